@@ -125,6 +125,8 @@ SYMBOLS = {
     "apt_gat_block": (_I, [_P, _I64, _P, _I, _P, _I64, _I, _I64, _I, _P, _P, C.c_float, _P, _P, _P]),
     "apt_gat_block_backward": (_I, [_P, _I64, _I, _P, _I64, _I, _I64, _I, _P, _P, C.c_float, _P, _P, _P, _P, _P, _P, _P]),
     "apt_spmm_heads": (_I, [_P, _P, _I64, _P, _I64, _P, _P, _I, _I64, _I, _I, _P, _I64, _P, _P, _P, _P]),
+    "apt_linear_wgrad_workspace_bytes": (_SZ, [_I64, _I64, _I64, _I]),
+    "apt_linear_wgrad": (_I, [_P, _P, _I64, _I64, _I64, _I, _P, _P, _P, _SZ, _P]),
     "apt_time_next_sample": (_I, [_I, _P, _P]),
     "apt_epoch_create": (_I, [C.POINTER(CEpochDesc), C.POINTER(_P)]),
     "apt_epoch_begin": (_I, [_P, _P, _I64, _U64, _P]),
@@ -1027,3 +1029,18 @@ def spmm_heads(row, col, x, head_weights, num_out, weight_row=None, grouped=Fals
     if flat:
         out = out.squeeze(1)
     return out if out2 is None else (out, out2)
+
+
+def linear_wgrad(dy, x, want_bias=True):
+    """dw = dy^T x and db = dy.sum(0) of y = x w^T + b: dy [m, n], x [m, k], fp32 or bf16 -> (dw [n, k], db [n] or None)."""
+    dy, x = _feat2d(dy, "dy"), _feat2d(x, "x")
+    if dy.dtype != x.dtype or dy.shape[0] != x.shape[0]:
+        raise AptError("linear_wgrad: dy and x differ in dtype or rows")
+    m, n, k = dy.shape[0], dy.shape[1], x.shape[1]
+    dw = torch.empty((n, k), dtype=x.dtype, device=x.device)
+    db = torch.empty(n, dtype=x.dtype, device=x.device) if want_bias else None
+    need = int(lib().apt_linear_wgrad_workspace_bytes(m, n, k, x.element_size()))
+    ws = torch.empty(max(need, 16), dtype=torch.uint8, device=x.device)
+    check(lib().apt_linear_wgrad(_ptr(dy), _ptr(x), m, n, k, x.element_size(), _ptr(dw), _ptr(db), _ptr(ws), ws.numel(),
+                                 _stream()))
+    return dw, db

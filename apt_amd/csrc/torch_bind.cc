@@ -926,6 +926,62 @@ Tensor UMulV(Tensor coo_row, Tensor coo_col, Tensor lhs, Tensor rhs, Tensor coo_
   return sddmm(1, coo_row, coo_col, lhs, rhs, coo_offset, lhs_offset, rhs_offset);
 }
 
+// ---------------------------------------------------------------- dense layers over a block's rows
+namespace {
+
+// Gradients of the weight [n, k] and the bias of y = x w^T + b (apt_linear_wgrad).
+std::tuple<Tensor, Tensor> linear_wgrad(const Tensor& dy_in, const Tensor& x_in, bool want_bias) {
+  auto dy = dy_in.contiguous(), x = x_in.contiguous();
+  const int64_t m = x.size(0), n = dy.size(1), k = x.size(1);
+  const int es = static_cast<int>(x.element_size());
+  const size_t need = apt_linear_wgrad_workspace_bytes(m, n, k, es);
+  TORCH_CHECK(need > 0, "npc: block_linear: a weight of ", n, " x ", k, " is out of range");
+  auto ws = torch::empty({static_cast<int64_t>(need)}, x.options().dtype(torch::kUInt8));
+  auto dw = torch::empty({n, k}, x.options());
+  Tensor db;
+  if (want_bias) db = torch::empty({n}, x.options());
+  check(apt_linear_wgrad(dy.data_ptr(), x.data_ptr(), m, n, k, es, dw.data_ptr(), want_bias ? db.data_ptr() : nullptr,
+                         ws.data_ptr(), need, stream()));
+  return {dw, db};
+}
+
+// y = x w^T + b (or x w with `kn`: w is [k, n]).  The product itself and the gradient towards x are plain GEMMs and
+// go to the library; the gradient of the weight reduces over the block's rows and has a kernel of its own.
+struct BlockLinearFn : public torch::autograd::Function<BlockLinearFn> {
+  static Tensor forward(torch::autograd::AutogradContext* ctx, const Tensor& x, const Tensor& w,
+                        const std::optional<Tensor>& b, bool kn) {
+    ctx->save_for_backward({x, w});
+    ctx->saved_data["kn"] = kn;
+    ctx->saved_data["bias"] = b.has_value();
+    return kn ? at::mm(x, w) : at::linear(x, w, b);
+  }
+  static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx,
+                                                 torch::autograd::variable_list grads) {
+    const auto saved = ctx->get_saved_variables();
+    const Tensor &x = saved[0], &w = saved[1], &dy = grads[0];
+    const bool kn = ctx->saved_data["kn"].toBool(), bias = ctx->saved_data["bias"].toBool();
+    Tensor dx, dw, db;
+    if (ctx->needs_input_grad(0)) dx = kn ? dy.mm(w.t()) : dy.mm(w);
+    if (torch::GradMode::is_enabled()) {   // a graph of the gradients is wanted: operations that carry one
+      dw = kn ? x.t().mm(dy) : dy.t().mm(x);
+      if (bias) db = dy.sum(0);
+    } else if (ctx->needs_input_grad(1) || bias) {
+      std::tie(dw, db) = kn ? linear_wgrad(x, dy, false) : linear_wgrad(dy, x, bias);
+    }
+    return {dx, dw, db, Tensor()};
+  }
+};
+
+}  // namespace
+
+Tensor BlockLinear(const Tensor& x, const Tensor& w, const std::optional<Tensor>& b, bool kn) {
+  TORCH_CHECK(x.is_cuda() && w.is_cuda() && x.dim() == 2 && w.dim() == 2 && x.scalar_type() == w.scalar_type() &&
+                  (x.scalar_type() == torch::kFloat32 || x.scalar_type() == torch::kBFloat16),
+              "npc: block_linear needs 2-D fp32 or bf16 GPU tensors of one dtype");
+  TORCH_CHECK(!kn || !b.has_value(), "npc: block_linear: a [k, n] weight takes no bias");
+  return BlockLinearFn::apply(x, w, b, kn);
+}
+
 // ---------------------------------------------------------------- peers only
 #define NPC_NEEDS_PEERS(name)                                                              \
   TORCH_CHECK(false, "npc." name " talks to other GPUs over NCCL in the reference; this " \
@@ -980,6 +1036,7 @@ TORCH_LIBRARY(npc, m) {
       .def("sample_neighbors", &SampleNeighbors)
       .def("sample_blocks", &SampleBlocks)
       .def("block_formats", &BlockFormats)
+      .def("block_linear", &BlockLinear)
       .def("cluster_and_permute", &ClusterAndPermuteLocal)
       .def("register_graph_partition", &RegisterGraphPartition)
       .def("set_topology", &SetTopology)

@@ -39,6 +39,23 @@ class BlockAggregate(torch.autograd.Function):
         return None, dX.to(dZ.dtype), None
 
 
+def _trains_natively(x, weight):
+    """Whether the gradient of `weight` can come from the library's kernel: a training step on fp32 or bf16 GPU rows
+    of the weight's dtype (autocast picks dtypes of its own)."""
+    return (x.is_cuda and x.dim() == 2 and x.dtype == weight.dtype and x.dtype in (torch.float32, torch.bfloat16)
+            and torch.is_grad_enabled() and weight.requires_grad and not torch.is_autocast_enabled("cuda"))
+
+
+def _linear(layer, x):
+    """layer(x); a plain nn.Linear takes its weight and bias gradients from npc.block_linear (hooks, subclasses and
+    everything else go through the module)."""
+    if (type(layer) is nn.Linear and _trains_natively(x, layer.weight)
+            and not (layer._forward_hooks or layer._forward_pre_hooks or layer._backward_hooks
+                     or layer._backward_pre_hooks)):
+        return torch.ops.npc.block_linear(x, layer.weight, layer.bias, False)
+    return layer(x)
+
+
 class SAGEConv(nn.Module):
     """GraphSAGE layer, mean aggregator, with the reference's arithmetic
     (python/npc/model/sageconv.py:118-188): fc_self(h_dst) + fc_neigh(mean of
@@ -58,10 +75,10 @@ class SAGEConv(nn.Module):
         """feat: [block.num_src, in_feats]; the first num_dst rows are the destinations."""
         h_self = feat[:block.num_dst]
         if self.in_feats > self.out_feats:
-            h_neigh = BlockAggregate.apply(block, self.fc_neigh(feat), True)
+            h_neigh = BlockAggregate.apply(block, _linear(self.fc_neigh, feat), True)
         else:
-            h_neigh = self.fc_neigh(BlockAggregate.apply(block, feat, True))
-        rst = self.fc_self(h_self) + h_neigh
+            h_neigh = _linear(self.fc_neigh, BlockAggregate.apply(block, feat, True))
+        rst = _linear(self.fc_self, h_self) + h_neigh
         return self.activation(rst) if self.activation is not None else rst
 
 
@@ -84,7 +101,9 @@ class GraphConv(nn.Module):
         fanout = float(block.fanout)
         if self.norm in ("left", "both"):
             feat = feat * (fanout ** -0.5 if self.norm == "both" else 1.0 / fanout)
-        rst = BlockAggregate.apply(block, torch.matmul(feat, self.weight), False)
+        h = (torch.ops.npc.block_linear(feat, self.weight, None, True) if _trains_natively(feat, self.weight)
+             else torch.matmul(feat, self.weight))
+        rst = BlockAggregate.apply(block, h, False)
         if self.norm in ("right", "both"):
             rst = rst * (fanout ** -0.5 if self.norm == "both" else 1.0 / fanout)
         if self.bias is not None:
@@ -145,7 +164,7 @@ class GATConv(nn.Module):
         nn.init.xavier_normal_(self.attn_r, gain=gain)
 
     def forward(self, block, feat):
-        ft = self.fc(feat).view(block.num_src, self.num_heads, self.out_feats).contiguous()
+        ft = _linear(self.fc, feat).view(block.num_src, self.num_heads, self.out_feats).contiguous()
         if torch.is_grad_enabled() and (ft.requires_grad or self.attn_l.requires_grad):
             el = (ft * self.attn_l).sum(-1)
             er = (ft[:block.num_dst] * self.attn_r).sum(-1)

@@ -778,6 +778,19 @@ int apt_spmm_heads(const int64_t* coo_row, const int64_t* coo_col, int64_t num_e
                    float* out, int64_t num_out_rows, const float* head_weights2, float* out2,
                    const int64_t* out_indptr, void* stream);
 
+/* Gradients of a dense layer y = x w^T + b over a block's rows (the fc_self /
+ * fc_neigh / fc of python/npc/model/sageconv.py:118-188 and gatconv.py:207-236,
+ * whose gradients the reference gets from cuBLAS through torch):
+ *   dw[n, k] = sum_m dy[m, n] * x[m, k],   db[n] = sum_m dy[m, n]
+ * dy [m, n], x [m, k], dw [n, k] and db [n] (NULL = not wanted) are row-major,
+ * fp32 (elem_size 4) or bf16 (2); sums are fp32 in an order that depends on the
+ * sizes only (reproducible).  n, k <= 2^20, n * k <= 2^30.  workspace:
+ * apt_linear_wgrad_workspace_bytes(m, n, k, elem_size) bytes of device scratch,
+ * 16-byte aligned; 0 = sizes out of range. */
+size_t apt_linear_wgrad_workspace_bytes(int64_t m, int64_t n, int64_t k, int elem_size);
+int apt_linear_wgrad(const void* dy, const void* x, int64_t m, int64_t n, int64_t k, int elem_size,
+                     void* dw, void* db, void* workspace, size_t workspace_bytes, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

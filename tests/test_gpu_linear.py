@@ -1,0 +1,60 @@
+"""Dense layers over a block's rows: weight and bias gradients of the library's kernel against float64, at the
+edges of its tiles (64 columns), steps (16 / 32 rows), vector widths and splits."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("m,n,k", [(1, 1, 1), (31, 64, 64), (33, 65, 63), (64, 16, 50), (65, 10, 32), (1000, 47, 256),
+                                   (4099, 188, 101), (9001, 256, 100), (2500, 320, 514), (70000, 3, 7)])
+def test_linear_wgrad(capi, m, n, k, dtype):
+    gen = torch.Generator(device=DEV).manual_seed(m + n + k)
+    dy = torch.randn(m, n, generator=gen, device=DEV).to(dtype)
+    x = torch.randn(m, k, generator=gen, device=DEV).to(dtype)
+    dw, db = capi.linear_wgrad(dy, x)
+    want_w, want_b = dy.double().t() @ x.double(), dy.double().sum(0)
+    # fp32 sums of m products of magnitude ~1: error ~ eps * m at the worst, sqrt(m) by chance; bf16 results round at 2^-9
+    tol = (2.0 ** -8 if dtype == torch.bfloat16 else 0.0)
+    for got, want in ((dw, want_w), (db, want_b)):
+        bound = tol * want.abs() + 2.0 ** -22 * (m ** 0.5) * 16 + 2.0 ** -22 * want.abs()
+        assert got.dtype == dtype and bool(((got.double() - want).abs() <= bound).all())
+    again, _ = capi.linear_wgrad(dy, x, want_bias=False)
+    assert torch.equal(again, dw)      # a fixed order of the sums
+
+
+def test_linear_wgrad_unaligned_and_empty(capi):
+    base = torch.randn(500 * 64 + 1, device=DEV)
+    dy = base[1:].view(500, 64)        # rows start at 4-byte, not 16-byte, addresses
+    x = torch.randn(500, 64, device=DEV)
+    dw, db = capi.linear_wgrad(dy, x)
+    assert torch.allclose(dw.double(), dy.double().t() @ x.double(), atol=1e-3) and torch.allclose(db, dy.sum(0), atol=1e-3)
+    dw, db = capi.linear_wgrad(torch.empty(0, 5, device=DEV), torch.empty(0, 7, device=DEV))
+    assert dw.shape == (5, 7) and not dw.any() and not db.any()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("kn", [False, True])
+def test_block_linear_gradients(dtype, kn):
+    import apt_amd  # noqa: F401  (loads the operators)
+    gen = torch.Generator(device=DEV).manual_seed(3)
+    x = torch.randn(777, 40, generator=gen, device=DEV).to(dtype).requires_grad_(True)
+    w = torch.randn((40, 24) if kn else (24, 40), generator=gen, device=DEV).to(dtype).requires_grad_(True)
+    b = None if kn else torch.randn(24, generator=gen, device=DEV).to(dtype).requires_grad_(True)
+    up = torch.randn(777, 24, generator=gen, device=DEV).to(dtype)
+    params = [x, w] + ([] if b is None else [b])
+    y = torch.ops.npc.block_linear(x, w, b, kn)
+    plain = x @ w if kn else torch.nn.functional.linear(x, w, b)
+    assert torch.equal(y, plain)
+    got = torch.autograd.grad(y, params, up)
+    want = torch.autograd.grad(plain, params, up)
+    for g, r in zip(got, want):
+        assert g.dtype == r.dtype and torch.allclose(g.float(), r.float(), rtol=2e-2 if dtype == torch.bfloat16 else 1e-5,
+                                                     atol=(0.3 if dtype == torch.bfloat16 else 1e-3))
+    # gradients of gradients still have a graph
+    y = torch.ops.npc.block_linear(x, w, b, kn)
+    gw, = torch.autograd.grad(y.float().square().sum(), w, create_graph=True)
+    gx, = torch.autograd.grad(gw.float().sum(), x)
+    assert gx.shape == x.shape and bool(torch.isfinite(gx).all())
