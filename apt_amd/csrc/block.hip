@@ -10,15 +10,20 @@
 //   CSC  csc_indptr over destinations; its indices are COO row, edge ids 0..E-1
 //   CSR  csr_indptr over sources, csr_indices = destination, csr_eids = COO
 //        position, edges of one source in increasing edge id
-// COO/CSC are a stream compaction (count per tile -> place).  CSR is a stable
-// least-significant-digit radix sort of (source, edge id) by source, 8 bits per
-// pass (histogram per tile -> scatter); a workgroup ranks its tile with wave
-// ballots, so equal keys keep their order and the result is reproducible (no
-// atomic tickets).  A block of a mini-batch has few tiles, so the place and
-// scatter workgroups add up the counts of the tiles before them themselves
-// (a few KB from L2) instead of waiting for a scan kernel: every launch saved
-// is worth more than the arithmetic here.  Large inputs take separate scan
-// launches.
+// COO/CSC are a stream compaction (count per tile -> place).  CSR of the blocks a
+// sampler makes is a partition by source range carried along with that
+// compaction, then a counting sort of every range in one workgroup (below, "CSR by
+// source ranges"): four launches for all three formats.  Blocks of more than 5 M
+// sources, 8 M slots or 2 M destinations take a stable least-significant-digit radix
+// sort of (source, edge id) by source, 8 bits per pass (histogram per tile ->
+// scatter).  Everywhere a workgroup ranks its tile with wave ballots, so equal keys
+// keep their order and the result is reproducible (no atomic tickets).  A block
+// of a mini-batch has few tiles, so the place and scatter workgroups add up the
+// counts of the tiles before them themselves (a few KB from L2) instead of waiting
+// for a scan kernel: every launch saved is worth more than the arithmetic here.
+// Large inputs take separate scan launches.
+#include <algorithm>
+
 #include "common.hpp"
 
 namespace apt {
@@ -446,6 +451,426 @@ __global__ __launch_bounds__(kSortBlock) void radix_scatter_kernel(SortParams p)
   }
 }
 
+// ---------------------------------------------------- CSR by source ranges
+// Sources are cut into ranges.  The compaction's count pass also counts a tile's
+// edges per range, one launch turns the counts into prefixes over the tiles, the
+// place pass (which knows an edge's id, source and destination) puts a packed
+// record of every edge into its range's part of a scratch array, in edge order, and
+// one workgroup per range sorts its records by source in LDS and writes offsets,
+// destinations and edge ids.  Two stable passes instead of three to four, and none
+// of them over a few tiles only (a radix pass over the 260 k edges of a batch of
+// 1024 is 64 workgroups on 256 CUs).  All three formats of a block, with radix
+// passes / with ranges, sizes exact: 8 k edges 40 / 22 us, 22 k 41 / 25, 260 k
+// (120 k sources) 79 / 33, 740 k (240 k) 88 / 49, 940 k (460 k) 89 / 50 us.
+// The relabel numbers nodes by first occurrence, so hubs have small ids and the
+// edges per source fall off about as 1 / id (2.4 M-node graph, 4096 seeds: 40 edges
+// per source at id 4500, 5 at 30 k, 1.4 at 200 k), and buffers sized by upper bounds
+// end in ids that do not occur.  Ranges of equal width would leave one workgroup with
+// 37 k records (93 us); three widths keep them between a few hundred and a few thousand.
+constexpr int kRangeMaxShift = 11;
+constexpr int64_t kRangeFrom1 = int64_t{1} << 15, kRangeFrom2 = int64_t{1} << 18;   // first sources of pieces 1, 2
+constexpr int kRangeShift0 = 5, kRangeShift1 = 8, kRangeShift2 = 10;
+constexpr int kRangeMaxCount = 4520;          // ranges: 12 bytes of LDS each in the place pass
+constexpr int64_t kRangeMaxTiles = 4096;
+constexpr int kRangeKeyBits = kRangeMaxShift;
+constexpr int kRangeEdgeBits = 31;
+constexpr int64_t kRangeMaxDst = int64_t{1} << (64 - kRangeKeyBits - kRangeEdgeBits - 1);
+constexpr int kRangeSortBlock = 256;
+constexpr int kRangeSortWaves = kRangeSortBlock / kWave;
+constexpr int kRangeSortRounds = 8;
+constexpr int kRangeSortChunk = kRangeSortBlock * kRangeSortRounds;
+constexpr int kRangeScanGroups = 16;          // tile groups of a scan workgroup
+
+struct RangeParams {
+  int shift2;                 // width of piece 2
+  int ranges;
+  uint32_t* hist;             // [tiles][ranges]: edges of a tile per range, then their prefix over the tiles
+  uint32_t* total;            // [ranges]
+  uint32_t* start;            // [ranges + 1]: a range's first record
+  uint64_t* rec;              // edges by range: destination | source within the range | edge id
+  int64_t num_src;
+  int64_t* csr_indptr;
+  int64_t* csr_indices;
+  int64_t* csr_eids;
+};
+
+constexpr int kRangeCount0 = static_cast<int>(kRangeFrom1 >> kRangeShift0);
+constexpr int kRangeCount1 = static_cast<int>((kRangeFrom2 - kRangeFrom1) >> kRangeShift1);
+
+__host__ __device__ __forceinline__ int64_t range_index(int64_t src, int shift2) {
+  return src < kRangeFrom1   ? src >> kRangeShift0
+         : src < kRangeFrom2 ? kRangeCount0 + ((src - kRangeFrom1) >> kRangeShift1)
+                             : kRangeCount0 + kRangeCount1 + ((src - kRangeFrom2) >> shift2);
+}
+__device__ __forceinline__ int range_shift(const RangeParams& r, int b) {
+  return b < kRangeCount0 ? kRangeShift0 : b < kRangeCount0 + kRangeCount1 ? kRangeShift1 : r.shift2;
+}
+__device__ __forceinline__ int64_t range_first(const RangeParams& r, int b) {
+  return b < kRangeCount0 ? static_cast<int64_t>(b) << kRangeShift0
+         : b < kRangeCount0 + kRangeCount1 ? kRangeFrom1 + (static_cast<int64_t>(b - kRangeCount0) << kRangeShift1)
+                                           : kRangeFrom2 + (static_cast<int64_t>(b - kRangeCount0 - kRangeCount1) << r.shift2);
+}
+// Sources past num_src (they have no offset of their own) sort behind those that have one, in the last range.
+__device__ __forceinline__ int range_of(const RangeParams& r, int64_t src) {
+  const int64_t b = range_index(src, r.shift2);
+  return b < r.ranges ? static_cast<int>(b) : r.ranges - 1;
+}
+__device__ __forceinline__ uint32_t range_key(const RangeParams& r, int b, int64_t src) {
+  const int64_t k = src - range_first(r, b), last = (int64_t{1} << range_shift(r, b)) - 1;
+  return static_cast<uint32_t>(k < last ? k : last);
+}
+
+// Lanes of the wavefront that hold the same value (its low `bits` bits) as this one, among `valid` lanes.
+__device__ __forceinline__ uint64_t same_value(uint32_t v, int bits, bool valid) {
+  uint64_t peers = ballot(valid);
+  for (int b = 0; b < bits; ++b) {
+    const bool bit = (v >> b) & 1u;
+    const uint64_t set = ballot(valid && bit);
+    peers &= bit ? set : ~set;
+  }
+  return peers;
+}
+
+__global__ __launch_bounds__(kFmtBlock) void range_count_kernel(CompactParams p, RangeParams r) {
+  extern __shared__ uint32_t s_range[];   // [ranges]
+  __shared__ uint32_t s_wave[kFmtWaves];
+  const int64_t slots = actual_count(p.num_dst, p.num_dst_dev) * p.fanout;
+  const int64_t base = static_cast<int64_t>(blockIdx.x) * kCompactTile;
+  if (base >= slots && blockIdx.x != 0) return;   // block-uniform: nobody reads an inactive tile's counts
+  int64_t v[kCompactIters];
+#pragma unroll
+  for (int it = 0; it < kCompactIters; ++it) {
+    const int64_t s = base + it * kFmtBlock + threadIdx.x;
+    v[it] = s < slots ? p.relabeled[s] : -1;
+  }
+  for (int b = threadIdx.x; b < r.ranges; b += kFmtBlock) s_range[b] = 0;
+  __syncthreads();
+  uint32_t c = 0;
+#pragma unroll
+  for (int it = 0; it < kCompactIters; ++it) {
+    if (v[it] < 0) continue;
+    ++c;
+    atomicAdd(&s_range[range_of(r, v[it])], 1u);
+  }
+  uint32_t all;
+  block_exclusive(c, s_wave, all);   // (its barriers also complete the counts)
+  if (threadIdx.x == 0) p.tile_cnt[blockIdx.x] = all;
+  uint32_t* row = r.hist + static_cast<int64_t>(blockIdx.x) * r.ranges;
+  for (int b = threadIdx.x; b < r.ranges; b += kFmtBlock) row[b] = s_range[b];
+}
+
+// 64 ranges per workgroup, the tiles in kRangeScanGroups groups: a group adds up its tiles, the groups' sums are
+// put in order in LDS, and a second walk leaves the prefixes.
+__global__ __launch_bounds__(kWave * kRangeScanGroups) void range_scan_kernel(CompactParams p, RangeParams r) {
+  constexpr int kUnroll = 8;
+  __shared__ uint32_t s_sum[kRangeScanGroups][kWave];
+  const int lane = threadIdx.x % kWave, group = threadIdx.x / kWave;
+  const int b = blockIdx.x * kWave + lane;
+  const int64_t slots = actual_count(p.num_dst, p.num_dst_dev) * p.fanout;
+  const int tiles = static_cast<int>(ceil_div_dev(slots, kCompactTile));
+  const int per = (tiles + kRangeScanGroups - 1) / kRangeScanGroups;
+  const int t0 = group * per, t1 = min(t0 + per, tiles);
+  const bool live = b < r.ranges;
+  uint32_t sum = 0;
+  for (int t = t0; t < t1 && live; t += kUnroll) {
+    uint32_t c[kUnroll];
+#pragma unroll
+    for (int u = 0; u < kUnroll; ++u) c[u] = r.hist[static_cast<int64_t>(min(t + u, t1 - 1)) * r.ranges + b];
+#pragma unroll
+    for (int u = 0; u < kUnroll; ++u) sum += t + u < t1 ? c[u] : 0u;
+  }
+  s_sum[group][lane] = sum;
+  __syncthreads();
+  uint32_t run = 0, all = 0;
+#pragma unroll
+  for (int g = 0; g < kRangeScanGroups; ++g) {
+    const uint32_t c = s_sum[g][lane];
+    if (g < group) run += c;
+    all += c;
+  }
+  if (!live) return;
+  for (int t = t0; t < t1; t += kUnroll) {
+    uint32_t c[kUnroll];
+#pragma unroll
+    for (int u = 0; u < kUnroll; ++u) c[u] = r.hist[static_cast<int64_t>(min(t + u, t1 - 1)) * r.ranges + b];
+#pragma unroll
+    for (int u = 0; u < kUnroll; ++u)
+      if (t + u < t1) {
+        r.hist[static_cast<int64_t>(t + u) * r.ranges + b] = run;
+        run += c[u];
+      }
+  }
+  if (group == 0) r.total[b] = all;
+}
+
+// The compaction's place pass (as fmt_place_kernel) with the partition: a wavefront owns consecutive slots, so that
+// walking the wavefronts, and the iterations inside one, is edge order.
+__global__ __launch_bounds__(kFmtBlock) void range_place_kernel(CompactParams p, RangeParams r) {
+  extern __shared__ uint32_t s_range[];
+  uint32_t* s_base = s_range;                                                // [ranges]
+  uint32_t* s_cnt2 = s_range + r.ranges;                                     // [waves][ranges / 2], 16-bit counts
+  const int words = (r.ranges + 1) / 2;                                      // 32-bit words of a wave's counts
+  __shared__ uint32_t s_edges[kFmtWaves * kCompactIters];
+  __shared__ uint32_t s_wave[kFmtWaves];
+  const int lane = lane_id();
+  const int wave = threadIdx.x / kWave;
+  const int64_t slots = actual_count(p.num_dst, p.num_dst_dev) * p.fanout;
+  const int64_t upper = p.num_dst * p.fanout;
+  const int64_t base = static_cast<int64_t>(blockIdx.x) * kCompactTile + wave * (kCompactIters * kWave);
+  int64_t v[kCompactIters];
+  uint32_t below[kCompactIters];
+#pragma unroll
+  for (int it = 0; it < kCompactIters; ++it) {
+    const int64_t s = base + it * kWave + lane;
+    v[it] = s < slots ? p.relabeled[s] : -1;
+  }
+  for (int i = threadIdx.x; i < words * kFmtWaves; i += kFmtBlock) s_cnt2[i] = 0;
+  __syncthreads();
+  uint32_t* cnt = s_cnt2 + wave * words;
+#pragma unroll
+  for (int it = 0; it < kCompactIters; ++it) {
+    const uint64_t m = ballot(v[it] >= 0);
+    below[it] = rank_below(m);
+    if (lane == 0) s_edges[wave * kCompactIters + it] = __popcll(m);
+    if (v[it] >= 0) {   // at most 512 per wavefront: a 16-bit half never overflows into the other
+      const int b = range_of(r, v[it]);
+      atomicAdd(&cnt[b >> 1], (b & 1) ? 0x10000u : 1u);
+    }
+  }
+  // edges of the tiles before this one, and of all tiles
+  const int64_t active = ceil_div_dev(slots, kCompactTile);
+  uint32_t before = 0, total = 0;
+  for (int64_t t = threadIdx.x; t < active; t += kFmtBlock) {
+    const uint32_t c = p.tile_cnt[t];
+    total += c;
+    if (t < blockIdx.x) before += c;
+  }
+  uint32_t first, all_total;
+  block_exclusive(before, s_wave, first);
+  block_exclusive(total, s_wave, all_total);
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    *p.num_edges_dev = all_total;
+    p.csc_indptr[p.num_dst] = all_total;
+  }
+  // where this tile's edges of a range start: the ranges before it, and the tiles before this one
+  const bool live = blockIdx.x < active || blockIdx.x == 0;   // block-uniform (workgroup 0 also writes the starts)
+  if (live) {
+    // (loads of a thread in batches: one at a time, a workgroup of a large launch would spend its time on them)
+    constexpr int kBatch = 6;
+    for (int b = threadIdx.x; b < r.ranges; b += kBatch * kFmtBlock) {
+      uint32_t c[kBatch];
+#pragma unroll
+      for (int u = 0; u < kBatch; ++u) c[u] = r.total[min(b + u * kFmtBlock, r.ranges - 1)];
+#pragma unroll
+      for (int u = 0; u < kBatch; ++u)
+        if (b + u * kFmtBlock < r.ranges) s_base[b + u * kFmtBlock] = c[u];
+    }
+    __syncthreads();
+    const int per = (r.ranges + kFmtBlock - 1) / kFmtBlock;
+    const int b0 = threadIdx.x * per, b1 = min(b0 + per, r.ranges);
+    uint32_t mine = 0;
+    for (int b = b0; b < b1; ++b) mine += s_base[b];
+    uint32_t all;
+    uint32_t run = block_exclusive(mine, s_wave, all);
+    for (int b = b0; b < b1; ++b) {
+      const uint32_t c = s_base[b];
+      s_base[b] = run;
+      run += c;
+    }
+    __syncthreads();
+    const uint32_t* row = r.hist + static_cast<int64_t>(blockIdx.x) * r.ranges;
+    for (int b = threadIdx.x; b < r.ranges; b += kBatch * kFmtBlock) {
+      uint32_t c[kBatch];
+#pragma unroll
+      for (int u = 0; u < kBatch; ++u) c[u] = row[min(b + u * kFmtBlock, r.ranges - 1)];
+#pragma unroll
+      for (int u = 0; u < kBatch; ++u) {
+        const int i = b + u * kFmtBlock;
+        if (i >= r.ranges) break;
+        if (blockIdx.x == 0) r.start[i] = s_base[i];
+        s_base[i] += c[u];
+      }
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) r.start[r.ranges] = all;
+    // counts of a wavefront -> counts of the wavefronts before it
+    for (int i = threadIdx.x; i < words; i += kFmtBlock) {
+      uint32_t sum = 0;
+#pragma unroll
+      for (int w = 0; w < kFmtWaves; ++w) {
+        const uint32_t c = s_cnt2[w * words + i];
+        s_cnt2[w * words + i] = sum;
+        sum += c;
+      }
+    }
+  }
+  static_assert(kCompactIters * kFmtWaves <= kWave, "one wavefront scans the tile's per-wave counts");
+  if (wave == 0) {
+    const uint32_t c = lane < kCompactIters * kFmtWaves ? s_edges[lane] : 0u;
+    uint32_t incl = c;
+#pragma unroll
+    for (int off = 1; off < kCompactIters * kFmtWaves; off <<= 1) {
+      const uint32_t y = __shfl_up(incl, off, kWave);
+      if (lane >= off) incl += y;
+    }
+    if (lane < kCompactIters * kFmtWaves) s_edges[lane] = first + incl - c;
+  }
+  __syncthreads();
+  const int bits = 32 - __clz(r.ranges - 1 > 0 ? r.ranges - 1 : 1);
+  volatile uint16_t* pos = reinterpret_cast<volatile uint16_t*>(cnt);
+  const uint32_t fan = static_cast<uint32_t>(p.fanout);
+#pragma unroll
+  for (int it = 0; it < kCompactIters; ++it) {
+    const int64_t s = base + it * kWave + lane;
+    const int64_t e = static_cast<int64_t>(s_edges[wave * kCompactIters + it]) + below[it];
+    const uint32_t d = static_cast<uint32_t>(s) / fan;
+    if (s < upper && static_cast<uint32_t>(s) - d * fan == 0) p.csc_indptr[d] = e;
+    const bool valid = v[it] >= 0;
+    if (ballot(valid) == 0) continue;   // wave-uniform
+    const uint32_t b = valid ? static_cast<uint32_t>(range_of(r, v[it])) : 0u;
+    const uint64_t peers = same_value(b, bits, valid);
+    const uint32_t rank = rank_below(peers);
+    uint32_t at = 0;
+    if (valid) at = pos[b] + rank;
+    __builtin_amdgcn_wave_barrier();
+    if (valid && rank + 1 == static_cast<uint32_t>(__popcll(peers))) pos[b] = static_cast<uint16_t>(at + 1);
+    __builtin_amdgcn_wave_barrier();
+    if (valid) {
+      p.coo_row[e] = v[it];
+      p.coo_col[e] = d;
+      r.rec[s_base[b] + at] = (static_cast<uint64_t>(d) << (kRangeKeyBits + kRangeEdgeBits)) |
+                              (static_cast<uint64_t>(range_key(r, static_cast<int>(b), v[it])) << kRangeEdgeBits) | static_cast<uint64_t>(e);
+    }
+  }
+}
+
+// One workgroup per range: stable counting sort of its records by source.  A range of a sampled block has about a
+// thousand; a range with more than a chunk of them (hubs) is walked chunk by chunk, after a counting walk.
+__global__ __launch_bounds__(kRangeSortBlock) void range_sort_kernel(RangeParams r) {
+  extern __shared__ uint32_t s_range[];
+  const int shift = range_shift(r, blockIdx.x);
+  const int keys = 1 << shift;
+  const int words = keys / 2;
+  uint32_t* s_start = s_range;              // [keys]: next position of a key's first record not yet placed
+  uint32_t* s_cnt2 = s_range + keys;        // [waves][keys / 2], 16-bit counts
+  __shared__ uint32_t s_wave[kRangeSortWaves];
+  const int tid = threadIdx.x, lane = lane_id(), wave = tid / kWave;
+  auto exclusive = [&](uint32_t x, uint32_t& all) {   // over the workgroup
+    uint32_t incl = x;
+#pragma unroll
+    for (int off = 1; off < kWave; off <<= 1) {
+      const uint32_t y = __shfl_up(incl, off, kWave);
+      if (lane >= off) incl += y;
+    }
+    __syncthreads();
+    if (lane == kWave - 1) s_wave[wave] = incl;
+    __syncthreads();
+    uint32_t before = 0;
+    all = 0;
+#pragma unroll
+    for (int w = 0; w < kRangeSortWaves; ++w) {
+      const uint32_t c = s_wave[w];
+      if (w < wave) before += c;
+      all += c;
+    }
+    return before + incl - x;
+  };
+  const uint32_t before = r.start[blockIdx.x], n = r.start[blockIdx.x + 1] - before;
+  const int64_t src0 = range_first(r, blockIdx.x);
+  if (n == 0) {
+    for (int k = tid; k < keys; k += kRangeSortBlock)
+      if (src0 + k <= r.num_src) r.csr_indptr[src0 + k] = before;
+    return;
+  }
+  const uint64_t* rec = r.rec + before;
+  auto key_of = [&](uint64_t x) { return static_cast<uint32_t>(x >> kRangeEdgeBits) & ((1u << kRangeKeyBits) - 1); };
+  const bool single = n <= kRangeSortChunk;   // block-uniform
+  const int per = (keys + kRangeSortBlock - 1) / kRangeSortBlock;
+  // counts per key in s_start -> the key's first position, and its offset
+  auto starts = [&]() {
+    const int k0 = tid * per, k1 = min(k0 + per, keys);
+    uint32_t mine = 0, all;
+    for (int k = k0; k < k1; ++k) mine += s_start[k];
+    uint32_t run = exclusive(mine, all);
+    for (int k = k0; k < k1; ++k) {
+      const uint32_t c = s_start[k];
+      s_start[k] = run;
+      if (src0 + k <= r.num_src) r.csr_indptr[src0 + k] = static_cast<int64_t>(before) + run;
+      run += c;
+    }
+  };
+  if (!single) {
+    for (int k = tid; k < keys; k += kRangeSortBlock) s_start[k] = 0;
+    __syncthreads();
+    for (uint32_t i = tid; i < n; i += kRangeSortBlock) atomicAdd(&s_start[key_of(rec[i])], 1u);
+    __syncthreads();
+    starts();
+  }
+  uint32_t* cnt = s_cnt2 + wave * words;
+  volatile uint16_t* pos = reinterpret_cast<volatile uint16_t*>(cnt);
+  for (uint32_t c0 = 0; c0 < n; c0 += kRangeSortChunk) {
+    const uint32_t left = min(n - c0, static_cast<uint32_t>(kRangeSortChunk));
+    const int rounds = static_cast<int>((left + kRangeSortBlock - 1) / kRangeSortBlock);
+    uint64_t x[kRangeSortRounds];
+#pragma unroll
+    for (int q = 0; q < kRangeSortRounds; ++q) {
+      const uint32_t i = (wave * rounds + q) * kWave + lane;
+      x[q] = q < rounds && i < left ? rec[c0 + i] : ~0ull;
+    }
+    __syncthreads();
+    for (int i = tid; i < words * kRangeSortWaves; i += kRangeSortBlock) s_cnt2[i] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < kRangeSortRounds; ++q)
+      if (x[q] != ~0ull) {
+        const uint32_t k = key_of(x[q]);
+        atomicAdd(&cnt[k >> 1], (k & 1) ? 0x10000u : 1u);
+      }
+    __syncthreads();
+    // counts of a wavefront -> counts of the wavefronts before it (a chunk's 2048 fit 16 bits)
+    for (int i = tid; i < words; i += kRangeSortBlock) {
+      uint32_t sum = 0;
+#pragma unroll
+      for (int w = 0; w < kRangeSortWaves; ++w) {
+        const uint32_t c = s_cnt2[w * words + i];
+        s_cnt2[w * words + i] = sum;
+        sum += c;
+      }
+      if (single) {
+        s_start[2 * i] = sum & 0xffffu;
+        s_start[2 * i + 1] = sum >> 16;
+      }
+    }
+    __syncthreads();
+    if (single) {
+      starts();
+      __syncthreads();
+    }
+#pragma unroll
+    for (int q = 0; q < kRangeSortRounds; ++q) {
+      if (q >= rounds) break;   // block-uniform
+      const bool valid = x[q] != ~0ull;
+      const uint32_t k = valid ? key_of(x[q]) : 0u;
+      const uint64_t peers = same_value(k, shift, valid);
+      const uint32_t rank = rank_below(peers);
+      uint32_t at = 0;
+      if (valid) at = pos[k] + rank;
+      __builtin_amdgcn_wave_barrier();
+      if (valid && rank + 1 == static_cast<uint32_t>(__popcll(peers))) pos[k] = static_cast<uint16_t>(at + 1);
+      __builtin_amdgcn_wave_barrier();
+      if (valid) {
+        const int64_t to = static_cast<int64_t>(before) + s_start[k] + at;
+        r.csr_eids[to] = static_cast<int64_t>(x[q] & ((1ull << kRangeEdgeBits) - 1));
+        r.csr_indices[to] = static_cast<int64_t>(x[q] >> (kRangeKeyBits + kRangeEdgeBits));
+      }
+    }
+    if (c0 + kRangeSortChunk >= n) break;
+    __syncthreads();
+    // every wavefront has moved its counters past its records: the last one's stand at the chunk's totals
+    const uint16_t* last = reinterpret_cast<const uint16_t*>(s_cnt2 + (kRangeSortWaves - 1) * words);
+    for (int k = tid; k < keys; k += kRangeSortBlock) s_start[k] += last[k];
+  }
+}
+
 // csr_indptr[s] = first position of a key >= s in the sorted keys, s in [0, num_src].
 // Position e starts a run of its key k when the key before it, kp, is smaller: then e is the answer for every
 // s in (kp, k].  One lane per position writes those entries itself when they are few (in a sampled block nearly
@@ -503,10 +928,23 @@ static size_t fmt_align(size_t x) { return (x + 255) / 256 * 256; }
 struct FmtLayout {
   int64_t slots, ctiles, stiles;
   size_t tile_cnt_off, sums_off, hist_off, bin_total_off, key_off[2], pay_off[2], total;
+  int range_shift2, ranges;   // CSR by source ranges; ranges == 0: by radix passes
+  size_t start_off, rec_off;
 };
 
-static FmtLayout fmt_layout(int64_t num_dst, int fanout, bool csr) {
+// The last piece's ranges are as narrow as their number allows.  num_src itself has a range: the last offset.
+static void choose_ranges(int64_t num_dst, int64_t num_src, FmtLayout& L) {
+  L.range_shift2 = kRangeShift2;
+  while (L.range_shift2 < kRangeMaxShift && range_index(num_src, L.range_shift2) >= kRangeMaxCount) ++L.range_shift2;
+  const int64_t ranges = range_index(num_src, L.range_shift2) + 1;
+  const bool fits = ranges <= kRangeMaxCount && L.ctiles <= kRangeMaxTiles && num_dst <= kRangeMaxDst &&
+                    tuning_block_fused_scan();
+  L.ranges = fits ? static_cast<int>(ranges) : 0;
+}
+
+static FmtLayout fmt_layout(int64_t num_dst, int fanout, int64_t num_src, bool csr) {
   FmtLayout L;
+  L.ranges = 0;
   L.slots = num_dst * fanout;
   L.ctiles = ceil_div(L.slots > 0 ? L.slots : 1, kCompactTile);
   L.stiles = ceil_div(L.slots > 0 ? L.slots : 1, kSortTile);
@@ -514,7 +952,13 @@ static FmtLayout fmt_layout(int64_t num_dst, int fanout, bool csr) {
   L.tile_cnt_off = off; off = fmt_align(off + sizeof(uint32_t) * static_cast<size_t>(L.ctiles));
   L.sums_off = off;     off = fmt_align(off + sizeof(uint32_t) * kScanChunk);
   L.hist_off = off;
-  if (csr) {
+  if (csr) choose_ranges(num_dst, num_src, L);
+  if (csr && L.ranges > 0) {
+    off = fmt_align(off + sizeof(uint32_t) * static_cast<size_t>(L.ctiles) * L.ranges);
+    L.bin_total_off = off; off = fmt_align(off + sizeof(uint32_t) * L.ranges);
+    L.start_off = off;     off = fmt_align(off + sizeof(uint32_t) * (L.ranges + 1));
+    L.rec_off = off;       off = fmt_align(off + sizeof(uint64_t) * static_cast<size_t>(L.slots > 0 ? L.slots : 1));
+  } else if (csr) {
     off = fmt_align(off + sizeof(uint32_t) * static_cast<size_t>(L.stiles) * kRadix);
     L.bin_total_off = off; off = fmt_align(off + sizeof(uint32_t) * kRadix);
     const size_t buf = sizeof(uint32_t) * static_cast<size_t>(L.slots > 0 ? L.slots : 1);
@@ -537,7 +981,7 @@ static bool fmt_sizes_ok(int64_t num_dst, int fanout, int64_t num_src) {
 extern "C" size_t apt_block_workspace_bytes(int64_t num_dst, int fanout, int64_t num_src, int want_csr) {
   using namespace apt;
   if (!fmt_sizes_ok(num_dst, fanout, num_src)) return 0;
-  return fmt_layout(num_dst, fanout, want_csr != 0).total;
+  return fmt_layout(num_dst, fanout, num_src, want_csr != 0).total;
 }
 
 extern "C" int apt_block_formats(const int64_t* relabeled, int64_t num_dst, const int64_t* num_dst_dev,
@@ -555,7 +999,7 @@ extern "C" int apt_block_formats(const int64_t* relabeled, int64_t num_dst, cons
   APT_REQUIRE(!csr || (csr_indices != nullptr && csr_eids != nullptr), APT_EINVAL,
               "apt_block_formats: csr_indices / csr_eids is NULL");
   hipStream_t st = static_cast<hipStream_t>(stream);
-  const FmtLayout L = fmt_layout(num_dst, fanout, csr);
+  const FmtLayout L = fmt_layout(num_dst, fanout, num_src, csr);
   if (L.slots == 0) {
     const int64_t longest = std::max<int64_t>(num_dst + 1, csr ? num_src + 1 : 0);
     hipLaunchKernelGGL(fmt_zero_kernel, dim3(static_cast<unsigned>(std::min<int64_t>(ceil_div(longest, kFmtBlock), 4096))),
@@ -584,6 +1028,34 @@ extern "C" int apt_block_formats(const int64_t* relabeled, int64_t num_dst, cons
   c.scanned = L.ctiles > kFusedCompactTiles || !tuning_block_fused_scan();
   c.num_edges_dev = num_edges_dev;
   const dim3 cgrid(static_cast<unsigned>(L.ctiles));
+  if (L.ranges > 0) {
+    RangeParams r;
+    r.shift2 = L.range_shift2;
+    r.ranges = L.ranges;
+    r.hist = reinterpret_cast<uint32_t*>(ws + L.hist_off);
+    r.total = reinterpret_cast<uint32_t*>(ws + L.bin_total_off);
+    r.start = reinterpret_cast<uint32_t*>(ws + L.start_off);
+    r.rec = reinterpret_cast<uint64_t*>(ws + L.rec_off);
+    r.num_src = num_src;
+    r.csr_indptr = csr_indptr;
+    r.csr_indices = csr_indices;
+    r.csr_eids = csr_eids;
+    hipLaunchKernelGGL(range_count_kernel, cgrid, dim3(kFmtBlock), sizeof(uint32_t) * L.ranges, st, c, r);
+    APT_LAUNCH_CHECK("range_count_kernel");
+    hipLaunchKernelGGL(range_scan_kernel, dim3(static_cast<unsigned>(ceil_div(L.ranges, kWave))),
+                       dim3(kWave * kRangeScanGroups), 0, st, c, r);
+    APT_LAUNCH_CHECK("range_scan_kernel");
+    const size_t place_lds = sizeof(uint32_t) * (L.ranges + kFmtWaves * ((L.ranges + 1) / 2));
+    hipLaunchKernelGGL(range_place_kernel, cgrid, dim3(kFmtBlock), place_lds, st, c, r);
+    APT_LAUNCH_CHECK("range_place_kernel");
+    const int keys = 1 << (L.ranges > kRangeCount0 + kRangeCount1 ? L.range_shift2
+                           : L.ranges > kRangeCount0              ? kRangeShift1
+                                                                  : kRangeShift0);
+    hipLaunchKernelGGL(range_sort_kernel, dim3(static_cast<unsigned>(L.ranges)), dim3(kRangeSortBlock),
+                       sizeof(uint32_t) * (keys + kRangeSortWaves * (keys / 2)), st, r);
+    APT_LAUNCH_CHECK("range_sort_kernel");
+    return APT_OK;
+  }
   hipLaunchKernelGGL(fmt_count_kernel, cgrid, dim3(kFmtBlock), 0, st, c);
   APT_LAUNCH_CHECK("fmt_count_kernel");
   // the edge total is also the last CSC offset

@@ -130,3 +130,23 @@ def test_gpu_pipeline_blocks_in_all_formats(orc, capi):
                     continue
                 assert f["csr_indptr"].numel() == num_src + 1
                 _same({k: (v.cpu().numpy() if hasattr(v, "cpu") else v) for k, v in f.items()}, ref)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("num_dst,fanout,num_src", [
+    (3000, 7, 32767), (3000, 7, 32768), (3000, 7, 32769),               # the first piece of source ranges ends at 2^15
+    (3000, 7, 2 ** 18 - 1), (3000, 7, 2 ** 18), (3000, 7, 2 ** 18 + 1),  # the second at 2^18
+    (2000, 3, 2 ** 18 + 2600 * 1024 - 1), (2000, 3, 2 ** 18 + 2600 * 1024), (2000, 3, 2 ** 18 + 2600 * 2048 - 1),
+    (2000, 3, 2 ** 18 + 2600 * 2048),                                    # one source more than the ranges hold: radix passes
+    (2 ** 21, 1, 50), (2 ** 21 + 1, 1, 50),                              # most destinations a record holds, and one more
+    (2048 * 4, 1, 33), (2048 * 4 + 1, 1, 33), (1, 2049, 64)])            # tiles, and a range of more than one chunk
+def test_gpu_csr_by_source_ranges(capi, num_dst, fanout, num_src):
+    import torch
+    rng = np.random.default_rng(num_dst + num_src)
+    r = _random_block(rng, num_dst, fanout, num_src)
+    # sources at both ends of the id range
+    r[: min(r.size, 50)] = np.minimum(np.arange(min(r.size, 50)) % 7, num_src - 1)
+    r[-min(r.size, 50):] = num_src - 1 - np.arange(min(r.size, 50)) % min(num_src, 5)
+    got = capi.block_formats(torch.from_numpy(r).cuda(), num_dst, fanout, num_src)
+    _same({k: (v.cpu().numpy() if hasattr(v, "cpu") else v) for k, v in got.items()},
+          _closed_form(r, num_dst, fanout, num_src))
