@@ -492,6 +492,8 @@ struct RangeParams {
   int64_t* csr_indptr;
   int64_t* csr_indices;
   int64_t* csr_eids;
+  uint32_t* t_indptr;         // transpose only (apt_block_transpose)
+  uint32_t* t_slots;
 };
 
 constexpr int kRangeCount0 = static_cast<int>(kRangeFrom1 >> kRangeShift0);
@@ -531,6 +533,9 @@ __device__ __forceinline__ uint64_t same_value(uint32_t v, int bits, bool valid)
   return peers;
 }
 
+// FORMATS: COO, CSC and CSR (an edge's id is its place in the COO).  Otherwise the transpose alone: the edges of a
+// source by slot, without a compaction.
+template <bool FORMATS>
 __global__ __launch_bounds__(kFmtBlock) void range_count_kernel(CompactParams p, RangeParams r) {
   extern __shared__ uint32_t s_range[];   // [ranges]
   __shared__ uint32_t s_wave[kFmtWaves];
@@ -552,9 +557,12 @@ __global__ __launch_bounds__(kFmtBlock) void range_count_kernel(CompactParams p,
     ++c;
     atomicAdd(&s_range[range_of(r, v[it])], 1u);
   }
-  uint32_t all;
-  block_exclusive(c, s_wave, all);   // (its barriers also complete the counts)
-  if (threadIdx.x == 0) p.tile_cnt[blockIdx.x] = all;
+  if (FORMATS) {
+    uint32_t all;
+    block_exclusive(c, s_wave, all);
+    if (threadIdx.x == 0) p.tile_cnt[blockIdx.x] = all;
+  }
+  __syncthreads();
   uint32_t* row = r.hist + static_cast<int64_t>(blockIdx.x) * r.ranges;
   for (int b = threadIdx.x; b < r.ranges; b += kFmtBlock) row[b] = s_range[b];
 }
@@ -605,6 +613,7 @@ __global__ __launch_bounds__(kWave * kRangeScanGroups) void range_scan_kernel(Co
 
 // The compaction's place pass (as fmt_place_kernel) with the partition: a wavefront owns consecutive slots, so that
 // walking the wavefronts, and the iterations inside one, is edge order.
+template <bool FORMATS>
 __global__ __launch_bounds__(kFmtBlock) void range_place_kernel(CompactParams p, RangeParams r) {
   extern __shared__ uint32_t s_range[];
   uint32_t* s_base = s_range;                                                // [ranges]
@@ -637,20 +646,23 @@ __global__ __launch_bounds__(kFmtBlock) void range_place_kernel(CompactParams p,
       atomicAdd(&cnt[b >> 1], (b & 1) ? 0x10000u : 1u);
     }
   }
-  // edges of the tiles before this one, and of all tiles
   const int64_t active = ceil_div_dev(slots, kCompactTile);
-  uint32_t before = 0, total = 0;
-  for (int64_t t = threadIdx.x; t < active; t += kFmtBlock) {
-    const uint32_t c = p.tile_cnt[t];
-    total += c;
-    if (t < blockIdx.x) before += c;
-  }
-  uint32_t first, all_total;
-  block_exclusive(before, s_wave, first);
-  block_exclusive(total, s_wave, all_total);
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    *p.num_edges_dev = all_total;
-    p.csc_indptr[p.num_dst] = all_total;
+  uint32_t first = 0;
+  if (FORMATS) {   // edges of the tiles before this one, and of all tiles
+    uint32_t before = 0, total = 0, all_total;
+    for (int64_t t = threadIdx.x; t < active; t += kFmtBlock) {
+      const uint32_t c = p.tile_cnt[t];
+      total += c;
+      if (t < blockIdx.x) before += c;
+    }
+    block_exclusive(before, s_wave, first);
+    block_exclusive(total, s_wave, all_total);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+      *p.num_edges_dev = all_total;
+      p.csc_indptr[p.num_dst] = all_total;
+    }
+  } else {
+    __syncthreads();   // the counts are complete
   }
   // where this tile's edges of a range start: the ranges before it, and the tiles before this one
   const bool live = blockIdx.x < active || blockIdx.x == 0;   // block-uniform (workgroup 0 also writes the starts)
@@ -704,7 +716,7 @@ __global__ __launch_bounds__(kFmtBlock) void range_place_kernel(CompactParams p,
     }
   }
   static_assert(kCompactIters * kFmtWaves <= kWave, "one wavefront scans the tile's per-wave counts");
-  if (wave == 0) {
+  if (FORMATS && wave == 0) {
     const uint32_t c = lane < kCompactIters * kFmtWaves ? s_edges[lane] : 0u;
     uint32_t incl = c;
 #pragma unroll
@@ -721,9 +733,9 @@ __global__ __launch_bounds__(kFmtBlock) void range_place_kernel(CompactParams p,
 #pragma unroll
   for (int it = 0; it < kCompactIters; ++it) {
     const int64_t s = base + it * kWave + lane;
-    const int64_t e = static_cast<int64_t>(s_edges[wave * kCompactIters + it]) + below[it];
-    const uint32_t d = static_cast<uint32_t>(s) / fan;
-    if (s < upper && static_cast<uint32_t>(s) - d * fan == 0) p.csc_indptr[d] = e;
+    const int64_t e = FORMATS ? static_cast<int64_t>(s_edges[wave * kCompactIters + it]) + below[it] : s;
+    const uint32_t d = FORMATS ? static_cast<uint32_t>(s) / fan : 0u;
+    if (FORMATS && s < upper && static_cast<uint32_t>(s) - d * fan == 0) p.csc_indptr[d] = e;
     const bool valid = v[it] >= 0;
     if (ballot(valid) == 0) continue;   // wave-uniform
     const uint32_t b = valid ? static_cast<uint32_t>(range_of(r, v[it])) : 0u;
@@ -735,8 +747,10 @@ __global__ __launch_bounds__(kFmtBlock) void range_place_kernel(CompactParams p,
     if (valid && rank + 1 == static_cast<uint32_t>(__popcll(peers))) pos[b] = static_cast<uint16_t>(at + 1);
     __builtin_amdgcn_wave_barrier();
     if (valid) {
-      p.coo_row[e] = v[it];
-      p.coo_col[e] = d;
+      if (FORMATS) {
+        p.coo_row[e] = v[it];
+        p.coo_col[e] = d;
+      }
       r.rec[s_base[b] + at] = (static_cast<uint64_t>(d) << (kRangeKeyBits + kRangeEdgeBits)) |
                               (static_cast<uint64_t>(range_key(r, static_cast<int>(b), v[it])) << kRangeEdgeBits) | static_cast<uint64_t>(e);
     }
@@ -745,6 +759,7 @@ __global__ __launch_bounds__(kFmtBlock) void range_place_kernel(CompactParams p,
 
 // One workgroup per range: stable counting sort of its records by source.  A range of a sampled block has about a
 // thousand; a range with more than a chunk of them (hubs) is walked chunk by chunk, after a counting walk.
+template <bool FORMATS>
 __global__ __launch_bounds__(kRangeSortBlock) void range_sort_kernel(RangeParams r) {
   extern __shared__ uint32_t s_range[];
   const int shift = range_shift(r, blockIdx.x);
@@ -776,9 +791,13 @@ __global__ __launch_bounds__(kRangeSortBlock) void range_sort_kernel(RangeParams
   };
   const uint32_t before = r.start[blockIdx.x], n = r.start[blockIdx.x + 1] - before;
   const int64_t src0 = range_first(r, blockIdx.x);
+  auto set_offset = [&](int k, uint32_t at) {
+    if (src0 + k > r.num_src) return;
+    if (FORMATS) r.csr_indptr[src0 + k] = at;
+    else r.t_indptr[src0 + k] = at;
+  };
   if (n == 0) {
-    for (int k = tid; k < keys; k += kRangeSortBlock)
-      if (src0 + k <= r.num_src) r.csr_indptr[src0 + k] = before;
+    for (int k = tid; k < keys; k += kRangeSortBlock) set_offset(k, before);
     return;
   }
   const uint64_t* rec = r.rec + before;
@@ -794,7 +813,7 @@ __global__ __launch_bounds__(kRangeSortBlock) void range_sort_kernel(RangeParams
     for (int k = k0; k < k1; ++k) {
       const uint32_t c = s_start[k];
       s_start[k] = run;
-      if (src0 + k <= r.num_src) r.csr_indptr[src0 + k] = static_cast<int64_t>(before) + run;
+      set_offset(k, before + run);
       run += c;
     }
   };
@@ -859,8 +878,13 @@ __global__ __launch_bounds__(kRangeSortBlock) void range_sort_kernel(RangeParams
       __builtin_amdgcn_wave_barrier();
       if (valid) {
         const int64_t to = static_cast<int64_t>(before) + s_start[k] + at;
-        r.csr_eids[to] = static_cast<int64_t>(x[q] & ((1ull << kRangeEdgeBits) - 1));
-        r.csr_indices[to] = static_cast<int64_t>(x[q] >> (kRangeKeyBits + kRangeEdgeBits));
+        const uint32_t e = static_cast<uint32_t>(x[q]) & ((1u << kRangeEdgeBits) - 1);
+        if (FORMATS) {
+          r.csr_eids[to] = e;
+          r.csr_indices[to] = static_cast<int64_t>(x[q] >> (kRangeKeyBits + kRangeEdgeBits));
+        } else {
+          r.t_slots[to] = e;
+        }
       }
     }
     if (c0 + kRangeSortChunk >= n) break;
@@ -976,7 +1000,67 @@ static bool fmt_sizes_ok(int64_t num_dst, int fanout, int64_t num_src) {
          (fanout == 0 || num_dst <= 0x7fffffffLL / fanout);
 }
 
+template <bool FORMATS>
+static int launch_ranges(const CompactParams& c, RangeParams& r, const FmtLayout& L, char* ws, int64_t num_src,
+                         hipStream_t st) {
+  r.shift2 = L.range_shift2;
+  r.ranges = L.ranges;
+  r.hist = reinterpret_cast<uint32_t*>(ws + L.hist_off);
+  r.total = reinterpret_cast<uint32_t*>(ws + L.bin_total_off);
+  r.start = reinterpret_cast<uint32_t*>(ws + L.start_off);
+  r.rec = reinterpret_cast<uint64_t*>(ws + L.rec_off);
+  r.num_src = num_src;
+  const dim3 tiles(static_cast<unsigned>(L.ctiles));
+  hipLaunchKernelGGL(range_count_kernel<FORMATS>, tiles, dim3(kFmtBlock), sizeof(uint32_t) * L.ranges, st, c, r);
+  APT_LAUNCH_CHECK("range_count_kernel");
+  hipLaunchKernelGGL(range_scan_kernel, dim3(static_cast<unsigned>(ceil_div(L.ranges, kWave))),
+                     dim3(kWave * kRangeScanGroups), 0, st, c, r);
+  APT_LAUNCH_CHECK("range_scan_kernel");
+  const size_t place_lds = sizeof(uint32_t) * (L.ranges + kFmtWaves * ((L.ranges + 1) / 2));
+  hipLaunchKernelGGL(range_place_kernel<FORMATS>, tiles, dim3(kFmtBlock), place_lds, st, c, r);
+  APT_LAUNCH_CHECK("range_place_kernel");
+  const int keys = 1 << (L.ranges > kRangeCount0 + kRangeCount1 ? L.range_shift2
+                         : L.ranges > kRangeCount0              ? kRangeShift1
+                                                                : kRangeShift0);
+  hipLaunchKernelGGL(range_sort_kernel<FORMATS>, dim3(static_cast<unsigned>(L.ranges)), dim3(kRangeSortBlock),
+                     sizeof(uint32_t) * (keys + kRangeSortWaves * (keys / 2)), st, r);
+  APT_LAUNCH_CHECK("range_sort_kernel");
+  return APT_OK;
+}
+
 }  // namespace apt
+
+extern "C" size_t apt_block_transpose_workspace_bytes(int64_t num_dst, int fanout, int64_t num_src) {
+  using namespace apt;
+  if (!fmt_sizes_ok(num_dst, fanout, num_src)) return 0;
+  const FmtLayout L = fmt_layout(num_dst, fanout, num_src, true);
+  return L.ranges > 0 ? L.total : 0;
+}
+
+extern "C" int apt_block_transpose(const int64_t* relabeled, int64_t num_dst, int fanout, int64_t num_src,
+                                   uint32_t* indptr, uint32_t* slots, void* workspace, size_t workspace_bytes,
+                                   void* stream) {
+  using namespace apt;
+  APT_REQUIRE(fmt_sizes_ok(num_dst, fanout, num_src), APT_ELIMIT,
+              "apt_block_transpose: sizes out of range (num_dst %lld, fanout %d, num_src %lld)",
+              static_cast<long long>(num_dst), fanout, static_cast<long long>(num_src));
+  const FmtLayout L = fmt_layout(num_dst, fanout, num_src, true);
+  APT_REQUIRE(L.ranges > 0, APT_ELIMIT, "apt_block_transpose: block too large (see apt_block_transpose_workspace_bytes)");
+  APT_REQUIRE(indptr != nullptr && (L.slots == 0 || (relabeled != nullptr && slots != nullptr)), APT_EINVAL,
+              "apt_block_transpose: an argument is NULL");
+  APT_REQUIRE(workspace != nullptr && workspace_bytes >= L.total, APT_EWORKSPACE,
+              "apt_block_transpose: workspace of %zu bytes, %zu needed", workspace_bytes, L.total);
+  CompactParams c{};
+  c.relabeled = relabeled;
+  c.num_dst = num_dst;
+  c.num_dst_dev = nullptr;
+  c.fanout = fanout;
+  c.tiles = L.ctiles;
+  RangeParams r{};
+  r.t_indptr = indptr;
+  r.t_slots = slots;
+  return launch_ranges<false>(c, r, L, static_cast<char*>(workspace), num_src, static_cast<hipStream_t>(stream));
+}
 
 extern "C" size_t apt_block_workspace_bytes(int64_t num_dst, int fanout, int64_t num_src, int want_csr) {
   using namespace apt;
@@ -1029,32 +1113,11 @@ extern "C" int apt_block_formats(const int64_t* relabeled, int64_t num_dst, cons
   c.num_edges_dev = num_edges_dev;
   const dim3 cgrid(static_cast<unsigned>(L.ctiles));
   if (L.ranges > 0) {
-    RangeParams r;
-    r.shift2 = L.range_shift2;
-    r.ranges = L.ranges;
-    r.hist = reinterpret_cast<uint32_t*>(ws + L.hist_off);
-    r.total = reinterpret_cast<uint32_t*>(ws + L.bin_total_off);
-    r.start = reinterpret_cast<uint32_t*>(ws + L.start_off);
-    r.rec = reinterpret_cast<uint64_t*>(ws + L.rec_off);
-    r.num_src = num_src;
+    RangeParams r{};
     r.csr_indptr = csr_indptr;
     r.csr_indices = csr_indices;
     r.csr_eids = csr_eids;
-    hipLaunchKernelGGL(range_count_kernel, cgrid, dim3(kFmtBlock), sizeof(uint32_t) * L.ranges, st, c, r);
-    APT_LAUNCH_CHECK("range_count_kernel");
-    hipLaunchKernelGGL(range_scan_kernel, dim3(static_cast<unsigned>(ceil_div(L.ranges, kWave))),
-                       dim3(kWave * kRangeScanGroups), 0, st, c, r);
-    APT_LAUNCH_CHECK("range_scan_kernel");
-    const size_t place_lds = sizeof(uint32_t) * (L.ranges + kFmtWaves * ((L.ranges + 1) / 2));
-    hipLaunchKernelGGL(range_place_kernel, cgrid, dim3(kFmtBlock), place_lds, st, c, r);
-    APT_LAUNCH_CHECK("range_place_kernel");
-    const int keys = 1 << (L.ranges > kRangeCount0 + kRangeCount1 ? L.range_shift2
-                           : L.ranges > kRangeCount0              ? kRangeShift1
-                                                                  : kRangeShift0);
-    hipLaunchKernelGGL(range_sort_kernel, dim3(static_cast<unsigned>(L.ranges)), dim3(kRangeSortBlock),
-                       sizeof(uint32_t) * (keys + kRangeSortWaves * (keys / 2)), st, r);
-    APT_LAUNCH_CHECK("range_sort_kernel");
-    return APT_OK;
+    return launch_ranges<true>(c, r, L, ws, num_src, st);
   }
   hipLaunchKernelGGL(fmt_count_kernel, cgrid, dim3(kFmtBlock), 0, st, c);
   APT_LAUNCH_CHECK("fmt_count_kernel");

@@ -1,0 +1,56 @@
+// Feature rows of the aggregation kernels: fp32 or bf16 (as bits) in memory, fp32 in registers.
+#pragma once
+
+#include "common.hpp"
+
+namespace apt {
+
+constexpr int kAggBlock = 256;
+constexpr int kAggWaves = kAggBlock / kWave;
+
+template <typename T> __device__ __forceinline__ float to_float(T v);
+template <> __device__ __forceinline__ float to_float<float>(float v) { return v; }
+template <> __device__ __forceinline__ float to_float<uint16_t>(uint16_t v) {  // bf16 bits
+  return __uint_as_float(static_cast<uint32_t>(v) << 16);
+}
+
+template <typename T> __device__ __forceinline__ T from_float(float v);
+template <> __device__ __forceinline__ float from_float<float>(float v) { return v; }
+template <> __device__ __forceinline__ uint16_t from_float<uint16_t>(float v) {
+  return __builtin_bit_cast(uint16_t, static_cast<__bf16>(v));   // round to nearest even
+}
+
+template <typename T, int VEC> struct Pack;
+template <> struct Pack<float, 4> { typedef float type __attribute__((ext_vector_type(4))); };
+template <> struct Pack<float, 1> { typedef float type; };
+template <> struct Pack<float, 8> { typedef float type __attribute__((ext_vector_type(8))); };
+template <> struct Pack<uint16_t, 4> { typedef uint16_t type __attribute__((ext_vector_type(4))); };
+template <> struct Pack<uint16_t, 1> { typedef uint16_t type; };
+template <> struct Pack<uint16_t, 8> { typedef uint16_t type __attribute__((ext_vector_type(8))); };
+
+template <typename T, int VEC>
+__device__ __forceinline__ void load_vec(const T* base, int64_t elem, float (&v)[VEC]) {
+  using P = typename Pack<T, VEC>::type;
+  const P raw = *reinterpret_cast<const P*>(base + elem);
+  if constexpr (VEC == 1) {
+    v[0] = to_float<T>(raw);
+  } else {
+#pragma unroll
+    for (int i = 0; i < VEC; ++i) v[i] = to_float<T>(raw[i]);
+  }
+}
+
+template <typename T, int VEC>
+__device__ __forceinline__ void store_vec(T* base, int64_t elem, const float (&v)[VEC]) {
+  using P = typename Pack<T, VEC>::type;
+  if constexpr (VEC == 1) {
+    base[elem] = from_float<T>(v[0]);
+  } else {
+    P raw;
+#pragma unroll
+    for (int i = 0; i < VEC; ++i) raw[i] = from_float<T>(v[i]);
+    *reinterpret_cast<P*>(base + elem) = raw;
+  }
+}
+
+}  // namespace apt

@@ -13,11 +13,10 @@
 // u_mul_e multiplies (the reference's kernel adds, src/cuda/spmm.cu:78, and
 // has no caller).
 #include "common.hpp"
+#include "feature_rows.hpp"
 
 namespace apt {
 
-constexpr int kAggBlock = 256;
-constexpr int kAggWaves = kAggBlock / kWave;
 constexpr int kEdgesPerWave = 64;
 constexpr int kMaxSegments = APT_MAX_BUCKETS + 1;
 
@@ -47,36 +46,11 @@ struct AggParams {
                               // span ranges, rows without edges) is zeroed by spmm_zero_rows_kernel: out need not be zero
 };
 
-template <typename T> __device__ __forceinline__ float to_float(T v);
-template <> __device__ __forceinline__ float to_float<float>(float v) { return v; }
-template <> __device__ __forceinline__ float to_float<uint16_t>(uint16_t v) {  // bf16 bits
-  return __uint_as_float(static_cast<uint32_t>(v) << 16);
-}
-
 // Segment of edge e: last k with coo_off[k] <= e (reference: cub::UpperBound - 1).
 __device__ __forceinline__ int segment_of(const int64_t* s_off, int num_seg, int64_t e) {
   int k = 0;
   while (k + 1 < num_seg && s_off[k + 1] <= e) ++k;
   return k;
-}
-
-template <typename T, int VEC> struct Pack;
-template <> struct Pack<float, 4> { typedef float type __attribute__((ext_vector_type(4))); };
-template <> struct Pack<float, 1> { typedef float type; };
-template <> struct Pack<uint16_t, 4> { typedef uint16_t type __attribute__((ext_vector_type(4))); };
-template <> struct Pack<uint16_t, 1> { typedef uint16_t type; };
-template <> struct Pack<uint16_t, 8> { typedef uint16_t type __attribute__((ext_vector_type(8))); };
-
-template <typename T, int VEC>
-__device__ __forceinline__ void load_vec(const T* base, int64_t elem, float (&v)[VEC]) {
-  using P = typename Pack<T, VEC>::type;
-  const P raw = *reinterpret_cast<const P*>(base + elem);
-  if constexpr (VEC == 1) {
-    v[0] = to_float<T>(raw);
-  } else {
-#pragma unroll
-    for (int i = 0; i < VEC; ++i) v[i] = to_float<T>(raw[i]);
-  }
 }
 
 // MODE 0: copy_u  acc += in[in_off + src]
@@ -286,12 +260,14 @@ __global__ __launch_bounds__(kAggBlock) void sddmm_kernel(AggParams p) {
 // destination i owns slots [i*fanout, (i+1)*fanout) of `nbr`, negative = no
 // edge.  A lane group owns a destination row, so there are no atomics, no
 // zero-fill and the sum order is fixed.  LPR lanes x VEC features cover `dim`.
-template <typename T, int VEC, int LPR>
+// OUT: fp32, or the input's type (a layer's result).  inv_degree, optional: 1 / number of valid slots per row.
+template <typename T, typename OUT, int VEC, int LPR>
 __global__ __launch_bounds__(kAggBlock) void spmm_ell_kernel(const int64_t* __restrict__ nbr,
                                                              int64_t num_dst, const int64_t* num_dst_dev,
                                                              int fanout, const T* __restrict__ x,
                                                              int64_t num_src, int64_t dim,
-                                                             float* __restrict__ out, int mean) {
+                                                             OUT* __restrict__ out, int mean,
+                                                             float* __restrict__ inv_degree) {
   constexpr int kGroups = kAggBlock / LPR;
   constexpr int kUnroll = 5;
   const int64_t n = actual_count(num_dst, num_dst_dev);
@@ -336,21 +312,25 @@ __global__ __launch_bounds__(kAggBlock) void spmm_ell_kernel(const int64_t* __re
       const float scale = (mean && cnt > 0) ? 1.0f / static_cast<float>(cnt) : 1.0f;
       if (live) {
 #pragma unroll
-        for (int k = 0; k < VEC; ++k) out[i * dim + d + k] = acc[k] * scale;
+        for (int k = 0; k < VEC; ++k) acc[k] *= scale;
+        store_vec<OUT, VEC>(out, i * dim + d, acc);
       }
+      if (inv_degree != nullptr && d0 == 0 && l == 0) inv_degree[i] = 1.0f / static_cast<float>(cnt > 0 ? cnt : 1);
     }
   }
 }
 
-template <typename T, int VEC>
+template <typename T, typename OUT, int VEC>
 static void launch_ell(const int64_t* nbr, int64_t num_dst, const int64_t* num_dst_dev, int fanout,
-                       const void* x, int64_t num_src, int64_t dim, float* out, int mean, hipStream_t st) {
+                       const void* x, int64_t num_src, int64_t dim, void* out, int mean, float* inv_degree,
+                       hipStream_t st) {
   const int64_t per_row = ceil_div(dim, VEC);
   const T* xt = static_cast<const T*>(x);
 #define APT_ELL(LPR)                                                                                 \
-  hipLaunchKernelGGL((spmm_ell_kernel<T, VEC, LPR>),                                                  \
+  hipLaunchKernelGGL((spmm_ell_kernel<T, OUT, VEC, LPR>),                                             \
                      dim3(static_cast<unsigned>(std::min<int64_t>(ceil_div(num_dst, kAggBlock / LPR), 1 << 20))), \
-                     dim3(kAggBlock), 0, st, nbr, num_dst, num_dst_dev, fanout, xt, num_src, dim, out, mean)
+                     dim3(kAggBlock), 0, st, nbr, num_dst, num_dst_dev, fanout, xt, num_src, dim, static_cast<OUT*>(out), mean, \
+                     inv_degree)
   if (per_row <= 8) APT_ELL(8);
   else if (per_row <= 16) APT_ELL(16);
   else if (per_row <= 32) APT_ELL(32);
@@ -957,31 +937,52 @@ extern "C" int apt_sddmm(int op, const int64_t* coo_row, const int64_t* coo_col,
   return APT_OK;
 }
 
-extern "C" int apt_spmm_block(const int64_t* neighbors, int64_t num_dst, const int64_t* num_dst_dev,
-                              int fanout, const void* input, int64_t num_src, int64_t dim, int elem_size,
-                              int mean, float* out, void* stream) {
-  using namespace apt;
+namespace apt {
+static int block_sum(const char* who, const int64_t* neighbors, int64_t num_dst, const int64_t* num_dst_dev, int fanout,
+                     const void* input, int64_t num_src, int64_t dim, int elem_size, int mean, void* out, bool out_like_input,
+                     float* inv_degree, void* stream) {
   APT_REQUIRE(num_dst >= 0 && fanout > 0 && dim > 0 && num_src >= 0, APT_EINVAL,
-              "apt_spmm_block: bad shape (num_dst %lld, fanout %d, dim %lld)", (long long)num_dst, fanout,
-              (long long)dim);
-  APT_REQUIRE(elem_size == 2 || elem_size == 4, APT_EINVAL, "apt_spmm_block: elem_size %d (4 = fp32, 2 = bf16)",
-              elem_size);
+              "%s: bad shape (num_dst %lld, fanout %d, dim %lld)", who, (long long)num_dst, fanout, (long long)dim);
+  APT_REQUIRE(elem_size == 2 || elem_size == 4, APT_EINVAL, "%s: elem_size %d (4 = fp32, 2 = bf16)", who, elem_size);
   if (num_dst == 0) return APT_OK;
   APT_REQUIRE(neighbors != nullptr && out != nullptr && (input != nullptr || num_src == 0), APT_EINVAL,
-              "apt_spmm_block: a tensor is NULL");
+              "%s: a tensor is NULL", who);
   hipStream_t st = static_cast<hipStream_t>(stream);
   const bool vec4 = dim % 4 == 0 && (reinterpret_cast<uintptr_t>(input) & 15) == 0 &&
                     (reinterpret_cast<uintptr_t>(out) & 15) == 0;
+#define APT_BLOCK_SUM(T, OUT, V) \
+  launch_ell<T, OUT, V>(neighbors, num_dst, num_dst_dev, fanout, input, num_src, dim, out, mean, inv_degree, st)
+#define APT_BLOCK_SUM_BF16(OUT)                                   \
+  if (vec4 && dim % 8 == 0) APT_BLOCK_SUM(uint16_t, OUT, 8);      \
+  else if (vec4) APT_BLOCK_SUM(uint16_t, OUT, 4);                 \
+  else APT_BLOCK_SUM(uint16_t, OUT, 1)
   if (elem_size == 4) {
-    if (vec4) launch_ell<float, 4>(neighbors, num_dst, num_dst_dev, fanout, input, num_src, dim, out, mean, st);
-    else launch_ell<float, 1>(neighbors, num_dst, num_dst_dev, fanout, input, num_src, dim, out, mean, st);
+    if (vec4) APT_BLOCK_SUM(float, float, 4);
+    else APT_BLOCK_SUM(float, float, 1);
+  } else if (out_like_input) {
+    APT_BLOCK_SUM_BF16(uint16_t);
   } else {
-    if (vec4 && dim % 8 == 0) launch_ell<uint16_t, 8>(neighbors, num_dst, num_dst_dev, fanout, input, num_src, dim, out, mean, st);
-    else if (vec4) launch_ell<uint16_t, 4>(neighbors, num_dst, num_dst_dev, fanout, input, num_src, dim, out, mean, st);
-    else launch_ell<uint16_t, 1>(neighbors, num_dst, num_dst_dev, fanout, input, num_src, dim, out, mean, st);
+    APT_BLOCK_SUM_BF16(float);
   }
+#undef APT_BLOCK_SUM_BF16
+#undef APT_BLOCK_SUM
   APT_LAUNCH_CHECK("spmm_ell_kernel");
   return APT_OK;
+}
+}  // namespace apt
+
+extern "C" int apt_spmm_block(const int64_t* neighbors, int64_t num_dst, const int64_t* num_dst_dev,
+                              int fanout, const void* input, int64_t num_src, int64_t dim, int elem_size,
+                              int mean, float* out, void* stream) {
+  return apt::block_sum("apt_spmm_block", neighbors, num_dst, num_dst_dev, fanout, input, num_src, dim, elem_size, mean,
+                        out, false, nullptr, stream);
+}
+
+extern "C" int apt_block_aggregate(const int64_t* neighbors, int64_t num_dst, int fanout, const void* input,
+                                   int64_t num_src, int64_t dim, int elem_size, int mean, void* out, float* inv_degree,
+                                   void* stream) {
+  return apt::block_sum("apt_block_aggregate", neighbors, num_dst, nullptr, fanout, input, num_src, dim, elem_size, mean,
+                        out, true, inv_degree, stream);
 }
 
 extern "C" int apt_gat_scores(const void* x, int64_t num_rows, int heads, int64_t dim, int elem_size,

@@ -982,6 +982,114 @@ Tensor BlockLinear(const Tensor& x, const Tensor& w, const std::optional<Tensor>
   return BlockLinearFn::apply(x, w, b, kn);
 }
 
+// ---------------------------------------------------------------- aggregation over a block, with its gradient
+namespace {
+
+void check_block(const char* who, const Tensor& relabeled, int64_t num_dst, int64_t fanout) {
+  TORCH_CHECK_TYPE(relabeled.is_cuda() && relabeled.scalar_type() == torch::kInt64 && relabeled.is_contiguous(), "npc: ", who,
+                   ": the block's slots must be a contiguous int64 tensor on the GPU");
+  TORCH_CHECK(num_dst >= 0 && fanout > 0 && relabeled.numel() >= num_dst * fanout, "npc: ", who,
+              ": the block has fewer than num_dst * fanout slots");
+}
+
+// The edges of every source of a block: slots (4-byte, apt_block_transpose), or, for a block too large for that, the
+// destinations of its CSR (8-byte).  Enqueued on the current stream; nothing is read back.
+struct SourceOrder {
+  Tensor indptr, index;
+  int bytes = 4;
+};
+SourceOrder source_order(const Tensor& relabeled, int64_t num_dst, int64_t fanout, int64_t num_src) {
+  SourceOrder o;
+  const int64_t slots = std::max<int64_t>(num_dst * fanout, 1);
+  const int f = static_cast<int>(fanout);
+  const auto u8 = relabeled.options().dtype(torch::kUInt8), i32 = relabeled.options().dtype(torch::kInt32);
+  if (const size_t need = apt_block_transpose_workspace_bytes(num_dst, f, num_src)) {
+    o.indptr = torch::empty({num_src + 1}, i32);
+    o.index = torch::empty({slots}, i32);
+    auto ws = torch::empty({static_cast<int64_t>(need)}, u8);
+    check(apt_block_transpose(i64(relabeled), num_dst, f, num_src, reinterpret_cast<uint32_t*>(o.indptr.data_ptr<int>()),
+                              reinterpret_cast<uint32_t*>(o.index.data_ptr<int>()), ws.data_ptr(), need, stream()));
+    return o;
+  }
+  const size_t need = apt_block_workspace_bytes(num_dst, f, num_src, 1);
+  TORCH_CHECK(need > 0, "npc: block of ", num_dst, " x ", fanout, " slots and ", num_src, " sources is out of range");
+  auto ws = torch::empty({static_cast<int64_t>(need)}, u8);
+  auto coo = torch::empty({2, slots}, relabeled.options()), csc = torch::empty({num_dst + 1}, relabeled.options());
+  auto edges = torch::empty({1}, relabeled.options()), eids = torch::empty({slots}, relabeled.options());
+  o.indptr = torch::empty({num_src + 1}, relabeled.options());
+  o.index = torch::empty({slots}, relabeled.options());
+  o.bytes = 8;
+  check(apt_block_formats(i64(relabeled), num_dst, nullptr, f, num_src, coo.data_ptr<int64_t>(),
+                          coo.data_ptr<int64_t>() + slots, csc.data_ptr<int64_t>(), edges.data_ptr<int64_t>(),
+                          o.indptr.data_ptr<int64_t>(), o.index.data_ptr<int64_t>(), eids.data_ptr<int64_t>(),
+                          ws.data_ptr(), need, stream()));
+  return o;
+}
+
+// The gradient of the block sum / mean towards its input, from the block's CSR if it has one.
+Tensor aggregate_backward(const Tensor& dz_in, const Tensor& relabeled, int64_t num_dst, int64_t fanout, int64_t num_src,
+                          const Tensor& dst_scale, const Tensor& csr_indptr, const Tensor& csr_indices) {
+  auto dz = dz_in.contiguous();
+  auto dx = torch::empty({num_src, dz.size(1)}, dz.options());
+  SourceOrder o;
+  if (csr_indptr.defined() && csr_indptr.numel() == num_src + 1) {
+    o.indptr = csr_indptr;
+    o.index = csr_indices;
+    o.bytes = 8;
+  } else {
+    o = source_order(relabeled, num_dst, fanout, num_src);
+  }
+  check(apt_block_aggregate_backward(o.indptr.data_ptr(), o.index.data_ptr(), o.bytes, static_cast<int>(fanout), num_src,
+                                     dst_scale.defined() ? dst_scale.data_ptr<float>() : nullptr, dz.data_ptr(), num_dst,
+                                     dz.size(1), static_cast<int>(dz.element_size()), dx.data_ptr(), stream()));
+  return dx;
+}
+
+// -> (sum or mean, 1 / degree per destination when `mean`)
+std::tuple<Tensor, Tensor> aggregate_forward(const Tensor& relabeled, int64_t num_dst, int64_t fanout, const Tensor& x,
+                                             bool mean) {
+  auto out = torch::empty({num_dst, x.size(1)}, x.options());
+  Tensor inv;
+  if (mean) inv = torch::empty({num_dst}, x.options().dtype(torch::kFloat32));
+  check(apt_block_aggregate(i64(relabeled), num_dst, static_cast<int>(fanout), x.data_ptr(), x.size(0), x.size(1),
+                            static_cast<int>(x.element_size()), mean, out.data_ptr(),
+                            mean ? inv.data_ptr<float>() : nullptr, stream()));
+  return {out, inv};
+}
+
+struct BlockAggregateFn : public torch::autograd::Function<BlockAggregateFn> {
+  static Tensor forward(torch::autograd::AutogradContext* ctx, const Tensor& x, const Tensor& relabeled, int64_t num_dst,
+                        int64_t fanout, bool mean, const std::optional<Tensor>& csr_indptr,
+                        const std::optional<Tensor>& csr_indices) {
+    auto r = aggregate_forward(relabeled, num_dst, fanout, x, mean);
+    ctx->save_for_backward({relabeled, std::get<1>(r), csr_indptr.value_or(Tensor()), csr_indices.value_or(Tensor())});
+    ctx->saved_data["num_dst"] = num_dst;
+    ctx->saved_data["fanout"] = fanout;
+    ctx->saved_data["num_src"] = x.size(0);
+    return std::get<0>(r);
+  }
+  static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx,
+                                                 torch::autograd::variable_list grads) {
+    const auto saved = ctx->get_saved_variables();
+    Tensor dx;
+    if (ctx->needs_input_grad(0))
+      dx = aggregate_backward(grads[0], saved[0], ctx->saved_data["num_dst"].toInt(), ctx->saved_data["fanout"].toInt(),
+                              ctx->saved_data["num_src"].toInt(), saved[1], saved[2], saved[3]);
+    return {dx, Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
+  }
+};
+
+}  // namespace
+
+Tensor BlockAggregate(const Tensor& relabeled, int64_t num_dst, int64_t fanout, const Tensor& x, bool mean,
+                      const std::optional<Tensor>& csr_indptr, const std::optional<Tensor>& csr_indices) {
+  check_block("block_aggregate", relabeled, num_dst, fanout);
+  TORCH_CHECK_TYPE(x.is_cuda() && x.dim() == 2 &&
+                       (x.scalar_type() == torch::kFloat32 || x.scalar_type() == torch::kBFloat16),
+                   "npc: block_aggregate: input must be a 2-D fp32 or bf16 GPU tensor");
+  return BlockAggregateFn::apply(x.contiguous(), relabeled, num_dst, fanout, mean, csr_indptr, csr_indices);
+}
+
 // ---------------------------------------------------------------- peers only
 #define NPC_NEEDS_PEERS(name)                                                              \
   TORCH_CHECK(false, "npc." name " talks to other GPUs over NCCL in the reference; this " \
@@ -1037,6 +1145,7 @@ TORCH_LIBRARY(npc, m) {
       .def("sample_blocks", &SampleBlocks)
       .def("block_formats", &BlockFormats)
       .def("block_linear", &BlockLinear)
+      .def("block_aggregate", &BlockAggregate)
       .def("cluster_and_permute", &ClusterAndPermuteLocal)
       .def("register_graph_partition", &RegisterGraphPartition)
       .def("set_topology", &SetTopology)

@@ -6,7 +6,7 @@ its own layers (python/npc/model/sageconv.py:118-188 MPSAGEConv, Aggregate
 from the same operator with the edges reversed.  The layers here keep that
 arithmetic on a Block of this package: the forward sum reads the sampler's
 fixed-stride layout directly (no atomics), the backward sum runs over the
-block's CSR order (edges grouped by source), so both directions are
+block's edges grouped by source (no atomics either), so both directions are
 reproducible.
 """
 import torch
@@ -15,28 +15,16 @@ from torch import nn
 from . import capi
 
 
-class BlockAggregate(torch.autograd.Function):
-    """out[d] = sum (or mean) over the block's edges (s -> d) of X[s]."""
+class BlockAggregate:
+    """out[d] = sum (or mean) over the block's edges (s -> d) of X[s], in X's dtype (sums are fp32 inside the kernels),
+    with its gradient: npc.block_aggregate.  The backward pass takes the block's CSR if it has been emitted and
+    otherwise orders the edges by source itself, without reading a size back."""
 
     @staticmethod
-    def forward(ctx, block, X, mean):
-        ctx.block, ctx.mean = block, mean
-        out = capi.spmm_block(block.relabeled, block.num_dst, block.fanout, X.contiguous(), mean=mean)
-        return out if X.dtype == torch.float32 else out.to(X.dtype)      # sums are fp32 inside the kernel
-
-    @staticmethod
-    def backward(ctx, dZ):
-        block = ctx.block
-        dZ = dZ.contiguous()
-        if ctx.mean:
-            indptr = block.csc()[0]
-            dZ = dZ / (indptr[1:] - indptr[:-1]).clamp(min=1).to(dZ.dtype)[:, None]
-        indptr, dst, eids = block.csr()                # edges grouped by source, by increasing edge id
-        src = block.row[eids]
-        # every source row is stored whole by the wavefront that holds its edges (or zeroed and added when it
-        # spans two): no zero-fill, no atomics for the bulk, sums in edge order
-        dX = capi.spmm_heads(dst, src, dZ, None, block.num_src, grouped=True, out_indptr=indptr)
-        return None, dX.to(dZ.dtype), None
+    def apply(block, X, mean):
+        f = block.formats or {}
+        return torch.ops.npc.block_aggregate(block.relabeled, block.num_dst, block.fanout, X, bool(mean),
+                                             f.get("csr_indptr"), f.get("csr_indices"))
 
 
 def _trains_natively(x, weight):

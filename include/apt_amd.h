@@ -778,6 +778,38 @@ int apt_spmm_heads(const int64_t* coo_row, const int64_t* coo_col, int64_t num_e
                    float* out, int64_t num_out_rows, const float* head_weights2, float* out2,
                    const int64_t* out_indptr, void* stream);
 
+/* The transpose of a sampled block by itself, for a backward pass: for every
+ * source the slots of relabeled[num_dst * fanout] that name it, in increasing order
+ * (the destination of slot s is s / fanout): indptr uint32[num_src + 1], slots
+ * uint32[num_dst * fanout] of which indptr[num_src] are written.  What
+ * apt_block_formats' CSR is, without the compaction, in half the bytes.
+ * workspace: apt_block_transpose_workspace_bytes; 0 = a block this large is not
+ * supported (take apt_block_formats). */
+size_t apt_block_transpose_workspace_bytes(int64_t num_dst, int fanout, int64_t num_src);
+int apt_block_transpose(const int64_t* relabeled, int64_t num_dst, int fanout, int64_t num_src,
+                        uint32_t* indptr, uint32_t* slots, void* workspace, size_t workspace_bytes,
+                        void* stream);
+
+/* Sum / mean over a block as a layer uses it, and its gradient (python/npc/model/
+ * sageconv.py:100-114: the reference's Aggregate, whose backward is the operator with
+ * the edges reversed).
+ *   apt_block_aggregate           apt_spmm_block with the result in the input's type;
+ *                                 inv_degree, optional: float[num_dst], 1 / number of
+ *                                 edges of the destination (1 where it has none)
+ *   apt_block_aggregate_backward  dx[s, :] = sum over the edges s -> d of
+ *                                 dst_scale[d] * dz[d, :] (dst_scale NULL: 1); every
+ *                                 row of dx [num_src, dim] is written, in the type of
+ *                                 dz (fp32 sums, fixed order).  The edges of a source:
+ *                                 index_bytes 8 = csr_indptr / csr_indices of
+ *                                 apt_block_formats (fanout ignored), 4 = indptr / slots
+ *                                 of apt_block_transpose. */
+int apt_block_aggregate(const int64_t* neighbors, int64_t num_dst, int fanout, const void* input,
+                        int64_t num_src, int64_t dim, int elem_size, int mean, void* out,
+                        float* inv_degree, void* stream);
+int apt_block_aggregate_backward(const void* indptr, const void* index, int index_bytes, int fanout,
+                                 int64_t num_src, const float* dst_scale, const void* dz,
+                                 int64_t num_dst, int64_t dim, int elem_size, void* dx, void* stream);
+
 /* Gradients of a dense layer y = x w^T + b over a block's rows (the fc_self /
  * fc_neigh / fc of python/npc/model/sageconv.py:118-188 and gatconv.py:207-236,
  * whose gradients the reference gets from cuBLAS through torch):
