@@ -137,6 +137,7 @@ __global__ __launch_bounds__(kAggBlock) void source_sum_kernel(SourceSumParams p
 #pragma unroll
         for (int k = 0; k < VEC; ++k) {
           float sum = 0.f;
+#pragma unroll 1
           for (int g = 0; g < kGroups; ++g) sum += s_sum[g][l * VEC + k];
           acc[k] = sum;
         }

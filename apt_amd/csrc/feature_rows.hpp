@@ -20,6 +20,9 @@ template <> __device__ __forceinline__ uint16_t from_float<uint16_t>(float v) {
   return __builtin_bit_cast(uint16_t, static_cast<__bf16>(v));   // round to nearest even
 }
 
+// A value as it would be after being stored as a T and read back.
+template <typename T> __device__ __forceinline__ float as_stored(float v) { return to_float<T>(from_float<T>(v)); }
+
 template <typename T, int VEC> struct Pack;
 template <> struct Pack<float, 4> { typedef float type __attribute__((ext_vector_type(4))); };
 template <> struct Pack<float, 1> { typedef float type; };

@@ -1,0 +1,600 @@
+// A GAT layer over a block between its dense product and its activation, forward and backward (python/npc/model/
+// gatconv.py:116-126,207-236; the arithmetic there is DGL's and torch's, an elementwise kernel or a reduction per
+// step over [num_src, heads, dim] temporaries):
+//   el = (ft * attn_l).sum(-1), er = (ft[:num_dst] * attn_r).sum(-1)      gat_pair_scores_*: one read of ft
+//   a = edge softmax of LeakyReLU(el[src] + er[dst]), out = sum a * ft[src] + bias      the block kernels of spmm.hip
+// and, from d_out,
+//   dz, d_er                                       the edge kernels of spmm.hip, in slot order
+//   d_ft = sum a * d_out[dst] + d_el * attn_l + d_er * attn_r, d_el = sum dz            gat_source_kernel
+//   d_attn_l = sum_s d_el * ft, d_attn_r = sum_d d_er * ft, d_bias = sum_d d_out        gat_param_grad_kernel
+// Everything is a stream over ft or d_out with a few registers of reduction per lane; nothing of the size of ft
+// but d_ft itself is written.
+// bf16: a model trained in bf16 gets what the separate operations give.  Their results are bf16 where both operands
+// are, so a value that was a bf16 tensor between two of them is rounded here too (as_stored, Terms); a gradient of the
+// attention vectors is what is left of large terms that cancel, and moves by several per cent with that rounding.
+#include <algorithm>
+
+#include "common.hpp"
+#include "feature_rows.hpp"
+#include "partial_sums.hpp"
+
+namespace apt {
+
+int gat_block(const char* who, const int64_t* neighbors, int64_t num_dst, const int64_t* num_dst_dev, int fanout,
+              const void* ft, int64_t num_src, int heads, int64_t dim, int elem_size, const float* el, const float* er,
+              float slope, void* out, bool like_input, float* attn_out, const void* bias, hipStream_t st);
+int gat_edge_grad(const char* who, const int64_t* neighbors, int64_t num_dst, int fanout, const void* ft, int64_t num_src,
+                  int heads, int64_t dim, int elem_size, const float* el, const float* er, float slope, const float* attn,
+                  const void* d_out, bool like_input, const int64_t* csc_indptr, float* a_edge, float* dz_edge, float* d_er,
+                  hipStream_t st);
+
+// A layer's parameters may be of another type than its rows (fp32 weights under bf16 features).
+struct ParamVec {
+  const void* p;
+  int elem_size;
+  __device__ __forceinline__ float at(int64_t i) const {
+    return elem_size == 4 ? static_cast<const float*>(p)[i] : to_float<uint16_t>(static_cast<const uint16_t*>(p)[i]);
+  }
+};
+
+// Type of what an operation of a row (T) and an attention parameter gives: bf16 only if both are.
+template <typename T>
+struct Terms {
+  bool bf16;
+  __device__ __forceinline__ explicit Terms(const ParamVec& attn) : bf16(sizeof(T) == 2 && attn.elem_size == 2) {}
+  __device__ __forceinline__ float operator()(float v) const { return bf16 ? as_stored<uint16_t>(v) : v; }
+};
+
+// el and er of a row by LPH lanes per head (VEC features each), heads * LPH lanes per row padded to LPR: the lanes of
+// a head reduce with xor shuffles.
+template <typename T, int VEC, int LPH, int LPR>
+__global__ __launch_bounds__(kAggBlock) void gat_pair_scores_kernel(const T* __restrict__ x, int64_t num_rows,
+                                                                    int64_t num_dst, int heads, ParamVec attn_l,
+                                                                    ParamVec attn_r, float* __restrict__ el,
+                                                                    float* __restrict__ er) {
+  constexpr int kGroups = kAggBlock / LPR;
+  constexpr int kRows = 4;
+  const int grp = threadIdx.x / LPR, l = threadIdx.x % LPR;
+  const bool live = l < heads * LPH;
+  const int h = live ? l / LPH : 0;
+  const int64_t row_len = static_cast<int64_t>(heads) * VEC * LPH;
+  float al[VEC], ar[VEC];
+#pragma unroll
+  for (int k = 0; k < VEC; ++k) {
+    al[k] = live ? attn_l.at(l * VEC + k) : 0.f;
+    ar[k] = live ? attn_r.at(l * VEC + k) : 0.f;
+  }
+  const Terms<T> term(attn_l);
+  const int64_t step = static_cast<int64_t>(gridDim.x) * kGroups;
+  for (int64_t r0 = static_cast<int64_t>(blockIdx.x) * kGroups + grp; r0 < num_rows; r0 += kRows * step) {
+    float v[kRows][VEC];
+#pragma unroll
+    for (int q = 0; q < kRows; ++q) {
+#pragma unroll
+      for (int k = 0; k < VEC; ++k) v[q][k] = 0.f;
+      if (live && r0 + q * step < num_rows) load_vec<T, VEC>(x, (r0 + q * step) * row_len + l * VEC, v[q]);
+    }
+#pragma unroll
+    for (int q = 0; q < kRows; ++q) {
+      const int64_t r = r0 + q * step;
+      if (r >= num_rows) break;   // group-uniform
+      float sl = 0.f, sr = 0.f;
+#pragma unroll
+      for (int k = 0; k < VEC; ++k) {
+        sl += term(v[q][k] * al[k]);
+        sr += term(v[q][k] * ar[k]);
+      }
+#pragma unroll
+      for (int off = LPH / 2; off > 0; off >>= 1) {
+        sl += __shfl_xor(sl, off, kWave);
+        sr += __shfl_xor(sr, off, kWave);
+      }
+      if (live && l % LPH == 0) {
+        el[r * heads + h] = term(sl);
+        if (r < num_dst) er[r * heads + h] = term(sr);
+      }
+    }
+  }
+}
+
+// Any heads and dim: a wavefront per (row, head).
+template <typename T>
+__global__ __launch_bounds__(kAggBlock) void gat_pair_scores_any_kernel(const T* __restrict__ x, int64_t num_rows,
+                                                                        int64_t num_dst, int heads, int64_t dim,
+                                                                        ParamVec attn_l, ParamVec attn_r,
+                                                                        float* __restrict__ el, float* __restrict__ er) {
+  const int lane = threadIdx.x % kWave;
+  const Terms<T> term(attn_l);
+  const int64_t items = num_rows * heads;
+  for (int64_t it = static_cast<int64_t>(blockIdx.x) * kAggWaves + threadIdx.x / kWave; it < items;
+       it += static_cast<int64_t>(gridDim.x) * kAggWaves) {
+    const int h = static_cast<int>(it % heads);
+    float sl = 0.f, sr = 0.f;
+    for (int64_t d = lane; d < dim; d += kWave) {
+      const float v = to_float<T>(x[it * dim + d]);
+      sl += term(v * attn_l.at(h * dim + d));
+      sr += term(v * attn_r.at(h * dim + d));
+    }
+#pragma unroll
+    for (int off = kWave / 2; off > 0; off >>= 1) {
+      sl += __shfl_down(sl, off, kWave);
+      sr += __shfl_down(sr, off, kWave);
+    }
+    if (lane == 0) {
+      el[it] = term(sl);
+      if (it < num_dst * heads) er[it] = term(sr);
+    }
+  }
+}
+
+template <typename T, int VEC, int LPH>
+static void launch_pair_scores_r(const void* x, int64_t n, int64_t num_dst, int heads, ParamVec al, ParamVec ar, float* el,
+                                 float* er, hipStream_t st) {
+#define APT_PAIR(LPR)                                                                                              \
+  hipLaunchKernelGGL((gat_pair_scores_kernel<T, VEC, LPH, LPR>),                                                    \
+                     dim3(static_cast<unsigned>(std::min<int64_t>(ceil_div(n, kAggBlock / LPR), 4096))),           \
+                     dim3(kAggBlock), 0, st, static_cast<const T*>(x), n, num_dst, heads, al, ar, el, er)
+  const int lanes = heads * LPH;
+  if constexpr (LPH <= 8) {
+    if (lanes <= 8) {
+      APT_PAIR(8);
+      return;
+    }
+  }
+  if constexpr (LPH <= 16) {
+    if (lanes <= 16) {
+      APT_PAIR(16);
+      return;
+    }
+  }
+  if constexpr (LPH <= 32) {
+    if (lanes <= 32) {
+      APT_PAIR(32);
+      return;
+    }
+  }
+  APT_PAIR(64);
+#undef APT_PAIR
+}
+
+template <typename T, int VEC>
+static bool launch_pair_scores(const void* x, int64_t n, int64_t num_dst, int heads, int64_t dim, ParamVec al, ParamVec ar,
+                               float* el, float* er, hipStream_t st) {
+  const int64_t lph = dim / VEC;
+  if (dim % VEC != 0 || (lph & (lph - 1)) != 0 || heads * lph > kWave || (reinterpret_cast<uintptr_t>(x) & 15) != 0)
+    return false;
+  switch (lph) {
+    case 1: launch_pair_scores_r<T, VEC, 1>(x, n, num_dst, heads, al, ar, el, er, st); return true;
+    case 2: launch_pair_scores_r<T, VEC, 2>(x, n, num_dst, heads, al, ar, el, er, st); return true;
+    case 4: launch_pair_scores_r<T, VEC, 4>(x, n, num_dst, heads, al, ar, el, er, st); return true;
+    case 8: launch_pair_scores_r<T, VEC, 8>(x, n, num_dst, heads, al, ar, el, er, st); return true;
+    case 16: launch_pair_scores_r<T, VEC, 16>(x, n, num_dst, heads, al, ar, el, er, st); return true;
+    case 32: launch_pair_scores_r<T, VEC, 32>(x, n, num_dst, heads, al, ar, el, er, st); return true;
+    default: launch_pair_scores_r<T, VEC, 64>(x, n, num_dst, heads, al, ar, el, er, st); return true;
+  }
+}
+
+// ------------------------------------------------------------------ backward, source half
+// As source_sum_kernel (block_grad.hip): a lane group per source row, hubs shared by the workgroup.
+constexpr int kGatHubEdges = 32;
+constexpr int kGatHubList = 1024;
+constexpr int kGatSourceBlocks = 2048;
+
+struct GatSourceParams {
+  const void* indptr;       // offsets of the sources in `index`
+  const void* index;        // per edge: its slot (uint32_t), or its destination (int64_t) with its edge id in `eids`
+  const int64_t* eids;
+  uint32_t fanout;
+  const float* attn;        // attention weight and logit gradient, [slot or edge id, heads]
+  const float* dz;
+  const void* d_out;        // [num_dst, heads * dim]
+  const float* d_er;        // [num_dst, heads]
+  ParamVec attn_l, attn_r;  // [heads, dim]
+  int64_t num_dst, num_src;
+  int heads;
+  int64_t dim;              // per head
+  void* d_ft;               // [num_src, heads * dim]
+  float* d_el;              // [num_src, heads]
+};
+
+// VEC consecutive features of a row belong to at most two heads (dim >= VEC): h0, and h1 from element `cut` on.
+template <typename T, int VEC, int LPR, typename I>
+__global__ __launch_bounds__(kAggBlock) void gat_source_kernel(GatSourceParams p) {
+  constexpr int kGroups = kAggBlock / LPR;
+  constexpr int kUnroll = 4;
+  __shared__ int s_hub[kGatHubList];
+  __shared__ int s_hubs;
+  __shared__ float s_sum[kGroups][LPR * (VEC + 2)];
+  const int grp = threadIdx.x / LPR, l = threadIdx.x % LPR;
+  const I* indptr = static_cast<const I*>(p.indptr);
+  const I* index = static_cast<const I*>(p.index);
+  const T* d_out = static_cast<const T*>(p.d_out);
+  T* d_ft = static_cast<T*>(p.d_ft);
+  const int64_t row_len = p.heads * p.dim;
+  const Terms<T> term(p.attn_l);
+  if (threadIdx.x == 0) s_hubs = 0;
+  __syncthreads();
+  struct Cols {
+    int64_t c;
+    int h0, h1, cut;
+    bool live;
+  };
+  auto columns = [&](int64_t c0) {
+    Cols k;
+    k.c = c0 + static_cast<int64_t>(l) * VEC;
+    k.live = k.c < row_len;
+    k.h0 = k.live ? static_cast<int>(k.c / p.dim) : 0;
+    k.cut = static_cast<int>(min(static_cast<int64_t>(VEC), (k.h0 + 1) * p.dim - k.c));
+    k.h1 = k.cut < VEC ? k.h0 + 1 : k.h0;
+    return k;
+  };
+  struct Acc {
+    float v[VEC];
+    float el0, el1;
+  };
+  auto clear = [](Acc& a) {
+#pragma unroll
+    for (int k = 0; k < VEC; ++k) a.v[k] = 0.f;
+    a.el0 = a.el1 = 0.f;
+  };
+  // lane j of the group holds edge j: its destination (-1: none) and where its weights are
+  auto edge_of = [&](int64_t at, int64_t end, int64_t& dst, int64_t& weight) {
+    dst = -1;
+    weight = 0;
+    if (at >= end) return;
+    if constexpr (sizeof(I) == 4) {
+      weight = static_cast<int64_t>(index[at]);
+      dst = static_cast<int64_t>(static_cast<uint32_t>(weight) / p.fanout);
+    } else {
+      dst = static_cast<int64_t>(index[at]);
+      weight = p.eids[at];
+    }
+    if (dst >= p.num_dst) dst = -1;
+  };
+  auto add_edges = [&](int64_t my_dst, int64_t my_weight, int n, const Cols& col, Acc& acc) {
+    for (int e0 = 0; e0 < n; e0 += kUnroll) {
+      float v[kUnroll][VEC], a0[kUnroll], a1[kUnroll], z0[kUnroll], z1[kUnroll];
+#pragma unroll
+      for (int u = 0; u < kUnroll; ++u) {
+#pragma unroll
+        for (int k = 0; k < VEC; ++k) v[u][k] = 0.f;
+        a0[u] = a1[u] = z0[u] = z1[u] = 0.f;
+        if (e0 + u < n) {
+          const int64_t d = __shfl(my_dst, e0 + u, LPR), w = __shfl(my_weight, e0 + u, LPR);
+          if (d >= 0 && col.live) {
+            load_vec<T, VEC>(d_out, d * row_len + col.c, v[u]);
+            a0[u] = p.attn[w * p.heads + col.h0];
+            z0[u] = p.dz[w * p.heads + col.h0];
+            if (VEC > 1 && col.h1 != col.h0) {
+              a1[u] = p.attn[w * p.heads + col.h1];
+              z1[u] = p.dz[w * p.heads + col.h1];
+            }
+          }
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < kUnroll; ++u) {
+#pragma unroll
+        for (int k = 0; k < VEC; ++k) acc.v[k] += (k < col.cut ? a0[u] : a1[u]) * v[u][k];
+        acc.el0 += z0[u];
+        acc.el1 += z1[u];
+      }
+    }
+  };
+  auto finish = [&](int64_t r, const Cols& col, const Acc& acc) {
+    if (!col.live) return;
+    const float e0 = term(acc.el0), e1 = term(acc.el1);
+    float r0 = 0.f, r1 = 0.f;
+    if (r < p.num_dst) {
+      r0 = term(p.d_er[r * p.heads + col.h0]);
+      r1 = term(p.d_er[r * p.heads + col.h1]);
+    }
+    float out[VEC];
+#pragma unroll
+    for (int k = 0; k < VEC; ++k) {
+      const bool first = k < col.cut;
+      out[k] = as_stored<T>(acc.v[k]);
+      if (r < p.num_dst) out[k] = as_stored<T>(out[k] + as_stored<T>((first ? r0 : r1) * p.attn_r.at(col.c + k)));
+      out[k] += as_stored<T>((first ? e0 : e1) * p.attn_l.at(col.c + k));
+      if ((col.c + k) % p.dim == 0) p.d_el[r * p.heads + (first ? col.h0 : col.h1)] = first ? e0 : e1;
+    }
+    store_vec<T, VEC>(d_ft, r * row_len + col.c, out);
+  };
+  const int64_t row_groups = static_cast<int64_t>(gridDim.x) * kGroups;
+  for (int64_t r = static_cast<int64_t>(grp) * gridDim.x + blockIdx.x; r < p.num_src; r += row_groups) {
+    const int64_t lo = static_cast<int64_t>(indptr[r]), hi = static_cast<int64_t>(indptr[r + 1]);
+    if (hi - lo > kGatHubEdges) {
+      if (l == 0) s_hub[atomicAdd(&s_hubs, 1)] = static_cast<int>(r);
+      continue;
+    }
+    int64_t dst, weight;
+    edge_of(lo + l, hi, dst, weight);
+    for (int64_t c0 = 0; c0 < row_len; c0 += LPR * VEC) {
+      const Cols col = columns(c0);
+      Acc acc;
+      clear(acc);
+      add_edges(dst, weight, static_cast<int>(min(hi - lo, static_cast<int64_t>(LPR))), col, acc);
+      for (int64_t e = lo + LPR; e < hi; e += LPR) {   // LPR < kGatHubEdges only
+        int64_t d, w;
+        edge_of(e + l, hi, d, w);
+        add_edges(d, w, static_cast<int>(min(hi - e, static_cast<int64_t>(LPR))), col, acc);
+      }
+      finish(r, col, acc);
+    }
+  }
+  __syncthreads();
+  const int hubs = s_hubs;
+  for (int i = 0; i < hubs; ++i) {
+    const int64_t r = s_hub[i];
+    const int64_t lo = static_cast<int64_t>(indptr[r]), hi = static_cast<int64_t>(indptr[r + 1]);
+    for (int64_t c0 = 0; c0 < row_len; c0 += LPR * VEC) {
+      const Cols col = columns(c0);
+      Acc acc;
+      clear(acc);
+      for (int64_t e = lo + grp * LPR; e < hi; e += kAggBlock) {
+        int64_t d, w;
+        edge_of(e + l, hi, d, w);
+        add_edges(d, w, static_cast<int>(min(hi - e, static_cast<int64_t>(LPR))), col, acc);
+      }
+#pragma unroll
+      for (int k = 0; k < VEC; ++k) s_sum[grp][k * LPR + l] = acc.v[k];
+      s_sum[grp][VEC * LPR + l] = acc.el0;
+      s_sum[grp][(VEC + 1) * LPR + l] = acc.el1;
+      __syncthreads();
+      if (grp == 0) {
+        clear(acc);
+#pragma unroll 1
+        for (int g = 0; g < kGroups; ++g) {
+#pragma unroll
+          for (int k = 0; k < VEC; ++k) acc.v[k] += s_sum[g][k * LPR + l];
+          acc.el0 += s_sum[g][VEC * LPR + l];
+          acc.el1 += s_sum[g][(VEC + 1) * LPR + l];
+        }
+        finish(r, col, acc);
+      }
+      __syncthreads();
+    }
+  }
+}
+
+template <typename T, int VEC, typename I>
+static void launch_gat_source(const GatSourceParams& p, hipStream_t st) {
+  const int64_t per_row = ceil_div(p.heads * p.dim, VEC);
+#define APT_GAT_SOURCE(LPR)                                                                                        \
+  do {                                                                                                            \
+    const int64_t blocks = std::max(ceil_div(p.num_src, kGatHubList),                                             \
+                                    std::min<int64_t>(ceil_div(p.num_src, kAggBlock / LPR), kGatSourceBlocks));   \
+    hipLaunchKernelGGL((gat_source_kernel<T, VEC, LPR, I>), dim3(static_cast<unsigned>(blocks)), dim3(kAggBlock), 0, \
+                       st, p);                                                                                    \
+  } while (0)
+  if (per_row <= 8) APT_GAT_SOURCE(8);
+  else if (per_row <= 16) APT_GAT_SOURCE(16);
+  else if (per_row <= 32) APT_GAT_SOURCE(32);
+  else APT_GAT_SOURCE(64);
+#undef APT_GAT_SOURCE
+}
+
+template <typename T, typename I>
+static void launch_gat_source_t(const GatSourceParams& p, hipStream_t st) {
+  const bool aligned = ((reinterpret_cast<uintptr_t>(p.d_out) | reinterpret_cast<uintptr_t>(p.d_ft)) & 15) == 0;
+  if (aligned && (p.heads * p.dim) % 4 == 0 && p.dim >= 4) launch_gat_source<T, 4, I>(p, st);
+  else launch_gat_source<T, 1, I>(p, st);
+}
+
+// ------------------------------------------------------------------ backward, parameters
+// Column sums over the rows: a workgroup has a run of rows, a thread VEC columns of every RG-th of them.
+constexpr int kParamBlocks = 512;
+
+template <typename T, int VEC>
+__global__ __launch_bounds__(kAggBlock) void gat_param_grad_kernel(const T* __restrict__ ft, const T* __restrict__ d_out,
+                                                                   const float* __restrict__ d_el,
+                                                                   const float* __restrict__ d_er, int64_t num_src,
+                                                                   int64_t num_dst, int heads, int64_t dim, int lanes,
+                                                                   int64_t rows_per_block, float* __restrict__ part,
+                                                                   ParamVec attn_l) {
+  constexpr int kUnroll = 4;
+  const Terms<T> term(attn_l);
+  __shared__ float s_sum[3 * VEC][kAggBlock];
+  const int64_t row_len = heads * dim;
+  const int groups = kAggBlock / lanes, grp = threadIdx.x / lanes, l = threadIdx.x % lanes;
+  const int64_t begin = blockIdx.x * rows_per_block, end = min(begin + rows_per_block, num_src);
+  float* out = part + static_cast<int64_t>(blockIdx.x) * 3 * row_len;
+  for (int64_t c0 = 0; c0 < row_len; c0 += static_cast<int64_t>(lanes) * VEC) {
+    const int64_t c = c0 + static_cast<int64_t>(l) * VEC;
+    const bool live = c < row_len;
+    const int h0 = live ? static_cast<int>(c / dim) : 0;
+    const int cut = static_cast<int>(min(static_cast<int64_t>(VEC), (h0 + 1) * dim - c));
+    const int h1 = cut < VEC ? h0 + 1 : h0;
+    float sl[VEC], sr[VEC], sb[VEC];
+#pragma unroll
+    for (int k = 0; k < VEC; ++k) sl[k] = sr[k] = sb[k] = 0.f;
+    for (int64_t r0 = begin + grp; r0 < end; r0 += static_cast<int64_t>(kUnroll) * groups) {
+      float v[kUnroll][VEC], o[kUnroll][VEC], l0[kUnroll], l1[kUnroll], e0[kUnroll], e1[kUnroll];
+#pragma unroll
+      for (int u = 0; u < kUnroll; ++u) {
+        const int64_t r = r0 + u * groups;
+#pragma unroll
+        for (int k = 0; k < VEC; ++k) v[u][k] = o[u][k] = 0.f;
+        l0[u] = l1[u] = e0[u] = e1[u] = 0.f;
+        if (r < end && live) {
+          load_vec<T, VEC>(ft, r * row_len + c, v[u]);
+          l0[u] = d_el[r * heads + h0];
+          l1[u] = d_el[r * heads + h1];
+          if (r < num_dst) {
+            load_vec<T, VEC>(d_out, r * row_len + c, o[u]);
+            e0[u] = term(d_er[r * heads + h0]);
+            e1[u] = term(d_er[r * heads + h1]);
+          }
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < kUnroll; ++u)
+#pragma unroll
+        for (int k = 0; k < VEC; ++k) {
+          sl[k] += term((k < cut ? l0[u] : l1[u]) * v[u][k]);
+          sr[k] += term((k < cut ? e0[u] : e1[u]) * v[u][k]);
+          sb[k] += o[u][k];
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < VEC; ++k) {
+      s_sum[k][threadIdx.x] = sl[k];
+      s_sum[VEC + k][threadIdx.x] = sr[k];
+      s_sum[2 * VEC + k][threadIdx.x] = sb[k];
+    }
+    __syncthreads();
+    if (grp == 0 && live) {
+#pragma unroll
+      for (int k = 0; k < VEC; ++k)
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+          float sum = 0.f;
+          for (int g = 0; g < groups; ++g) sum += s_sum[q * VEC + k][g * lanes + l];
+          out[q * row_len + c + k] = sum;
+        }
+    }
+    __syncthreads();
+  }
+}
+
+static int64_t param_blocks(int64_t num_src) { return std::min<int64_t>(std::max<int64_t>(ceil_div(num_src, 64), 1), kParamBlocks); }
+
+template <typename T>
+static void launch_param_grad(const void* ft, const void* d_out, const float* d_el, const float* d_er, int64_t num_src,
+                              int64_t num_dst, int heads, int64_t dim, float* part, ParamVec attn_l, hipStream_t st) {
+  const int64_t blocks = param_blocks(num_src), rows = ceil_div(num_src, blocks), row_len = heads * dim;
+  const bool vec4 = row_len % 4 == 0 && dim >= 4 && ((reinterpret_cast<uintptr_t>(ft) | reinterpret_cast<uintptr_t>(d_out)) & 15) == 0;
+  int lanes = 8;
+  while (lanes < kAggBlock && lanes * (vec4 ? 4 : 1) < row_len) lanes <<= 1;
+  const dim3 grid(static_cast<unsigned>(blocks)), block(kAggBlock);
+#define APT_PARAM(V)                                                                                               \
+  hipLaunchKernelGGL((gat_param_grad_kernel<T, V>), grid, block, 0, st, static_cast<const T*>(ft),                  \
+                     static_cast<const T*>(d_out), d_el, d_er, num_src, num_dst, heads, dim, lanes, rows, part, attn_l)
+  if (vec4) APT_PARAM(4);
+  else APT_PARAM(1);
+#undef APT_PARAM
+}
+
+static size_t align256(size_t x) { return (x + 255) / 256 * 256; }
+
+}  // namespace apt
+
+extern "C" int apt_gat_layer(const int64_t* neighbors, int64_t num_dst, int fanout, const void* ft, int64_t num_src,
+                             int heads, int64_t dim, int elem_size, const void* attn_l, const void* attn_r,
+                             int attn_elem_size, const void* bias, float negative_slope, float* el, float* er, void* out,
+                             float* attn_out, void* stream) {
+  using namespace apt;
+  const char* who = "apt_gat_layer";
+  APT_REQUIRE(num_dst >= 0 && num_dst <= num_src && fanout > 0 && heads > 0 && dim > 0, APT_EINVAL,
+              "%s: bad shape (num_dst %lld, num_src %lld, fanout %d, heads %d, dim %lld)", who, (long long)num_dst,
+              (long long)num_src, fanout, heads, (long long)dim);
+  APT_REQUIRE((elem_size == 2 || elem_size == 4) && (attn_elem_size == 2 || attn_elem_size == 4), APT_EINVAL,
+              "%s: elem_size %d, attn_elem_size %d (4 = fp32, 2 = bf16)", who, elem_size, attn_elem_size);
+  if (num_src == 0) return APT_OK;
+  APT_REQUIRE(ft != nullptr && attn_l != nullptr && attn_r != nullptr && el != nullptr && (num_dst == 0 || er != nullptr),
+              APT_EINVAL, "%s: a tensor is NULL", who);
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  const ParamVec al{attn_l, attn_elem_size}, ar{attn_r, attn_elem_size};
+  const bool done = elem_size == 4 ? launch_pair_scores<float, 4>(ft, num_src, num_dst, heads, dim, al, ar, el, er, st)
+                                   : launch_pair_scores<uint16_t, 8>(ft, num_src, num_dst, heads, dim, al, ar, el, er, st) ||
+                                         launch_pair_scores<uint16_t, 4>(ft, num_src, num_dst, heads, dim, al, ar, el, er, st);
+  if (!done) {
+    const dim3 grid(static_cast<unsigned>(std::min<int64_t>(ceil_div(num_src * heads, kAggWaves), 1 << 16))), block(kAggBlock);
+    if (elem_size == 4)
+      hipLaunchKernelGGL(gat_pair_scores_any_kernel<float>, grid, block, 0, st, static_cast<const float*>(ft), num_src, num_dst,
+                         heads, dim, al, ar, el, er);
+    else
+      hipLaunchKernelGGL(gat_pair_scores_any_kernel<uint16_t>, grid, block, 0, st, static_cast<const uint16_t*>(ft), num_src,
+                         num_dst, heads, dim, al, ar, el, er);
+  }
+  APT_LAUNCH_CHECK("gat_pair_scores_kernel");
+  return gat_block(who, neighbors, num_dst, nullptr, fanout, ft, num_src, heads, dim, elem_size, el, er, negative_slope, out,
+                   true, attn_out, bias, st);
+}
+
+extern "C" size_t apt_gat_layer_backward_workspace_bytes(int64_t num_dst, int fanout, int64_t num_src, int heads, int64_t dim,
+                                                         int64_t num_edges) {
+  using namespace apt;
+  if (num_dst < 0 || fanout <= 0 || num_src < 0 || heads <= 0 || dim <= 0 || num_edges < 0) return 0;
+  const int64_t weights = std::max(num_dst * fanout, num_edges) * heads;
+  return align256(sizeof(float) * 2 * weights) + align256(sizeof(float) * (num_dst + num_src) * heads) +
+         align256(sizeof(float) * 3 * heads * dim * param_blocks(num_src)) + 256;
+}
+
+extern "C" int apt_gat_layer_backward(const int64_t* neighbors, int64_t num_dst, int fanout, const void* ft,
+                                      int64_t num_src, int heads, int64_t dim, int elem_size, const void* attn_l,
+                                      const void* attn_r, int attn_elem_size, float negative_slope, const float* el,
+                                      const float* er, const float* attn, const void* d_out, const void* indptr,
+                                      const void* index, int index_bytes, const int64_t* eids, const int64_t* csc_indptr,
+                                      int64_t num_edges, void* d_ft, void* d_attn_l, void* d_attn_r, void* d_bias,
+                                      void* workspace, size_t workspace_bytes, void* stream) {
+  using namespace apt;
+  const char* who = "apt_gat_layer_backward";
+  APT_REQUIRE(num_dst >= 0 && num_dst <= num_src && num_src <= 0x7fffffffLL && fanout > 0 && heads > 0 && dim > 0 && num_edges >= 0,
+              APT_EINVAL, "%s: bad shape (num_dst %lld, num_src %lld, fanout %d, heads %d, dim %lld)", who,
+              (long long)num_dst, (long long)num_src, fanout, heads, (long long)dim);
+  APT_REQUIRE((elem_size == 2 || elem_size == 4) && (attn_elem_size == 2 || attn_elem_size == 4), APT_EINVAL,
+              "%s: elem_size %d, attn_elem_size %d (4 = fp32, 2 = bf16)", who, elem_size, attn_elem_size);
+  APT_REQUIRE(index_bytes == 4 || (index_bytes == 8 && eids != nullptr && csc_indptr != nullptr), APT_EINVAL,
+              "%s: index_bytes %d (4 = slots, 8 = destinations, with eids and csc_indptr)", who, index_bytes);
+  APT_REQUIRE(workspace != nullptr && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0 &&
+                  workspace_bytes >= apt_gat_layer_backward_workspace_bytes(num_dst, fanout, num_src, heads, dim, num_edges),
+              APT_EWORKSPACE, "%s: workspace too small or not 16-byte aligned", who);
+  if (num_src == 0) return APT_OK;
+  APT_REQUIRE(ft != nullptr && attn_l != nullptr && attn_r != nullptr && el != nullptr && indptr != nullptr && d_ft != nullptr &&
+                  (num_dst == 0 || (neighbors != nullptr && er != nullptr && attn != nullptr && d_out != nullptr && index != nullptr)),
+              APT_EINVAL, "%s: a tensor is NULL", who);
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  const bool by_slot = index_bytes == 4;
+  char* ws = static_cast<char*>(workspace);
+  const int64_t weights = std::max(num_dst * fanout, num_edges) * heads;
+  float* dz = reinterpret_cast<float*>(ws);
+  float* a_edge = dz + weights;
+  ws += align256(sizeof(float) * 2 * weights);
+  float* d_er = reinterpret_cast<float*>(ws);
+  float* d_el = d_er + num_dst * heads;
+  ws += align256(sizeof(float) * (num_dst + num_src) * heads);
+  float* part = reinterpret_cast<float*>(ws);
+  if (const int rc = gat_edge_grad(who, neighbors, num_dst, fanout, ft, num_src, heads, dim, elem_size, el, er,
+                                   negative_slope, attn, d_out, true, by_slot ? nullptr : csc_indptr, a_edge, dz, d_er, st))
+    return rc;
+  GatSourceParams p;
+  p.indptr = indptr;
+  p.index = index;
+  p.eids = eids;
+  p.fanout = static_cast<uint32_t>(fanout);
+  p.attn = by_slot ? attn : a_edge;
+  p.dz = dz;
+  p.d_out = d_out;
+  p.d_er = d_er;
+  p.attn_l = ParamVec{attn_l, attn_elem_size};
+  p.attn_r = ParamVec{attn_r, attn_elem_size};
+  p.num_dst = num_dst;
+  p.num_src = num_src;
+  p.heads = heads;
+  p.dim = dim;
+  p.d_ft = d_ft;
+  p.d_el = d_el;
+  if (elem_size == 4) {
+    if (by_slot) launch_gat_source_t<float, uint32_t>(p, st);
+    else launch_gat_source_t<float, int64_t>(p, st);
+  } else {
+    if (by_slot) launch_gat_source_t<uint16_t, uint32_t>(p, st);
+    else launch_gat_source_t<uint16_t, int64_t>(p, st);
+  }
+  APT_LAUNCH_CHECK("gat_source_kernel");
+  if (d_attn_l == nullptr && d_attn_r == nullptr && d_bias == nullptr) return APT_OK;
+  if (elem_size == 4) launch_param_grad<float>(ft, d_out, d_el, d_er, num_src, num_dst, heads, dim, part, p.attn_l, st);
+  else launch_param_grad<uint16_t>(ft, d_out, d_el, d_er, num_src, num_dst, heads, dim, part, p.attn_l, st);
+  APT_LAUNCH_CHECK("gat_param_grad_kernel");
+  const int64_t n = heads * dim;
+  const int splits = static_cast<int>(param_blocks(num_src));
+  if (attn_elem_size == 4) launch_partial_sums<float, float>(part, 3 * n, splits, d_attn_l, n, d_attn_r, n, nullptr, 0, st);
+  else launch_partial_sums<uint16_t, uint16_t>(part, 3 * n, splits, d_attn_l, n, d_attn_r, n, nullptr, 0, st);
+  APT_LAUNCH_CHECK("partial_sums_kernel");
+  if (d_bias == nullptr) return APT_OK;
+  if (elem_size == 4) launch_partial_sums<float, float>(part + 2 * n, 3 * n, splits, d_bias, n, nullptr, 0, nullptr, 0, st);
+  else launch_partial_sums<uint16_t, uint16_t>(part + 2 * n, 3 * n, splits, d_bias, n, nullptr, 0, nullptr, 0, st);
+  APT_LAUNCH_CHECK("partial_sums_kernel");
+  return APT_OK;
+}

@@ -17,6 +17,7 @@
 #include <algorithm>
 
 #include "common.hpp"
+#include "partial_sums.hpp"
 
 namespace apt {
 
@@ -265,49 +266,6 @@ __global__ __launch_bounds__(kWgradWaves * kWave) void wgrad_kernel(WgradParams 
   }
 }
 
-// out[e] = sum over the splits of part[s][e], e over the weight and then the bias.  64 elements per workgroup,
-// the splits dealt to its wavefronts.
-constexpr int kWgradReduceBlock = 1024;
-constexpr int kWgradReduceWaves = kWgradReduceBlock / kWave;
-
-template <typename T> __device__ __forceinline__ T wgrad_out(float v);
-template <> __device__ __forceinline__ float wgrad_out<float>(float v) { return v; }
-template <> __device__ __forceinline__ uint16_t wgrad_out<uint16_t>(float v) {
-  return __builtin_bit_cast(uint16_t, static_cast<__bf16>(v));
-}
-
-template <typename T>
-__global__ __launch_bounds__(kWgradReduceBlock) void wgrad_reduce_kernel(const float* __restrict__ part, int64_t stride,
-                                                                         int splits, int64_t nk, int64_t n,
-                                                                         T* __restrict__ dw, T* __restrict__ db) {
-  constexpr int kUnroll = 8;
-  __shared__ float s_sum[kWgradReduceWaves][kWave];
-  const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
-  const int64_t e = static_cast<int64_t>(blockIdx.x) * kWave + lane;
-  const int64_t total = nk + (db != nullptr ? n : 0);
-  float sum = 0.f;
-  if (e < total) {
-    const float* src = part + e;
-    for (int s = wave; s < splits; s += kWgradReduceWaves * kUnroll) {
-      float v[kUnroll];
-#pragma unroll
-      for (int u = 0; u < kUnroll; ++u) {
-        const int t = s + u * kWgradReduceWaves;
-        v[u] = t < splits ? src[static_cast<int64_t>(t) * stride] : 0.f;
-      }
-#pragma unroll
-      for (int u = 0; u < kUnroll; ++u) sum += v[u];
-    }
-  }
-  s_sum[wave][lane] = sum;
-  __syncthreads();
-  if (wave != 0 || e >= total) return;
-#pragma unroll
-  for (int w = 1; w < kWgradReduceWaves; ++w) sum += s_sum[w][lane];
-  if (e < nk) dw[e] = wgrad_out<T>(sum);
-  else db[e - nk] = wgrad_out<T>(sum);
-}
-
 // How the rows are split: into as many parts as keep eight wavefronts on every CU, while a part keeps a few steps of
 // its loop and the partials (written once, read once) stay below half of the inputs they come from or a few
 // megabytes.  Both launches, against the library's GEMM and column sum, for n x k = 256 x 128:
@@ -400,14 +358,8 @@ extern "C" int apt_linear_wgrad(const void* dy, const void* x, int64_t m, int64_
     else launch_wgrad<uint16_t>(p, va, vb, st);
     APT_LAUNCH_CHECK("wgrad_kernel");
   }
-  const int64_t total = n * k + (db != nullptr ? n : 0);
-  const dim3 grid(static_cast<unsigned>(ceil_div(total, kWave)));
-  if (elem_size == 4)
-    hipLaunchKernelGGL(wgrad_reduce_kernel<float>, grid, dim3(kWgradReduceBlock), 0, st, p.part, p.part_stride, p.splits,
-                       n * k, n, static_cast<float*>(dw), static_cast<float*>(db));
-  else
-    hipLaunchKernelGGL(wgrad_reduce_kernel<uint16_t>, grid, dim3(kWgradReduceBlock), 0, st, p.part, p.part_stride,
-                       p.splits, n * k, n, static_cast<uint16_t*>(dw), static_cast<uint16_t*>(db));
-  APT_LAUNCH_CHECK("wgrad_reduce_kernel");
+  if (elem_size == 4) launch_partial_sums<float, float>(p.part, p.part_stride, p.splits, dw, n * k, db, n, nullptr, 0, st);
+  else launch_partial_sums<uint16_t, uint16_t>(p.part, p.part_stride, p.splits, dw, n * k, db, n, nullptr, 0, st);
+  APT_LAUNCH_CHECK("partial_sums_kernel");
   return APT_OK;
 }

@@ -12,6 +12,8 @@
 // edge order it degrades to the reference's atomic-per-edge behaviour.
 // u_mul_e multiplies (the reference's kernel adds, src/cuda/spmm.cu:78, and
 // has no caller).
+#include <algorithm>
+
 #include "common.hpp"
 #include "feature_rows.hpp"
 
@@ -393,15 +395,18 @@ __global__ __launch_bounds__(kAggBlock) void gat_scores_vec_kernel(const T* __re
 // row (all heads); the softmax runs online over the slots (running maximum,
 // rescaled sum), so a row's features are read once and nothing is written but
 // the result: no per-edge score, exponent or weight arrays, no atomics.
-template <typename T, int VEC, int LPR>
+// OUT: fp32, or the input's type with the layer's bias (optional, [heads, dim] of that type) added to the result as
+// it would be stored without one.
+template <typename T, typename OUT, int VEC, int LPR>
 __global__ __launch_bounds__(kAggBlock) void gat_ell_kernel(const int64_t* __restrict__ nbr, int64_t num_dst,
                                                             const int64_t* num_dst_dev, int fanout,
                                                             const T* __restrict__ ft, int64_t num_src,
                                                             int heads, int64_t dim,
                                                             const float* __restrict__ el,
                                                             const float* __restrict__ er, float slope,
-                                                            float* __restrict__ out,
-                                                            float* __restrict__ attn_out) {
+                                                            OUT* __restrict__ out,
+                                                            float* __restrict__ attn_out,
+                                                            const OUT* __restrict__ bias) {
   constexpr int kGroups = kAggBlock / LPR;
   constexpr int kUnroll = 5;
   const int64_t n = actual_count(num_dst, num_dst_dev);
@@ -456,7 +461,11 @@ __global__ __launch_bounds__(kAggBlock) void gat_ell_kernel(const int64_t* __res
       }
       const float inv = denom > 0.f ? 1.0f / denom : 0.f;
 #pragma unroll
-      for (int k = 0; k < VEC; ++k) out[i * row_len + d + k] = acc[k] * inv;
+      for (int k = 0; k < VEC; ++k) {
+        acc[k] *= inv;
+        if (bias != nullptr) acc[k] = as_stored<OUT>(acc[k]) + to_float<OUT>(bias[d + k]);
+      }
+      store_vec<OUT, VEC>(out, i * row_len + d, acc);
       // the lane that holds a head's first features also writes its attention weights
       if (attn_out != nullptr && d % dim == 0) {
         for (int s = 0; s < fanout; ++s) {
@@ -482,12 +491,12 @@ __global__ __launch_bounds__(kAggBlock) void gat_ell_kernel(const int64_t* __res
 // cross-lane reductions.  Feature layout: lane l holds VEC features of head
 // l / lph and adds up the source rows, fetching each slot's weight from the slot
 // layout with one shuffle.
-template <typename T, int VEC>
+template <typename T, typename OUT, int VEC>
 __global__ __launch_bounds__(kAggBlock) void gat_ell_wave_kernel(
     const int64_t* __restrict__ nbr, int64_t num_dst, const int64_t* num_dst_dev, int fanout,
     const T* __restrict__ ft, int64_t num_src, int heads, int log2_heads, int64_t dim,
-    const float* __restrict__ el, const float* __restrict__ er, float slope, float* __restrict__ out,
-    float* __restrict__ attn_out) {
+    const float* __restrict__ el, const float* __restrict__ er, float slope, OUT* __restrict__ out,
+    float* __restrict__ attn_out, const OUT* __restrict__ bias) {
   constexpr int kUnroll = 5;
   const int64_t n = actual_count(num_dst, num_dst_dev);
   const int lane = threadIdx.x % kWave;
@@ -539,38 +548,42 @@ __global__ __launch_bounds__(kAggBlock) void gat_ell_wave_kernel(
         for (int q = 0; q < VEC; ++q) acc[q] += au[u] * v[u][q];
     }
     if (live) {
+      if (bias != nullptr) {
 #pragma unroll
-      for (int q = 0; q < VEC; ++q) out[i * row_len + d + q] = acc[q];
+        for (int q = 0; q < VEC; ++q) acc[q] = as_stored<OUT>(acc[q]) + to_float<OUT>(bias[d + q]);
+      }
+      store_vec<OUT, VEC>(out, i * row_len + d, acc);
     }
   }
 }
 
-template <typename T, int VEC>
+template <typename T, typename OUT, int VEC>
 static bool launch_gat_wave(const int64_t* nbr, int64_t num_dst, const int64_t* num_dst_dev, int fanout,
                             const void* ft, int64_t num_src, int heads, int64_t dim, const float* el,
-                            const float* er, float slope, float* out, float* attn_out, hipStream_t st) {
+                            const float* er, float slope, void* out, float* attn_out, const void* bias, hipStream_t st) {
   if (dim % VEC != 0 || (heads & (heads - 1)) != 0 || heads * fanout > kWave) return false;
   const int64_t lph = dim / VEC;
   if ((lph & (lph - 1)) != 0 || heads * lph > kWave) return false;
   int log2_heads = 0;
   while ((1 << log2_heads) < heads) ++log2_heads;
   const unsigned blocks = static_cast<unsigned>(std::min<int64_t>(ceil_div(num_dst, kAggWaves), 1 << 20));
-  hipLaunchKernelGGL((gat_ell_wave_kernel<T, VEC>), dim3(blocks), dim3(kAggBlock), 0, st, nbr, num_dst, num_dst_dev,
-                     fanout, static_cast<const T*>(ft), num_src, heads, log2_heads, dim, el, er, slope, out, attn_out);
+  hipLaunchKernelGGL((gat_ell_wave_kernel<T, OUT, VEC>), dim3(blocks), dim3(kAggBlock), 0, st, nbr, num_dst, num_dst_dev,
+                     fanout, static_cast<const T*>(ft), num_src, heads, log2_heads, dim, el, er, slope,
+                     static_cast<OUT*>(out), attn_out, static_cast<const OUT*>(bias));
   return true;
 }
 
-template <typename T, int VEC>
+template <typename T, typename OUT, int VEC>
 static void launch_gat(const int64_t* nbr, int64_t num_dst, const int64_t* num_dst_dev, int fanout,
                        const void* ft, int64_t num_src, int heads, int64_t dim, const float* el,
-                       const float* er, float slope, float* out, float* attn_out, hipStream_t st) {
+                       const float* er, float slope, void* out, float* attn_out, const void* bias, hipStream_t st) {
   const int64_t per_row = ceil_div(static_cast<int64_t>(heads) * dim, VEC);
   const T* x = static_cast<const T*>(ft);
 #define APT_GAT(LPR)                                                                                  \
-  hipLaunchKernelGGL((gat_ell_kernel<T, VEC, LPR>),                                                   \
+  hipLaunchKernelGGL((gat_ell_kernel<T, OUT, VEC, LPR>),                                              \
                      dim3(static_cast<unsigned>(std::min<int64_t>(ceil_div(num_dst, kAggBlock / LPR), 1 << 20))), \
                      dim3(kAggBlock), 0, st, nbr, num_dst, num_dst_dev, fanout, x, num_src, heads, dim, el, er, \
-                     slope, out, attn_out)
+                     slope, static_cast<OUT*>(out), attn_out, static_cast<const OUT*>(bias))
   if (per_row <= 8) APT_GAT(8);
   else if (per_row <= 16) APT_GAT(16);
   else if (per_row <= 32) APT_GAT(32);
@@ -588,11 +601,13 @@ static void launch_gat(const int64_t* nbr, int64_t num_dst, const int64_t* num_d
 // weight a and dz per edge and head, and der[i, h] = sum_k dz_k.  The source half
 // (d ft[s] = sum a dOut[dst], d el[s] = sum dz) is a sum over the edges of a
 // source and runs through the SpMM kernels on the block's CSR order.
-template <typename T>
+// Without csc_indptr the edges stay where their slots are: dz_edge is [num_dst * fanout, heads] and a_edge is not
+// written (the attention weights are in that order already).  DT: type of d_out.
+template <typename T, typename DT>
 __global__ __launch_bounds__(kAggBlock) void gat_bwd_edge_kernel(
     const int64_t* __restrict__ nbr, int64_t num_dst, int fanout, const T* __restrict__ ft, int64_t num_src,
     int heads, int64_t dim, const float* __restrict__ el, const float* __restrict__ er, float slope,
-    const float* __restrict__ attn, const float* __restrict__ d_out, const int64_t* __restrict__ csc_indptr,
+    const float* __restrict__ attn, const DT* __restrict__ d_out, const int64_t* __restrict__ csc_indptr,
     float* __restrict__ a_edge, float* __restrict__ dz_edge, float* __restrict__ d_er) {
   const int lane = threadIdx.x % kWave;
   const int64_t items = num_dst * heads;
@@ -609,7 +624,7 @@ __global__ __launch_bounds__(kAggBlock) void gat_bwd_edge_kernel(
       if (src < 0 || src >= num_src) continue;   // wave-uniform
       float part = 0.f;
       for (int64_t d = lane; d < dim; d += kWave)
-        part += d_out[it * dim + d] * to_float<T>(ft[(src * heads + h) * dim + d]);
+        part += to_float<DT>(d_out[it * dim + d]) * to_float<T>(ft[(src * heads + h) * dim + d]);
 #pragma unroll
       for (int off = kWave / 2; off > 0; off >>= 1) part += __shfl_xor(part, off, kWave);
       if (lane == k) g = part;
@@ -628,8 +643,8 @@ __global__ __launch_bounds__(kAggBlock) void gat_bwd_edge_kernel(
     for (int off = kWave / 2; off > 0; off >>= 1) sum_dz += __shfl_xor(sum_dz, off, kWave);
     const uint64_t m = ballot(valid);
     if (valid) {
-      const int64_t e = csc_indptr[i] + rank_below(m);
-      a_edge[e * heads + h] = a;
+      const int64_t e = csc_indptr != nullptr ? csc_indptr[i] + rank_below(m) : i * fanout + lane;
+      if (csc_indptr != nullptr) a_edge[e * heads + h] = a;
       dz_edge[e * heads + h] = dz;
     }
     if (lane == 0) d_er[it] = sum_dz;
@@ -641,11 +656,11 @@ __global__ __launch_bounds__(kAggBlock) void gat_bwd_edge_kernel(
 // lanes.  The row's source features are read once, VEC per lane; the dot of a
 // slot is reduced over the head's lanes with xor shuffles and parked in
 // dz_edge until the row's sum is known.
-template <typename T, int VEC, int G>
+template <typename T, typename DT, int VEC, int G>
 __global__ __launch_bounds__(kAggBlock) void gat_bwd_edge_group_kernel(
     const int64_t* __restrict__ nbr, int64_t num_dst, int fanout, const T* __restrict__ ft, int64_t num_src,
     int heads, int64_t dim, const float* __restrict__ el, const float* __restrict__ er, float slope,
-    const float* __restrict__ attn, const float* __restrict__ d_out, const int64_t* __restrict__ csc_indptr,
+    const float* __restrict__ attn, const DT* __restrict__ d_out, const int64_t* __restrict__ csc_indptr,
     float* __restrict__ a_edge, float* __restrict__ dz_edge, float* __restrict__ d_er) {
   constexpr int kGroups = kAggBlock / G;
   constexpr int kUnroll = 5;
@@ -659,10 +674,11 @@ __global__ __launch_bounds__(kAggBlock) void gat_bwd_edge_group_kernel(
   for (int64_t i = static_cast<int64_t>(blockIdx.x) * kGroups + grp; i < num_dst;
        i += static_cast<int64_t>(gridDim.x) * kGroups) {
     const int64_t* ids = nbr + i * fanout;
-    const int64_t e0 = csc_indptr[i];
+    const bool by_slot = csc_indptr == nullptr;
+    const int64_t e0 = by_slot ? i * fanout : csc_indptr[i];
     float go[VEC];
 #pragma unroll
-    for (int q = 0; q < VEC; ++q) go[q] = live ? d_out[i * row_len + d + q] : 0.f;
+    for (int q = 0; q < VEC; ++q) go[q] = live ? to_float<DT>(d_out[i * row_len + d + q]) : 0.f;
     float s = 0.f;
     int64_t e = e0;
     for (int k0 = 0; k0 < fanout; k0 += kUnroll) {
@@ -683,6 +699,7 @@ __global__ __launch_bounds__(kAggBlock) void gat_bwd_edge_group_kernel(
       }
 #pragma unroll
       for (int u = 0; u < kUnroll; ++u) {
+        if (by_slot) e = e0 + k0 + u;
         if (!ok[u]) continue;  // group-uniform
         float part = 0.f;
 #pragma unroll
@@ -701,11 +718,12 @@ __global__ __launch_bounds__(kAggBlock) void gat_bwd_edge_group_kernel(
       e = e0;
       for (int k = 0; k < fanout; ++k) {
         const int64_t src = ids[k];
+        if (by_slot) e = e0 + k;
         if (src < 0 || src >= num_src) continue;
         const float a = attn[(i * fanout + k) * heads + h];
         const float z = el[src * heads + h] + er_i;
         const float dz = a * (dz_edge[e * heads + h] - s) * (z > 0.f ? 1.f : slope);
-        a_edge[e * heads + h] = a;
+        if (!by_slot) a_edge[e * heads + h] = a;
         dz_edge[e * heads + h] = dz;
         sum_dz += dz;
         ++e;
@@ -724,11 +742,11 @@ __global__ __launch_bounds__(kAggBlock) void gat_bwd_edge_group_kernel(
 // destination instead of six accesses per slot and head by one lane in sixteen).
 // Needs heads and lph to be powers of two, heads * lph <= 64 and
 // heads * fanout <= 64.
-template <typename T, int VEC>
+template <typename T, typename DT, int VEC>
 __global__ __launch_bounds__(kAggBlock) void gat_bwd_edge_wave_kernel(
     const int64_t* __restrict__ nbr, int64_t num_dst, int fanout, const T* __restrict__ ft, int64_t num_src,
     int heads, int log2_heads, int64_t dim, const float* __restrict__ el, const float* __restrict__ er, float slope,
-    const float* __restrict__ attn, const float* __restrict__ d_out, const int64_t* __restrict__ csc_indptr,
+    const float* __restrict__ attn, const DT* __restrict__ d_out, const int64_t* __restrict__ csc_indptr,
     float* __restrict__ a_edge, float* __restrict__ dz_edge, float* __restrict__ d_er) {
   constexpr int kUnroll = 5;
   const int lane = threadIdx.x % kWave;
@@ -744,10 +762,11 @@ __global__ __launch_bounds__(kAggBlock) void gat_bwd_edge_wave_kernel(
     const bool valid = id >= 0 && id < num_src;
     const float a = valid ? attn[(i * fanout + k) * heads + hs] : 0.f;
     const float z = valid ? el[id * heads + hs] + er[i * heads + hs] : 0.f;
-    const int64_t e0 = csc_indptr[i];
+    const int64_t e0 = csc_indptr != nullptr ? csc_indptr[i] : 0;
     float go[VEC];
 #pragma unroll
-    for (int q = 0; q < VEC; ++q) go[q] = live ? d_out[i * row_len + d + q] : 0.f;
+    for (int q = 0; q < VEC; ++q) go[q] = 0.f;
+    if (live) load_vec<DT, VEC>(d_out, i * row_len + d, go);
     float my_part = 0.f;   // slot layout: dOut[i, hs] . ft[id, hs]
     for (int u0 = 0; u0 < fanout; u0 += kUnroll) {
       float v[kUnroll][VEC];
@@ -786,7 +805,9 @@ __global__ __launch_bounds__(kAggBlock) void gat_bwd_edge_wave_kernel(
     const uint64_t vm = ballot(valid && hs == 0);
     const int first = k << log2_heads;
     const int rank = __popcll(vm & (first == 0 ? 0ull : (~0ull >> (kWave - first))));
-    if (valid) {
+    if (csc_indptr == nullptr) {
+      if (slot) dz_edge[(i * fanout + k) * heads + hs] = dz;
+    } else if (valid) {
       const int64_t e = e0 + rank;
       a_edge[e * heads + hs] = a;
       dz_edge[e * heads + hs] = dz;
@@ -795,40 +816,41 @@ __global__ __launch_bounds__(kAggBlock) void gat_bwd_edge_wave_kernel(
   }
 }
 
-template <typename T, int VEC>
+template <typename T, typename DT, int VEC>
 static bool launch_gat_bwd_wave(const int64_t* nbr, int64_t num_dst, int fanout, const void* ft, int64_t num_src,
                                 int heads, int64_t dim, const float* el, const float* er, float slope,
-                                const float* attn, const float* d_out, const int64_t* csc_indptr, float* a_edge,
+                                const float* attn, const void* d_out, const int64_t* csc_indptr, float* a_edge,
                                 float* dz_edge, float* d_er, hipStream_t st) {
   if (dim % VEC != 0 || (heads & (heads - 1)) != 0 || heads * fanout > kWave) return false;
   const int64_t lph = dim / VEC;
   if ((lph & (lph - 1)) != 0 || heads * lph > kWave) return false;
-  if ((reinterpret_cast<uintptr_t>(ft) & 15) != 0) return false;
+  if (((reinterpret_cast<uintptr_t>(ft) | reinterpret_cast<uintptr_t>(d_out)) & 15) != 0) return false;
   int log2_heads = 0;
   while ((1 << log2_heads) < heads) ++log2_heads;
   const unsigned blocks = static_cast<unsigned>(std::min<int64_t>(ceil_div(num_dst, kAggWaves), 1 << 20));
-  hipLaunchKernelGGL((gat_bwd_edge_wave_kernel<T, VEC>), dim3(blocks), dim3(kAggBlock), 0, st, nbr, num_dst, fanout,
-                     static_cast<const T*>(ft), num_src, heads, log2_heads, dim, el, er, slope, attn, d_out,
+  hipLaunchKernelGGL((gat_bwd_edge_wave_kernel<T, DT, VEC>), dim3(blocks), dim3(kAggBlock), 0, st, nbr, num_dst, fanout,
+                     static_cast<const T*>(ft), num_src, heads, log2_heads, dim, el, er, slope, attn,
+                     static_cast<const DT*>(d_out),
                      csc_indptr, a_edge, dz_edge, d_er);
   return true;
 }
 
-template <typename T, int VEC>
+template <typename T, typename DT, int VEC>
 static bool launch_gat_bwd_group(const int64_t* nbr, int64_t num_dst, int fanout, const void* ft, int64_t num_src,
                                  int heads, int64_t dim, const float* el, const float* er, float slope,
-                                 const float* attn, const float* d_out, const int64_t* csc_indptr, float* a_edge,
+                                 const float* attn, const void* d_out, const int64_t* csc_indptr, float* a_edge,
                                  float* dz_edge, float* d_er, hipStream_t st) {
   if (dim % VEC != 0) return false;
   const int64_t lph = dim / VEC;
   if (lph > kWave || (lph & (lph - 1)) != 0 || heads * lph > kWave) return false;
-  if ((reinterpret_cast<uintptr_t>(ft) & 15) != 0) return false;
+  if (((reinterpret_cast<uintptr_t>(ft) | reinterpret_cast<uintptr_t>(d_out)) & 15) != 0) return false;
   const int64_t lanes = heads * lph;
   const T* x = static_cast<const T*>(ft);
 #define APT_GATB(G)                                                                                   \
-  hipLaunchKernelGGL((gat_bwd_edge_group_kernel<T, VEC, G>),                                          \
+  hipLaunchKernelGGL((gat_bwd_edge_group_kernel<T, DT, VEC, G>),                                          \
                      dim3(static_cast<unsigned>(std::min<int64_t>(ceil_div(num_dst, kAggBlock / G), 1 << 20))), \
                      dim3(kAggBlock), 0, st, nbr, num_dst, fanout, x, num_src, heads, dim, el, er, slope, attn, \
-                     d_out, csc_indptr, a_edge, dz_edge, d_er)
+                     static_cast<const DT*>(d_out), csc_indptr, a_edge, dz_edge, d_er)
   if (lanes <= 8) APT_GATB(8);
   else if (lanes <= 16) APT_GATB(16);
   else if (lanes <= 32) APT_GATB(32);
@@ -1034,41 +1056,57 @@ extern "C" int apt_gat_scores(const void* x, int64_t num_rows, int heads, int64_
   return APT_OK;
 }
 
+namespace apt {
+template <typename T, typename OUT>
+static void gat_block_as(const int64_t* neighbors, int64_t num_dst, const int64_t* num_dst_dev, int fanout, const void* ft,
+                         int64_t num_src, int heads, int64_t dim, const float* el, const float* er, float slope, void* out,
+                         float* attn_out, const void* bias, hipStream_t st) {
+  const bool vec4 = dim % 4 == 0 && ((reinterpret_cast<uintptr_t>(ft) | reinterpret_cast<uintptr_t>(out)) & 15) == 0;
+  if (vec4 && num_src > 0 &&
+      launch_gat_wave<T, OUT, 4>(neighbors, num_dst, num_dst_dev, fanout, ft, num_src, heads, dim, el, er, slope, out,
+                                 attn_out, bias, st))
+    return;
+#define APT_GAT_BLOCK(V) \
+  launch_gat<T, OUT, V>(neighbors, num_dst, num_dst_dev, fanout, ft, num_src, heads, dim, el, er, slope, out, attn_out, bias, st)
+  if constexpr (sizeof(T) == 2) {
+    if (vec4 && dim % 8 == 0) {
+      APT_GAT_BLOCK(8);
+      return;
+    }
+  }
+  if (vec4) APT_GAT_BLOCK(4);
+  else APT_GAT_BLOCK(1);
+#undef APT_GAT_BLOCK
+}
+
+// out: fp32 without a bias, or (like_input) the input's type with one.  Shared with the GAT layer (gat_layer.hip).
+int gat_block(const char* who, const int64_t* neighbors, int64_t num_dst, const int64_t* num_dst_dev, int fanout,
+              const void* ft, int64_t num_src, int heads, int64_t dim, int elem_size, const float* el, const float* er,
+              float slope, void* out, bool like_input, float* attn_out, const void* bias, hipStream_t st) {
+  APT_REQUIRE(num_dst >= 0 && fanout > 0 && heads > 0 && dim > 0 && num_src >= 0, APT_EINVAL,
+              "%s: bad shape (num_dst %lld, fanout %d, heads %d, dim %lld)", who, (long long)num_dst, fanout, heads,
+              (long long)dim);
+  APT_REQUIRE(elem_size == 2 || elem_size == 4, APT_EINVAL, "%s: elem_size %d (4 = fp32, 2 = bf16)", who, elem_size);
+  if (num_dst == 0) return APT_OK;
+  APT_REQUIRE(neighbors != nullptr && out != nullptr && er != nullptr && ((ft != nullptr && el != nullptr) || num_src == 0),
+              APT_EINVAL, "%s: a tensor is NULL", who);
+#define APT_GAT_AS(T, OUT) \
+  gat_block_as<T, OUT>(neighbors, num_dst, num_dst_dev, fanout, ft, num_src, heads, dim, el, er, slope, out, attn_out, bias, st)
+  if (elem_size == 4) APT_GAT_AS(float, float);
+  else if (like_input) APT_GAT_AS(uint16_t, uint16_t);
+  else APT_GAT_AS(uint16_t, float);
+#undef APT_GAT_AS
+  APT_LAUNCH_CHECK("gat_ell_kernel");
+  return APT_OK;
+}
+}  // namespace apt
+
 extern "C" int apt_gat_block(const int64_t* neighbors, int64_t num_dst, const int64_t* num_dst_dev, int fanout,
                              const void* ft, int64_t num_src, int heads, int64_t dim, int elem_size,
                              const float* el, const float* er, float negative_slope, float* out,
                              float* attn_out, void* stream) {
-  using namespace apt;
-  APT_REQUIRE(num_dst >= 0 && fanout > 0 && heads > 0 && dim > 0 && num_src >= 0, APT_EINVAL,
-              "apt_gat_block: bad shape (num_dst %lld, fanout %d, heads %d, dim %lld)", (long long)num_dst,
-              fanout, heads, (long long)dim);
-  APT_REQUIRE(elem_size == 2 || elem_size == 4, APT_EINVAL, "apt_gat_block: elem_size %d (4 = fp32, 2 = bf16)",
-              elem_size);
-  if (num_dst == 0) return APT_OK;
-  APT_REQUIRE(neighbors != nullptr && out != nullptr && er != nullptr &&
-                  ((ft != nullptr && el != nullptr) || num_src == 0),
-              APT_EINVAL, "apt_gat_block: a tensor is NULL");
-  hipStream_t st = static_cast<hipStream_t>(stream);
-  const bool vec4 = dim % 4 == 0 && (reinterpret_cast<uintptr_t>(ft) & 15) == 0 &&
-                    (reinterpret_cast<uintptr_t>(out) & 15) == 0;
-  if (vec4 && num_src > 0 &&
-      (elem_size == 4 ? launch_gat_wave<float, 4>(neighbors, num_dst, num_dst_dev, fanout, ft, num_src, heads, dim, el,
-                                                  er, negative_slope, out, attn_out, st)
-                      : launch_gat_wave<uint16_t, 4>(neighbors, num_dst, num_dst_dev, fanout, ft, num_src, heads, dim,
-                                                     el, er, negative_slope, out, attn_out, st))) {
-    APT_LAUNCH_CHECK("gat_ell_wave_kernel");
-    return APT_OK;
-  }
-  if (elem_size == 4) {
-    if (vec4) launch_gat<float, 4>(neighbors, num_dst, num_dst_dev, fanout, ft, num_src, heads, dim, el, er, negative_slope, out, attn_out, st);
-    else launch_gat<float, 1>(neighbors, num_dst, num_dst_dev, fanout, ft, num_src, heads, dim, el, er, negative_slope, out, attn_out, st);
-  } else {
-    if (vec4 && dim % 8 == 0) launch_gat<uint16_t, 8>(neighbors, num_dst, num_dst_dev, fanout, ft, num_src, heads, dim, el, er, negative_slope, out, attn_out, st);
-    else if (vec4) launch_gat<uint16_t, 4>(neighbors, num_dst, num_dst_dev, fanout, ft, num_src, heads, dim, el, er, negative_slope, out, attn_out, st);
-    else launch_gat<uint16_t, 1>(neighbors, num_dst, num_dst_dev, fanout, ft, num_src, heads, dim, el, er, negative_slope, out, attn_out, st);
-  }
-  APT_LAUNCH_CHECK("gat_ell_kernel");
-  return APT_OK;
+  return apt::gat_block("apt_gat_block", neighbors, num_dst, num_dst_dev, fanout, ft, num_src, heads, dim, elem_size, el, er,
+                        negative_slope, out, false, attn_out, nullptr, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int apt_spmm_heads(const int64_t* coo_row, const int64_t* coo_col, int64_t num_edges,
@@ -1122,55 +1160,61 @@ extern "C" int apt_spmm_heads(const int64_t* coo_row, const int64_t* coo_col, in
   return APT_OK;
 }
 
+namespace apt {
+template <typename T, typename DT>
+static void gat_edge_grad_as(const int64_t* neighbors, int64_t num_dst, int fanout, const void* ft, int64_t num_src, int heads,
+                             int64_t dim, const float* el, const float* er, float slope, const float* attn, const void* d_out,
+                             const int64_t* csc_indptr, float* a_edge, float* dz_edge, float* d_er, hipStream_t st) {
+  if (launch_gat_bwd_wave<T, DT, 4>(neighbors, num_dst, fanout, ft, num_src, heads, dim, el, er, slope, attn, d_out,
+                                    csc_indptr, a_edge, dz_edge, d_er, st))
+    return;
+  if constexpr (sizeof(T) == 2) {
+    if (launch_gat_bwd_group<T, DT, 8>(neighbors, num_dst, fanout, ft, num_src, heads, dim, el, er, slope, attn, d_out,
+                                       csc_indptr, a_edge, dz_edge, d_er, st))
+      return;
+  }
+  if (launch_gat_bwd_group<T, DT, 4>(neighbors, num_dst, fanout, ft, num_src, heads, dim, el, er, slope, attn, d_out,
+                                     csc_indptr, a_edge, dz_edge, d_er, st))
+    return;
+  const unsigned blocks = static_cast<unsigned>(std::min<int64_t>(ceil_div(num_dst * heads, kAggWaves), 1 << 20));
+  hipLaunchKernelGGL((gat_bwd_edge_kernel<T, DT>), dim3(blocks), dim3(kAggBlock), 0, st, neighbors, num_dst, fanout,
+                     static_cast<const T*>(ft), num_src, heads, dim, el, er, slope, attn, static_cast<const DT*>(d_out),
+                     csc_indptr, a_edge, dz_edge, d_er);
+}
+
+// The edge half of the GAT gradient; d_out fp32, or (like_input) of the input's type.  csc_indptr NULL: slot order.
+// Shared with the GAT layer (gat_layer.hip).
+int gat_edge_grad(const char* who, const int64_t* neighbors, int64_t num_dst, int fanout, const void* ft, int64_t num_src,
+                  int heads, int64_t dim, int elem_size, const float* el, const float* er, float slope, const float* attn,
+                  const void* d_out, bool like_input, const int64_t* csc_indptr, float* a_edge, float* dz_edge, float* d_er,
+                  hipStream_t st) {
+  APT_REQUIRE(num_dst >= 0 && fanout > 0 && fanout <= kWave && heads > 0 && dim > 0 && num_src >= 0, APT_EINVAL,
+              "%s: bad shape (num_dst %lld, fanout %d (1..64), heads %d, dim %lld)", who, (long long)num_dst, fanout, heads,
+              (long long)dim);
+  APT_REQUIRE(elem_size == 2 || elem_size == 4, APT_EINVAL, "%s: elem_size %d (4 = fp32, 2 = bf16)", who, elem_size);
+  if (num_dst == 0) return APT_OK;
+  APT_REQUIRE(neighbors != nullptr && ft != nullptr && el != nullptr && er != nullptr && attn != nullptr && d_out != nullptr &&
+                  (csc_indptr == nullptr || a_edge != nullptr) && dz_edge != nullptr && d_er != nullptr,
+              APT_EINVAL, "%s: a tensor is NULL", who);
+#define APT_EDGE_GRAD(T, DT)                                                                                         \
+  gat_edge_grad_as<T, DT>(neighbors, num_dst, fanout, ft, num_src, heads, dim, el, er, slope, attn, d_out, csc_indptr, \
+                          a_edge, dz_edge, d_er, st)
+  if (elem_size == 4) APT_EDGE_GRAD(float, float);
+  else if (like_input) APT_EDGE_GRAD(uint16_t, uint16_t);
+  else APT_EDGE_GRAD(uint16_t, float);
+#undef APT_EDGE_GRAD
+  APT_LAUNCH_CHECK("gat_bwd_edge_kernel");
+  return APT_OK;
+}
+}  // namespace apt
+
 extern "C" int apt_gat_block_backward(const int64_t* neighbors, int64_t num_dst, int fanout, const void* ft,
                                       int64_t num_src, int heads, int64_t dim, int elem_size, const float* el,
                                       const float* er, float negative_slope, const float* attn,
                                       const float* d_out, const int64_t* csc_indptr, float* a_edge,
                                       float* dz_edge, float* d_er, void* stream) {
-  using namespace apt;
-  APT_REQUIRE(num_dst >= 0 && fanout > 0 && fanout <= kWave && heads > 0 && dim > 0 && num_src >= 0, APT_EINVAL,
-              "apt_gat_block_backward: bad shape (num_dst %lld, fanout %d (1..64), heads %d, dim %lld)",
-              (long long)num_dst, fanout, heads, (long long)dim);
-  APT_REQUIRE(elem_size == 2 || elem_size == 4, APT_EINVAL,
-              "apt_gat_block_backward: elem_size %d (4 = fp32, 2 = bf16)", elem_size);
-  if (num_dst == 0) return APT_OK;
-  APT_REQUIRE(neighbors != nullptr && ft != nullptr && el != nullptr && er != nullptr && attn != nullptr &&
-                  d_out != nullptr && csc_indptr != nullptr && a_edge != nullptr && dz_edge != nullptr &&
-                  d_er != nullptr,
-              APT_EINVAL, "apt_gat_block_backward: a tensor is NULL");
-  const unsigned blocks =
-      static_cast<unsigned>(std::min<int64_t>(ceil_div(num_dst * heads, kAggWaves), 1 << 20));
-  hipStream_t st = static_cast<hipStream_t>(stream);
-  const bool by_wave =
-      elem_size == 4 ? launch_gat_bwd_wave<float, 4>(neighbors, num_dst, fanout, ft, num_src, heads, dim, el, er,
-                                                     negative_slope, attn, d_out, csc_indptr, a_edge, dz_edge, d_er, st)
-                     : launch_gat_bwd_wave<uint16_t, 4>(neighbors, num_dst, fanout, ft, num_src, heads, dim, el, er,
-                                                        negative_slope, attn, d_out, csc_indptr, a_edge, dz_edge, d_er,
-                                                        st);
-  if (by_wave) {
-    APT_LAUNCH_CHECK("gat_bwd_edge_wave_kernel");
-    return APT_OK;
-  }
-  const bool grouped =
-      elem_size == 4
-          ? launch_gat_bwd_group<float, 4>(neighbors, num_dst, fanout, ft, num_src, heads, dim, el, er,
-                                           negative_slope, attn, d_out, csc_indptr, a_edge, dz_edge, d_er, st)
-          : (launch_gat_bwd_group<uint16_t, 8>(neighbors, num_dst, fanout, ft, num_src, heads, dim, el, er,
-                                               negative_slope, attn, d_out, csc_indptr, a_edge, dz_edge, d_er, st) ||
-             launch_gat_bwd_group<uint16_t, 4>(neighbors, num_dst, fanout, ft, num_src, heads, dim, el, er,
-                                               negative_slope, attn, d_out, csc_indptr, a_edge, dz_edge, d_er, st));
-  if (grouped) {
-    APT_LAUNCH_CHECK("gat_bwd_edge_group_kernel");
-    return APT_OK;
-  }
-  if (elem_size == 4)
-    hipLaunchKernelGGL(gat_bwd_edge_kernel<float>, dim3(blocks), dim3(kAggBlock), 0, st, neighbors, num_dst,
-                       fanout, static_cast<const float*>(ft), num_src, heads, dim, el, er, negative_slope, attn,
-                       d_out, csc_indptr, a_edge, dz_edge, d_er);
-  else
-    hipLaunchKernelGGL(gat_bwd_edge_kernel<uint16_t>, dim3(blocks), dim3(kAggBlock), 0, st, neighbors, num_dst,
-                       fanout, static_cast<const uint16_t*>(ft), num_src, heads, dim, el, er, negative_slope, attn,
-                       d_out, csc_indptr, a_edge, dz_edge, d_er);
-  APT_LAUNCH_CHECK("gat_bwd_edge_kernel");
-  return APT_OK;
+  APT_REQUIRE(csc_indptr != nullptr || num_dst <= 0, APT_EINVAL, "apt_gat_block_backward: a tensor is NULL");
+  return apt::gat_edge_grad("apt_gat_block_backward", neighbors, num_dst, fanout, ft, num_src, heads, dim, elem_size, el, er,
+                            negative_slope, attn, d_out, false, csc_indptr, a_edge, dz_edge, d_er,
+                            static_cast<hipStream_t>(stream));
 }

@@ -1090,6 +1090,124 @@ Tensor BlockAggregate(const Tensor& relabeled, int64_t num_dst, int64_t fanout, 
   return BlockAggregateFn::apply(x.contiguous(), relabeled, num_dst, fanout, mean, csr_indptr, csr_indices);
 }
 
+// ---------------------------------------------------------------- GAT layer, from the dense product to the bias
+namespace {
+
+struct GatLayerFn : public torch::autograd::Function<GatLayerFn> {
+  static Tensor forward(torch::autograd::AutogradContext* ctx, const Tensor& ft, const Tensor& attn_l, const Tensor& attn_r,
+                        const std::optional<Tensor>& bias, const Tensor& relabeled, int64_t num_dst, int64_t fanout,
+                        double slope, bool want_grad, const std::optional<Tensor>& csr_indptr,
+                        const std::optional<Tensor>& csr_indices, const std::optional<Tensor>& csr_eids,
+                        const std::optional<Tensor>& csc_indptr) {
+    const int64_t n = ft.size(0), heads = ft.size(1), dim = ft.size(2);
+    const auto f32 = ft.options().dtype(torch::kFloat32);
+    auto scores = torch::empty({(n + num_dst) * heads}, f32);   // el, then er
+    float* el = scores.data_ptr<float>();
+    float* er = el + n * heads;
+    auto out = torch::empty({num_dst, heads, dim}, ft.options());
+    Tensor attn;
+    if (want_grad) attn = torch::empty({num_dst * fanout, heads}, f32);
+    Tensor b = bias.has_value() ? bias->contiguous() : Tensor();
+    check(apt_gat_layer(i64(relabeled), num_dst, static_cast<int>(fanout), ft.data_ptr(), n, static_cast<int>(heads), dim,
+                        static_cast<int>(ft.element_size()), attn_l.data_ptr(), attn_r.data_ptr(),
+                        static_cast<int>(attn_l.element_size()), b.defined() ? b.data_ptr() : nullptr,
+                        static_cast<float>(slope), el, er, out.data_ptr(), want_grad ? attn.data_ptr<float>() : nullptr,
+                        stream()));
+    if (want_grad) {
+      const bool csr = csr_indptr.has_value() && csr_indices.has_value() && csr_eids.has_value() && csc_indptr.has_value() &&
+                       csr_indptr->numel() == n + 1;
+      ctx->save_for_backward({ft, attn_l, attn_r, relabeled, scores, attn, csr ? *csr_indptr : Tensor(),
+                              csr ? *csr_indices : Tensor(), csr ? *csr_eids : Tensor(), csr ? *csc_indptr : Tensor()});
+      ctx->saved_data["num_dst"] = num_dst;
+      ctx->saved_data["fanout"] = fanout;
+      ctx->saved_data["slope"] = slope;
+      ctx->saved_data["bias"] = bias.has_value();
+    }
+    return out;
+  }
+  static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx,
+                                                 torch::autograd::variable_list grads) {
+    const auto saved = ctx->get_saved_variables();
+    const Tensor &ft = saved[0], &attn_l = saved[1], &attn_r = saved[2], &relabeled = saved[3], &scores = saved[4],
+                 &attn = saved[5];
+    const int64_t num_dst = ctx->saved_data["num_dst"].toInt(), fanout = ctx->saved_data["fanout"].toInt();
+    const int64_t n = ft.size(0), heads = ft.size(1), dim = ft.size(2);
+    const bool bias = ctx->saved_data["bias"].toBool();
+    auto d_out = grads[0].contiguous();
+    SourceOrder o;
+    Tensor eids, csc;
+    int64_t edges = 0;
+    if (saved[6].defined()) {
+      o.indptr = saved[6];
+      o.index = saved[7];
+      o.bytes = 8;
+      eids = saved[8];
+      csc = saved[9];
+      edges = eids.numel();
+    } else if (apt_block_transpose_workspace_bytes(num_dst, static_cast<int>(fanout), n) > 0) {
+      o = source_order(relabeled, num_dst, fanout, n);
+    } else {
+      auto f = BlockFormats(relabeled, num_dst, fanout, n, true);
+      csc = f[2];
+      o.indptr = f[3];
+      o.index = f[4];
+      o.bytes = 8;
+      eids = f[5];
+      edges = eids.numel();
+    }
+    auto d_ft = torch::empty_like(ft), d_al = torch::empty_like(attn_l), d_ar = torch::empty_like(attn_r);
+    Tensor d_bias;
+    if (bias) d_bias = torch::empty({heads, dim}, ft.options());
+    const size_t need = apt_gat_layer_backward_workspace_bytes(num_dst, static_cast<int>(fanout), n, static_cast<int>(heads),
+                                                               dim, edges);
+    auto ws = torch::empty({static_cast<int64_t>(need)}, ft.options().dtype(torch::kUInt8));
+    const float* el = scores.data_ptr<float>();
+    check(apt_gat_layer_backward(i64(relabeled), num_dst, static_cast<int>(fanout), ft.data_ptr(), n,
+                                 static_cast<int>(heads), dim, static_cast<int>(ft.element_size()), attn_l.data_ptr(),
+                                 attn_r.data_ptr(), static_cast<int>(attn_l.element_size()),
+                                 static_cast<float>(ctx->saved_data["slope"].toDouble()), el, el + n * heads,
+                                 attn.data_ptr<float>(), d_out.data_ptr(), o.indptr.data_ptr(), o.index.data_ptr(), o.bytes,
+                                 o.bytes == 8 ? i64(eids) : nullptr, o.bytes == 8 ? i64(csc) : nullptr, edges,
+                                 d_ft.data_ptr(), d_al.data_ptr(), d_ar.data_ptr(), bias ? d_bias.data_ptr() : nullptr,
+                                 ws.data_ptr(), need, stream()));
+    torch::autograd::variable_list out(13);
+    out[0] = d_ft;
+    out[1] = d_al;
+    out[2] = d_ar;
+    if (bias) out[3] = d_bias;
+    return out;
+  }
+};
+
+}  // namespace
+
+// ft [num_src, heads, dim] -> [num_dst, heads, dim] (apt_gat_layer), with its gradients.  attn_l, attn_r [heads, dim]
+// fp32 or bf16, bias [heads, dim] (or any shape of that many elements) of ft's type.
+Tensor GatLayer(const Tensor& relabeled, int64_t num_dst, int64_t fanout, const Tensor& ft, const Tensor& attn_l,
+                const Tensor& attn_r, const std::optional<Tensor>& bias, double slope,
+                const std::optional<Tensor>& csr_indptr, const std::optional<Tensor>& csr_indices,
+                const std::optional<Tensor>& csr_eids, const std::optional<Tensor>& csc_indptr) {
+  check_block("gat_layer", relabeled, num_dst, fanout);
+  const auto good = [](const Tensor& t) {
+    return t.is_cuda() && (t.scalar_type() == torch::kFloat32 || t.scalar_type() == torch::kBFloat16);
+  };
+  TORCH_CHECK_TYPE(good(ft) && ft.dim() == 3, "npc: gat_layer: ft must be a [num_src, heads, dim] fp32 or bf16 GPU tensor");
+  TORCH_CHECK_TYPE(good(attn_l) && attn_r.scalar_type() == attn_l.scalar_type() && attn_r.is_cuda(),
+                   "npc: gat_layer: attn_l and attn_r must be fp32 or bf16 GPU tensors of one type");
+  TORCH_CHECK(attn_l.numel() == ft.size(1) * ft.size(2) && attn_r.numel() == attn_l.numel() && num_dst <= ft.size(0),
+              "npc: gat_layer: attn_l / attn_r must be [heads, dim], num_dst at most num_src");
+  std::optional<Tensor> b = bias;
+  if (b.has_value()) {
+    TORCH_CHECK(b->is_cuda() && b->scalar_type() == ft.scalar_type() && b->numel() == ft.size(1) * ft.size(2),
+                "npc: gat_layer: bias must have heads * dim elements of ft's type");
+    b = b->reshape({ft.size(1), ft.size(2)});
+  }
+  const bool want_grad = torch::GradMode::is_enabled() && (ft.requires_grad() || attn_l.requires_grad() || attn_r.requires_grad() ||
+                                                          (b.has_value() && b->requires_grad()));
+  return GatLayerFn::apply(ft.contiguous(), attn_l.contiguous(), attn_r.contiguous(), b, relabeled, num_dst, fanout, slope,
+                           want_grad, csr_indptr, csr_indices, csr_eids, csc_indptr);
+}
+
 // ---------------------------------------------------------------- peers only
 #define NPC_NEEDS_PEERS(name)                                                              \
   TORCH_CHECK(false, "npc." name " talks to other GPUs over NCCL in the reference; this " \
@@ -1146,6 +1264,7 @@ TORCH_LIBRARY(npc, m) {
       .def("block_formats", &BlockFormats)
       .def("block_linear", &BlockLinear)
       .def("block_aggregate", &BlockAggregate)
+      .def("gat_layer", &GatLayer)
       .def("cluster_and_permute", &ClusterAndPermuteLocal)
       .def("register_graph_partition", &RegisterGraphPartition)
       .def("set_topology", &SetTopology)

@@ -810,6 +810,35 @@ int apt_block_aggregate_backward(const void* indptr, const void* index, int inde
                                  int64_t num_src, const float* dst_scale, const void* dz,
                                  int64_t num_dst, int64_t dim, int elem_size, void* dx, void* stream);
 
+/* A GAT layer between its dense product and its activation (python/npc/model/
+ * gatconv.py:116-126,207-236), forward and backward.  ft, out, d_out, d_ft and the
+ * bias are of one type (elem_size 4 = fp32, 2 = bf16), attn_l / attn_r and their
+ * gradients of another (attn_elem_size); all sums are fp32, in a fixed order.
+ * num_dst <= num_src: the first num_dst sources are the destinations.
+ *   apt_gat_layer           el = (ft * attn_l).sum(-1) [num_src, heads], er likewise on
+ *                           the first num_dst rows, then apt_gat_block and + bias
+ *                           ([heads, dim], may be NULL): out [num_dst, heads, dim];
+ *                           attn_out [num_dst * fanout, heads], optional, as there
+ *   apt_gat_layer_backward  fanout <= 64; every row of d_ft [num_src, heads, dim] is
+ *                           written; d_attn_l, d_attn_r, d_bias [heads, dim] may be
+ *                           NULL.  The edges by source: index_bytes 4 = indptr / slots
+ *                           of apt_block_transpose (eids, csc_indptr NULL, num_edges
+ *                           0), 8 = csr_indptr / csr_indices with csr_eids, csc_indptr
+ *                           and the edge count of apt_block_formats. */
+int apt_gat_layer(const int64_t* neighbors, int64_t num_dst, int fanout, const void* ft, int64_t num_src,
+                  int heads, int64_t dim, int elem_size, const void* attn_l, const void* attn_r,
+                  int attn_elem_size, const void* bias, float negative_slope, float* el, float* er, void* out,
+                  float* attn_out, void* stream);
+size_t apt_gat_layer_backward_workspace_bytes(int64_t num_dst, int fanout, int64_t num_src, int heads, int64_t dim,
+                                              int64_t num_edges);
+int apt_gat_layer_backward(const int64_t* neighbors, int64_t num_dst, int fanout, const void* ft,
+                           int64_t num_src, int heads, int64_t dim, int elem_size, const void* attn_l,
+                           const void* attn_r, int attn_elem_size, float negative_slope, const float* el,
+                           const float* er, const float* attn, const void* d_out, const void* indptr,
+                           const void* index, int index_bytes, const int64_t* eids, const int64_t* csc_indptr,
+                           int64_t num_edges, void* d_ft, void* d_attn_l, void* d_attn_r, void* d_bias,
+                           void* workspace, size_t workspace_bytes, void* stream);
+
 /* Gradients of a dense layer y = x w^T + b over a block's rows (the fc_self /
  * fc_neigh / fc of python/npc/model/sageconv.py:118-188 and gatconv.py:207-236,
  * whose gradients the reference gets from cuBLAS through torch):

@@ -1,0 +1,64 @@
+"""The fused GAT layer (scores, edge softmax, weighted sum, bias, and all gradients) against the separate operations in
+torch, sums over edges in float64 (bf16 rows: the operations between them in bf16, as a bf16 model has them): heads and widths on every path (a wavefront per destination, lane groups, features that cross a head's
+edge inside a vector), hubs, destinations without edges, both edge orders."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _separate(rel, num_dst, fanout, ft_row, al, ar, bias, slope):
+    el_row, er_row = (ft_row * al).sum(-1), (ft_row[:num_dst] * ar).sum(-1)
+    ft, el, er = ft_row.double(), el_row.double(), er_row.double()
+    keep = (rel >= 0).nonzero().flatten()
+    src, dst = rel[keep], keep // fanout
+    heads, dim = ft.shape[1:]
+    e = torch.nn.functional.leaky_relu(el[src] + er[dst], slope)
+    top = torch.full((num_dst, heads), -1e30, device=DEV, dtype=ft.dtype).scatter_reduce(0, dst[:, None].expand(-1, heads), e.detach(), "amax")
+    w = torch.exp(e - top[dst])
+    den = torch.zeros(num_dst, heads, device=DEV, dtype=ft.dtype).index_add(0, dst, w)
+    out = torch.zeros(num_dst, heads, dim, device=DEV, dtype=ft.dtype).index_add(0, dst, (w / den[dst])[:, :, None] * ft[src])
+    return out.to(ft_row.dtype) + bias
+
+
+@pytest.mark.parametrize("dtype,attn_dtype", [(torch.float32, torch.float32), (torch.bfloat16, torch.bfloat16),
+                                              (torch.bfloat16, torch.float32)])
+@pytest.mark.parametrize("num_dst,fanout,num_src,heads,dim", [
+    (300, 15, 2500, 4, 64), (300, 10, 2500, 4, 47), (200, 7, 900, 3, 8), (150, 9, 700, 1, 5), (150, 9, 700, 8, 8),
+    (100, 25, 800, 2, 100), (100, 20, 800, 8, 64), (64, 64, 500, 1, 256), (1, 1, 1, 1, 1), (90, 5, 400, 4, 6), (80, 5, 300, 5, 3)])
+@pytest.mark.parametrize("with_csr", [False, True])
+def test_gat_layer(capi, num_dst, fanout, num_src, heads, dim, dtype, attn_dtype, with_csr):
+    import apt_amd  # noqa: F401
+    rng = np.random.default_rng(num_dst + dim)
+    r = rng.integers(0, num_src, size=num_dst * fanout)
+    if r.size > 800:
+        r[rng.choice(r.size, 300, replace=False)] = min(3, num_src - 1)         # a hub
+    r[rng.random(r.size) < 0.2] = -1
+    r[:fanout] = -1 if num_dst > 1 else 0                                       # a destination without edges
+    rel = torch.from_numpy(r.astype(np.int64)).to(DEV)
+    gen = torch.Generator(device=DEV).manual_seed(heads * dim)
+    rand = lambda *s: torch.randn(*s, generator=gen, device=DEV)
+    ft = rand(num_src, heads, dim).to(dtype).requires_grad_(True)
+    al, ar = (rand(heads, dim) * 0.3).to(attn_dtype).requires_grad_(True), (rand(heads, dim) * 0.3).to(attn_dtype).requires_grad_(True)
+    bias = rand(heads * dim).to(dtype).requires_grad_(True)
+    up = rand(num_dst, heads, dim).to(dtype)
+    f = capi.block_formats(rel, num_dst, fanout, num_src) if with_csr else {}
+    csr = [f.get(k) for k in ("csr_indptr", "csr_indices", "csr_eids", "csc_indptr")]
+    out = torch.ops.npc.gat_layer(rel, num_dst, fanout, ft, al, ar, bias, 0.2, *csr)
+    got = torch.autograd.grad(out, [ft, al, ar, bias], up)
+    wide = torch.float64 if dtype == torch.float32 else None      # fp32: everything in float64
+    leaves = [(t.detach() if wide is None else t.detach().to(wide)).requires_grad_(True) for t in (ft, al, ar, bias.view(heads, dim))]
+    ref = _separate(rel, num_dst, fanout, *leaves, 0.2)
+    want = torch.autograd.grad(ref, leaves, up.to(ref.dtype))
+    # fp32: sums of a few thousand products.  bf16: an fp32 sum next to a rounding boundary may round the other way in
+    # another order, 2^-8 of that value; the attention vectors' gradients are sums of terms that cancel, so there
+    # it weighs more.
+    for a, b, name in zip((out,) + got, (ref,) + want, ("out", "ft", "attn_l", "attn_r", "bias")):
+        assert a.dtype == (attn_dtype if name.startswith("attn") else dtype)
+        tol = 1e-4 if dtype == torch.float32 else 3e-2 if name.startswith("attn") else 1e-2
+        err = (a.double().reshape(-1) - b.double().reshape(-1)).abs().max().item()
+        assert err <= tol * (b.abs().max().item() + 1e-2), (name, err, b.abs().max().item())
+    with torch.no_grad():
+        assert torch.equal(torch.ops.npc.gat_layer(rel, num_dst, fanout, ft, al, ar, bias, 0.2, *csr), out)
