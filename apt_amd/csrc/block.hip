@@ -957,16 +957,16 @@ struct FmtLayout {
 };
 
 // The last piece's ranges are as narrow as their number allows.  num_src itself has a range: the last offset.
-static void choose_ranges(int64_t num_dst, int64_t num_src, FmtLayout& L) {
+static void choose_ranges(int64_t num_dst, int64_t num_src, bool records_hold_dst, FmtLayout& L) {
   L.range_shift2 = kRangeShift2;
   while (L.range_shift2 < kRangeMaxShift && range_index(num_src, L.range_shift2) >= kRangeMaxCount) ++L.range_shift2;
   const int64_t ranges = range_index(num_src, L.range_shift2) + 1;
-  const bool fits = ranges <= kRangeMaxCount && L.ctiles <= kRangeMaxTiles && num_dst <= kRangeMaxDst &&
-                    tuning_block_fused_scan();
+  const bool fits = ranges <= kRangeMaxCount && L.ctiles <= kRangeMaxTiles &&
+                    (!records_hold_dst || num_dst <= kRangeMaxDst) && tuning_block_fused_scan();
   L.ranges = fits ? static_cast<int>(ranges) : 0;
 }
 
-static FmtLayout fmt_layout(int64_t num_dst, int fanout, int64_t num_src, bool csr) {
+static FmtLayout fmt_layout(int64_t num_dst, int fanout, int64_t num_src, bool csr, bool transpose = false) {
   FmtLayout L;
   L.ranges = 0;
   L.slots = num_dst * fanout;
@@ -976,7 +976,7 @@ static FmtLayout fmt_layout(int64_t num_dst, int fanout, int64_t num_src, bool c
   L.tile_cnt_off = off; off = fmt_align(off + sizeof(uint32_t) * static_cast<size_t>(L.ctiles));
   L.sums_off = off;     off = fmt_align(off + sizeof(uint32_t) * kScanChunk);
   L.hist_off = off;
-  if (csr) choose_ranges(num_dst, num_src, L);
+  if (csr) choose_ranges(num_dst, num_src, !transpose, L);
   if (csr && L.ranges > 0) {
     off = fmt_align(off + sizeof(uint32_t) * static_cast<size_t>(L.ctiles) * L.ranges);
     L.bin_total_off = off; off = fmt_align(off + sizeof(uint32_t) * L.ranges);
@@ -1033,7 +1033,7 @@ static int launch_ranges(const CompactParams& c, RangeParams& r, const FmtLayout
 extern "C" size_t apt_block_transpose_workspace_bytes(int64_t num_dst, int fanout, int64_t num_src) {
   using namespace apt;
   if (!fmt_sizes_ok(num_dst, fanout, num_src)) return 0;
-  const FmtLayout L = fmt_layout(num_dst, fanout, num_src, true);
+  const FmtLayout L = fmt_layout(num_dst, fanout, num_src, true, true);
   return L.ranges > 0 ? L.total : 0;
 }
 
@@ -1044,7 +1044,7 @@ extern "C" int apt_block_transpose(const int64_t* relabeled, int64_t num_dst, in
   APT_REQUIRE(fmt_sizes_ok(num_dst, fanout, num_src), APT_ELIMIT,
               "apt_block_transpose: sizes out of range (num_dst %lld, fanout %d, num_src %lld)",
               static_cast<long long>(num_dst), fanout, static_cast<long long>(num_src));
-  const FmtLayout L = fmt_layout(num_dst, fanout, num_src, true);
+  const FmtLayout L = fmt_layout(num_dst, fanout, num_src, true, true);
   APT_REQUIRE(L.ranges > 0, APT_ELIMIT, "apt_block_transpose: block too large (see apt_block_transpose_workspace_bytes)");
   APT_REQUIRE(indptr != nullptr && (L.slots == 0 || (relabeled != nullptr && slots != nullptr)), APT_EINVAL,
               "apt_block_transpose: an argument is NULL");

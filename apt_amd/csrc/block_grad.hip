@@ -1,5 +1,6 @@
-// Source side of a block's aggregation: dx[s, :] = sum over the edges s -> d of w(e) * dz[d, :], the gradient of the
-// block sum / mean (and, weighted per edge and head, of the GAT aggregation) towards its input.
+// Sums over grouped edges: dx[s, :] = sum over the edges e of s of w(e) * dz[d(e), :].  With the edges of a sampled
+// block grouped by source this is the gradient of the block sum / mean towards its input; with the edges of a COO
+// grouped by destination it is the COO sum (apt_coo_sum).  "Source" below is the row that is written.
 //
 // A lane group owns a source row, so every row is written once, in its own type, whole and in a fixed order: no
 // zero-fill, no atomics, no fp32 copy of a bf16 result.  Nearly all sources of a sampled block have one or two edges;
@@ -19,8 +20,10 @@ constexpr int kSourceBlocks = 2048;
 
 struct SourceSumParams {
   const void* indptr;      // offsets of the sources in `index`
-  const void* index;       // per edge: its destination, or its slot (fanout > 0: destination = slot / fanout)
-  uint32_t fanout;
+  const void* index;       // per edge: its destination (int64_t), or its slot (uint32_t; NULL: edge e is slot e)
+  uint32_t fanout;         // slots: the destination is slot / fanout ...
+  const int64_t* via;      // ... or, if given, via[slot]
+  const void* edata;       // slots, optional: [slots, dim] of dz's type, multiplies the destination's row
   const float* dst_scale;  // per destination, or NULL
   const void* dz;          // [num_dst, dim]
   int64_t num_dst;
@@ -30,7 +33,7 @@ struct SourceSumParams {
 };
 
 // I: int64_t = a block's CSR (offsets, destinations), uint32_t = apt_block_transpose (offsets, slots).
-template <typename T, int VEC, int LPR, typename I>
+template <typename T, int VEC, int LPR, typename I, bool EDATA>
 __global__ __launch_bounds__(kAggBlock) void source_sum_kernel(SourceSumParams p) {
   constexpr int kGroups = kAggBlock / LPR;
   constexpr int kRows = 2;
@@ -45,12 +48,28 @@ __global__ __launch_bounds__(kAggBlock) void source_sum_kernel(SourceSumParams p
   T* dx = static_cast<T*>(p.dx);
   if (threadIdx.x == 0) s_hubs = 0;
   __syncthreads();
-  auto destination = [&](I i) -> int64_t {
-    const int64_t d = sizeof(I) == 4 ? static_cast<int64_t>(static_cast<uint32_t>(i) / p.fanout) : static_cast<int64_t>(i);
-    return d >= 0 && d < p.num_dst ? d : -1;
+  struct Edge {      // lane j of a group: edge j of the row
+    int64_t dst;     // -1: none
+    uint32_t slot;   // EDATA only
+    float scale;
   };
-  // acc += the rows of up to LPR edges whose destinations the group's lanes hold (lane j: edge j)
-  auto add_edges = [&](int64_t my_dst, float my_scale, int n, int64_t c, bool live, float (&acc)[VEC]) {
+  auto slot_of = [&](int64_t at) { return index != nullptr ? index[at] : static_cast<I>(at); };
+  auto edge = [&](int64_t at, bool mine) {
+    Edge e{-1, 0u, 1.f};
+    if (!mine) return e;
+    if constexpr (sizeof(I) == 8) {
+      e.dst = static_cast<int64_t>(index[at]);
+    } else {
+      e.slot = static_cast<uint32_t>(slot_of(at));
+      e.dst = p.via != nullptr ? p.via[e.slot] : static_cast<int64_t>(e.slot / p.fanout);
+    }
+    if (e.dst < 0 || e.dst >= p.num_dst) e.dst = -1;
+    if (p.dst_scale != nullptr && e.dst >= 0) e.scale = p.dst_scale[e.dst];
+    return e;
+  };
+  const T* edata = static_cast<const T*>(p.edata);
+  // acc += the rows of up to LPR edges that the group's lanes hold
+  auto add_edges = [&](const Edge& my, int n, int64_t c, bool live, float (&acc)[VEC]) {
     for (int e0 = 0; e0 < n; e0 += kUnroll) {
       float v[kUnroll][VEC];
       float w[kUnroll];
@@ -60,9 +79,18 @@ __global__ __launch_bounds__(kAggBlock) void source_sum_kernel(SourceSumParams p
         for (int k = 0; k < VEC; ++k) v[u][k] = 0.f;
         w[u] = 0.f;
         if (e0 + u < n) {
-          const int64_t d = __shfl(my_dst, e0 + u, LPR);
-          w[u] = __shfl(my_scale, e0 + u, LPR);
-          if (d >= 0 && live) load_vec<T, VEC>(dz, d * p.dim + c, v[u]);
+          const int64_t d = __shfl(my.dst, e0 + u, LPR);
+          w[u] = __shfl(my.scale, e0 + u, LPR);
+          const uint32_t slot = EDATA ? __shfl(my.slot, e0 + u, LPR) : 0u;
+          if (d >= 0 && live) {
+            load_vec<T, VEC>(dz, d * p.dim + c, v[u]);
+            if constexpr (EDATA) {
+              float m[VEC];
+              load_vec<T, VEC>(edata, static_cast<int64_t>(slot) * p.dim + c, m);
+#pragma unroll
+              for (int k = 0; k < VEC; ++k) v[u][k] *= m[k];
+            }
+          }
         }
       }
 #pragma unroll
@@ -85,12 +113,9 @@ __global__ __launch_bounds__(kAggBlock) void source_sum_kernel(SourceSumParams p
         n[q] = static_cast<int>(static_cast<int64_t>(indptr[r + 1]) - lo[q]);
       }
     }
-    int64_t dst[kRows];
-    float scale[kRows];
+    Edge first[kRows];
 #pragma unroll
-    for (int q = 0; q < kRows; ++q) dst[q] = l < n[q] && n[q] <= kHubEdges ? destination(index[lo[q] + l]) : -1;
-#pragma unroll
-    for (int q = 0; q < kRows; ++q) scale[q] = p.dst_scale != nullptr && dst[q] >= 0 ? p.dst_scale[dst[q]] : 1.f;
+    for (int q = 0; q < kRows; ++q) first[q] = edge(lo[q] + l, l < n[q] && n[q] <= kHubEdges);
     for (int64_t c0 = 0; c0 < p.dim; c0 += LPR * VEC) {
       const int64_t c = c0 + static_cast<int64_t>(l) * VEC;
       const bool live = c < p.dim;
@@ -101,12 +126,9 @@ __global__ __launch_bounds__(kAggBlock) void source_sum_kernel(SourceSumParams p
         float acc[VEC];
 #pragma unroll
         for (int k = 0; k < VEC; ++k) acc[k] = 0.f;
-        add_edges(dst[q], scale[q], min(n[q], LPR), c, live, acc);
-        for (int e = LPR; e < n[q]; e += LPR) {   // LPR < kHubEdges only
-          const int64_t d = e + l < n[q] ? destination(index[lo[q] + e + l]) : -1;
-          const float s = p.dst_scale != nullptr && d >= 0 ? p.dst_scale[d] : 1.f;
-          add_edges(d, s, min(n[q] - e, LPR), c, live, acc);
-        }
+        add_edges(first[q], min(n[q], LPR), c, live, acc);
+        for (int e = LPR; e < n[q]; e += LPR)   // LPR < kHubEdges only
+          add_edges(edge(lo[q] + e + l, e + l < n[q]), min(n[q] - e, LPR), c, live, acc);
         if (live) store_vec<T, VEC>(dx, r * p.dim + c, acc);
       }
     }
@@ -126,9 +148,7 @@ __global__ __launch_bounds__(kAggBlock) void source_sum_kernel(SourceSumParams p
 #pragma unroll
       for (int k = 0; k < VEC; ++k) acc[k] = 0.f;
       for (int64_t e = lo + grp * LPR; e < hi; e += kAggBlock) {
-        const int64_t d = e + l < hi ? destination(index[e + l]) : -1;
-        const float s = p.dst_scale != nullptr && d >= 0 ? p.dst_scale[d] : 1.f;
-        add_edges(d, s, static_cast<int>(min(hi - e, static_cast<int64_t>(LPR))), c, live, acc);
+        add_edges(edge(e + l, e + l < hi), static_cast<int>(min(hi - e, static_cast<int64_t>(LPR))), c, live, acc);
       }
 #pragma unroll
       for (int k = 0; k < VEC; ++k) s_sum[grp][l * VEC + k] = acc[k];
@@ -148,7 +168,7 @@ __global__ __launch_bounds__(kAggBlock) void source_sum_kernel(SourceSumParams p
   }
 }
 
-template <typename T, int VEC, typename I>
+template <typename T, int VEC, typename I, bool EDATA>
 static void launch_source_sum(const SourceSumParams& p, hipStream_t st) {
   const int64_t per_row = ceil_div(p.dim, VEC);
 #define APT_SOURCE_SUM(LPR)                                                                                        \
@@ -156,7 +176,7 @@ static void launch_source_sum(const SourceSumParams& p, hipStream_t st) {
     constexpr int64_t groups = kAggBlock / LPR;                                                                    \
     const int64_t blocks = std::max(ceil_div(p.num_src, kHubList),                                                \
                                     std::min<int64_t>(ceil_div(p.num_src, groups * 2), kSourceBlocks));           \
-    hipLaunchKernelGGL((source_sum_kernel<T, VEC, LPR, I>), dim3(static_cast<unsigned>(blocks)), dim3(kAggBlock), 0, \
+    hipLaunchKernelGGL((source_sum_kernel<T, VEC, LPR, I, EDATA>), dim3(static_cast<unsigned>(blocks)), dim3(kAggBlock), 0, \
                        st, p);                                                                                    \
   } while (0)
   if (per_row <= 8) APT_SOURCE_SUM(8);
@@ -166,22 +186,184 @@ static void launch_source_sum(const SourceSumParams& p, hipStream_t st) {
 #undef APT_SOURCE_SUM
 }
 
-template <typename I>
+template <typename I, bool EDATA>
 static int source_sum(const SourceSumParams& p, int elem_size, hipStream_t st) {
-  const bool aligned = ((reinterpret_cast<uintptr_t>(p.dz) | reinterpret_cast<uintptr_t>(p.dx)) & 15) == 0;
+  const bool aligned = ((reinterpret_cast<uintptr_t>(p.dz) | reinterpret_cast<uintptr_t>(p.dx) |
+                         reinterpret_cast<uintptr_t>(p.edata)) & 15) == 0;
   if (elem_size == 4) {
-    if (aligned && p.dim % 4 == 0) launch_source_sum<float, 4, I>(p, st);
-    else launch_source_sum<float, 1, I>(p, st);
+    if (aligned && p.dim % 4 == 0) launch_source_sum<float, 4, I, EDATA>(p, st);
+    else launch_source_sum<float, 1, I, EDATA>(p, st);
   } else {
-    if (aligned && p.dim % 8 == 0) launch_source_sum<uint16_t, 8, I>(p, st);
-    else if (aligned && p.dim % 4 == 0) launch_source_sum<uint16_t, 4, I>(p, st);
-    else launch_source_sum<uint16_t, 1, I>(p, st);
+    if (aligned && p.dim % 8 == 0) launch_source_sum<uint16_t, 8, I, EDATA>(p, st);
+    else if (aligned && p.dim % 4 == 0) launch_source_sum<uint16_t, 4, I, EDATA>(p, st);
+    else launch_source_sum<uint16_t, 1, I, EDATA>(p, st);
   }
   APT_LAUNCH_CHECK("source_sum_kernel");
   return APT_OK;
 }
 
+// ------------------------------------------------------------------ sums over a COO
+// The edges of a COO by absolute output row (`key`) and input row, whatever segments they come in, and whether the
+// keys are non-decreasing.
+struct CooParams {
+  const int64_t* row;
+  const int64_t* col;
+  int64_t num_edges;
+  const int64_t* coo_off;   // [num_seg + 1]
+  const int64_t* in_off;    // [num_seg] or NULL
+  const int64_t* out_off;   // [num_seg] or NULL
+  int num_seg;
+  int64_t* keys;
+  int64_t* sources;
+  int64_t* grouped;         // 1 on entry
+};
+constexpr int kCooSegments = APT_MAX_BUCKETS + 1;
+
+__global__ void coo_grouped_init_kernel(int64_t* grouped, const int64_t* last_offset, int64_t* num_out) {
+  *grouped = 1;
+  if (num_out != nullptr) *num_out = last_offset != nullptr ? *last_offset : 0;
+}
+
+__global__ __launch_bounds__(kAggBlock) void coo_prepare_kernel(CooParams p) {
+  __shared__ int64_t s_off[kCooSegments + 1], s_in[kCooSegments], s_out[kCooSegments];
+  if (static_cast<int>(threadIdx.x) <= p.num_seg) s_off[threadIdx.x] = p.coo_off[threadIdx.x];
+  if (static_cast<int>(threadIdx.x) < p.num_seg) {
+    s_in[threadIdx.x] = p.in_off != nullptr ? p.in_off[threadIdx.x] : 0;
+    s_out[threadIdx.x] = p.out_off != nullptr ? p.out_off[threadIdx.x] : 0;
+  }
+  __syncthreads();
+  auto segment = [&](int64_t e) {   // last k with coo_off[k] <= e (reference: cub::UpperBound - 1)
+    int k = 0;
+    while (k + 1 < p.num_seg && s_off[k + 1] <= e) ++k;
+    return k;
+  };
+  bool bad = false;
+  for (int64_t e = static_cast<int64_t>(blockIdx.x) * kAggBlock + threadIdx.x; e < p.num_edges;
+       e += static_cast<int64_t>(gridDim.x) * kAggBlock) {
+    const int k = segment(e);
+    const int64_t key = s_out[k] + p.col[e];
+    p.keys[e] = key;
+    p.sources[e] = s_in[k] + p.row[e];
+    if (e + 1 < p.num_edges) {
+      const int q = segment(e + 1);
+      bad |= key > s_out[q] + p.col[e + 1];
+    }
+  }
+  if (bad) *p.grouped = 0;
+}
+
+// Offsets of the rows in non-decreasing keys: position e, where the key before it is kp and its own k, is the offset
+// of the rows in (kp, k]; a long stretch of rows without edges is filled by the whole wavefront.
+__global__ __launch_bounds__(kAggBlock) void coo_offsets_kernel(const int64_t* __restrict__ keys, int64_t n,
+                                                                int64_t num_rows, uint32_t* __restrict__ indptr) {
+  constexpr int kShortGap = 4;
+  const int lane = threadIdx.x % kWave;
+  const int64_t tid = static_cast<int64_t>(blockIdx.x) * kAggBlock + threadIdx.x;
+  const int64_t stride = static_cast<int64_t>(gridDim.x) * kAggBlock;
+  auto clamp = [&](int64_t k) { return k < -1 ? -1 : k > num_rows ? num_rows : k; };
+  for (int64_t e0 = tid - lane; e0 < n; e0 += stride) {   // wave-uniform
+    const int64_t e = e0 + lane;
+    int64_t k = -1, kp = -1;
+    if (e < n) {
+      k = clamp(keys[e]);
+      if (e > 0) kp = clamp(keys[e - 1]);
+    }
+    const int64_t gap = k - kp;
+    if (gap > 0 && gap <= kShortGap)
+      for (int64_t t = kp + 1; t <= k; ++t) indptr[t] = static_cast<uint32_t>(e);
+    uint64_t wide = ballot(gap > kShortGap);
+    while (wide != 0) {
+      const int src = __ffsll(static_cast<long long>(wide)) - 1;
+      wide &= wide - 1;
+      const int64_t a = __shfl(kp, src, kWave) + 1, b = __shfl(k, src, kWave);
+      for (int64_t t = a + lane; t <= b; t += kWave) indptr[t] = static_cast<uint32_t>(e0 + src);
+    }
+  }
+  const int64_t last = n > 0 ? clamp(keys[n - 1]) : -1;
+  for (int64_t t = last + 1 + tid; t <= num_rows; t += stride) indptr[t] = static_cast<uint32_t>(n);
+}
+
+static size_t coo_align(size_t x) { return (x + 255) / 256 * 256; }
+
 }  // namespace apt
+
+extern "C" int apt_coo_prepare(const int64_t* coo_row, const int64_t* coo_col, int64_t num_edges, const int64_t* coo_offset,
+                               const int64_t* input_offset, const int64_t* output_offset, int num_segments,
+                               const int64_t* last_offset, int64_t* keys, int64_t* sources, int64_t* result, void* stream) {
+  using namespace apt;
+  APT_REQUIRE(num_edges >= 0 && result != nullptr, APT_EINVAL, "apt_coo_prepare: bad arguments");
+  APT_REQUIRE(num_segments >= 1 && num_segments < kCooSegments, APT_ELIMIT, "apt_coo_prepare: %d segments outside [1, %d]",
+              num_segments, kCooSegments - 1);
+  APT_REQUIRE(num_edges == 0 || (coo_row != nullptr && coo_col != nullptr && coo_offset != nullptr && keys != nullptr &&
+                                 sources != nullptr),
+              APT_EINVAL, "apt_coo_prepare: a tensor is NULL");
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  hipLaunchKernelGGL(coo_grouped_init_kernel, dim3(1), dim3(1), 0, st, result, last_offset, result + 1);
+  APT_LAUNCH_CHECK("coo_grouped_init_kernel");
+  if (num_edges == 0) return APT_OK;
+  const CooParams p{coo_row, coo_col, num_edges, coo_offset, input_offset, output_offset, num_segments, keys, sources, result};
+  hipLaunchKernelGGL(coo_prepare_kernel, dim3(static_cast<unsigned>(std::min<int64_t>(ceil_div(num_edges, kAggBlock), 4096))),
+                     dim3(kAggBlock), 0, st, p);
+  APT_LAUNCH_CHECK("coo_prepare_kernel");
+  return APT_OK;
+}
+
+extern "C" size_t apt_coo_sum_workspace_bytes(int64_t num_edges, int64_t num_out_rows, int grouped) {
+  using namespace apt;
+  if (num_edges < 0 || num_edges > 0x7fffffffLL || num_out_rows < 0 || num_out_rows > 0x7fffffffLL) return 0;
+  const size_t offsets = coo_align(sizeof(uint32_t) * (num_out_rows + 1));
+  if (grouped != 0) return offsets;
+  const size_t order = apt_block_transpose_workspace_bytes(num_edges, 1, num_out_rows);
+  return order == 0 ? 0 : offsets + coo_align(sizeof(uint32_t) * (num_edges + 1)) + order;
+}
+
+extern "C" int apt_coo_sum(int mode, const int64_t* keys, const int64_t* sources, int64_t num_edges, int grouped,
+                           const void* input, int64_t num_in_rows, const void* edata, int64_t dim, int elem_size, void* out,
+                           int64_t num_out_rows, void* workspace, size_t workspace_bytes, void* stream) {
+  using namespace apt;
+  APT_REQUIRE(mode >= 0 && mode <= 2, APT_EINVAL, "apt_coo_sum: mode %d (0 copy_u, 1 copy_e, 2 u_mul_e)", mode);
+  APT_REQUIRE(num_edges >= 0 && num_in_rows >= 0 && num_out_rows >= 0 && dim > 0, APT_EINVAL,
+              "apt_coo_sum: bad shape (E %lld, rows %lld -> %lld, dim %lld)", (long long)num_edges, (long long)num_in_rows,
+              (long long)num_out_rows, (long long)dim);
+  APT_REQUIRE(elem_size == 2 || elem_size == 4, APT_EINVAL, "apt_coo_sum: elem_size %d (4 = fp32, 2 = bf16)", elem_size);
+  if (num_out_rows == 0) return APT_OK;
+  const size_t need = apt_coo_sum_workspace_bytes(num_edges, num_out_rows, grouped);
+  APT_REQUIRE(need > 0, APT_ELIMIT, "apt_coo_sum: %lld edges or %lld rows out of range", (long long)num_edges,
+              (long long)num_out_rows);
+  APT_REQUIRE(out != nullptr && (num_edges == 0 || (keys != nullptr && sources != nullptr && input != nullptr)) &&
+                  (mode != 2 || edata != nullptr || num_edges == 0),
+              APT_EINVAL, "apt_coo_sum: a tensor is NULL");
+  APT_REQUIRE(workspace != nullptr && workspace_bytes >= need && (reinterpret_cast<uintptr_t>(workspace) & 255) == 0,
+              APT_EWORKSPACE, "apt_coo_sum: workspace too small or not 256-byte aligned (see apt_coo_sum_workspace_bytes)");
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  char* ws = static_cast<char*>(workspace);
+  uint32_t* indptr = reinterpret_cast<uint32_t*>(ws);
+  ws += coo_align(sizeof(uint32_t) * (num_out_rows + 1));
+  uint32_t* order = nullptr;
+  if (grouped != 0) {
+    const int64_t work = std::max(num_edges, num_out_rows + 1);
+    hipLaunchKernelGGL(coo_offsets_kernel, dim3(static_cast<unsigned>(std::min<int64_t>(ceil_div(work, kAggBlock), 4096))),
+                       dim3(kAggBlock), 0, st, keys, num_edges, num_out_rows, indptr);
+    APT_LAUNCH_CHECK("coo_offsets_kernel");
+  } else {
+    order = reinterpret_cast<uint32_t*>(ws);
+    ws += coo_align(sizeof(uint32_t) * (num_edges + 1));
+    const size_t left = workspace_bytes - static_cast<size_t>(ws - static_cast<char*>(workspace));
+    if (const int rc = apt_block_transpose(keys, num_edges, 1, num_out_rows, indptr, order, ws, left, stream)) return rc;
+  }
+  SourceSumParams p{};
+  p.indptr = indptr;
+  p.index = order;
+  p.fanout = 1;
+  p.via = mode == 1 ? nullptr : sources;
+  p.edata = mode == 2 ? edata : nullptr;
+  p.dz = input;
+  p.num_dst = mode == 1 ? num_edges : num_in_rows;
+  p.dim = dim;
+  p.num_src = num_out_rows;
+  p.dx = out;
+  return mode == 2 ? source_sum<uint32_t, true>(p, elem_size, st) : source_sum<uint32_t, false>(p, elem_size, st);
+}
 
 extern "C" int apt_block_aggregate_backward(const void* indptr, const void* index, int index_bytes, int fanout,
                                             int64_t num_src, const float* dst_scale, const void* dz, int64_t num_dst,
@@ -197,7 +379,7 @@ extern "C" int apt_block_aggregate_backward(const void* indptr, const void* inde
   if (num_src == 0) return APT_OK;
   APT_REQUIRE(indptr != nullptr && dx != nullptr && (num_dst == 0 || (index != nullptr && dz != nullptr)), APT_EINVAL,
               "apt_block_aggregate_backward: a tensor is NULL");
-  SourceSumParams p;
+  SourceSumParams p{};
   p.indptr = indptr;
   p.index = index;
   p.fanout = static_cast<uint32_t>(fanout);
@@ -208,5 +390,5 @@ extern "C" int apt_block_aggregate_backward(const void* indptr, const void* inde
   p.num_src = num_src;
   p.dx = dx;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  return index_bytes == 8 ? source_sum<int64_t>(p, elem_size, st) : source_sum<uint32_t>(p, elem_size, st);
+  return index_bytes == 8 ? source_sum<int64_t, false>(p, elem_size, st) : source_sum<uint32_t, false>(p, elem_size, st);
 }

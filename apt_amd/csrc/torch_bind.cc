@@ -130,6 +130,16 @@ int64_t* pinned_counts() {
   return s.pinned_counts.data_ptr<int64_t>();
 }
 
+// A few device counts on the host, through pinned memory of the calling thread (operators of a backward pass run on
+// autograd's threads).  Waits for the current stream.
+const int64_t* read_counts(const Tensor& dev) {
+  static thread_local Tensor host;
+  if (!host.defined()) host = torch::zeros({8}, torch::TensorOptions().dtype(torch::kInt64).pinned_memory(true));
+  host.narrow(0, 0, dev.numel()).copy_(dev, /*non_blocking=*/true);
+  c10::hip::getCurrentHIPStream().synchronize();
+  return host.data_ptr<int64_t>();
+}
+
 }  // namespace
 
 // ---------------------------------------------------------------- registries
@@ -865,7 +875,6 @@ Tensor spmm(int mode, Tensor coo_row, Tensor coo_col, Tensor input, const Tensor
   TORCH_CHECK(coo.numel() >= 2 && oo.numel() >= coo.numel() - 1 && row.numel() == col.numel(),
               "npc: spmm: bad offsets or edge lists");
   const int nseg = static_cast<int>(coo.numel() - 1);
-  const int64_t out_num = oo.index({-1}).item<int64_t>();
   Tensor io, ed;
   if (input_offset) io = ids_on_device(*input_offset, "input_offset");
   if (edata) {
@@ -874,14 +883,32 @@ Tensor spmm(int mode, Tensor coo_row, Tensor coo_col, Tensor input, const Tensor
                 "npc: spmm: edata must be [E, dim] of the input dtype");
   }
   if (mode == 1) TORCH_CHECK(x.size(0) == row.numel(), "npc: spmm_copy_e_sum needs one input row per edge");
+  TORCH_CHECK(!input_offset || io.numel() >= nseg, "npc: spmm: input_offset is shorter than the segments");
+  // every edge's rows, whether the edges come grouped by output row (a block's COO does), and the number of output
+  // rows: the last two are read back in one copy
+  auto keys = torch::empty({2, row.numel()}, i64_opts());
+  auto probe = torch::empty({2}, i64_opts());
+  check(apt_coo_prepare(i64(row), i64(col), row.numel(), i64(coo), input_offset ? i64(io) : nullptr, i64(oo), nseg,
+                        i64(oo) + oo.numel() - 1, keys.data_ptr<int64_t>(), keys.data_ptr<int64_t>() + row.numel(),
+                        probe.data_ptr<int64_t>(), stream()));
+  const int64_t* host = read_counts(probe);
+  const int grouped = host[0] != 0;
+  const int64_t out_num = host[1];
+  const int64_t E = row.numel();
+  const size_t need = apt_coo_sum_workspace_bytes(E, out_num, grouped);
+  if (need > 0) {
+    auto ws = torch::empty({static_cast<int64_t>(need)}, x.options().dtype(torch::kUInt8));
+    auto out = torch::empty({out_num, x.size(1)}, x.options());
+    check(apt_coo_sum(mode, i64(keys), E ? i64(keys) + E : nullptr, E, grouped, x.data_ptr(), x.size(0),
+                      edata ? ed.data_ptr() : nullptr, x.size(1), static_cast<int>(x.element_size()), out.data_ptr(),
+                      out_num, ws.data_ptr(), need, stream()));
+    return out;
+  }
+  // more edges or rows than the ordering takes: the edge-parallel sum, atomics where a row's edges are apart
   auto out = torch::zeros({out_num, x.size(1)}, x.options().dtype(torch::kFloat32));
-  // a block's COO is destination-major: found out on the device, rows inside a wavefront's edges skip the atomics
-  auto grouped = torch::empty({1}, torch::TensorOptions().dtype(torch::kInt32).device(device()));
-  check(apt_coo_is_grouped(i64(col), col.numel(), grouped.data_ptr<int>(), stream()));
-  check(apt_spmm_sum(mode, i64(row), i64(col), row.numel(), x.data_ptr(), x.size(0),
-                     edata ? ed.data_ptr() : nullptr, x.size(1), static_cast<int>(x.element_size()),
-                     i64(coo), input_offset ? i64(io) : nullptr, i64(oo), nseg, out.data_ptr<float>(),
-                     out_num, grouped.data_ptr<int>(), stream()));
+  check(apt_spmm_sum(mode, i64(row), i64(col), E, x.data_ptr(), x.size(0), edata ? ed.data_ptr() : nullptr, x.size(1),
+                     static_cast<int>(x.element_size()), i64(coo), input_offset ? i64(io) : nullptr, i64(oo), nseg,
+                     out.data_ptr<float>(), out_num, nullptr, stream()));
   return out.to(x.scalar_type());
 }
 
@@ -895,11 +922,11 @@ Tensor sddmm(int op, Tensor coo_row, Tensor coo_col, Tensor lhs, Tensor rhs, Ten
   auto lo = ids_on_device(lhs_offset, "lhs_offset"), ro = ids_on_device(rhs_offset, "rhs_offset");
   TORCH_CHECK(coo.numel() >= 2 && lo.numel() >= coo.numel() - 1 && ro.numel() >= coo.numel() - 1,
               "npc: sddmm: bad offsets");
-  auto out = torch::empty({row.numel(), l.size(1)}, l.options().dtype(torch::kFloat32));
-  check(apt_sddmm(op, i64(row), i64(col), row.numel(), l.data_ptr(), l.size(0), r.data_ptr(), r.size(0),
+  auto out = torch::empty({row.numel(), l.size(1)}, l.options());
+  check(apt_coo_combine(op, i64(row), i64(col), row.numel(), l.data_ptr(), l.size(0), r.data_ptr(), r.size(0),
                   l.size(1), static_cast<int>(l.element_size()), i64(coo), i64(lo), i64(ro),
-                  static_cast<int>(coo.numel() - 1), out.data_ptr<float>(), stream()));
-  return out.to(l.scalar_type());
+                  static_cast<int>(coo.numel() - 1), out.data_ptr(), stream()));
+  return out;
 }
 
 }  // namespace

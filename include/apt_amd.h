@@ -810,6 +810,32 @@ int apt_block_aggregate_backward(const void* indptr, const void* index, int inde
                                  int64_t num_src, const float* dst_scale, const void* dz,
                                  int64_t num_dst, int64_t dim, int elem_size, void* dx, void* stream);
 
+/* Sums over a COO in any order (apt_spmm_sum's three modes) without atomics, with the
+ * result in the input's type; what the spmm_* operators do.
+ *   apt_coo_prepare  keys[e] = output_offset[k] + col[e], sources[e] = input_offset[k] +
+ *                    row[e] (k = segment of e as in apt_spmm_sum, offsets NULL = 0);
+ *                    result[0] = 1 if the keys are non-decreasing, else 0; result[1] =
+ *                    *last_offset (0 if NULL): what a caller reads back in one copy
+ *   apt_coo_sum      out[r, :] = sum over the edges with key r, in edge order; every
+ *                    row is written; edges with a key or source out of range do not
+ *                    count.  grouped: result[0]; otherwise the edges are ordered by key
+ *                    first (apt_block_transpose).  workspace:
+ *                    apt_coo_sum_workspace_bytes, 256-byte aligned; 0 = sizes out of
+ *                    range (take apt_spmm_sum)
+ *   apt_coo_combine  apt_sddmm with the result in the input's type */
+int apt_coo_prepare(const int64_t* coo_row, const int64_t* coo_col, int64_t num_edges,
+                    const int64_t* coo_offset, const int64_t* input_offset, const int64_t* output_offset,
+                    int num_segments, const int64_t* last_offset, int64_t* keys, int64_t* sources,
+                    int64_t* result, void* stream);
+size_t apt_coo_sum_workspace_bytes(int64_t num_edges, int64_t num_out_rows, int grouped);
+int apt_coo_sum(int mode, const int64_t* keys, const int64_t* sources, int64_t num_edges, int grouped,
+                const void* input, int64_t num_in_rows, const void* edata, int64_t dim, int elem_size,
+                void* out, int64_t num_out_rows, void* workspace, size_t workspace_bytes, void* stream);
+int apt_coo_combine(int op, const int64_t* coo_row, const int64_t* coo_col, int64_t num_edges,
+                    const void* lhs, int64_t num_lhs_rows, const void* rhs, int64_t num_rhs_rows,
+                    int64_t dim, int elem_size, const int64_t* coo_offset, const int64_t* lhs_offset,
+                    const int64_t* rhs_offset, int num_segments, void* out, void* stream);
+
 /* A GAT layer between its dense product and its activation (python/npc/model/
  * gatconv.py:116-126,207-236), forward and backward.  ft, out, d_out, d_ft and the
  * bias are of one type (elem_size 4 = fp32, 2 = bf16), attn_l / attn_r and their
