@@ -137,6 +137,8 @@ SYMBOLS = {
     "apt_gat_layer_backward_workspace_bytes": (_SZ, [_I64, _I, _I64, _I, _I64, _I64]),
     "apt_gat_layer_backward": (_I, [_P, _I64, _I, _P, _I64, _I, _I64, _I, _P, _P, _I, C.c_float, _P, _P, _P, _P, _P, _P, _I, _P,
                                     _P, _I64, _P, _P, _P, _P, _P, _SZ, _P]),
+    "apt_rows_gemm_workspace_bytes": (_SZ, [_I64, _I64, _I64]),
+    "apt_rows_gemm": (_I, [_P, _I64, _P, _I64, _I64, _P, _I64, _P, _I64, _I64, _I64, _I64, _I64, _P, _I, _P, _P, _SZ, _P]),
     "apt_linear_wgrad_workspace_bytes": (_SZ, [_I64, _I64, _I64, _I]),
     "apt_linear_wgrad": (_I, [_P, _P, _I64, _I64, _I64, _I, _P, _P, _P, _SZ, _P]),
     "apt_time_next_sample": (_I, [_I, _P, _P]),
@@ -1056,3 +1058,28 @@ def linear_wgrad(dy, x, want_bias=True):
     check(lib().apt_linear_wgrad(_ptr(dy), _ptr(x), m, n, k, x.element_size(), _ptr(dw), _ptr(db), _ptr(ws), ws.numel(),
                                  _stream()))
     return dw, db
+
+
+def rows_gemm(x1, w1, x2=None, w2=None, bias=None, out=None):
+    """x1 w1^T (+ x2 w2^T on the first rows) (+ bias) in fp32; out: added to.  Weights may have any strides."""
+    x1 = x1.contiguous()
+    x2 = None if x2 is None else x2.contiguous()
+    if any(t is not None and (not t.is_cuda or t.dtype != torch.float32) for t in (x1, w1, x2, w2, bias, out)):
+        raise AptError("rows_gemm takes fp32 GPU tensors")
+    m, k1 = x1.shape
+    n = w1.shape[0]
+    k2, m2 = (0, 0) if x2 is None else (x2.shape[1], x2.shape[0])
+    if (w1.shape[1] != k1 or (x2 is not None and (w2 is None or tuple(w2.shape) != (n, k2) or m2 > m))
+            or (bias is not None and bias.numel() != n)
+            or (out is not None and (tuple(out.shape) != (m, n) or not out.is_contiguous()))):
+        raise AptError("rows_gemm: shapes do not fit")
+    bias = None if bias is None else bias.contiguous()
+    accumulate = out is not None
+    if out is None:
+        out = torch.empty((m, n), dtype=torch.float32, device=x1.device)
+    need = int(lib().apt_rows_gemm_workspace_bytes(n, k1, k2))
+    ws = torch.empty(max(need, 256), dtype=torch.uint8, device=x1.device)
+    s2 = (0, 0) if w2 is None else w2.stride()
+    check(lib().apt_rows_gemm(_ptr(x1), k1, _ptr(w1), w1.stride(0), w1.stride(1), _ptr(x2), k2, _ptr(w2), s2[0], s2[1], m, m2,
+                              n, _ptr(bias), int(accumulate), _ptr(out), _ptr(ws), ws.numel(), _stream()))
+    return out

@@ -962,25 +962,55 @@ std::tuple<Tensor, Tensor> linear_wgrad(const Tensor& dy_in, const Tensor& x_in,
   const int64_t m = x.size(0), n = dy.size(1), k = x.size(1);
   const int es = static_cast<int>(x.element_size());
   const size_t need = apt_linear_wgrad_workspace_bytes(m, n, k, es);
-  TORCH_CHECK(need > 0, "npc: block_linear: a weight of ", n, " x ", k, " is out of range");
+  Tensor db;
+  if (need == 0) {   // a weight beyond the kernel's sizes
+    if (want_bias) db = dy.sum(0);
+    return {dy.t().mm(x), db};
+  }
   auto ws = torch::empty({static_cast<int64_t>(need)}, x.options().dtype(torch::kUInt8));
   auto dw = torch::empty({n, k}, x.options());
-  Tensor db;
   if (want_bias) db = torch::empty({n}, x.options());
   check(apt_linear_wgrad(dy.data_ptr(), x.data_ptr(), m, n, k, es, dw.data_ptr(), want_bias ? db.data_ptr() : nullptr,
                          ws.data_ptr(), need, stream()));
   return {dw, db};
 }
 
-// y = x w^T + b (or x w with `kn`: w is [k, n]).  The product itself and the gradient towards x are plain GEMMs and
-// go to the library; the gradient of the weight reduces over the block's rows and has a kernel of its own.
+// x w^T (+ x2 w2^T on the first rows) (+ b) with w [n, k] of any strides; `onto`: added to (and returned).  fp32 rows
+// take apt_rows_gemm, bf16 rows, whose products are bound by memory in the library's kernels already, at::mm.
+Tensor dense(const Tensor& x_in, const Tensor& w, const Tensor& x2_in = Tensor(), const Tensor& w2 = Tensor(),
+             const Tensor& b = Tensor(), Tensor onto = Tensor()) {
+  const int64_t m = x_in.size(0), k = x_in.size(1), n = w.size(0);
+  const bool pair = x2_in.defined();
+  const int64_t m2 = pair ? x2_in.size(0) : 0, k2 = pair ? x2_in.size(1) : 0;
+  TORCH_CHECK(w.size(1) == k && (!pair || (w2.size(0) == n && w2.size(1) == k2 && m2 <= m)) && (!b.defined() || b.numel() == n),
+              "npc: a layer's rows have ", k, " columns, its weight is ", n, " x ", w.size(1), " (or the bias does not fit)");
+  const size_t need = x_in.scalar_type() == torch::kFloat32 ? apt_rows_gemm_workspace_bytes(n, k, k2) : 0;
+  if (need > 0) {
+    auto x = x_in.contiguous();
+    Tensor x2 = pair ? x2_in.contiguous() : Tensor(), bias = b.defined() ? b.contiguous() : Tensor();
+    const bool accumulate = onto.defined();
+    auto y = accumulate ? onto : torch::empty({m, n}, x.options());
+    auto ws = torch::empty({static_cast<int64_t>(need)}, x.options().dtype(torch::kUInt8));
+    check(apt_rows_gemm(x.data_ptr<float>(), k, w.data_ptr<float>(), w.stride(0), w.stride(1),
+                        pair ? x2.data_ptr<float>() : nullptr, k2, pair ? w2.data_ptr<float>() : nullptr,
+                        pair ? w2.stride(0) : 0, pair ? w2.stride(1) : 0, m, m2, n,
+                        bias.defined() ? bias.data_ptr<float>() : nullptr, accumulate, y.data_ptr<float>(), ws.data_ptr(),
+                        need, stream()));
+    return y;
+  }
+  Tensor y = at::linear(x_in, w, b.defined() ? std::optional<Tensor>(b) : std::nullopt);
+  if (pair) y.narrow(0, 0, m2).addmm_(x2_in, w2.t());
+  return onto.defined() ? onto.add_(y) : y;
+}
+
+// y = x w^T + b (or x w with `kn`: w is [k, n]).
 struct BlockLinearFn : public torch::autograd::Function<BlockLinearFn> {
   static Tensor forward(torch::autograd::AutogradContext* ctx, const Tensor& x, const Tensor& w,
                         const std::optional<Tensor>& b, bool kn) {
     ctx->save_for_backward({x, w});
     ctx->saved_data["kn"] = kn;
     ctx->saved_data["bias"] = b.has_value();
-    return kn ? at::mm(x, w) : at::linear(x, w, b);
+    return dense(x, kn ? w.t() : w, Tensor(), Tensor(), b.value_or(Tensor()));
   }
   static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx,
                                                  torch::autograd::variable_list grads) {
@@ -988,12 +1018,13 @@ struct BlockLinearFn : public torch::autograd::Function<BlockLinearFn> {
     const Tensor &x = saved[0], &w = saved[1], &dy = grads[0];
     const bool kn = ctx->saved_data["kn"].toBool(), bias = ctx->saved_data["bias"].toBool();
     Tensor dx, dw, db;
-    if (ctx->needs_input_grad(0)) dx = kn ? dy.mm(w.t()) : dy.mm(w);
     if (torch::GradMode::is_enabled()) {   // a graph of the gradients is wanted: operations that carry one
+      if (ctx->needs_input_grad(0)) dx = kn ? dy.mm(w.t()) : dy.mm(w);
       dw = kn ? x.t().mm(dy) : dy.t().mm(x);
       if (bias) db = dy.sum(0);
-    } else if (ctx->needs_input_grad(1) || bias) {
-      std::tie(dw, db) = kn ? linear_wgrad(x, dy, false) : linear_wgrad(dy, x, bias);
+    } else {
+      if (ctx->needs_input_grad(0)) dx = dense(dy, kn ? w : w.t());
+      if (ctx->needs_input_grad(1) || bias) std::tie(dw, db) = kn ? linear_wgrad(x, dy, false) : linear_wgrad(dy, x, bias);
     }
     return {dx, dw, db, Tensor()};
   }
@@ -1115,6 +1146,91 @@ Tensor BlockAggregate(const Tensor& relabeled, int64_t num_dst, int64_t fanout, 
                        (x.scalar_type() == torch::kFloat32 || x.scalar_type() == torch::kBFloat16),
                    "npc: block_aggregate: input must be a 2-D fp32 or bf16 GPU tensor");
   return BlockAggregateFn::apply(x.contiguous(), relabeled, num_dst, fanout, mean, csr_indptr, csr_indices);
+}
+
+// ---------------------------------------------------------------- GraphSAGE layer
+namespace {
+
+// x[:num_dst] w_self^T + bias + mean over the block of x, times w_neigh^T; the product comes before the mean where it
+// makes the rows shorter.  As one function the two products and their gradients are added up in the kernels that form
+// them: no pass over the result to add them, no zero-filled gradient of the destinations' rows.
+struct SageLayerFn : public torch::autograd::Function<SageLayerFn> {
+  static Tensor forward(torch::autograd::AutogradContext* ctx, const Tensor& x, const Tensor& w_neigh, const Tensor& w_self,
+                        const std::optional<Tensor>& bias, const Tensor& relabeled, int64_t num_dst, int64_t fanout,
+                        const std::optional<Tensor>& csr_indptr, const std::optional<Tensor>& csr_indices) {
+    const Tensor b = bias.value_or(Tensor()), self = x.narrow(0, 0, num_dst);
+    const bool first = x.size(1) > w_self.size(0);
+    Tensor mean, inv, out;
+    if (first) {
+      std::tie(out, inv) = aggregate_forward(relabeled, num_dst, fanout, dense(x, w_neigh), true);
+      out = dense(self, w_self, Tensor(), Tensor(), b, out);
+    } else {
+      std::tie(mean, inv) = aggregate_forward(relabeled, num_dst, fanout, x, true);
+      out = dense(self, w_self, mean, w_neigh, b);
+    }
+    ctx->save_for_backward({x, w_neigh, w_self, relabeled, inv, mean, csr_indptr.value_or(Tensor()),
+                            csr_indices.value_or(Tensor())});
+    ctx->saved_data["bias"] = bias.has_value();
+    ctx->saved_data["num_dst"] = num_dst;
+    ctx->saved_data["fanout"] = fanout;
+    return out;
+  }
+  static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx,
+                                                 torch::autograd::variable_list grads) {
+    const auto saved = ctx->get_saved_variables();
+    const Tensor &x = saved[0], &w_neigh = saved[1], &w_self = saved[2], &relabeled = saved[3], &inv = saved[4];
+    const bool bias = ctx->saved_data["bias"].toBool(), first = x.size(1) > w_self.size(0);
+    const int64_t num_dst = ctx->saved_data["num_dst"].toInt(), fanout = ctx->saved_data["fanout"].toInt();
+    const int64_t num_src = x.size(0);
+    const auto spread = [&](const Tensor& d) {
+      return aggregate_backward(d, relabeled, num_dst, fanout, num_src, inv, saved[6], saved[7]);
+    };
+    const Tensor dz = grads[0].contiguous(), self = x.narrow(0, 0, num_dst);
+    const bool want_x = ctx->needs_input_grad(0), want_w = ctx->needs_input_grad(1) || ctx->needs_input_grad(2) || bias;
+    Tensor dx, dwn, dws, db;
+    if (torch::GradMode::is_enabled()) {   // a graph of the gradients is wanted: operations that carry one
+      const Tensor dzn = first ? spread(dz) : dz.mm(w_neigh);
+      const Tensor mean = first ? Tensor() : BlockAggregateFn::apply(x, relabeled, num_dst, fanout, true, std::nullopt, std::nullopt);
+      dx = (first ? dzn.mm(w_neigh) : spread(dzn)) + at::constant_pad_nd(dz.mm(w_self), {0, 0, 0, num_src - num_dst});
+      dwn = first ? dzn.t().mm(x) : dz.t().mm(mean);
+      dws = dz.t().mm(self);
+      if (bias) db = dz.sum(0);
+    } else {
+      Tensor dpre;
+      if (first) dpre = spread(dz);
+      if (want_w) {
+        std::tie(dws, db) = linear_wgrad(dz, self, bias);
+        dwn = std::get<0>(first ? linear_wgrad(dpre, x, false) : linear_wgrad(dz, saved[5], false));
+      }
+      if (want_x)
+        dx = first ? dense(dpre, w_neigh.t(), dz, w_self.t()) : [&] {
+          Tensor d = spread(dense(dz, w_neigh.t()));
+          if (d.scalar_type() == torch::kFloat32) dense(dz, w_self.t(), Tensor(), Tensor(), Tensor(), d.narrow(0, 0, num_dst));
+          else d.narrow(0, 0, num_dst).addmm_(dz, w_self);
+          return d;
+        }();
+    }
+    return {dx, dwn, dws, db, Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
+  }
+};
+
+}  // namespace
+
+Tensor SageLayer(const Tensor& relabeled, int64_t num_dst, int64_t fanout, const Tensor& x, const Tensor& w_neigh,
+                 const Tensor& w_self, const std::optional<Tensor>& bias, const std::optional<Tensor>& csr_indptr,
+                 const std::optional<Tensor>& csr_indices) {
+  check_block("sage_layer", relabeled, num_dst, fanout);
+  const auto t = x.scalar_type();
+  TORCH_CHECK_TYPE(x.is_cuda() && x.dim() == 2 && (t == torch::kFloat32 || t == torch::kBFloat16),
+                   "npc: sage_layer: input must be a 2-D fp32 or bf16 GPU tensor");
+  const auto fits = [&](const Tensor& w) {
+    return w.is_cuda() && w.dim() == 2 && w.scalar_type() == t && w.size(1) == x.size(1) && w.size(0) == w_self.size(0);
+  };
+  TORCH_CHECK(fits(w_neigh) && fits(w_self) && x.size(1) > 0 && w_self.size(0) > 0 && num_dst <= x.size(0) &&
+                  (!bias.has_value() || (bias->is_cuda() && bias->scalar_type() == t && bias->dim() == 1 &&
+                                         bias->size(0) == w_self.size(0))),
+              "npc: sage_layer: weights, bias and input do not fit each other");
+  return SageLayerFn::apply(x.contiguous(), w_neigh, w_self, bias, relabeled, num_dst, fanout, csr_indptr, csr_indices);
 }
 
 // ---------------------------------------------------------------- GAT layer, from the dense product to the bias
@@ -1291,6 +1407,7 @@ TORCH_LIBRARY(npc, m) {
       .def("block_formats", &BlockFormats)
       .def("block_linear", &BlockLinear)
       .def("block_aggregate", &BlockAggregate)
+      .def("sage_layer", &SageLayer)
       .def("gat_layer", &GatLayer)
       .def("cluster_and_permute", &ClusterAndPermuteLocal)
       .def("register_graph_partition", &RegisterGraphPartition)

@@ -11,6 +11,7 @@ reproducible.
 """
 import torch
 from torch import nn
+from torch.nn.modules.module import _has_any_global_hook
 
 from . import ops  # noqa: F401  (loads the npc operators)
 
@@ -27,19 +28,25 @@ class BlockAggregate:
                                              f.get("csr_indptr"), f.get("csr_indices"))
 
 
-def _trains_natively(x, weight):
-    """Whether the gradient of `weight` can come from the library's kernel: a training step on fp32 or bf16 GPU rows
-    of the weight's dtype (autocast picks dtypes of its own)."""
-    return (x.is_cuda and x.dim() == 2 and x.dtype == weight.dtype and x.dtype in (torch.float32, torch.bfloat16)
-            and torch.is_grad_enabled() and weight.requires_grad and not torch.is_autocast_enabled("cuda"))
+def _native_rows(x, weight):
+    """Whether the library's products can take x (fp32 or bf16 GPU rows of the weight's dtype; autocast picks dtypes of
+    its own).  A bf16 product without gradients is the same one either way."""
+    if not (x.is_cuda and x.dim() == 2 and x.dtype == weight.dtype and weight.is_cuda and weight.numel() > 0
+            and not torch.is_autocast_enabled("cuda")):
+        return False
+    return x.dtype == torch.float32 or (x.dtype == torch.bfloat16 and torch.is_grad_enabled() and weight.requires_grad)
+
+
+def _plain(layer):
+    """A plain nn.Linear: no subclass, parametrization, replaced forward or hooks, all of which are the module's to run."""
+    return (type(layer) is nn.Linear and "forward" not in layer.__dict__
+            and not (layer._forward_hooks or layer._forward_pre_hooks or layer._backward_hooks
+                     or layer._backward_pre_hooks or _has_any_global_hook()))
 
 
 def _linear(layer, x):
-    """layer(x); a plain nn.Linear takes its weight and bias gradients from npc.block_linear (hooks, subclasses and
-    everything else go through the module)."""
-    if (type(layer) is nn.Linear and _trains_natively(x, layer.weight)
-            and not (layer._forward_hooks or layer._forward_pre_hooks or layer._backward_hooks
-                     or layer._backward_pre_hooks)):
+    """layer(x), its products and gradients from npc.block_linear where they can be."""
+    if _plain(layer) and _native_rows(x, layer.weight) and (layer.bias is None or layer.bias.dtype == x.dtype):
         return torch.ops.npc.block_linear(x, layer.weight, layer.bias, False)
     return layer(x)
 
@@ -61,6 +68,16 @@ class SAGEConv(nn.Module):
 
     def forward(self, block, feat):
         """feat: [block.num_src, in_feats]; the first num_dst rows are the destinations."""
+        wn, ws, b = self.fc_neigh.weight, self.fc_self.weight, self.fc_self.bias
+        if (_plain(self.fc_neigh) and _plain(self.fc_self) and self.fc_neigh.bias is None and feat.is_cuda
+                and feat.dim() == 2 and feat.dtype in (torch.float32, torch.bfloat16)
+                and feat.dtype == wn.dtype == ws.dtype and (b is None or b.dtype == feat.dtype)
+                and wn.shape == ws.shape == (self.out_feats, self.in_feats) and feat.shape[1] == self.in_feats > 0
+                and self.out_feats > 0 and feat.shape[0] >= block.num_dst and not torch.is_autocast_enabled("cuda")):
+            f = block.formats or {}
+            rst = torch.ops.npc.sage_layer(block.relabeled, block.num_dst, block.fanout, feat, wn, ws, b,
+                                           f.get("csr_indptr"), f.get("csr_indices"))
+            return self.activation(rst) if self.activation is not None else rst
         h_self = feat[:block.num_dst]
         if self.in_feats > self.out_feats:
             h_neigh = BlockAggregate.apply(block, _linear(self.fc_neigh, feat), True)
@@ -89,7 +106,7 @@ class GraphConv(nn.Module):
         fanout = float(block.fanout)
         if self.norm in ("left", "both"):
             feat = feat * (fanout ** -0.5 if self.norm == "both" else 1.0 / fanout)
-        h = (torch.ops.npc.block_linear(feat, self.weight, None, True) if _trains_natively(feat, self.weight)
+        h = (torch.ops.npc.block_linear(feat, self.weight, None, True) if _native_rows(feat, self.weight)
              else torch.matmul(feat, self.weight))
         rst = BlockAggregate.apply(block, h, False)
         if self.norm in ("right", "both"):

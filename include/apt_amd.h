@@ -790,6 +790,19 @@ int apt_block_transpose(const int64_t* relabeled, int64_t num_dst, int fanout, i
                         uint32_t* indptr, uint32_t* slots, void* workspace, size_t workspace_bytes,
                         void* stream);
 
+/* The dense product of a layer in fp32, of two operand pairs at once:
+ *   y[r, j] (+)= sum_k x1[r, k] w1[j, k] + (r < m2: sum_k x2[r, k] w2[j, k]) + bias[j]
+ * x1 [m, k1], x2 [m2, k2] (k2 = 0: none), y [m, n], all row by row; the element (j, k) of a
+ * weight is at j * stride_n + k * stride_k; bias may be NULL; accumulate: y is added to.
+ * The products are formed from bf16 parts of the operands, to at least the accuracy of
+ * an fp32 sum; infinities and NaN come out as such a sum has them. */
+size_t apt_rows_gemm_workspace_bytes(int64_t n, int64_t k1, int64_t k2);   /* 0 = out of range */
+int apt_rows_gemm(const float* x1, int64_t k1, const float* w1, int64_t w1_stride_n,
+                  int64_t w1_stride_k, const float* x2, int64_t k2, const float* w2,
+                  int64_t w2_stride_n, int64_t w2_stride_k, int64_t m, int64_t m2, int64_t n,
+                  const float* bias, int accumulate, float* y, void* workspace,
+                  size_t workspace_bytes, void* stream);
+
 /* Sum / mean over a block as a layer uses it, and its gradient (python/npc/model/
  * sageconv.py:100-114: the reference's Aggregate, whose backward is the operator with
  * the edges reversed).
