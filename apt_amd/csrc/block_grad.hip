@@ -14,7 +14,7 @@
 
 namespace apt {
 
-constexpr int kHubEdges = 32;
+constexpr int kHubEdges = 16;
 constexpr int kHubList = 1024;             // rows of a workgroup at the most, so its list of hubs never overflows
 constexpr int kSourceBlocks = 2048;
 
@@ -147,8 +147,10 @@ __global__ __launch_bounds__(kAggBlock) void source_sum_kernel(SourceSumParams p
       float acc[VEC];
 #pragma unroll
       for (int k = 0; k < VEC; ++k) acc[k] = 0.f;
-      for (int64_t e = lo + grp * LPR; e < hi; e += kAggBlock) {
-        add_edges(edge(e + l, e + l < hi), static_cast<int>(min(hi - e, static_cast<int64_t>(LPR))), c, live, acc);
+      for (int64_t e = lo + grp; e < hi; e += kAggBlock) {   // every kGroups-th edge, so that all groups have some
+        const int64_t at = e + static_cast<int64_t>(l) * kGroups;
+        add_edges(edge(at, at < hi), static_cast<int>(min((hi - e + kGroups - 1) / kGroups, static_cast<int64_t>(LPR))), c, live,
+                  acc);
       }
 #pragma unroll
       for (int k = 0; k < VEC; ++k) s_sum[grp][l * VEC + k] = acc[k];

@@ -43,6 +43,20 @@ __device__ __forceinline__ void load_vec(const T* base, int64_t elem, float (&v)
   }
 }
 
+// The same in two halves, for loads that should be in flight together: load every row from an address that is valid
+// in any case (row 0 in the place of a missing one), then convert and use those that exist.  A load or a conversion
+// inside a branch is waited for there.
+template <typename T, int VEC> using Row = typename Pack<T, VEC>::type;
+template <typename T, int VEC>
+__device__ __forceinline__ Row<T, VEC> load_row(const T* base, int64_t elem) {
+  return *reinterpret_cast<const Row<T, VEC>*>(base + elem);
+}
+template <typename T, int VEC>
+__device__ __forceinline__ float row_elem(const Row<T, VEC>& raw, int k) {
+  if constexpr (VEC == 1) return to_float<T>(raw);
+  else return to_float<T>(raw[k]);
+}
+
 template <typename T, int VEC>
 __device__ __forceinline__ void store_vec(T* base, int64_t elem, const float (&v)[VEC]) {
   using P = typename Pack<T, VEC>::type;

@@ -35,6 +35,19 @@ struct ParamVec {
   __device__ __forceinline__ float at(int64_t i) const {
     return elem_size == 4 ? static_cast<const float*>(p)[i] : to_float<uint16_t>(static_cast<const uint16_t*>(p)[i]);
   }
+  // elements i .. i + N - 1, all on their way together
+  template <int N> __device__ __forceinline__ void load(int64_t i, float (&v)[N]) const {
+    if (elem_size == 4) {
+#pragma unroll
+      for (int k = 0; k < N; ++k) v[k] = static_cast<const float*>(p)[i + k];
+    } else {
+      uint16_t raw[N];
+#pragma unroll
+      for (int k = 0; k < N; ++k) raw[k] = static_cast<const uint16_t*>(p)[i + k];
+#pragma unroll
+      for (int k = 0; k < N; ++k) v[k] = to_float<uint16_t>(raw[k]);
+    }
+  }
 };
 
 // Type of what an operation of a row (T) and an attention parameter gives: bf16 only if both are.
@@ -59,21 +72,15 @@ __global__ __launch_bounds__(kAggBlock) void gat_pair_scores_kernel(const T* __r
   const int h = live ? l / LPH : 0;
   const int64_t row_len = static_cast<int64_t>(heads) * VEC * LPH;
   float al[VEC], ar[VEC];
-#pragma unroll
-  for (int k = 0; k < VEC; ++k) {
-    al[k] = live ? attn_l.at(l * VEC + k) : 0.f;
-    ar[k] = live ? attn_r.at(l * VEC + k) : 0.f;
-  }
+  attn_l.load(live ? l * VEC : 0, al);
+  attn_r.load(live ? l * VEC : 0, ar);
   const Terms<T> term(attn_l);
   const int64_t step = static_cast<int64_t>(gridDim.x) * kGroups;
   for (int64_t r0 = static_cast<int64_t>(blockIdx.x) * kGroups + grp; r0 < num_rows; r0 += kRows * step) {
-    float v[kRows][VEC];
+    Row<T, VEC> v[kRows];
 #pragma unroll
-    for (int q = 0; q < kRows; ++q) {
-#pragma unroll
-      for (int k = 0; k < VEC; ++k) v[q][k] = 0.f;
-      if (live && r0 + q * step < num_rows) load_vec<T, VEC>(x, (r0 + q * step) * row_len + l * VEC, v[q]);
-    }
+    for (int q = 0; q < kRows; ++q)
+      v[q] = load_row<T, VEC>(x, min(r0 + q * step, num_rows - 1) * row_len + (live ? l * VEC : 0));
 #pragma unroll
     for (int q = 0; q < kRows; ++q) {
       const int64_t r = r0 + q * step;
@@ -81,8 +88,9 @@ __global__ __launch_bounds__(kAggBlock) void gat_pair_scores_kernel(const T* __r
       float sl = 0.f, sr = 0.f;
 #pragma unroll
       for (int k = 0; k < VEC; ++k) {
-        sl += term(v[q][k] * al[k]);
-        sr += term(v[q][k] * ar[k]);
+        const float f = live ? row_elem<T, VEC>(v[q], k) : 0.f;
+        sl += term(f * al[k]);
+        sr += term(f * ar[k]);
       }
 #pragma unroll
       for (int off = LPH / 2; off > 0; off >>= 1) {
@@ -176,7 +184,7 @@ static bool launch_pair_scores(const void* x, int64_t n, int64_t num_dst, int he
 
 // ------------------------------------------------------------------ backward, source half
 // As source_sum_kernel (block_grad.hip): a lane group per source row, hubs shared by the workgroup.
-constexpr int kGatHubEdges = 32;
+constexpr int kGatHubEdges = 16;
 constexpr int kGatHubList = 1024;
 constexpr int kGatSourceBlocks = 2048;
 
@@ -198,9 +206,17 @@ struct GatSourceParams {
 };
 
 // VEC consecutive features of a row belong to at most two heads (dim >= VEC): h0, and h1 from element `cut` on.
-template <typename T, int VEC, int LPR, typename I>
+// Nearly all sources have one or two edges, so a row is a chain of three dependent reads (offsets, edges, rows of the
+// destinations) and little else: a group has kRows rows in flight with their first edges, loads stand outside branches
+// (a conversion inside one waits for its load), and what depends on the columns alone (heads, parameters) is taken out
+// of the loop over the rows.  124 k rows of 4 x 64 bf16, 261 k edges: 68 us; 193 us with a wavefront per row, loads in
+// branches and the heads worked out per row (63 MB written, 134 MB of destinations' rows read from the caches).
+// TWO: a lane's features may belong to two heads.
+template <typename T, int VEC, int LPR, typename I, bool TWO>
 __global__ __launch_bounds__(kAggBlock) void gat_source_kernel(GatSourceParams p) {
   constexpr int kGroups = kAggBlock / LPR;
+  constexpr int kRows = 4;     // rows of a group in flight,
+  constexpr int kHead = 2;     // with their first edges
   constexpr int kUnroll = 4;
   __shared__ int s_hub[kGatHubList];
   __shared__ int s_hubs;
@@ -217,15 +233,19 @@ __global__ __launch_bounds__(kAggBlock) void gat_source_kernel(GatSourceParams p
   struct Cols {
     int64_t c;
     int h0, h1, cut;
-    bool live;
+    bool live, start;   // start: the lane's first feature is its head's
+    float al[VEC], ar[VEC];
   };
   auto columns = [&](int64_t c0) {
     Cols k;
     k.c = c0 + static_cast<int64_t>(l) * VEC;
     k.live = k.c < row_len;
     k.h0 = k.live ? static_cast<int>(k.c / p.dim) : 0;
+    k.start = k.c == k.h0 * p.dim;
     k.cut = static_cast<int>(min(static_cast<int64_t>(VEC), (k.h0 + 1) * p.dim - k.c));
     k.h1 = k.cut < VEC ? k.h0 + 1 : k.h0;
+    p.attn_l.load(k.live ? k.c : 0, k.al);
+    p.attn_r.load(k.live ? k.c : 0, k.ar);
     return k;
   };
   struct Acc {
@@ -239,46 +259,57 @@ __global__ __launch_bounds__(kAggBlock) void gat_source_kernel(GatSourceParams p
   };
   // lane j of the group holds edge j: its destination (-1: none) and where its weights are
   auto edge_of = [&](int64_t at, int64_t end, int64_t& dst, int64_t& weight) {
-    dst = -1;
-    weight = 0;
-    if (at >= end) return;
+    const bool mine = at < end;
+    const I v = index[mine ? at : 0];
     if constexpr (sizeof(I) == 4) {
-      weight = static_cast<int64_t>(index[at]);
-      dst = static_cast<int64_t>(static_cast<uint32_t>(weight) / p.fanout);
+      weight = static_cast<int64_t>(v);
+      dst = static_cast<int64_t>(v / p.fanout);
     } else {
-      dst = static_cast<int64_t>(index[at]);
-      weight = p.eids[at];
+      weight = p.eids[mine ? at : 0];
+      dst = static_cast<int64_t>(v);
     }
-    if (dst >= p.num_dst) dst = -1;
+    if (!mine || dst >= p.num_dst) dst = -1;
   };
-  auto add_edges = [&](int64_t my_dst, int64_t my_weight, int n, const Cols& col, Acc& acc) {
-    for (int e0 = 0; e0 < n; e0 += kUnroll) {
-      float v[kUnroll][VEC], a0[kUnroll], a1[kUnroll], z0[kUnroll], z1[kUnroll];
+  // Edges that the group's lanes hold (none beyond n), all on their way before the first is used.
+  struct Loaded {
+    Row<T, VEC> v[kUnroll];
+    float a0[kUnroll], z0[kUnroll], a1[kUnroll], z1[kUnroll];
+    bool ok[kUnroll];
+  };
+  auto load_edges = [&](int64_t my_dst, int64_t my_weight, int e0, int n, const Cols& col, int count, Loaded& o) {
 #pragma unroll
-      for (int u = 0; u < kUnroll; ++u) {
-#pragma unroll
-        for (int k = 0; k < VEC; ++k) v[u][k] = 0.f;
-        a0[u] = a1[u] = z0[u] = z1[u] = 0.f;
-        if (e0 + u < n) {
-          const int64_t d = __shfl(my_dst, e0 + u, LPR), w = __shfl(my_weight, e0 + u, LPR);
-          if (d >= 0 && col.live) {
-            load_vec<T, VEC>(d_out, d * row_len + col.c, v[u]);
-            a0[u] = p.attn[w * p.heads + col.h0];
-            z0[u] = p.dz[w * p.heads + col.h0];
-            if (VEC > 1 && col.h1 != col.h0) {
-              a1[u] = p.attn[w * p.heads + col.h1];
-              z1[u] = p.dz[w * p.heads + col.h1];
-            }
-          }
-        }
+    for (int u = 0; u < kUnroll; ++u) {
+      if (u >= count) break;
+      // in the place of a missing edge, the last one again: its lines are on their way already
+      const int j = max(min(min(e0 + u, n - 1), LPR - 1), 0);
+      const int64_t d = __shfl(my_dst, j, LPR), w = __shfl(my_weight, j, LPR);
+      o.ok[u] = e0 + u < n && d >= 0;
+      const int64_t at = d >= 0 ? w * p.heads : 0;
+      o.v[u] = load_row<T, VEC>(d_out, (d >= 0 ? d * row_len : 0) + (col.live ? col.c : 0));
+      o.a0[u] = p.attn[at + col.h0];
+      o.z0[u] = p.dz[at + col.h0];
+      if (TWO) {
+        o.a1[u] = p.attn[at + (col.live ? col.h1 : 0)];
+        o.z1[u] = p.dz[at + (col.live ? col.h1 : 0)];
       }
+    }
+  };
+  auto sum_edges = [&](const Loaded& o, const Cols& col, int count, Acc& acc) {
 #pragma unroll
-      for (int u = 0; u < kUnroll; ++u) {
+    for (int u = 0; u < kUnroll; ++u) {
+      if (u >= count) break;
+      if (!o.ok[u]) continue;
 #pragma unroll
-        for (int k = 0; k < VEC; ++k) acc.v[k] += (k < col.cut ? a0[u] : a1[u]) * v[u][k];
-        acc.el0 += z0[u];
-        acc.el1 += z1[u];
-      }
+      for (int k = 0; k < VEC; ++k) acc.v[k] += (!TWO || k < col.cut ? o.a0[u] : o.a1[u]) * row_elem<T, VEC>(o.v[u], k);
+      acc.el0 += o.z0[u];
+      if (TWO) acc.el1 += o.z1[u];
+    }
+  };
+  auto add_edges = [&](int64_t my_dst, int64_t my_weight, int from, int n, const Cols& col, Acc& acc) {
+    for (int e0 = from; e0 < n; e0 += kUnroll) {
+      Loaded o;
+      load_edges(my_dst, my_weight, e0, n, col, kUnroll, o);
+      sum_edges(o, col, kUnroll, acc);
     }
   };
   auto finish = [&](int64_t r, const Cols& col, const Acc& acc) {
@@ -287,39 +318,60 @@ __global__ __launch_bounds__(kAggBlock) void gat_source_kernel(GatSourceParams p
     float r0 = 0.f, r1 = 0.f;
     if (r < p.num_dst) {
       r0 = term(p.d_er[r * p.heads + col.h0]);
-      r1 = term(p.d_er[r * p.heads + col.h1]);
+      if (TWO) r1 = term(p.d_er[r * p.heads + col.h1]);
     }
     float out[VEC];
 #pragma unroll
     for (int k = 0; k < VEC; ++k) {
-      const bool first = k < col.cut;
+      const bool first = !TWO || k < col.cut;
       out[k] = as_stored<T>(acc.v[k]);
-      if (r < p.num_dst) out[k] = as_stored<T>(out[k] + as_stored<T>((first ? r0 : r1) * p.attn_r.at(col.c + k)));
-      out[k] += as_stored<T>((first ? e0 : e1) * p.attn_l.at(col.c + k));
-      if ((col.c + k) % p.dim == 0) p.d_el[r * p.heads + (first ? col.h0 : col.h1)] = first ? e0 : e1;
+      if (r < p.num_dst) out[k] = as_stored<T>(out[k] + as_stored<T>((first ? r0 : r1) * col.ar[k]));
+      out[k] += as_stored<T>((first ? e0 : e1) * col.al[k]);
     }
+    if (col.start) p.d_el[r * p.heads + col.h0] = e0;
+    if (TWO && col.cut < VEC) p.d_el[r * p.heads + col.h1] = e1;
     store_vec<T, VEC>(d_ft, r * row_len + col.c, out);
   };
   const int64_t row_groups = static_cast<int64_t>(gridDim.x) * kGroups;
-  for (int64_t r = static_cast<int64_t>(grp) * gridDim.x + blockIdx.x; r < p.num_src; r += row_groups) {
-    const int64_t lo = static_cast<int64_t>(indptr[r]), hi = static_cast<int64_t>(indptr[r + 1]);
-    if (hi - lo > kGatHubEdges) {
-      if (l == 0) s_hub[atomicAdd(&s_hubs, 1)] = static_cast<int>(r);
-      continue;
-    }
-    int64_t dst, weight;
-    edge_of(lo + l, hi, dst, weight);
-    for (int64_t c0 = 0; c0 < row_len; c0 += LPR * VEC) {
-      const Cols col = columns(c0);
-      Acc acc;
-      clear(acc);
-      add_edges(dst, weight, static_cast<int>(min(hi - lo, static_cast<int64_t>(LPR))), col, acc);
-      for (int64_t e = lo + LPR; e < hi; e += LPR) {   // LPR < kGatHubEdges only
-        int64_t d, w;
-        edge_of(e + l, hi, d, w);
-        add_edges(d, w, static_cast<int>(min(hi - e, static_cast<int64_t>(LPR))), col, acc);
+  for (int64_t c0 = 0; c0 < row_len; c0 += LPR * VEC) {
+    const Cols col = columns(c0);
+    for (int64_t r0 = static_cast<int64_t>(grp) * gridDim.x + blockIdx.x; r0 < p.num_src; r0 += kRows * row_groups) {
+      int64_t lo[kRows], hi[kRows], dst[kRows], weight[kRows];
+      int n[kRows];     // edges; a hub's are left for later
+#pragma unroll
+      for (int q = 0; q < kRows; ++q) {
+        const int64_t r = r0 + q * row_groups;
+        const I a = indptr[min(r, p.num_src - 1)], b = indptr[min(r, p.num_src - 1) + 1];
+        lo[q] = static_cast<int64_t>(a);
+        hi[q] = lo[q] + static_cast<int64_t>(b - a) * (r < p.num_src);   // (a condition would wait for the load)
       }
-      finish(r, col, acc);
+#pragma unroll
+      for (int q = 0; q < kRows; ++q) edge_of(lo[q] + l, hi[q], dst[q], weight[q]);
+      Loaded head[kRows];
+#pragma unroll
+      for (int q = 0; q < kRows; ++q) {
+        n[q] = hi[q] - lo[q] > kGatHubEdges ? 0 : static_cast<int>(hi[q] - lo[q]);
+        load_edges(dst[q], weight[q], 0, n[q], col, kHead, head[q]);
+      }
+#pragma unroll
+      for (int q = 0; q < kRows; ++q) {
+        const int64_t r = r0 + q * row_groups;
+        if (r >= p.num_src) break;
+        if (hi[q] - lo[q] > kGatHubEdges) {
+          if (l == 0 && c0 == 0) s_hub[atomicAdd(&s_hubs, 1)] = static_cast<int>(r);
+          continue;
+        }
+        Acc acc;
+        clear(acc);
+        sum_edges(head[q], col, kHead, acc);
+        add_edges(dst[q], weight[q], kHead, min(n[q], LPR), col, acc);
+        for (int e = LPR; e < n[q]; e += LPR) {   // LPR < kGatHubEdges only
+          int64_t d, w;
+          edge_of(lo[q] + e + l, hi[q], d, w);
+          add_edges(d, w, 0, min(n[q] - e, LPR), col, acc);
+        }
+        finish(r, col, acc);
+      }
     }
   }
   __syncthreads();
@@ -331,10 +383,10 @@ __global__ __launch_bounds__(kAggBlock) void gat_source_kernel(GatSourceParams p
       const Cols col = columns(c0);
       Acc acc;
       clear(acc);
-      for (int64_t e = lo + grp * LPR; e < hi; e += kAggBlock) {
+      for (int64_t e = lo + grp; e < hi; e += kAggBlock) {   // every kGroups-th edge, so that all groups have some
         int64_t d, w;
-        edge_of(e + l, hi, d, w);
-        add_edges(d, w, static_cast<int>(min(hi - e, static_cast<int64_t>(LPR))), col, acc);
+        edge_of(e + l * kGroups, hi, d, w);
+        add_edges(d, w, 0, static_cast<int>(min((hi - e + kGroups - 1) / kGroups, static_cast<int64_t>(LPR))), col, acc);
       }
 #pragma unroll
       for (int k = 0; k < VEC; ++k) s_sum[grp][k * LPR + l] = acc.v[k];
@@ -357,14 +409,14 @@ __global__ __launch_bounds__(kAggBlock) void gat_source_kernel(GatSourceParams p
   }
 }
 
-template <typename T, int VEC, typename I>
-static void launch_gat_source(const GatSourceParams& p, hipStream_t st) {
+template <typename T, int VEC, typename I, bool TWO>
+static void launch_gat_source_as(const GatSourceParams& p, hipStream_t st) {
   const int64_t per_row = ceil_div(p.heads * p.dim, VEC);
 #define APT_GAT_SOURCE(LPR)                                                                                        \
   do {                                                                                                            \
     const int64_t blocks = std::max(ceil_div(p.num_src, kGatHubList),                                             \
-                                    std::min<int64_t>(ceil_div(p.num_src, kAggBlock / LPR), kGatSourceBlocks));   \
-    hipLaunchKernelGGL((gat_source_kernel<T, VEC, LPR, I>), dim3(static_cast<unsigned>(blocks)), dim3(kAggBlock), 0, \
+                                    std::min<int64_t>(ceil_div(p.num_src, 4 * kAggBlock / LPR), kGatSourceBlocks));   \
+    hipLaunchKernelGGL((gat_source_kernel<T, VEC, LPR, I, TWO>), dim3(static_cast<unsigned>(blocks)), dim3(kAggBlock), 0, \
                        st, p);                                                                                    \
   } while (0)
   if (per_row <= 8) APT_GAT_SOURCE(8);
@@ -374,16 +426,28 @@ static void launch_gat_source(const GatSourceParams& p, hipStream_t st) {
 #undef APT_GAT_SOURCE
 }
 
+template <typename T, int VEC, typename I>
+static void launch_gat_source(const GatSourceParams& p, hipStream_t st) {
+  if (VEC > 1 && p.dim % VEC != 0) launch_gat_source_as<T, VEC, I, (VEC > 1)>(p, st);
+  else launch_gat_source_as<T, VEC, I, false>(p, st);
+}
+
 template <typename T, typename I>
 static void launch_gat_source_t(const GatSourceParams& p, hipStream_t st) {
   const bool aligned = ((reinterpret_cast<uintptr_t>(p.d_out) | reinterpret_cast<uintptr_t>(p.d_ft)) & 15) == 0;
+  if constexpr (sizeof(T) == 2) {   // 16 bytes a lane: twice the rows in a wavefront
+    if (aligned && (p.heads * p.dim) % 8 == 0 && p.dim >= 8) {
+      launch_gat_source<T, 8, I>(p, st);
+      return;
+    }
+  }
   if (aligned && (p.heads * p.dim) % 4 == 0 && p.dim >= 4) launch_gat_source<T, 4, I>(p, st);
   else launch_gat_source<T, 1, I>(p, st);
 }
 
 // ------------------------------------------------------------------ backward, parameters
 // Column sums over the rows: a workgroup has a run of rows, a thread VEC columns of every RG-th of them.
-constexpr int kParamBlocks = 512;
+constexpr int kParamBlocks = 1024;
 
 template <typename T, int VEC>
 __global__ __launch_bounds__(kAggBlock) void gat_param_grad_kernel(const T* __restrict__ ft, const T* __restrict__ d_out,
@@ -463,14 +527,17 @@ template <typename T>
 static void launch_param_grad(const void* ft, const void* d_out, const float* d_el, const float* d_er, int64_t num_src,
                               int64_t num_dst, int heads, int64_t dim, float* part, ParamVec attn_l, hipStream_t st) {
   const int64_t blocks = param_blocks(num_src), rows = ceil_div(num_src, blocks), row_len = heads * dim;
-  const bool vec4 = row_len % 4 == 0 && dim >= 4 && ((reinterpret_cast<uintptr_t>(ft) | reinterpret_cast<uintptr_t>(d_out)) & 15) == 0;
+  const bool aligned = ((reinterpret_cast<uintptr_t>(ft) | reinterpret_cast<uintptr_t>(d_out)) & 15) == 0;
+  constexpr int kWide = 16 / sizeof(T);
+  const int vec = aligned && row_len % kWide == 0 && dim >= kWide ? kWide : aligned && row_len % 4 == 0 && dim >= 4 ? 4 : 1;
   int lanes = 8;
-  while (lanes < kAggBlock && lanes * (vec4 ? 4 : 1) < row_len) lanes <<= 1;
+  while (lanes < kAggBlock && lanes * vec < row_len) lanes <<= 1;
   const dim3 grid(static_cast<unsigned>(blocks)), block(kAggBlock);
 #define APT_PARAM(V)                                                                                               \
   hipLaunchKernelGGL((gat_param_grad_kernel<T, V>), grid, block, 0, st, static_cast<const T*>(ft),                  \
                      static_cast<const T*>(d_out), d_el, d_er, num_src, num_dst, heads, dim, lanes, rows, part, attn_l)
-  if (vec4) APT_PARAM(4);
+  if (vec == kWide) APT_PARAM(kWide);
+  else if (vec == 4) APT_PARAM(4);
   else APT_PARAM(1);
 #undef APT_PARAM
 }
@@ -575,6 +642,12 @@ extern "C" int apt_gat_layer_backward(const int64_t* neighbors, int64_t num_dst,
   p.dim = dim;
   p.d_ft = d_ft;
   p.d_el = d_el;
+  if (num_dst == 0) {   // entry 0 of every array is read in the place of a missing edge
+    p.d_out = ft;
+    p.attn = p.dz = el;
+  }
+  if (index == nullptr || num_dst == 0) p.index = indptr;
+  if (!by_slot && (eids == nullptr || num_edges == 0)) p.eids = static_cast<const int64_t*>(indptr);
   if (elem_size == 4) {
     if (by_slot) launch_gat_source_t<float, uint32_t>(p, st);
     else launch_gat_source_t<float, int64_t>(p, st);
@@ -589,6 +662,12 @@ extern "C" int apt_gat_layer_backward(const int64_t* neighbors, int64_t num_dst,
   APT_LAUNCH_CHECK("gat_param_grad_kernel");
   const int64_t n = heads * dim;
   const int splits = static_cast<int>(param_blocks(num_src));
+  if (attn_elem_size == elem_size) {
+    if (elem_size == 4) launch_partial_sums<float, float>(part, 3 * n, splits, d_attn_l, n, d_attn_r, n, d_bias, n, st);
+    else launch_partial_sums<uint16_t, uint16_t>(part, 3 * n, splits, d_attn_l, n, d_attn_r, n, d_bias, n, st);
+    APT_LAUNCH_CHECK("partial_sums_kernel");
+    return APT_OK;
+  }
   if (attn_elem_size == 4) launch_partial_sums<float, float>(part, 3 * n, splits, d_attn_l, n, d_attn_r, n, nullptr, 0, st);
   else launch_partial_sums<uint16_t, uint16_t>(part, 3 * n, splits, d_attn_l, n, d_attn_r, n, nullptr, 0, st);
   APT_LAUNCH_CHECK("partial_sums_kernel");

@@ -284,36 +284,34 @@ __global__ __launch_bounds__(kAggBlock) void spmm_ell_kernel(const int64_t* __re
     // lane s of the group fetches slot s's id (one coalesced load for the destination); the slot loop reads
     // it with a shuffle.  (Ids that do not fit 32 bits, or more slots than lanes: every lane loads them itself.)
     const bool shared_ids = fanout <= LPR && num_src <= 0x7fffffffLL;
-    int my_id = -1;
-    if (shared_ids && l < fanout) {
-      const int64_t v = ids[l];
-      my_id = (v >= 0 && v < num_src) ? static_cast<int>(v) : -1;
-    }
+    const int64_t mine = ids[min(l, fanout - 1)];
+    const int my_id = mine >= 0 && mine < num_src ? static_cast<int>(mine) : -1;   // used if shared_ids
+    const int64_t spare = max(min(i, num_src - 1), int64_t{0});   // read in the place of a missing edge
     for (int64_t d0 = 0; d0 < dim; d0 += LPR * VEC) {   // every lane of the group stays in the loop (shuffles)
       const int64_t d = d0 + static_cast<int64_t>(l) * VEC;
       const bool live = d < dim;
+      const int64_t at = live ? d : 0;
       float acc[VEC];
 #pragma unroll
       for (int k = 0; k < VEC; ++k) acc[k] = 0.f;
       int cnt = 0;
       for (int s0 = 0; s0 < fanout; s0 += kUnroll) {
-        float v[kUnroll][VEC];
+        Row<T, VEC> v[kUnroll];
+        bool ok[kUnroll];
 #pragma unroll
         for (int u = 0; u < kUnroll; ++u) {
-#pragma unroll
-          for (int k = 0; k < VEC; ++k) v[u][k] = 0.f;
-          if (s0 + u < fanout) {
-            const int64_t src = shared_ids ? static_cast<int64_t>(__shfl(my_id, s0 + u, LPR)) : ids[s0 + u];
-            if (src >= 0 && src < num_src) {
-              if (live) load_vec<T, VEC>(x, src * dim + d, v[u]);
-              ++cnt;
-            }
-          }
+          const int s = min(s0 + u, fanout - 1);
+          const int64_t src = shared_ids ? static_cast<int64_t>(__shfl(my_id, s, LPR)) : ids[s];
+          ok[u] = s0 + u < fanout && src >= 0 && src < num_src;
+          v[u] = load_row<T, VEC>(x, (ok[u] ? src : spare) * dim + at);
+          cnt += ok[u];
         }
 #pragma unroll
-        for (int u = 0; u < kUnroll; ++u)
+        for (int u = 0; u < kUnroll; ++u) {
+          if (!ok[u]) continue;
 #pragma unroll
-          for (int k = 0; k < VEC; ++k) acc[k] += v[u][k];
+          for (int k = 0; k < VEC; ++k) acc[k] += row_elem<T, VEC>(v[u], k);
+        }
       }
       const float scale = (mean && cnt > 0) ? 1.0f / static_cast<float>(cnt) : 1.0f;
       if (live) {
@@ -531,25 +529,23 @@ __global__ __launch_bounds__(kAggBlock) void gat_ell_wave_kernel(
 #pragma unroll
     for (int q = 0; q < VEC; ++q) acc[q] = 0.f;
     for (int u0 = 0; u0 < fanout; u0 += kUnroll) {
-      float v[kUnroll][VEC];
+      Row<T, VEC> v[kUnroll];
       float au[kUnroll];
+      bool ok[kUnroll];
 #pragma unroll
       for (int u = 0; u < kUnroll; ++u) {
-        au[u] = 0.f;
-#pragma unroll
-        for (int q = 0; q < VEC; ++q) v[u][q] = 0.f;
-        if (u0 + u < fanout) {
-          const int64_t src = wave_read(id, (u0 + u) << log2_heads);
-          if (src >= 0 && src < num_src) {
-            au[u] = __shfl(a, ((u0 + u) << log2_heads) + hf, kWave);
-            if (live) load_vec<T, VEC>(ft, src * row_len + d, v[u]);
-          }
-        }
+        const int at = min(u0 + u, fanout - 1);
+        const int64_t src = wave_read(id, at << log2_heads);
+        ok[u] = u0 + u < fanout && src >= 0 && src < num_src;
+        au[u] = __shfl(a, (at << log2_heads) + hf, kWave);
+        v[u] = load_row<T, VEC>(ft, (ok[u] ? src : min(i, num_src - 1)) * row_len + (live ? d : 0));   // in any case a row
       }
 #pragma unroll
-      for (int u = 0; u < kUnroll; ++u)
+      for (int u = 0; u < kUnroll; ++u) {
+        if (!ok[u]) continue;   // the same in all lanes
 #pragma unroll
-        for (int q = 0; q < VEC; ++q) acc[q] += au[u] * v[u][q];
+        for (int q = 0; q < VEC; ++q) acc[q] += au[u] * row_elem<T, VEC>(v[u], q);
+      }
     }
     if (live) {
       if (bias != nullptr) {
@@ -565,6 +561,7 @@ template <typename T, typename OUT, int VEC>
 static bool launch_gat_wave(const int64_t* nbr, int64_t num_dst, const int64_t* num_dst_dev, int fanout,
                             const void* ft, int64_t num_src, int heads, int64_t dim, const float* el,
                             const float* er, float slope, void* out, float* attn_out, const void* bias, hipStream_t st) {
+  if (num_src == 0) return false;   // the kernel reads a row for every slot
   if (dim % VEC != 0 || (heads & (heads - 1)) != 0 || heads * fanout > kWave) return false;
   const int64_t lph = dim / VEC;
   if ((lph & (lph - 1)) != 0 || heads * lph > kWave) return false;
@@ -773,27 +770,20 @@ __global__ __launch_bounds__(kAggBlock) void gat_bwd_edge_wave_kernel(
     if (live) load_vec<DT, VEC>(d_out, i * row_len + d, go);
     float my_part = 0.f;   // slot layout: dOut[i, hs] . ft[id, hs]
     for (int u0 = 0; u0 < fanout; u0 += kUnroll) {
-      float v[kUnroll][VEC];
+      Row<T, VEC> v[kUnroll];
       bool ok[kUnroll];
 #pragma unroll
       for (int u = 0; u < kUnroll; ++u) {
-        ok[u] = false;
-#pragma unroll
-        for (int q = 0; q < VEC; ++q) v[u][q] = 0.f;
-        if (u0 + u < fanout) {
-          const int64_t src = wave_read(id, (u0 + u) << log2_heads);
-          if (src >= 0 && src < num_src) {
-            ok[u] = true;
-            if (live) load_vec<T, VEC>(ft, src * row_len + d, v[u]);
-          }
-        }
+        const int64_t src = wave_read(id, min(u0 + u, fanout - 1) << log2_heads);
+        ok[u] = u0 + u < fanout && src >= 0 && src < num_src;
+        v[u] = load_row<T, VEC>(ft, (ok[u] ? src : min(i, num_src - 1)) * row_len + (live ? d : 0));   // in any case a row
       }
 #pragma unroll
       for (int u = 0; u < kUnroll; ++u) {
         if (!ok[u]) continue;  // the same in all lanes
         float part = 0.f;
 #pragma unroll
-        for (int q = 0; q < VEC; ++q) part += go[q] * v[u][q];
+        for (int q = 0; q < VEC; ++q) part += go[q] * row_elem<T, VEC>(v[u], q);
         for (int off = lph / 2; off > 0; off >>= 1) part += __shfl_xor(part, off, kWave);
         const float got = __shfl(part, hs * lph, kWave);   // the dot product of head hs
         if (k == u0 + u) my_part = got;
@@ -825,6 +815,7 @@ static bool launch_gat_bwd_wave(const int64_t* nbr, int64_t num_dst, int fanout,
                                 int heads, int64_t dim, const float* el, const float* er, float slope,
                                 const float* attn, const void* d_out, const int64_t* csc_indptr, float* a_edge,
                                 float* dz_edge, float* d_er, hipStream_t st) {
+  if (num_src == 0) return false;   // the kernel reads a row for every slot
   if (dim % VEC != 0 || (heads & (heads - 1)) != 0 || heads * fanout > kWave) return false;
   const int64_t lph = dim / VEC;
   if ((lph & (lph - 1)) != 0 || heads * lph > kWave) return false;
@@ -1001,6 +992,7 @@ static int block_sum(const char* who, const int64_t* neighbors, int64_t num_dst,
   APT_REQUIRE(neighbors != nullptr && out != nullptr && (input != nullptr || num_src == 0), APT_EINVAL,
               "%s: a tensor is NULL", who);
   hipStream_t st = static_cast<hipStream_t>(stream);
+  if (num_src == 0) input = out;   // no edge is valid: the kernel reads a row, and uses none
   const bool vec4 = dim % 4 == 0 && (reinterpret_cast<uintptr_t>(input) & 15) == 0 &&
                     (reinterpret_cast<uintptr_t>(out) & 15) == 0;
 #define APT_BLOCK_SUM(T, OUT, V) \
