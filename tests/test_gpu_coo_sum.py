@@ -24,7 +24,8 @@ def _sum(key, x, n_out, ok):
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("order", ["grouped", "any"])
 @pytest.mark.parametrize("E,n_in,n_out,dim", [(1, 1, 1, 1), (5000, 700, 900, 47), (20000, 3000, 70, 100), (3000, 500, 100000, 8),
-                                              (9000, 2000, 1500, 256), (0, 4, 6, 16)])
+                                              (9000, 2000, 1500, 256), (60000, 3000, 900, 41), (40000, 3000, 70, 100),
+                                              (300000, 500, 200000, 8), (0, 4, 6, 16)])
 def test_spmm_operators(E, n_in, n_out, dim, order, dtype):
     import apt_amd as npc
     row, col = _edges(E, n_in, n_out, order, E + dim)
