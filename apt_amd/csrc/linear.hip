@@ -9,15 +9,19 @@
 // of its rows in MFMA accumulators and leaves it in a partial buffer, and a second
 // launch adds the partials in a fixed order (reproducible, no atomics).
 //
+// fp32 operands are multiplied as bf16 parts (split_bf16.hpp): the fp32 matrix
+// instruction would bound the product (57 us of its rate alone for 71 k rows of
+// 256 x 100 in tiles of 64; the four 256-wide gradients of a GraphSAGE step of
+// 4096 seeds took 169 us with it and take 132).
 // Both operands have the reduced dimension as their row index, which is what an
-// MFMA operand wants *inside* a lane (8 consecutive rows of one column for bf16,
-// one for fp32).  No LDS transpose: a lane loads VEC consecutive columns of each
+// MFMA operand wants *inside* a lane (8 consecutive rows of one column).  No LDS transpose: a lane loads VEC consecutive columns of each
 // of its rows and the 16-bit halves are regrouped by column in registers
 // (v_perm); the columns of the MFMA tiles are simply numbered lane * VEC + j.
 #include <algorithm>
 
 #include "common.hpp"
 #include "partial_sums.hpp"
+#include "split_bf16.hpp"
 
 namespace apt {
 
@@ -54,15 +58,8 @@ struct WgradParams {
   int64_t rows_per_split;
 };
 
-template <typename T> struct WgradType;
-template <> struct WgradType<float> {
-  static constexpr int kRows = 16;       // rows per step: 4 MFMAs of depth 4
-  static constexpr int kLoads = 4;       // rows of a lane in a step
-};
-template <> struct WgradType<uint16_t> {
-  static constexpr int kRows = 32;       // one MFMA of depth 32
-  static constexpr int kLoads = 8;
-};
+constexpr int kWgradRows = 32;     // rows per step: one MFMA of depth 32 (fp32: six, of its bf16 parts)
+constexpr int kWgradLoads = 8;     // consecutive rows of a lane in a step; the lanes of a 16-lane group share them
 
 // The lane's rows of one operand as they come from memory: VEC consecutive columns of each row (VEC 4), two pairs
 // (VEC 2) or kWgradFrags single columns (VEC 1), at the byte offsets off[].  What an MFMA wants is taken out of it
@@ -70,10 +67,10 @@ template <> struct WgradType<uint16_t> {
 template <typename T, int VEC> struct WgradRows {
   static constexpr int kWords = sizeof(T) == 4 || VEC == 1 ? kWgradFrags : 2;   // 32-bit registers per row
   static constexpr int kOffsets = kWgradFrags / VEC;
-  uint32_t v[WgradType<T>::kLoads][kWords];
+  uint32_t v[kWgradLoads][kWords];
   __device__ __forceinline__ void load(buffer_t buf, uint32_t at, uint32_t row_bytes, const uint32_t (&off)[kOffsets]) {
 #pragma unroll
-    for (int r = 0; r < WgradType<T>::kLoads; ++r, at += row_bytes) {
+    for (int r = 0; r < kWgradLoads; ++r, at += row_bytes) {
       if constexpr (VEC * sizeof(T) == 16) {
         const u32x4_v w = __builtin_amdgcn_raw_buffer_load_b128(buf, off[0] + at, 0, 0);
 #pragma unroll
@@ -96,11 +93,6 @@ template <typename T, int VEC> struct WgradRows {
   }
 };
 
-// Row r of a lane inside a step is wgrad_row0(group) + r * wgrad_row_step (the lanes of a 16-lane group share the
-// rows).
-template <typename T> __device__ __forceinline__ int wgrad_row0(int group) { return sizeof(T) == 2 ? group * 8 : group; }
-template <typename T> constexpr int wgrad_row_step = sizeof(T) == 2 ? 1 : 4;
-
 // Column of the output that element i (0..15) of tile fragment f stands for, relative to the tile.
 template <int VEC>
 __device__ __forceinline__ int wgrad_col(int f, int i) {
@@ -110,12 +102,17 @@ __device__ __forceinline__ int wgrad_col(int f, int i) {
 // MFMA operands of one step: fragment f = 16 columns, the lane's rows of one of them.
 template <typename T> struct WgradOperand;
 template <> struct WgradOperand<float> {
-  float v[kWgradFrags][4];
+  uint32_t v[3][kWgradFrags][4];   // the parts of eight values of a column, two rows to a register
   template <int VEC> __device__ __forceinline__ explicit WgradOperand(const WgradRows<float, VEC>& rows) {
 #pragma unroll
     for (int f = 0; f < kWgradFrags; ++f)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) v[f][r] = __uint_as_float(rows.v[r][f]);
+      for (int d = 0; d < 4; ++d) {
+        const SplitPair s = split_pair(__uint_as_float(rows.v[2 * d][f]), __uint_as_float(rows.v[2 * d + 1][f]));
+        v[0][f][d] = s.hi;
+        v[1][f][d] = s.mid;
+        v[2][f][d] = s.lo;
+      }
   }
 };
 template <> struct WgradOperand<uint16_t> {
@@ -134,20 +131,20 @@ template <> struct WgradOperand<uint16_t> {
 
 // acc[fa][fb] += a[fa]^T b[fb] over the step's rows; products of one accumulator are kept apart (a chain of them
 // would wait for each other).
-__device__ __forceinline__ void wgrad_products(const WgradOperand<float>& a, const WgradOperand<float>& b,
-                                               f32x4_t (&acc)[kWgradFrags][kWgradFrags]) {
-#pragma unroll
-  for (int r = 0; r < 4; ++r)
-#pragma unroll
-    for (int fa = 0; fa < kWgradFrags; ++fa)
-#pragma unroll
-      for (int fb = 0; fb < kWgradFrags; ++fb)
-        acc[fa][fb] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.v[fa][r], b.v[fb][r], acc[fa][fb], 0, 0, 0);
-}
 __device__ __forceinline__ f32x4_t wgrad_mfma(const uint32_t (&a)[4], const uint32_t (&b)[4], f32x4_t acc) {
   const u32x4_v av = {a[0], a[1], a[2], a[3]}, bv = {b[0], b[1], b[2], b[3]};
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, av), __builtin_bit_cast(bf16x8_t, bv), acc,
                                                  0, 0, 0);
+}
+__device__ __forceinline__ void wgrad_products(const WgradOperand<float>& a, const WgradOperand<float>& b,
+                                               f32x4_t (&acc)[kWgradFrags][kWgradFrags]) {
+#pragma unroll
+  for (int t = 0; t < kSplitProducts; ++t)
+#pragma unroll
+    for (int fa = 0; fa < kWgradFrags; ++fa)
+#pragma unroll
+      for (int fb = 0; fb < kWgradFrags; ++fb)
+        acc[fa][fb] = wgrad_mfma(a.v[kSplitA[t]][fa], b.v[kSplitB[t]][fb], acc[fa][fb]);
 }
 __device__ __forceinline__ void wgrad_products(const WgradOperand<uint16_t>& a, const WgradOperand<uint16_t>& b,
                                                f32x4_t (&acc)[kWgradFrags][kWgradFrags]) {
@@ -157,23 +154,26 @@ __device__ __forceinline__ void wgrad_products(const WgradOperand<uint16_t>& a, 
     for (int fb = 0; fb < kWgradFrags; ++fb) acc[fa][fb] = wgrad_mfma(a.v[fa], b.v[fb], acc[fa][fb]);
 }
 // Column sums of dy.  bf16: a product with ones (4 more MFMAs beside 16; unpacking the halves would cost more), the
-// sum of column i in accumulator row i.  fp32: MFMAs are the bound, so the vector units add; the lane's sum covers
-// its own rows of columns l16.
-__device__ __forceinline__ void wgrad_sums(const WgradOperand<uint16_t>& a, f32x4_t (&sum)[kWgradFrags]) {
+// sum of column i in accumulator row i.  fp32: the vector units add; the lane's sum covers its own rows of columns l16.
+template <int VEC>
+__device__ __forceinline__ void wgrad_sums(const WgradRows<uint16_t, VEC>&, const WgradOperand<uint16_t>& a,
+                                           f32x4_t (&sum)[kWgradFrags]) {
   const uint32_t ones[4] = {0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u};
 #pragma unroll
   for (int f = 0; f < kWgradFrags; ++f) sum[f] = wgrad_mfma(a.v[f], ones, sum[f]);
 }
-__device__ __forceinline__ void wgrad_sums(const WgradOperand<float>& a, f32x4_t (&sum)[kWgradFrags]) {
+template <int VEC>
+__device__ __forceinline__ void wgrad_sums(const WgradRows<float, VEC>& rows, const WgradOperand<float>&,
+                                           f32x4_t (&sum)[kWgradFrags]) {
 #pragma unroll
   for (int f = 0; f < kWgradFrags; ++f)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) sum[f][r] += a.v[f][r];
+    for (int r = 0; r < kWgradLoads; ++r) sum[f][r & 1] += __uint_as_float(rows.v[r][f]);
 }
 
 template <typename T, int VA, int VB>
 __global__ __launch_bounds__(kWgradWaves * kWave) void wgrad_kernel(WgradParams p) {
-  constexpr int kRows = WgradType<T>::kRows;
+  constexpr int kRows = kWgradRows;
   const int lane = threadIdx.x % kWave;
   const int l16 = lane % 16, group = lane / 16;
   // A wavefront has one tile of one split.  The workgroups of a split read the same rows: they are numbered eight
@@ -203,41 +203,82 @@ __global__ __launch_bounds__(kWgradWaves * kWave) void wgrad_kernel(WgradParams 
   uint32_t off_a[kWgradFrags / VA], off_b[kWgradFrags / VB];
 #pragma unroll
   for (int o = 0; o < kWgradFrags / VA; ++o)
-    off_a[o] = static_cast<uint32_t>((wgrad_row0<T>(group) * p.n + n0 + wgrad_col<VA>(o * VA, l16)) * sizeof(T));
+    off_a[o] = static_cast<uint32_t>((group * kWgradLoads * p.n + n0 + wgrad_col<VA>(o * VA, l16)) * sizeof(T));
 #pragma unroll
   for (int o = 0; o < kWgradFrags / VB; ++o)
-    off_b[o] = static_cast<uint32_t>((wgrad_row0<T>(group) * p.k + k0 + wgrad_col<VB>(o * VB, l16)) * sizeof(T));
-  const uint32_t row_a = static_cast<uint32_t>(wgrad_row_step<T> * p.n * sizeof(T)),
-                 row_b = static_cast<uint32_t>(wgrad_row_step<T> * p.k * sizeof(T));
+    off_b[o] = static_cast<uint32_t>((group * kWgradLoads * p.k + k0 + wgrad_col<VB>(o * VB, l16)) * sizeof(T));
+  const uint32_t row_a = static_cast<uint32_t>(p.n * sizeof(T)), row_b = static_cast<uint32_t>(p.k * sizeof(T));
   const uint32_t step_a = static_cast<uint32_t>(kRows * p.n * sizeof(T)), step_b = static_cast<uint32_t>(kRows * p.k * sizeof(T));
   f32x4_t acc[kWgradFrags][kWgradFrags] = {};
   f32x4_t sum[kWgradFrags] = {};
   const bool bias = tile % p.tiles_k == 0;
 
-  auto multiply = [&](const WgradRows<T, VA>& a, const WgradRows<T, VB>& b) {
-    const WgradOperand<T> oa(a), ob(b);
-    wgrad_products(oa, ob, acc);
-    if (bias) wgrad_sums(oa, sum);
-  };
-  // Two steps in registers: the rows of one are on their way during the products of the other.  A step past the
-  // split's end reads zeros.
-  WgradRows<T, VA> a0, a1;
-  WgradRows<T, VB> b0, b1;
   const int steps = static_cast<int>((m1 - m0 + kRows - 1) / kRows);
   uint32_t at_a = 0, at_b = 0;
+  WgradRows<T, VA> a0;
+  WgradRows<T, VB> b0;
   a0.load(dy, at_a, row_a, off_a);
   b0.load(x, at_b, row_b, off_b);
-  for (int s = 0; s < steps; s += 2) {
-    at_a += step_a;
-    at_b += step_b;
-    a1.load(dy, at_a, row_a, off_a);
-    b1.load(x, at_b, row_b, off_b);
-    multiply(a0, b0);
-    at_a += step_a;
-    at_b += step_b;
-    a0.load(dy, at_a, row_a, off_a);
-    b0.load(x, at_b, row_b, off_b);
-    multiply(a1, b1);
+  if constexpr (sizeof(T) == 4) {
+    // The parts take the place of the second step's rows (registers): the next rows are on their way during the products.
+    for (int s = 0; s < steps; ++s) {
+      const WgradOperand<T> oa(a0), ob(b0);
+      if (bias) wgrad_sums(a0, oa, sum);
+      at_a += step_a;
+      at_b += step_b;
+      a0.load(dy, at_a, row_a, off_a);
+      b0.load(x, at_b, row_b, off_b);
+      wgrad_products(oa, ob, acc);
+    }
+    bool finite = true;
+#pragma unroll
+    for (int fa = 0; fa < kWgradFrags; ++fa)
+#pragma unroll
+      for (int fb = 0; fb < kWgradFrags; ++fb)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) finite &= __builtin_isfinite(acc[fa][fb][q]);
+    if (__any(!finite)) {   // again with the fp32 instruction (rows r, 8 + r, 16 + r, 24 + r of a step at a time)
+#pragma unroll
+      for (int fa = 0; fa < kWgradFrags; ++fa)
+#pragma unroll
+        for (int fb = 0; fb < kWgradFrags; ++fb) acc[fa][fb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      at_a = at_b = 0;
+#pragma unroll 1
+      for (int s = 0; s < steps; ++s, at_a += step_a, at_b += step_b) {
+        a0.load(dy, at_a, row_a, off_a);
+        b0.load(x, at_b, row_b, off_b);
+#pragma unroll
+        for (int r = 0; r < kWgradLoads; ++r)
+#pragma unroll
+          for (int fa = 0; fa < kWgradFrags; ++fa)
+#pragma unroll
+            for (int fb = 0; fb < kWgradFrags; ++fb)
+              acc[fa][fb] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a0.v[r][fa]), __uint_as_float(b0.v[r][fb]),
+                                                                 acc[fa][fb], 0, 0, 0);
+      }
+    }
+  } else {
+    auto multiply = [&](const WgradRows<T, VA>& a, const WgradRows<T, VB>& b) {
+      const WgradOperand<T> oa(a), ob(b);
+      wgrad_products(oa, ob, acc);
+      if (bias) wgrad_sums(a, oa, sum);
+    };
+    // Two steps in registers: the rows of one are on their way during the products of the other.  A step past the
+    // split's end reads zeros.
+    WgradRows<T, VA> a1;
+    WgradRows<T, VB> b1;
+    for (int s = 0; s < steps; s += 2) {
+      at_a += step_a;
+      at_b += step_b;
+      a1.load(dy, at_a, row_a, off_a);
+      b1.load(x, at_b, row_b, off_b);
+      multiply(a0, b0);
+      at_a += step_a;
+      at_b += step_b;
+      a0.load(dy, at_a, row_a, off_a);
+      b0.load(x, at_b, row_b, off_b);
+      multiply(a1, b1);
+    }
   }
   // Element q of a lane's accumulator is row (dy column) group * 4 + q, column (x column) l16 of the tile fragment.
   float* part = p.part + static_cast<int64_t>(split) * p.part_stride;
@@ -257,7 +298,7 @@ __global__ __launch_bounds__(kWgradWaves * kWave) void wgrad_kernel(WgradParams 
   if (sizeof(T) == 4 && bias) {
 #pragma unroll
     for (int f = 0; f < kWgradFrags; ++f) {
-      float v = (sum[f][0] + sum[f][1]) + (sum[f][2] + sum[f][3]);
+      float v = sum[f][0] + sum[f][1];
       v += __shfl_xor(v, 16, kWave);
       v += __shfl_xor(v, 32, kWave);
       const int64_t n = n0 + wgrad_col<VA>(f, l16);
@@ -270,10 +311,10 @@ __global__ __launch_bounds__(kWgradWaves * kWave) void wgrad_kernel(WgradParams 
 // its loop and the partials (written once, read once) stay below half of the inputs they come from or a few
 // megabytes.  Both launches, against the library's GEMM and column sum, for n x k = 256 x 128:
 //   rows      bf16: here / library     fp32: here / library
-//   256              18 / 27 us              21 / 42 us
-//   17 k             25 / 108 us             40 / 120 us
-//   170 k            46 / 403 us            118 / 350 us   (bytes alone 26 / 52 us; the fp32 products 72 us)
-//   700 k           171 / 1435 us           431 / 1378 us
+//   256              18 / 27 us              20 / 42 us
+//   17 k             25 / 108 us             33 / 120 us     (fp32 instruction:  40)
+//   170 k            46 / 403 us            101 / 358 us     (118; bytes alone 52, products 66 at the bf16 rate)
+//   700 k           171 / 1435 us           436 / 1385 us    (431)
 static void wgrad_shape(int64_t m, int64_t n, int64_t k, int elem_size, WgradParams& p) {
   const int64_t tiles_n = ceil_div(n, kWgradTile);
   p.tiles_k = static_cast<int>(ceil_div(k, kWgradTile));
@@ -287,8 +328,7 @@ static void wgrad_shape(int64_t m, int64_t n, int64_t k, int elem_size, WgradPar
   s = std::max<int64_t>(1, std::min(s, ceil_div(m, kWgradMinRows)));
   // a split's rows are addressed with 32-bit offsets, and the loop reads up to three steps past its last one
   s = std::max(s, ceil_div(m * std::max(n, k) * elem_size, int64_t{1} << 30));
-  const int64_t step = elem_size == 2 ? WgradType<uint16_t>::kRows : WgradType<float>::kRows;
-  p.rows_per_split = ceil_div(ceil_div(m, s), step) * step;
+  p.rows_per_split = ceil_div(ceil_div(m, s), kWgradRows) * kWgradRows;
   p.splits = static_cast<int>(ceil_div(m, p.rows_per_split));
 }
 

@@ -4,11 +4,10 @@
 // A GraphSAGE layer is the sum of two such products and its gradient towards the features is another; one pass
 // over the result saves writing one product, adding the other and, backward, a zero-filled copy of the rows.
 //
-// fp32 operands are split into three bf16 parts (8 + 8 + 8 bits, rounded to nearest: the parts add up to the value)
-// and six of the nine partial products are formed on the bf16 matrix units with fp32 accumulators; what is left out is
-// below 2^-25 of a product.  The six take less than half the time of the fp32 matrix instruction, whose rate (157
-// TFLOP/s, one sixteenth of bf16's) bounds these products otherwise.  A result that is not finite is formed again with
-// the fp32 instruction: the parts of an infinity, or of a value that rounds to one in bf16, would make NaNs.
+// fp32 operands are split into three bf16 parts (split_bf16.hpp) and multiplied on the bf16 matrix units with fp32
+// accumulators: six products take less than half the time of the fp32 matrix instruction, whose rate (157 TFLOP/s, one
+// sixteenth of bf16's) bounds these products otherwise.  A result that is not finite is formed again with that
+// instruction.
 //
 // Tile: a workgroup has 64 x (64 or 16) result elements per wavefront; the rows go through LDS, already split (every
 // wavefront of a row range shares them), and the weights come from the workspace, where rows_gemm_weights_kernel left
@@ -25,6 +24,7 @@
 #include <algorithm>
 
 #include "common.hpp"
+#include "split_bf16.hpp"
 
 namespace apt {
 
@@ -57,27 +57,6 @@ struct GemmParams {
   float* y;
 };
 
-// Two fp32 values as three pairs of bf16.
-struct SplitPair {
-  uint32_t hi, mid, lo;
-};
-typedef __bf16 gemm_bf16x2 __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ uint32_t bf16_pair(float a, float b) {
-  const gemm_bf16x2 v = {static_cast<__bf16>(a), static_cast<__bf16>(b)};
-  return __builtin_bit_cast(uint32_t, v);
-}
-__device__ __forceinline__ SplitPair split_pair(float a, float b) {
-  SplitPair s;
-  s.hi = bf16_pair(a, b);
-  a -= __uint_as_float(s.hi << 16);
-  b -= __uint_as_float(s.hi & 0xffff0000u);
-  s.mid = bf16_pair(a, b);
-  a -= __uint_as_float(s.mid << 16);
-  b -= __uint_as_float(s.mid & 0xffff0000u);
-  s.lo = bf16_pair(a, b);
-  return s;
-}
-
 __device__ __forceinline__ float gemm_weight(const GemmParams& p, int64_t n, int64_t k) {
   if (n >= p.n) return 0.f;
   if (k < p.k1) return p.w1.w[n * p.w1.stride_n + k * p.w1.stride_k];
@@ -94,9 +73,18 @@ __global__ __launch_bounds__(kGemmBlock) void rows_gemm_weights_kernel(GemmParam
   const int64_t n = frag % p.frags * 16 + lane % 16;
   const int64_t k = frag / p.frags * kGemmStep + lane / 16 * 8;
   gemm_u32x4 part[kGemmParts];
+  float w[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {   // all on their way together: the address of a missing element is one that exists
+    const bool first = k + j < p.k1, in = n < p.n && k + j < p.k1 + p.k2;
+    const int64_t kj = first ? k + j : k + j - p.k1;
+    const float* at = first ? p.w1.w + n * p.w1.stride_n + kj * p.w1.stride_k : p.w2.w + n * p.w2.stride_n + kj * p.w2.stride_k;
+    w[j] = *(in ? at : p.w1.w);
+  }
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    const SplitPair s = split_pair(gemm_weight(p, n, k + 2 * j), gemm_weight(p, n, k + 2 * j + 1));
+    const bool in0 = n < p.n && k + 2 * j < p.k1 + p.k2, in1 = n < p.n && k + 2 * j + 1 < p.k1 + p.k2;
+    const SplitPair s = split_pair(in0 ? w[2 * j] : 0.f, in1 ? w[2 * j + 1] : 0.f);
     part[0][j] = s.hi;
     part[1][j] = s.mid;
     part[2][j] = s.lo;
@@ -194,13 +182,12 @@ __global__ __launch_bounds__(kGemmBlock, 2) void rows_gemm_kernel(GemmParams p) 
       for (int q = 0; q < kGemmParts; ++q)
         x[q] = *reinterpret_cast<const gemm_u32x4*>(&s_x[buf][q][((wm * MF + m) * kWave + lane) * 4]);
       // A step's products are added up on their own, the small ones first: one rounding of the long sum per step
-      constexpr int kPartW[6] = {2, 0, 1, 1, 0, 0}, kPartX[6] = {0, 2, 1, 0, 1, 0};
       gemm_f32x4 sum[kGemmFragsN];
 #pragma unroll
-      for (int t = 0; t < 6; ++t)
+      for (int t = 0; t < kSplitProducts; ++t)
 #pragma unroll
         for (int f = 0; f < kGemmFragsN; ++f)
-          sum[f] = gemm_mfma(v[f][kPartW[t]], x[kPartX[t]], t == 0 ? gemm_f32x4{0.f, 0.f, 0.f, 0.f} : sum[f]);
+          sum[f] = gemm_mfma(v[f][kSplitA[t]], x[kSplitB[t]], t == 0 ? gemm_f32x4{0.f, 0.f, 0.f, 0.f} : sum[f]);
 #pragma unroll
       for (int f = 0; f < kGemmFragsN; ++f) acc[m][f] += sum[f];
     }
