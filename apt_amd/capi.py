@@ -127,18 +127,19 @@ SYMBOLS = {
     "apt_spmm_heads": (_I, [_P, _P, _I64, _P, _I64, _P, _P, _I, _I64, _I, _I, _P, _I64, _P, _P, _P, _P]),
     "apt_block_transpose_workspace_bytes": (_SZ, [_I64, _I, _I64]),
     "apt_block_transpose": (_I, [_P, _I64, _I, _I64, _P, _P, _P, _SZ, _P]),
-    "apt_block_aggregate": (_I, [_P, _I64, _I, _P, _I64, _I64, _I, _I, _P, _P, _P]),
-    "apt_block_aggregate_backward": (_I, [_P, _P, _I, _I, _I64, _P, _P, _I64, _I64, _I, _P, _P]),
+    "apt_block_aggregate": (_I, [_P, _I64, _I, _P, _I64, _I64, _I, _I, C.c_float, _P, _P, _I, _P, _P, _P]),
+    "apt_block_aggregate_backward": (_I, [_P, _P, _I, _I, _I64, _P, C.c_float, _P, _I64, _I64, _I, _P, _P]),
     "apt_coo_prepare": (_I, [_P, _P, _I64, _P, _P, _P, _I, _P, _P, _P, _P, _P]),
     "apt_coo_sum_workspace_bytes": (_SZ, [_I64, _I64, _I]),
     "apt_coo_sum": (_I, [_I, _P, _P, _I64, _I, _P, _I64, _P, _I64, _I, _P, _I64, _P, _SZ, _P]),
     "apt_coo_combine": (_I, [_I, _P, _P, _I64, _P, _I64, _P, _I64, _I64, _I, _P, _P, _P, _I, _P, _P]),
-    "apt_gat_layer": (_I, [_P, _I64, _I, _P, _I64, _I, _I64, _I, _P, _P, _I, _P, C.c_float, _P, _P, _P, _P, _P]),
+    "apt_gat_layer": (_I, [_P, _I64, _I, _P, _I64, _I, _I64, _I, _P, _P, _I, _P, _I, C.c_float, _P, _P, _P, _P, _P]),
     "apt_gat_layer_backward_workspace_bytes": (_SZ, [_I64, _I, _I64, _I, _I64, _I64]),
     "apt_gat_layer_backward": (_I, [_P, _I64, _I, _P, _I64, _I, _I64, _I, _P, _P, _I, C.c_float, _P, _P, _P, _P, _P, _P, _I, _P,
                                     _P, _I64, _P, _P, _P, _P, _P, _SZ, _P]),
+    "apt_add_rows": (_I, [_P, _P, _I64, _I, _I, _P]),
     "apt_rows_gemm_workspace_bytes": (_SZ, [_I64, _I64, _I64]),
-    "apt_rows_gemm": (_I, [_P, _I64, _P, _I64, _I64, _P, _I64, _P, _I64, _I64, _I64, _I64, _I64, _P, _I, _P, _P, _SZ, _P]),
+    "apt_rows_gemm": (_I, [_P, _I64, _P, _I64, _I64, _P, _I64, _P, _I64, _I64, _I64, _I64, _I64, _P, _I, _I, _P, _P, _SZ, _P]),
     "apt_linear_wgrad_workspace_bytes": (_SZ, [_I64, _I64, _I64, _I]),
     "apt_linear_wgrad": (_I, [_P, _P, _I64, _I64, _I64, _I, _P, _P, _P, _SZ, _P]),
     "apt_time_next_sample": (_I, [_I, _P, _P]),
@@ -1060,7 +1061,7 @@ def linear_wgrad(dy, x, want_bias=True):
     return dw, db
 
 
-def rows_gemm(x1, w1, x2=None, w2=None, bias=None, out=None):
+def rows_gemm(x1, w1, x2=None, w2=None, bias=None, out=None, relu=False):
     """x1 w1^T (+ x2 w2^T on the first rows) (+ bias) in fp32; out: added to.  Weights may have any strides."""
     x1 = x1.contiguous()
     x2 = None if x2 is None else x2.contiguous()
@@ -1081,5 +1082,5 @@ def rows_gemm(x1, w1, x2=None, w2=None, bias=None, out=None):
     ws = torch.empty(max(need, 256), dtype=torch.uint8, device=x1.device)
     s2 = (0, 0) if w2 is None else w2.stride()
     check(lib().apt_rows_gemm(_ptr(x1), k1, _ptr(w1), w1.stride(0), w1.stride(1), _ptr(x2), k2, _ptr(w2), s2[0], s2[1], m, m2,
-                              n, _ptr(bias), int(accumulate), _ptr(out), _ptr(ws), ws.numel(), _stream()))
+                              n, _ptr(bias), int(accumulate), int(relu), _ptr(out), _ptr(ws), ws.numel(), _stream()))
     return out

@@ -25,6 +25,7 @@ struct SourceSumParams {
   const int64_t* via;      // ... or, if given, via[slot]
   const void* edata;       // slots, optional: [slots, dim] of dz's type, multiplies the destination's row
   const float* dst_scale;  // per destination, or NULL
+  float scale;             // of every sum
   const void* dz;          // [num_dst, dim]
   int64_t num_dst;
   int64_t dim;
@@ -129,7 +130,11 @@ __global__ __launch_bounds__(kAggBlock) void source_sum_kernel(SourceSumParams p
         add_edges(first[q], min(n[q], LPR), c, live, acc);
         for (int e = LPR; e < n[q]; e += LPR)   // LPR < kHubEdges only
           add_edges(edge(lo[q] + e + l, e + l < n[q]), min(n[q] - e, LPR), c, live, acc);
-        if (live) store_vec<T, VEC>(dx, r * p.dim + c, acc);
+        if (live) {
+#pragma unroll
+          for (int k = 0; k < VEC; ++k) acc[k] *= p.scale;
+          store_vec<T, VEC>(dx, r * p.dim + c, acc);
+        }
       }
     }
 #pragma unroll
@@ -161,7 +166,7 @@ __global__ __launch_bounds__(kAggBlock) void source_sum_kernel(SourceSumParams p
           float sum = 0.f;
 #pragma unroll 1
           for (int g = 0; g < kGroups; ++g) sum += s_sum[g][l * VEC + k];
-          acc[k] = sum;
+          acc[k] = sum * p.scale;
         }
         store_vec<T, VEC>(dx, r * p.dim + c, acc);
       }
@@ -354,6 +359,7 @@ extern "C" int apt_coo_sum(int mode, const int64_t* keys, const int64_t* sources
     if (const int rc = apt_block_transpose(keys, num_edges, 1, num_out_rows, indptr, order, ws, left, stream)) return rc;
   }
   SourceSumParams p{};
+  p.scale = 1.f;
   p.indptr = indptr;
   p.index = order;
   p.fanout = 1;
@@ -368,7 +374,7 @@ extern "C" int apt_coo_sum(int mode, const int64_t* keys, const int64_t* sources
 }
 
 extern "C" int apt_block_aggregate_backward(const void* indptr, const void* index, int index_bytes, int fanout,
-                                            int64_t num_src, const float* dst_scale, const void* dz, int64_t num_dst,
+                                            int64_t num_src, const float* dst_scale, float scale, const void* dz, int64_t num_dst,
                                             int64_t dim, int elem_size, void* dx, void* stream) {
   using namespace apt;
   APT_REQUIRE(num_src >= 0 && num_src <= 0x7fffffffLL && num_dst >= 0 && dim > 0, APT_EINVAL,
@@ -386,6 +392,7 @@ extern "C" int apt_block_aggregate_backward(const void* indptr, const void* inde
   p.index = index;
   p.fanout = static_cast<uint32_t>(fanout);
   p.dst_scale = dst_scale;
+  p.scale = scale;
   p.dz = dz;
   p.num_dst = num_dst;
   p.dim = dim;

@@ -57,6 +57,9 @@ __device__ __forceinline__ float row_elem(const Row<T, VEC>& raw, int k) {
   else return to_float<T>(raw[k]);
 }
 
+// max(v, 0) as torch has it: NaN stays NaN.
+__device__ __forceinline__ float relu(float v) { return v < 0.f ? 0.f : v; }
+
 template <typename T, int VEC>
 __device__ __forceinline__ void store_vec(T* base, int64_t elem, const float (&v)[VEC]) {
   using P = typename Pack<T, VEC>::type;

@@ -22,7 +22,7 @@ namespace apt {
 
 int gat_block(const char* who, const int64_t* neighbors, int64_t num_dst, const int64_t* num_dst_dev, int fanout,
               const void* ft, int64_t num_src, int heads, int64_t dim, int elem_size, const float* el, const float* er,
-              float slope, void* out, bool like_input, float* attn_out, const void* bias, hipStream_t st);
+              float slope, void* out, bool like_input, float* attn_out, const void* bias, int act, hipStream_t st);
 int gat_edge_grad(const char* who, const int64_t* neighbors, int64_t num_dst, int fanout, const void* ft, int64_t num_src,
                   int heads, int64_t dim, int elem_size, const float* el, const float* er, float slope, const float* attn,
                   const void* d_out, bool like_input, const int64_t* csc_indptr, float* a_edge, float* dz_edge, float* d_er,
@@ -548,8 +548,8 @@ static size_t align256(size_t x) { return (x + 255) / 256 * 256; }
 
 extern "C" int apt_gat_layer(const int64_t* neighbors, int64_t num_dst, int fanout, const void* ft, int64_t num_src,
                              int heads, int64_t dim, int elem_size, const void* attn_l, const void* attn_r,
-                             int attn_elem_size, const void* bias, float negative_slope, float* el, float* er, void* out,
-                             float* attn_out, void* stream) {
+                             int attn_elem_size, const void* bias, int relu, float negative_slope, float* el, float* er,
+                             void* out,                             float* attn_out, void* stream) {
   using namespace apt;
   const char* who = "apt_gat_layer";
   APT_REQUIRE(num_dst >= 0 && num_dst <= num_src && fanout > 0 && heads > 0 && dim > 0, APT_EINVAL,
@@ -576,7 +576,7 @@ extern "C" int apt_gat_layer(const int64_t* neighbors, int64_t num_dst, int fano
   }
   APT_LAUNCH_CHECK("gat_pair_scores_kernel");
   return gat_block(who, neighbors, num_dst, nullptr, fanout, ft, num_src, heads, dim, elem_size, el, er, negative_slope, out,
-                   true, attn_out, bias, st);
+                   true, attn_out, bias, relu, st);
 }
 
 extern "C" size_t apt_gat_layer_backward_workspace_bytes(int64_t num_dst, int fanout, int64_t num_src, int heads, int64_t dim,

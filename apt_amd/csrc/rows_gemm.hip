@@ -24,6 +24,7 @@
 #include <algorithm>
 
 #include "common.hpp"
+#include "feature_rows.hpp"
 #include "split_bf16.hpp"
 
 namespace apt {
@@ -53,7 +54,7 @@ struct GemmParams {
   const gemm_u32x4* parts;   // [step][column fragment][part][lane]
   int frags;                 // column fragments: ceil(n / 64) * 4
   const float* bias;
-  int accumulate;
+  int accumulate, relu;
   float* y;
 };
 
@@ -268,6 +269,10 @@ __global__ __launch_bounds__(kGemmBlock, 2) void rows_gemm_kernel(GemmParams p) 
           for (int q = 0; q < 4; ++q) v[q] += p.bias[n + q];
         }
         if (p.accumulate) v += *reinterpret_cast<const gemm_f32x4*>(out);
+        if (p.relu) {
+#pragma unroll
+          for (int q = 0; q < 4; ++q) v[q] = relu(v[q]);
+        }
         *reinterpret_cast<gemm_f32x4*>(out) = v;
       } else {
 #pragma unroll
@@ -276,11 +281,37 @@ __global__ __launch_bounds__(kGemmBlock, 2) void rows_gemm_kernel(GemmParams p) 
           float v = acc[m][f][q];
           if (p.bias != nullptr) v += p.bias[n + q];
           if (p.accumulate) v += out[q];
+          if (p.relu) v = relu(v);
           out[q] = v;
         }
       }
     }
   }
+}
+
+// The sum of two products that the library formed, with the ReLU: one pass instead of two.
+template <typename T, int VEC>
+__global__ __launch_bounds__(kGemmBlock) void add_rows_kernel(T* __restrict__ y, const T* __restrict__ x, int64_t vecs,
+                                                              int act) {
+  for (int64_t i = static_cast<int64_t>(blockIdx.x) * kGemmBlock + threadIdx.x; i < vecs;
+       i += static_cast<int64_t>(gridDim.x) * kGemmBlock) {
+    float a[VEC], b[VEC];
+    load_vec<T, VEC>(y, i * VEC, a);
+    load_vec<T, VEC>(x, i * VEC, b);
+#pragma unroll
+    for (int k = 0; k < VEC; ++k) {
+      a[k] += b[k];
+      if (act) a[k] = relu(a[k]);
+    }
+    store_vec<T, VEC>(y, i * VEC, a);
+  }
+}
+
+template <typename T, int VEC>
+static void launch_add_rows(void* y, const void* x, int64_t count, int act, hipStream_t st) {
+  const int64_t vecs = count / VEC;
+  hipLaunchKernelGGL((add_rows_kernel<T, VEC>), dim3(static_cast<unsigned>(std::min<int64_t>(ceil_div(vecs, kGemmBlock), 1 << 16))),
+                     dim3(kGemmBlock), 0, st, static_cast<T*>(y), static_cast<const T*>(x), vecs, act);
 }
 
 static bool gemm_sizes_ok(int64_t m, int64_t m2, int64_t n, int64_t k1, int64_t k2) {
@@ -314,7 +345,7 @@ extern "C" size_t apt_rows_gemm_workspace_bytes(int64_t n, int64_t k1, int64_t k
 
 extern "C" int apt_rows_gemm(const float* x1, int64_t k1, const float* w1, int64_t w1_stride_n, int64_t w1_stride_k,
                              const float* x2, int64_t k2, const float* w2, int64_t w2_stride_n, int64_t w2_stride_k,
-                             int64_t m, int64_t m2, int64_t n, const float* bias, int accumulate, float* y,
+                             int64_t m, int64_t m2, int64_t n, const float* bias, int accumulate, int relu, float* y,
                              void* workspace, size_t workspace_bytes, void* stream) {
   using namespace apt;
   APT_REQUIRE(gemm_sizes_ok(m, m2, n, k1, k2), APT_ELIMIT, "apt_rows_gemm: sizes out of range (m %lld, m2 %lld, n %lld, k %lld + %lld)",
@@ -328,7 +359,7 @@ extern "C" int apt_rows_gemm(const float* x1, int64_t k1, const float* w1, int64
   APT_REQUIRE(n % 4 != 0 || (reinterpret_cast<uintptr_t>(y) & 15) == 0, APT_EINVAL, "apt_rows_gemm: y is not 16-byte aligned");
   hipStream_t st = static_cast<hipStream_t>(stream);
   GemmParams p{x1, x2, k1, k2, m, k2 > 0 ? m2 : 0, n, {w1, w1_stride_n, w1_stride_k}, {w2, w2_stride_n, w2_stride_k},
-               static_cast<const gemm_u32x4*>(workspace), gemm_frags(n), bias, accumulate, y};
+               static_cast<const gemm_u32x4*>(workspace), gemm_frags(n), bias, accumulate, relu, y};
   const int steps = static_cast<int>(ceil_div(k1 + k2, kGemmStep));
   hipLaunchKernelGGL(rows_gemm_weights_kernel,
                      dim3(static_cast<unsigned>(ceil_div(static_cast<int64_t>(steps) * p.frags * kWave, kGemmBlock))),
@@ -345,5 +376,24 @@ extern "C" int apt_rows_gemm(const float* x1, int64_t k1, const float* w1, int64
   else { APT_ROWS_GEMM(4); }
 #undef APT_ROWS_GEMM
   APT_LAUNCH_CHECK("rows_gemm_kernel");
+  return APT_OK;
+}
+
+extern "C" int apt_add_rows(void* y, const void* x, int64_t count, int elem_size, int relu, void* stream) {
+  using namespace apt;
+  APT_REQUIRE(count >= 0 && (elem_size == 2 || elem_size == 4), APT_EINVAL, "apt_add_rows: count %lld, elem_size %d",
+              (long long)count, elem_size);
+  if (count == 0) return APT_OK;
+  APT_REQUIRE(y != nullptr && x != nullptr, APT_EINVAL, "apt_add_rows: a tensor is NULL");
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  const bool wide = ((reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(x)) & 15) == 0;
+  if (elem_size == 4) {
+    if (wide && count % 4 == 0) launch_add_rows<float, 4>(y, x, count, relu, st);
+    else launch_add_rows<float, 1>(y, x, count, relu, st);
+  } else {
+    if (wide && count % 8 == 0) launch_add_rows<uint16_t, 8>(y, x, count, relu, st);
+    else launch_add_rows<uint16_t, 1>(y, x, count, relu, st);
+  }
+  APT_LAUNCH_CHECK("add_rows_kernel");
   return APT_OK;
 }

@@ -267,13 +267,20 @@ __global__ __launch_bounds__(kAggBlock) void sddmm_kernel(AggParams p, OUT* __re
 // edge.  A lane group owns a destination row, so there are no atomics, no
 // zero-fill and the sum order is fixed.  LPR lanes x VEC features cover `dim`.
 // OUT: fp32, or the input's type (a layer's result).  inv_degree, optional: 1 / number of valid slots per row.
+// What a layer does to the sum before it is stored comes along (a pass over the result each otherwise).
+struct EllEpilogue {
+  float scale;        // factor of the sum or mean
+  const void* bias;   // [dim] of OUT, or NULL
+  const void* base;   // [num_dst, dim] of OUT to add to, or NULL
+  int relu;
+};
 template <typename T, typename OUT, int VEC, int LPR>
 __global__ __launch_bounds__(kAggBlock) void spmm_ell_kernel(const int64_t* __restrict__ nbr,
                                                              int64_t num_dst, const int64_t* num_dst_dev,
                                                              int fanout, const T* __restrict__ x,
                                                              int64_t num_src, int64_t dim,
                                                              OUT* __restrict__ out, int mean,
-                                                             float* __restrict__ inv_degree) {
+                                                             float* __restrict__ inv_degree, EllEpilogue ep) {
   constexpr int kGroups = kAggBlock / LPR;
   constexpr int kUnroll = 5;
   const int64_t n = actual_count(num_dst, num_dst_dev);
@@ -313,10 +320,24 @@ __global__ __launch_bounds__(kAggBlock) void spmm_ell_kernel(const int64_t* __re
           for (int k = 0; k < VEC; ++k) acc[k] += row_elem<T, VEC>(v[u], k);
         }
       }
-      const float scale = (mean && cnt > 0) ? 1.0f / static_cast<float>(cnt) : 1.0f;
+      const float scale = (mean && cnt > 0 ? 1.0f / static_cast<float>(cnt) : 1.0f) * ep.scale;
       if (live) {
 #pragma unroll
-        for (int k = 0; k < VEC; ++k) acc[k] *= scale;
+        for (int k = 0; k < VEC; ++k) acc[k] = __fmul_rn(acc[k], scale);   // each step rounds, as operations of their own do
+        if (ep.bias != nullptr) {
+#pragma unroll
+          for (int k = 0; k < VEC; ++k) acc[k] = __fadd_rn(acc[k], to_float<OUT>(static_cast<const OUT*>(ep.bias)[d + k]));
+        }
+        if (ep.base != nullptr) {
+          float b[VEC];
+          load_vec<OUT, VEC>(static_cast<const OUT*>(ep.base), i * dim + d, b);
+#pragma unroll
+          for (int k = 0; k < VEC; ++k) acc[k] = __fadd_rn(as_stored<OUT>(acc[k]), b[k]);
+        }
+        if (ep.relu) {
+#pragma unroll
+          for (int k = 0; k < VEC; ++k) acc[k] = relu(acc[k]);
+        }
         store_vec<OUT, VEC>(out, i * dim + d, acc);
       }
       if (inv_degree != nullptr && d0 == 0 && l == 0) inv_degree[i] = 1.0f / static_cast<float>(cnt > 0 ? cnt : 1);
@@ -327,14 +348,14 @@ __global__ __launch_bounds__(kAggBlock) void spmm_ell_kernel(const int64_t* __re
 template <typename T, typename OUT, int VEC>
 static void launch_ell(const int64_t* nbr, int64_t num_dst, const int64_t* num_dst_dev, int fanout,
                        const void* x, int64_t num_src, int64_t dim, void* out, int mean, float* inv_degree,
-                       hipStream_t st) {
+                       EllEpilogue ep, hipStream_t st) {
   const int64_t per_row = ceil_div(dim, VEC);
   const T* xt = static_cast<const T*>(x);
 #define APT_ELL(LPR)                                                                                 \
   hipLaunchKernelGGL((spmm_ell_kernel<T, OUT, VEC, LPR>),                                             \
                      dim3(static_cast<unsigned>(std::min<int64_t>(ceil_div(num_dst, kAggBlock / LPR), 1 << 20))), \
                      dim3(kAggBlock), 0, st, nbr, num_dst, num_dst_dev, fanout, xt, num_src, dim, static_cast<OUT*>(out), mean, \
-                     inv_degree)
+                     inv_degree, ep)
   if (per_row <= 8) APT_ELL(8);
   else if (per_row <= 16) APT_ELL(16);
   else if (per_row <= 32) APT_ELL(32);
@@ -408,7 +429,7 @@ __global__ __launch_bounds__(kAggBlock) void gat_ell_kernel(const int64_t* __res
                                                             const float* __restrict__ er, float slope,
                                                             OUT* __restrict__ out,
                                                             float* __restrict__ attn_out,
-                                                            const OUT* __restrict__ bias) {
+                                                            const OUT* __restrict__ bias, int act) {
   constexpr int kGroups = kAggBlock / LPR;
   constexpr int kUnroll = 5;
   const int64_t n = actual_count(num_dst, num_dst_dev);
@@ -466,6 +487,7 @@ __global__ __launch_bounds__(kAggBlock) void gat_ell_kernel(const int64_t* __res
       for (int k = 0; k < VEC; ++k) {
         acc[k] *= inv;
         if (bias != nullptr) acc[k] = as_stored<OUT>(acc[k]) + to_float<OUT>(bias[d + k]);
+        if (act) acc[k] = relu(acc[k]);
       }
       store_vec<OUT, VEC>(out, i * row_len + d, acc);
       // the lane that holds a head's first features also writes its attention weights
@@ -498,7 +520,7 @@ __global__ __launch_bounds__(kAggBlock) void gat_ell_wave_kernel(
     const int64_t* __restrict__ nbr, int64_t num_dst, const int64_t* num_dst_dev, int fanout,
     const T* __restrict__ ft, int64_t num_src, int heads, int log2_heads, int64_t dim,
     const float* __restrict__ el, const float* __restrict__ er, float slope, OUT* __restrict__ out,
-    float* __restrict__ attn_out, const OUT* __restrict__ bias) {
+    float* __restrict__ attn_out, const OUT* __restrict__ bias, int act) {
   constexpr int kUnroll = 5;
   const int64_t n = actual_count(num_dst, num_dst_dev);
   const int lane = threadIdx.x % kWave;
@@ -552,6 +574,10 @@ __global__ __launch_bounds__(kAggBlock) void gat_ell_wave_kernel(
 #pragma unroll
         for (int q = 0; q < VEC; ++q) acc[q] = as_stored<OUT>(acc[q]) + to_float<OUT>(bias[d + q]);
       }
+      if (act) {
+#pragma unroll
+        for (int q = 0; q < VEC; ++q) acc[q] = relu(acc[q]);
+      }
       store_vec<OUT, VEC>(out, i * row_len + d, acc);
     }
   }
@@ -560,7 +586,7 @@ __global__ __launch_bounds__(kAggBlock) void gat_ell_wave_kernel(
 template <typename T, typename OUT, int VEC>
 static bool launch_gat_wave(const int64_t* nbr, int64_t num_dst, const int64_t* num_dst_dev, int fanout,
                             const void* ft, int64_t num_src, int heads, int64_t dim, const float* el,
-                            const float* er, float slope, void* out, float* attn_out, const void* bias, hipStream_t st) {
+                            const float* er, float slope, void* out, float* attn_out, const void* bias, int act, hipStream_t st) {
   if (num_src == 0) return false;   // the kernel reads a row for every slot
   if (dim % VEC != 0 || (heads & (heads - 1)) != 0 || heads * fanout > kWave) return false;
   const int64_t lph = dim / VEC;
@@ -570,21 +596,21 @@ static bool launch_gat_wave(const int64_t* nbr, int64_t num_dst, const int64_t* 
   const unsigned blocks = static_cast<unsigned>(std::min<int64_t>(ceil_div(num_dst, kAggWaves), 1 << 20));
   hipLaunchKernelGGL((gat_ell_wave_kernel<T, OUT, VEC>), dim3(blocks), dim3(kAggBlock), 0, st, nbr, num_dst, num_dst_dev,
                      fanout, static_cast<const T*>(ft), num_src, heads, log2_heads, dim, el, er, slope,
-                     static_cast<OUT*>(out), attn_out, static_cast<const OUT*>(bias));
+                     static_cast<OUT*>(out), attn_out, static_cast<const OUT*>(bias), act);
   return true;
 }
 
 template <typename T, typename OUT, int VEC>
 static void launch_gat(const int64_t* nbr, int64_t num_dst, const int64_t* num_dst_dev, int fanout,
                        const void* ft, int64_t num_src, int heads, int64_t dim, const float* el,
-                       const float* er, float slope, void* out, float* attn_out, const void* bias, hipStream_t st) {
+                       const float* er, float slope, void* out, float* attn_out, const void* bias, int act, hipStream_t st) {
   const int64_t per_row = ceil_div(static_cast<int64_t>(heads) * dim, VEC);
   const T* x = static_cast<const T*>(ft);
 #define APT_GAT(LPR)                                                                                  \
   hipLaunchKernelGGL((gat_ell_kernel<T, OUT, VEC, LPR>),                                              \
                      dim3(static_cast<unsigned>(std::min<int64_t>(ceil_div(num_dst, kAggBlock / LPR), 1 << 20))), \
                      dim3(kAggBlock), 0, st, nbr, num_dst, num_dst_dev, fanout, x, num_src, heads, dim, el, er, \
-                     slope, static_cast<OUT*>(out), attn_out, static_cast<const OUT*>(bias))
+                     slope, static_cast<OUT*>(out), attn_out, static_cast<const OUT*>(bias), act)
   if (per_row <= 8) APT_GAT(8);
   else if (per_row <= 16) APT_GAT(16);
   else if (per_row <= 32) APT_GAT(32);
@@ -984,7 +1010,7 @@ extern "C" int apt_coo_combine(int op, const int64_t* coo_row, const int64_t* co
 namespace apt {
 static int block_sum(const char* who, const int64_t* neighbors, int64_t num_dst, const int64_t* num_dst_dev, int fanout,
                      const void* input, int64_t num_src, int64_t dim, int elem_size, int mean, void* out, bool out_like_input,
-                     float* inv_degree, void* stream) {
+                     float* inv_degree, EllEpilogue ep, void* stream) {
   APT_REQUIRE(num_dst >= 0 && fanout > 0 && dim > 0 && num_src >= 0, APT_EINVAL,
               "%s: bad shape (num_dst %lld, fanout %d, dim %lld)", who, (long long)num_dst, fanout, (long long)dim);
   APT_REQUIRE(elem_size == 2 || elem_size == 4, APT_EINVAL, "%s: elem_size %d (4 = fp32, 2 = bf16)", who, elem_size);
@@ -994,9 +1020,9 @@ static int block_sum(const char* who, const int64_t* neighbors, int64_t num_dst,
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (num_src == 0) input = out;   // no edge is valid: the kernel reads a row, and uses none
   const bool vec4 = dim % 4 == 0 && (reinterpret_cast<uintptr_t>(input) & 15) == 0 &&
-                    (reinterpret_cast<uintptr_t>(out) & 15) == 0;
+                    ((reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(ep.base)) & 15) == 0;
 #define APT_BLOCK_SUM(T, OUT, V) \
-  launch_ell<T, OUT, V>(neighbors, num_dst, num_dst_dev, fanout, input, num_src, dim, out, mean, inv_degree, st)
+  launch_ell<T, OUT, V>(neighbors, num_dst, num_dst_dev, fanout, input, num_src, dim, out, mean, inv_degree, ep, st)
 #define APT_BLOCK_SUM_BF16(OUT)                                   \
   if (vec4 && dim % 8 == 0) APT_BLOCK_SUM(uint16_t, OUT, 8);      \
   else if (vec4) APT_BLOCK_SUM(uint16_t, OUT, 4);                 \
@@ -1020,14 +1046,14 @@ extern "C" int apt_spmm_block(const int64_t* neighbors, int64_t num_dst, const i
                               int fanout, const void* input, int64_t num_src, int64_t dim, int elem_size,
                               int mean, float* out, void* stream) {
   return apt::block_sum("apt_spmm_block", neighbors, num_dst, num_dst_dev, fanout, input, num_src, dim, elem_size, mean,
-                        out, false, nullptr, stream);
+                        out, false, nullptr, apt::EllEpilogue{1.f, nullptr, nullptr, 0}, stream);
 }
 
 extern "C" int apt_block_aggregate(const int64_t* neighbors, int64_t num_dst, int fanout, const void* input,
-                                   int64_t num_src, int64_t dim, int elem_size, int mean, void* out, float* inv_degree,
-                                   void* stream) {
+                                   int64_t num_src, int64_t dim, int elem_size, int mean, float scale, const void* bias,
+                                   const void* base, int relu, void* out, float* inv_degree, void* stream) {
   return apt::block_sum("apt_block_aggregate", neighbors, num_dst, nullptr, fanout, input, num_src, dim, elem_size, mean,
-                        out, true, inv_degree, stream);
+                        out, true, inv_degree, apt::EllEpilogue{scale, bias, base, relu}, stream);
 }
 
 extern "C" int apt_gat_scores(const void* x, int64_t num_rows, int heads, int64_t dim, int elem_size,
@@ -1083,14 +1109,14 @@ namespace apt {
 template <typename T, typename OUT>
 static void gat_block_as(const int64_t* neighbors, int64_t num_dst, const int64_t* num_dst_dev, int fanout, const void* ft,
                          int64_t num_src, int heads, int64_t dim, const float* el, const float* er, float slope, void* out,
-                         float* attn_out, const void* bias, hipStream_t st) {
+                         float* attn_out, const void* bias, int act, hipStream_t st) {
   const bool vec4 = dim % 4 == 0 && ((reinterpret_cast<uintptr_t>(ft) | reinterpret_cast<uintptr_t>(out)) & 15) == 0;
   if (vec4 && num_src > 0 &&
       launch_gat_wave<T, OUT, 4>(neighbors, num_dst, num_dst_dev, fanout, ft, num_src, heads, dim, el, er, slope, out,
-                                 attn_out, bias, st))
+                                 attn_out, bias, act, st))
     return;
 #define APT_GAT_BLOCK(V) \
-  launch_gat<T, OUT, V>(neighbors, num_dst, num_dst_dev, fanout, ft, num_src, heads, dim, el, er, slope, out, attn_out, bias, st)
+  launch_gat<T, OUT, V>(neighbors, num_dst, num_dst_dev, fanout, ft, num_src, heads, dim, el, er, slope, out, attn_out, bias, act, st)
   if constexpr (sizeof(T) == 2) {
     if (vec4 && dim % 8 == 0) {
       APT_GAT_BLOCK(8);
@@ -1105,7 +1131,7 @@ static void gat_block_as(const int64_t* neighbors, int64_t num_dst, const int64_
 // out: fp32 without a bias, or (like_input) the input's type with one.  Shared with the GAT layer (gat_layer.hip).
 int gat_block(const char* who, const int64_t* neighbors, int64_t num_dst, const int64_t* num_dst_dev, int fanout,
               const void* ft, int64_t num_src, int heads, int64_t dim, int elem_size, const float* el, const float* er,
-              float slope, void* out, bool like_input, float* attn_out, const void* bias, hipStream_t st) {
+              float slope, void* out, bool like_input, float* attn_out, const void* bias, int act, hipStream_t st) {
   APT_REQUIRE(num_dst >= 0 && fanout > 0 && heads > 0 && dim > 0 && num_src >= 0, APT_EINVAL,
               "%s: bad shape (num_dst %lld, fanout %d, heads %d, dim %lld)", who, (long long)num_dst, fanout, heads,
               (long long)dim);
@@ -1114,7 +1140,7 @@ int gat_block(const char* who, const int64_t* neighbors, int64_t num_dst, const 
   APT_REQUIRE(neighbors != nullptr && out != nullptr && er != nullptr && ((ft != nullptr && el != nullptr) || num_src == 0),
               APT_EINVAL, "%s: a tensor is NULL", who);
 #define APT_GAT_AS(T, OUT) \
-  gat_block_as<T, OUT>(neighbors, num_dst, num_dst_dev, fanout, ft, num_src, heads, dim, el, er, slope, out, attn_out, bias, st)
+  gat_block_as<T, OUT>(neighbors, num_dst, num_dst_dev, fanout, ft, num_src, heads, dim, el, er, slope, out, attn_out, bias, act, st)
   if (elem_size == 4) APT_GAT_AS(float, float);
   else if (like_input) APT_GAT_AS(uint16_t, uint16_t);
   else APT_GAT_AS(uint16_t, float);
@@ -1129,7 +1155,7 @@ extern "C" int apt_gat_block(const int64_t* neighbors, int64_t num_dst, const in
                              const float* el, const float* er, float negative_slope, float* out,
                              float* attn_out, void* stream) {
   return apt::gat_block("apt_gat_block", neighbors, num_dst, num_dst_dev, fanout, ft, num_src, heads, dim, elem_size, el, er,
-                        negative_slope, out, false, attn_out, nullptr, static_cast<hipStream_t>(stream));
+                        negative_slope, out, false, attn_out, nullptr, 0, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int apt_spmm_heads(const int64_t* coo_row, const int64_t* coo_col, int64_t num_edges,

@@ -986,7 +986,7 @@ std::tuple<Tensor, Tensor> linear_wgrad(const Tensor& dy_in, const Tensor& x_in,
 // x w^T (+ x2 w2^T on the first rows) (+ b) with w [n, k] of any strides; `onto`: added to (and returned).  fp32 rows
 // take apt_rows_gemm, bf16 rows, whose products are bound by memory in the library's kernels already, at::mm.
 Tensor dense(const Tensor& x_in, const Tensor& w, const Tensor& x2_in = Tensor(), const Tensor& w2 = Tensor(),
-             const Tensor& b = Tensor(), Tensor onto = Tensor()) {
+             const Tensor& b = Tensor(), Tensor onto = Tensor(), bool relu = false) {
   const int64_t m = x_in.size(0), k = x_in.size(1), n = w.size(0);
   const bool pair = x2_in.defined();
   const int64_t m2 = pair ? x2_in.size(0) : 0, k2 = pair ? x2_in.size(1) : 0;
@@ -1002,23 +1002,36 @@ Tensor dense(const Tensor& x_in, const Tensor& w, const Tensor& x2_in = Tensor()
     check(apt_rows_gemm(x.data_ptr<float>(), k, w.data_ptr<float>(), w.stride(0), w.stride(1),
                         pair ? x2.data_ptr<float>() : nullptr, k2, pair ? w2.data_ptr<float>() : nullptr,
                         pair ? w2.stride(0) : 0, pair ? w2.stride(1) : 0, m, m2, n,
-                        bias.defined() ? bias.data_ptr<float>() : nullptr, accumulate, y.data_ptr<float>(), ws.data_ptr(),
+                        bias.defined() ? bias.data_ptr<float>() : nullptr, accumulate, relu, y.data_ptr<float>(), ws.data_ptr(),
                         need, stream()));
     return y;
   }
   Tensor y = at::linear(x_in, w, b.defined() ? std::optional<Tensor>(b) : std::nullopt);
   if (pair) y.narrow(0, 0, m2).addmm_(x2_in, w2.t());
-  return onto.defined() ? onto.add_(y) : y;
+  if (onto.defined()) y = onto.add_(y);
+  return relu ? y.relu_() : y;
+}
+
+// Whether a call is part of a training step.  Its fp32 products are the library's: they give the bits of nn.Linear, and a
+// ReLU whose input changes sign with the last bit (one or two of 10^7) moves a weight's gradient by up to 6e-5.
+template <typename... Tensors>
+bool trains(const Tensors&... t) {
+  return torch::GradMode::is_enabled() && (t.requires_grad() || ...);
+}
+Tensor product(bool train, const Tensor& x, const Tensor& w, const Tensor& b = Tensor()) {
+  return train ? at::linear(x, w, b.defined() ? std::optional<Tensor>(b) : std::nullopt)
+               : dense(x, w, Tensor(), Tensor(), b);
 }
 
 // y = x w^T + b (or x w with `kn`: w is [k, n]).
 struct BlockLinearFn : public torch::autograd::Function<BlockLinearFn> {
   static Tensor forward(torch::autograd::AutogradContext* ctx, const Tensor& x, const Tensor& w,
-                        const std::optional<Tensor>& b, bool kn) {
+                        const std::optional<Tensor>& b, bool kn, bool train) {
     ctx->save_for_backward({x, w});
     ctx->saved_data["kn"] = kn;
     ctx->saved_data["bias"] = b.has_value();
-    return dense(x, kn ? w.t() : w, Tensor(), Tensor(), b.value_or(Tensor()));
+    if (train && kn) return at::mm(x, w);
+    return product(train, x, kn ? w.t() : w, b.value_or(Tensor()));
   }
   static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx,
                                                  torch::autograd::variable_list grads) {
@@ -1034,7 +1047,7 @@ struct BlockLinearFn : public torch::autograd::Function<BlockLinearFn> {
       if (ctx->needs_input_grad(0)) dx = dense(dy, kn ? w : w.t());
       if (ctx->needs_input_grad(1) || bias) std::tie(dw, db) = kn ? linear_wgrad(x, dy, false) : linear_wgrad(dy, x, bias);
     }
-    return {dx, dw, db, Tensor()};
+    return {dx, dw, db, Tensor(), Tensor()};
   }
 };
 
@@ -1045,7 +1058,7 @@ Tensor BlockLinear(const Tensor& x, const Tensor& w, const std::optional<Tensor>
                   (x.scalar_type() == torch::kFloat32 || x.scalar_type() == torch::kBFloat16),
               "npc: block_linear needs 2-D fp32 or bf16 GPU tensors of one dtype");
   TORCH_CHECK(!kn || !b.has_value(), "npc: block_linear: a [k, n] weight takes no bias");
-  return BlockLinearFn::apply(x, w, b, kn);
+  return BlockLinearFn::apply(x, w, b, kn, trains(x, w) || (b.has_value() && trains(*b)));
 }
 
 // ---------------------------------------------------------------- aggregation over a block, with its gradient
@@ -1094,7 +1107,7 @@ SourceOrder source_order(const Tensor& relabeled, int64_t num_dst, int64_t fanou
 
 // The gradient of the block sum / mean towards its input, from the block's CSR if it has one.
 Tensor aggregate_backward(const Tensor& dz_in, const Tensor& relabeled, int64_t num_dst, int64_t fanout, int64_t num_src,
-                          const Tensor& dst_scale, const Tensor& csr_indptr, const Tensor& csr_indices) {
+                          const Tensor& dst_scale, const Tensor& csr_indptr, const Tensor& csr_indices, float scale = 1.f) {
   auto dz = dz_in.contiguous();
   auto dx = torch::empty({num_src, dz.size(1)}, dz.options());
   SourceOrder o;
@@ -1106,19 +1119,21 @@ Tensor aggregate_backward(const Tensor& dz_in, const Tensor& relabeled, int64_t 
     o = source_order(relabeled, num_dst, fanout, num_src);
   }
   check(apt_block_aggregate_backward(o.indptr.data_ptr(), o.index.data_ptr(), o.bytes, static_cast<int>(fanout), num_src,
-                                     dst_scale.defined() ? dst_scale.data_ptr<float>() : nullptr, dz.data_ptr(), num_dst,
+                                     dst_scale.defined() ? dst_scale.data_ptr<float>() : nullptr, scale, dz.data_ptr(), num_dst,
                                      dz.size(1), static_cast<int>(dz.element_size()), dx.data_ptr(), stream()));
   return dx;
 }
 
 // -> (sum or mean, 1 / degree per destination when `mean`)
 std::tuple<Tensor, Tensor> aggregate_forward(const Tensor& relabeled, int64_t num_dst, int64_t fanout, const Tensor& x,
-                                             bool mean) {
+                                             bool mean, float scale = 1.f, const Tensor& bias = Tensor(), bool relu = false,
+                                             const Tensor& base = Tensor()) {
   auto out = torch::empty({num_dst, x.size(1)}, x.options());
   Tensor inv;
   if (mean) inv = torch::empty({num_dst}, x.options().dtype(torch::kFloat32));
   check(apt_block_aggregate(i64(relabeled), num_dst, static_cast<int>(fanout), x.data_ptr(), x.size(0), x.size(1),
-                            static_cast<int>(x.element_size()), mean, out.data_ptr(),
+                            static_cast<int>(x.element_size()), mean, scale, bias.defined() ? bias.data_ptr() : nullptr,
+                            base.defined() ? base.data_ptr() : nullptr, relu, out.data_ptr(),
                             mean ? inv.data_ptr<float>() : nullptr, stream()));
   return {out, inv};
 }
@@ -1159,25 +1174,39 @@ Tensor BlockAggregate(const Tensor& relabeled, int64_t num_dst, int64_t fanout, 
 // ---------------------------------------------------------------- GraphSAGE layer
 namespace {
 
+// The gradient towards what a layer's ReLU was applied to (`out`: its result; undefined: no ReLU).
+Tensor before_relu(const Tensor& grad, const Tensor& out) {
+  return (out.defined() ? at::threshold_backward(grad, out, 0) : grad).contiguous();
+}
+
 // x[:num_dst] w_self^T + bias + mean over the block of x, times w_neigh^T; the product comes before the mean where it
 // makes the rows shorter.  As one function the two products and their gradients are added up in the kernels that form
 // them: no pass over the result to add them, no zero-filled gradient of the destinations' rows.
 struct SageLayerFn : public torch::autograd::Function<SageLayerFn> {
   static Tensor forward(torch::autograd::AutogradContext* ctx, const Tensor& x, const Tensor& w_neigh, const Tensor& w_self,
                         const std::optional<Tensor>& bias, const Tensor& relabeled, int64_t num_dst, int64_t fanout,
-                        const std::optional<Tensor>& csr_indptr, const std::optional<Tensor>& csr_indices) {
+                        const std::optional<Tensor>& csr_indptr, const std::optional<Tensor>& csr_indices, bool relu,
+                        bool train) {
     const Tensor b = bias.value_or(Tensor()), self = x.narrow(0, 0, num_dst);
     const bool first = x.size(1) > w_self.size(0);
     Tensor mean, inv, out;
+    const bool apart = train || x.scalar_type() != torch::kFloat32;   // the products by the library
     if (first) {
-      std::tie(out, inv) = aggregate_forward(relabeled, num_dst, fanout, dense(x, w_neigh), true);
-      out = dense(self, w_self, Tensor(), Tensor(), b, out);
+      const Tensor base = product(apart, self, w_self, b);
+      std::tie(out, inv) = aggregate_forward(relabeled, num_dst, fanout, product(apart, x, w_neigh), true, 1.f, Tensor(), relu,
+                                             base);
     } else {
       std::tie(mean, inv) = aggregate_forward(relabeled, num_dst, fanout, x, true);
-      out = dense(self, w_self, mean, w_neigh, b);
+      if (apart) {
+        out = product(true, self, w_self, b);
+        const Tensor neigh = product(true, mean, w_neigh);
+        check(apt_add_rows(out.data_ptr(), neigh.data_ptr(), out.numel(), static_cast<int>(out.element_size()), relu, stream()));
+      } else {
+        out = dense(self, w_self, mean, w_neigh, b, Tensor(), relu);
+      }
     }
     ctx->save_for_backward({x, w_neigh, w_self, relabeled, inv, mean, csr_indptr.value_or(Tensor()),
-                            csr_indices.value_or(Tensor())});
+                            csr_indices.value_or(Tensor()), relu ? out : Tensor()});
     ctx->saved_data["bias"] = bias.has_value();
     ctx->saved_data["num_dst"] = num_dst;
     ctx->saved_data["fanout"] = fanout;
@@ -1193,7 +1222,7 @@ struct SageLayerFn : public torch::autograd::Function<SageLayerFn> {
     const auto spread = [&](const Tensor& d) {
       return aggregate_backward(d, relabeled, num_dst, fanout, num_src, inv, saved[6], saved[7]);
     };
-    const Tensor dz = grads[0].contiguous(), self = x.narrow(0, 0, num_dst);
+    const Tensor dz = before_relu(grads[0], saved[8]), self = x.narrow(0, 0, num_dst);
     const bool want_x = ctx->needs_input_grad(0), want_w = ctx->needs_input_grad(1) || ctx->needs_input_grad(2) || bias;
     Tensor dx, dwn, dws, db;
     if (torch::GradMode::is_enabled()) {   // a graph of the gradients is wanted: operations that carry one
@@ -1218,7 +1247,7 @@ struct SageLayerFn : public torch::autograd::Function<SageLayerFn> {
           return d;
         }();
     }
-    return {dx, dwn, dws, db, Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
+    return {dx, dwn, dws, db, Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
   }
 };
 
@@ -1226,7 +1255,7 @@ struct SageLayerFn : public torch::autograd::Function<SageLayerFn> {
 
 Tensor SageLayer(const Tensor& relabeled, int64_t num_dst, int64_t fanout, const Tensor& x, const Tensor& w_neigh,
                  const Tensor& w_self, const std::optional<Tensor>& bias, const std::optional<Tensor>& csr_indptr,
-                 const std::optional<Tensor>& csr_indices) {
+                 const std::optional<Tensor>& csr_indices, bool relu) {
   check_block("sage_layer", relabeled, num_dst, fanout);
   const auto t = x.scalar_type();
   TORCH_CHECK_TYPE(x.is_cuda() && x.dim() == 2 && (t == torch::kFloat32 || t == torch::kBFloat16),
@@ -1238,7 +1267,71 @@ Tensor SageLayer(const Tensor& relabeled, int64_t num_dst, int64_t fanout, const
                   (!bias.has_value() || (bias->is_cuda() && bias->scalar_type() == t && bias->dim() == 1 &&
                                          bias->size(0) == w_self.size(0))),
               "npc: sage_layer: weights, bias and input do not fit each other");
-  return SageLayerFn::apply(x.contiguous(), w_neigh, w_self, bias, relabeled, num_dst, fanout, csr_indptr, csr_indices);
+  return SageLayerFn::apply(x.contiguous(), w_neigh, w_self, bias, relabeled, num_dst, fanout, csr_indptr, csr_indices, relu,
+                            trains(x, w_neigh, w_self) || (bias.has_value() && trains(*bias)));
+}
+
+// ---------------------------------------------------------------- GCN layer
+namespace {
+
+// right * (sum over the block of (left * x) w) + bias, w [in, out]: the factors of the normalisation, of the rows before
+// and after.  Without gradients both are one factor of the sum (a training step keeps the bits of separate operations,
+// see `trains`); in the gradients they are one.  Factor, bias and ReLU are applied where the sum is stored.
+struct GcnLayerFn : public torch::autograd::Function<GcnLayerFn> {
+  static Tensor forward(torch::autograd::AutogradContext* ctx, const Tensor& x, const Tensor& w,
+                        const std::optional<Tensor>& bias, const Tensor& relabeled, int64_t num_dst, int64_t fanout,
+                        double left, double right, const std::optional<Tensor>& csr_indptr,
+                        const std::optional<Tensor>& csr_indices, bool relu, bool train) {
+    const Tensor b = bias.has_value() ? bias->contiguous() : Tensor();
+    const bool exact = train && x.scalar_type() == torch::kFloat32;
+    const Tensor h = exact ? at::mm(left == 1.0 ? x : at::mul(x, left), w) : dense(x, w.t());
+    const double scale = left * right;
+    const Tensor out = std::get<0>(aggregate_forward(relabeled, num_dst, fanout, h, false,
+                                                     static_cast<float>(exact ? right : scale), b, relu));
+    ctx->save_for_backward({x, w, relabeled, csr_indptr.value_or(Tensor()), csr_indices.value_or(Tensor()),
+                            relu ? out : Tensor()});
+    ctx->saved_data["bias"] = bias.has_value();
+    ctx->saved_data["num_dst"] = num_dst;
+    ctx->saved_data["fanout"] = fanout;
+    ctx->saved_data["scale"] = scale;
+    return out;
+  }
+  static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx,
+                                                 torch::autograd::variable_list grads) {
+    const auto saved = ctx->get_saved_variables();
+    const Tensor &x = saved[0], &w = saved[1];
+    const Tensor dz = before_relu(grads[0], saved[5]);
+    const Tensor dh = aggregate_backward(dz, saved[2], ctx->saved_data["num_dst"].toInt(), ctx->saved_data["fanout"].toInt(),
+                                         x.size(0), Tensor(), saved[3], saved[4],
+                                         static_cast<float>(ctx->saved_data["scale"].toDouble()));
+    Tensor dx, dw, db;
+    if (ctx->saved_data["bias"].toBool()) db = dz.sum(0);
+    if (torch::GradMode::is_enabled()) {   // a graph of the gradients is wanted: operations that carry one
+      if (ctx->needs_input_grad(0)) dx = dh.mm(w.t());
+      dw = x.t().mm(dh);
+    } else {
+      if (ctx->needs_input_grad(0)) dx = dense(dh, w);
+      if (ctx->needs_input_grad(1)) dw = std::get<0>(linear_wgrad(x, dh, false));
+    }
+    return {dx, dw, db, Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
+  }
+};
+
+}  // namespace
+
+Tensor GcnLayer(const Tensor& relabeled, int64_t num_dst, int64_t fanout, const Tensor& x, const Tensor& w,
+                const std::optional<Tensor>& bias, double left, double right, const std::optional<Tensor>& csr_indptr,
+                const std::optional<Tensor>& csr_indices, bool relu) {
+  check_block("gcn_layer", relabeled, num_dst, fanout);
+  const auto t = x.scalar_type();
+  TORCH_CHECK_TYPE(x.is_cuda() && x.dim() == 2 && (t == torch::kFloat32 || t == torch::kBFloat16),
+                   "npc: gcn_layer: input must be a 2-D fp32 or bf16 GPU tensor");
+  TORCH_CHECK(w.is_cuda() && w.dim() == 2 && w.scalar_type() == t && w.size(0) == x.size(1) && w.numel() > 0 &&
+                  (!bias.has_value() || (bias->is_cuda() && bias->scalar_type() == t && bias->dim() == 1 &&
+                                         bias->size(0) == w.size(1))),
+              "npc: gcn_layer: weight, bias and input do not fit each other");
+  return GcnLayerFn::apply(x.contiguous(), w, bias, relabeled, num_dst, fanout, left, right, csr_indptr, csr_indices, relu,
+                           trains(x, w) || (bias.has_value() && trains(*bias)));
 }
 
 // ---------------------------------------------------------------- GAT layer, from the dense product to the bias
@@ -1249,7 +1342,7 @@ struct GatLayerFn : public torch::autograd::Function<GatLayerFn> {
                         const std::optional<Tensor>& bias, const Tensor& relabeled, int64_t num_dst, int64_t fanout,
                         double slope, bool want_grad, const std::optional<Tensor>& csr_indptr,
                         const std::optional<Tensor>& csr_indices, const std::optional<Tensor>& csr_eids,
-                        const std::optional<Tensor>& csc_indptr) {
+                        const std::optional<Tensor>& csc_indptr, bool relu) {
     const int64_t n = ft.size(0), heads = ft.size(1), dim = ft.size(2);
     const auto f32 = ft.options().dtype(torch::kFloat32);
     auto scores = torch::empty({(n + num_dst) * heads}, f32);   // el, then er
@@ -1261,14 +1354,15 @@ struct GatLayerFn : public torch::autograd::Function<GatLayerFn> {
     Tensor b = bias.has_value() ? bias->contiguous() : Tensor();
     check(apt_gat_layer(i64(relabeled), num_dst, static_cast<int>(fanout), ft.data_ptr(), n, static_cast<int>(heads), dim,
                         static_cast<int>(ft.element_size()), attn_l.data_ptr(), attn_r.data_ptr(),
-                        static_cast<int>(attn_l.element_size()), b.defined() ? b.data_ptr() : nullptr,
+                        static_cast<int>(attn_l.element_size()), b.defined() ? b.data_ptr() : nullptr, relu,
                         static_cast<float>(slope), el, er, out.data_ptr(), want_grad ? attn.data_ptr<float>() : nullptr,
                         stream()));
     if (want_grad) {
       const bool csr = csr_indptr.has_value() && csr_indices.has_value() && csr_eids.has_value() && csc_indptr.has_value() &&
                        csr_indptr->numel() == n + 1;
       ctx->save_for_backward({ft, attn_l, attn_r, relabeled, scores, attn, csr ? *csr_indptr : Tensor(),
-                              csr ? *csr_indices : Tensor(), csr ? *csr_eids : Tensor(), csr ? *csc_indptr : Tensor()});
+                              csr ? *csr_indices : Tensor(), csr ? *csr_eids : Tensor(), csr ? *csc_indptr : Tensor(),
+                              relu ? out : Tensor()});
       ctx->saved_data["num_dst"] = num_dst;
       ctx->saved_data["fanout"] = fanout;
       ctx->saved_data["slope"] = slope;
@@ -1284,7 +1378,7 @@ struct GatLayerFn : public torch::autograd::Function<GatLayerFn> {
     const int64_t num_dst = ctx->saved_data["num_dst"].toInt(), fanout = ctx->saved_data["fanout"].toInt();
     const int64_t n = ft.size(0), heads = ft.size(1), dim = ft.size(2);
     const bool bias = ctx->saved_data["bias"].toBool();
-    auto d_out = grads[0].contiguous();
+    const Tensor d_out = before_relu(grads[0], saved[10]);
     SourceOrder o;
     Tensor eids, csc;
     int64_t edges = 0;
@@ -1321,7 +1415,7 @@ struct GatLayerFn : public torch::autograd::Function<GatLayerFn> {
                                  o.bytes == 8 ? i64(eids) : nullptr, o.bytes == 8 ? i64(csc) : nullptr, edges,
                                  d_ft.data_ptr(), d_al.data_ptr(), d_ar.data_ptr(), bias ? d_bias.data_ptr() : nullptr,
                                  ws.data_ptr(), need, stream()));
-    torch::autograd::variable_list out(13);
+    torch::autograd::variable_list out(14);
     out[0] = d_ft;
     out[1] = d_al;
     out[2] = d_ar;
@@ -1337,7 +1431,7 @@ struct GatLayerFn : public torch::autograd::Function<GatLayerFn> {
 Tensor GatLayer(const Tensor& relabeled, int64_t num_dst, int64_t fanout, const Tensor& ft, const Tensor& attn_l,
                 const Tensor& attn_r, const std::optional<Tensor>& bias, double slope,
                 const std::optional<Tensor>& csr_indptr, const std::optional<Tensor>& csr_indices,
-                const std::optional<Tensor>& csr_eids, const std::optional<Tensor>& csc_indptr) {
+                const std::optional<Tensor>& csr_eids, const std::optional<Tensor>& csc_indptr, bool relu) {
   check_block("gat_layer", relabeled, num_dst, fanout);
   const auto good = [](const Tensor& t) {
     return t.is_cuda() && (t.scalar_type() == torch::kFloat32 || t.scalar_type() == torch::kBFloat16);
@@ -1356,7 +1450,7 @@ Tensor GatLayer(const Tensor& relabeled, int64_t num_dst, int64_t fanout, const 
   const bool want_grad = torch::GradMode::is_enabled() && (ft.requires_grad() || attn_l.requires_grad() || attn_r.requires_grad() ||
                                                           (b.has_value() && b->requires_grad()));
   return GatLayerFn::apply(ft.contiguous(), attn_l.contiguous(), attn_r.contiguous(), b, relabeled, num_dst, fanout, slope,
-                           want_grad, csr_indptr, csr_indices, csr_eids, csc_indptr);
+                           want_grad, csr_indptr, csr_indices, csr_eids, csc_indptr, relu);
 }
 
 // ---------------------------------------------------------------- peers only
@@ -1415,8 +1509,13 @@ TORCH_LIBRARY(npc, m) {
       .def("block_formats", &BlockFormats)
       .def("block_linear", &BlockLinear)
       .def("block_aggregate", &BlockAggregate)
-      .def("sage_layer", &SageLayer)
-      .def("gat_layer", &GatLayer)
+      .def("sage_layer(Tensor relabeled, int num_dst, int fanout, Tensor x, Tensor w_neigh, Tensor w_self, Tensor? bias, "
+           "Tensor? csr_indptr, Tensor? csr_indices, bool relu=False) -> Tensor", &SageLayer)
+      .def("gcn_layer(Tensor relabeled, int num_dst, int fanout, Tensor x, Tensor w, Tensor? bias, float left, float right, "
+           "Tensor? csr_indptr, Tensor? csr_indices, bool relu=False) -> Tensor", &GcnLayer)
+      .def("gat_layer(Tensor relabeled, int num_dst, int fanout, Tensor ft, Tensor attn_l, Tensor attn_r, Tensor? bias, "
+           "float slope, Tensor? csr_indptr, Tensor? csr_indices, Tensor? csr_eids, Tensor? csc_indptr, bool relu=False) "
+           "-> Tensor", &GatLayer)
       .def("cluster_and_permute", &ClusterAndPermuteLocal)
       .def("register_graph_partition", &RegisterGraphPartition)
       .def("set_topology", &SetTopology)

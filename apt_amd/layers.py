@@ -51,6 +51,13 @@ def _linear(layer, x):
     return layer(x)
 
 
+_RELU = (torch.relu, nn.functional.relu)      # activations that the kernels apply where they store a layer's result
+
+
+def _is_relu(activation):
+    return any(activation is f for f in _RELU)
+
+
 class SAGEConv(nn.Module):
     """GraphSAGE layer, mean aggregator, with the reference's arithmetic
     (python/npc/model/sageconv.py:118-188): fc_self(h_dst) + fc_neigh(mean of
@@ -75,9 +82,10 @@ class SAGEConv(nn.Module):
                 and wn.shape == ws.shape == (self.out_feats, self.in_feats) and feat.shape[1] == self.in_feats > 0
                 and self.out_feats > 0 and feat.shape[0] >= block.num_dst and not torch.is_autocast_enabled("cuda")):
             f = block.formats or {}
+            relu = _is_relu(self.activation)
             rst = torch.ops.npc.sage_layer(block.relabeled, block.num_dst, block.fanout, feat, wn, ws, b,
-                                           f.get("csr_indptr"), f.get("csr_indices"))
-            return self.activation(rst) if self.activation is not None else rst
+                                           f.get("csr_indptr"), f.get("csr_indices"), relu)
+            return rst if relu or self.activation is None else self.activation(rst)
         h_self = feat[:block.num_dst]
         if self.in_feats > self.out_feats:
             h_neigh = BlockAggregate.apply(block, _linear(self.fc_neigh, feat), True)
@@ -104,16 +112,32 @@ class GraphConv(nn.Module):
 
     def forward(self, block, feat):
         fanout = float(block.fanout)
+        w, b = self.weight, self.bias
+        if (feat.is_cuda and feat.dim() == 2 and feat.dtype in (torch.float32, torch.bfloat16) and feat.dtype == w.dtype
+                and w.is_cuda and w.dim() == 2 and feat.shape[1] == w.shape[0] and w.numel() > 0
+                and (b is None or (b.is_cuda and b.dtype == feat.dtype and b.shape == w.shape[1:]))
+                and not torch.is_autocast_enabled("cuda")):
+            f = block.formats or {}
+            relu = _is_relu(self.activation)
+            rst = torch.ops.npc.gcn_layer(block.relabeled, block.num_dst, block.fanout, feat, w, b,
+                                          *self._factors(fanout), f.get("csr_indptr"), f.get("csr_indices"), relu)
+            return rst if relu or self.activation is None else self.activation(rst)
+        left, right = self._factors(fanout)
         if self.norm in ("left", "both"):
-            feat = feat * (fanout ** -0.5 if self.norm == "both" else 1.0 / fanout)
+            feat = feat * left
         h = (torch.ops.npc.block_linear(feat, self.weight, None, True) if _native_rows(feat, self.weight)
              else torch.matmul(feat, self.weight))
         rst = BlockAggregate.apply(block, h, False)
         if self.norm in ("right", "both"):
-            rst = rst * (fanout ** -0.5 if self.norm == "both" else 1.0 / fanout)
+            rst = rst * right
         if self.bias is not None:
             rst = rst + self.bias
         return self.activation(rst) if self.activation is not None else rst
+
+    def _factors(self, fanout):
+        """What the rows are multiplied with before and after the sum."""
+        return {"none": (1.0, 1.0), "left": (1.0 / fanout, 1.0), "right": (1.0, 1.0 / fanout),
+                "both": (fanout ** -0.5, fanout ** -0.5)}[self.norm]
 
 
 class GATConv(nn.Module):
@@ -140,9 +164,10 @@ class GATConv(nn.Module):
         ft = _linear(self.fc, feat).view(block.num_src, self.num_heads, self.out_feats)
         f = block.formats or {}
         inside = self.bias is not None and self.bias.dtype == ft.dtype
+        relu = _is_relu(self.activation) and (inside or self.bias is None)
         rst = torch.ops.npc.gat_layer(block.relabeled, block.num_dst, block.fanout, ft, self.attn_l, self.attn_r,
                                       self.bias if inside else None, self.negative_slope, f.get("csr_indptr"),
-                                      f.get("csr_indices"), f.get("csr_eids"), f.get("csc_indptr"))
+                                      f.get("csr_indices"), f.get("csr_eids"), f.get("csc_indptr"), relu)
         if self.bias is not None and not inside:      # a bias of another type than the rows: torch's promotion
             rst = rst + self.bias.view(1, self.num_heads, self.out_feats)
-        return self.activation(rst) if self.activation is not None else rst
+        return rst if relu or self.activation is None else self.activation(rst)

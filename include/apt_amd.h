@@ -793,23 +793,29 @@ int apt_block_transpose(const int64_t* relabeled, int64_t num_dst, int fanout, i
 /* The dense product of a layer in fp32, of two operand pairs at once:
  *   y[r, j] (+)= sum_k x1[r, k] w1[j, k] + (r < m2: sum_k x2[r, k] w2[j, k]) + bias[j]
  * x1 [m, k1], x2 [m2, k2] (k2 = 0: none), y [m, n], all row by row; the element (j, k) of a
- * weight is at j * stride_n + k * stride_k; bias may be NULL; accumulate: y is added to.
+ * weight is at j * stride_n + k * stride_k; bias may be NULL; accumulate: y is added to;
+ * relu: what is negative in the end becomes 0.
  * The products are formed from bf16 parts of the operands, to at least the accuracy of
  * an fp32 sum; infinities and NaN come out as such a sum has them. */
 size_t apt_rows_gemm_workspace_bytes(int64_t n, int64_t k1, int64_t k2);   /* 0 = out of range */
 int apt_rows_gemm(const float* x1, int64_t k1, const float* w1, int64_t w1_stride_n,
                   int64_t w1_stride_k, const float* x2, int64_t k2, const float* w2,
                   int64_t w2_stride_n, int64_t w2_stride_k, int64_t m, int64_t m2, int64_t n,
-                  const float* bias, int accumulate, float* y, void* workspace,
+                  const float* bias, int accumulate, int relu, float* y, void* workspace,
                   size_t workspace_bytes, void* stream);
+
+/* y[i] = y[i] + x[i], what is negative then 0 if relu; fp32 (elem_size 4) or bf16 (2). */
+int apt_add_rows(void* y, const void* x, int64_t count, int elem_size, int relu, void* stream);
 
 /* Sum / mean over a block as a layer uses it, and its gradient (python/npc/model/
  * sageconv.py:100-114: the reference's Aggregate, whose backward is the operator with
  * the edges reversed).
- *   apt_block_aggregate           apt_spmm_block with the result in the input's type;
+ *   apt_block_aggregate           scale * apt_spmm_block + bias [dim] + base [num_dst, dim]
+ *                                 (of the input's type, or NULL), what is negative then 0
+ *                                 if relu, in the input's type; base may be out;
  *                                 inv_degree, optional: float[num_dst], 1 / number of
  *                                 edges of the destination (1 where it has none)
- *   apt_block_aggregate_backward  dx[s, :] = sum over the edges s -> d of
+ *   apt_block_aggregate_backward  dx[s, :] = scale * sum over the edges s -> d of
  *                                 dst_scale[d] * dz[d, :] (dst_scale NULL: 1); every
  *                                 row of dx [num_src, dim] is written, in the type of
  *                                 dz (fp32 sums, fixed order).  The edges of a source:
@@ -817,10 +823,11 @@ int apt_rows_gemm(const float* x1, int64_t k1, const float* w1, int64_t w1_strid
  *                                 apt_block_formats (fanout ignored), 4 = indptr / slots
  *                                 of apt_block_transpose. */
 int apt_block_aggregate(const int64_t* neighbors, int64_t num_dst, int fanout, const void* input,
-                        int64_t num_src, int64_t dim, int elem_size, int mean, void* out,
+                        int64_t num_src, int64_t dim, int elem_size, int mean, float scale,
+                        const void* bias, const void* base, int relu, void* out,
                         float* inv_degree, void* stream);
 int apt_block_aggregate_backward(const void* indptr, const void* index, int index_bytes, int fanout,
-                                 int64_t num_src, const float* dst_scale, const void* dz,
+                                 int64_t num_src, const float* dst_scale, float scale, const void* dz,
                                  int64_t num_dst, int64_t dim, int elem_size, void* dx, void* stream);
 
 /* Sums over a COO in any order (apt_spmm_sum's three modes) without atomics, with the
@@ -856,7 +863,8 @@ int apt_coo_combine(int op, const int64_t* coo_row, const int64_t* coo_col, int6
  * num_dst <= num_src: the first num_dst sources are the destinations.
  *   apt_gat_layer           el = (ft * attn_l).sum(-1) [num_src, heads], er likewise on
  *                           the first num_dst rows, then apt_gat_block and + bias
- *                           ([heads, dim], may be NULL): out [num_dst, heads, dim];
+ *                           ([heads, dim], may be NULL), what is negative then 0 if
+ *                           relu: out [num_dst, heads, dim];
  *                           attn_out [num_dst * fanout, heads], optional, as there
  *   apt_gat_layer_backward  fanout <= 64; every row of d_ft [num_src, heads, dim] is
  *                           written; d_attn_l, d_attn_r, d_bias [heads, dim] may be
@@ -866,7 +874,7 @@ int apt_coo_combine(int op, const int64_t* coo_row, const int64_t* coo_col, int6
  *                           and the edge count of apt_block_formats. */
 int apt_gat_layer(const int64_t* neighbors, int64_t num_dst, int fanout, const void* ft, int64_t num_src,
                   int heads, int64_t dim, int elem_size, const void* attn_l, const void* attn_r,
-                  int attn_elem_size, const void* bias, float negative_slope, float* el, float* er, void* out,
+                  int attn_elem_size, const void* bias, int relu, float negative_slope, float* el, float* er, void* out,
                   float* attn_out, void* stream);
 size_t apt_gat_layer_backward_workspace_bytes(int64_t num_dst, int fanout, int64_t num_src, int heads, int64_t dim,
                                               int64_t num_edges);

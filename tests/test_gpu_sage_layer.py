@@ -47,8 +47,14 @@ def test_sage_layer(capi, num_dst, fanout, num_src, k, n, dtype, bias, with_csr)
     for a, b in zip((out,) + got, (want,) + grads):
         assert a.dtype == dtype and a.shape == b.shape
         assert bool((a.double() - b).norm() <= rel_err * b.norm() + 1e-30)
-    with torch.no_grad():
-        assert torch.equal(torch.ops.npc.sage_layer(*args(leaves)), out)
+    # a training step has the bits of separate operations 
+    lin, agg = torch.nn.functional.linear, lambda t: torch.ops.npc.block_aggregate(rel, num_dst, fanout, t, True, None, None)
+    xd, wn, ws = (t.detach() for t in leaves[:3])
+    apart = lin(xd[:num_dst], ws, leaves[3].detach() if bias else None) + (agg(lin(xd, wn)) if k > n else lin(agg(xd), wn))
+    assert torch.equal(out, apart)
+    with torch.no_grad():      # fp32 without gradients: the library's own products
+        plain = torch.ops.npc.sage_layer(*args(leaves))
+    assert bool((plain.double() - want).norm() <= rel_err * want.norm() + 1e-30)
 
 
 def test_sage_layer_second_order_and_hooks():
