@@ -472,6 +472,12 @@ constexpr int64_t kRangeFrom1 = int64_t{1} << 15, kRangeFrom2 = int64_t{1} << 18
 constexpr int kRangeShift0 = 5, kRangeShift1 = 8, kRangeShift2 = 10;
 constexpr int kRangeMaxCount = 4520;          // ranges: 12 bytes of LDS each in the place pass
 constexpr int64_t kRangeMaxTiles = 4096;
+// A tile of the partition: 1024 slots (four per thread) instead of 2048 while the edges are few and workgroups with them.
+// Every tile walks all ranges, so a large block is better off with half the tiles.  CSR of 8 k / 260 k / 730 k / 950 k /
+// 3.4 M edges with 2048 and 1024: 51 / 47, 114 / 108, 183 / 191, 198 / 210, 476 / 542 us (host reads included).
+// A row count in device memory is a third of its bound or less.
+constexpr int64_t kRangeSmallSlots = int64_t{1} << 19, kRangeSmallBound = int64_t{1} << 21;
+constexpr int kRangeSmallIters = 4;
 constexpr int kRangeKeyBits = kRangeMaxShift;
 constexpr int kRangeEdgeBits = 31;
 constexpr int64_t kRangeMaxDst = int64_t{1} << (64 - kRangeKeyBits - kRangeEdgeBits - 1);
@@ -484,6 +490,7 @@ constexpr int kRangeScanGroups = 16;          // tile groups of a scan workgroup
 struct RangeParams {
   int shift2;                 // width of piece 2
   int ranges;
+  int tile;                   // slots of a workgroup
   uint32_t* hist;             // [tiles][ranges]: edges of a tile per range, then their prefix over the tiles
   uint32_t* total;            // [ranges]
   uint32_t* start;            // [ranges + 1]: a range's first record
@@ -535,16 +542,16 @@ __device__ __forceinline__ uint64_t same_value(uint32_t v, int bits, bool valid)
 
 // FORMATS: COO, CSC and CSR (an edge's id is its place in the COO).  Otherwise the transpose alone: the edges of a
 // source by slot, without a compaction.
-template <bool FORMATS>
+template <bool FORMATS, int ITERS>
 __global__ __launch_bounds__(kFmtBlock) void range_count_kernel(CompactParams p, RangeParams r) {
   extern __shared__ uint32_t s_range[];   // [ranges]
   __shared__ uint32_t s_wave[kFmtWaves];
   const int64_t slots = actual_count(p.num_dst, p.num_dst_dev) * p.fanout;
-  const int64_t base = static_cast<int64_t>(blockIdx.x) * kCompactTile;
+  const int64_t base = static_cast<int64_t>(blockIdx.x) * (kFmtBlock * ITERS);
   if (base >= slots && blockIdx.x != 0) return;   // block-uniform: nobody reads an inactive tile's counts
-  int64_t v[kCompactIters];
+  int64_t v[ITERS];
 #pragma unroll
-  for (int it = 0; it < kCompactIters; ++it) {
+  for (int it = 0; it < ITERS; ++it) {
     const int64_t s = base + it * kFmtBlock + threadIdx.x;
     v[it] = s < slots ? p.relabeled[s] : -1;
   }
@@ -552,7 +559,7 @@ __global__ __launch_bounds__(kFmtBlock) void range_count_kernel(CompactParams p,
   __syncthreads();
   uint32_t c = 0;
 #pragma unroll
-  for (int it = 0; it < kCompactIters; ++it) {
+  for (int it = 0; it < ITERS; ++it) {
     if (v[it] < 0) continue;
     ++c;
     atomicAdd(&s_range[range_of(r, v[it])], 1u);
@@ -575,7 +582,7 @@ __global__ __launch_bounds__(kWave * kRangeScanGroups) void range_scan_kernel(Co
   const int lane = threadIdx.x % kWave, group = threadIdx.x / kWave;
   const int b = blockIdx.x * kWave + lane;
   const int64_t slots = actual_count(p.num_dst, p.num_dst_dev) * p.fanout;
-  const int tiles = static_cast<int>(ceil_div_dev(slots, kCompactTile));
+  const int tiles = static_cast<int>(ceil_div_dev(slots, r.tile));
   const int per = (tiles + kRangeScanGroups - 1) / kRangeScanGroups;
   const int t0 = group * per, t1 = min(t0 + per, tiles);
   const bool live = b < r.ranges;
@@ -613,23 +620,23 @@ __global__ __launch_bounds__(kWave * kRangeScanGroups) void range_scan_kernel(Co
 
 // The compaction's place pass (as fmt_place_kernel) with the partition: a wavefront owns consecutive slots, so that
 // walking the wavefronts, and the iterations inside one, is edge order.
-template <bool FORMATS>
+template <bool FORMATS, int ITERS>
 __global__ __launch_bounds__(kFmtBlock) void range_place_kernel(CompactParams p, RangeParams r) {
   extern __shared__ uint32_t s_range[];
   uint32_t* s_base = s_range;                                                // [ranges]
   uint32_t* s_cnt2 = s_range + r.ranges;                                     // [waves][ranges / 2], 16-bit counts
   const int words = (r.ranges + 1) / 2;                                      // 32-bit words of a wave's counts
-  __shared__ uint32_t s_edges[kFmtWaves * kCompactIters];
+  __shared__ uint32_t s_edges[kFmtWaves * ITERS];
   __shared__ uint32_t s_wave[kFmtWaves];
   const int lane = lane_id();
   const int wave = threadIdx.x / kWave;
   const int64_t slots = actual_count(p.num_dst, p.num_dst_dev) * p.fanout;
   const int64_t upper = p.num_dst * p.fanout;
-  const int64_t base = static_cast<int64_t>(blockIdx.x) * kCompactTile + wave * (kCompactIters * kWave);
-  int64_t v[kCompactIters];
-  uint32_t below[kCompactIters];
+  const int64_t base = static_cast<int64_t>(blockIdx.x) * (kFmtBlock * ITERS) + wave * (ITERS * kWave);
+  int64_t v[ITERS];
+  uint32_t below[ITERS];
 #pragma unroll
-  for (int it = 0; it < kCompactIters; ++it) {
+  for (int it = 0; it < ITERS; ++it) {
     const int64_t s = base + it * kWave + lane;
     v[it] = s < slots ? p.relabeled[s] : -1;
   }
@@ -637,16 +644,16 @@ __global__ __launch_bounds__(kFmtBlock) void range_place_kernel(CompactParams p,
   __syncthreads();
   uint32_t* cnt = s_cnt2 + wave * words;
 #pragma unroll
-  for (int it = 0; it < kCompactIters; ++it) {
+  for (int it = 0; it < ITERS; ++it) {
     const uint64_t m = ballot(v[it] >= 0);
     below[it] = rank_below(m);
-    if (lane == 0) s_edges[wave * kCompactIters + it] = __popcll(m);
+    if (lane == 0) s_edges[wave * ITERS + it] = __popcll(m);
     if (v[it] >= 0) {   // at most 512 per wavefront: a 16-bit half never overflows into the other
       const int b = range_of(r, v[it]);
       atomicAdd(&cnt[b >> 1], (b & 1) ? 0x10000u : 1u);
     }
   }
-  const int64_t active = ceil_div_dev(slots, kCompactTile);
+  const int64_t active = ceil_div_dev(slots, (kFmtBlock * ITERS));
   uint32_t first = 0;
   if (FORMATS) {   // edges of the tiles before this one, and of all tiles
     uint32_t before = 0, total = 0, all_total;
@@ -715,25 +722,25 @@ __global__ __launch_bounds__(kFmtBlock) void range_place_kernel(CompactParams p,
       }
     }
   }
-  static_assert(kCompactIters * kFmtWaves <= kWave, "one wavefront scans the tile's per-wave counts");
+  static_assert(ITERS * kFmtWaves <= kWave, "one wavefront scans the tile's per-wave counts");
   if (FORMATS && wave == 0) {
-    const uint32_t c = lane < kCompactIters * kFmtWaves ? s_edges[lane] : 0u;
+    const uint32_t c = lane < ITERS * kFmtWaves ? s_edges[lane] : 0u;
     uint32_t incl = c;
 #pragma unroll
-    for (int off = 1; off < kCompactIters * kFmtWaves; off <<= 1) {
+    for (int off = 1; off < ITERS * kFmtWaves; off <<= 1) {
       const uint32_t y = __shfl_up(incl, off, kWave);
       if (lane >= off) incl += y;
     }
-    if (lane < kCompactIters * kFmtWaves) s_edges[lane] = first + incl - c;
+    if (lane < ITERS * kFmtWaves) s_edges[lane] = first + incl - c;
   }
   __syncthreads();
   const int bits = 32 - __clz(r.ranges - 1 > 0 ? r.ranges - 1 : 1);
   volatile uint16_t* pos = reinterpret_cast<volatile uint16_t*>(cnt);
   const uint32_t fan = static_cast<uint32_t>(p.fanout);
 #pragma unroll
-  for (int it = 0; it < kCompactIters; ++it) {
+  for (int it = 0; it < ITERS; ++it) {
     const int64_t s = base + it * kWave + lane;
-    const int64_t e = FORMATS ? static_cast<int64_t>(s_edges[wave * kCompactIters + it]) + below[it] : s;
+    const int64_t e = FORMATS ? static_cast<int64_t>(s_edges[wave * ITERS + it]) + below[it] : s;
     const uint32_t d = FORMATS ? static_cast<uint32_t>(s) / fan : 0u;
     if (FORMATS && s < upper && static_cast<uint32_t>(s) - d * fan == 0) p.csc_indptr[d] = e;
     const bool valid = v[it] >= 0;
@@ -950,7 +957,7 @@ int tuning_block_fused_scan();  // 0 = always take the separate scan launches
 static size_t fmt_align(size_t x) { return (x + 255) / 256 * 256; }
 
 struct FmtLayout {
-  int64_t slots, ctiles, stiles;
+  int64_t slots, ctiles, stiles, rtiles;
   size_t tile_cnt_off, sums_off, hist_off, bin_total_off, key_off[2], pay_off[2], total;
   int range_shift2, ranges;   // CSR by source ranges; ranges == 0: by radix passes
   size_t start_off, rec_off;
@@ -976,9 +983,15 @@ static FmtLayout fmt_layout(int64_t num_dst, int fanout, int64_t num_src, bool c
   L.tile_cnt_off = off; off = fmt_align(off + sizeof(uint32_t) * static_cast<size_t>(L.ctiles));
   L.sums_off = off;     off = fmt_align(off + sizeof(uint32_t) * kScanChunk);
   L.hist_off = off;
+  L.rtiles = 0;
   if (csr) choose_ranges(num_dst, num_src, !transpose, L);
+  if (L.ranges > 0) {   // by either tile: which one is the launch's choice
+    L.rtiles = L.slots <= kRangeSmallBound ? ceil_div(std::max<int64_t>(L.slots, 1), kFmtBlock * kRangeSmallIters) : L.ctiles;
+    L.tile_cnt_off = off; off = fmt_align(off + sizeof(uint32_t) * static_cast<size_t>(L.rtiles));
+    L.hist_off = off;
+  }
   if (csr && L.ranges > 0) {
-    off = fmt_align(off + sizeof(uint32_t) * static_cast<size_t>(L.ctiles) * L.ranges);
+    off = fmt_align(off + sizeof(uint32_t) * static_cast<size_t>(L.rtiles) * L.ranges);
     L.bin_total_off = off; off = fmt_align(off + sizeof(uint32_t) * L.ranges);
     L.start_off = off;     off = fmt_align(off + sizeof(uint32_t) * (L.ranges + 1));
     L.rec_off = off;       off = fmt_align(off + sizeof(uint64_t) * static_cast<size_t>(L.slots > 0 ? L.slots : 1));
@@ -1010,14 +1023,23 @@ static int launch_ranges(const CompactParams& c, RangeParams& r, const FmtLayout
   r.start = reinterpret_cast<uint32_t*>(ws + L.start_off);
   r.rec = reinterpret_cast<uint64_t*>(ws + L.rec_off);
   r.num_src = num_src;
-  const dim3 tiles(static_cast<unsigned>(L.ctiles));
-  hipLaunchKernelGGL(range_count_kernel<FORMATS>, tiles, dim3(kFmtBlock), sizeof(uint32_t) * L.ranges, st, c, r);
+  const bool small = L.slots <= (c.num_dst_dev != nullptr ? kRangeSmallBound : kRangeSmallSlots);
+  r.tile = small ? kFmtBlock * kRangeSmallIters : kCompactTile;
+  const dim3 tiles(static_cast<unsigned>(ceil_div(std::max<int64_t>(L.slots, 1), r.tile)));
+  const size_t count_lds = sizeof(uint32_t) * L.ranges;
+  if (small)
+    hipLaunchKernelGGL((range_count_kernel<FORMATS, kRangeSmallIters>), tiles, dim3(kFmtBlock), count_lds, st, c, r);
+  else
+    hipLaunchKernelGGL((range_count_kernel<FORMATS, kCompactIters>), tiles, dim3(kFmtBlock), count_lds, st, c, r);
   APT_LAUNCH_CHECK("range_count_kernel");
   hipLaunchKernelGGL(range_scan_kernel, dim3(static_cast<unsigned>(ceil_div(L.ranges, kWave))),
                      dim3(kWave * kRangeScanGroups), 0, st, c, r);
   APT_LAUNCH_CHECK("range_scan_kernel");
   const size_t place_lds = sizeof(uint32_t) * (L.ranges + kFmtWaves * ((L.ranges + 1) / 2));
-  hipLaunchKernelGGL(range_place_kernel<FORMATS>, tiles, dim3(kFmtBlock), place_lds, st, c, r);
+  if (small)
+    hipLaunchKernelGGL((range_place_kernel<FORMATS, kRangeSmallIters>), tiles, dim3(kFmtBlock), place_lds, st, c, r);
+  else
+    hipLaunchKernelGGL((range_place_kernel<FORMATS, kCompactIters>), tiles, dim3(kFmtBlock), place_lds, st, c, r);
   APT_LAUNCH_CHECK("range_place_kernel");
   const int keys = 1 << (L.ranges > kRangeCount0 + kRangeCount1 ? L.range_shift2
                          : L.ranges > kRangeCount0              ? kRangeShift1

@@ -21,7 +21,8 @@ def _block(num_dst, fanout, num_src, seed):
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("num_dst,fanout,num_src,dim", [(1, 1, 1, 1), (700, 15, 5000, 47), (700, 15, 400, 4), (900, 10, 3000, 32),
                                                         (900, 10, 3000, 36), (900, 10, 3000, 100), (500, 25, 9000, 256),
-                                                        (300, 20, 2000, 264), (300, 20, 2000, 600), (4000, 5, 70000, 8)])
+                                                        (300, 20, 2000, 264), (300, 20, 2000, 600), (4000, 5, 70000, 8),
+                                                        (40000, 15, 90000, 4)])
 @pytest.mark.parametrize("mean", [False, True])
 @pytest.mark.parametrize("with_csr", [False, True])
 def test_block_aggregate_backward(capi, num_dst, fanout, num_src, dim, dtype, mean, with_csr):
