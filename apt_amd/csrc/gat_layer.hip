@@ -542,6 +542,26 @@ static void launch_param_grad(const void* ft, const void* d_out, const float* d_
 #undef APT_PARAM
 }
 
+// d_attn_l, d_attn_r (of one type) and d_bias (of the rows') from `splits` partials of 3 * n; zeros from none.
+static int gat_param_sums(const float* part, int splits, int64_t n, int elem_size, int attn_elem_size, void* d_attn_l,
+                          void* d_attn_r, void* d_bias, hipStream_t st) {
+  if (d_attn_l == nullptr && d_attn_r == nullptr && d_bias == nullptr) return APT_OK;
+  if (attn_elem_size == elem_size) {
+    if (elem_size == 4) launch_partial_sums<float, float>(part, 3 * n, splits, d_attn_l, n, d_attn_r, n, d_bias, n, st);
+    else launch_partial_sums<uint16_t, uint16_t>(part, 3 * n, splits, d_attn_l, n, d_attn_r, n, d_bias, n, st);
+    APT_LAUNCH_CHECK("partial_sums_kernel");
+    return APT_OK;
+  }
+  if (attn_elem_size == 4) launch_partial_sums<float, float>(part, 3 * n, splits, d_attn_l, n, d_attn_r, n, nullptr, 0, st);
+  else launch_partial_sums<uint16_t, uint16_t>(part, 3 * n, splits, d_attn_l, n, d_attn_r, n, nullptr, 0, st);
+  APT_LAUNCH_CHECK("partial_sums_kernel");
+  if (d_bias == nullptr) return APT_OK;
+  if (elem_size == 4) launch_partial_sums<float, float>(part + 2 * n, 3 * n, splits, d_bias, n, nullptr, 0, nullptr, 0, st);
+  else launch_partial_sums<uint16_t, uint16_t>(part + 2 * n, 3 * n, splits, d_bias, n, nullptr, 0, nullptr, 0, st);
+  APT_LAUNCH_CHECK("partial_sums_kernel");
+  return APT_OK;
+}
+
 static size_t align256(size_t x) { return (x + 255) / 256 * 256; }
 
 }  // namespace apt
@@ -607,7 +627,9 @@ extern "C" int apt_gat_layer_backward(const int64_t* neighbors, int64_t num_dst,
   APT_REQUIRE(workspace != nullptr && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0 &&
                   workspace_bytes >= apt_gat_layer_backward_workspace_bytes(num_dst, fanout, num_src, heads, dim, num_edges),
               APT_EWORKSPACE, "%s: workspace too small or not 16-byte aligned", who);
-  if (num_src == 0) return APT_OK;
+  if (num_src == 0)   // no rows: the parameters' gradients are zeros
+    return gat_param_sums(static_cast<const float*>(workspace), 0, static_cast<int64_t>(heads) * dim, elem_size, attn_elem_size,
+                          d_attn_l, d_attn_r, d_bias, static_cast<hipStream_t>(stream));
   APT_REQUIRE(ft != nullptr && attn_l != nullptr && attn_r != nullptr && el != nullptr && indptr != nullptr && d_ft != nullptr &&
                   (num_dst == 0 || (neighbors != nullptr && er != nullptr && attn != nullptr && d_out != nullptr && index != nullptr)),
               APT_EINVAL, "%s: a tensor is NULL", who);
@@ -660,20 +682,6 @@ extern "C" int apt_gat_layer_backward(const int64_t* neighbors, int64_t num_dst,
   if (elem_size == 4) launch_param_grad<float>(ft, d_out, d_el, d_er, num_src, num_dst, heads, dim, part, p.attn_l, st);
   else launch_param_grad<uint16_t>(ft, d_out, d_el, d_er, num_src, num_dst, heads, dim, part, p.attn_l, st);
   APT_LAUNCH_CHECK("gat_param_grad_kernel");
-  const int64_t n = heads * dim;
-  const int splits = static_cast<int>(param_blocks(num_src));
-  if (attn_elem_size == elem_size) {
-    if (elem_size == 4) launch_partial_sums<float, float>(part, 3 * n, splits, d_attn_l, n, d_attn_r, n, d_bias, n, st);
-    else launch_partial_sums<uint16_t, uint16_t>(part, 3 * n, splits, d_attn_l, n, d_attn_r, n, d_bias, n, st);
-    APT_LAUNCH_CHECK("partial_sums_kernel");
-    return APT_OK;
-  }
-  if (attn_elem_size == 4) launch_partial_sums<float, float>(part, 3 * n, splits, d_attn_l, n, d_attn_r, n, nullptr, 0, st);
-  else launch_partial_sums<uint16_t, uint16_t>(part, 3 * n, splits, d_attn_l, n, d_attn_r, n, nullptr, 0, st);
-  APT_LAUNCH_CHECK("partial_sums_kernel");
-  if (d_bias == nullptr) return APT_OK;
-  if (elem_size == 4) launch_partial_sums<float, float>(part + 2 * n, 3 * n, splits, d_bias, n, nullptr, 0, nullptr, 0, st);
-  else launch_partial_sums<uint16_t, uint16_t>(part + 2 * n, 3 * n, splits, d_bias, n, nullptr, 0, nullptr, 0, st);
-  APT_LAUNCH_CHECK("partial_sums_kernel");
-  return APT_OK;
+  return gat_param_sums(part, static_cast<int>(param_blocks(num_src)), static_cast<int64_t>(heads) * dim, elem_size, attn_elem_size,
+                        d_attn_l, d_attn_r, d_bias, st);
 }

@@ -62,3 +62,23 @@ def test_gat_layer(capi, num_dst, fanout, num_src, heads, dim, dtype, attn_dtype
         assert err <= tol * (b.abs().max().item() + 1e-2), (name, err, b.abs().max().item())
     with torch.no_grad():
         assert torch.equal(torch.ops.npc.gat_layer(rel, num_dst, fanout, ft, al, ar, bias, 0.2, *csr), out)
+
+
+@pytest.mark.parametrize("dtype,attn_dtype", [(torch.float32, torch.float32), (torch.bfloat16, torch.bfloat16),
+                                              (torch.bfloat16, torch.float32), (torch.float32, torch.bfloat16)])
+@pytest.mark.parametrize("num_dst,num_src", [(0, 0), (0, 70)])
+def test_gat_layer_without_destinations(capi, num_dst, num_src, dtype, attn_dtype):
+    """No row and no edge: every gradient is zero, as torch's sums over nothing are."""
+    import apt_amd  # noqa: F401
+    heads, dim, fanout = 4, 24, 5
+    rel = torch.empty(0, dtype=torch.int64, device=DEV)
+    ft = torch.randn(num_src, heads, dim, device=DEV).to(dtype).requires_grad_(True)
+    al, ar = (torch.randn(heads, dim, device=DEV).to(attn_dtype).requires_grad_(True) for _ in range(2))
+    bias = torch.randn(heads * dim, device=DEV).to(dtype).requires_grad_(True)
+    out = torch.ops.npc.gat_layer(rel, num_dst, fanout, ft, al, ar, bias, 0.2, None, None, None, None)
+    assert out.shape == (num_dst, heads, dim)
+    # what the gradients are allocated from: blocks of their sizes that hold something else
+    dirty = [torch.full((heads, dim), float("nan"), device=DEV, dtype=t) for t in (dtype, attn_dtype) for _ in range(8)]
+    del dirty
+    for g, t in zip(torch.autograd.grad(out, [ft, al, ar, bias], torch.zeros_like(out)), (ft, al, ar, bias)):
+        assert g.shape == t.shape and g.dtype == t.dtype and bool((g == 0).all())
