@@ -39,7 +39,7 @@ class CFeatStore(C.Structure):
 MAX_HOPS, MAX_SLOTS = 8, 16
 
 
-ABI_VERSION = 2          # APT_ABI_VERSION of include/apt_amd.h
+ABI_VERSION = 3          # APT_ABI_VERSION of include/apt_amd.h
 
 
 class CBlockBuffers(C.Structure):    # apt_block_buffers
@@ -133,7 +133,7 @@ SYMBOLS = {
     "apt_coo_sum_workspace_bytes": (_SZ, [_I64, _I64, _I]),
     "apt_coo_sum": (_I, [_I, _P, _P, _I64, _I, _P, _I64, _P, _I64, _I, _P, _I64, _P, _SZ, _P]),
     "apt_coo_combine": (_I, [_I, _P, _P, _I64, _P, _I64, _P, _I64, _I64, _I, _P, _P, _P, _I, _P, _P]),
-    "apt_gat_layer": (_I, [_P, _I64, _I, _P, _I64, _I, _I64, _I, _P, _P, _I, _P, _I, C.c_float, _P, _P, _P, _P, _P]),
+    "apt_gat_layer": (_I, [_P, _I64, _I, _P, _I64, _I, _I64, _I, _P, _P, _I, _P, _I, C.c_float, _I, _P, _P, _P, _P, _P]),
     "apt_gat_layer_backward_workspace_bytes": (_SZ, [_I64, _I, _I64, _I, _I64, _I64]),
     "apt_gat_layer_backward": (_I, [_P, _I64, _I, _P, _I64, _I, _I64, _I, _P, _P, _I, C.c_float, _P, _P, _P, _P, _P, _P, _I, _P,
                                     _P, _I64, _P, _P, _P, _P, _P, _SZ, _P]),

@@ -12,6 +12,7 @@
 // bf16: a model trained in bf16 gets what the separate operations give.  Their results are bf16 where both operands
 // are, so a value that was a bf16 tensor between two of them is rounded here too (as_stored, Terms); a gradient of the
 // attention vectors is what is left of large terms that cancel, and moves by several per cent with that rounding.
+// Without gradients (`wide`) nothing is rounded between the rows and the result: scores, sum and result are fp32.
 #include <algorithm>
 
 #include "common.hpp"
@@ -54,7 +55,8 @@ struct ParamVec {
 template <typename T>
 struct Terms {
   bool bf16;
-  __device__ __forceinline__ explicit Terms(const ParamVec& attn) : bf16(sizeof(T) == 2 && attn.elem_size == 2) {}
+  __device__ __forceinline__ explicit Terms(const ParamVec& attn, int wide = 0)
+      : bf16(sizeof(T) == 2 && attn.elem_size == 2 && !wide) {}
   __device__ __forceinline__ float operator()(float v) const { return bf16 ? as_stored<uint16_t>(v) : v; }
 };
 
@@ -63,7 +65,7 @@ struct Terms {
 template <typename T, int VEC, int LPH, int LPR>
 __global__ __launch_bounds__(kAggBlock) void gat_pair_scores_kernel(const T* __restrict__ x, int64_t num_rows,
                                                                     int64_t num_dst, int heads, ParamVec attn_l,
-                                                                    ParamVec attn_r, float* __restrict__ el,
+                                                                    ParamVec attn_r, int wide, float* __restrict__ el,
                                                                     float* __restrict__ er) {
   constexpr int kGroups = kAggBlock / LPR;
   constexpr int kRows = 4;
@@ -74,7 +76,7 @@ __global__ __launch_bounds__(kAggBlock) void gat_pair_scores_kernel(const T* __r
   float al[VEC], ar[VEC];
   attn_l.load(live ? l * VEC : 0, al);
   attn_r.load(live ? l * VEC : 0, ar);
-  const Terms<T> term(attn_l);
+  const Terms<T> term(attn_l, wide);
   const int64_t step = static_cast<int64_t>(gridDim.x) * kGroups;
   for (int64_t r0 = static_cast<int64_t>(blockIdx.x) * kGroups + grp; r0 < num_rows; r0 += kRows * step) {
     Row<T, VEC> v[kRows];
@@ -109,10 +111,10 @@ __global__ __launch_bounds__(kAggBlock) void gat_pair_scores_kernel(const T* __r
 template <typename T>
 __global__ __launch_bounds__(kAggBlock) void gat_pair_scores_any_kernel(const T* __restrict__ x, int64_t num_rows,
                                                                         int64_t num_dst, int heads, int64_t dim,
-                                                                        ParamVec attn_l, ParamVec attn_r,
+                                                                        ParamVec attn_l, ParamVec attn_r, int wide,
                                                                         float* __restrict__ el, float* __restrict__ er) {
   const int lane = threadIdx.x % kWave;
-  const Terms<T> term(attn_l);
+  const Terms<T> term(attn_l, wide);
   const int64_t items = num_rows * heads;
   for (int64_t it = static_cast<int64_t>(blockIdx.x) * kAggWaves + threadIdx.x / kWave; it < items;
        it += static_cast<int64_t>(gridDim.x) * kAggWaves) {
@@ -136,12 +138,12 @@ __global__ __launch_bounds__(kAggBlock) void gat_pair_scores_any_kernel(const T*
 }
 
 template <typename T, int VEC, int LPH>
-static void launch_pair_scores_r(const void* x, int64_t n, int64_t num_dst, int heads, ParamVec al, ParamVec ar, float* el,
-                                 float* er, hipStream_t st) {
+static void launch_pair_scores_r(const void* x, int64_t n, int64_t num_dst, int heads, ParamVec al, ParamVec ar, int wide,
+                                 float* el, float* er, hipStream_t st) {
 #define APT_PAIR(LPR)                                                                                              \
   hipLaunchKernelGGL((gat_pair_scores_kernel<T, VEC, LPH, LPR>),                                                    \
                      dim3(static_cast<unsigned>(std::min<int64_t>(ceil_div(n, kAggBlock / LPR), 4096))),           \
-                     dim3(kAggBlock), 0, st, static_cast<const T*>(x), n, num_dst, heads, al, ar, el, er)
+                     dim3(kAggBlock), 0, st, static_cast<const T*>(x), n, num_dst, heads, al, ar, wide, el, er)
   const int lanes = heads * LPH;
   if constexpr (LPH <= 8) {
     if (lanes <= 8) {
@@ -167,18 +169,18 @@ static void launch_pair_scores_r(const void* x, int64_t n, int64_t num_dst, int 
 
 template <typename T, int VEC>
 static bool launch_pair_scores(const void* x, int64_t n, int64_t num_dst, int heads, int64_t dim, ParamVec al, ParamVec ar,
-                               float* el, float* er, hipStream_t st) {
+                               int wide, float* el, float* er, hipStream_t st) {
   const int64_t lph = dim / VEC;
   if (dim % VEC != 0 || (lph & (lph - 1)) != 0 || heads * lph > kWave || (reinterpret_cast<uintptr_t>(x) & 15) != 0)
     return false;
   switch (lph) {
-    case 1: launch_pair_scores_r<T, VEC, 1>(x, n, num_dst, heads, al, ar, el, er, st); return true;
-    case 2: launch_pair_scores_r<T, VEC, 2>(x, n, num_dst, heads, al, ar, el, er, st); return true;
-    case 4: launch_pair_scores_r<T, VEC, 4>(x, n, num_dst, heads, al, ar, el, er, st); return true;
-    case 8: launch_pair_scores_r<T, VEC, 8>(x, n, num_dst, heads, al, ar, el, er, st); return true;
-    case 16: launch_pair_scores_r<T, VEC, 16>(x, n, num_dst, heads, al, ar, el, er, st); return true;
-    case 32: launch_pair_scores_r<T, VEC, 32>(x, n, num_dst, heads, al, ar, el, er, st); return true;
-    default: launch_pair_scores_r<T, VEC, 64>(x, n, num_dst, heads, al, ar, el, er, st); return true;
+    case 1: launch_pair_scores_r<T, VEC, 1>(x, n, num_dst, heads, al, ar, wide, el, er, st); return true;
+    case 2: launch_pair_scores_r<T, VEC, 2>(x, n, num_dst, heads, al, ar, wide, el, er, st); return true;
+    case 4: launch_pair_scores_r<T, VEC, 4>(x, n, num_dst, heads, al, ar, wide, el, er, st); return true;
+    case 8: launch_pair_scores_r<T, VEC, 8>(x, n, num_dst, heads, al, ar, wide, el, er, st); return true;
+    case 16: launch_pair_scores_r<T, VEC, 16>(x, n, num_dst, heads, al, ar, wide, el, er, st); return true;
+    case 32: launch_pair_scores_r<T, VEC, 32>(x, n, num_dst, heads, al, ar, wide, el, er, st); return true;
+    default: launch_pair_scores_r<T, VEC, 64>(x, n, num_dst, heads, al, ar, wide, el, er, st); return true;
   }
 }
 
@@ -568,8 +570,8 @@ static size_t align256(size_t x) { return (x + 255) / 256 * 256; }
 
 extern "C" int apt_gat_layer(const int64_t* neighbors, int64_t num_dst, int fanout, const void* ft, int64_t num_src,
                              int heads, int64_t dim, int elem_size, const void* attn_l, const void* attn_r,
-                             int attn_elem_size, const void* bias, int relu, float negative_slope, float* el, float* er,
-                             void* out,                             float* attn_out, void* stream) {
+                             int attn_elem_size, const void* bias, int relu, float negative_slope, int wide, float* el,
+                             float* er, void* out, float* attn_out, void* stream) {
   using namespace apt;
   const char* who = "apt_gat_layer";
   APT_REQUIRE(num_dst >= 0 && num_dst <= num_src && fanout > 0 && heads > 0 && dim > 0, APT_EINVAL,
@@ -582,21 +584,21 @@ extern "C" int apt_gat_layer(const int64_t* neighbors, int64_t num_dst, int fano
               APT_EINVAL, "%s: a tensor is NULL", who);
   hipStream_t st = static_cast<hipStream_t>(stream);
   const ParamVec al{attn_l, attn_elem_size}, ar{attn_r, attn_elem_size};
-  const bool done = elem_size == 4 ? launch_pair_scores<float, 4>(ft, num_src, num_dst, heads, dim, al, ar, el, er, st)
-                                   : launch_pair_scores<uint16_t, 8>(ft, num_src, num_dst, heads, dim, al, ar, el, er, st) ||
-                                         launch_pair_scores<uint16_t, 4>(ft, num_src, num_dst, heads, dim, al, ar, el, er, st);
+  const bool done = elem_size == 4 ? launch_pair_scores<float, 4>(ft, num_src, num_dst, heads, dim, al, ar, wide, el, er, st)
+                                   : launch_pair_scores<uint16_t, 8>(ft, num_src, num_dst, heads, dim, al, ar, wide, el, er, st) ||
+                                         launch_pair_scores<uint16_t, 4>(ft, num_src, num_dst, heads, dim, al, ar, wide, el, er, st);
   if (!done) {
     const dim3 grid(static_cast<unsigned>(std::min<int64_t>(ceil_div(num_src * heads, kAggWaves), 1 << 16))), block(kAggBlock);
     if (elem_size == 4)
       hipLaunchKernelGGL(gat_pair_scores_any_kernel<float>, grid, block, 0, st, static_cast<const float*>(ft), num_src, num_dst,
-                         heads, dim, al, ar, el, er);
+                         heads, dim, al, ar, wide, el, er);
     else
       hipLaunchKernelGGL(gat_pair_scores_any_kernel<uint16_t>, grid, block, 0, st, static_cast<const uint16_t*>(ft), num_src,
-                         num_dst, heads, dim, al, ar, el, er);
+                         num_dst, heads, dim, al, ar, wide, el, er);
   }
   APT_LAUNCH_CHECK("gat_pair_scores_kernel");
   return gat_block(who, neighbors, num_dst, nullptr, fanout, ft, num_src, heads, dim, elem_size, el, er, negative_slope, out,
-                   true, attn_out, bias, relu, st);
+                   wide == 0, attn_out, bias, relu, st);
 }
 
 extern "C" size_t apt_gat_layer_backward_workspace_bytes(int64_t num_dst, int fanout, int64_t num_src, int heads, int64_t dim,

@@ -418,8 +418,8 @@ __global__ __launch_bounds__(kAggBlock) void gat_scores_vec_kernel(const T* __re
 // row (all heads); the softmax runs online over the slots (running maximum,
 // rescaled sum), so a row's features are read once and nothing is written but
 // the result: no per-edge score, exponent or weight arrays, no atomics.
-// OUT: fp32, or the input's type with the layer's bias (optional, [heads, dim] of that type) added to the result as
-// it would be stored without one.
+// OUT: fp32 or the input's type, with the layer's bias (optional, [heads, dim] of OUT) added to the result as it would
+// be stored without one.
 template <typename T, typename OUT, int VEC, int LPR>
 __global__ __launch_bounds__(kAggBlock) void gat_ell_kernel(const int64_t* __restrict__ nbr, int64_t num_dst,
                                                             const int64_t* num_dst_dev, int fanout,
@@ -1128,7 +1128,7 @@ static void gat_block_as(const int64_t* neighbors, int64_t num_dst, const int64_
 #undef APT_GAT_BLOCK
 }
 
-// out: fp32 without a bias, or (like_input) the input's type with one.  Shared with the GAT layer (gat_layer.hip).
+// out and bias: fp32, or (like_input) the input's type.  Shared with the GAT layer (gat_layer.hip).
 int gat_block(const char* who, const int64_t* neighbors, int64_t num_dst, const int64_t* num_dst_dev, int fanout,
               const void* ft, int64_t num_src, int heads, int64_t dim, int elem_size, const float* el, const float* er,
               float slope, void* out, bool like_input, float* attn_out, const void* bias, int act, hipStream_t st) {

@@ -1342,20 +1342,20 @@ struct GatLayerFn : public torch::autograd::Function<GatLayerFn> {
                         const std::optional<Tensor>& bias, const Tensor& relabeled, int64_t num_dst, int64_t fanout,
                         double slope, bool want_grad, const std::optional<Tensor>& csr_indptr,
                         const std::optional<Tensor>& csr_indices, const std::optional<Tensor>& csr_eids,
-                        const std::optional<Tensor>& csc_indptr, bool relu) {
+                        const std::optional<Tensor>& csc_indptr, bool relu, bool wide) {
     const int64_t n = ft.size(0), heads = ft.size(1), dim = ft.size(2);
     const auto f32 = ft.options().dtype(torch::kFloat32);
     auto scores = torch::empty({(n + num_dst) * heads}, f32);   // el, then er
     float* el = scores.data_ptr<float>();
     float* er = el + n * heads;
-    auto out = torch::empty({num_dst, heads, dim}, ft.options());
+    auto out = torch::empty({num_dst, heads, dim}, wide ? f32 : ft.options());
     Tensor attn;
     if (want_grad) attn = torch::empty({num_dst * fanout, heads}, f32);
-    Tensor b = bias.has_value() ? bias->contiguous() : Tensor();
+    Tensor b = bias.has_value() ? bias->to(out.scalar_type()).contiguous() : Tensor();
     check(apt_gat_layer(i64(relabeled), num_dst, static_cast<int>(fanout), ft.data_ptr(), n, static_cast<int>(heads), dim,
                         static_cast<int>(ft.element_size()), attn_l.data_ptr(), attn_r.data_ptr(),
                         static_cast<int>(attn_l.element_size()), b.defined() ? b.data_ptr() : nullptr, relu,
-                        static_cast<float>(slope), el, er, out.data_ptr(), want_grad ? attn.data_ptr<float>() : nullptr,
+                        static_cast<float>(slope), wide, el, er, out.data_ptr(), want_grad ? attn.data_ptr<float>() : nullptr,
                         stream()));
     if (want_grad) {
       const bool csr = csr_indptr.has_value() && csr_indices.has_value() && csr_eids.has_value() && csc_indptr.has_value() &&
@@ -1415,7 +1415,7 @@ struct GatLayerFn : public torch::autograd::Function<GatLayerFn> {
                                  o.bytes == 8 ? i64(eids) : nullptr, o.bytes == 8 ? i64(csc) : nullptr, edges,
                                  d_ft.data_ptr(), d_al.data_ptr(), d_ar.data_ptr(), bias ? d_bias.data_ptr() : nullptr,
                                  ws.data_ptr(), need, stream()));
-    torch::autograd::variable_list out(14);
+    torch::autograd::variable_list out(15);
     out[0] = d_ft;
     out[1] = d_al;
     out[2] = d_ar;
@@ -1427,11 +1427,12 @@ struct GatLayerFn : public torch::autograd::Function<GatLayerFn> {
 }  // namespace
 
 // ft [num_src, heads, dim] -> [num_dst, heads, dim] (apt_gat_layer), with its gradients.  attn_l, attn_r [heads, dim]
-// fp32 or bf16, bias [heads, dim] (or any shape of that many elements) of ft's type.
+// fp32 or bf16, bias [heads, dim] (or any shape of that many elements) of ft's type.  fp32_result: of bf16 rows too, and
+// nothing rounded on the way to it, if no gradient is wanted.
 Tensor GatLayer(const Tensor& relabeled, int64_t num_dst, int64_t fanout, const Tensor& ft, const Tensor& attn_l,
                 const Tensor& attn_r, const std::optional<Tensor>& bias, double slope,
                 const std::optional<Tensor>& csr_indptr, const std::optional<Tensor>& csr_indices,
-                const std::optional<Tensor>& csr_eids, const std::optional<Tensor>& csc_indptr, bool relu) {
+                const std::optional<Tensor>& csr_eids, const std::optional<Tensor>& csc_indptr, bool relu, bool fp32_result) {
   check_block("gat_layer", relabeled, num_dst, fanout);
   const auto good = [](const Tensor& t) {
     return t.is_cuda() && (t.scalar_type() == torch::kFloat32 || t.scalar_type() == torch::kBFloat16);
@@ -1450,7 +1451,8 @@ Tensor GatLayer(const Tensor& relabeled, int64_t num_dst, int64_t fanout, const 
   const bool want_grad = torch::GradMode::is_enabled() && (ft.requires_grad() || attn_l.requires_grad() || attn_r.requires_grad() ||
                                                           (b.has_value() && b->requires_grad()));
   return GatLayerFn::apply(ft.contiguous(), attn_l.contiguous(), attn_r.contiguous(), b, relabeled, num_dst, fanout, slope,
-                           want_grad, csr_indptr, csr_indices, csr_eids, csc_indptr, relu);
+                           want_grad, csr_indptr, csr_indices, csr_eids, csc_indptr, relu,
+                           fp32_result && !want_grad && ft.scalar_type() == torch::kBFloat16);
 }
 
 // ---------------------------------------------------------------- peers only
@@ -1514,8 +1516,8 @@ TORCH_LIBRARY(npc, m) {
       .def("gcn_layer(Tensor relabeled, int num_dst, int fanout, Tensor x, Tensor w, Tensor? bias, float left, float right, "
            "Tensor? csr_indptr, Tensor? csr_indices, bool relu=False) -> Tensor", &GcnLayer)
       .def("gat_layer(Tensor relabeled, int num_dst, int fanout, Tensor ft, Tensor attn_l, Tensor attn_r, Tensor? bias, "
-           "float slope, Tensor? csr_indptr, Tensor? csr_indices, Tensor? csr_eids, Tensor? csc_indptr, bool relu=False) "
-           "-> Tensor", &GatLayer)
+           "float slope, Tensor? csr_indptr, Tensor? csr_indices, Tensor? csr_eids, Tensor? csc_indptr, bool relu=False, "
+           "bool fp32_result=False) -> Tensor", &GatLayer)
       .def("cluster_and_permute", &ClusterAndPermuteLocal)
       .def("register_graph_partition", &RegisterGraphPartition)
       .def("set_topology", &SetTopology)

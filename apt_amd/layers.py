@@ -145,7 +145,9 @@ class GATConv(nn.Module):
     LeakyReLU, edge softmax, weighted sum, bias).  Everything between the dense
     product and the activation is npc.gat_layer, forward and backward: two
     kernels from the fixed-stride block, and for the gradients one over the
-    destinations' edges, one over the sources and one for the parameters."""
+    destinations' edges, one over the sources and one for the parameters.
+    A bf16 layer without gradients returns the fp32 sum (scores in fp32 too); the
+    next bf16 layer takes it as its input."""
 
     def __init__(self, in_feats, out_feats, num_heads, negative_slope=0.2, bias=True, activation=None):
         super().__init__()
@@ -161,13 +163,15 @@ class GATConv(nn.Module):
         nn.init.xavier_normal_(self.attn_r, gain=gain)
 
     def forward(self, block, feat):
+        if not torch.is_grad_enabled() and feat.dtype == torch.float32 and self.fc.weight.dtype == torch.bfloat16:
+            feat = feat.bfloat16()
         ft = _linear(self.fc, feat).view(block.num_src, self.num_heads, self.out_feats)
         f = block.formats or {}
         inside = self.bias is not None and self.bias.dtype == ft.dtype
         relu = _is_relu(self.activation) and (inside or self.bias is None)
         rst = torch.ops.npc.gat_layer(block.relabeled, block.num_dst, block.fanout, ft, self.attn_l, self.attn_r,
                                       self.bias if inside else None, self.negative_slope, f.get("csr_indptr"),
-                                      f.get("csr_indices"), f.get("csr_eids"), f.get("csc_indptr"), relu)
+                                      f.get("csr_indices"), f.get("csr_eids"), f.get("csc_indptr"), relu, True)
         if self.bias is not None and not inside:      # a bias of another type than the rows: torch's promotion
             rst = rst + self.bias.view(1, self.num_heads, self.out_feats)
         return rst if relu or self.activation is None else self.activation(rst)

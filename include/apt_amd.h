@@ -58,7 +58,7 @@ const char* apt_last_error(void);
 /* Raised whenever a struct of this header or a signature changes; a binding
  * compares apt_abi_version() of the library it loaded with the header it was
  * written against. */
-#define APT_ABI_VERSION 2
+#define APT_ABI_VERSION 3
 int apt_abi_version(void);
 
 /* Kernel-variant knobs for measurement (process-wide, not thread-safe, no
@@ -864,7 +864,9 @@ int apt_coo_combine(int op, const int64_t* coo_row, const int64_t* coo_col, int6
  *   apt_gat_layer           el = (ft * attn_l).sum(-1) [num_src, heads], er likewise on
  *                           the first num_dst rows, then apt_gat_block and + bias
  *                           ([heads, dim], may be NULL), what is negative then 0 if
- *                           relu: out [num_dst, heads, dim];
+ *                           relu: out [num_dst, heads, dim].  wide: bf16 rows keep fp32
+ *                           from there on (scores, out; the bias is fp32 too); 0:
+ *                           rounded where separate bf16 operations round;
  *                           attn_out [num_dst * fanout, heads], optional, as there
  *   apt_gat_layer_backward  fanout <= 64; every row of d_ft [num_src, heads, dim] is
  *                           written; d_attn_l, d_attn_r, d_bias [heads, dim] may be
@@ -874,8 +876,8 @@ int apt_coo_combine(int op, const int64_t* coo_row, const int64_t* coo_col, int6
  *                           and the edge count of apt_block_formats. */
 int apt_gat_layer(const int64_t* neighbors, int64_t num_dst, int fanout, const void* ft, int64_t num_src,
                   int heads, int64_t dim, int elem_size, const void* attn_l, const void* attn_r,
-                  int attn_elem_size, const void* bias, int relu, float negative_slope, float* el, float* er, void* out,
-                  float* attn_out, void* stream);
+                  int attn_elem_size, const void* bias, int relu, float negative_slope, int wide, float* el, float* er,
+                  void* out, float* attn_out, void* stream);
 size_t apt_gat_layer_backward_workspace_bytes(int64_t num_dst, int fanout, int64_t num_src, int heads, int64_t dim,
                                               int64_t num_edges);
 int apt_gat_layer_backward(const int64_t* neighbors, int64_t num_dst, int fanout, const void* ft,

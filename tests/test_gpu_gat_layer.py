@@ -82,3 +82,38 @@ def test_gat_layer_without_destinations(capi, num_dst, num_src, dtype, attn_dtyp
     del dirty
     for g, t in zip(torch.autograd.grad(out, [ft, al, ar, bias], torch.zeros_like(out)), (ft, al, ar, bias)):
         assert g.shape == t.shape and g.dtype == t.dtype and bool((g == 0).all())
+
+
+@pytest.mark.parametrize("heads,dim,fanout", [(4, 16, 9), (3, 24, 9), (2, 100, 9), (4, 64, 20), (1, 5, 7)])
+@pytest.mark.parametrize("attn_dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("activation", [None, torch.relu])
+def test_gat_layer_bf16_without_gradients_keeps_fp32(capi, heads, dim, fanout, attn_dtype, activation):
+    """Scores, softmax, sum and result of a bf16 layer are fp32 under no_grad: 1e-5 of the same bf16 rows' float64
+    result (a rounding of a score or of the result to bf16 is 4e-3).  The next layer takes that result."""
+    from apt_amd.layers import GATConv
+    from apt_amd.sampler import Block
+    num_dst, num_src = 400, 1500
+    rng = np.random.default_rng(heads * dim + fanout)
+    r = rng.integers(0, num_src, size=num_dst * fanout)
+    r[rng.random(r.size) < 0.2] = -1
+    r[:fanout] = -1
+    rel = torch.from_numpy(r.astype(np.int64)).to(DEV)
+    torch.manual_seed(3)
+    layer = GATConv(40, dim, heads, activation=activation).to(DEV, torch.bfloat16)
+    with torch.no_grad():
+        layer.bias.normal_()
+    for p in (layer.attn_l, layer.attn_r):
+        p.data = p.data.to(attn_dtype)
+    blk = Block(num_src, num_dst, None, rel, fanout)
+    feat = torch.randn(num_src, 40, device=DEV).bfloat16()
+    with torch.no_grad():
+        got = layer(blk, feat)
+        ft, al, ar = layer.fc(feat).view(num_src, heads, dim).double(), layer.attn_l.double(), layer.attn_r.double()
+        want = _separate(rel, num_dst, fanout, ft, al, ar, layer.bias.view(heads, dim).double(), 0.2)
+        want = want if activation is None else activation(want)
+        assert got.dtype == torch.float32
+        assert (got.double() - want).abs().max().item() <= 1e-5 * want.abs().max().item()
+        upper = GATConv(heads * dim, 8, 2).to(DEV, torch.bfloat16)
+        top = Block(num_dst, 50, None, torch.randint(0, num_dst, (50 * 4,), device=DEV), 4)
+        assert torch.equal(upper(top, got.flatten(1)), upper(top, got.flatten(1).bfloat16()))
+    assert layer(blk, feat).dtype == torch.bfloat16     # a training step
