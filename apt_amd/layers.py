@@ -16,6 +16,16 @@ from torch.nn.modules.module import _has_any_global_hook
 from . import ops  # noqa: F401  (loads the npc operators)
 
 
+@torch._disable_dynamo      # (imports the compiler on its first call, which is made while compiling)
+def _untraced(op, *args):
+    return op(*args)
+
+
+def _call(op, *args):
+    """op(*args).  A compiler cannot look into an operator that launches kernels: it breaks its graph around the call."""
+    return _untraced(op, *args) if torch.compiler.is_compiling() else op(*args)
+
+
 class BlockAggregate:
     """out[d] = sum (or mean) over the block's edges (s -> d) of X[s], in X's dtype (sums are fp32 inside the kernels),
     with its gradient: npc.block_aggregate.  The backward pass takes the block's CSR if it has been emitted and
@@ -24,8 +34,8 @@ class BlockAggregate:
     @staticmethod
     def apply(block, X, mean):
         f = block.formats or {}
-        return torch.ops.npc.block_aggregate(block.relabeled, block.num_dst, block.fanout, X, bool(mean),
-                                             f.get("csr_indptr"), f.get("csr_indices"))
+        return _call(torch.ops.npc.block_aggregate, block.relabeled, block.num_dst, block.fanout, X, bool(mean),
+                     f.get("csr_indptr"), f.get("csr_indices"))
 
 
 def _native_rows(x, weight):
@@ -47,7 +57,7 @@ def _plain(layer):
 def _linear(layer, x):
     """layer(x), its products and gradients from npc.block_linear where they can be."""
     if _plain(layer) and _native_rows(x, layer.weight) and (layer.bias is None or layer.bias.dtype == x.dtype):
-        return torch.ops.npc.block_linear(x, layer.weight, layer.bias, False)
+        return _call(torch.ops.npc.block_linear, x, layer.weight, layer.bias, False)
     return layer(x)
 
 
@@ -83,8 +93,8 @@ class SAGEConv(nn.Module):
                 and self.out_feats > 0 and feat.shape[0] >= block.num_dst and not torch.is_autocast_enabled("cuda")):
             f = block.formats or {}
             relu = _is_relu(self.activation)
-            rst = torch.ops.npc.sage_layer(block.relabeled, block.num_dst, block.fanout, feat, wn, ws, b,
-                                           f.get("csr_indptr"), f.get("csr_indices"), relu)
+            rst = _call(torch.ops.npc.sage_layer, block.relabeled, block.num_dst, block.fanout, feat, wn, ws, b,
+                        f.get("csr_indptr"), f.get("csr_indices"), relu)
             return rst if relu or self.activation is None else self.activation(rst)
         h_self = feat[:block.num_dst]
         if self.in_feats > self.out_feats:
@@ -119,13 +129,13 @@ class GraphConv(nn.Module):
                 and not torch.is_autocast_enabled("cuda")):
             f = block.formats or {}
             relu = _is_relu(self.activation)
-            rst = torch.ops.npc.gcn_layer(block.relabeled, block.num_dst, block.fanout, feat, w, b,
-                                          *self._factors(fanout), f.get("csr_indptr"), f.get("csr_indices"), relu)
+            rst = _call(torch.ops.npc.gcn_layer, block.relabeled, block.num_dst, block.fanout, feat, w, b,
+                        *self._factors(fanout), f.get("csr_indptr"), f.get("csr_indices"), relu)
             return rst if relu or self.activation is None else self.activation(rst)
         left, right = self._factors(fanout)
         if self.norm in ("left", "both"):
             feat = feat * left
-        h = (torch.ops.npc.block_linear(feat, self.weight, None, True) if _native_rows(feat, self.weight)
+        h = (_call(torch.ops.npc.block_linear, feat, self.weight, None, True) if _native_rows(feat, self.weight)
              else torch.matmul(feat, self.weight))
         rst = BlockAggregate.apply(block, h, False)
         if self.norm in ("right", "both"):
@@ -169,9 +179,9 @@ class GATConv(nn.Module):
         f = block.formats or {}
         inside = self.bias is not None and self.bias.dtype == ft.dtype
         relu = _is_relu(self.activation) and (inside or self.bias is None)
-        rst = torch.ops.npc.gat_layer(block.relabeled, block.num_dst, block.fanout, ft, self.attn_l, self.attn_r,
-                                      self.bias if inside else None, self.negative_slope, f.get("csr_indptr"),
-                                      f.get("csr_indices"), f.get("csr_eids"), f.get("csc_indptr"), relu, True)
+        rst = _call(torch.ops.npc.gat_layer, block.relabeled, block.num_dst, block.fanout, ft, self.attn_l, self.attn_r,
+                    self.bias if inside else None, self.negative_slope, f.get("csr_indptr"),
+                    f.get("csr_indices"), f.get("csr_eids"), f.get("csc_indptr"), relu, True)
         if self.bias is not None and not inside:      # a bias of another type than the rows: torch's promotion
             rst = rst + self.bias.view(1, self.num_heads, self.out_feats)
         return rst if relu or self.activation is None else self.activation(rst)

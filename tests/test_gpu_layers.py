@@ -189,3 +189,39 @@ def test_sage_trains_on_sampled_batches():
         opt.step()
         losses.append(loss.item())
     assert np.mean(losses[-10:]) < 0.6 * np.mean(losses[:5]), (losses[:5], losses[-10:])
+
+
+@pytest.mark.parametrize("backend", ["eager", "aot_eager"])
+@pytest.mark.parametrize("kind", ["sage", "gcn", "gat", "sage_hooked"])
+def test_layers_inside_a_compiled_model(kind, backend):
+    """torch.compile breaks its graph around the layers' operators: same outputs and gradients as without it."""
+    from apt_amd.layers import GATConv, GraphConv, SAGEConv
+    from apt_amd.sampler import Block
+    make = dict(sage=SAGEConv, sage_hooked=SAGEConv, gcn=GraphConv, gat=lambda a, b, activation: GATConv(a, b, 1, activation=activation))[kind]
+    gen = torch.Generator(device=DEV).manual_seed(7)
+    slots = [torch.randint(-1, n, (m * 5,), device=DEV, generator=gen) for n, m in ((900, 300), (300, 40))]
+    blocks = [Block(900, 300, None, slots[0], 5), Block(300, 40, None, slots[1], 5)]
+
+    class Model(torch.nn.Module):
+        def __init__(self):
+            super().__init__()
+            self.first, self.second = make(16, 32, activation=torch.relu), make(32, 8, activation=None)
+            if kind == "sage_hooked":      # the separate operations
+                self.first.fc_self.register_forward_hook(lambda module, args, out: out * 2)
+
+        def forward(self, x):
+            return self.second(blocks[1], self.first(blocks[0], x).flatten(1) * 0.5).flatten(1)
+
+    torch.manual_seed(5)
+    model = Model().to(DEV)
+    x = torch.randn(900, 16, device=DEV)
+    want = model(x)
+    grads = torch.autograd.grad(want.square().sum(), list(model.parameters()))
+    torch._dynamo.reset()
+    compiled = torch.compile(model, backend=backend)
+    got = compiled(x)
+    assert torch.allclose(got, want, rtol=1e-6, atol=1e-6)
+    for a, b in zip(torch.autograd.grad(got.square().sum(), list(model.parameters())), grads):
+        assert torch.allclose(a, b, rtol=1e-5, atol=1e-5)
+    with torch.no_grad():
+        assert torch.allclose(compiled(x), want, rtol=1e-5, atol=1e-5)
