@@ -1138,6 +1138,12 @@ std::tuple<Tensor, Tensor> aggregate_forward(const Tensor& relabeled, int64_t nu
   return {out, inv};
 }
 
+std::optional<Tensor> maybe(const Tensor& t) { return t.defined() ? std::optional<Tensor>(t) : std::nullopt; }
+
+// The same inside a backward pass whose own graph may be wanted (create_graph).
+Tensor aggregate_gradient(const Tensor& dz, const Tensor& relabeled, int64_t num_dst, int64_t fanout, int64_t num_src,
+                          const Tensor& dst_scale, const Tensor& csr_indptr, const Tensor& csr_indices, double scale = 1.0);
+
 struct BlockAggregateFn : public torch::autograd::Function<BlockAggregateFn> {
   static Tensor forward(torch::autograd::AutogradContext* ctx, const Tensor& x, const Tensor& relabeled, int64_t num_dst,
                         int64_t fanout, bool mean, const std::optional<Tensor>& csr_indptr,
@@ -1154,11 +1160,45 @@ struct BlockAggregateFn : public torch::autograd::Function<BlockAggregateFn> {
     const auto saved = ctx->get_saved_variables();
     Tensor dx;
     if (ctx->needs_input_grad(0))
-      dx = aggregate_backward(grads[0], saved[0], ctx->saved_data["num_dst"].toInt(), ctx->saved_data["fanout"].toInt(),
+      dx = aggregate_gradient(grads[0], saved[0], ctx->saved_data["num_dst"].toInt(), ctx->saved_data["fanout"].toInt(),
                               ctx->saved_data["num_src"].toInt(), saved[1], saved[2], saved[3]);
     return {dx, Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
   }
 };
+
+// That gradient is linear in dz, and its own gradient is the sum (or mean) again.
+struct AggregateGradientFn : public torch::autograd::Function<AggregateGradientFn> {
+  static Tensor forward(torch::autograd::AutogradContext* ctx, const Tensor& dz, const Tensor& relabeled, int64_t num_dst,
+                        int64_t fanout, int64_t num_src, const std::optional<Tensor>& dst_scale,
+                        const std::optional<Tensor>& csr_indptr, const std::optional<Tensor>& csr_indices, double scale) {
+    ctx->save_for_backward({relabeled, csr_indptr.value_or(Tensor()), csr_indices.value_or(Tensor())});
+    ctx->saved_data["num_dst"] = num_dst;
+    ctx->saved_data["fanout"] = fanout;
+    ctx->saved_data["mean"] = dst_scale.has_value();
+    ctx->saved_data["scale"] = scale;
+    return aggregate_backward(dz, relabeled, num_dst, fanout, num_src, dst_scale.value_or(Tensor()), csr_indptr.value_or(Tensor()),
+                              csr_indices.value_or(Tensor()), static_cast<float>(scale));
+  }
+  static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx,
+                                                 torch::autograd::variable_list grads) {
+    const auto saved = ctx->get_saved_variables();
+    Tensor ddz = BlockAggregateFn::apply(grads[0].contiguous(), saved[0], ctx->saved_data["num_dst"].toInt(),
+                                         ctx->saved_data["fanout"].toInt(), ctx->saved_data["mean"].toBool(), maybe(saved[1]),
+                                         maybe(saved[2]));
+    const double scale = ctx->saved_data["scale"].toDouble();
+    if (scale != 1.0) ddz = ddz * scale;
+    return {ddz, Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
+  }
+};
+
+Tensor aggregate_gradient(const Tensor& dz, const Tensor& relabeled, int64_t num_dst, int64_t fanout, int64_t num_src,
+                          const Tensor& dst_scale, const Tensor& csr_indptr, const Tensor& csr_indices, double scale) {
+  if (torch::GradMode::is_enabled())
+    return AggregateGradientFn::apply(dz, relabeled, num_dst, fanout, num_src, maybe(dst_scale), maybe(csr_indptr),
+                                      maybe(csr_indices), scale);
+  return aggregate_backward(dz, relabeled, num_dst, fanout, num_src, dst_scale, csr_indptr, csr_indices,
+                            static_cast<float>(scale));
+}
 
 }  // namespace
 
@@ -1220,7 +1260,7 @@ struct SageLayerFn : public torch::autograd::Function<SageLayerFn> {
     const int64_t num_dst = ctx->saved_data["num_dst"].toInt(), fanout = ctx->saved_data["fanout"].toInt();
     const int64_t num_src = x.size(0);
     const auto spread = [&](const Tensor& d) {
-      return aggregate_backward(d, relabeled, num_dst, fanout, num_src, inv, saved[6], saved[7]);
+      return aggregate_gradient(d, relabeled, num_dst, fanout, num_src, inv, saved[6], saved[7]);
     };
     const Tensor dz = before_relu(grads[0], saved[8]), self = x.narrow(0, 0, num_dst);
     const bool want_x = ctx->needs_input_grad(0), want_w = ctx->needs_input_grad(1) || ctx->needs_input_grad(2) || bias;
@@ -1301,9 +1341,8 @@ struct GcnLayerFn : public torch::autograd::Function<GcnLayerFn> {
     const auto saved = ctx->get_saved_variables();
     const Tensor &x = saved[0], &w = saved[1];
     const Tensor dz = before_relu(grads[0], saved[5]);
-    const Tensor dh = aggregate_backward(dz, saved[2], ctx->saved_data["num_dst"].toInt(), ctx->saved_data["fanout"].toInt(),
-                                         x.size(0), Tensor(), saved[3], saved[4],
-                                         static_cast<float>(ctx->saved_data["scale"].toDouble()));
+    const Tensor dh = aggregate_gradient(dz, saved[2], ctx->saved_data["num_dst"].toInt(), ctx->saved_data["fanout"].toInt(),
+                                         x.size(0), Tensor(), saved[3], saved[4], ctx->saved_data["scale"].toDouble());
     Tensor dx, dw, db;
     if (ctx->saved_data["bias"].toBool()) db = dz.sum(0);
     if (torch::GradMode::is_enabled()) {   // a graph of the gradients is wanted: operations that carry one
@@ -1337,6 +1376,33 @@ Tensor GcnLayer(const Tensor& relabeled, int64_t num_dst, int64_t fanout, const 
 // ---------------------------------------------------------------- GAT layer, from the dense product to the bias
 namespace {
 
+// The layer's gradients as operations that carry a graph (create_graph): it is stated again in torch, with the slots as an
+// index, and differentiated.  v: ft, attn_l, attn_r and the bias, or undefined.
+torch::autograd::variable_list gat_gradients_with_graph(const std::vector<Tensor>& v, const Tensor& relabeled, int64_t num_dst,
+                                                        int64_t fanout, double slope, const Tensor& d_out) {
+  std::vector<Tensor> in, wanted;   // aliases: a tensor that is given twice has a gradient in each place
+  for (const Tensor& t : v) {
+    in.push_back(t.defined() ? t.view_as(t) : t);
+    if (t.defined() && t.requires_grad()) wanted.push_back(in.back());
+  }
+  const int64_t n = v[0].size(0), heads = v[0].size(1), dim = v[0].size(2);
+  const Tensor ids = relabeled.narrow(0, 0, num_dst * fanout).view({num_dst, fanout});
+  const Tensor missing = (ids < 0).logical_or(ids >= n).unsqueeze(-1);
+  const Tensor at = ids.clamp(0, std::max<int64_t>(n - 1, 0)).view(-1);
+  const Tensor ft = in[0].to(torch::kFloat32);
+  const Tensor el = (ft * in[1].view({heads, dim})).sum(-1), er = (ft.narrow(0, 0, num_dst) * in[2].view({heads, dim})).sum(-1);
+  const Tensor e = at::leaky_relu(el.index_select(0, at).view({num_dst, fanout, heads}) + er.unsqueeze(1), slope);
+  const Tensor a = at::softmax(e.masked_fill(missing, -1e30), 1).masked_fill(missing, 0);
+  Tensor out = (a.unsqueeze(-1) * ft.index_select(0, at).view({num_dst, fanout, heads, dim})).sum(1).to(v[0].scalar_type());
+  if (in[3].defined()) out = out + in[3].view({heads, dim});
+  auto grads = torch::autograd::grad({out}, wanted, {d_out}, /*retain_graph=*/true, /*create_graph=*/true, /*allow_unused=*/true);
+  torch::autograd::variable_list result(v.size());
+  size_t next = 0;
+  for (size_t i = 0; i < v.size(); ++i)
+    if (v[i].defined() && v[i].requires_grad()) result[i] = grads[next++];
+  return result;
+}
+
 struct GatLayerFn : public torch::autograd::Function<GatLayerFn> {
   static Tensor forward(torch::autograd::AutogradContext* ctx, const Tensor& ft, const Tensor& attn_l, const Tensor& attn_r,
                         const std::optional<Tensor>& bias, const Tensor& relabeled, int64_t num_dst, int64_t fanout,
@@ -1362,7 +1428,7 @@ struct GatLayerFn : public torch::autograd::Function<GatLayerFn> {
                        csr_indptr->numel() == n + 1;
       ctx->save_for_backward({ft, attn_l, attn_r, relabeled, scores, attn, csr ? *csr_indptr : Tensor(),
                               csr ? *csr_indices : Tensor(), csr ? *csr_eids : Tensor(), csr ? *csc_indptr : Tensor(),
-                              relu ? out : Tensor()});
+                              relu ? out : Tensor(), bias.value_or(Tensor())});
       ctx->saved_data["num_dst"] = num_dst;
       ctx->saved_data["fanout"] = fanout;
       ctx->saved_data["slope"] = slope;
@@ -1379,6 +1445,12 @@ struct GatLayerFn : public torch::autograd::Function<GatLayerFn> {
     const int64_t n = ft.size(0), heads = ft.size(1), dim = ft.size(2);
     const bool bias = ctx->saved_data["bias"].toBool();
     const Tensor d_out = before_relu(grads[0], saved[10]);
+    if (torch::GradMode::is_enabled()) {
+      auto out = gat_gradients_with_graph({ft, attn_l, attn_r, saved[11]}, relabeled, num_dst, fanout,
+                                          ctx->saved_data["slope"].toDouble(), d_out);
+      out.resize(15);
+      return out;
+    }
     SourceOrder o;
     Tensor eids, csc;
     int64_t edges = 0;

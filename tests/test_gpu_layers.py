@@ -225,3 +225,71 @@ def test_layers_inside_a_compiled_model(kind, backend):
         assert torch.allclose(a, b, rtol=1e-5, atol=1e-5)
     with torch.no_grad():
         assert torch.allclose(compiled(x), want, rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("kind", ["aggregate", "aggregate_mean", "sage", "sage_first", "gcn", "gat", "gat_relu"])
+@pytest.mark.parametrize("with_csr", [False, True])
+def test_gradients_of_gradients(kind, with_csr):
+    """A gradient taken with create_graph, squared and differentiated again, against float64: every leaf's first and second
+    derivative (fp32 chains of six products and sums of up to a hundred terms: 1e-5 of a result's norm; bound 1e-4)."""
+    from apt_amd.layers import BlockAggregate, GATConv, GraphConv, SAGEConv
+    from apt_amd.sampler import Block
+    gen = torch.Generator(device=DEV).manual_seed(11)
+    num_dst, num_src, fanout = 30, 80, 6
+    rel = torch.randint(0, num_src, (num_dst * fanout,), device=DEV, generator=gen)
+    rel[torch.rand(rel.numel(), device=DEV, generator=gen) < 0.2] = -1
+    rel[:fanout] = -1
+    blk = Block(num_src, num_dst, None, rel, fanout)
+    if with_csr:
+        blk.csr()
+    keep = (rel >= 0).nonzero().flatten()
+    src, dst = rel[keep], keep // fanout
+    deg = torch.bincount(dst, minlength=num_dst).clamp(min=1)[:, None].double()
+    total = lambda h: torch.zeros(num_dst, h.shape[1], device=DEV, dtype=h.dtype).index_add(0, dst, h[src])  # noqa: E731
+    torch.manual_seed(2)
+    k, n = (12, 20) if kind != "sage_first" else (20, 12)
+    x = torch.randn(num_src, k, device=DEV, generator=gen)
+    if kind.startswith("aggregate"):
+        layer, mean = torch.nn.Linear(k, n).to(DEV), kind == "aggregate_mean"
+        run = lambda: BlockAggregate.apply(blk, layer(leaves[0]), mean)  # noqa: E731
+        state = lambda x, w, b: total(x @ w.t() + b) / (deg if mean else 1.0)  # noqa: E731
+    elif kind.startswith("sage"):
+        layer = SAGEConv(k, n, activation=torch.tanh).to(DEV)
+        run = lambda: layer(blk, leaves[0])  # noqa: E731
+        state = lambda x, wn, ws, b: torch.tanh(x[:num_dst] @ ws.t() + b + (total(x) / deg) @ wn.t())  # noqa: E731
+    elif kind == "gcn":
+        layer = GraphConv(k, n, activation=torch.tanh).to(DEV)
+        run = lambda: layer(blk, leaves[0])  # noqa: E731
+        state = lambda x, w, b: torch.tanh(total(x @ w) / fanout + b)  # noqa: E731
+    else:
+        layer = GATConv(k, 5, 3, activation=torch.relu if kind == "gat_relu" else None).to(DEV)
+        run = lambda: layer(blk, leaves[0])  # noqa: E731
+
+        def state(x, al, ar, b, w):
+            ft = (x @ w.t()).view(num_src, 3, 5)
+            el, er = (ft * al).sum(-1), (ft[:num_dst] * ar).sum(-1)
+            e = torch.exp(torch.nn.functional.leaky_relu(el[src] + er[dst], 0.2))
+            den = torch.zeros(num_dst, 3, device=DEV, dtype=e.dtype).index_add(0, dst, e)
+            out = torch.zeros(num_dst, 3, 5, device=DEV, dtype=e.dtype).index_add(0, dst, (e / den[dst])[:, :, None] * ft[src])
+            out = out + b.view(3, 5)
+            return out * (got_out > 0) if kind == "gat_relu" else out
+    with torch.no_grad():
+        for p in layer.parameters():
+            if p.dim() == 1:
+                p.normal_()
+    names = [name for name, _ in layer.named_parameters()]
+    order = {"sage": ["fc_neigh.weight", "fc_self.weight", "fc_self.bias"], "gcn": ["weight", "bias"],
+             "gat": ["attn_l", "attn_r", "bias", "fc.weight"], "aggregate": ["weight", "bias"]}[kind.split("_")[0]]
+    assert sorted(order) == sorted(names)
+    params = dict(layer.named_parameters())
+    leaves = [x.requires_grad_(True)] + [params[name] for name in order]
+    got_out = run()
+    w = torch.randn(got_out.shape, device=DEV, generator=gen)
+    exact = [t.detach().double().requires_grad_(True) for t in leaves]
+    want_out = state(*exact)
+    first = torch.autograd.grad((got_out.square() * w).sum(), leaves, create_graph=True)
+    want = torch.autograd.grad((want_out.square() * w.double()).sum(), exact, create_graph=True)
+    second = torch.autograd.grad(sum(g.square().sum() for g in first), leaves)
+    want2 = torch.autograd.grad(sum(g.square().sum() for g in want), exact)
+    for a, b, name in zip(first + second, want + want2, 2 * (["x"] + order)):
+        assert (a.double() - b).norm().item() <= 1e-4 * b.norm().item() + 1e-9, name
