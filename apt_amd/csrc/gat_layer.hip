@@ -624,7 +624,7 @@ extern "C" int apt_gat_layer_backward(const int64_t* neighbors, int64_t num_dst,
               (long long)num_dst, (long long)num_src, fanout, heads, (long long)dim);
   APT_REQUIRE((elem_size == 2 || elem_size == 4) && (attn_elem_size == 2 || attn_elem_size == 4), APT_EINVAL,
               "%s: elem_size %d, attn_elem_size %d (4 = fp32, 2 = bf16)", who, elem_size, attn_elem_size);
-  APT_REQUIRE(index_bytes == 4 || (index_bytes == 8 && eids != nullptr && csc_indptr != nullptr), APT_EINVAL,
+  APT_REQUIRE(index_bytes == 4 || (index_bytes == 8 && (eids != nullptr || num_edges == 0) && csc_indptr != nullptr), APT_EINVAL,
               "%s: index_bytes %d (4 = slots, 8 = destinations, with eids and csc_indptr)", who, index_bytes);
   APT_REQUIRE(workspace != nullptr && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0 &&
                   workspace_bytes >= apt_gat_layer_backward_workspace_bytes(num_dst, fanout, num_src, heads, dim, num_edges),
@@ -633,7 +633,8 @@ extern "C" int apt_gat_layer_backward(const int64_t* neighbors, int64_t num_dst,
     return gat_param_sums(static_cast<const float*>(workspace), 0, static_cast<int64_t>(heads) * dim, elem_size, attn_elem_size,
                           d_attn_l, d_attn_r, d_bias, static_cast<hipStream_t>(stream));
   APT_REQUIRE(ft != nullptr && attn_l != nullptr && attn_r != nullptr && el != nullptr && indptr != nullptr && d_ft != nullptr &&
-                  (num_dst == 0 || (neighbors != nullptr && er != nullptr && attn != nullptr && d_out != nullptr && index != nullptr)),
+                  (num_dst == 0 || (neighbors != nullptr && er != nullptr && attn != nullptr && d_out != nullptr &&
+                                    (index != nullptr || (index_bytes == 8 && num_edges == 0)))),
               APT_EINVAL, "%s: a tensor is NULL", who);
   hipStream_t st = static_cast<hipStream_t>(stream);
   const bool by_slot = index_bytes == 4;

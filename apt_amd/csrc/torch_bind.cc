@@ -1113,7 +1113,7 @@ Tensor aggregate_backward(const Tensor& dz_in, const Tensor& relabeled, int64_t 
   SourceOrder o;
   if (csr_indptr.defined() && csr_indptr.numel() == num_src + 1) {
     o.indptr = csr_indptr;
-    o.index = csr_indices;
+    o.index = csr_indices.numel() > 0 ? csr_indices : csr_indptr;   // (no edge: never read, and not NULL)
     o.bytes = 8;
   } else {
     o = source_order(relabeled, num_dst, fanout, num_src);

@@ -293,3 +293,27 @@ def test_gradients_of_gradients(kind, with_csr):
     want2 = torch.autograd.grad(sum(g.square().sum() for g in want), exact)
     for a, b, name in zip(first + second, want + want2, 2 * (["x"] + order)):
         assert (a.double() - b).norm().item() <= 1e-4 * b.norm().item() + 1e-9, name
+
+
+@pytest.mark.parametrize("kind", ["sage", "sage_first", "gcn", "gat"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_block_without_edges_whose_csr_was_emitted(kind, dtype):
+    """Destinations none of which has a neighbour: the CSR's index arrays are empty, and no gradient crosses the block."""
+    from apt_amd.layers import GATConv, GraphConv, SAGEConv
+    from apt_amd.sampler import Block
+    num_dst, num_src, fanout = 40, 70, 4
+    layer = {"sage": lambda: SAGEConv(8, 16), "sage_first": lambda: SAGEConv(16, 8), "gcn": lambda: GraphConv(8, 16),
+             "gat": lambda: GATConv(8, 8, 4)}[kind]().to(DEV, dtype)
+    x = torch.randn(num_src, 16 if kind == "sage_first" else 8, device=DEV).to(dtype).requires_grad_(True)
+    grads = []
+    for csr in (False, True):
+        blk = Block(num_src, num_dst, None, torch.full((num_dst * fanout,), -1, device=DEV), fanout)
+        if csr:
+            assert blk.csr()[1].numel() == 0
+        out = layer(blk, x)
+        grads.append(torch.autograd.grad(out.float().square().sum() + out.float().sum(), [x] + list(layer.parameters())))
+    for a, b in zip(*grads):
+        assert torch.equal(a, b)
+    want = layer.fc_self(x)[:num_dst] if kind.startswith("sage") else layer.bias.view(1, -1).expand(num_dst, -1)
+    assert torch.allclose(out.flatten(1).float(), want.float(), rtol=1e-5, atol=1e-6)
+    assert bool((grads[0][0][num_dst:] == 0).all())
