@@ -973,39 +973,65 @@ static void choose_ranges(int64_t num_dst, int64_t num_src, bool records_hold_ds
   L.ranges = fits ? static_cast<int>(ranges) : 0;
 }
 
+static void lay_out_ranges(size_t off, int64_t tiles, int64_t ranges, int64_t slots, FmtLayout& L) {
+  L.rtiles = tiles;
+  L.tile_cnt_off = off;  off = fmt_align(off + sizeof(uint32_t) * static_cast<size_t>(tiles));
+  L.hist_off = off;      off = fmt_align(off + sizeof(uint32_t) * static_cast<size_t>(tiles) * ranges);
+  L.bin_total_off = off; off = fmt_align(off + sizeof(uint32_t) * ranges);
+  L.start_off = off;     off = fmt_align(off + sizeof(uint32_t) * (ranges + 1));
+  L.rec_off = off;       L.total = fmt_align(off + sizeof(uint64_t) * static_cast<size_t>(slots));
+}
+
+static void lay_out_radix(size_t off, int64_t slots, FmtLayout& L) {
+  L.hist_off = off;      off = fmt_align(off + sizeof(uint32_t) * static_cast<size_t>(L.stiles) * kRadix);
+  L.bin_total_off = off; off = fmt_align(off + sizeof(uint32_t) * kRadix);
+  for (int k = 0; k < 2; ++k) {
+    L.key_off[k] = off; off = fmt_align(off + sizeof(uint32_t) * static_cast<size_t>(slots));
+    L.pay_off[k] = off; off = fmt_align(off + sizeof(uint32_t) * static_cast<size_t>(slots));
+  }
+  L.total = off;
+}
+
 static FmtLayout fmt_layout(int64_t num_dst, int fanout, int64_t num_src, bool csr, bool transpose = false) {
   FmtLayout L;
   L.ranges = 0;
+  L.rtiles = 0;
   L.slots = num_dst * fanout;
-  L.ctiles = ceil_div(L.slots > 0 ? L.slots : 1, kCompactTile);
-  L.stiles = ceil_div(L.slots > 0 ? L.slots : 1, kSortTile);
+  const int64_t slots = std::max<int64_t>(L.slots, 1);
+  L.ctiles = ceil_div(slots, kCompactTile);
+  L.stiles = ceil_div(slots, kSortTile);
   size_t off = 0;
   L.tile_cnt_off = off; off = fmt_align(off + sizeof(uint32_t) * static_cast<size_t>(L.ctiles));
   L.sums_off = off;     off = fmt_align(off + sizeof(uint32_t) * kScanChunk);
-  L.hist_off = off;
-  L.rtiles = 0;
-  if (csr) choose_ranges(num_dst, num_src, !transpose, L);
-  if (L.ranges > 0) {   // by either tile: which one is the launch's choice
-    L.rtiles = L.slots <= kRangeSmallBound ? ceil_div(std::max<int64_t>(L.slots, 1), kFmtBlock * kRangeSmallIters) : L.ctiles;
-    L.tile_cnt_off = off; off = fmt_align(off + sizeof(uint32_t) * static_cast<size_t>(L.rtiles));
-    L.hist_off = off;
-  }
-  if (csr && L.ranges > 0) {
-    off = fmt_align(off + sizeof(uint32_t) * static_cast<size_t>(L.rtiles) * L.ranges);
-    L.bin_total_off = off; off = fmt_align(off + sizeof(uint32_t) * L.ranges);
-    L.start_off = off;     off = fmt_align(off + sizeof(uint32_t) * (L.ranges + 1));
-    L.rec_off = off;       off = fmt_align(off + sizeof(uint64_t) * static_cast<size_t>(L.slots > 0 ? L.slots : 1));
-  } else if (csr) {
-    off = fmt_align(off + sizeof(uint32_t) * static_cast<size_t>(L.stiles) * kRadix);
-    L.bin_total_off = off; off = fmt_align(off + sizeof(uint32_t) * kRadix);
-    const size_t buf = sizeof(uint32_t) * static_cast<size_t>(L.slots > 0 ? L.slots : 1);
-    for (int k = 0; k < 2; ++k) {
-      L.key_off[k] = off; off = fmt_align(off + buf);
-      L.pay_off[k] = off; off = fmt_align(off + buf);
-    }
-  }
-  L.total = off;
+  L.total = L.hist_off = off;
+  if (!csr) return L;
+  choose_ranges(num_dst, num_src, !transpose, L);
+  // ranges: by either tile, which one is the launch's choice
+  if (L.ranges > 0)
+    lay_out_ranges(off, slots <= kRangeSmallBound ? ceil_div(slots, kFmtBlock * kRangeSmallIters) : L.ctiles, L.ranges, slots, L);
+  else
+    lay_out_radix(off, slots, L);
   return L;
+}
+
+// What a block within these bounds takes at the most: a caller may size one workspace for its largest block.  A smaller
+// block can have more ranges (narrower ones), more tiles (shorter ones) or other passes than the largest.
+static size_t fmt_workspace(int64_t num_dst, int fanout, int64_t num_src, bool csr, bool transpose = false) {
+  const FmtLayout L = fmt_layout(num_dst, fanout, num_src, csr, transpose);
+  if (!csr) return L.total;
+  const int64_t slots = std::max<int64_t>(L.slots, 1);
+  FmtLayout most = L;
+  const int64_t tiles = std::max(ceil_div(std::min(slots, kRangeSmallBound), kFmtBlock * kRangeSmallIters),
+                                 std::min(L.ctiles, kRangeMaxTiles));
+  const size_t head = fmt_align(sizeof(uint32_t) * static_cast<size_t>(L.ctiles)) + fmt_align(sizeof(uint32_t) * kScanChunk);
+  lay_out_ranges(head, tiles, std::min<int64_t>(range_index(num_src, kRangeShift2) + 1, kRangeMaxCount),
+                 std::min(slots, kRangeMaxTiles * kCompactTile), most);
+  size_t total = std::max(L.total, most.total);
+  if (!transpose) {
+    lay_out_radix(head, slots, most);
+    total = std::max(total, most.total);
+  }
+  return total;
 }
 
 static bool fmt_sizes_ok(int64_t num_dst, int fanout, int64_t num_src) {
@@ -1055,8 +1081,7 @@ static int launch_ranges(const CompactParams& c, RangeParams& r, const FmtLayout
 extern "C" size_t apt_block_transpose_workspace_bytes(int64_t num_dst, int fanout, int64_t num_src) {
   using namespace apt;
   if (!fmt_sizes_ok(num_dst, fanout, num_src)) return 0;
-  const FmtLayout L = fmt_layout(num_dst, fanout, num_src, true, true);
-  return L.ranges > 0 ? L.total : 0;
+  return fmt_layout(num_dst, fanout, num_src, true, true).ranges > 0 ? fmt_workspace(num_dst, fanout, num_src, true, true) : 0;
 }
 
 extern "C" int apt_block_transpose(const int64_t* relabeled, int64_t num_dst, int fanout, int64_t num_src,
@@ -1087,7 +1112,7 @@ extern "C" int apt_block_transpose(const int64_t* relabeled, int64_t num_dst, in
 extern "C" size_t apt_block_workspace_bytes(int64_t num_dst, int fanout, int64_t num_src, int want_csr) {
   using namespace apt;
   if (!fmt_sizes_ok(num_dst, fanout, num_src)) return 0;
-  return fmt_layout(num_dst, fanout, num_src, want_csr != 0).total;
+  return fmt_workspace(num_dst, fanout, num_src, want_csr != 0);
 }
 
 extern "C" int apt_block_formats(const int64_t* relabeled, int64_t num_dst, const int64_t* num_dst_dev,

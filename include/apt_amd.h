@@ -658,7 +658,7 @@ int apt_vir_send_offset(int world_size, int64_t base, const int64_t* sorted_node
  * (num_dst_dev as n_dev in apt_sample_neighbors; sources need no count): the
  * offsets of rows past the real counts equal the edge total, i.e. empty rows.
  * workspace: apt_block_workspace_bytes(num_dst, fanout, num_src, csr != NULL)
- * bytes of device scratch; 0 = sizes out of range. */
+ * bytes of device scratch, which do for every smaller block too; 0 = sizes out of range. */
 size_t apt_block_workspace_bytes(int64_t num_dst, int fanout, int64_t num_src, int want_csr);
 int apt_block_formats(const int64_t* relabeled, int64_t num_dst, const int64_t* num_dst_dev,
                       int fanout, int64_t num_src, int64_t* coo_row, int64_t* coo_col,

@@ -150,3 +150,38 @@ def test_gpu_csr_by_source_ranges(capi, num_dst, fanout, num_src):
     got = capi.block_formats(torch.from_numpy(r).cuda(), num_dst, fanout, num_src)
     _same({k: (v.cpu().numpy() if hasattr(v, "cpu") else v) for k, v in got.items()},
           _closed_form(r, num_dst, fanout, num_src))
+
+
+# (a block, a smaller one that takes more ranges of sources, shorter tiles or other passes)
+SMALLER = [((3000, 7, 2 ** 18 + 2700 * 1024), (3000, 7, 2 ** 18 + 2599 * 1024)), ((2 ** 21 + 2048, 1, 40000), (2 ** 21, 1, 40000)),
+           ((2 ** 20, 9, 2 ** 18 + 2600 * 1024 - 1), (2 ** 20, 8, 2 ** 18 + 2600 * 1024 - 1)),
+           ((2 ** 22, 2, 2 ** 22), (2 ** 21, 4, 2 ** 22)), ((300000, 10, 6_000_000), (300000, 10, 2_000_000))]
+
+
+def test_block_workspace_of_a_block_does_for_smaller_ones():
+    from apt_amd import capi
+    L = capi.lib()
+    rng = np.random.default_rng(5)
+    pairs = list(SMALLER)
+    for _ in range(3000):
+        big = [int(np.exp(rng.uniform(0, np.log(m)))) for m in (4e6, 30, 1e7)]
+        small = [int(v * rng.choice([1.0, 0.99, 0.5, rng.random()])) for v in big]
+        pairs.append((big, small))
+    for big, small in pairs:
+        for csr in (0, 1):
+            assert L.apt_block_workspace_bytes(*small, csr) <= L.apt_block_workspace_bytes(*big, csr), (big, small)
+        need = L.apt_block_transpose_workspace_bytes(*big)
+        if need:
+            assert 0 < L.apt_block_transpose_workspace_bytes(*small) <= need, (big, small)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("big,small", SMALLER[:2])
+def test_gpu_formats_of_a_smaller_block_in_the_same_buffers(capi, big, small):
+    import torch
+    f = capi.BlockFormats(*big)
+    r = _random_block(np.random.default_rng(1), *small)
+    f.num_dst, f.fanout, f.num_src = small
+    f.emit(torch.from_numpy(r).cuda())
+    got = f.narrow()
+    _same({k: (v.cpu().numpy() if hasattr(v, "cpu") else v) for k, v in got.items()}, _closed_form(r, *small))
