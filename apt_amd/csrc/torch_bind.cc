@@ -1023,6 +1023,12 @@ Tensor product(bool train, const Tensor& x, const Tensor& w, const Tensor& b = T
                : dense(x, w, Tensor(), Tensor(), b);
 }
 
+// Slots and CSR of a block that was made in inference mode: autograd keeps no such tensor, but a copy of it.
+Tensor keepable(bool train, const Tensor& t) { return train && t.is_inference() ? t.clone() : t; }
+std::optional<Tensor> keepable(bool train, const std::optional<Tensor>& t) {
+  return t.has_value() ? std::optional<Tensor>(keepable(train, *t)) : t;
+}
+
 // y = x w^T + b (or x w with `kn`: w is [k, n]).
 struct BlockLinearFn : public torch::autograd::Function<BlockLinearFn> {
   static Tensor forward(torch::autograd::AutogradContext* ctx, const Tensor& x, const Tensor& w,
@@ -1208,7 +1214,9 @@ Tensor BlockAggregate(const Tensor& relabeled, int64_t num_dst, int64_t fanout, 
   TORCH_CHECK_TYPE(x.is_cuda() && x.dim() == 2 &&
                        (x.scalar_type() == torch::kFloat32 || x.scalar_type() == torch::kBFloat16),
                    "npc: block_aggregate: input must be a 2-D fp32 or bf16 GPU tensor");
-  return BlockAggregateFn::apply(x.contiguous(), relabeled, num_dst, fanout, mean, csr_indptr, csr_indices);
+  const bool train = trains(x);
+  return BlockAggregateFn::apply(x.contiguous(), keepable(train, relabeled), num_dst, fanout, mean, keepable(train, csr_indptr),
+                                 keepable(train, csr_indices));
 }
 
 // ---------------------------------------------------------------- GraphSAGE layer
@@ -1307,8 +1315,9 @@ Tensor SageLayer(const Tensor& relabeled, int64_t num_dst, int64_t fanout, const
                   (!bias.has_value() || (bias->is_cuda() && bias->scalar_type() == t && bias->dim() == 1 &&
                                          bias->size(0) == w_self.size(0))),
               "npc: sage_layer: weights, bias and input do not fit each other");
-  return SageLayerFn::apply(x.contiguous(), w_neigh, w_self, bias, relabeled, num_dst, fanout, csr_indptr, csr_indices, relu,
-                            trains(x, w_neigh, w_self) || (bias.has_value() && trains(*bias)));
+  const bool train = trains(x, w_neigh, w_self) || (bias.has_value() && trains(*bias));
+  return SageLayerFn::apply(x.contiguous(), w_neigh, w_self, bias, keepable(train, relabeled), num_dst, fanout,
+                            keepable(train, csr_indptr), keepable(train, csr_indices), relu, train);
 }
 
 // ---------------------------------------------------------------- GCN layer
@@ -1369,8 +1378,9 @@ Tensor GcnLayer(const Tensor& relabeled, int64_t num_dst, int64_t fanout, const 
                   (!bias.has_value() || (bias->is_cuda() && bias->scalar_type() == t && bias->dim() == 1 &&
                                          bias->size(0) == w.size(1))),
               "npc: gcn_layer: weight, bias and input do not fit each other");
-  return GcnLayerFn::apply(x.contiguous(), w, bias, relabeled, num_dst, fanout, left, right, csr_indptr, csr_indices, relu,
-                           trains(x, w) || (bias.has_value() && trains(*bias)));
+  const bool train = trains(x, w) || (bias.has_value() && trains(*bias));
+  return GcnLayerFn::apply(x.contiguous(), w, bias, keepable(train, relabeled), num_dst, fanout, left, right,
+                           keepable(train, csr_indptr), keepable(train, csr_indices), relu, train);
 }
 
 // ---------------------------------------------------------------- GAT layer, from the dense product to the bias
@@ -1522,8 +1532,9 @@ Tensor GatLayer(const Tensor& relabeled, int64_t num_dst, int64_t fanout, const 
   }
   const bool want_grad = torch::GradMode::is_enabled() && (ft.requires_grad() || attn_l.requires_grad() || attn_r.requires_grad() ||
                                                           (b.has_value() && b->requires_grad()));
-  return GatLayerFn::apply(ft.contiguous(), attn_l.contiguous(), attn_r.contiguous(), b, relabeled, num_dst, fanout, slope,
-                           want_grad, csr_indptr, csr_indices, csr_eids, csc_indptr, relu,
+  return GatLayerFn::apply(ft.contiguous(), attn_l.contiguous(), attn_r.contiguous(), b, keepable(want_grad, relabeled), num_dst, fanout,
+                           slope, want_grad, keepable(want_grad, csr_indptr), keepable(want_grad, csr_indices),
+                           keepable(want_grad, csr_eids), keepable(want_grad, csc_indptr), relu,
                            fp32_result && !want_grad && ft.scalar_type() == torch::kBFloat16);
 }
 

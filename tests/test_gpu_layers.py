@@ -317,3 +317,27 @@ def test_block_without_edges_whose_csr_was_emitted(kind, dtype):
     want = layer.fc_self(x)[:num_dst] if kind.startswith("sage") else layer.bias.view(1, -1).expand(num_dst, -1)
     assert torch.allclose(out.flatten(1).float(), want.float(), rtol=1e-5, atol=1e-6)
     assert bool((grads[0][0][num_dst:] == 0).all())
+
+
+@pytest.mark.parametrize("kind", ["aggregate", "sage", "sage_first", "gcn", "gat"])
+@pytest.mark.parametrize("with_csr", [False, True])
+def test_training_on_a_block_made_in_inference_mode(kind, with_csr):
+    """Sampling needs no autograd, so a program may do it under torch.inference_mode()."""
+    from apt_amd.layers import BlockAggregate, GATConv, GraphConv, SAGEConv
+    from apt_amd.sampler import Block
+    slots = torch.from_numpy(np.random.default_rng(3).integers(-1, 90, size=30 * 5)).to(DEV)
+    torch.manual_seed(4)
+    layer = {"aggregate": lambda: torch.nn.Identity(), "sage": lambda: SAGEConv(8, 16), "sage_first": lambda: SAGEConv(8, 4),
+             "gcn": lambda: GraphConv(8, 16), "gat": lambda: GATConv(8, 8, 2)}[kind]().to(DEV)
+    x = torch.randn(90, 8, device=DEV, requires_grad=True)
+    grads = []
+    for mode in (False, True):
+        with torch.inference_mode(mode):
+            blk = Block(90, 30, None, slots.clone(), 5)
+            if with_csr:
+                blk.csr()
+            assert blk.relabeled.is_inference() == mode
+        out = BlockAggregate.apply(blk, x, True) if kind == "aggregate" else layer(blk, x)
+        grads.append(torch.autograd.grad(out.square().sum(), [x] + list(layer.parameters())))
+    for a, b in zip(*grads):
+        assert torch.equal(a, b)
