@@ -1023,6 +1023,8 @@ Tensor product(bool train, const Tensor& x, const Tensor& w, const Tensor& b = T
                : dense(x, w, Tensor(), Tensor(), b);
 }
 
+// What a gradient needs is kept until then; the rest stays free to be changed in place.
+Tensor kept_if(bool needed, const Tensor& t) { return needed ? t : Tensor(); }
 // Slots and CSR of a block that was made in inference mode: autograd keeps no such tensor, but a copy of it.
 Tensor keepable(bool train, const Tensor& t) { return train && t.is_inference() ? t.clone() : t; }
 std::optional<Tensor> keepable(bool train, const std::optional<Tensor>& t) {
@@ -1033,9 +1035,9 @@ std::optional<Tensor> keepable(bool train, const std::optional<Tensor>& t) {
 struct BlockLinearFn : public torch::autograd::Function<BlockLinearFn> {
   static Tensor forward(torch::autograd::AutogradContext* ctx, const Tensor& x, const Tensor& w,
                         const std::optional<Tensor>& b, bool kn, bool train) {
-    ctx->save_for_backward({x, w});
+    ctx->save_for_backward({kept_if(w.requires_grad(), x), kept_if(x.requires_grad(), w)});
     ctx->saved_data["kn"] = kn;
-    ctx->saved_data["bias"] = b.has_value();
+    ctx->saved_data["bias"] = b.has_value() && b->requires_grad();
     if (train && kn) return at::mm(x, w);
     return product(train, x, kn ? w.t() : w, b.value_or(Tensor()));
   }
@@ -1047,11 +1049,12 @@ struct BlockLinearFn : public torch::autograd::Function<BlockLinearFn> {
     Tensor dx, dw, db;
     if (torch::GradMode::is_enabled()) {   // a graph of the gradients is wanted: operations that carry one
       if (ctx->needs_input_grad(0)) dx = kn ? dy.mm(w.t()) : dy.mm(w);
-      dw = kn ? x.t().mm(dy) : dy.t().mm(x);
+      if (ctx->needs_input_grad(1)) dw = kn ? x.t().mm(dy) : dy.t().mm(x);
       if (bias) db = dy.sum(0);
     } else {
       if (ctx->needs_input_grad(0)) dx = dense(dy, kn ? w : w.t());
-      if (ctx->needs_input_grad(1) || bias) std::tie(dw, db) = kn ? linear_wgrad(x, dy, false) : linear_wgrad(dy, x, bias);
+      if (ctx->needs_input_grad(1)) std::tie(dw, db) = kn ? linear_wgrad(x, dy, false) : linear_wgrad(dy, x, bias);
+      else if (bias) db = dy.sum(0);
     }
     return {dx, dw, db, Tensor(), Tensor()};
   }
@@ -1253,9 +1256,12 @@ struct SageLayerFn : public torch::autograd::Function<SageLayerFn> {
         out = dense(self, w_self, mean, w_neigh, b, Tensor(), relu);
       }
     }
-    ctx->save_for_backward({x, w_neigh, w_self, relabeled, inv, mean, csr_indptr.value_or(Tensor()),
-                            csr_indices.value_or(Tensor()), relu ? out : Tensor()});
-    ctx->saved_data["bias"] = bias.has_value();
+    ctx->save_for_backward({kept_if(w_neigh.requires_grad() || w_self.requires_grad(), x), kept_if(x.requires_grad(), w_neigh),
+                            kept_if(x.requires_grad(), w_self), relabeled, inv, kept_if(w_neigh.requires_grad(), mean),
+                            csr_indptr.value_or(Tensor()), csr_indices.value_or(Tensor()), relu ? out : Tensor()});
+    ctx->saved_data["bias"] = bias.has_value() && bias->requires_grad();
+    ctx->saved_data["first"] = first;
+    ctx->saved_data["num_src"] = x.size(0);
     ctx->saved_data["num_dst"] = num_dst;
     ctx->saved_data["fanout"] = fanout;
     return out;
@@ -1264,29 +1270,29 @@ struct SageLayerFn : public torch::autograd::Function<SageLayerFn> {
                                                  torch::autograd::variable_list grads) {
     const auto saved = ctx->get_saved_variables();
     const Tensor &x = saved[0], &w_neigh = saved[1], &w_self = saved[2], &relabeled = saved[3], &inv = saved[4];
-    const bool bias = ctx->saved_data["bias"].toBool(), first = x.size(1) > w_self.size(0);
+    const bool bias = ctx->saved_data["bias"].toBool(), first = ctx->saved_data["first"].toBool();
     const int64_t num_dst = ctx->saved_data["num_dst"].toInt(), fanout = ctx->saved_data["fanout"].toInt();
-    const int64_t num_src = x.size(0);
+    const int64_t num_src = ctx->saved_data["num_src"].toInt();
     const auto spread = [&](const Tensor& d) {
       return aggregate_gradient(d, relabeled, num_dst, fanout, num_src, inv, saved[6], saved[7]);
     };
-    const Tensor dz = before_relu(grads[0], saved[8]), self = x.narrow(0, 0, num_dst);
-    const bool want_x = ctx->needs_input_grad(0), want_w = ctx->needs_input_grad(1) || ctx->needs_input_grad(2) || bias;
-    Tensor dx, dwn, dws, db;
+    const Tensor dz = before_relu(grads[0], saved[8]), self = x.defined() ? x.narrow(0, 0, num_dst) : x;
+    const bool want_x = ctx->needs_input_grad(0), want_n = ctx->needs_input_grad(1), want_s = ctx->needs_input_grad(2);
+    Tensor dpre, dx, dwn, dws, db;
+    if (first && (want_x || want_n)) dpre = spread(dz);
     if (torch::GradMode::is_enabled()) {   // a graph of the gradients is wanted: operations that carry one
-      const Tensor dzn = first ? spread(dz) : dz.mm(w_neigh);
-      const Tensor mean = first ? Tensor() : BlockAggregateFn::apply(x, relabeled, num_dst, fanout, true, std::nullopt, std::nullopt);
-      dx = (first ? dzn.mm(w_neigh) : spread(dzn)) + at::constant_pad_nd(dz.mm(w_self), {0, 0, 0, num_src - num_dst});
-      dwn = first ? dzn.t().mm(x) : dz.t().mm(mean);
-      dws = dz.t().mm(self);
+      if (want_x)
+        dx = (first ? dpre.mm(w_neigh) : spread(dz.mm(w_neigh))) +
+             at::constant_pad_nd(dz.mm(w_self), {0, 0, 0, num_src - num_dst});
+      if (want_n)
+        dwn = first ? dpre.t().mm(x)
+                    : dz.t().mm(BlockAggregateFn::apply(x, relabeled, num_dst, fanout, true, std::nullopt, std::nullopt));
+      if (want_s) dws = dz.t().mm(self);
       if (bias) db = dz.sum(0);
     } else {
-      Tensor dpre;
-      if (first) dpre = spread(dz);
-      if (want_w) {
-        std::tie(dws, db) = linear_wgrad(dz, self, bias);
-        dwn = std::get<0>(first ? linear_wgrad(dpre, x, false) : linear_wgrad(dz, saved[5], false));
-      }
+      if (want_s) std::tie(dws, db) = linear_wgrad(dz, self, bias);
+      else if (bias) db = dz.sum(0);
+      if (want_n) dwn = std::get<0>(first ? linear_wgrad(dpre, x, false) : linear_wgrad(dz, saved[5], false));
       if (want_x)
         dx = first ? dense(dpre, w_neigh.t(), dz, w_self.t()) : [&] {
           Tensor d = spread(dense(dz, w_neigh.t()));
@@ -1337,9 +1343,10 @@ struct GcnLayerFn : public torch::autograd::Function<GcnLayerFn> {
     const double scale = left * right;
     const Tensor out = std::get<0>(aggregate_forward(relabeled, num_dst, fanout, h, false,
                                                      static_cast<float>(exact ? right : scale), b, relu));
-    ctx->save_for_backward({x, w, relabeled, csr_indptr.value_or(Tensor()), csr_indices.value_or(Tensor()),
-                            relu ? out : Tensor()});
-    ctx->saved_data["bias"] = bias.has_value();
+    ctx->save_for_backward({kept_if(w.requires_grad(), x), kept_if(x.requires_grad(), w), relabeled,
+                            csr_indptr.value_or(Tensor()), csr_indices.value_or(Tensor()), relu ? out : Tensor()});
+    ctx->saved_data["bias"] = bias.has_value() && bias->requires_grad();
+    ctx->saved_data["num_src"] = x.size(0);
     ctx->saved_data["num_dst"] = num_dst;
     ctx->saved_data["fanout"] = fanout;
     ctx->saved_data["scale"] = scale;
@@ -1350,13 +1357,15 @@ struct GcnLayerFn : public torch::autograd::Function<GcnLayerFn> {
     const auto saved = ctx->get_saved_variables();
     const Tensor &x = saved[0], &w = saved[1];
     const Tensor dz = before_relu(grads[0], saved[5]);
-    const Tensor dh = aggregate_gradient(dz, saved[2], ctx->saved_data["num_dst"].toInt(), ctx->saved_data["fanout"].toInt(),
-                                         x.size(0), Tensor(), saved[3], saved[4], ctx->saved_data["scale"].toDouble());
-    Tensor dx, dw, db;
+    Tensor dh, dx, dw, db;
+    if (ctx->needs_input_grad(0) || ctx->needs_input_grad(1))
+      dh = aggregate_gradient(dz, saved[2], ctx->saved_data["num_dst"].toInt(), ctx->saved_data["fanout"].toInt(),
+                              ctx->saved_data["num_src"].toInt(), Tensor(), saved[3], saved[4],
+                              ctx->saved_data["scale"].toDouble());
     if (ctx->saved_data["bias"].toBool()) db = dz.sum(0);
     if (torch::GradMode::is_enabled()) {   // a graph of the gradients is wanted: operations that carry one
       if (ctx->needs_input_grad(0)) dx = dh.mm(w.t());
-      dw = x.t().mm(dh);
+      if (ctx->needs_input_grad(1)) dw = x.t().mm(dh);
     } else {
       if (ctx->needs_input_grad(0)) dx = dense(dh, w);
       if (ctx->needs_input_grad(1)) dw = std::get<0>(linear_wgrad(x, dh, false));

@@ -341,3 +341,33 @@ def test_training_on_a_block_made_in_inference_mode(kind, with_csr):
         grads.append(torch.autograd.grad(out.square().sum(), [x] + list(layer.parameters())))
     for a, b in zip(*grads):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("kind", ["sage", "sage_first", "gcn", "gat"])
+@pytest.mark.parametrize("change", ["rows", "weights"])
+def test_what_no_gradient_needs_may_be_changed_in_place(kind, change):
+    """Rows under frozen weights, and weights above rows that need no gradient, between forward and backward: nn.Linear
+    keeps neither, and so do the layers."""
+    from apt_amd.layers import GATConv, GraphConv, SAGEConv
+    from apt_amd.sampler import Block
+    blk = Block(90, 30, None, torch.from_numpy(np.random.default_rng(3).integers(-1, 90, size=30 * 5)).to(DEV), 5)
+    grads = []
+    for touched in (False, True):
+        torch.manual_seed(4)
+        layer = {"sage": lambda: SAGEConv(8, 16), "sage_first": lambda: SAGEConv(8, 4), "gcn": lambda: GraphConv(8, 16),
+                 "gat": lambda: GATConv(8, 8, 2)}[kind]().to(DEV)
+        weights = [p for n, p in layer.named_parameters() if n.endswith("weight")]
+        leaf = torch.randn(90, 8, device=DEV, requires_grad=change == "rows")
+        if change == "rows":
+            for p in weights:
+                p.requires_grad_(False)
+        x = leaf * 1.0
+        out = layer(blk, x)
+        if touched:
+            with torch.no_grad():
+                for t in [x] if change == "rows" else weights:
+                    t.mul_(3.0)
+        wanted = [leaf, layer.bias if kind in ("gcn", "gat") else layer.fc_self.bias] if change == "rows" else weights
+        grads.append(torch.autograd.grad((out * torch.linspace(-1, 1, out.numel(), device=DEV).view(out.shape)).sum(), wanted))
+    for a, b in zip(*grads):
+        assert torch.equal(a, b) and bool((a != 0).any())
