@@ -13,9 +13,9 @@
 // COO/CSC are a stream compaction (count per tile -> place).  CSR of the blocks a
 // sampler makes is a partition by source range carried along with that
 // compaction, then a counting sort of every range in one workgroup (below, "CSR by
-// source ranges"): four launches for all three formats.  Blocks of more than 5 M
-// sources, 8 M slots or 2 M destinations take a stable least-significant-digit radix
-// sort of (source, edge id) by source, 8 bits per pass (histogram per tile ->
+// source ranges"): four launches for all three formats.  Blocks of more than 6 M
+// sources, 8 M slots or 2 M destinations, and blocks of very few sources, take a stable
+// least-significant-digit radix sort of (source, edge id) by source, 8 bits per pass (histogram per tile ->
 // scatter).  Everywhere a workgroup ranks its tile with wave ballots, so equal keys
 // keep their order and the result is reproducible (no atomic tickets).  A block
 // of a mini-batch has few tiles, so the place and scatter workgroups add up the
@@ -461,16 +461,21 @@ __global__ __launch_bounds__(kSortBlock) void radix_scatter_kernel(SortParams p)
 // of them over a few tiles only (a radix pass over the 260 k edges of a batch of
 // 1024 is 64 workgroups on 256 CUs).  All three formats of a block, with radix
 // passes / with ranges, sizes exact: 8 k edges 40 / 22 us, 22 k 41 / 25, 260 k
-// (120 k sources) 79 / 33, 740 k (240 k) 88 / 49, 940 k (460 k) 89 / 50 us.
+// (120 k sources) 79 / 33, 740 k (240 k) 88 / 49, 940 k (460 k) 89 / 50 us.  With edges in long ranges (1 M edges; one
+// source in every tenth slot, with a low / a high id): 98 / 55, 98 / 73; all edges in one: 96 / 64, 294 / 132; four
+// sources in four of ten slots: 97 / 86 us.
 // The relabel numbers nodes by first occurrence, so hubs have small ids and the
 // edges per source fall off about as 1 / id (2.4 M-node graph, 4096 seeds: 40 edges
 // per source at id 4500, 5 at 30 k, 1.4 at 200 k), and buffers sized by upper bounds
 // end in ids that do not occur.  Ranges of equal width would leave one workgroup with
-// 37 k records (93 us); three widths keep them between a few hundred and a few thousand.
+// 37 k records (93 us); four widths keep them between a few hundred and a few thousand.
 constexpr int kRangeMaxShift = 11;
+// The first sources have a range each: the worst hubs, and all sources of a block that has few.  Such a range needs no
+// sort, so any number of workgroups may share it (range_sort_kernel).
+constexpr int64_t kRangeFrom0 = 256;                                                // sources with a range each
 constexpr int64_t kRangeFrom1 = int64_t{1} << 15, kRangeFrom2 = int64_t{1} << 18;   // first sources of pieces 1, 2
 constexpr int kRangeShift0 = 5, kRangeShift1 = 8, kRangeShift2 = 10;
-constexpr int kRangeMaxCount = 4520;          // ranges: 12 bytes of LDS each in the place pass
+constexpr int kRangeMaxCount = 5016;          // ranges: 12 bytes of LDS each in the place pass
 constexpr int64_t kRangeMaxTiles = 4096;
 // A tile of the partition: 1024 slots (four per thread) instead of 2048 while the edges are few and workgroups with them.
 // Every tile walks all ranges, so a large block is better off with half the tiles.  CSR of 8 k / 260 k / 730 k / 950 k /
@@ -479,18 +484,30 @@ constexpr int64_t kRangeMaxTiles = 4096;
 constexpr int64_t kRangeSmallSlots = int64_t{1} << 19, kRangeSmallBound = int64_t{1} << 21;
 constexpr int kRangeSmallIters = 4;
 constexpr int kRangeKeyBits = kRangeMaxShift;
-constexpr int kRangeEdgeBits = 31;
-constexpr int64_t kRangeMaxDst = int64_t{1} << (64 - kRangeKeyBits - kRangeEdgeBits - 1);
+constexpr int kRangeEdgeBits = 32;
+constexpr int64_t kRangeMaxDst = int64_t{1} << (64 - kRangeKeyBits - kRangeEdgeBits);
 constexpr int kRangeSortBlock = 256;
 constexpr int kRangeSortWaves = kRangeSortBlock / kWave;
 constexpr int kRangeSortRounds = 8;
 constexpr int kRangeSortChunk = kRangeSortBlock * kRangeSortRounds;
+// A range of more records than four times the mean is sorted in parts, within these bounds.
+constexpr int64_t kRangeLong = 2 * kRangeSortChunk, kRangeLongest = 8 * kRangeSortChunk;
+constexpr int kRangePart = kRangeSortChunk;            // records of a part: this many, or a 64th of the range
+constexpr int kRangeMaxParts = 64;
+constexpr int kRangePartGroups = 512;
 constexpr int kRangeScanGroups = 16;          // tile groups of a scan workgroup
 
 struct RangeParams {
   int shift2;                 // width of piece 2
   int ranges;
   int tile;                   // slots of a workgroup
+  int part_groups;            // workgroups of the sort that take parts of long ranges
+  uint32_t long_from;         // a range of more records is sorted in parts
+  int row_words;              // keys of the widest range
+  uint32_t* parts;            // [1]: number of parts
+  uint32_t* part0;            // [ranges]: a long range's first part
+  uint32_t* part_range;       // [parts]
+  uint32_t* part_keys;        // [parts][row_words]: records of a part per source
   uint32_t* hist;             // [tiles][ranges]: edges of a tile per range, then their prefix over the tiles
   uint32_t* total;            // [ranges]
   uint32_t* start;            // [ranges + 1]: a range's first record
@@ -503,19 +520,22 @@ struct RangeParams {
   uint32_t* t_slots;
 };
 
-constexpr int kRangeCount0 = static_cast<int>(kRangeFrom1 >> kRangeShift0);
+constexpr int kRangeSingles = static_cast<int>(kRangeFrom0);
+constexpr int kRangeCount0 = kRangeSingles + static_cast<int>((kRangeFrom1 - kRangeFrom0) >> kRangeShift0);   // ranges up to piece 1
 constexpr int kRangeCount1 = static_cast<int>((kRangeFrom2 - kRangeFrom1) >> kRangeShift1);
 
 __host__ __device__ __forceinline__ int64_t range_index(int64_t src, int shift2) {
-  return src < kRangeFrom1   ? src >> kRangeShift0
+  return src < kRangeFrom0   ? src
+         : src < kRangeFrom1 ? kRangeSingles + ((src - kRangeFrom0) >> kRangeShift0)
          : src < kRangeFrom2 ? kRangeCount0 + ((src - kRangeFrom1) >> kRangeShift1)
                              : kRangeCount0 + kRangeCount1 + ((src - kRangeFrom2) >> shift2);
 }
 __device__ __forceinline__ int range_shift(const RangeParams& r, int b) {
-  return b < kRangeCount0 ? kRangeShift0 : b < kRangeCount0 + kRangeCount1 ? kRangeShift1 : r.shift2;
+  return b < kRangeSingles ? 0 : b < kRangeCount0 ? kRangeShift0 : b < kRangeCount0 + kRangeCount1 ? kRangeShift1 : r.shift2;
 }
 __device__ __forceinline__ int64_t range_first(const RangeParams& r, int b) {
-  return b < kRangeCount0 ? static_cast<int64_t>(b) << kRangeShift0
+  return b < kRangeSingles ? b
+         : b < kRangeCount0 ? kRangeFrom0 + (static_cast<int64_t>(b - kRangeSingles) << kRangeShift0)
          : b < kRangeCount0 + kRangeCount1 ? kRangeFrom1 + (static_cast<int64_t>(b - kRangeCount0) << kRangeShift1)
                                            : kRangeFrom2 + (static_cast<int64_t>(b - kRangeCount0 - kRangeCount1) << r.shift2);
 }
@@ -528,6 +548,11 @@ __device__ __forceinline__ uint32_t range_key(const RangeParams& r, int b, int64
   const int64_t k = src - range_first(r, b), last = (int64_t{1} << range_shift(r, b)) - 1;
   return static_cast<uint32_t>(k < last ? k : last);
 }
+
+__device__ __forceinline__ uint32_t part_length(uint32_t n) {   // a multiple of a chunk
+  return max(static_cast<uint32_t>(kRangePart), (n / kRangeMaxParts + kRangeSortChunk) / kRangeSortChunk * kRangeSortChunk);
+}
+__device__ __forceinline__ uint32_t part_count(uint32_t n) { return (n + part_length(n) - 1) / part_length(n); }
 
 // Lanes of the wavefront that hold the same value (its low `bits` bits) as this one, among `valid` lanes.
 __device__ __forceinline__ uint64_t same_value(uint32_t v, int bits, bool valid) {
@@ -549,6 +574,7 @@ __global__ __launch_bounds__(kFmtBlock) void range_count_kernel(CompactParams p,
   const int64_t slots = actual_count(p.num_dst, p.num_dst_dev) * p.fanout;
   const int64_t base = static_cast<int64_t>(blockIdx.x) * (kFmtBlock * ITERS);
   if (base >= slots && blockIdx.x != 0) return;   // block-uniform: nobody reads an inactive tile's counts
+  if (blockIdx.x == 0 && threadIdx.x == 0) *r.parts = 0;
   int64_t v[ITERS];
 #pragma unroll
   for (int it = 0; it < ITERS; ++it) {
@@ -579,6 +605,7 @@ __global__ __launch_bounds__(kFmtBlock) void range_count_kernel(CompactParams p,
 __global__ __launch_bounds__(kWave * kRangeScanGroups) void range_scan_kernel(CompactParams p, RangeParams r) {
   constexpr int kUnroll = 8;
   __shared__ uint32_t s_sum[kRangeScanGroups][kWave];
+  __shared__ uint32_t s_part0[kWave];
   const int lane = threadIdx.x % kWave, group = threadIdx.x / kWave;
   const int b = blockIdx.x * kWave + lane;
   const int64_t slots = actual_count(p.num_dst, p.num_dst_dev) * p.fanout;
@@ -602,6 +629,22 @@ __global__ __launch_bounds__(kWave * kRangeScanGroups) void range_scan_kernel(Co
     const uint32_t c = s_sum[g][lane];
     if (g < group) run += c;
     all += c;
+  }
+  uint64_t lengthy = ballot(live && all > r.long_from);   // (every wavefront has the same lanes' totals)
+  if (lengthy != 0) {   // block-uniform: number their parts, and clear the counts that the place pass adds to
+    if (group == 0 && ((lengthy >> lane) & 1)) {
+      const uint32_t parts = part_count(all), part0 = atomicAdd(r.parts, parts);
+      r.part0[b] = s_part0[lane] = part0;
+      for (uint32_t q = 0; q < parts; ++q) r.part_range[part0 + q] = b;
+    }
+    __syncthreads();
+    for (; lengthy != 0; lengthy &= lengthy - 1) {
+      const int src = __ffsll(static_cast<long long>(lengthy)) - 1;
+      const int keys = 1 << range_shift(r, blockIdx.x * kWave + src);
+      const uint32_t words = keys > 1 ? part_count(__shfl(all, src, kWave)) * r.row_words : 0u;
+      uint32_t* row = r.part_keys + static_cast<int64_t>(s_part0[src]) * r.row_words;
+      for (uint32_t i = threadIdx.x; i < words; i += kWave * kRangeScanGroups) row[i] = 0;
+    }
   }
   if (!live) return;
   for (int t = t0; t < t1; t += kUnroll) {
@@ -628,13 +671,16 @@ __global__ __launch_bounds__(kFmtBlock) void range_place_kernel(CompactParams p,
   const int words = (r.ranges + 1) / 2;                                      // 32-bit words of a wave's counts
   __shared__ uint32_t s_edges[kFmtWaves * ITERS];
   __shared__ uint32_t s_wave[kFmtWaves];
+  __shared__ int s_long;                                                     // whether there are long ranges
   const int lane = lane_id();
   const int wave = threadIdx.x / kWave;
   const int64_t slots = actual_count(p.num_dst, p.num_dst_dev) * p.fanout;
   const int64_t upper = p.num_dst * p.fanout;
+  if (threadIdx.x == 0) s_long = 0;
   const int64_t base = static_cast<int64_t>(blockIdx.x) * (kFmtBlock * ITERS) + wave * (ITERS * kWave);
   int64_t v[ITERS];
   uint32_t below[ITERS];
+  int range[ITERS];
 #pragma unroll
   for (int it = 0; it < ITERS; ++it) {
     const int64_t s = base + it * kWave + lane;
@@ -648,10 +694,9 @@ __global__ __launch_bounds__(kFmtBlock) void range_place_kernel(CompactParams p,
     const uint64_t m = ballot(v[it] >= 0);
     below[it] = rank_below(m);
     if (lane == 0) s_edges[wave * ITERS + it] = __popcll(m);
-    if (v[it] >= 0) {   // at most 512 per wavefront: a 16-bit half never overflows into the other
-      const int b = range_of(r, v[it]);
-      atomicAdd(&cnt[b >> 1], (b & 1) ? 0x10000u : 1u);
-    }
+    range[it] = v[it] >= 0 ? range_of(r, v[it]) : 0;
+    if (v[it] >= 0)   // at most 512 per wavefront: a 16-bit half never overflows into the other
+      atomicAdd(&cnt[range[it] >> 1], (range[it] & 1) ? 0x10000u : 1u);
   }
   const int64_t active = ceil_div_dev(slots, (kFmtBlock * ITERS));
   uint32_t first = 0;
@@ -682,7 +727,10 @@ __global__ __launch_bounds__(kFmtBlock) void range_place_kernel(CompactParams p,
       for (int u = 0; u < kBatch; ++u) c[u] = r.total[min(b + u * kFmtBlock, r.ranges - 1)];
 #pragma unroll
       for (int u = 0; u < kBatch; ++u)
-        if (b + u * kFmtBlock < r.ranges) s_base[b + u * kFmtBlock] = c[u];
+        if (b + u * kFmtBlock < r.ranges) {
+          s_base[b + u * kFmtBlock] = c[u];
+          if (c[u] > r.long_from && b + u * kFmtBlock >= kRangeSingles) s_long = 1;
+        }
     }
     __syncthreads();
     const int per = (r.ranges + kFmtBlock - 1) / kFmtBlock;
@@ -745,7 +793,7 @@ __global__ __launch_bounds__(kFmtBlock) void range_place_kernel(CompactParams p,
     if (FORMATS && s < upper && static_cast<uint32_t>(s) - d * fan == 0) p.csc_indptr[d] = e;
     const bool valid = v[it] >= 0;
     if (ballot(valid) == 0) continue;   // wave-uniform
-    const uint32_t b = valid ? static_cast<uint32_t>(range_of(r, v[it])) : 0u;
+    const uint32_t b = static_cast<uint32_t>(range[it]);
     const uint64_t peers = same_value(b, bits, valid);
     const uint32_t rank = rank_below(peers);
     uint32_t at = 0;
@@ -761,19 +809,33 @@ __global__ __launch_bounds__(kFmtBlock) void range_place_kernel(CompactParams p,
       r.rec[s_base[b] + at] = (static_cast<uint64_t>(d) << (kRangeKeyBits + kRangeEdgeBits)) |
                               (static_cast<uint64_t>(range_key(r, static_cast<int>(b), v[it])) << kRangeEdgeBits) | static_cast<uint64_t>(e);
     }
+    if (s_long != 0) {   // block-uniform: count the edges of a long range's part per source
+      const uint32_t n = r.total[b];
+      const bool count = valid && b >= static_cast<uint32_t>(kRangeSingles) && n > r.long_from;
+      uint32_t cell = 0;
+      if (count) {
+        const uint32_t before = r.hist[static_cast<int64_t>(blockIdx.x) * r.ranges + b] + at;   // records of the range
+        cell = (r.part0[b] + before / part_length(n)) * r.row_words + range_key(r, static_cast<int>(b), v[it]);
+      }
+      uint64_t todo = ballot(count);
+      for (int t = 0; t < 4 && todo != 0; ++t) {   // a hub's lanes together, the others by themselves
+        const int leader = __ffsll(static_cast<long long>(todo)) - 1;
+        const uint64_t same = ballot(cell == __shfl(cell, leader, kWave)) & todo;
+        if (lane == leader) atomicAdd(&r.part_keys[cell], static_cast<uint32_t>(__popcll(same)));
+        todo &= ~same;
+      }
+      if ((todo >> lane) & 1) atomicAdd(&r.part_keys[cell], 1u);
+    }
   }
 }
 
 // One workgroup per range: stable counting sort of its records by source.  A range of a sampled block has about a
-// thousand; a range with more than a chunk of them (hubs) is walked chunk by chunk, after a counting walk.
+// thousand; one with more than a chunk of them is walked chunk by chunk, after a counting walk.  A long range (a hub, or
+// a block of few sources) would keep its workgroup busy long after the others are done: it is cut into parts for the
+// first `part_groups` workgroups of the launch.  The place pass has counted a long range's records per part and source.
 template <bool FORMATS>
 __global__ __launch_bounds__(kRangeSortBlock) void range_sort_kernel(RangeParams r) {
   extern __shared__ uint32_t s_range[];
-  const int shift = range_shift(r, blockIdx.x);
-  const int keys = 1 << shift;
-  const int words = keys / 2;
-  uint32_t* s_start = s_range;              // [keys]: next position of a key's first record not yet placed
-  uint32_t* s_cnt2 = s_range + keys;        // [waves][keys / 2], 16-bit counts
   __shared__ uint32_t s_wave[kRangeSortWaves];
   const int tid = threadIdx.x, lane = lane_id(), wave = tid / kWave;
   auto exclusive = [&](uint32_t x, uint32_t& all) {   // over the workgroup
@@ -796,109 +858,159 @@ __global__ __launch_bounds__(kRangeSortBlock) void range_sort_kernel(RangeParams
     }
     return before + incl - x;
   };
-  const uint32_t before = r.start[blockIdx.x], n = r.start[blockIdx.x + 1] - before;
-  const int64_t src0 = range_first(r, blockIdx.x);
-  auto set_offset = [&](int k, uint32_t at) {
-    if (src0 + k > r.num_src) return;
-    if (FORMATS) r.csr_indptr[src0 + k] = at;
-    else r.t_indptr[src0 + k] = at;
-  };
-  if (n == 0) {
-    for (int k = tid; k < keys; k += kRangeSortBlock) set_offset(k, before);
-    return;
-  }
-  const uint64_t* rec = r.rec + before;
-  auto key_of = [&](uint64_t x) { return static_cast<uint32_t>(x >> kRangeEdgeBits) & ((1u << kRangeKeyBits) - 1); };
-  const bool single = n <= kRangeSortChunk;   // block-uniform
-  const int per = (keys + kRangeSortBlock - 1) / kRangeSortBlock;
-  // counts per key in s_start -> the key's first position, and its offset
-  auto starts = [&]() {
-    const int k0 = tid * per, k1 = min(k0 + per, keys);
-    uint32_t mine = 0, all;
-    for (int k = k0; k < k1; ++k) mine += s_start[k];
-    uint32_t run = exclusive(mine, all);
-    for (int k = k0; k < k1; ++k) {
-      const uint32_t c = s_start[k];
-      s_start[k] = run;
-      set_offset(k, before + run);
-      run += c;
+  // Records [first, last) of range b (of which it has n, from position `before` on); part0: the range's first part if
+  // it is long.
+  auto sort = [&](int b, uint32_t before, uint32_t n, uint32_t first, uint32_t last, bool part, uint32_t part0) {
+    const int shift = range_shift(r, b);
+    const int keys = 1 << shift;
+    const int words = keys / 2;
+    uint32_t* s_start = s_range;              // [keys]: next position of a key's first record not yet placed
+    uint32_t* s_cnt2 = s_range + keys;        // [waves][keys / 2], 16-bit counts
+    uint32_t* s_before = s_cnt2;              // [keys], before those: records ahead of `first`
+    const int64_t src0 = range_first(r, b);
+    auto set_offset = [&](int k, uint32_t at) {
+      if (src0 + k > r.num_src) return;
+      if (FORMATS) r.csr_indptr[src0 + k] = at;
+      else r.t_indptr[src0 + k] = at;
+    };
+    if (n == 0) {
+      for (int k = tid; k < keys; k += kRangeSortBlock) set_offset(k, before);
+      return;
     }
-  };
-  if (!single) {
-    for (int k = tid; k < keys; k += kRangeSortBlock) s_start[k] = 0;
-    __syncthreads();
-    for (uint32_t i = tid; i < n; i += kRangeSortBlock) atomicAdd(&s_start[key_of(rec[i])], 1u);
-    __syncthreads();
-    starts();
-  }
-  uint32_t* cnt = s_cnt2 + wave * words;
-  volatile uint16_t* pos = reinterpret_cast<volatile uint16_t*>(cnt);
-  for (uint32_t c0 = 0; c0 < n; c0 += kRangeSortChunk) {
-    const uint32_t left = min(n - c0, static_cast<uint32_t>(kRangeSortChunk));
-    const int rounds = static_cast<int>((left + kRangeSortBlock - 1) / kRangeSortBlock);
-    uint64_t x[kRangeSortRounds];
-#pragma unroll
-    for (int q = 0; q < kRangeSortRounds; ++q) {
-      const uint32_t i = (wave * rounds + q) * kWave + lane;
-      x[q] = q < rounds && i < left ? rec[c0 + i] : ~0ull;
+    const uint64_t* rec = r.rec + before;
+    auto place = [&](int64_t to, uint64_t x) {
+      const uint32_t e = static_cast<uint32_t>(x);
+      if (FORMATS) {
+        r.csr_eids[to] = e;
+        r.csr_indices[to] = static_cast<int64_t>(x >> (kRangeKeyBits + kRangeEdgeBits));
+      } else {
+        r.t_slots[to] = e;
+      }
+    };
+    if (keys == 1) {   // one source: its records are in order already
+      if (first == 0 && tid == 0) set_offset(0, before);
+      for (uint32_t i = first + tid; i < last; i += kRangeSortBlock) place(static_cast<int64_t>(before) + i, rec[i]);
+      return;
     }
-    __syncthreads();
-    for (int i = tid; i < words * kRangeSortWaves; i += kRangeSortBlock) s_cnt2[i] = 0;
-    __syncthreads();
+    auto key_of = [&](uint64_t x) { return static_cast<uint32_t>(x >> kRangeEdgeBits) & ((1u << kRangeKeyBits) - 1); };
+    const bool single = n <= kRangeSortChunk;   // block-uniform
+    const int per = (keys + kRangeSortBlock - 1) / kRangeSortBlock;
+    // counts per key in s_start -> the key's first position, and its offset
+    auto starts = [&]() {
+      const int k0 = tid * per, k1 = min(k0 + per, keys);
+      uint32_t mine = 0, all;
+      for (int k = k0; k < k1; ++k) mine += s_start[k];
+      uint32_t run = exclusive(mine, all);
+      for (int k = k0; k < k1; ++k) {
+        const uint32_t c = s_start[k];
+        s_start[k] = run;
+        if (first == 0) set_offset(k, before + run);
+        run += c;
+      }
+    };
+    if (part) {
+      constexpr int kBatch = 8;
+      const uint32_t parts = part_count(n), mine = first / part_length(n);
+      for (int k = tid; k < keys; k += kRangeSortBlock) {
+        const uint32_t* col = r.part_keys + static_cast<int64_t>(part0) * r.row_words + k;
+        uint32_t total = 0, ahead = 0;
+        for (uint32_t q = 0; q < parts; q += kBatch) {
+          uint32_t c[kBatch];
 #pragma unroll
-    for (int q = 0; q < kRangeSortRounds; ++q)
-      if (x[q] != ~0ull) {
-        const uint32_t k = key_of(x[q]);
-        atomicAdd(&cnt[k >> 1], (k & 1) ? 0x10000u : 1u);
-      }
-    __syncthreads();
-    // counts of a wavefront -> counts of the wavefronts before it (a chunk's 2048 fit 16 bits)
-    for (int i = tid; i < words; i += kRangeSortBlock) {
-      uint32_t sum = 0;
+          for (int u = 0; u < kBatch; ++u) c[u] = col[static_cast<int64_t>(min(q + u, parts - 1)) * r.row_words];
 #pragma unroll
-      for (int w = 0; w < kRangeSortWaves; ++w) {
-        const uint32_t c = s_cnt2[w * words + i];
-        s_cnt2[w * words + i] = sum;
-        sum += c;
+          for (int u = 0; u < kBatch; ++u) {
+            total += q + u < parts ? c[u] : 0u;
+            ahead += q + u < mine ? c[u] : 0u;
+          }
+        }
+        s_start[k] = total;
+        s_before[k] = ahead;
       }
-      if (single) {
-        s_start[2 * i] = sum & 0xffffu;
-        s_start[2 * i + 1] = sum >> 16;
-      }
-    }
-    __syncthreads();
-    if (single) {
+      __syncthreads();
       starts();
       __syncthreads();
+      for (int k = tid; k < keys; k += kRangeSortBlock) s_start[k] += s_before[k];
+    } else if (!single) {
+      for (int k = tid; k < keys; k += kRangeSortBlock) s_start[k] = 0;
+      __syncthreads();
+      for (uint32_t i = tid; i < n; i += kRangeSortBlock) atomicAdd(&s_start[key_of(rec[i])], 1u);
+      __syncthreads();
+      starts();
     }
+    uint32_t* cnt = s_cnt2 + wave * words;
+    volatile uint16_t* pos = reinterpret_cast<volatile uint16_t*>(cnt);
+    for (uint32_t c0 = first; c0 < last; c0 += kRangeSortChunk) {
+      const uint32_t left = min(last - c0, static_cast<uint32_t>(kRangeSortChunk));
+      const int rounds = static_cast<int>((left + kRangeSortBlock - 1) / kRangeSortBlock);
+      uint64_t x[kRangeSortRounds];
 #pragma unroll
-    for (int q = 0; q < kRangeSortRounds; ++q) {
-      if (q >= rounds) break;   // block-uniform
-      const bool valid = x[q] != ~0ull;
-      const uint32_t k = valid ? key_of(x[q]) : 0u;
-      const uint64_t peers = same_value(k, shift, valid);
-      const uint32_t rank = rank_below(peers);
-      uint32_t at = 0;
-      if (valid) at = pos[k] + rank;
-      __builtin_amdgcn_wave_barrier();
-      if (valid && rank + 1 == static_cast<uint32_t>(__popcll(peers))) pos[k] = static_cast<uint16_t>(at + 1);
-      __builtin_amdgcn_wave_barrier();
-      if (valid) {
-        const int64_t to = static_cast<int64_t>(before) + s_start[k] + at;
-        const uint32_t e = static_cast<uint32_t>(x[q]) & ((1u << kRangeEdgeBits) - 1);
-        if (FORMATS) {
-          r.csr_eids[to] = e;
-          r.csr_indices[to] = static_cast<int64_t>(x[q] >> (kRangeKeyBits + kRangeEdgeBits));
-        } else {
-          r.t_slots[to] = e;
+      for (int q = 0; q < kRangeSortRounds; ++q) {
+        const uint32_t i = (wave * rounds + q) * kWave + lane;
+        x[q] = q < rounds && i < left ? rec[c0 + i] : ~0ull;
+      }
+      __syncthreads();
+      for (int i = tid; i < words * kRangeSortWaves; i += kRangeSortBlock) s_cnt2[i] = 0;
+      __syncthreads();
+#pragma unroll
+      for (int q = 0; q < kRangeSortRounds; ++q)
+        if (x[q] != ~0ull) {
+          const uint32_t k = key_of(x[q]);
+          atomicAdd(&cnt[k >> 1], (k & 1) ? 0x10000u : 1u);
+        }
+      __syncthreads();
+      // counts of a wavefront -> counts of the wavefronts before it (a chunk's 2048 fit 16 bits)
+      for (int i = tid; i < words; i += kRangeSortBlock) {
+        uint32_t sum = 0;
+#pragma unroll
+        for (int w = 0; w < kRangeSortWaves; ++w) {
+          const uint32_t c = s_cnt2[w * words + i];
+          s_cnt2[w * words + i] = sum;
+          sum += c;
+        }
+        if (single) {
+          s_start[2 * i] = sum & 0xffffu;
+          s_start[2 * i + 1] = sum >> 16;
         }
       }
+      __syncthreads();
+      if (single) {
+        starts();
+        __syncthreads();
+      }
+#pragma unroll
+      for (int q = 0; q < kRangeSortRounds; ++q) {
+        if (q >= rounds) break;   // block-uniform
+        const bool valid = x[q] != ~0ull;
+        const uint32_t k = valid ? key_of(x[q]) : 0u;
+        const uint64_t peers = same_value(k, shift, valid);
+        const uint32_t rank = rank_below(peers);
+        uint32_t at = 0;
+        if (valid) at = pos[k] + rank;
+        __builtin_amdgcn_wave_barrier();
+        if (valid && rank + 1 == static_cast<uint32_t>(__popcll(peers))) pos[k] = static_cast<uint16_t>(at + 1);
+        __builtin_amdgcn_wave_barrier();
+        if (valid) place(static_cast<int64_t>(before) + s_start[k] + at, x[q]);
+      }
+      if (c0 + kRangeSortChunk >= last) break;
+      __syncthreads();
+      // every wavefront has moved its counters past its records: the last one's stand at the chunk's totals
+      const uint16_t* moved = reinterpret_cast<const uint16_t*>(s_cnt2 + (kRangeSortWaves - 1) * words);
+      for (int k = tid; k < keys; k += kRangeSortBlock) s_start[k] += moved[k];
     }
-    if (c0 + kRangeSortChunk >= n) break;
-    __syncthreads();
-    // every wavefront has moved its counters past its records: the last one's stand at the chunk's totals
-    const uint16_t* last = reinterpret_cast<const uint16_t*>(s_cnt2 + (kRangeSortWaves - 1) * words);
-    for (int k = tid; k < keys; k += kRangeSortBlock) s_start[k] += last[k];
+  };
+  const bool whole = static_cast<int>(blockIdx.x) >= r.part_groups;   // a range of its own
+  const uint32_t parts = whole ? 0u : *r.parts;
+  for (uint32_t p = blockIdx.x;; p += r.part_groups) {   // block-uniform
+    if (!whole && p >= parts) return;
+    const int b = whole ? static_cast<int>(blockIdx.x) - r.part_groups : static_cast<int>(r.part_range[p]);
+    const uint32_t before = r.start[b], n = r.start[b + 1] - before;
+    const bool part = n > r.long_from;
+    if (whole && part) return;
+    const uint32_t part0 = whole ? 0u : r.part0[b], first = whole ? 0u : (p - part0) * part_length(n);
+    sort(b, before, n, first, whole ? n : min(first + part_length(n), n), part, part0);
+    if (whole) return;
+    __syncthreads();   // (the counters)
   }
 }
 
@@ -960,16 +1072,30 @@ struct FmtLayout {
   int64_t slots, ctiles, stiles, rtiles;
   size_t tile_cnt_off, sums_off, hist_off, bin_total_off, key_off[2], pay_off[2], total;
   int range_shift2, ranges;   // CSR by source ranges; ranges == 0: by radix passes
-  size_t start_off, rec_off;
+  size_t start_off, rec_off, part0_off, part_range_off, part_keys_off;
 };
 
+// Keys of the widest of so many ranges.
+static int range_keys(int64_t ranges, int shift2) {
+  return 1 << (ranges > kRangeCount0 + kRangeCount1 ? shift2 : ranges > kRangeCount0 ? kRangeShift1 : kRangeShift0);
+}
+// Long ranges have more than kRangeLong = 2 kRangePart records each: at most 3 parts to 2 kRangePart records.
+static int64_t most_parts(int64_t slots) { return 3 * slots / (2 * kRangePart) + 1; }
+static_assert(kRangeLong >= 2 * kRangePart && kRangePart % kRangeSortChunk == 0);
+
 // The last piece's ranges are as narrow as their number allows.  num_src itself has a range: the last offset.
+// A block of so few sources that every range is long is better off with the radix passes, of which it needs one or two:
+// 1 M edges of 31 / 1000 / 2000 / 4000 sources, radix 42 / 70 / 69 / 69, ranges 40 / 95 / 106 / 61 us.  (The transpose has no
+// radix passes.)
+constexpr int64_t kRangeMostMean = 3000;
 static void choose_ranges(int64_t num_dst, int64_t num_src, bool records_hold_dst, FmtLayout& L) {
   L.range_shift2 = kRangeShift2;
   while (L.range_shift2 < kRangeMaxShift && range_index(num_src, L.range_shift2) >= kRangeMaxCount) ++L.range_shift2;
   const int64_t ranges = range_index(num_src, L.range_shift2) + 1;
   const bool fits = ranges <= kRangeMaxCount && L.ctiles <= kRangeMaxTiles &&
-                    (!records_hold_dst || num_dst <= kRangeMaxDst) && tuning_block_fused_scan();
+                    (!records_hold_dst || (num_dst <= kRangeMaxDst &&
+                                           (num_src >= kRangeFrom1 || L.slots <= kRangeMostMean * ranges))) &&
+                    tuning_block_fused_scan();
   L.ranges = fits ? static_cast<int>(ranges) : 0;
 }
 
@@ -979,6 +1105,9 @@ static void lay_out_ranges(size_t off, int64_t tiles, int64_t ranges, int64_t sl
   L.hist_off = off;      off = fmt_align(off + sizeof(uint32_t) * static_cast<size_t>(tiles) * ranges);
   L.bin_total_off = off; off = fmt_align(off + sizeof(uint32_t) * ranges);
   L.start_off = off;     off = fmt_align(off + sizeof(uint32_t) * (ranges + 1));
+  L.part0_off = off;     off = fmt_align(off + sizeof(uint32_t) * (ranges + 1));   // (and the number of parts)
+  L.part_range_off = off; off = fmt_align(off + sizeof(uint32_t) * static_cast<size_t>(most_parts(slots)));
+  L.part_keys_off = off; off = fmt_align(off + sizeof(uint32_t) * static_cast<size_t>(most_parts(slots)) * range_keys(ranges, L.range_shift2));
   L.rec_off = off;       L.total = fmt_align(off + sizeof(uint64_t) * static_cast<size_t>(slots));
 }
 
@@ -1047,8 +1176,15 @@ static int launch_ranges(const CompactParams& c, RangeParams& r, const FmtLayout
   r.hist = reinterpret_cast<uint32_t*>(ws + L.hist_off);
   r.total = reinterpret_cast<uint32_t*>(ws + L.bin_total_off);
   r.start = reinterpret_cast<uint32_t*>(ws + L.start_off);
+  r.part0 = reinterpret_cast<uint32_t*>(ws + L.part0_off);
+  r.parts = r.part0 + L.ranges;
+  r.part_range = reinterpret_cast<uint32_t*>(ws + L.part_range_off);
+  r.part_keys = reinterpret_cast<uint32_t*>(ws + L.part_keys_off);
   r.rec = reinterpret_cast<uint64_t*>(ws + L.rec_off);
   r.num_src = num_src;
+  const int keys = r.row_words = range_keys(L.ranges, L.range_shift2);
+  r.long_from = static_cast<uint32_t>(std::min<int64_t>(std::max<int64_t>(kRangeLong, 4 * L.slots / L.ranges), kRangeLongest));
+  r.part_groups = L.slots > r.long_from ? static_cast<int>(std::min<int64_t>(ceil_div(L.slots, kRangePart), kRangePartGroups)) : 0;
   const bool small = L.slots <= (c.num_dst_dev != nullptr ? kRangeSmallBound : kRangeSmallSlots);
   r.tile = small ? kFmtBlock * kRangeSmallIters : kCompactTile;
   const dim3 tiles(static_cast<unsigned>(ceil_div(std::max<int64_t>(L.slots, 1), r.tile)));
@@ -1067,10 +1203,7 @@ static int launch_ranges(const CompactParams& c, RangeParams& r, const FmtLayout
   else
     hipLaunchKernelGGL((range_place_kernel<FORMATS, kCompactIters>), tiles, dim3(kFmtBlock), place_lds, st, c, r);
   APT_LAUNCH_CHECK("range_place_kernel");
-  const int keys = 1 << (L.ranges > kRangeCount0 + kRangeCount1 ? L.range_shift2
-                         : L.ranges > kRangeCount0              ? kRangeShift1
-                                                                : kRangeShift0);
-  hipLaunchKernelGGL(range_sort_kernel<FORMATS>, dim3(static_cast<unsigned>(L.ranges)), dim3(kRangeSortBlock),
+  hipLaunchKernelGGL(range_sort_kernel<FORMATS>, dim3(static_cast<unsigned>(r.part_groups + L.ranges)), dim3(kRangeSortBlock),
                      sizeof(uint32_t) * (keys + kRangeSortWaves * (keys / 2)), st, r);
   APT_LAUNCH_CHECK("range_sort_kernel");
   return APT_OK;
