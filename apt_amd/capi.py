@@ -126,17 +126,20 @@ SYMBOLS = {
     "apt_gat_block_backward": (_I, [_P, _I64, _I, _P, _I64, _I, _I64, _I, _P, _P, C.c_float, _P, _P, _P, _P, _P, _P, _P]),
     "apt_spmm_heads": (_I, [_P, _P, _I64, _P, _I64, _P, _P, _I, _I64, _I, _I, _P, _I64, _P, _P, _P, _P]),
     "apt_block_transpose_workspace_bytes": (_SZ, [_I64, _I, _I64]),
-    "apt_block_transpose": (_I, [_P, _I64, _I, _I64, _P, _P, _P, _SZ, _P]),
+    "apt_block_transpose": (_I, [_P, _I64, _I, _I64, _P, _P, _P, _P, _SZ, _P]),
+    "apt_long_rows_bytes": (_SZ, [_I64]),
+    "apt_find_long_rows": (_I, [_P, _I, _I64, _I64, _P, _P]),
     "apt_block_aggregate": (_I, [_P, _I64, _I, _P, _I64, _I64, _I, _I, C.c_float, _P, _P, _I, _P, _P, _P]),
-    "apt_block_aggregate_backward": (_I, [_P, _P, _I, _I, _I64, _P, C.c_float, _P, _I64, _I64, _I, _P, _P]),
+    "apt_block_aggregate_backward_workspace_bytes": (_SZ, [_I64, _I64]),
+    "apt_block_aggregate_backward": (_I, [_P, _P, _I, _I, _I64, _I64, _P, _P, C.c_float, _P, _I64, _I64, _I, _P, _P, _SZ, _P]),
     "apt_coo_prepare": (_I, [_P, _P, _I64, _P, _P, _P, _I, _P, _P, _P, _P, _P]),
-    "apt_coo_sum_workspace_bytes": (_SZ, [_I64, _I64, _I]),
-    "apt_coo_sum": (_I, [_I, _P, _P, _I64, _I, _P, _I64, _P, _I64, _I, _P, _I64, _P, _SZ, _P]),
+    "apt_coo_sum_workspace_bytes": (_SZ, [_I64, _I64, _I, _I, _I64]),
+    "apt_coo_sum": (_I, [_I, _P, _P, _I64, _I, _I, _P, _I64, _P, _I64, _I, _P, _I64, _P, _SZ, _P]),
     "apt_coo_combine": (_I, [_I, _P, _P, _I64, _P, _I64, _P, _I64, _I64, _I, _P, _P, _P, _I, _P, _P]),
     "apt_gat_layer": (_I, [_P, _I64, _I, _P, _I64, _I, _I64, _I, _P, _P, _I, _P, _I, C.c_float, _I, _P, _P, _P, _P, _P]),
     "apt_gat_layer_backward_workspace_bytes": (_SZ, [_I64, _I, _I64, _I, _I64, _I64]),
     "apt_gat_layer_backward": (_I, [_P, _I64, _I, _P, _I64, _I, _I64, _I, _P, _P, _I, C.c_float, _P, _P, _P, _P, _P, _P, _I, _P,
-                                    _P, _I64, _P, _P, _P, _P, _P, _SZ, _P]),
+                                    _P, _I64, _P, _P, _P, _P, _P, _P, _SZ, _P]),
     "apt_add_rows": (_I, [_P, _P, _I64, _I, _I, _P]),
     "apt_rows_gemm_workspace_bytes": (_SZ, [_I64, _I64, _I64]),
     "apt_rows_gemm": (_I, [_P, _I64, _P, _I64, _I64, _P, _I64, _P, _I64, _I64, _I64, _I64, _I64, _P, _I, _I, _P, _P, _SZ, _P]),

@@ -25,6 +25,7 @@
 #include <algorithm>
 
 #include "common.hpp"
+#include "long_rows.hpp"
 
 namespace apt {
 
@@ -518,6 +519,7 @@ struct RangeParams {
   int64_t* csr_eids;
   uint32_t* t_indptr;         // transpose only (apt_block_transpose)
   uint32_t* t_slots;
+  LongRows lng;               // sources with very many edges: the table that the sums over them read
 };
 
 constexpr int kRangeSingles = static_cast<int>(kRangeFrom0);
@@ -575,6 +577,10 @@ __global__ __launch_bounds__(kFmtBlock) void range_count_kernel(CompactParams p,
   const int64_t base = static_cast<int64_t>(blockIdx.x) * (kFmtBlock * ITERS);
   if (base >= slots && blockIdx.x != 0) return;   // block-uniform: nobody reads an inactive tile's counts
   if (blockIdx.x == 0 && threadIdx.x == 0) *r.parts = 0;
+  if (!FORMATS)
+    for (int64_t i = static_cast<int64_t>(blockIdx.x) * kFmtBlock + threadIdx.x; i < r.lng.slots;
+         i += static_cast<int64_t>(gridDim.x) * kFmtBlock)
+      r.lng.row[i] = r.lng.arrived[i] = 0;
   int64_t v[ITERS];
 #pragma unroll
   for (int it = 0; it < ITERS; ++it) {
@@ -868,13 +874,18 @@ __global__ __launch_bounds__(kRangeSortBlock) void range_sort_kernel(RangeParams
     uint32_t* s_cnt2 = s_range + keys;        // [waves][keys / 2], 16-bit counts
     uint32_t* s_before = s_cnt2;              // [keys], before those: records ahead of `first`
     const int64_t src0 = range_first(r, b);
-    auto set_offset = [&](int k, uint32_t at) {
+    auto set_offset = [&](int k, uint32_t at, uint32_t count) {
       if (src0 + k > r.num_src) return;
-      if (FORMATS) r.csr_indptr[src0 + k] = at;
-      else r.t_indptr[src0 + k] = at;
+      if (FORMATS) {
+        r.csr_indptr[src0 + k] = at;
+      } else {
+        r.t_indptr[src0 + k] = at;
+        if (r.lng.slots > 0 && count > r.lng.longer && src0 + k < r.num_src)
+          r.lng.row[at / r.lng.longer] = static_cast<uint32_t>(src0 + k) + 1;
+      }
     };
     if (n == 0) {
-      for (int k = tid; k < keys; k += kRangeSortBlock) set_offset(k, before);
+      for (int k = tid; k < keys; k += kRangeSortBlock) set_offset(k, before, 0);
       return;
     }
     const uint64_t* rec = r.rec + before;
@@ -888,7 +899,7 @@ __global__ __launch_bounds__(kRangeSortBlock) void range_sort_kernel(RangeParams
       }
     };
     if (keys == 1) {   // one source: its records are in order already
-      if (first == 0 && tid == 0) set_offset(0, before);
+      if (first == 0 && tid == 0) set_offset(0, before, n);
       for (uint32_t i = first + tid; i < last; i += kRangeSortBlock) place(static_cast<int64_t>(before) + i, rec[i]);
       return;
     }
@@ -904,7 +915,7 @@ __global__ __launch_bounds__(kRangeSortBlock) void range_sort_kernel(RangeParams
       for (int k = k0; k < k1; ++k) {
         const uint32_t c = s_start[k];
         s_start[k] = run;
-        if (first == 0) set_offset(k, before + run);
+        if (first == 0) set_offset(k, before + run, c);
         run += c;
       }
     };
@@ -1218,8 +1229,8 @@ extern "C" size_t apt_block_transpose_workspace_bytes(int64_t num_dst, int fanou
 }
 
 extern "C" int apt_block_transpose(const int64_t* relabeled, int64_t num_dst, int fanout, int64_t num_src,
-                                   uint32_t* indptr, uint32_t* slots, void* workspace, size_t workspace_bytes,
-                                   void* stream) {
+                                   uint32_t* indptr, uint32_t* slots, void* long_table, void* workspace,
+                                   size_t workspace_bytes, void* stream) {
   using namespace apt;
   APT_REQUIRE(fmt_sizes_ok(num_dst, fanout, num_src), APT_ELIMIT,
               "apt_block_transpose: sizes out of range (num_dst %lld, fanout %d, num_src %lld)",
@@ -1239,6 +1250,7 @@ extern "C" int apt_block_transpose(const int64_t* relabeled, int64_t num_dst, in
   RangeParams r{};
   r.t_indptr = indptr;
   r.t_slots = slots;
+  r.lng = long_rows(long_table, L.slots, nullptr);
   return launch_ranges<false>(c, r, L, static_cast<char*>(workspace), num_src, static_cast<hipStream_t>(stream));
 }
 

@@ -7,16 +7,19 @@
 // two rows per group are in flight.  The few hubs (hundreds of edges) would each occupy one group for the length of
 // the launch: rows longer than kHubEdges are put aside and added up by all groups of the workgroup afterwards.  Hubs
 // have neighbouring ids (the relabel numbers nodes by first occurrence), so a workgroup's rows are taken a grid apart.
+// Rows that are too long for one workgroup as well are cut into chunks (long_rows.hpp).
 #include <algorithm>
 
 #include "common.hpp"
 #include "feature_rows.hpp"
+#include "long_rows.hpp"
 
 namespace apt {
 
 constexpr int kHubEdges = 16;
 constexpr int kHubList = 1024;             // rows of a workgroup at the most, so its list of hubs never overflows
 constexpr int kSourceBlocks = 2048;
+constexpr int kLongBlocks = 512;           // (without a long row the launch takes 3 us)
 
 struct SourceSumParams {
   const void* indptr;      // offsets of the sources in `index`
@@ -31,24 +34,34 @@ struct SourceSumParams {
   int64_t dim;
   int64_t num_src;
   void* dx;                // [num_src, dim]
+  LongRows lng;
 };
 
 // I: int64_t = a block's CSR (offsets, destinations), uint32_t = apt_block_transpose (offsets, slots).
-template <typename T, int VEC, int LPR, typename I, bool EDATA>
+// LONG: the long rows alone, a launch after the one that takes all others (in one kernel with them, the compiler makes the
+// loop over the rows 18 % slower: 282 us instead of 239 for 500 k rows of 256 fp32).
+template <typename T, int VEC, int LPR, typename I, bool EDATA, bool LONG>
 __global__ __launch_bounds__(kAggBlock) void source_sum_kernel(SourceSumParams p) {
   constexpr int kGroups = kAggBlock / LPR;
   constexpr int kRows = 2;
   constexpr int kUnroll = 4;
-  __shared__ int s_hub[kHubList];
+  __shared__ int s_hub[LONG ? 1 : kHubList];
   __shared__ int s_hubs;
   __shared__ float s_sum[kGroups][LPR * VEC];
+  __shared__ uint32_t s_wave[kAggWaves], s_where[2];   // LONG
   const int grp = threadIdx.x / LPR, l = threadIdx.x % LPR;
   const I* indptr = static_cast<const I*>(p.indptr);
   const I* index = static_cast<const I*>(p.index);
   const T* dz = static_cast<const T*>(p.dz);
   T* dx = static_cast<T*>(p.dx);
-  if (threadIdx.x == 0) s_hubs = 0;
-  __syncthreads();
+  LongChunks<kAggBlock, I> chunks(p.lng, indptr);
+  if constexpr (LONG) {
+    chunks.number(s_wave);
+    if (blockIdx.x >= chunks.all) return;
+  } else {
+    if (threadIdx.x == 0) s_hubs = 0;
+    __syncthreads();
+  }
   struct Edge {      // lane j of a group: edge j of the row
     int64_t dst;     // -1: none
     uint32_t slot;   // EDATA only
@@ -100,6 +113,61 @@ __global__ __launch_bounds__(kAggBlock) void source_sum_kernel(SourceSumParams p
         for (int k = 0; k < VEC; ++k) acc[k] += w[u] * v[u][k];
     }
   };
+  // acc += the edges [lo, hi), every kGroups-th by this group
+  auto add_span = [&](int64_t lo, int64_t hi, int64_t c, bool live, float (&acc)[VEC]) {
+    for (int64_t e = lo + grp; e < hi; e += kAggBlock) {
+      const int64_t at = e + static_cast<int64_t>(l) * kGroups;
+      add_edges(edge(at, at < hi), static_cast<int>(min((hi - e + kGroups - 1) / kGroups, static_cast<int64_t>(LPR))), c, live, acc);
+    }
+  };
+  // The groups' sums together, in order, for the first group.
+  auto over_groups = [&](float (&acc)[VEC]) {
+#pragma unroll
+    for (int k = 0; k < VEC; ++k) s_sum[grp][l * VEC + k] = acc[k];
+    __syncthreads();
+    if (grp == 0) {
+#pragma unroll
+      for (int k = 0; k < VEC; ++k) {
+        float sum = 0.f;
+#pragma unroll 1
+        for (int g = 0; g < kGroups; ++g) sum += s_sum[g][l * VEC + k];
+        acc[k] = sum;
+      }
+    }
+    __syncthreads();
+  };
+  if constexpr (LONG) {
+    for (uint32_t q = blockIdx.x; q < chunks.all; q += gridDim.x) {   // block-uniform
+      const auto chunk = chunks.find(q, s_where);
+      const float* part = p.lng.part + static_cast<int64_t>(q - chunk.index) * p.dim;   // of the row's chunks
+      bool whole = false;
+      for (;;) {   // the chunk's edges; then, for the workgroup that completes the row, its chunks' sums
+        for (int64_t c0 = 0; c0 < p.dim; c0 += LPR * VEC) {
+          const int64_t c = c0 + static_cast<int64_t>(l) * VEC;
+          const bool live = c < p.dim;
+          float acc[VEC];
+#pragma unroll
+          for (int k = 0; k < VEC; ++k) acc[k] = 0.f;
+          if (!whole) add_span(chunk.from, chunk.to, c, live, acc);
+          for (uint32_t g = grp; whole && g < chunk.count && live; g += kGroups)
+#pragma unroll
+            for (int k = 0; k < VEC; ++k) acc[k] += part[static_cast<int64_t>(g) * p.dim + c + k];
+          over_groups(acc);
+          if (grp == 0 && live && !whole) {
+#pragma unroll
+            for (int k = 0; k < VEC; ++k) p.lng.part[static_cast<int64_t>(q) * p.dim + c + k] = acc[k];
+          } else if (grp == 0 && live) {
+#pragma unroll
+            for (int k = 0; k < VEC; ++k) acc[k] *= p.scale;
+            store_vec<T, VEC>(dx, chunk.row * p.dim + c, acc);
+          }
+        }
+        if (whole || !chunks.last_of_row(chunk, s_where)) break;
+        whole = true;
+      }
+    }
+    return;
+  }
   const int64_t row_groups = static_cast<int64_t>(gridDim.x) * kGroups;
   for (int64_t r0 = static_cast<int64_t>(grp) * gridDim.x + blockIdx.x; r0 < p.num_src; r0 += kRows * row_groups) {
     int64_t lo[kRows];
@@ -139,7 +207,8 @@ __global__ __launch_bounds__(kAggBlock) void source_sum_kernel(SourceSumParams p
     }
 #pragma unroll
     for (int q = 0; q < kRows; ++q)
-      if (n[q] > kHubEdges && l == 0) s_hub[atomicAdd(&s_hubs, 1)] = static_cast<int>(r0 + q * row_groups);
+      if (n[q] > kHubEdges && l == 0 && (p.lng.slots == 0 || n[q] <= static_cast<int>(p.lng.longer)))
+        s_hub[atomicAdd(&s_hubs, 1)] = static_cast<int>(r0 + q * row_groups);
   }
   __syncthreads();
   const int hubs = s_hubs;
@@ -152,39 +221,35 @@ __global__ __launch_bounds__(kAggBlock) void source_sum_kernel(SourceSumParams p
       float acc[VEC];
 #pragma unroll
       for (int k = 0; k < VEC; ++k) acc[k] = 0.f;
-      for (int64_t e = lo + grp; e < hi; e += kAggBlock) {   // every kGroups-th edge, so that all groups have some
-        const int64_t at = e + static_cast<int64_t>(l) * kGroups;
-        add_edges(edge(at, at < hi), static_cast<int>(min((hi - e + kGroups - 1) / kGroups, static_cast<int64_t>(LPR))), c, live,
-                  acc);
-      }
-#pragma unroll
-      for (int k = 0; k < VEC; ++k) s_sum[grp][l * VEC + k] = acc[k];
-      __syncthreads();
+      add_span(lo, hi, c, live, acc);   // (all groups have some of the edges)
+      over_groups(acc);
       if (grp == 0 && live) {
 #pragma unroll
-        for (int k = 0; k < VEC; ++k) {
-          float sum = 0.f;
-#pragma unroll 1
-          for (int g = 0; g < kGroups; ++g) sum += s_sum[g][l * VEC + k];
-          acc[k] = sum * p.scale;
-        }
+        for (int k = 0; k < VEC; ++k) acc[k] *= p.scale;
         store_vec<T, VEC>(dx, r * p.dim + c, acc);
       }
-      __syncthreads();
     }
   }
 }
 
+// A workgroup for two rows per lane group, or, where rows have many edges, for sixteen edges per lane group (1 M edges of
+// 16 fp32 into 4096 rows: 481 us with the 64 workgroups of the rows alone).
 template <typename T, int VEC, typename I, bool EDATA>
-static void launch_source_sum(const SourceSumParams& p, hipStream_t st) {
+static void launch_source_sum(const SourceSumParams& p, int64_t num_edges, hipStream_t st) {
   const int64_t per_row = ceil_div(p.dim, VEC);
 #define APT_SOURCE_SUM(LPR)                                                                                        \
   do {                                                                                                            \
     constexpr int64_t groups = kAggBlock / LPR;                                                                    \
     const int64_t blocks = std::max(ceil_div(p.num_src, kHubList),                                                \
-                                    std::min<int64_t>(ceil_div(p.num_src, groups * 2), kSourceBlocks));           \
-    hipLaunchKernelGGL((source_sum_kernel<T, VEC, LPR, I, EDATA>), dim3(static_cast<unsigned>(blocks)), dim3(kAggBlock), 0, \
-                       st, p);                                                                                    \
+                                    std::min<int64_t>(std::max(ceil_div(p.num_src, groups * 2),                   \
+                                                               std::min(p.num_src, num_edges / (groups * kHubEdges))), \
+                                                      kSourceBlocks));                                            \
+    hipLaunchKernelGGL((source_sum_kernel<T, VEC, LPR, I, EDATA, false>), dim3(static_cast<unsigned>(blocks)),    \
+                       dim3(kAggBlock), 0, st, p);                                                                \
+    if (p.lng.slots > 0)                                                                                          \
+      hipLaunchKernelGGL((source_sum_kernel<T, VEC, LPR, I, EDATA, true>),                                        \
+                         dim3(static_cast<unsigned>(std::min<int64_t>(long_chunks(num_edges), kLongBlocks))),     \
+                         dim3(kAggBlock), 0, st, p);                                                              \
   } while (0)
   if (per_row <= 8) APT_SOURCE_SUM(8);
   else if (per_row <= 16) APT_SOURCE_SUM(16);
@@ -194,19 +259,49 @@ static void launch_source_sum(const SourceSumParams& p, hipStream_t st) {
 }
 
 template <typename I, bool EDATA>
-static int source_sum(const SourceSumParams& p, int elem_size, hipStream_t st) {
+static int source_sum(const SourceSumParams& p, int64_t num_edges, int elem_size, hipStream_t st) {
   const bool aligned = ((reinterpret_cast<uintptr_t>(p.dz) | reinterpret_cast<uintptr_t>(p.dx) |
                          reinterpret_cast<uintptr_t>(p.edata)) & 15) == 0;
   if (elem_size == 4) {
-    if (aligned && p.dim % 4 == 0) launch_source_sum<float, 4, I, EDATA>(p, st);
-    else launch_source_sum<float, 1, I, EDATA>(p, st);
+    if (aligned && p.dim % 4 == 0) launch_source_sum<float, 4, I, EDATA>(p, num_edges, st);
+    else launch_source_sum<float, 1, I, EDATA>(p, num_edges, st);
   } else {
-    if (aligned && p.dim % 8 == 0) launch_source_sum<uint16_t, 8, I, EDATA>(p, st);
-    else if (aligned && p.dim % 4 == 0) launch_source_sum<uint16_t, 4, I, EDATA>(p, st);
-    else launch_source_sum<uint16_t, 1, I, EDATA>(p, st);
+    if (aligned && p.dim % 8 == 0) launch_source_sum<uint16_t, 8, I, EDATA>(p, num_edges, st);
+    else if (aligned && p.dim % 4 == 0) launch_source_sum<uint16_t, 4, I, EDATA>(p, num_edges, st);
+    else launch_source_sum<uint16_t, 1, I, EDATA>(p, num_edges, st);
   }
   APT_LAUNCH_CHECK("source_sum_kernel");
   return APT_OK;
+}
+
+// ------------------------------------------------------------------ long rows of given offsets
+// A wavefront per slot of the table: the last row that begins in the slot's edges is the only one that can be
+// long (a long row reaches beyond them).  Offsets are searched 64 at a time.
+template <typename I>
+__global__ __launch_bounds__(kAggBlock) void find_long_rows_kernel(const I* __restrict__ indptr, int64_t num_rows, LongRows l) {
+  const int lane = threadIdx.x % kWave;
+  const int64_t slot = static_cast<int64_t>(blockIdx.x) * kAggWaves + threadIdx.x / kWave;
+  if (slot >= l.slots) return;   // wave-uniform
+  const int64_t from = slot * l.longer, to = from + l.longer;
+  int64_t lo = 0, len = num_rows;   // rows that begin before `to`: lo + some of the next len
+  while (len > 0) {
+    const int64_t step = (len + kWave - 1) / kWave;
+    const int64_t at = lo + lane * step + step - 1;   // the last row of the lane's stretch
+    const uint64_t below = ballot(at < lo + len && static_cast<int64_t>(indptr[min(at, num_rows - 1)]) < to);
+    const int64_t whole = __popcll(below);            // (offsets do not decrease: the lanes below are the first ones)
+    const int64_t end = lo + len;
+    lo += whole * step;
+    len = min(step - 1, end - lo);
+  }
+  uint32_t found = 0;
+  if (lo > 0) {
+    const int64_t first = static_cast<int64_t>(indptr[lo - 1]), last = static_cast<int64_t>(indptr[lo]);
+    if (first >= from && last - first > l.longer) found = static_cast<uint32_t>(lo);   // row lo - 1, plus one
+  }
+  if (lane == 0) {
+    l.row[slot] = found;
+    l.arrived[slot] = 0;
+  }
 }
 
 // ------------------------------------------------------------------ sums over a COO
@@ -222,13 +317,15 @@ struct CooParams {
   int num_seg;
   int64_t* keys;
   int64_t* sources;
-  int64_t* grouped;         // 1 on entry
+  int64_t* grouped;         // [0]: 1 on entry; [2]: 0 on entry, 1 if grouped keys may have a long row
+  int64_t half;             // half of the edges that make a row long
 };
 constexpr int kCooSegments = APT_MAX_BUCKETS + 1;
 
 __global__ void coo_grouped_init_kernel(int64_t* grouped, const int64_t* last_offset, int64_t* num_out) {
-  *grouped = 1;
-  if (num_out != nullptr) *num_out = last_offset != nullptr ? *last_offset : 0;
+  grouped[0] = 1;
+  grouped[2] = 0;
+  *num_out = last_offset != nullptr ? *last_offset : 0;
 }
 
 __global__ __launch_bounds__(kAggBlock) void coo_prepare_kernel(CooParams p) {
@@ -244,7 +341,7 @@ __global__ __launch_bounds__(kAggBlock) void coo_prepare_kernel(CooParams p) {
     while (k + 1 < p.num_seg && s_off[k + 1] <= e) ++k;
     return k;
   };
-  bool bad = false;
+  bool bad = false, lengthy = false;
   for (int64_t e = static_cast<int64_t>(blockIdx.x) * kAggBlock + threadIdx.x; e < p.num_edges;
        e += static_cast<int64_t>(gridDim.x) * kAggBlock) {
     const int k = segment(e);
@@ -255,8 +352,11 @@ __global__ __launch_bounds__(kAggBlock) void coo_prepare_kernel(CooParams p) {
       const int q = segment(e + 1);
       bad |= key > s_out[q] + p.col[e + 1];
     }
+    // a long row of equal keys: a multiple of half its length at least, and the key half that further on, are both in it
+    if (e % p.half == 0 && e + p.half < p.num_edges) lengthy |= key == s_out[segment(e + p.half)] + p.col[e + p.half];
   }
-  if (bad) *p.grouped = 0;
+  if (bad) p.grouped[0] = 0;
+  if (lengthy) p.grouped[2] = 1;
 }
 
 // Offsets of the rows in non-decreasing keys: position e, where the key before it is kp and its own k, is the offset
@@ -308,23 +408,57 @@ extern "C" int apt_coo_prepare(const int64_t* coo_row, const int64_t* coo_col, i
   hipLaunchKernelGGL(coo_grouped_init_kernel, dim3(1), dim3(1), 0, st, result, last_offset, result + 1);
   APT_LAUNCH_CHECK("coo_grouped_init_kernel");
   if (num_edges == 0) return APT_OK;
-  const CooParams p{coo_row, coo_col, num_edges, coo_offset, input_offset, output_offset, num_segments, keys, sources, result};
+  const CooParams p{coo_row, coo_col, num_edges, coo_offset, input_offset, output_offset, num_segments, keys, sources, result,
+                    long_from(num_edges) / 2};
   hipLaunchKernelGGL(coo_prepare_kernel, dim3(static_cast<unsigned>(std::min<int64_t>(ceil_div(num_edges, kAggBlock), 4096))),
                      dim3(kAggBlock), 0, st, p);
   APT_LAUNCH_CHECK("coo_prepare_kernel");
   return APT_OK;
 }
 
-extern "C" size_t apt_coo_sum_workspace_bytes(int64_t num_edges, int64_t num_out_rows, int grouped) {
+namespace apt {
+// A sum's scratch: the table of its long rows, if it makes one itself, and their chunks' sums.
+static size_t long_table_bytes(int64_t num_edges) { return coo_align(sizeof(uint32_t) * 2 * long_slots(num_edges)); }
+static size_t long_part_bytes(int64_t num_edges, int64_t width) { return coo_align(sizeof(float) * long_chunks(num_edges) * width); }
+
+template <typename I>
+static int find_long_rows(const void* indptr, int64_t num_rows, const LongRows& l, hipStream_t st) {
+  if (l.slots == 0) return APT_OK;
+  hipLaunchKernelGGL(find_long_rows_kernel<I>, dim3(static_cast<unsigned>(ceil_div(l.slots, kAggWaves))), dim3(kAggBlock), 0, st,
+                     static_cast<const I*>(indptr), num_rows, l);
+  APT_LAUNCH_CHECK("find_long_rows_kernel");
+  return APT_OK;
+}
+}  // namespace apt
+
+extern "C" size_t apt_long_rows_bytes(int64_t num_edges) {
+  return num_edges < 0 || num_edges > 0x7fffffffLL ? 0 : apt::long_table_bytes(num_edges);
+}
+
+extern "C" int apt_find_long_rows(const void* indptr, int index_bytes, int64_t num_src, int64_t num_edges, void* long_table,
+                                  void* stream) {
   using namespace apt;
-  if (num_edges < 0 || num_edges > 0x7fffffffLL || num_out_rows < 0 || num_out_rows > 0x7fffffffLL) return 0;
-  const size_t offsets = coo_align(sizeof(uint32_t) * (num_out_rows + 1));
+  APT_REQUIRE(num_src >= 0 && num_src <= 0x7fffffffLL && num_edges >= 0 && num_edges <= 0x7fffffffLL, APT_ELIMIT,
+              "apt_find_long_rows: sizes out of range (num_src %lld, edges %lld)", (long long)num_src, (long long)num_edges);
+  APT_REQUIRE(index_bytes == 4 || index_bytes == 8, APT_EINVAL, "apt_find_long_rows: index_bytes %d", index_bytes);
+  if (long_slots(num_edges) == 0) return APT_OK;
+  APT_REQUIRE(indptr != nullptr && long_table != nullptr, APT_EINVAL, "apt_find_long_rows: a tensor is NULL");
+  const LongRows l = long_rows(long_table, num_edges, nullptr);
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  return index_bytes == 8 ? find_long_rows<int64_t>(indptr, num_src, l, st) : find_long_rows<uint32_t>(indptr, num_src, l, st);
+}
+
+extern "C" size_t apt_coo_sum_workspace_bytes(int64_t num_edges, int64_t num_out_rows, int grouped, int has_long, int64_t dim) {
+  using namespace apt;
+  if (num_edges < 0 || num_edges > 0x7fffffffLL || num_out_rows < 0 || num_out_rows > 0x7fffffffLL || dim <= 0) return 0;
+  size_t offsets = coo_align(sizeof(uint32_t) * (num_out_rows + 1));
+  if (grouped == 0 || has_long != 0) offsets += long_table_bytes(num_edges) + long_part_bytes(num_edges, dim);
   if (grouped != 0) return offsets;
   const size_t order = apt_block_transpose_workspace_bytes(num_edges, 1, num_out_rows);
   return order == 0 ? 0 : offsets + coo_align(sizeof(uint32_t) * (num_edges + 1)) + order;
 }
 
-extern "C" int apt_coo_sum(int mode, const int64_t* keys, const int64_t* sources, int64_t num_edges, int grouped,
+extern "C" int apt_coo_sum(int mode, const int64_t* keys, const int64_t* sources, int64_t num_edges, int grouped, int has_long,
                            const void* input, int64_t num_in_rows, const void* edata, int64_t dim, int elem_size, void* out,
                            int64_t num_out_rows, void* workspace, size_t workspace_bytes, void* stream) {
   using namespace apt;
@@ -334,7 +468,7 @@ extern "C" int apt_coo_sum(int mode, const int64_t* keys, const int64_t* sources
               (long long)num_out_rows, (long long)dim);
   APT_REQUIRE(elem_size == 2 || elem_size == 4, APT_EINVAL, "apt_coo_sum: elem_size %d (4 = fp32, 2 = bf16)", elem_size);
   if (num_out_rows == 0) return APT_OK;
-  const size_t need = apt_coo_sum_workspace_bytes(num_edges, num_out_rows, grouped);
+  const size_t need = apt_coo_sum_workspace_bytes(num_edges, num_out_rows, grouped, has_long, dim);
   APT_REQUIRE(need > 0, APT_ELIMIT, "apt_coo_sum: %lld edges or %lld rows out of range", (long long)num_edges,
               (long long)num_out_rows);
   APT_REQUIRE(out != nullptr && (num_edges == 0 || (keys != nullptr && sources != nullptr && input != nullptr)) &&
@@ -346,17 +480,23 @@ extern "C" int apt_coo_sum(int mode, const int64_t* keys, const int64_t* sources
   char* ws = static_cast<char*>(workspace);
   uint32_t* indptr = reinterpret_cast<uint32_t*>(ws);
   ws += coo_align(sizeof(uint32_t) * (num_out_rows + 1));
+  LongRows lng{};
+  if (grouped == 0 || has_long != 0) {
+    lng = long_rows(ws, num_edges, reinterpret_cast<float*>(ws + long_table_bytes(num_edges)));
+    ws += long_table_bytes(num_edges) + long_part_bytes(num_edges, dim);
+  }
   uint32_t* order = nullptr;
   if (grouped != 0) {
     const int64_t work = std::max(num_edges, num_out_rows + 1);
     hipLaunchKernelGGL(coo_offsets_kernel, dim3(static_cast<unsigned>(std::min<int64_t>(ceil_div(work, kAggBlock), 4096))),
                        dim3(kAggBlock), 0, st, keys, num_edges, num_out_rows, indptr);
     APT_LAUNCH_CHECK("coo_offsets_kernel");
+    if (const int rc = find_long_rows<uint32_t>(indptr, num_out_rows, lng, st)) return rc;
   } else {
     order = reinterpret_cast<uint32_t*>(ws);
     ws += coo_align(sizeof(uint32_t) * (num_edges + 1));
     const size_t left = workspace_bytes - static_cast<size_t>(ws - static_cast<char*>(workspace));
-    if (const int rc = apt_block_transpose(keys, num_edges, 1, num_out_rows, indptr, order, ws, left, stream)) return rc;
+    if (const int rc = apt_block_transpose(keys, num_edges, 1, num_out_rows, indptr, order, lng.row, ws, left, stream)) return rc;
   }
   SourceSumParams p{};
   p.scale = 1.f;
@@ -370,26 +510,37 @@ extern "C" int apt_coo_sum(int mode, const int64_t* keys, const int64_t* sources
   p.dim = dim;
   p.num_src = num_out_rows;
   p.dx = out;
-  return mode == 2 ? source_sum<uint32_t, true>(p, elem_size, st) : source_sum<uint32_t, false>(p, elem_size, st);
+  p.lng = lng;
+  return mode == 2 ? source_sum<uint32_t, true>(p, num_edges, elem_size, st)
+                   : source_sum<uint32_t, false>(p, num_edges, elem_size, st);
+}
+
+extern "C" size_t apt_block_aggregate_backward_workspace_bytes(int64_t num_edges, int64_t dim) {
+  return num_edges < 0 || num_edges > 0x7fffffffLL || dim <= 0 ? 0 : apt::long_part_bytes(num_edges, dim);
 }
 
 extern "C" int apt_block_aggregate_backward(const void* indptr, const void* index, int index_bytes, int fanout,
-                                            int64_t num_src, const float* dst_scale, float scale, const void* dz, int64_t num_dst,
-                                            int64_t dim, int elem_size, void* dx, void* stream) {
+                                            int64_t num_src, int64_t num_edges, void* long_table, const float* dst_scale,
+                                            float scale, const void* dz, int64_t num_dst, int64_t dim, int elem_size, void* dx,
+                                            void* workspace, size_t workspace_bytes, void* stream) {
   using namespace apt;
-  APT_REQUIRE(num_src >= 0 && num_src <= 0x7fffffffLL && num_dst >= 0 && dim > 0, APT_EINVAL,
-              "apt_block_aggregate_backward: bad shape (num_src %lld, num_dst %lld, dim %lld)", (long long)num_src,
-              (long long)num_dst, (long long)dim);
+  APT_REQUIRE(num_src >= 0 && num_src <= 0x7fffffffLL && num_edges >= 0 && num_edges <= 0x7fffffffLL && num_dst >= 0 && dim > 0,
+              APT_EINVAL, "apt_block_aggregate_backward: bad shape (num_src %lld, edges %lld, num_dst %lld, dim %lld)",
+              (long long)num_src, (long long)num_edges, (long long)num_dst, (long long)dim);
   APT_REQUIRE(elem_size == 2 || elem_size == 4, APT_EINVAL,
               "apt_block_aggregate_backward: elem_size %d (4 = fp32, 2 = bf16)", elem_size);
   APT_REQUIRE(index_bytes == 8 || (index_bytes == 4 && fanout > 0), APT_EINVAL,
               "apt_block_aggregate_backward: index_bytes %d (8 = destinations, 4 = slots, with the fanout)", index_bytes);
   if (num_src == 0) return APT_OK;
-  APT_REQUIRE(indptr != nullptr && dx != nullptr && (num_dst == 0 || (index != nullptr && dz != nullptr)), APT_EINVAL,
-              "apt_block_aggregate_backward: a tensor is NULL");
+  APT_REQUIRE(indptr != nullptr && dx != nullptr && (num_dst == 0 || dz != nullptr) && (num_edges == 0 || index != nullptr),
+              APT_EINVAL, "apt_block_aggregate_backward: a tensor is NULL");
+  const size_t need = long_table == nullptr ? 0 : apt_block_aggregate_backward_workspace_bytes(num_edges, dim);
+  APT_REQUIRE(need == 0 || (workspace != nullptr && workspace_bytes >= need && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0),
+              APT_EWORKSPACE, "apt_block_aggregate_backward: workspace too small or not 16-byte aligned "
+                              "(see apt_block_aggregate_backward_workspace_bytes)");
   SourceSumParams p{};
   p.indptr = indptr;
-  p.index = index;
+  p.index = index != nullptr ? index : indptr;   // (no edge: never read)
   p.fanout = static_cast<uint32_t>(fanout);
   p.dst_scale = dst_scale;
   p.scale = scale;
@@ -398,6 +549,8 @@ extern "C" int apt_block_aggregate_backward(const void* indptr, const void* inde
   p.dim = dim;
   p.num_src = num_src;
   p.dx = dx;
+  p.lng = long_rows(long_table, num_edges, static_cast<float*>(workspace));
   hipStream_t st = static_cast<hipStream_t>(stream);
-  return index_bytes == 8 ? source_sum<int64_t, false>(p, elem_size, st) : source_sum<uint32_t, false>(p, elem_size, st);
+  return index_bytes == 8 ? source_sum<int64_t, false>(p, num_edges, elem_size, st)
+                          : source_sum<uint32_t, false>(p, num_edges, elem_size, st);
 }

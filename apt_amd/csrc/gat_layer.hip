@@ -17,6 +17,7 @@
 
 #include "common.hpp"
 #include "feature_rows.hpp"
+#include "long_rows.hpp"
 #include "partial_sums.hpp"
 
 namespace apt {
@@ -185,7 +186,8 @@ static bool launch_pair_scores(const void* x, int64_t n, int64_t num_dst, int he
 }
 
 // ------------------------------------------------------------------ backward, source half
-// As source_sum_kernel (block_grad.hip): a lane group per source row, hubs shared by the workgroup.
+// As source_sum_kernel (block_grad.hip): a lane group per source row, hubs shared by the workgroup, rows too long for one
+// workgroup cut into chunks (long_rows.hpp; a chunk's sum: the row's features, then the heads' logit gradients).
 constexpr int kGatHubEdges = 16;
 constexpr int kGatHubList = 1024;
 constexpr int kGatSourceBlocks = 2048;
@@ -205,6 +207,7 @@ struct GatSourceParams {
   int64_t dim;              // per head
   void* d_ft;               // [num_src, heads * dim]
   float* d_el;              // [num_src, heads]
+  LongRows lng;
 };
 
 // VEC consecutive features of a row belong to at most two heads (dim >= VEC): h0, and h1 from element `cut` on.
@@ -223,6 +226,7 @@ __global__ __launch_bounds__(kAggBlock) void gat_source_kernel(GatSourceParams p
   __shared__ int s_hub[kGatHubList];
   __shared__ int s_hubs;
   __shared__ float s_sum[kGroups][LPR * (VEC + 2)];
+  __shared__ uint32_t s_wave[kAggWaves], s_where[2];
   const int grp = threadIdx.x / LPR, l = threadIdx.x % LPR;
   const I* indptr = static_cast<const I*>(p.indptr);
   const I* index = static_cast<const I*>(p.index);
@@ -334,6 +338,35 @@ __global__ __launch_bounds__(kAggBlock) void gat_source_kernel(GatSourceParams p
     if (TWO && col.cut < VEC) p.d_el[r * p.heads + col.h1] = e1;
     store_vec<T, VEC>(d_ft, r * row_len + col.c, out);
   };
+  // acc += the edges [lo, hi), every kGroups-th by this group
+  auto add_span = [&](int64_t lo, int64_t hi, const Cols& col, Acc& acc) {
+    for (int64_t e = lo + grp; e < hi; e += kAggBlock) {
+      int64_t d, w;
+      edge_of(e + l * kGroups, hi, d, w);
+      add_edges(d, w, 0, static_cast<int>(min((hi - e + kGroups - 1) / kGroups, static_cast<int64_t>(LPR))), col, acc);
+    }
+  };
+  // The groups' sums together, in order, for the first group.
+  auto over_groups = [&](Acc& acc) {
+#pragma unroll
+    for (int k = 0; k < VEC; ++k) s_sum[grp][k * LPR + l] = acc.v[k];
+    s_sum[grp][VEC * LPR + l] = acc.el0;
+    s_sum[grp][(VEC + 1) * LPR + l] = acc.el1;
+    __syncthreads();
+    if (grp == 0) {
+      clear(acc);
+#pragma unroll 1
+      for (int g = 0; g < kGroups; ++g) {
+#pragma unroll
+        for (int k = 0; k < VEC; ++k) acc.v[k] += s_sum[g][k * LPR + l];
+        acc.el0 += s_sum[g][VEC * LPR + l];
+        acc.el1 += s_sum[g][(VEC + 1) * LPR + l];
+      }
+    }
+    __syncthreads();
+  };
+  uint32_t lengthy = 0;   // asked for now, looked at in the end
+  for (int s = threadIdx.x; s < p.lng.slots; s += kAggBlock) lengthy |= p.lng.row[s];
   const int64_t row_groups = static_cast<int64_t>(gridDim.x) * kGroups;
   for (int64_t c0 = 0; c0 < row_len; c0 += LPR * VEC) {
     const Cols col = columns(c0);
@@ -360,7 +393,8 @@ __global__ __launch_bounds__(kAggBlock) void gat_source_kernel(GatSourceParams p
         const int64_t r = r0 + q * row_groups;
         if (r >= p.num_src) break;
         if (hi[q] - lo[q] > kGatHubEdges) {
-          if (l == 0 && c0 == 0) s_hub[atomicAdd(&s_hubs, 1)] = static_cast<int>(r);
+          if (l == 0 && c0 == 0 && (p.lng.slots == 0 || hi[q] - lo[q] <= p.lng.longer))
+            s_hub[atomicAdd(&s_hubs, 1)] = static_cast<int>(r);
           continue;
         }
         Acc acc;
@@ -385,41 +419,61 @@ __global__ __launch_bounds__(kAggBlock) void gat_source_kernel(GatSourceParams p
       const Cols col = columns(c0);
       Acc acc;
       clear(acc);
-      for (int64_t e = lo + grp; e < hi; e += kAggBlock) {   // every kGroups-th edge, so that all groups have some
-        int64_t d, w;
-        edge_of(e + l * kGroups, hi, d, w);
-        add_edges(d, w, 0, static_cast<int>(min((hi - e + kGroups - 1) / kGroups, static_cast<int64_t>(LPR))), col, acc);
-      }
+      add_span(lo, hi, col, acc);   // (all groups have some of the edges)
+      over_groups(acc);
+      if (grp == 0) finish(r, col, acc);
+    }
+  }
+  if (p.lng.slots == 0 || !__syncthreads_or(lengthy != 0)) return;
+  LongChunks<kAggBlock, I> chunks(p.lng, indptr);
+  chunks.number(s_wave);
+  const int64_t width = row_len + p.heads;
+  for (uint32_t q = blockIdx.x; q < chunks.all; q += gridDim.x) {   // block-uniform
+    const auto chunk = chunks.find(q, s_where);
+    float* sum = p.lng.part + static_cast<int64_t>(q) * width;
+    for (int64_t c0 = 0; c0 < row_len; c0 += LPR * VEC) {
+      const Cols col = columns(c0);
+      Acc acc;
+      clear(acc);
+      add_span(chunk.from, chunk.to, col, acc);
+      over_groups(acc);
+      if (grp == 0 && col.live) {
 #pragma unroll
-      for (int k = 0; k < VEC; ++k) s_sum[grp][k * LPR + l] = acc.v[k];
-      s_sum[grp][VEC * LPR + l] = acc.el0;
-      s_sum[grp][(VEC + 1) * LPR + l] = acc.el1;
-      __syncthreads();
-      if (grp == 0) {
-        clear(acc);
-#pragma unroll 1
-        for (int g = 0; g < kGroups; ++g) {
-#pragma unroll
-          for (int k = 0; k < VEC; ++k) acc.v[k] += s_sum[g][k * LPR + l];
-          acc.el0 += s_sum[g][VEC * LPR + l];
-          acc.el1 += s_sum[g][(VEC + 1) * LPR + l];
-        }
-        finish(r, col, acc);
+        for (int k = 0; k < VEC; ++k) sum[col.c + k] = acc.v[k];
+        if (col.start) sum[row_len + col.h0] = acc.el0;
+        if (TWO && col.cut < VEC) sum[row_len + col.h1] = acc.el1;
       }
-      __syncthreads();
+    }
+    if (!chunks.last_of_row(chunk, s_where)) continue;
+    const float* part = p.lng.part + static_cast<int64_t>(q - chunk.index) * width;
+    for (int64_t c0 = 0; c0 < row_len; c0 += LPR * VEC) {
+      const Cols col = columns(c0);
+      Acc acc;
+      clear(acc);
+      for (uint32_t g = grp; g < chunk.count && col.live; g += kGroups) {
+        const float* at = part + static_cast<int64_t>(g) * width;
+#pragma unroll
+        for (int k = 0; k < VEC; ++k) acc.v[k] += at[col.c + k];
+        acc.el0 += at[row_len + col.h0];
+        if (TWO) acc.el1 += at[row_len + col.h1];
+      }
+      over_groups(acc);
+      if (grp == 0) finish(chunk.row, col, acc);
     }
   }
 }
 
 template <typename T, int VEC, typename I, bool TWO>
-static void launch_gat_source_as(const GatSourceParams& p, hipStream_t st) {
+static void launch_gat_source_as(const GatSourceParams& p, int64_t num_edges, hipStream_t st) {
   const int64_t per_row = ceil_div(p.heads * p.dim, VEC);
 #define APT_GAT_SOURCE(LPR)                                                                                        \
   do {                                                                                                            \
+    const int64_t for_edges = std::max(std::min(p.num_src, num_edges / (kAggBlock / LPR * kGatHubEdges)),         \
+                                       p.lng.slots > 0 ? long_chunks(num_edges) : 0);                             \
     const int64_t blocks = std::max(ceil_div(p.num_src, kGatHubList),                                             \
-                                    std::min<int64_t>(ceil_div(p.num_src, 4 * kAggBlock / LPR), kGatSourceBlocks));   \
-    hipLaunchKernelGGL((gat_source_kernel<T, VEC, LPR, I, TWO>), dim3(static_cast<unsigned>(blocks)), dim3(kAggBlock), 0, \
-                       st, p);                                                                                    \
+                                    std::min<int64_t>(std::max(ceil_div(p.num_src, 4 * kAggBlock / LPR), for_edges), \
+                                                      kGatSourceBlocks));                                         \
+    hipLaunchKernelGGL((gat_source_kernel<T, VEC, LPR, I, TWO>), dim3(static_cast<unsigned>(blocks)), dim3(kAggBlock), 0, st, p); \
   } while (0)
   if (per_row <= 8) APT_GAT_SOURCE(8);
   else if (per_row <= 16) APT_GAT_SOURCE(16);
@@ -429,22 +483,22 @@ static void launch_gat_source_as(const GatSourceParams& p, hipStream_t st) {
 }
 
 template <typename T, int VEC, typename I>
-static void launch_gat_source(const GatSourceParams& p, hipStream_t st) {
-  if (VEC > 1 && p.dim % VEC != 0) launch_gat_source_as<T, VEC, I, (VEC > 1)>(p, st);
-  else launch_gat_source_as<T, VEC, I, false>(p, st);
+static void launch_gat_source(const GatSourceParams& p, int64_t num_edges, hipStream_t st) {
+  if (VEC > 1 && p.dim % VEC != 0) launch_gat_source_as<T, VEC, I, (VEC > 1)>(p, num_edges, st);
+  else launch_gat_source_as<T, VEC, I, false>(p, num_edges, st);
 }
 
 template <typename T, typename I>
-static void launch_gat_source_t(const GatSourceParams& p, hipStream_t st) {
+static void launch_gat_source_t(const GatSourceParams& p, int64_t num_edges, hipStream_t st) {
   const bool aligned = ((reinterpret_cast<uintptr_t>(p.d_out) | reinterpret_cast<uintptr_t>(p.d_ft)) & 15) == 0;
   if constexpr (sizeof(T) == 2) {   // 16 bytes a lane: twice the rows in a wavefront
     if (aligned && (p.heads * p.dim) % 8 == 0 && p.dim >= 8) {
-      launch_gat_source<T, 8, I>(p, st);
+      launch_gat_source<T, 8, I>(p, num_edges, st);
       return;
     }
   }
-  if (aligned && (p.heads * p.dim) % 4 == 0 && p.dim >= 4) launch_gat_source<T, 4, I>(p, st);
-  else launch_gat_source<T, 1, I>(p, st);
+  if (aligned && (p.heads * p.dim) % 4 == 0 && p.dim >= 4) launch_gat_source<T, 4, I>(p, num_edges, st);
+  else launch_gat_source<T, 1, I>(p, num_edges, st);
 }
 
 // ------------------------------------------------------------------ backward, parameters
@@ -607,7 +661,8 @@ extern "C" size_t apt_gat_layer_backward_workspace_bytes(int64_t num_dst, int fa
   if (num_dst < 0 || fanout <= 0 || num_src < 0 || heads <= 0 || dim <= 0 || num_edges < 0) return 0;
   const int64_t weights = std::max(num_dst * fanout, num_edges) * heads;
   return align256(sizeof(float) * 2 * weights) + align256(sizeof(float) * (num_dst + num_src) * heads) +
-         align256(sizeof(float) * 3 * heads * dim * param_blocks(num_src)) + 256;
+         align256(sizeof(float) * 3 * heads * dim * param_blocks(num_src)) +
+         align256(sizeof(float) * long_chunks(std::max(num_dst * fanout, num_edges)) * (heads * dim + heads)) + 256;
 }
 
 extern "C" int apt_gat_layer_backward(const int64_t* neighbors, int64_t num_dst, int fanout, const void* ft,
@@ -615,7 +670,7 @@ extern "C" int apt_gat_layer_backward(const int64_t* neighbors, int64_t num_dst,
                                       const void* attn_r, int attn_elem_size, float negative_slope, const float* el,
                                       const float* er, const float* attn, const void* d_out, const void* indptr,
                                       const void* index, int index_bytes, const int64_t* eids, const int64_t* csc_indptr,
-                                      int64_t num_edges, void* d_ft, void* d_attn_l, void* d_attn_r, void* d_bias,
+                                      int64_t num_edges, void* long_table, void* d_ft, void* d_attn_l, void* d_attn_r, void* d_bias,
                                       void* workspace, size_t workspace_bytes, void* stream) {
   using namespace apt;
   const char* who = "apt_gat_layer_backward";
@@ -647,6 +702,7 @@ extern "C" int apt_gat_layer_backward(const int64_t* neighbors, int64_t num_dst,
   float* d_el = d_er + num_dst * heads;
   ws += align256(sizeof(float) * (num_dst + num_src) * heads);
   float* part = reinterpret_cast<float*>(ws);
+  ws += align256(sizeof(float) * 3 * heads * dim * param_blocks(num_src));
   if (const int rc = gat_edge_grad(who, neighbors, num_dst, fanout, ft, num_src, heads, dim, elem_size, el, er,
                                    negative_slope, attn, d_out, true, by_slot ? nullptr : csc_indptr, a_edge, dz, d_er, st))
     return rc;
@@ -667,6 +723,8 @@ extern "C" int apt_gat_layer_backward(const int64_t* neighbors, int64_t num_dst,
   p.dim = dim;
   p.d_ft = d_ft;
   p.d_el = d_el;
+  const int64_t edges = by_slot ? num_dst * fanout : num_edges;
+  p.lng = long_rows(long_table, edges, reinterpret_cast<float*>(ws));
   if (num_dst == 0) {   // entry 0 of every array is read in the place of a missing edge
     p.d_out = ft;
     p.attn = p.dz = el;
@@ -674,11 +732,11 @@ extern "C" int apt_gat_layer_backward(const int64_t* neighbors, int64_t num_dst,
   if (index == nullptr || num_dst == 0) p.index = indptr;
   if (!by_slot && (eids == nullptr || num_edges == 0)) p.eids = static_cast<const int64_t*>(indptr);
   if (elem_size == 4) {
-    if (by_slot) launch_gat_source_t<float, uint32_t>(p, st);
-    else launch_gat_source_t<float, int64_t>(p, st);
+    if (by_slot) launch_gat_source_t<float, uint32_t>(p, edges, st);
+    else launch_gat_source_t<float, int64_t>(p, edges, st);
   } else {
-    if (by_slot) launch_gat_source_t<uint16_t, uint32_t>(p, st);
-    else launch_gat_source_t<uint16_t, int64_t>(p, st);
+    if (by_slot) launch_gat_source_t<uint16_t, uint32_t>(p, edges, st);
+    else launch_gat_source_t<uint16_t, int64_t>(p, edges, st);
   }
   APT_LAUNCH_CHECK("gat_source_kernel");
   if (d_attn_l == nullptr && d_attn_r == nullptr && d_bias == nullptr) return APT_OK;

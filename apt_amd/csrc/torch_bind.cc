@@ -898,21 +898,21 @@ Tensor spmm(int mode, Tensor coo_row, Tensor coo_col, Tensor input, const Tensor
   // Ordering the edges costs some 40 us of launches, as much as about 3.5 M atomic additions: few edges or short rows
   // are added up as they come (951 seeds' edges of 16 fp32, both directions and scores: 90 us, ordered 103 us).
   if (E * x.size(1) <= int64_t{1} << 21) return by_edge(oo.index({-1}).item<int64_t>());
-  // every edge's rows, whether the edges come grouped by output row (a block's COO does), and the number of output
-  // rows: the last two are read back in one copy
+  // every edge's rows, whether the edges come grouped by output row (a block's COO does), the number of output rows, and
+  // whether some may have very many edges: the last three are read back in one copy
   auto keys = torch::empty({2, E}, i64_opts());
-  auto probe = torch::empty({2}, i64_opts());
+  auto probe = torch::empty({3}, i64_opts());
   check(apt_coo_prepare(i64(row), i64(col), E, i64(coo), input_offset ? i64(io) : nullptr, i64(oo), nseg,
                         i64(oo) + oo.numel() - 1, keys.data_ptr<int64_t>(), keys.data_ptr<int64_t>() + E,
                         probe.data_ptr<int64_t>(), stream()));
   const int64_t* host = read_counts(probe);
-  const int grouped = host[0] != 0;
+  const int grouped = host[0] != 0, has_long = host[2] != 0;
   const int64_t out_num = host[1];
-  const size_t need = apt_coo_sum_workspace_bytes(E, out_num, grouped);
+  const size_t need = apt_coo_sum_workspace_bytes(E, out_num, grouped, has_long, x.size(1));
   if (need > 0) {
     auto ws = torch::empty({static_cast<int64_t>(need)}, x.options().dtype(torch::kUInt8));
     auto out = torch::empty({out_num, x.size(1)}, x.options());
-    check(apt_coo_sum(mode, i64(keys), E ? i64(keys) + E : nullptr, E, grouped, x.data_ptr(), x.size(0),
+    check(apt_coo_sum(mode, i64(keys), E ? i64(keys) + E : nullptr, E, grouped, has_long, x.data_ptr(), x.size(0),
                       edata ? ed.data_ptr() : nullptr, x.size(1), static_cast<int>(x.element_size()), out.data_ptr(),
                       out_num, ws.data_ptr(), need, stream()));
     return out;
@@ -1081,22 +1081,57 @@ void check_block(const char* who, const Tensor& relabeled, int64_t num_dst, int6
 }
 
 // The edges of every source of a block: slots (4-byte, apt_block_transpose), or, for a block too large for that, the
-// destinations of its CSR (8-byte).  Enqueued on the current stream; nothing is read back.
+// destinations of its CSR (8-byte), with the table of the sources that have very many and `scratch` bytes beside it.
+// Enqueued on the current stream; nothing is read back.
 struct SourceOrder {
-  Tensor indptr, index;
+  Tensor memory, csr_indptr, csr_index;
+  const void* indptr = nullptr;
+  const void* index = nullptr;
+  void* table = nullptr;        // NULL: no source can have so many
+  void* scratch = nullptr;
+  size_t scratch_bytes = 0;
   int bytes = 4;
+  int64_t edges = 0;            // what index holds
 };
-SourceOrder source_order(const Tensor& relabeled, int64_t num_dst, int64_t fanout, int64_t num_src) {
+size_t aligned(size_t x) { return (x + 255) / 256 * 256; }
+
+// of a CSR
+SourceOrder source_order_csr(const Tensor& csr_indptr, const Tensor& csr_index, int64_t num_src, size_t scratch) {
   SourceOrder o;
+  o.csr_indptr = csr_indptr;
+  o.csr_index = csr_index;
+  o.indptr = csr_indptr.data_ptr();
+  o.index = csr_index.numel() > 0 ? csr_index.data_ptr() : nullptr;
+  o.bytes = 8;
+  o.edges = csr_index.numel();
+  if (const size_t need = apt_long_rows_bytes(o.edges)) {
+    o.memory = torch::empty({static_cast<int64_t>(aligned(need) + scratch)}, csr_indptr.options().dtype(torch::kUInt8));
+    o.table = o.memory.data_ptr();
+    o.scratch = static_cast<char*>(o.table) + aligned(need);
+    o.scratch_bytes = scratch;
+    check(apt_find_long_rows(o.indptr, 8, num_src, o.edges, o.table, stream()));
+  }
+  return o;
+}
+
+SourceOrder source_order(const Tensor& relabeled, int64_t num_dst, int64_t fanout, int64_t num_src, size_t scratch) {
   const int64_t slots = std::max<int64_t>(num_dst * fanout, 1);
   const int f = static_cast<int>(fanout);
-  const auto u8 = relabeled.options().dtype(torch::kUInt8), i32 = relabeled.options().dtype(torch::kInt32);
+  const auto u8 = relabeled.options().dtype(torch::kUInt8);
   if (const size_t need = apt_block_transpose_workspace_bytes(num_dst, f, num_src)) {
-    o.indptr = torch::empty({num_src + 1}, i32);
-    o.index = torch::empty({slots}, i32);
-    auto ws = torch::empty({static_cast<int64_t>(need)}, u8);
-    check(apt_block_transpose(i64(relabeled), num_dst, f, num_src, reinterpret_cast<uint32_t*>(o.indptr.data_ptr<int>()),
-                              reinterpret_cast<uint32_t*>(o.index.data_ptr<int>()), ws.data_ptr(), need, stream()));
+    SourceOrder o;
+    o.edges = num_dst * fanout;
+    const size_t offsets = aligned(4 * (static_cast<size_t>(num_src) + 1)), entries = aligned(4 * static_cast<size_t>(slots)),
+                 table = aligned(apt_long_rows_bytes(o.edges));
+    o.scratch_bytes = std::max(need, scratch);   // first the transpose's, then the caller's
+    o.memory = torch::empty({static_cast<int64_t>(offsets + entries + table + o.scratch_bytes)}, u8);
+    char* at = static_cast<char*>(o.memory.data_ptr());
+    o.indptr = at;
+    o.index = at + offsets;
+    o.table = table > 0 ? at + offsets + entries : nullptr;
+    o.scratch = at + offsets + entries + table;
+    check(apt_block_transpose(i64(relabeled), num_dst, f, num_src, reinterpret_cast<uint32_t*>(at),
+                              reinterpret_cast<uint32_t*>(at + offsets), o.table, o.scratch, need, stream()));
     return o;
   }
   const size_t need = apt_block_workspace_bytes(num_dst, f, num_src, 1);
@@ -1104,14 +1139,12 @@ SourceOrder source_order(const Tensor& relabeled, int64_t num_dst, int64_t fanou
   auto ws = torch::empty({static_cast<int64_t>(need)}, u8);
   auto coo = torch::empty({2, slots}, relabeled.options()), csc = torch::empty({num_dst + 1}, relabeled.options());
   auto edges = torch::empty({1}, relabeled.options()), eids = torch::empty({slots}, relabeled.options());
-  o.indptr = torch::empty({num_src + 1}, relabeled.options());
-  o.index = torch::empty({slots}, relabeled.options());
-  o.bytes = 8;
+  auto indptr = torch::empty({num_src + 1}, relabeled.options()), index = torch::empty({slots}, relabeled.options());
   check(apt_block_formats(i64(relabeled), num_dst, nullptr, f, num_src, coo.data_ptr<int64_t>(),
                           coo.data_ptr<int64_t>() + slots, csc.data_ptr<int64_t>(), edges.data_ptr<int64_t>(),
-                          o.indptr.data_ptr<int64_t>(), o.index.data_ptr<int64_t>(), eids.data_ptr<int64_t>(),
-                          ws.data_ptr(), need, stream()));
-  return o;
+                          indptr.data_ptr<int64_t>(), index.data_ptr<int64_t>(), eids.data_ptr<int64_t>(), ws.data_ptr(), need,
+                          stream()));
+  return source_order_csr(indptr, index, num_src, scratch);
 }
 
 // The gradient of the block sum / mean towards its input, from the block's CSR if it has one.
@@ -1119,17 +1152,15 @@ Tensor aggregate_backward(const Tensor& dz_in, const Tensor& relabeled, int64_t 
                           const Tensor& dst_scale, const Tensor& csr_indptr, const Tensor& csr_indices, float scale = 1.f) {
   auto dz = dz_in.contiguous();
   auto dx = torch::empty({num_src, dz.size(1)}, dz.options());
-  SourceOrder o;
-  if (csr_indptr.defined() && csr_indptr.numel() == num_src + 1) {
-    o.indptr = csr_indptr;
-    o.index = csr_indices.numel() > 0 ? csr_indices : csr_indptr;   // (no edge: never read, and not NULL)
-    o.bytes = 8;
-  } else {
-    o = source_order(relabeled, num_dst, fanout, num_src);
-  }
-  check(apt_block_aggregate_backward(o.indptr.data_ptr(), o.index.data_ptr(), o.bytes, static_cast<int>(fanout), num_src,
+  const bool csr = csr_indptr.defined() && csr_indptr.numel() == num_src + 1;
+  const size_t scratch =
+      apt_block_aggregate_backward_workspace_bytes(csr ? csr_indices.numel() : num_dst * fanout, dz.size(1));
+  const SourceOrder o = csr ? source_order_csr(csr_indptr, csr_indices, num_src, scratch)
+                            : source_order(relabeled, num_dst, fanout, num_src, scratch);
+  check(apt_block_aggregate_backward(o.indptr, o.index, o.bytes, static_cast<int>(fanout), num_src, o.edges, o.table,
                                      dst_scale.defined() ? dst_scale.data_ptr<float>() : nullptr, scale, dz.data_ptr(), num_dst,
-                                     dz.size(1), static_cast<int>(dz.element_size()), dx.data_ptr(), stream()));
+                                     dz.size(1), static_cast<int>(dz.element_size()), dx.data_ptr(), o.scratch, o.scratch_bytes,
+                                     stream()));
   return dx;
 }
 
@@ -1474,23 +1505,18 @@ struct GatLayerFn : public torch::autograd::Function<GatLayerFn> {
     Tensor eids, csc;
     int64_t edges = 0;
     if (saved[6].defined()) {
-      o.indptr = saved[6];
-      o.index = saved[7];
-      o.bytes = 8;
       eids = saved[8];
       csc = saved[9];
-      edges = eids.numel();
+      o = source_order_csr(saved[6], saved[7], n, 0);
     } else if (apt_block_transpose_workspace_bytes(num_dst, static_cast<int>(fanout), n) > 0) {
-      o = source_order(relabeled, num_dst, fanout, n);
+      o = source_order(relabeled, num_dst, fanout, n, 0);
     } else {
       auto f = BlockFormats(relabeled, num_dst, fanout, n, true);
       csc = f[2];
-      o.indptr = f[3];
-      o.index = f[4];
-      o.bytes = 8;
       eids = f[5];
-      edges = eids.numel();
+      o = source_order_csr(f[3], f[4], n, 0);
     }
+    if (o.bytes == 8) edges = o.edges;
     auto d_ft = torch::empty_like(ft), d_al = torch::empty_like(attn_l), d_ar = torch::empty_like(attn_r);
     Tensor d_bias;
     if (bias) d_bias = torch::empty({heads, dim}, ft.options());
@@ -1502,9 +1528,9 @@ struct GatLayerFn : public torch::autograd::Function<GatLayerFn> {
                                  static_cast<int>(heads), dim, static_cast<int>(ft.element_size()), attn_l.data_ptr(),
                                  attn_r.data_ptr(), static_cast<int>(attn_l.element_size()),
                                  static_cast<float>(ctx->saved_data["slope"].toDouble()), el, el + n * heads,
-                                 attn.data_ptr<float>(), d_out.data_ptr(), o.indptr.data_ptr(), o.index.data_ptr(), o.bytes,
+                                 attn.data_ptr<float>(), d_out.data_ptr(), o.indptr, o.index, o.bytes,
                                  o.bytes == 8 ? i64(eids) : nullptr, o.bytes == 8 ? i64(csc) : nullptr, edges,
-                                 d_ft.data_ptr(), d_al.data_ptr(), d_ar.data_ptr(), bias ? d_bias.data_ptr() : nullptr,
+                                 o.table, d_ft.data_ptr(), d_al.data_ptr(), d_ar.data_ptr(), bias ? d_bias.data_ptr() : nullptr,
                                  ws.data_ptr(), need, stream()));
     torch::autograd::variable_list out(15);
     out[0] = d_ft;

@@ -783,12 +783,21 @@ int apt_spmm_heads(const int64_t* coo_row, const int64_t* coo_col, int64_t num_e
  * (the destination of slot s is s / fanout): indptr uint32[num_src + 1], slots
  * uint32[num_dst * fanout] of which indptr[num_src] are written.  What
  * apt_block_formats' CSR is, without the compaction, in half the bytes.
- * workspace: apt_block_transpose_workspace_bytes; 0 = a block this large is not
- * supported (take apt_block_formats). */
+ * workspace: apt_block_transpose_workspace_bytes (does for smaller blocks too); 0 = a
+ * block this large is not supported (take apt_block_formats).
+ *
+ * long_table, or NULL: the rows with very many edges, which the sums over a transposed
+ * block or a CSR then share out to several workgroups: device scratch of
+ * apt_long_rows_bytes(num_edges) bytes for a block of at most so many edges (slots;
+ * 0: it can have none, and NULL will do), 16-byte aligned.  apt_find_long_rows makes it
+ * from offsets of 4 or 8 bytes (index_bytes). */
 size_t apt_block_transpose_workspace_bytes(int64_t num_dst, int fanout, int64_t num_src);
 int apt_block_transpose(const int64_t* relabeled, int64_t num_dst, int fanout, int64_t num_src,
-                        uint32_t* indptr, uint32_t* slots, void* workspace, size_t workspace_bytes,
-                        void* stream);
+                        uint32_t* indptr, uint32_t* slots, void* long_table, void* workspace,
+                        size_t workspace_bytes, void* stream);
+size_t apt_long_rows_bytes(int64_t num_edges);
+int apt_find_long_rows(const void* indptr, int index_bytes, int64_t num_src, int64_t num_edges,
+                       void* long_table, void* stream);
 
 /* The dense product of a layer in fp32, of two operand pairs at once:
  *   y[r, j] (+)= sum_k x1[r, k] w1[j, k] + (r < m2: sum_k x2[r, k] w2[j, k]) + bias[j]
@@ -821,24 +830,32 @@ int apt_add_rows(void* y, const void* x, int64_t count, int elem_size, int relu,
  *                                 dz (fp32 sums, fixed order).  The edges of a source:
  *                                 index_bytes 8 = csr_indptr / csr_indices of
  *                                 apt_block_formats (fanout ignored), 4 = indptr / slots
- *                                 of apt_block_transpose. */
+ *                                 of apt_block_transpose.  num_edges: what index holds;
+ *                                 long_table: of that many edges, or NULL (a row is then
+ *                                 one workgroup's at the most); workspace for it:
+ *                                 apt_block_aggregate_backward_workspace_bytes, 16-byte
+ *                                 aligned. */
 int apt_block_aggregate(const int64_t* neighbors, int64_t num_dst, int fanout, const void* input,
                         int64_t num_src, int64_t dim, int elem_size, int mean, float scale,
                         const void* bias, const void* base, int relu, void* out,
                         float* inv_degree, void* stream);
+size_t apt_block_aggregate_backward_workspace_bytes(int64_t num_edges, int64_t dim);
 int apt_block_aggregate_backward(const void* indptr, const void* index, int index_bytes, int fanout,
-                                 int64_t num_src, const float* dst_scale, float scale, const void* dz,
-                                 int64_t num_dst, int64_t dim, int elem_size, void* dx, void* stream);
+                                 int64_t num_src, int64_t num_edges, void* long_table, const float* dst_scale,
+                                 float scale, const void* dz, int64_t num_dst, int64_t dim, int elem_size,
+                                 void* dx, void* workspace, size_t workspace_bytes, void* stream);
 
 /* Sums over a COO in any order (apt_spmm_sum's three modes) without atomics, with the
  * result in the input's type; what the spmm_* operators do.
  *   apt_coo_prepare  keys[e] = output_offset[k] + col[e], sources[e] = input_offset[k] +
  *                    row[e] (k = segment of e as in apt_spmm_sum, offsets NULL = 0);
  *                    result[0] = 1 if the keys are non-decreasing, else 0; result[1] =
- *                    *last_offset (0 if NULL): what a caller reads back in one copy
+ *                    *last_offset (0 if NULL); result[2] = 1 if non-decreasing keys may
+ *                    have a row with very many edges: what a caller reads back in one
+ *                    copy
  *   apt_coo_sum      out[r, :] = sum over the edges with key r, in edge order; every
  *                    row is written; edges with a key or source out of range do not
- *                    count.  grouped: result[0]; otherwise the edges are ordered by key
+ *                    count.  grouped: result[0], has_long: result[2]; otherwise the edges are ordered by key
  *                    first (apt_block_transpose).  workspace:
  *                    apt_coo_sum_workspace_bytes, 256-byte aligned; 0 = sizes out of
  *                    range (take apt_spmm_sum)
@@ -847,8 +864,8 @@ int apt_coo_prepare(const int64_t* coo_row, const int64_t* coo_col, int64_t num_
                     const int64_t* coo_offset, const int64_t* input_offset, const int64_t* output_offset,
                     int num_segments, const int64_t* last_offset, int64_t* keys, int64_t* sources,
                     int64_t* result, void* stream);
-size_t apt_coo_sum_workspace_bytes(int64_t num_edges, int64_t num_out_rows, int grouped);
-int apt_coo_sum(int mode, const int64_t* keys, const int64_t* sources, int64_t num_edges, int grouped,
+size_t apt_coo_sum_workspace_bytes(int64_t num_edges, int64_t num_out_rows, int grouped, int has_long, int64_t dim);
+int apt_coo_sum(int mode, const int64_t* keys, const int64_t* sources, int64_t num_edges, int grouped, int has_long,
                 const void* input, int64_t num_in_rows, const void* edata, int64_t dim, int elem_size,
                 void* out, int64_t num_out_rows, void* workspace, size_t workspace_bytes, void* stream);
 int apt_coo_combine(int op, const int64_t* coo_row, const int64_t* coo_col, int64_t num_edges,
@@ -873,7 +890,8 @@ int apt_coo_combine(int op, const int64_t* coo_row, const int64_t* coo_col, int6
  *                           NULL.  The edges by source: index_bytes 4 = indptr / slots
  *                           of apt_block_transpose (eids, csc_indptr NULL, num_edges
  *                           0), 8 = csr_indptr / csr_indices with csr_eids, csc_indptr
- *                           and the edge count of apt_block_formats. */
+ *                           and the edge count of apt_block_formats; long_table: of
+ *                           num_dst * fanout or num_edges edges, or NULL. */
 int apt_gat_layer(const int64_t* neighbors, int64_t num_dst, int fanout, const void* ft, int64_t num_src,
                   int heads, int64_t dim, int elem_size, const void* attn_l, const void* attn_r,
                   int attn_elem_size, const void* bias, int relu, float negative_slope, int wide, float* el, float* er,
@@ -885,7 +903,7 @@ int apt_gat_layer_backward(const int64_t* neighbors, int64_t num_dst, int fanout
                            const void* attn_r, int attn_elem_size, float negative_slope, const float* el,
                            const float* er, const float* attn, const void* d_out, const void* indptr,
                            const void* index, int index_bytes, const int64_t* eids, const int64_t* csc_indptr,
-                           int64_t num_edges, void* d_ft, void* d_attn_l, void* d_attn_r, void* d_bias,
+                           int64_t num_edges, void* long_table, void* d_ft, void* d_attn_l, void* d_attn_r, void* d_bias,
                            void* workspace, size_t workspace_bytes, void* stream);
 
 /* Gradients of a dense layer y = x w^T + b over a block's rows (the fc_self /

@@ -217,7 +217,7 @@ def test_gpu_csr_of_ranges_that_are_sorted_in_parts(capi, num_dst, fanout, num_s
     indptr = torch.empty(num_src + 1, dtype=torch.int32, device="cuda")
     slots = torch.empty(num_dst * fanout, dtype=torch.int32, device="cuda")
     ws = torch.empty(L.apt_block_transpose_workspace_bytes(num_dst, fanout, num_src), dtype=torch.uint8, device="cuda")
-    assert L.apt_block_transpose(rel.data_ptr(), num_dst, fanout, num_src, indptr.data_ptr(), slots.data_ptr(), ws.data_ptr(),
+    assert L.apt_block_transpose(rel.data_ptr(), num_dst, fanout, num_src, indptr.data_ptr(), slots.data_ptr(), None, ws.data_ptr(),
                                  ws.numel(), torch.cuda.current_stream().cuda_stream) == 0
     assert np.array_equal(indptr.cpu().numpy(), want["csr_indptr"])
     assert np.array_equal(slots.cpu().numpy()[: want["num_edges"]], np.nonzero(r >= 0)[0][want["csr_eids"]])

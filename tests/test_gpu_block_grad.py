@@ -1,5 +1,7 @@
 """The gradient of a block's sum / mean towards its input (every source row written once): widths at the edges of the
-lane groups, rows without edges, rows around the length a group adds up alone (32), hubs, and both edge orders."""
+lane groups, rows without edges, rows of the lengths at which the way of adding them up changes (8: the lanes of the smallest
+group; 16: what a group adds up alone; 512, or a 512th of all edges: what a workgroup adds up alone), hubs, and both edge
+orders."""
 import numpy as np
 import pytest
 import torch
@@ -11,7 +13,7 @@ DEV = "cuda:0"
 def _block(num_dst, fanout, num_src, seed):
     rng = np.random.default_rng(seed)
     r = rng.integers(0, num_src, size=num_dst * fanout)
-    for s, n in ((0, 32), (1, 33), (2, 64), (3, 65), (4, 700)):          # sources with a given number of edges
+    for s, n in ((0, 32), (1, 33), (2, 64), (3, 65), (4, 700)):          # sources with about so many edges
         if s < num_src and n <= r.size // 8:
             r[rng.choice(r.size, n, replace=False)] = s
     r[rng.random(r.size) < 0.2] = -1
@@ -49,6 +51,75 @@ def test_block_aggregate_backward(capi, num_dst, fanout, num_src, dim, dtype, me
     again, = torch.autograd.grad(torch.ops.npc.block_aggregate(rel, num_dst, fanout, x, mean, f.get("csr_indptr"),
                                                                f.get("csr_indices")), x, up)
     assert torch.equal(dx, again)
+
+
+# Sources with exactly so many edges.  A row of more than 512 is summed in chunks of 256.  With 400 k more edges in a row,
+# one of more than 812 is (a 512th of the slots), in chunks of 406.
+COUNTS = [0, 1, 7, 8, 9, 15, 16, 17, 18, 31, 32, 33, 64, 65, 255, 256, 257, 511, 512, 513, 514, 767, 768, 769, 811, 812, 813, 814, 1025, 5000, 0, 2]
+
+
+def _counted_block(counts, fanout, holes, seed):
+    """Slots in random order that name source s counts[s] times, and -1."""
+    rng = np.random.default_rng(seed)
+    r = np.concatenate([np.repeat(np.arange(len(counts)), counts), np.full(holes, -1)])
+    r = np.concatenate([r, np.full(-r.size % fanout, -1)])
+    return torch.from_numpy(rng.permutation(r).astype(np.int64)).to(DEV), r.size // fanout
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("dim", [4, 8, 33, 64, 256, 264])
+@pytest.mark.parametrize("with_csr", [False, True])
+@pytest.mark.parametrize("last", [0, 400_000])
+def test_rows_of_every_length(capi, dim, dtype, with_csr, last):
+    import apt_amd  # noqa: F401
+    if last and dim not in (8, 64):
+        pytest.skip("one narrow and one wide row are enough for the longest")
+    counts = COUNTS + [last, 3, 0]
+    num_src = len(counts)
+    rel, num_dst = _counted_block(counts, 5, 777, dim)
+    gen = torch.Generator(device=DEV).manual_seed(dim)
+    x = torch.randn(num_src, dim, generator=gen, device=DEV).to(dtype).requires_grad_(True)
+    up = torch.randn(num_dst, dim, generator=gen, device=DEV).to(dtype)
+    f = capi.block_formats(rel, num_dst, 5, num_src) if with_csr else {}
+    grad = lambda: torch.autograd.grad(torch.ops.npc.block_aggregate(rel, num_dst, 5, x, True, f.get("csr_indptr"),  # noqa: E731
+                                                                     f.get("csr_indices")), x, up)[0]
+    keep = (rel >= 0).nonzero().flatten()
+    src, dst = rel[keep], keep // 5
+    assert torch.bincount(src, minlength=num_src).tolist() == counts
+    w = 1.0 / torch.bincount(dst, minlength=num_dst).clamp(min=1).double()[dst]
+    terms = up.double()[dst] * w[:, None]
+    pick = (torch.arange(num_src, device=DEV)[:, None] == src).double()
+    want, size = pick @ terms, pick @ terms.abs()
+    dx = grad()
+    half = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -22
+    assert bool(((dx.double() - want).abs() <= 1e-6 * size + half * want.abs()).all())
+    for _ in range(3):      # whichever workgroup adds a row's chunks up
+        assert torch.equal(grad(), dx)
+
+
+def test_a_hub_takes_no_longer_than_an_even_block(capi):
+    """100 k edges of one source, 64 features: 13 times the even block's backward pass while one workgroup added a row up
+    (1660 against 122 us; the bound leaves room for a busy machine)."""
+    import apt_amd  # noqa: F401
+    num_dst, fanout, num_src, dim = 100_000, 10, 300_000, 64
+    rel = torch.randint(0, num_src, (num_dst * fanout,), device=DEV)
+    x = torch.randn(num_src, dim, device=DEV, requires_grad=True)
+    up = torch.randn(num_dst, dim, device=DEV)
+
+    def fastest():
+        times = []
+        for _ in range(8):
+            out = torch.ops.npc.block_aggregate(rel, num_dst, fanout, x, False, None, None)
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            torch.autograd.grad(out, x, up)
+            b.record()
+            b.synchronize()
+            times.append(a.elapsed_time(b))
+        return min(times)
+    even = fastest()
+    rel.view(num_dst, fanout)[:, 3] = 70_000
+    assert fastest() <= 4 * even
 
 
 def test_block_aggregate_empty_and_wrong_inputs():

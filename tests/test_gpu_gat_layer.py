@@ -117,3 +117,38 @@ def test_gat_layer_bf16_without_gradients_keeps_fp32(capi, heads, dim, fanout, a
         top = Block(num_dst, 50, None, torch.randint(0, num_dst, (50 * 4,), device=DEV), 4)
         assert torch.equal(upper(top, got.flatten(1)), upper(top, got.flatten(1).bfloat16()))
     assert layer(blk, feat).dtype == torch.bfloat16     # a training step
+
+
+@pytest.mark.parametrize("dtype,attn_dtype", [(torch.float32, torch.float32), (torch.bfloat16, torch.bfloat16)])
+@pytest.mark.parametrize("heads,dim", [(4, 64), (8, 8), (3, 6), (1, 5), (5, 3), (2, 100)])
+@pytest.mark.parametrize("with_csr", [False, True])
+def test_gat_layer_sources_with_given_numbers_of_edges(capi, heads, dim, dtype, attn_dtype, with_csr):
+    """Rows of the source half at the lengths where the way of adding them up changes: 8 (the lanes of the smallest group),
+    16 (a group alone), 512 (a workgroup alone), several chunks, a 512th of the row to a chunk."""
+    import apt_amd  # noqa: F401
+    counts = [0, 7, 8, 9, 15, 16, 17, 18, 33, 255, 511, 512, 513, 769, 5000, 140_000 if heads * dim <= 64 else 900, 1]
+    fanout, rng = 6, np.random.default_rng(heads * dim)
+    r = np.concatenate([np.repeat(np.arange(len(counts)), counts), np.full(1000, -1)])
+    r = rng.permutation(np.concatenate([r, np.full(-r.size % fanout, -1)]))
+    num_dst, rel = r.size // fanout, torch.from_numpy(r.astype(np.int64)).to(DEV)
+    num_src = max(num_dst, len(counts))                     # the destinations are the first sources
+    gen = torch.Generator(device=DEV).manual_seed(dim)
+    rand = lambda *s: torch.randn(*s, generator=gen, device=DEV)  # noqa: E731
+    ft = rand(num_src, heads, dim).to(dtype).requires_grad_(True)
+    al, ar = ((rand(heads, dim) * 0.3).to(attn_dtype).requires_grad_(True) for _ in range(2))
+    up = rand(num_dst, heads, dim).to(dtype)
+    f = capi.block_formats(rel, num_dst, fanout, num_src) if with_csr else {}
+    csr = [f.get(k) for k in ("csr_indptr", "csr_indices", "csr_eids", "csc_indptr")]
+    grads = lambda: torch.autograd.grad(torch.ops.npc.gat_layer(rel, num_dst, fanout, ft, al, ar, None, 0.2, *csr), [ft, al, ar], up)  # noqa: E731
+    got = grads()
+    wide = torch.float64 if dtype == torch.float32 else None
+    leaves = [(t.detach() if wide is None else t.detach().to(wide)).requires_grad_(True) for t in (ft, al, ar)]
+    ref = _separate(rel, num_dst, fanout, *leaves, torch.zeros((), device=DEV, dtype=leaves[0].dtype), 0.2)
+    want = torch.autograd.grad(ref, leaves, up.to(ref.dtype))
+    # As in test_gat_layer; a source's gradient is a sum of up to 140 k terms of its own magnitude: to the sum's norm.
+    for a, b, name in zip(got, want, ("ft", "attn_l", "attn_r")):
+        tol = 2e-5 if dtype == torch.float32 else 5e-2 if name.startswith("attn") else 1e-2
+        a, b = a.double().reshape(-1), b.double().reshape(-1)
+        assert bool((a - b).norm() <= tol * b.norm()), (name, ((a - b).norm() / b.norm()).item())
+    for a, b in zip(got, grads()):
+        assert torch.equal(a, b)
