@@ -365,8 +365,6 @@ __global__ __launch_bounds__(kAggBlock) void gat_source_kernel(GatSourceParams p
     }
     __syncthreads();
   };
-  uint32_t lengthy = 0;   // asked for now, looked at in the end
-  for (int s = threadIdx.x; s < p.lng.slots; s += kAggBlock) lengthy |= p.lng.row[s];
   const int64_t row_groups = static_cast<int64_t>(gridDim.x) * kGroups;
   for (int64_t c0 = 0; c0 < row_len; c0 += LPR * VEC) {
     const Cols col = columns(c0);
@@ -424,7 +422,7 @@ __global__ __launch_bounds__(kAggBlock) void gat_source_kernel(GatSourceParams p
       if (grp == 0) finish(r, col, acc);
     }
   }
-  if (p.lng.slots == 0 || !__syncthreads_or(lengthy != 0)) return;
+  if (p.lng.slots == 0) return;
   LongChunks<kAggBlock, I> chunks(p.lng, indptr);
   chunks.number(s_wave);
   const int64_t width = row_len + p.heads;

@@ -105,3 +105,39 @@ def test_minibatch_kernels_do_not_spill(tmp_path):
     assert any("mb_place_kernel" in n for n in res) and any("mb_count_kernel" in n for n in res)
     for name, k in res.items():
         assert k["ScratchSize"] == 0 and k["VGPRs Spill"] == 0, (name, k)
+
+
+# Waves per SIMD of the layers' and block formats' kernels in the shapes that a training step takes (512 VGPRs per SIMD
+# lane): the fewest that each was measured with.
+LAYER_BUDGETS = {
+    "block.hip": {"void apt::range_count_kernel<false, 8>(": 8, "apt::range_scan_kernel(": 8, "void apt::range_place_kernel<false, 8>(": 8,
+                  "void apt::range_place_kernel<true, 4>(": 8, "void apt::range_place_kernel<true, 8>(": 6,
+                  "void apt::range_sort_kernel<false>(": 7, "void apt::range_sort_kernel<true>(": 7},
+    # fp32 rows of 256, bf16 rows of 256, from slots and from a CSR
+    "block_grad.hip": {"void apt::source_sum_kernel<float, 4, 64, unsigned int, false, false>(": 8,
+                       "void apt::source_sum_kernel<float, 4, 64, long, false, false>(": 8,
+                       "void apt::source_sum_kernel<unsigned short, 8, 32, unsigned int, false, false>(": 5,
+                       "void apt::source_sum_kernel<unsigned short, 8, 32, long, false, false>(": 5},
+    # 4 heads of 64
+    "gat_layer.hip": {"void apt::gat_source_kernel<unsigned short, 8, 32, unsigned int, false>(": 3,
+                      "void apt::gat_source_kernel<unsigned short, 8, 32, long, false>(": 3,
+                      "void apt::gat_source_kernel<float, 4, 64, unsigned int, false>(": 3,
+                      "void apt::gat_pair_scores_kernel<unsigned short, 8, 8, 32>(": 6,
+                      "void apt::gat_pair_scores_kernel<float, 4, 16, 64>(": 8,
+                      "void apt::gat_param_grad_kernel<unsigned short, 8>(": 2, "void apt::gat_param_grad_kernel<float, 4>(": 3},
+    "linear.hip": {"void apt::wgrad_kernel<float, 4, 4>(": 2, "void apt::wgrad_kernel<unsigned short, 4, 4>(": 2},
+    "rows_gemm.hip": {"void apt::rows_gemm_kernel<4, 4, 4>(": 2, "void apt::rows_gemm_kernel<4, 1, 4>(": 3,
+                      "void apt::rows_gemm_kernel<1, 2, 4>(": 2, "void apt::add_rows_kernel<float, 4>(": 8},
+    "spmm.hip": {"void apt::spmm_ell_kernel<float, float, 4, 64>(": 8, "void apt::spmm_ell_kernel<unsigned short, unsigned short, 8, 32>(": 8,
+                 "void apt::gat_ell_wave_kernel<float, float, 4>(": 8, "void apt::gat_bwd_edge_wave_kernel<unsigned short, unsigned short, 4>(": 8},
+}
+
+
+@pytest.mark.parametrize("source", sorted(LAYER_BUDGETS))
+def test_layer_kernels_keep_their_occupancy_and_do_not_spill(source, tmp_path):
+    res = _resources(source, tmp_path)
+    for name, waves in LAYER_BUDGETS[source].items():
+        assert _one(res, name)["Occupancy"] >= waves, (name, _one(res, name))
+    for name, k in res.items():
+        assert k["ScratchSize"] == 0 and k["VGPRs Spill"] == 0, (name, k)
+        assert k["LDS Size"] <= 64 * 1024, (name, k)
