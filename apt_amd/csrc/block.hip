@@ -481,7 +481,8 @@ constexpr int64_t kRangeMaxTiles = 4096;
 // A tile of the partition: 1024 slots (four per thread) instead of 2048 while the edges are few and workgroups with them.
 // Every tile walks all ranges, so a large block is better off with half the tiles.  CSR of 8 k / 260 k / 730 k / 950 k /
 // 3.4 M edges with 2048 and 1024: 51 / 47, 114 / 108, 183 / 191, 198 / 210, 476 / 542 us (host reads included).
-// A row count in device memory is a third of its bound or less.
+// A row count in device memory is usually a fraction of its bound (a batch of the 111 M-node graph: 1.07 M edges for bounds
+// of 4.3 M slots), so the bound may be four times that; a block that fills it pays the 6 to 8 % above.
 constexpr int64_t kRangeSmallSlots = int64_t{1} << 19, kRangeSmallBound = int64_t{1} << 21;
 constexpr int kRangeSmallIters = 4;
 constexpr int kRangeKeyBits = kRangeMaxShift;

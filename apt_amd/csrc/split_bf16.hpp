@@ -1,6 +1,8 @@
 // fp32 values as sums of three bf16 (8 bits each, rounded to nearest): the products of the parts on the bf16 matrix units
-// stand for an fp32 product.  Six of the nine are formed; those left out are below 2^-25 of the product.  An infinity, or
-// a value that rounds to one in bf16, has parts that are NaN: a result that is not finite is formed again in fp32.
+// stand for an fp32 product.  Six of the nine are formed; those left out are below 2^-25 of the product.  (The low parts of
+// a value below 2^-110 are subnormal bf16 or zero: such a value counts with fewer bits, down to the eight of its high part.)
+// An infinity, or a value that rounds to one in bf16, has parts that are NaN: a result that is not finite is formed
+// again in fp32.
 #pragma once
 
 #include "common.hpp"

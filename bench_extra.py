@@ -60,7 +60,8 @@ def graph_replay_us(torch, fn, reps=10, replays=5):
 def stage_aggregation(capi, dev, synth, torch, pipe, seeds, rng_seed, data_seed=1):
     """The aggregation stage on the outermost block of one batch: GraphSAGE mean SpMM
     (hidden 256, fp32 and bf16 rows, fp32 accumulation) and a GAT layer of 4 heads x 64 (logits, then fused
-    LeakyReLU + edge softmax + weighted sum), each with the bytes it has to move and its duration."""
+    LeakyReLU + edge softmax + weighted sum), each with the bytes it has to move and its duration; the backward passes
+    as the layers of apt_amd.layers run them (the edges ordered by source included), and the COO operators."""
     pipe.run(seeds, rng_seed)
     res = pipe.result()
     blk = res["blocks"][0]
@@ -74,7 +75,7 @@ def stage_aggregation(capi, dev, synth, torch, pipe, seeds, rng_seed, data_seed=
            "bytes": "SpMM mean: E x hidden x s read + num_dst x hidden x 4 written + 8 x num_dst x fanout of ids"}
     for name, dt, es in (("fp32", torch.float32, 4), ("bf16", torch.bfloat16, 2)):
         h = synth.random_features(n_src, hid, dt, data_seed + 7, dev)
-        fn = lambda: capi.spmm_sum(0, row_e, col_e, h, n_dst)
+        fn = lambda: capi.spmm_sum(0, row_e, col_e, h, n_dst)   # the edge-parallel C entry
         t = seconds_per_call(torch, fn)
         nbytes = E * hid * es + 2 * n_dst * hid * 4 + 16 * E   # rows read, zero-fill + sums written, ids
         agg[f"spmm_copy_u_sum_{name}_us"] = t * 1e6
@@ -86,6 +87,16 @@ def stage_aggregation(capi, dev, synth, torch, pipe, seeds, rng_seed, data_seed=
         agg[f"spmm_block_mean_{name}_us"] = t * 1e6
         agg[f"spmm_block_mean_{name}_bytes"] = nbytes
         agg[f"spmm_block_mean_{name}_GBps"] = nbytes / t / 1e9
+        # the operator (edges grouped by destination already, two host reads), and the gradient of the mean
+        i64 = dict(dtype=torch.int64, device=dev)
+        coo, zero, dst_off = torch.tensor([0, E], **i64), torch.zeros(1, **i64), torch.tensor([0, n_dst], **i64)
+        agg[f"npc_spmm_copy_u_sum_{name}_us"] = seconds_per_call(
+            torch, lambda: torch.ops.npc.spmm_copy_u_sum(row_e, col_e, h, coo, zero, dst_off)) * 1e6
+        x = h.requires_grad_(True)
+        out, d_out = torch.ops.npc.block_aggregate(rel, n_dst, f, x, True, None, None), torch.randn(n_dst, hid, device=dev).to(dt)
+        agg[f"block_aggregate_backward_{name}_us"] = seconds_per_call(
+            torch, lambda: torch.autograd.grad(out, x, d_out, retain_graph=True)) * 1e6
+        del h, x, out, d_out
     # GAT layer of the same block: 4 heads x 64, logits then fused LeakyReLU + edge softmax + weighted sum
     heads, hdim = 4, 64
     for name, dt, es in (("fp32", torch.float32, 4), ("bf16", torch.bfloat16, 2)):
@@ -101,29 +112,14 @@ def stage_aggregation(capi, dev, synth, torch, pipe, seeds, rng_seed, data_seed=
             agg[f"{tag}_{name}_us"] = t * 1e6
             agg[f"{tag}_{name}_bytes"] = nbytes
             agg[f"{tag}_{name}_GBps"] = nbytes / t / 1e9
-        # backward of the aggregation: logit gradients per (destination, head), then the sums over the
-        # edges of a source on the block's CSR order
-        fmt_b = capi.block_formats(rel, n_dst, f, n_src)
-        _, attn_w = capi.gat_block(rel, n_dst, f, ft, el, er, 0.2, want_attn=True)
-        d_out = torch.randn(n_dst, heads, hdim, device=dev)
-        csr_ip = fmt_b["csr_indptr"][:n_src + 1].contiguous()
-        src_csr = fmt_b["coo_row"][fmt_b["csr_eids"]].contiguous()
-        d2 = d_out.view(n_dst, heads * hdim)
-
-        def gat_bwd():
-            a_e, dz_e, d_er = capi.gat_block_backward(rel, n_dst, f, ft, el, er, 0.2, attn_w, d_out,
-                                                      fmt_b["csc_indptr"], fmt_b["num_edges"])
-            capi.spmm_heads(fmt_b["csr_indices"], src_csr, d_out, a_e, n_src, weight_row=fmt_b["csr_eids"],
-                            grouped=True, head_weights2=dz_e, out_indptr=csr_ip)
-
-        # backward of the plain sum / mean (SAGE, GCN): the same sum over the CSR order, no weights
-        for tag, fn in (("gat_block_backward", gat_bwd),
-                        ("spmm_block_backward", lambda: capi.spmm_heads(
-                            fmt_b["csr_indices"], src_csr, d2, None, n_src, grouped=True, out_indptr=csr_ip))):
-            if tag.startswith("spmm_block_backward") and name != "fp32":
-                continue
-            agg[f"{tag}_{name}_us"] = seconds_per_call(torch, fn) * 1e6
-        del ft, el, er, fmt_b, attn_w, d_out
+        # the layer from the dense product on (scores, softmax, sum), and all its gradients
+        leaves = [t.detach().to(dt).requires_grad_(True) for t in (ft, al, ar)]
+        layer = lambda: torch.ops.npc.gat_layer(rel, n_dst, f, *leaves, None, 0.2, None, None, None, None)
+        agg[f"gat_layer_{name}_us"] = seconds_per_call(torch, layer) * 1e6
+        out, d_out = layer(), torch.randn(n_dst, heads, hdim, device=dev).to(dt)
+        agg[f"gat_layer_backward_{name}_us"] = seconds_per_call(
+            torch, lambda: torch.autograd.grad(out, leaves, d_out, retain_graph=True)) * 1e6
+        del ft, el, er, leaves, out, d_out
     hd = synth.random_features(n_dst, hid, torch.float32, data_seed + 8, dev)
     h = synth.random_features(n_src, hid, torch.float32, data_seed + 7, dev)
     fn = lambda: capi.sddmm(0, row_e, col_e, h, hd)
