@@ -68,6 +68,11 @@ class CEpochDesc(C.Structure):       # apt_epoch_desc
                 ("slots", CBatchSlot * MAX_SLOTS)]
 
 
+class CWgradProduct(C.Structure):    # apt_wgrad_product
+    _fields_ = [("dy", C.c_void_p), ("out", C.c_void_p), ("x", C.c_void_p), ("m", C.c_int64), ("n", C.c_int64),
+                ("k", C.c_int64), ("dw", C.c_void_p), ("db", C.c_void_p)]
+
+
 class CEpochCost(C.Structure):       # apt_epoch_cost
     _fields_ = [("batches", C.c_int64), ("enqueue_seconds", C.c_double), ("wait_enqueue_seconds", C.c_double),
                 ("wait_gpu_seconds", C.c_double), ("release_seconds", C.c_double)]
@@ -145,6 +150,8 @@ SYMBOLS = {
     "apt_rows_gemm": (_I, [_P, _I64, _P, _I64, _I64, _P, _I64, _P, _I64, _I64, _I64, _I64, _I64, _P, _I, _I, _P, _P, _SZ, _P]),
     "apt_linear_wgrad_workspace_bytes": (_SZ, [_I64, _I64, _I64, _I]),
     "apt_linear_wgrad": (_I, [_P, _P, _I64, _I64, _I64, _I, _P, _P, _P, _SZ, _P]),
+    "apt_linear_wgrads_workspace_bytes": (_SZ, [C.POINTER(CWgradProduct), _I, _I]),
+    "apt_linear_wgrads": (_I, [C.POINTER(CWgradProduct), _I, _I, _P, _SZ, _P]),
     "apt_time_next_sample": (_I, [_I, _P, _P]),
     "apt_epoch_create": (_I, [C.POINTER(CEpochDesc), C.POINTER(_P)]),
     "apt_epoch_begin": (_I, [_P, _P, _I64, _U64, _P]),
@@ -1062,6 +1069,26 @@ def linear_wgrad(dy, x, want_bias=True):
     check(lib().apt_linear_wgrad(_ptr(dy), _ptr(x), m, n, k, x.element_size(), _ptr(dw), _ptr(db), _ptr(ws), ws.numel(),
                                  _stream()))
     return dw, db
+
+
+def linear_wgrads(products):
+    """Weight and bias gradients of one or two products (dy, x or None, the ReLU's result or None, want_bias) in one launch
+    -> [(dw or None, db or None), ...]; dy counts where the ReLU's result is positive, x None: db alone."""
+    arr, out = (CWgradProduct * len(products))(), []
+    es = products[0][0].element_size()
+    for q, (dy, x, relu_out, want_bias) in zip(arr, products):
+        dy = _feat2d(dy, "dy")
+        if any(t is not None and (t.dtype != products[0][0].dtype or t.shape[0] != dy.shape[0] or not t.is_contiguous())
+               for t in (dy, x, relu_out)) or (relu_out is not None and relu_out.shape != dy.shape):
+            raise AptError("linear_wgrads: tensors do not fit each other")
+        n, k = dy.shape[1], 0 if x is None else x.shape[1]
+        dw = None if x is None else torch.empty((n, k), dtype=dy.dtype, device=dy.device)
+        db = torch.empty(n, dtype=dy.dtype, device=dy.device) if want_bias else None
+        q.dy, q.out, q.x, q.m, q.n, q.k, q.dw, q.db = _ptr(dy), _ptr(relu_out), _ptr(x), dy.shape[0], n, k, _ptr(dw), _ptr(db)
+        out.append((dw, db))
+    ws = torch.empty(max(int(lib().apt_linear_wgrads_workspace_bytes(arr, len(arr), es)), 16), dtype=torch.uint8, device=dy.device)
+    check(lib().apt_linear_wgrads(arr, len(arr), es, _ptr(ws), ws.numel(), _stream()))
+    return out
 
 
 def rows_gemm(x1, w1, x2=None, w2=None, bias=None, out=None, relu=False):

@@ -1,26 +1,22 @@
-// Gradients of a dense layer's weight and bias over the rows of a block:
+// Gradients of dense layers' weights and biases over the rows of a block:
 //   dw[n, k] = sum_m dy[m, n] * x[m, k],   db[n] = sum_m dy[m, n]
+// for one or two such products in one launch (a GraphSAGE layer has two, a GCN layer one and the column sums of
+// another matrix); dy may still need the mask of the ReLU that it passed.
 //
-// A block has 10^4..10^6 rows and a layer a few hundred columns, so this product
-// reduces over the one long dimension and its output is a few tiles: bound by
-// reading dy and x once (bf16) or by the fp32 matrix rate.  A GEMM that gives
-// every output tile to one workgroup keeps a handful of the 256 CUs busy; here
-// the rows are split over the chip, every workgroup accumulates the whole output
-// of its rows in MFMA accumulators and leaves it in a partial buffer, and a second
-// launch adds the partials in a fixed order (reproducible, no atomics).
+// A block has 10^4..10^6 rows and a layer a few hundred columns, so a product reduces over the one long dimension
+// and its output is a few tiles.  The rows are split over the chip, a workgroup accumulates one output tile of its
+// rows in MFMA accumulators and leaves it in a partial buffer, and a second launch adds the partials in a fixed
+// order (reproducible, no atomics).
 //
-// fp32 operands are multiplied as bf16 parts (split_bf16.hpp): the fp32 matrix
-// instruction would bound the product (57 us of its rate alone for 71 k rows of
-// 256 x 100 in tiles of 64; the four 256-wide gradients of a GraphSAGE step of
-// 4096 seeds took 169 us with it and take 132).
-// Both operands have the reduced dimension as their row index, which is what an
-// MFMA operand wants *inside* a lane (8 consecutive rows of one column).  No LDS transpose: a lane loads VEC consecutive columns of each
-// of its rows and the 16-bit halves are regrouped by column in registers
-// (v_perm); the columns of the MFMA tiles are simply numbered lane * VEC + j.
+// fp32 operands are multiplied as bf16 parts (split_bf16.hpp): the fp32 matrix instruction would bound the product.
+// Splitting costs as many cycles of the vector units as its six products cost the matrix units, so a step's rows
+// are split once, into LDS, and read from there by all wavefronts that need them.  Both operands have the reduced
+// dimension as their row index, which is what an MFMA operand wants *inside* a lane (8 consecutive rows of one
+// column): a thread loads 8 rows of a few columns and regroups them by column on the way into LDS.
 #include <algorithm>
 
 #include "common.hpp"
-#include "partial_sums.hpp"
+#include "feature_rows.hpp"
 #include "split_bf16.hpp"
 
 namespace apt {
@@ -38,368 +34,559 @@ __device__ __forceinline__ buffer_t make_buffer(const void* base, int64_t bytes)
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, static_cast<uint32_t>(bytes), 0x00020000);
 }
 
-constexpr int kWgradTile = 64;      // output columns of dy / of x per wavefront
-constexpr int kWgradFrags = kWgradTile / 16;
-constexpr int kWgradWaves = 8;
-constexpr int kWgradGroups = 256;                     // workgroups aimed at: one per CU
-constexpr int64_t kWgradMinRows = 64;                 // rows a split has at least
-constexpr int64_t kWgradPartBytes = int64_t{12} << 20;
+constexpr int kWgradWaves = 4;      // that multiply, two by two; as many more prepare their operands
+constexpr int kWgradHalf = kWgradWaves * kWave;
+constexpr int kWgradBlock = 2 * kWgradHalf;
+constexpr int kWgradGroups = 256;   // workgroups aimed at: one per CU ...
+constexpr int kWgradSmallGroups = 512;   // ... or, of small tiles, two while each has kWgradSmallSteps of its loop
+constexpr int kWgradSmallSteps = 16;
+constexpr int kWgradJobs = 2;
+constexpr int64_t kWgradPartBytes = int64_t{16} << 20;
+
+struct WgradJob {
+  const void* dy;      // [m, n]
+  const void* out;     // [m, n] or NULL: dy counts where out > 0
+  const void* x;       // [m, k]; k == 0: the column sums alone
+  int64_t m, n, k;
+  float* part;         // [splits][stride]: dw, then db
+  int64_t stride;
+  int tiles_k, tiles;  // output tiles: tiles_n * tiles_k
+  int splits;
+  void *dw, *db;
+};
 
 struct WgradParams {
-  const void* dy;      // [m, n]
-  const void* x;       // [m, k]
-  int64_t m, n, k;
-  float* part;         // [splits][n * k + n]
-  int64_t part_stride;
-  int tiles_k, tiles;  // wavefront tiles of the output (tiles_n * tiles_k)
-  int tile_groups;     // workgroups per split: ceil(tiles / waves)
-  int splits_per_group;  // splits in a workgroup where tile_groups == 1
-  int splits;
+  WgradJob job[kWgradJobs];
+  int jobs, tiles;          // of all jobs
   int64_t rows_per_split;
 };
 
-constexpr int kWgradRows = 32;     // rows per step: one MFMA of depth 32 (fp32: six, of its bf16 parts)
-constexpr int kWgradLoads = 8;     // consecutive rows of a lane in a step; the lanes of a 16-lane group share them
+// Rows of a step and how a thread reads them: a unit is 8 rows (one lane's share of an MFMA operand) of kCols columns.
+// WgradOdd: bf16 rows of an odd length or address, whose elements are read one by one.
+// WgradRelu: products may have a mask.
+struct WgradOdd {};
+template <typename T> struct WgradRelu {};
+template <typename T> struct WgradType;
+template <> struct WgradType<float> {
+  using Elem = float;
+  static constexpr int kRows = 32, kCols = 2, kWords = 2, kParts = 3;
+  static constexpr bool kMask = false;
+};
+template <> struct WgradType<uint16_t> {
+  using Elem = uint16_t;
+  static constexpr int kRows = 64, kCols = 4, kWords = 2, kParts = 1;
+  static constexpr bool kMask = false;
+};
+template <> struct WgradType<WgradOdd> : WgradType<uint16_t> {
+  static constexpr int kWords = 4;
+};
+template <typename T> struct WgradType<WgradRelu<T>> : WgradType<T> {
+  static constexpr bool kMask = true;
+};
+constexpr int kUnitRows = 8;
+constexpr int kWgradAhead = 2;   // steps whose rows are on their way
+// Where column c of a fragment stands in LDS, and the reverse: a thread's columns are apart from each other, those of its
+// neighbours together, so that a store of a wavefront meets every bank alike.  The lanes of an operand have the columns in
+// this order.
+template <typename T> __host__ __device__ constexpr int wgrad_place(int c) {
+  return c % WgradType<T>::kCols * (16 / WgradType<T>::kCols) + c / WgradType<T>::kCols;
+}
+template <typename T> __host__ __device__ constexpr int wgrad_col(int place) {
+  return place % (16 / WgradType<T>::kCols) * WgradType<T>::kCols + place / (16 / WgradType<T>::kCols);
+}
+// A workgroup's output tile, 2 FN x 2 FK fragments, and its LDS: a step's operands twice, and the column sums.
+template <typename T, int FN, int FK> struct WgradTile {
+  static constexpr int kTileN = 2 * FN * 16, kTileK = 2 * FK * 16;
+  static constexpr int kGroups = WgradType<T>::kRows / kUnitRows;
+  static constexpr int kBuffer = WgradType<T>::kParts * WgradType<T>::kRows * (kTileN + kTileK) * 2;
+  static constexpr int kLds = 2 * kBuffer + kGroups * kTileN * 4;
+};
 
-// The lane's rows of one operand as they come from memory: VEC consecutive columns of each row (VEC 4), two pairs
-// (VEC 2) or kWgradFrags single columns (VEC 1), at the byte offsets off[].  What an MFMA wants is taken out of it
-// only when it is used: regrouping at the load would wait for it.
-template <typename T, int VEC> struct WgradRows {
-  static constexpr int kWords = sizeof(T) == 4 || VEC == 1 ? kWgradFrags : 2;   // 32-bit registers per row
-  static constexpr int kOffsets = kWgradFrags / VEC;
-  uint32_t v[kWgradLoads][kWords];
-  __device__ __forceinline__ void load(buffer_t buf, uint32_t at, uint32_t row_bytes, const uint32_t (&off)[kOffsets]) {
+template <typename T> struct WgradUnit {
+  using Type = WgradType<T>;
+  uint32_t v[kUnitRows][Type::kWords];
+  // (no choice between kinds of loads here: registers that two branches load are moved, and waited for, behind them.
+  // Every dword of a load has a range check of its own.)
+  __device__ __forceinline__ void load(buffer_t buf, uint32_t at, uint32_t row_bytes) {
 #pragma unroll
-    for (int r = 0; r < kWgradLoads; ++r, at += row_bytes) {
-      if constexpr (VEC * sizeof(T) == 16) {
-        const u32x4_v w = __builtin_amdgcn_raw_buffer_load_b128(buf, off[0] + at, 0, 0);
-#pragma unroll
-        for (int c = 0; c < 4; ++c) v[r][c] = w[c];
-      } else if constexpr (VEC * sizeof(T) == 8) {
-#pragma unroll
-        for (int o = 0; o < kOffsets; ++o) {
-          const u32x2_v w = __builtin_amdgcn_raw_buffer_load_b64(buf, off[o] + at, 0, 0);
-          v[r][2 * o] = w[0];
-          v[r][2 * o + 1] = w[1];
-        }
+    for (int r = 0; r < kUnitRows; ++r, at += row_bytes) {
+      if constexpr (Type::kWords == 2) {
+        const u32x2_v w = __builtin_amdgcn_raw_buffer_load_b64(buf, at, 0, 0);
+        v[r][0] = w[0];
+        v[r][1] = w[1];
       } else {
 #pragma unroll
-        for (int o = 0; o < kOffsets; ++o) {
-          if constexpr (VEC * sizeof(T) == 4) v[r][o] = __builtin_amdgcn_raw_buffer_load_b32(buf, off[o] + at, 0, 0);
-          else v[r][o] = __builtin_amdgcn_raw_buffer_load_b16(buf, off[o] + at, 0, 0);
+        for (int c = 0; c < Type::kWords; ++c) v[r][c] = __builtin_amdgcn_raw_buffer_load_b16(buf, at + 2 * c, 0, 0);
+      }
+    }
+  }
+  // Single elements -> pairs of columns, as the wide loads leave them.
+  __device__ __forceinline__ void pack() {
+    if constexpr (Type::kWords == 4) {
+#pragma unroll
+      for (int r = 0; r < kUnitRows; ++r) {
+        v[r][0] |= v[r][1] << 16;
+        v[r][1] = v[r][2] | v[r][3] << 16;
+      }
+    }
+  }
+  // Zero where the ReLU's result is (as torch has it: a NaN passes).
+  __device__ __forceinline__ void mask(const WgradUnit& out) {
+#pragma unroll
+    for (int r = 0; r < kUnitRows; ++r)
+#pragma unroll
+      for (int w = 0; w < 2; ++w) {
+        if constexpr (Type::kParts == 3) {
+          v[r][w] = __uint_as_float(out.v[r][w]) <= 0.f ? 0u : v[r][w];
+        } else {
+          const uint32_t lo = __uint_as_float(out.v[r][w] << 16) <= 0.f ? 0u : 0xffffu;
+          const uint32_t hi = __uint_as_float(out.v[r][w] & 0xffff0000u) <= 0.f ? 0u : 0xffff0000u;
+          v[r][w] &= lo | hi;
+        }
+      }
+  }
+  __device__ __forceinline__ void add_to(float (&sum)[Type::kCols]) const {
+#pragma unroll
+    for (int c = 0; c < Type::kCols; ++c) {
+      float even = 0.f, odd = 0.f;
+#pragma unroll
+      for (int r = 0; r < kUnitRows; r += 2) {
+        if constexpr (Type::kParts == 3) {
+          even += __uint_as_float(v[r][c]);
+          odd += __uint_as_float(v[r + 1][c]);
+        } else {
+          even += __uint_as_float((c & 1) != 0 ? v[r][c / 2] & 0xffff0000u : v[r][c / 2] << 16);
+          odd += __uint_as_float((c & 1) != 0 ? v[r + 1][c / 2] & 0xffff0000u : v[r + 1][c / 2] << 16);
+        }
+      }
+      sum[c] += even + odd;
+    }
+  }
+  // Column c of the unit as MFMA operand: eight bf16 (per part), two rows to a register.
+  __device__ __forceinline__ void column(int c, u32x4_v (&o)[Type::kParts]) const {
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+      if constexpr (Type::kParts == 3) {
+        const SplitPair s = split_pair(__uint_as_float(v[2 * d][c]), __uint_as_float(v[2 * d + 1][c]));
+        o[0][d] = s.hi;
+        o[1][d] = s.mid;
+        o[2][d] = s.lo;
+      } else {
+        o[0][d] = __builtin_amdgcn_perm(v[2 * d + 1][c / 2], v[2 * d][c / 2], (c & 1) != 0 ? 0x07060302u : 0x05040100u);
+      }
+    }
+  }
+};
+
+__device__ __forceinline__ f32x4_t wgrad_mfma(u32x4_v a, u32x4_v b, f32x4_t acc) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), acc, 0, 0, 0);
+}
+
+// FN x FK fragments (of 16 x 16 outputs) per wavefront.  Four wavefronts read the rows, split them and leave them in LDS
+// (producers), the other four multiply what the step before left there (consumers): with one of either on a SIMD the
+// vector units and the matrix units work at the same time.
+template <typename T, int FN, int FK>
+__global__ __launch_bounds__(kWgradBlock) void wgrad_kernel(WgradParams p) {
+  using Type = WgradType<T>;
+  using Elem = typename Type::Elem;
+  using Tile = WgradTile<T, FN, FK>;
+  constexpr int kRows = Type::kRows, kCols = Type::kCols, kParts = Type::kParts;
+  constexpr int kGroups = Tile::kGroups, kSubs = kRows / 32;
+  constexpr int kTileN = Tile::kTileN, kTileK = Tile::kTileK;
+  static_assert(FN == FK, "as many units of dy as of x");
+  constexpr int kOperandUnits = kTileN / kCols * kGroups;         // of dy, and of x
+  constexpr int kUnits = 2 * kOperandUnits / kWgradHalf;          // of a producer: 2 = one of either, 1 = of dy or of x
+  static_assert(kUnits == 1 || kUnits == 2);
+  constexpr int kFrags = 2 * FN + 2 * FK;                         // of the tile's operands: dy's, then x's
+  constexpr int kFlip = kCols == 4 ? 4 : 0;                       // four lanes to a fragment: its neighbour the other way round
+  static_assert(kWgradAhead % 2 == 0 && FN % 2 == 0);
+  extern __shared__ __align__(16) char s_wgrad[];
+  u32x4_v* s_part = reinterpret_cast<u32x4_v*>(s_wgrad);          // [buffer][part][sub][fragment][lane]
+  float(*s_sum)[kTileN] = reinterpret_cast<float(*)[kTileN]>(s_wgrad + 2 * Tile::kBuffer);
+  constexpr int kBufferVecs = Tile::kBuffer / 16, kPartVecs = kBufferVecs / kParts;
+  const int lane = threadIdx.x % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int group = lane / 16, col16 = wgrad_col<T>(lane % 16);
+  // The workgroups of a split read the same rows: they are numbered eight apart, i.e. on one XCD, whose L2 then serves
+  // the others.
+  const int i = blockIdx.x / 8;
+  const int split = __builtin_amdgcn_readfirstlane((i / p.tiles) * 8 + blockIdx.x % 8);   // (a division leaves them in
+  int tile = __builtin_amdgcn_readfirstlane(i % p.tiles);                                  // vector registers)
+  const int which = p.jobs > 1 && tile >= p.job[0].tiles ? 1 : 0;
+  const WgradJob& job = p.job[which];
+  if (which == 1) tile -= p.job[0].tiles;
+  if (split >= job.splits) return;   // block-uniform
+  const int tile_n = __builtin_amdgcn_readfirstlane(tile / job.tiles_k), tile_k = tile - tile_n * job.tiles_k;
+  const int64_t n0 = static_cast<int64_t>(tile_n) * kTileN, k0 = static_cast<int64_t>(tile_k) * kTileK;
+  const int64_t m0 = static_cast<int64_t>(split) * p.rows_per_split;
+  const int64_t m1 = min(m0 + p.rows_per_split, job.m);
+  const bool bias = job.db != nullptr && tile_k == 0;
+  const bool masked = job.out != nullptr;
+  const buffer_t dy = make_buffer(static_cast<const Elem*>(job.dy) + m0 * job.n, (m1 - m0) * job.n * sizeof(Elem));
+  const buffer_t out = make_buffer(static_cast<const Elem*>(masked ? job.out : job.dy) + m0 * job.n, (m1 - m0) * job.n * sizeof(Elem));
+  const buffer_t x = make_buffer(static_cast<const Elem*>(job.x) + m0 * job.k, (m1 - m0) * job.k * sizeof(Elem));
+  // (whole turns of the producers' loop; a step past the end reads zeros)
+  const int steps = static_cast<int>((m1 - m0 + kWgradAhead * kRows - 1) / (kWgradAhead * kRows)) * kWgradAhead;
+
+  const int wn = (wave & 3) / 2, wk = wave % 2;
+  const int64_t wave_n = n0 + wn * FN * 16, wave_k = k0 + wk * FK * 16;
+  const bool active = wave < kWgradWaves && wave_n < job.n && wave_k < job.k;   // wave-uniform
+  f32x4_t acc[FN][FK] = {};
+  if (wave >= kWgradWaves) {
+    // A thread's units: columns kCols * (u % units per row), rows 8 * (u / units per row) of a step.  Columns past the
+    // edge read the row after (or zero): they only reach outputs past the edge, which are not stored.
+    const int u = (threadIdx.x - kWgradHalf) % kOperandUnits;
+    const int col = u % (kTileN / kCols) * kCols, rg = u / (kTileN / kCols);
+    const bool has_dy = kUnits == 2 || wave - kWgradWaves < kOperandUnits / kWave;   // wave-uniform; otherwise x alone
+    const uint32_t row_a = static_cast<uint32_t>(job.n * sizeof(Elem)), row_b = static_cast<uint32_t>(job.k * sizeof(Elem));
+    const uint32_t at_a = static_cast<uint32_t>((rg * kUnitRows * job.n + n0 + col) * sizeof(Elem));
+    const uint32_t at_b = static_cast<uint32_t>((rg * kUnitRows * job.k + k0 + col) * sizeof(Elem));
+    const bool sum_here = bias && has_dy;
+    struct Source {
+      buffer_t buffer;
+      uint32_t row, at;
+      int frag0;
+    } source[kUnits];
+    source[0] = has_dy ? Source{dy, row_a, at_a, 0} : Source{x, row_b, at_b, 2 * FN};
+    if constexpr (kUnits == 2) source[1] = Source{x, row_b, at_b, 2 * FN};
+    WgradUnit<T> unit[kWgradAhead][kUnits], relu[kWgradAhead];
+    auto load = [&](int q) {
+      if constexpr (Type::kMask) relu[q].load(has_dy ? out : x, source[0].at, source[0].row);
+#pragma unroll
+      for (int i = 0; i < kUnits; ++i) {
+        unit[q][i].load(source[i].buffer, source[i].at, source[i].row);
+        source[i].at += kRows * source[i].row;
+      }
+      __builtin_amdgcn_sched_barrier(0);   // (in this order: the first step's are waited for alone)
+    };
+    float sum[kCols] = {};
+#pragma unroll
+    for (int q = 0; q < kWgradAhead; ++q) load(q);
+    for (int s = 0; s < steps; s += kWgradAhead) {
+#pragma unroll
+      for (int q = 0; q < kWgradAhead; ++q) {
+#pragma unroll
+        for (int i = 0; i < kUnits; ++i) {
+          WgradUnit<T> now = unit[q][i];
+          now.pack();
+          if constexpr (Type::kMask) {
+            if (i == 0 && masked && has_dy) {
+              WgradUnit<T> result = relu[q];
+              result.pack();
+              now.mask(result);
+            }
+          }
+          if (i == 0 && sum_here) now.add_to(sum);
+#pragma unroll
+          for (int c = 0; c < kCols; ++c) {
+            u32x4_v o[kParts];
+            now.column(c, o);
+            const int frag = source[i].frag0 + col / 16;
+            const int at = (q & 1) * kBufferVecs + ((rg / 4 * kFrags + frag) * 4 + rg % 4) * 16 + (wgrad_place<T>(col % 16 + c) ^ (frag & 1) * kFlip);
+#pragma unroll
+            for (int d = 0; d < kParts; ++d) s_part[d * kPartVecs + at] = o[d];
+          }
+        }
+        load(q);
+        __syncthreads();   // (one per step, of the producers and of the consumers)
+      }
+    }
+    if (sum_here)
+#pragma unroll
+      for (int q = 0; q < kCols; ++q) s_sum[rg][col + q] = sum[q];
+  } else {
+    for (int s = 0; s < steps; ++s) {
+      __syncthreads();
+      if (!active) continue;
+      const u32x4_v* from[2] = {s_part + (s & 1) * kBufferVecs + lane, s_part + (s & 1) * kBufferVecs + (lane ^ kFlip)};
+#pragma unroll
+      for (int h = 0; h < kSubs; ++h) {
+        u32x4_v fa[FN][kParts];
+#pragma unroll
+        for (int f = 0; f < FN; ++f)
+#pragma unroll
+          for (int t = 0; t < kParts; ++t) fa[f][t] = from[f & 1][t * kPartVecs + (h * kFrags + wn * FN + f) * kWave];
+#pragma unroll
+        for (int g = 0; g < FK; ++g) {
+          u32x4_v fb[kParts];
+#pragma unroll
+          for (int t = 0; t < kParts; ++t) fb[t] = from[g & 1][t * kPartVecs + (h * kFrags + 2 * FN + wk * FK + g) * kWave];
+          // products of one accumulator are kept apart (a chain of them would wait for each other)
+          if constexpr (kParts == 3) {
+            // a step's are added up on their own, the small ones first: one rounding of the long sum per step
+            f32x4_t sum[FN];
+#pragma unroll
+            for (int t = 0; t < kSplitProducts; ++t)
+#pragma unroll
+              for (int f = 0; f < FN; ++f)
+                sum[f] = wgrad_mfma(fa[f][kSplitA[t]], fb[kSplitB[t]], t == 0 ? f32x4_t{0.f, 0.f, 0.f, 0.f} : sum[f]);
+#pragma unroll
+            for (int f = 0; f < FN; ++f) acc[f][g] += sum[f];
+          } else {
+#pragma unroll
+            for (int f = 0; f < FN; ++f) acc[f][g] = wgrad_mfma(fa[f][0], fb[0], acc[f][g]);
+          }
         }
       }
     }
   }
-};
-
-// Column of the output that element i (0..15) of tile fragment f stands for, relative to the tile.
-template <int VEC>
-__device__ __forceinline__ int wgrad_col(int f, int i) {
-  return VEC == 4 ? i * 4 + f : VEC == 2 ? (f / 2) * 32 + i * 2 + (f & 1) : f * 16 + i;
-}
-
-// MFMA operands of one step: fragment f = 16 columns, the lane's rows of one of them.
-template <typename T> struct WgradOperand;
-template <> struct WgradOperand<float> {
-  uint32_t v[3][kWgradFrags][4];   // the parts of eight values of a column, two rows to a register
-  template <int VEC> __device__ __forceinline__ explicit WgradOperand(const WgradRows<float, VEC>& rows) {
+  float* part = job.part + static_cast<int64_t>(split) * job.stride;
+  if (bias) {   // block-uniform
+    __syncthreads();
+    if (threadIdx.x < kTileN && n0 + threadIdx.x < job.n) {
+      float v = 0.f;
 #pragma unroll
-    for (int f = 0; f < kWgradFrags; ++f)
-#pragma unroll
-      for (int d = 0; d < 4; ++d) {
-        const SplitPair s = split_pair(__uint_as_float(rows.v[2 * d][f]), __uint_as_float(rows.v[2 * d + 1][f]));
-        v[0][f][d] = s.hi;
-        v[1][f][d] = s.mid;
-        v[2][f][d] = s.lo;
-      }
-  }
-};
-template <> struct WgradOperand<uint16_t> {
-  uint32_t v[kWgradFrags][4];   // eight bf16 of a column, two rows to a register
-  template <int VEC> __device__ __forceinline__ explicit WgradOperand(const WgradRows<uint16_t, VEC>& rows) {
-#pragma unroll
-    for (int f = 0; f < kWgradFrags; ++f)
-#pragma unroll
-      for (int d = 0; d < 4; ++d) {
-        const int w = VEC == 1 ? f : f / 2;
-        v[f][d] = __builtin_amdgcn_perm(rows.v[2 * d + 1][w], rows.v[2 * d][w],
-                                        VEC != 1 && (f & 1) != 0 ? 0x07060302u : 0x05040100u);
-      }
-  }
-};
-
-// acc[fa][fb] += a[fa]^T b[fb] over the step's rows; products of one accumulator are kept apart (a chain of them
-// would wait for each other).
-__device__ __forceinline__ f32x4_t wgrad_mfma(const uint32_t (&a)[4], const uint32_t (&b)[4], f32x4_t acc) {
-  const u32x4_v av = {a[0], a[1], a[2], a[3]}, bv = {b[0], b[1], b[2], b[3]};
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, av), __builtin_bit_cast(bf16x8_t, bv), acc,
-                                                 0, 0, 0);
-}
-__device__ __forceinline__ void wgrad_products(const WgradOperand<float>& a, const WgradOperand<float>& b,
-                                               f32x4_t (&acc)[kWgradFrags][kWgradFrags]) {
-#pragma unroll
-  for (int t = 0; t < kSplitProducts; ++t)
-#pragma unroll
-    for (int fa = 0; fa < kWgradFrags; ++fa)
-#pragma unroll
-      for (int fb = 0; fb < kWgradFrags; ++fb)
-        acc[fa][fb] = wgrad_mfma(a.v[kSplitA[t]][fa], b.v[kSplitB[t]][fb], acc[fa][fb]);
-}
-__device__ __forceinline__ void wgrad_products(const WgradOperand<uint16_t>& a, const WgradOperand<uint16_t>& b,
-                                               f32x4_t (&acc)[kWgradFrags][kWgradFrags]) {
-#pragma unroll
-  for (int fa = 0; fa < kWgradFrags; ++fa)
-#pragma unroll
-    for (int fb = 0; fb < kWgradFrags; ++fb) acc[fa][fb] = wgrad_mfma(a.v[fa], b.v[fb], acc[fa][fb]);
-}
-// Column sums of dy.  bf16: a product with ones (4 more MFMAs beside 16; unpacking the halves would cost more), the
-// sum of column i in accumulator row i.  fp32: the vector units add; the lane's sum covers its own rows of columns l16.
-template <int VEC>
-__device__ __forceinline__ void wgrad_sums(const WgradRows<uint16_t, VEC>&, const WgradOperand<uint16_t>& a,
-                                           f32x4_t (&sum)[kWgradFrags]) {
-  const uint32_t ones[4] = {0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u};
-#pragma unroll
-  for (int f = 0; f < kWgradFrags; ++f) sum[f] = wgrad_mfma(a.v[f], ones, sum[f]);
-}
-template <int VEC>
-__device__ __forceinline__ void wgrad_sums(const WgradRows<float, VEC>& rows, const WgradOperand<float>&,
-                                           f32x4_t (&sum)[kWgradFrags]) {
-#pragma unroll
-  for (int f = 0; f < kWgradFrags; ++f)
-#pragma unroll
-    for (int r = 0; r < kWgradLoads; ++r) sum[f][r & 1] += __uint_as_float(rows.v[r][f]);
-}
-
-template <typename T, int VA, int VB>
-__global__ __launch_bounds__(kWgradWaves * kWave) void wgrad_kernel(WgradParams p) {
-  constexpr int kRows = kWgradRows;
-  const int lane = threadIdx.x % kWave;
-  const int l16 = lane % 16, group = lane / 16;
-  // A wavefront has one tile of one split.  The workgroups of a split read the same rows: they are numbered eight
-  // apart, i.e. on one XCD, whose L2 then serves the second reader.
-  int split, tile;
-  const int wave = threadIdx.x / kWave;
-  if (p.tile_groups == 1) {
-    split = blockIdx.x * p.splits_per_group + wave / p.tiles;
-    tile = wave % p.tiles;
-    if (wave >= p.splits_per_group * p.tiles) return;
-  } else {
-    const int i = blockIdx.x / 8;
-    split = (i / p.tile_groups) * 8 + blockIdx.x % 8;
-    tile = (i % p.tile_groups) * kWgradWaves + wave;
-  }
-  split = __builtin_amdgcn_readfirstlane(split);
-  tile = __builtin_amdgcn_readfirstlane(tile);
-  if (split >= p.splits || tile >= p.tiles) return;   // wave-uniform, no barriers below
-  const int64_t n0 = static_cast<int64_t>(tile / p.tiles_k) * kWgradTile;
-  const int64_t k0 = static_cast<int64_t>(tile % p.tiles_k) * kWgradTile;
-  const int64_t m0 = static_cast<int64_t>(split) * p.rows_per_split;
-  const int64_t m1 = min(m0 + p.rows_per_split, p.m);
-  const buffer_t dy = make_buffer(static_cast<const T*>(p.dy) + m0 * p.n, (m1 - m0) * p.n * sizeof(T));
-  const buffer_t x = make_buffer(static_cast<const T*>(p.x) + m0 * p.k, (m1 - m0) * p.k * sizeof(T));
-  // A lane's offsets inside a step do not change.  Columns past the edge read the row after (or zero): they only
-  // reach outputs past the edge, which are not stored.
-  uint32_t off_a[kWgradFrags / VA], off_b[kWgradFrags / VB];
-#pragma unroll
-  for (int o = 0; o < kWgradFrags / VA; ++o)
-    off_a[o] = static_cast<uint32_t>((group * kWgradLoads * p.n + n0 + wgrad_col<VA>(o * VA, l16)) * sizeof(T));
-#pragma unroll
-  for (int o = 0; o < kWgradFrags / VB; ++o)
-    off_b[o] = static_cast<uint32_t>((group * kWgradLoads * p.k + k0 + wgrad_col<VB>(o * VB, l16)) * sizeof(T));
-  const uint32_t row_a = static_cast<uint32_t>(p.n * sizeof(T)), row_b = static_cast<uint32_t>(p.k * sizeof(T));
-  const uint32_t step_a = static_cast<uint32_t>(kRows * p.n * sizeof(T)), step_b = static_cast<uint32_t>(kRows * p.k * sizeof(T));
-  f32x4_t acc[kWgradFrags][kWgradFrags] = {};
-  f32x4_t sum[kWgradFrags] = {};
-  const bool bias = tile % p.tiles_k == 0;
-
-  const int steps = static_cast<int>((m1 - m0 + kRows - 1) / kRows);
-  uint32_t at_a = 0, at_b = 0;
-  WgradRows<T, VA> a0;
-  WgradRows<T, VB> b0;
-  a0.load(dy, at_a, row_a, off_a);
-  b0.load(x, at_b, row_b, off_b);
-  if constexpr (sizeof(T) == 4) {
-    // The parts take the place of the second step's rows (registers): the next rows are on their way during the products.
-    for (int s = 0; s < steps; ++s) {
-      const WgradOperand<T> oa(a0), ob(b0);
-      if (bias) wgrad_sums(a0, oa, sum);
-      at_a += step_a;
-      at_b += step_b;
-      a0.load(dy, at_a, row_a, off_a);
-      b0.load(x, at_b, row_b, off_b);
-      wgrad_products(oa, ob, acc);
+      for (int g = 0; g < kGroups; ++g) v += s_sum[g][threadIdx.x];
+      part[job.n * job.k + n0 + threadIdx.x] = v;
     }
+  }
+  if (!active) return;
+  if constexpr (kParts == 3) {
     bool finite = true;
 #pragma unroll
-    for (int fa = 0; fa < kWgradFrags; ++fa)
+    for (int f = 0; f < FN; ++f)
 #pragma unroll
-      for (int fb = 0; fb < kWgradFrags; ++fb)
+      for (int g = 0; g < FK; ++g)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) finite &= __builtin_isfinite(acc[fa][fb][q]);
-    if (__any(!finite)) {   // again with the fp32 instruction (rows r, 8 + r, 16 + r, 24 + r of a step at a time)
+        for (int q = 0; q < 4; ++q) finite &= __builtin_isfinite(acc[f][g][q]);
+    if (__any(!finite)) {   // again with the fp32 instruction, four rows at a time
 #pragma unroll
-      for (int fa = 0; fa < kWgradFrags; ++fa)
+      for (int f = 0; f < FN; ++f)
 #pragma unroll
-        for (int fb = 0; fb < kWgradFrags; ++fb) acc[fa][fb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-      at_a = at_b = 0;
+        for (int g = 0; g < FK; ++g) acc[f][g] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll 1
-      for (int s = 0; s < steps; ++s, at_a += step_a, at_b += step_b) {
-        a0.load(dy, at_a, row_a, off_a);
-        b0.load(x, at_b, row_b, off_b);
+      for (int64_t r = group; r < m1 - m0 + group; r += 4) {
+        float av[FN], bv[FK];
 #pragma unroll
-        for (int r = 0; r < kWgradLoads; ++r)
+        for (int f = 0; f < FN; ++f) {
+          const uint32_t at = static_cast<uint32_t>((r * job.n + wave_n + f * 16 + col16) * 4);
+          av[f] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(dy, at, 0, 0));
+          if (masked && __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(out, at, 0, 0)) <= 0.f) av[f] = 0.f;
+        }
 #pragma unroll
-          for (int fa = 0; fa < kWgradFrags; ++fa)
+        for (int g = 0; g < FK; ++g)
+          bv[g] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+              x, static_cast<uint32_t>((r * job.k + wave_k + g * 16 + col16) * 4), 0, 0));
 #pragma unroll
-            for (int fb = 0; fb < kWgradFrags; ++fb)
-              acc[fa][fb] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a0.v[r][fa]), __uint_as_float(b0.v[r][fb]),
-                                                                 acc[fa][fb], 0, 0, 0);
+        for (int f = 0; f < FN; ++f)
+#pragma unroll
+          for (int g = 0; g < FK; ++g) acc[f][g] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[f], bv[g], acc[f][g], 0, 0, 0);
       }
     }
-  } else {
-    auto multiply = [&](const WgradRows<T, VA>& a, const WgradRows<T, VB>& b) {
-      const WgradOperand<T> oa(a), ob(b);
-      wgrad_products(oa, ob, acc);
-      if (bias) wgrad_sums(a, oa, sum);
-    };
-    // Two steps in registers: the rows of one are on their way during the products of the other.  A step past the
-    // split's end reads zeros.
-    WgradRows<T, VA> a1;
-    WgradRows<T, VB> b1;
-    for (int s = 0; s < steps; s += 2) {
-      at_a += step_a;
-      at_b += step_b;
-      a1.load(dy, at_a, row_a, off_a);
-      b1.load(x, at_b, row_b, off_b);
-      multiply(a0, b0);
-      at_a += step_a;
-      at_b += step_b;
-      a0.load(dy, at_a, row_a, off_a);
-      b0.load(x, at_b, row_b, off_b);
-      multiply(a1, b1);
-    }
   }
-  // Element q of a lane's accumulator is row (dy column) group * 4 + q, column (x column) l16 of the tile fragment.
-  float* part = p.part + static_cast<int64_t>(split) * p.part_stride;
+  // Element q of a lane's accumulator is row (dy column) group * 4 + q, column (x column) lane % 16 of the fragment.
 #pragma unroll
-  for (int fa = 0; fa < kWgradFrags; ++fa)
+  for (int f = 0; f < FN; ++f)
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      const int64_t n = n0 + wgrad_col<VA>(fa, group * 4 + q);
-      if (n >= p.n) continue;
+      const int64_t n = wave_n + f * 16 + wgrad_col<T>(group * 4 + q);
+      if (n >= job.n) continue;
 #pragma unroll
-      for (int fb = 0; fb < kWgradFrags; ++fb) {
-        const int64_t k = k0 + wgrad_col<VB>(fb, l16);
-        if (k < p.k) part[n * p.k + k] = acc[fa][fb][q];
+      for (int g = 0; g < FK; ++g) {
+        const int64_t k = wave_k + g * 16 + col16;
+        if (k < job.k) part[n * job.k + k] = acc[f][g][q];
       }
-      if (sizeof(T) == 2 && bias && l16 == 0) part[p.n * p.k + n] = sum[fa][q];
     }
-  if (sizeof(T) == 4 && bias) {
+}
+
+// Sums of the partials of all products, in the order of the splits: 256 elements per workgroup, four per lane, the splits
+// dealt to its wavefronts.
+constexpr int kWgradSumBlock = 512;
+constexpr int kWgradSumWaves = kWgradSumBlock / kWave;
+
+template <typename E>
+__global__ __launch_bounds__(kWgradSumBlock) void wgrad_sums_kernel(WgradParams p, int blocks0) {
+  constexpr int kUnroll = 8;
+  __shared__ __align__(16) f32x4_t s_sum[kWgradSumWaves][kWave];
+  const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+  const int which = static_cast<int>(blockIdx.x) >= blocks0 ? 1 : 0;
+  const WgradJob& job = p.job[which];
+  const int64_t e = (static_cast<int64_t>(blockIdx.x) - (which ? blocks0 : 0)) * (4 * kWave) + lane * 4;
+  const bool live = e < job.stride;                     // (a multiple of four)
+  const f32x4_t* src = reinterpret_cast<const f32x4_t*>(job.part + (live ? e : 0));
+  const int64_t step = job.stride / 4;
+  f32x4_t sum = {0.f, 0.f, 0.f, 0.f};
+  for (int s = wave; s < job.splits; s += kWgradSumWaves * kUnroll) {
+    f32x4_t v[kUnroll];
 #pragma unroll
-    for (int f = 0; f < kWgradFrags; ++f) {
-      float v = sum[f][0] + sum[f][1];
-      v += __shfl_xor(v, 16, kWave);
-      v += __shfl_xor(v, 32, kWave);
-      const int64_t n = n0 + wgrad_col<VA>(f, l16);
-      if (group == 0 && n < p.n) part[p.n * p.k + n] = v;
+    for (int u = 0; u < kUnroll; ++u) v[u] = src[min(s + u * kWgradSumWaves, job.splits - 1) * step];
+#pragma unroll
+    for (int u = 0; u < kUnroll; ++u)
+      if (s + u * kWgradSumWaves < job.splits) sum += v[u];
+  }
+  s_sum[wave][lane] = sum;
+  __syncthreads();
+  if (wave != 0 || !live) return;
+#pragma unroll
+  for (int w = 1; w < kWgradSumWaves; ++w) sum += s_sum[w][lane];
+  const int64_t nk = job.n * job.k;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    if (e + q < nk) {
+      if (job.dw != nullptr) static_cast<E*>(job.dw)[e + q] = from_float<E>(sum[q]);
+    } else if (e + q < nk + job.n) {
+      if (job.db != nullptr) static_cast<E*>(job.db)[e + q - nk] = from_float<E>(sum[q]);
     }
   }
-}
-
-// How the rows are split: into as many parts as keep eight wavefronts on every CU, while a part keeps a few steps of
-// its loop and the partials (written once, read once) stay below half of the inputs they come from or a few
-// megabytes.  Both launches, against the library's GEMM and column sum, for n x k = 256 x 128:
-//   rows      bf16: here / library     fp32: here / library
-//   256              18 / 27 us              20 / 42 us
-//   17 k             25 / 108 us             33 / 120 us     (fp32 instruction:  40)
-//   170 k            46 / 403 us            101 / 358 us     (118; bytes alone 52, products 66 at the bf16 rate)
-//   700 k           171 / 1435 us           436 / 1385 us    (431)
-static void wgrad_shape(int64_t m, int64_t n, int64_t k, int elem_size, WgradParams& p) {
-  const int64_t tiles_n = ceil_div(n, kWgradTile);
-  p.tiles_k = static_cast<int>(ceil_div(k, kWgradTile));
-  p.tiles = static_cast<int>(tiles_n * p.tiles_k);
-  p.tile_groups = static_cast<int>(ceil_div(p.tiles, kWgradWaves));
-  p.splits_per_group = p.tile_groups == 1 ? kWgradWaves / p.tiles : 1;
-  p.part_stride = n * k + n;
-  const int64_t part_bytes = p.part_stride * 4;
-  int64_t s = p.tile_groups == 1 ? kWgradGroups * p.splits_per_group : ceil_div(kWgradGroups, p.tile_groups);
-  s = std::min(s, std::max(kWgradPartBytes, m * (n + k) * elem_size / 2) / part_bytes);
-  s = std::max<int64_t>(1, std::min(s, ceil_div(m, kWgradMinRows)));
-  // a split's rows are addressed with 32-bit offsets, and the loop reads up to three steps past its last one
-  s = std::max(s, ceil_div(m * std::max(n, k) * elem_size, int64_t{1} << 30));
-  p.rows_per_split = ceil_div(ceil_div(m, s), kWgradRows) * kWgradRows;
-  p.splits = static_cast<int>(ceil_div(m, p.rows_per_split));
-}
-
-template <typename T>
-static void launch_wgrad(const WgradParams& p, int va, int vb, hipStream_t st) {
-  const int64_t groups = p.tile_groups == 1 ? ceil_div(p.splits, p.splits_per_group)
-                                            : ceil_div(p.splits, 8) * 8 * p.tile_groups;
-  const dim3 grid(static_cast<unsigned>(groups)), block(kWgradWaves * kWave);
-#define APT_WGRAD(VA, VB) hipLaunchKernelGGL((wgrad_kernel<T, VA, VB>), grid, block, 0, st, p)
-#define APT_WGRAD_B(VA)              \
-  if (vb == 4) APT_WGRAD(VA, 4);     \
-  else if (vb == 2) APT_WGRAD(VA, 2); \
-  else APT_WGRAD(VA, 1)
-  if (va == 4) { APT_WGRAD_B(4); }
-  else if (va == 2) { APT_WGRAD_B(2); }
-  else { APT_WGRAD_B(1); }
-#undef APT_WGRAD_B
-#undef APT_WGRAD
-}
-
-static int wgrad_vec(const void* p, int64_t cols, int elem_size) {
-  for (int v = 4; v > 1; v >>= 1)
-    if (cols % v == 0 && (reinterpret_cast<uintptr_t>(p) & (v * elem_size - 1)) == 0) return v;
-  return 1;
 }
 
 static bool wgrad_sizes_ok(int64_t m, int64_t n, int64_t k) {
-  return m >= 0 && n > 0 && k > 0 && n <= (1 << 20) && k <= (1 << 20) && n * k <= (int64_t{1} << 30);
+  return m >= 0 && n > 0 && k >= 0 && n <= (1 << 20) && k <= (1 << 20) && n * k <= (int64_t{1} << 30);
+}
+
+// Tiles of 128 x 128 where both sides of a product are longer than 64 and its rows make a workgroup for every CU, of
+// 64 x 64 otherwise (the tile of 128 with half of it empty: 20 against 12 us for 10 k rows of 47 x 256 fp32).  The rows are
+// split into as many parts as keep the CUs busy, while a part keeps two steps of its loop and the partials (written once,
+// read once) stay below half of the inputs they come from or a few megabytes.  Both launches; before: a wavefront for
+// itself loaded, regrouped and (fp32) split its operands, every tile's again.  us:
+//   rows n x k            fp32 before / now      bf16 before / now
+//   700 k 256 x 128           391 / 385              170 / 131
+//   124 k 256 x 128            74 /  71               38 /  29
+//   54 k  256 x 100            43 /  37               26 /  20
+//   54 k  256 x (100 + 100)    87 /  60               53 /  26      (two products in one launch)
+//   11 k  256 x (256 + 256)    77 /  34               52 /  22
+//   11 k   47 x 256            21 /  12               18 /  14
+//   200 k  64 x 256            68 /  68               40 /  27
+//   460 k 256 x 64            166 / 178               77 /  62
+// fp32, 700 k rows: 3800 cycles a step and CU, of which 1540 on the matrix units, 770 in LDS and 1100 splitting; bf16:
+// 4.3 TB/s of rows.
+static bool wgrad_shape(WgradParams& p, int elem_size) {
+  const int64_t step = elem_size == 4 ? 32 : 64;
+  bool big = false;
+  for (int j = 0; j < p.jobs; ++j) {
+    const WgradJob& w = p.job[j];
+    big |= w.n > 64 && w.k > 64 && ceil_div(w.n, 128) * ceil_div(w.k, 128) * ceil_div(w.m, 2 * step) >= 256;
+  }
+  const int64_t tile = big ? 128 : 64;
+  int64_t work = 0, part_row = 0, bytes = 0, most = 1, widest = 1;
+  p.tiles = 0;
+  for (int j = 0; j < p.jobs; ++j) {
+    WgradJob& w = p.job[j];
+    w.tiles_k = static_cast<int>(std::max<int64_t>(ceil_div(w.k, tile), 1));
+    w.tiles = static_cast<int>(ceil_div(w.n, tile) * w.tiles_k);
+    w.stride = ceil_div(w.n * w.k + w.n, 4) * 4;
+    p.tiles += w.tiles;
+    work += w.m * w.tiles;
+    part_row += w.m * w.stride * 4;
+    bytes += w.m * (w.n + w.k) * elem_size;
+    most = std::max(most, w.m);
+    widest = std::max(widest, std::max(w.n, w.k) * elem_size);
+  }
+  // rows of a split: from the workgroups aimed at, and from the partials' bytes (part_row / rows)
+  int64_t rows = std::max(ceil_div(work, kWgradGroups), 2 * step);
+  if (!big) rows = std::max({ceil_div(work, kWgradSmallGroups), std::min(rows, kWgradSmallSteps * step), 2 * step});
+  rows = std::max(rows, ceil_div(part_row, std::max(kWgradPartBytes, bytes / 2)));
+  rows = std::min(ceil_div(rows, step) * step, ceil_div(most, step) * step);
+  // a split's rows are addressed with 32-bit offsets, and the loop reads up to 2 kWgradAhead steps past its last one
+  rows = std::min(rows, std::max<int64_t>((int64_t{1} << 30) / widest / step, 1) * step);
+  p.rows_per_split = rows;
+  for (int j = 0; j < p.jobs; ++j) p.job[j].splits = static_cast<int>(ceil_div(p.job[j].m, rows));
+  return big;
+}
+
+static size_t wgrad_bytes(const WgradParams& p) {
+  size_t bytes = 0;
+  for (int j = 0; j < p.jobs; ++j) bytes += static_cast<size_t>(std::max(p.job[j].splits, 1)) * p.job[j].stride * sizeof(float);
+  return bytes;
+}
+
+// Whether rows of bf16 can be read in pairs of columns.
+static bool wgrad_pairs(const void* p, int64_t cols) { return cols % 2 == 0 && (reinterpret_cast<uintptr_t>(p) & 3) == 0; }
+
+template <typename T>
+static void launch_wgrad(const WgradParams& p, bool big, hipStream_t st) {
+  int splits = 0;
+  for (int j = 0; j < p.jobs; ++j) splits = std::max(splits, p.job[j].splits);
+  const dim3 grid(static_cast<unsigned>(ceil_div(splits, 8) * 8 * p.tiles)), block(kWgradBlock);
+  const bool masked = p.job[0].out != nullptr || p.job[1].out != nullptr;
+#define APT_WGRAD(TYPE, F) hipLaunchKernelGGL((wgrad_kernel<TYPE, F, F>), grid, block, (WgradTile<TYPE, F, F>::kLds), st, p)
+  if (masked && big) APT_WGRAD(WgradRelu<T>, 4);
+  else if (masked) APT_WGRAD(WgradRelu<T>, 2);
+  else if (big) APT_WGRAD(T, 4);
+  else APT_WGRAD(T, 2);
+#undef APT_WGRAD
+}
+
+static int wgrad_params(const char* who, const apt_wgrad_product* products, int count, int elem_size, WgradParams& p) {
+  APT_REQUIRE(products != nullptr && count >= 1 && count <= kWgradJobs, APT_EINVAL, "%s: %d products", who, count);
+  APT_REQUIRE(elem_size == 2 || elem_size == 4, APT_EINVAL, "%s: elem_size %d (4 = fp32, 2 = bf16)", who, elem_size);
+  p.jobs = count;
+  for (int j = 0; j < count; ++j) {
+    const apt_wgrad_product& q = products[j];
+    APT_REQUIRE(wgrad_sizes_ok(q.m, q.n, q.k), APT_ELIMIT, "%s: sizes out of range (m %lld, n %lld, k %lld)", who,
+                (long long)q.m, (long long)q.n, (long long)q.k);
+    WgradJob& w = p.job[j];
+    w.dy = q.dy;
+    w.out = q.out;
+    w.x = q.x;
+    w.m = q.m;
+    w.n = q.n;
+    w.k = q.k;
+    w.dw = q.dw;
+    w.db = q.db;
+  }
+  return APT_OK;
 }
 
 }  // namespace apt
 
-extern "C" size_t apt_linear_wgrad_workspace_bytes(int64_t m, int64_t n, int64_t k, int elem_size) {
+extern "C" size_t apt_linear_wgrads_workspace_bytes(const apt_wgrad_product* products, int count, int elem_size) {
   using namespace apt;
-  if (!wgrad_sizes_ok(m, n, k) || (elem_size != 2 && elem_size != 4)) return 0;
   WgradParams p{};
-  wgrad_shape(std::max<int64_t>(m, 1), n, k, elem_size, p);
-  return static_cast<size_t>(p.splits) * p.part_stride * sizeof(float);
+  if (wgrad_params("apt_linear_wgrads_workspace_bytes", products, count, elem_size, p) != APT_OK) return 0;
+  wgrad_shape(p, elem_size);
+  return wgrad_bytes(p);
+}
+
+extern "C" int apt_linear_wgrads(const apt_wgrad_product* products, int count, int elem_size, void* workspace,
+                                 size_t workspace_bytes, void* stream) {
+  using namespace apt;
+  const char* who = "apt_linear_wgrads";
+  WgradParams p{};
+  if (const int rc = wgrad_params(who, products, count, elem_size, p)) return rc;
+  const bool big = wgrad_shape(p, elem_size);
+  APT_REQUIRE(workspace != nullptr && workspace_bytes >= wgrad_bytes(p) && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0,
+              APT_EWORKSPACE, "%s: workspace too small or not 16-byte aligned (see apt_linear_wgrads_workspace_bytes)", who);
+  float* part = static_cast<float*>(workspace);
+  bool odd = false, any = false;
+  int64_t sum_blocks[kWgradJobs] = {};
+  for (int j = 0; j < p.jobs; ++j) {
+    WgradJob& w = p.job[j];
+    APT_REQUIRE((w.k == 0 || w.dw != nullptr) && (w.k > 0 || w.db != nullptr) &&
+                    (w.m == 0 || (w.dy != nullptr && (w.k == 0 || w.x != nullptr))),
+                APT_EINVAL, "%s: a tensor is NULL", who);
+    w.part = part;
+    part += static_cast<int64_t>(std::max(w.splits, 1)) * w.stride;
+    odd |= !wgrad_pairs(w.dy, w.n) || !wgrad_pairs(w.out, w.n) || (w.k > 0 && !wgrad_pairs(w.x, w.k));
+    any |= w.splits > 0;
+    sum_blocks[j] = ceil_div(w.stride, 4 * kWave);   // (no rows: zeros)
+  }
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  if (any) {
+    if (elem_size == 4) launch_wgrad<float>(p, big, st);
+    else if (odd) launch_wgrad<WgradOdd>(p, big, st);
+    else launch_wgrad<uint16_t>(p, big, st);
+    APT_LAUNCH_CHECK("wgrad_kernel");
+  }
+  const dim3 grid(static_cast<unsigned>(sum_blocks[0] + sum_blocks[1])), block(kWgradSumBlock);
+  const int blocks0 = static_cast<int>(sum_blocks[0]);
+  if (elem_size == 4) hipLaunchKernelGGL(wgrad_sums_kernel<float>, grid, block, 0, st, p, blocks0);
+  else hipLaunchKernelGGL(wgrad_sums_kernel<uint16_t>, grid, block, 0, st, p, blocks0);
+  APT_LAUNCH_CHECK("wgrad_sums_kernel");
+  return APT_OK;
+}
+
+extern "C" size_t apt_linear_wgrad_workspace_bytes(int64_t m, int64_t n, int64_t k, int elem_size) {
+  if (k < 1) return 0;
+  const apt_wgrad_product q{nullptr, nullptr, nullptr, m, n, k, nullptr, nullptr};
+  return apt_linear_wgrads_workspace_bytes(&q, 1, elem_size);
 }
 
 extern "C" int apt_linear_wgrad(const void* dy, const void* x, int64_t m, int64_t n, int64_t k, int elem_size, void* dw,
                                 void* db, void* workspace, size_t workspace_bytes, void* stream) {
   using namespace apt;
-  APT_REQUIRE(wgrad_sizes_ok(m, n, k), APT_ELIMIT, "apt_linear_wgrad: sizes out of range (m %lld, n %lld, k %lld)",
-              (long long)m, (long long)n, (long long)k);
-  APT_REQUIRE(elem_size == 2 || elem_size == 4, APT_EINVAL, "apt_linear_wgrad: elem_size %d (4 = fp32, 2 = bf16)",
-              elem_size);
-  APT_REQUIRE(dw != nullptr && (m == 0 || (dy != nullptr && x != nullptr)), APT_EINVAL,
-              "apt_linear_wgrad: a tensor is NULL");
-  WgradParams p{};
-  p.dy = dy;
-  p.x = x;
-  p.m = m;
-  p.n = n;
-  p.k = k;
-  p.part = static_cast<float*>(workspace);
-  wgrad_shape(std::max<int64_t>(m, 1), n, k, elem_size, p);
-  APT_REQUIRE(workspace != nullptr && workspace_bytes >= static_cast<size_t>(p.splits) * p.part_stride * sizeof(float) &&
-                  (reinterpret_cast<uintptr_t>(workspace) & 15) == 0,
-              APT_EWORKSPACE, "apt_linear_wgrad: workspace too small or not 16-byte aligned "
-                              "(see apt_linear_wgrad_workspace_bytes)");
-  hipStream_t st = static_cast<hipStream_t>(stream);
-  if (m == 0) p.splits = 0;   // the reduction then writes zeros
-  if (p.splits > 0) {
-    const int va = wgrad_vec(dy, n, elem_size), vb = wgrad_vec(x, k, elem_size);
-    if (elem_size == 4) launch_wgrad<float>(p, va, vb, st);
-    else launch_wgrad<uint16_t>(p, va, vb, st);
-    APT_LAUNCH_CHECK("wgrad_kernel");
-  }
-  if (elem_size == 4) launch_partial_sums<float, float>(p.part, p.part_stride, p.splits, dw, n * k, db, n, nullptr, 0, st);
-  else launch_partial_sums<uint16_t, uint16_t>(p.part, p.part_stride, p.splits, dw, n * k, db, n, nullptr, 0, st);
-  APT_LAUNCH_CHECK("partial_sums_kernel");
-  return APT_OK;
+  APT_REQUIRE(k > 0, APT_ELIMIT, "apt_linear_wgrad: sizes out of range (m %lld, n %lld, k %lld)", (long long)m, (long long)n,
+              (long long)k);
+  const apt_wgrad_product q{dy, nullptr, x, m, n, k, dw, db};
+  return apt_linear_wgrads(&q, 1, elem_size, workspace, workspace_bytes, stream);
 }

@@ -12,6 +12,7 @@
 #include <torch/library.h>
 #include <torch/torch.h>
 
+#include <array>
 #include <deque>
 #include <memory>
 #include <string>
@@ -966,23 +967,57 @@ Tensor UMulV(Tensor coo_row, Tensor coo_col, Tensor lhs, Tensor rhs, Tensor coo_
 // ---------------------------------------------------------------- dense layers over a block's rows
 namespace {
 
-// Gradients of the weight [n, k] and the bias of y = x w^T + b (apt_linear_wgrad).
-std::tuple<Tensor, Tensor> linear_wgrad(const Tensor& dy_in, const Tensor& x_in, bool want_bias) {
-  auto dy = dy_in.contiguous(), x = x_in.contiguous();
-  const int64_t m = x.size(0), n = dy.size(1), k = x.size(1);
-  const int es = static_cast<int>(x.element_size());
-  const size_t need = apt_linear_wgrad_workspace_bytes(m, n, k, es);
-  Tensor db;
-  if (need == 0) {   // a weight beyond the kernel's sizes
-    if (want_bias) db = dy.sum(0);
-    return {dy.t().mm(x), db};
+// A product whose weight's gradient is wanted, dw = dy^T x, and its bias's, the column sums of dy; dy counts where `relu`
+// is positive if that is given.  Without x the sums alone.
+struct WeightGrad {
+  Tensor dy, x;
+  bool want_bias = false;
+  Tensor relu;
+  Tensor dw{}, db{};
+};
+// Gradients of one or two products, of one type, in one launch (apt_linear_wgrads).
+template <size_t N>
+void weight_grads(std::array<WeightGrad, N>& all, size_t count = N) {
+  apt_wgrad_product products[N] = {};
+  int es = 0;
+  for (size_t i = 0; i < count; ++i) {
+    WeightGrad& g = all[i];
+    g.dy = g.dy.contiguous();
+    if (g.x.defined()) g.x = g.x.contiguous();
+    if (g.relu.defined()) g.relu = g.relu.contiguous();
+    es = static_cast<int>(g.dy.element_size());
+    products[i].m = g.dy.size(0);
+    products[i].n = g.dy.size(1);
+    products[i].k = g.x.defined() ? g.x.size(1) : 0;
   }
-  auto ws = torch::empty({static_cast<int64_t>(need)}, x.options().dtype(torch::kUInt8));
-  auto dw = torch::empty({n, k}, x.options());
-  if (want_bias) db = torch::empty({n}, x.options());
-  check(apt_linear_wgrad(dy.data_ptr(), x.data_ptr(), m, n, k, es, dw.data_ptr(), want_bias ? db.data_ptr() : nullptr,
-                         ws.data_ptr(), need, stream()));
-  return {dw, db};
+  const size_t need = apt_linear_wgrads_workspace_bytes(products, static_cast<int>(count), es);
+  if (need == 0) {   // a weight beyond the kernel's sizes
+    for (size_t i = 0; i < count; ++i) {
+      WeightGrad& g = all[i];
+      const Tensor dy = g.relu.defined() ? at::threshold_backward(g.dy, g.relu, 0) : g.dy;
+      if (g.x.defined()) g.dw = dy.t().mm(g.x);
+      if (g.want_bias) g.db = dy.sum(0);
+    }
+    return;
+  }
+  auto ws = torch::empty({static_cast<int64_t>(need)}, all[0].dy.options().dtype(torch::kUInt8));
+  for (size_t i = 0; i < count; ++i) {
+    WeightGrad& g = all[i];
+    apt_wgrad_product& q = products[i];
+    if (g.x.defined()) g.dw = torch::empty({q.n, q.k}, g.dy.options());
+    if (g.want_bias) g.db = torch::empty({q.n}, g.dy.options());
+    q.dy = g.dy.data_ptr();
+    q.out = g.relu.defined() ? g.relu.data_ptr() : nullptr;
+    q.x = g.x.defined() ? g.x.data_ptr() : nullptr;
+    q.dw = g.dw.defined() ? g.dw.data_ptr() : nullptr;
+    q.db = g.db.defined() ? g.db.data_ptr() : nullptr;
+  }
+  check(apt_linear_wgrads(products, static_cast<int>(count), es, ws.data_ptr(), need, stream()));
+}
+std::tuple<Tensor, Tensor> linear_wgrad(const Tensor& dy, const Tensor& x, bool want_bias) {
+  std::array<WeightGrad, 1> g{WeightGrad{dy, x, want_bias}};
+  weight_grads(g);
+  return {g[0].dw, g[0].db};
 }
 
 // x w^T (+ x2 w2^T on the first rows) (+ b) with w [n, k] of any strides; `onto`: added to (and returned).  fp32 rows
@@ -1309,8 +1344,11 @@ struct SageLayerFn : public torch::autograd::Function<SageLayerFn> {
     const auto spread = [&](const Tensor& d) {
       return aggregate_gradient(d, relabeled, num_dst, fanout, num_src, inv, saved[6], saved[7]);
     };
-    const Tensor dz = before_relu(grads[0], saved[8]), self = x.defined() ? x.narrow(0, 0, num_dst) : x;
+    const Tensor self = x.defined() ? x.narrow(0, 0, num_dst) : x;
     const bool want_x = ctx->needs_input_grad(0), want_n = ctx->needs_input_grad(1), want_s = ctx->needs_input_grad(2);
+    // where the weights' gradients alone read the gradient, the ReLU's mask is applied as they do
+    const bool masked = saved[8].defined() && !want_x && !(first && want_n) && !torch::GradMode::is_enabled();
+    const Tensor dz = masked ? grads[0] : before_relu(grads[0], saved[8]);
     Tensor dpre, dx, dwn, dws, db;
     if (first && (want_x || want_n)) dpre = spread(dz);
     if (torch::GradMode::is_enabled()) {   // a graph of the gradients is wanted: operations that carry one
@@ -1323,9 +1361,15 @@ struct SageLayerFn : public torch::autograd::Function<SageLayerFn> {
       if (want_s) dws = dz.t().mm(self);
       if (bias) db = dz.sum(0);
     } else {
-      if (want_s) std::tie(dws, db) = linear_wgrad(dz, self, bias);
-      else if (bias) db = dz.sum(0);
-      if (want_n) dwn = std::get<0>(first ? linear_wgrad(dpre, x, false) : linear_wgrad(dz, saved[5], false));
+      const Tensor relu = masked ? saved[8] : Tensor();
+      std::array<WeightGrad, 2> g;
+      size_t count = 0;
+      if (want_s || bias) g[count++] = WeightGrad{dz, want_s ? self : Tensor(), bias, relu};
+      if (want_n) g[count++] = first ? WeightGrad{dpre, x} : WeightGrad{dz, saved[5], false, relu};
+      if (count > 0) weight_grads(g, count);
+      if (want_s) dws = g[0].dw;
+      if (bias) db = g[0].db;
+      if (want_n) dwn = g[count - 1].dw;
       if (want_x)
         dx = first ? dense(dpre, w_neigh.t(), dz, w_self.t()) : [&] {
           Tensor d = spread(dense(dz, w_neigh.t()));
@@ -1395,13 +1439,20 @@ struct GcnLayerFn : public torch::autograd::Function<GcnLayerFn> {
       dh = aggregate_gradient(dz, saved[2], ctx->saved_data["num_dst"].toInt(), ctx->saved_data["fanout"].toInt(),
                               ctx->saved_data["num_src"].toInt(), Tensor(), saved[3], saved[4],
                               ctx->saved_data["scale"].toDouble());
-    if (ctx->saved_data["bias"].toBool()) db = dz.sum(0);
+    const bool bias = ctx->saved_data["bias"].toBool();
     if (torch::GradMode::is_enabled()) {   // a graph of the gradients is wanted: operations that carry one
       if (ctx->needs_input_grad(0)) dx = dh.mm(w.t());
       if (ctx->needs_input_grad(1)) dw = x.t().mm(dh);
+      if (bias) db = dz.sum(0);
     } else {
       if (ctx->needs_input_grad(0)) dx = dense(dh, w);
-      if (ctx->needs_input_grad(1)) dw = std::get<0>(linear_wgrad(x, dh, false));
+      std::array<WeightGrad, 2> g;
+      size_t count = 0;
+      if (bias) g[count++] = WeightGrad{dz, Tensor(), true};
+      if (ctx->needs_input_grad(1)) g[count++] = WeightGrad{x, dh};
+      if (count > 0) weight_grads(g, count);
+      if (bias) db = g[0].db;
+      if (ctx->needs_input_grad(1)) dw = g[count - 1].dw;
     }
     return {dx, dw, db, Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
   }

@@ -919,6 +919,23 @@ size_t apt_linear_wgrad_workspace_bytes(int64_t m, int64_t n, int64_t k, int ele
 int apt_linear_wgrad(const void* dy, const void* x, int64_t m, int64_t n, int64_t k, int elem_size,
                      void* dw, void* db, void* workspace, size_t workspace_bytes, void* stream);
 
+/* One or two such products (count) of one type in one launch, each with its own
+ * rows and sizes.  out [m, n], optional: the result of a ReLU that dy is the
+ * gradient of; dy counts where out > 0.  k = 0: the column sums alone (x and dw
+ * NULL).  workspace: apt_linear_wgrads_workspace_bytes of the same sizes (the
+ * pointers are not looked at); 0 = sizes out of range. */
+typedef struct apt_wgrad_product {
+  const void* dy;
+  const void* out;
+  const void* x;
+  int64_t m, n, k;
+  void* dw;
+  void* db;
+} apt_wgrad_product;
+size_t apt_linear_wgrads_workspace_bytes(const apt_wgrad_product* products, int count, int elem_size);
+int apt_linear_wgrads(const apt_wgrad_product* products, int count, int elem_size, void* workspace,
+                      size_t workspace_bytes, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

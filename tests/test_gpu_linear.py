@@ -61,3 +61,41 @@ def test_block_linear_gradients(dtype, kn):
     gw, = torch.autograd.grad(y.float().square().sum(), w, create_graph=True)
     gx, = torch.autograd.grad(gw.float().sum(), x)
     assert gx.shape == x.shape and bool(torch.isfinite(gx).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("m,m2,n,k,k2", [(1, 1, 1, 1, 1), (129, 65, 65, 129, 64), (6000, 6000, 256, 100, 100), (4097, 900, 47, 256, 256),
+                                         (9000, 257, 130, 0, 70), (40000, 40000, 96, 101, 33), (300, 0, 20, 12, 7)])
+def test_two_weight_gradients_in_one_launch(capi, m, m2, n, k, k2, dtype):
+    """Products of different rows and columns, column sums alone (k = 0), the mask of a ReLU with NaN, infinite and zero
+    results, and the edges of both tiles (64, 128) and of a split."""
+    gen = torch.Generator(device=DEV).manual_seed(m + n)
+    draw = lambda r, c: torch.randn(r, c, generator=gen, device=DEV).to(dtype)
+    dy, x, relu = draw(m, n), draw(m, k) if k else None, torch.relu(draw(m, n))
+    relu.view(-1)[:3:2] = torch.tensor([float("nan"), float("inf")], device=DEV, dtype=dtype)[:relu.view(-1)[:3:2].numel()]
+    dy2, x2 = draw(m2, n + 3), draw(m2, k2)
+    (dw, db), (dw2, db2) = capi.linear_wgrads([(dy, x, relu, True), (dy2, x2, None, False)])
+    live = torch.where(relu <= 0, torch.zeros_like(dy), dy).double()      # (a NaN passes, as in torch)
+    # as in test_linear_wgrad: fp32 sums of m products of magnitude ~1, bf16 results round at 2^-9
+    tol = 2.0 ** -8 if dtype == torch.bfloat16 else 0.0
+    for got, want, rows in ((dw, None if x is None else live.t() @ x.double(), m), (db, live.sum(0), m),
+                            (dw2, dy2.double().t() @ x2.double(), m2)):
+        if want is None:
+            assert got is None
+            continue
+        bound = tol * want.abs() + 2.0 ** -22 * (rows ** 0.5) * 16 + 2.0 ** -22 * want.abs()
+        assert got.dtype == dtype and bool(((got.double() - want).abs() <= bound).all())
+    assert db2 is None
+
+
+def test_weight_gradient_of_infinite_rows(capi):
+    """The parts of an infinity are NaN: the tile is formed again in fp32, and gives what fp32 gives."""
+    dy, x = torch.randn(500, 70, device=DEV), torch.randn(500, 80, device=DEV)
+    dy[77, 3], x[401, 5], relu = float("inf"), float("-inf"), torch.ones(500, 70, device=DEV)
+    relu[401] = 0
+    (dw, db), = capi.linear_wgrads([(dy, x, relu, True)])
+    live = torch.where(relu <= 0, torch.zeros_like(dy), dy)
+    want = live.double().t() @ x.double()     # (0 * inf: NaN, in column 5 and in row 3 where x is not)
+    assert torch.equal(dw.isnan(), want.isnan()) and torch.equal(dw.isinf(), want.isinf())
+    ok = want.isfinite()
+    assert torch.allclose(dw[ok].double(), want[ok], atol=2.0 ** -22 * 500 ** 0.5 * 16) and db[3].isinf()
