@@ -14,6 +14,7 @@
 // attention vectors is what is left of large terms that cancel, and moves by several per cent with that rounding.
 // Without gradients (`wide`) nothing is rounded between the rows and the result: scores, sum and result are fp32.
 #include <algorithm>
+#include <type_traits>
 
 #include "common.hpp"
 #include "feature_rows.hpp"
@@ -500,60 +501,87 @@ static void launch_gat_source_t(const GatSourceParams& p, int64_t num_edges, hip
 }
 
 // ------------------------------------------------------------------ backward, parameters
-// Column sums over the rows: a workgroup has a run of rows, a thread VEC columns of every RG-th of them.
-constexpr int kParamBlocks = 1024;
+// Column sums over the rows: a thread has VEC columns of every so many-th row, first of those that are destinations too,
+// then of the others, which have nothing but ft.  Bound by reading ft and d_out once; kUnroll rows of a lane group are on
+// their way (loads outside branches: a conversion inside one waits for its load).  99 k rows of 4 x 64 bf16, 19 k of them
+// destinations: PARAM_US us with the sum of the partials, 40 with the loads in branches and rows in one piece per workgroup.
+// TwoHeads: a lane's features may belong to two heads.
+constexpr int kParamBlocks = 512;
 
-template <typename T, int VEC>
-__global__ __launch_bounds__(kAggBlock) void gat_param_grad_kernel(const T* __restrict__ ft, const T* __restrict__ d_out,
+template <typename T> struct TwoHeads {};
+template <typename T> struct ParamRow {
+  using Elem = T;
+  static constexpr bool kTwo = false;
+};
+template <typename T> struct ParamRow<TwoHeads<T>> {
+  using Elem = T;
+  static constexpr bool kTwo = true;
+};
+
+template <typename R, int VEC>
+__global__ __launch_bounds__(kAggBlock) void gat_param_grad_kernel(const typename ParamRow<R>::Elem* __restrict__ ft,
+                                                                   const typename ParamRow<R>::Elem* __restrict__ d_out,
                                                                    const float* __restrict__ d_el,
                                                                    const float* __restrict__ d_er, int64_t num_src,
                                                                    int64_t num_dst, int heads, int64_t dim, int lanes,
-                                                                   int64_t rows_per_block, float* __restrict__ part,
-                                                                   ParamVec attn_l) {
-  constexpr int kUnroll = 4;
+                                                                   float* __restrict__ part, ParamVec attn_l) {
+  using T = typename ParamRow<R>::Elem;
+  constexpr bool TWO = ParamRow<R>::kTwo;
+  constexpr int kUnroll = 8;
   const Terms<T> term(attn_l);
   __shared__ float s_sum[3 * VEC][kAggBlock];
   const int64_t row_len = heads * dim;
   const int groups = kAggBlock / lanes, grp = threadIdx.x / lanes, l = threadIdx.x % lanes;
-  const int64_t begin = blockIdx.x * rows_per_block, end = min(begin + rows_per_block, num_src);
+  const int64_t first = static_cast<int64_t>(grp) * gridDim.x + blockIdx.x, step = static_cast<int64_t>(groups) * gridDim.x;
   float* out = part + static_cast<int64_t>(blockIdx.x) * 3 * row_len;
   for (int64_t c0 = 0; c0 < row_len; c0 += static_cast<int64_t>(lanes) * VEC) {
     const int64_t c = c0 + static_cast<int64_t>(l) * VEC;
     const bool live = c < row_len;
-    const int h0 = live ? static_cast<int>(c / dim) : 0;
-    const int cut = static_cast<int>(min(static_cast<int64_t>(VEC), (h0 + 1) * dim - c));
+    const int64_t at = live ? c : 0;
+    const int h0 = static_cast<int>(at / dim);
+    const int cut = static_cast<int>(min(static_cast<int64_t>(VEC), (h0 + 1) * dim - at));
     const int h1 = cut < VEC ? h0 + 1 : h0;
     float sl[VEC], sr[VEC], sb[VEC];
 #pragma unroll
     for (int k = 0; k < VEC; ++k) sl[k] = sr[k] = sb[k] = 0.f;
-    for (int64_t r0 = begin + grp; r0 < end; r0 += static_cast<int64_t>(kUnroll) * groups) {
-      float v[kUnroll][VEC], o[kUnroll][VEC], l0[kUnroll], l1[kUnroll], e0[kUnroll], e1[kUnroll];
+    auto rows = [&](int64_t from, int64_t to, auto both) {
+      for (int64_t r0 = from + first; r0 < to; r0 += kUnroll * step) {
+        Row<T, VEC> v[kUnroll], o[kUnroll];
+        float l0[kUnroll], l1[kUnroll], e0[kUnroll], e1[kUnroll];
 #pragma unroll
-      for (int u = 0; u < kUnroll; ++u) {
-        const int64_t r = r0 + u * groups;
-#pragma unroll
-        for (int k = 0; k < VEC; ++k) v[u][k] = o[u][k] = 0.f;
-        l0[u] = l1[u] = e0[u] = e1[u] = 0.f;
-        if (r < end && live) {
-          load_vec<T, VEC>(ft, r * row_len + c, v[u]);
+        for (int u = 0; u < kUnroll; ++u) {
+          const int64_t r = min(r0 + u * step, to - 1);
+          v[u] = load_row<T, VEC>(ft, r * row_len + at);
           l0[u] = d_el[r * heads + h0];
-          l1[u] = d_el[r * heads + h1];
-          if (r < num_dst) {
-            load_vec<T, VEC>(d_out, r * row_len + c, o[u]);
-            e0[u] = term(d_er[r * heads + h0]);
-            e1[u] = term(d_er[r * heads + h1]);
+          if (TWO) l1[u] = d_el[r * heads + h1];
+          if constexpr (decltype(both)::value) {
+            o[u] = load_row<T, VEC>(d_out, r * row_len + at);
+            e0[u] = d_er[r * heads + h0];
+            if (TWO) e1[u] = d_er[r * heads + h1];
+          }
+        }
+#pragma unroll
+        for (int u = 0; u < kUnroll; ++u) {
+          if (r0 + u * step >= to) break;   // group-uniform
+          if constexpr (decltype(both)::value) {
+            e0[u] = term(e0[u]);
+            if (TWO) e1[u] = term(e1[u]);
+          }
+#pragma unroll
+          for (int k = 0; k < VEC; ++k) {
+            const bool own = !TWO || k < cut;
+            const float f = row_elem<T, VEC>(v[u], k);
+            sl[k] += term((own ? l0[u] : l1[u]) * f);
+            if constexpr (decltype(both)::value) {
+              sr[k] += term((own ? e0[u] : e1[u]) * f);
+              sb[k] += row_elem<T, VEC>(o[u], k);
+            }
           }
         }
       }
-#pragma unroll
-      for (int u = 0; u < kUnroll; ++u)
-#pragma unroll
-        for (int k = 0; k < VEC; ++k) {
-          sl[k] += term((k < cut ? l0[u] : l1[u]) * v[u][k]);
-          sr[k] += term((k < cut ? e0[u] : e1[u]) * v[u][k]);
-          sb[k] += o[u][k];
-        }
-    }
+    };
+    rows(0, num_dst, std::true_type{});
+    rows(num_dst, num_src, std::false_type{});
 #pragma unroll
     for (int k = 0; k < VEC; ++k) {
       s_sum[k][threadIdx.x] = sl[k];
@@ -575,24 +603,30 @@ __global__ __launch_bounds__(kAggBlock) void gat_param_grad_kernel(const T* __re
   }
 }
 
-static int64_t param_blocks(int64_t num_src) { return std::min<int64_t>(std::max<int64_t>(ceil_div(num_src, 64), 1), kParamBlocks); }
+static int64_t param_blocks(int64_t num_src) { return std::min<int64_t>(std::max<int64_t>(ceil_div(num_src, 16), 1), kParamBlocks); }
 
 template <typename T>
 static void launch_param_grad(const void* ft, const void* d_out, const float* d_el, const float* d_er, int64_t num_src,
                               int64_t num_dst, int heads, int64_t dim, float* part, ParamVec attn_l, hipStream_t st) {
-  const int64_t blocks = param_blocks(num_src), rows = ceil_div(num_src, blocks), row_len = heads * dim;
+  const int64_t blocks = param_blocks(num_src), row_len = heads * dim;
   const bool aligned = ((reinterpret_cast<uintptr_t>(ft) | reinterpret_cast<uintptr_t>(d_out)) & 15) == 0;
   constexpr int kWide = 16 / sizeof(T);
   const int vec = aligned && row_len % kWide == 0 && dim >= kWide ? kWide : aligned && row_len % 4 == 0 && dim >= 4 ? 4 : 1;
   int lanes = 8;
   while (lanes < kAggBlock && lanes * vec < row_len) lanes <<= 1;
   const dim3 grid(static_cast<unsigned>(blocks)), block(kAggBlock);
-#define APT_PARAM(V)                                                                                               \
-  hipLaunchKernelGGL((gat_param_grad_kernel<T, V>), grid, block, 0, st, static_cast<const T*>(ft),                  \
-                     static_cast<const T*>(d_out), d_el, d_er, num_src, num_dst, heads, dim, lanes, rows, part, attn_l)
-  if (vec == kWide) APT_PARAM(kWide);
-  else if (vec == 4) APT_PARAM(4);
-  else APT_PARAM(1);
+#define APT_PARAM(R, V)                                                                                            \
+  hipLaunchKernelGGL((gat_param_grad_kernel<R, V>), grid, block, 0, st, static_cast<const T*>(ft),                  \
+                     static_cast<const T*>(d_out), d_el, d_er, num_src, num_dst, heads, dim, lanes, part, attn_l)
+  if (vec == kWide) {
+    if (dim % kWide == 0) APT_PARAM(T, kWide);
+    else APT_PARAM(TwoHeads<T>, kWide);
+  } else if (vec == 4) {
+    if (dim % 4 == 0) APT_PARAM(T, 4);
+    else APT_PARAM(TwoHeads<T>, 4);
+  } else {
+    APT_PARAM(T, 1);
+  }
 #undef APT_PARAM
 }
 
