@@ -503,8 +503,9 @@ static void launch_gat_source_t(const GatSourceParams& p, int64_t num_edges, hip
 // ------------------------------------------------------------------ backward, parameters
 // Column sums over the rows: a thread has VEC columns of every so many-th row, first of those that are destinations too,
 // then of the others, which have nothing but ft.  Bound by reading ft and d_out once; kUnroll rows of a lane group are on
-// their way (loads outside branches: a conversion inside one waits for its load).  99 k rows of 4 x 64 bf16, 19 k of them
-// destinations: PARAM_US us with the sum of the partials, 40 with the loads in branches and rows in one piece per workgroup.
+// their way (loads outside branches: a conversion inside one waits for its load).  124 k rows of 4 x 64 bf16, 19 k of
+// them destinations: 22 us (73 MB), 33 with the loads in branches and the rows in one
+// piece per workgroup.
 // TwoHeads: a lane's features may belong to two heads.
 constexpr int kParamBlocks = 512;
 
