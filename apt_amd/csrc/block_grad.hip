@@ -4,10 +4,15 @@
 //
 // A lane group owns a source row, so every row is written once, in its own type, whole and in a fixed order: no
 // zero-fill, no atomics, no fp32 copy of a bf16 result.  Nearly all sources of a sampled block have one or two edges;
-// two rows per group are in flight.  The few hubs (hundreds of edges) would each occupy one group for the length of
-// the launch: rows longer than kHubEdges are put aside and added up by all groups of the workgroup afterwards.  Hubs
-// have neighbouring ids (the relabel numbers nodes by first occurrence), so a workgroup's rows are taken a grid apart.
-// Rows that are too long for one workgroup as well are cut into chunks (long_rows.hpp).
+// two rows per group are looked up at once.  Rows longer than kHubEdges are put aside: the shorter of them are added up
+// by a group each afterwards, the longer by all groups of the workgroup.  Hubs have neighbouring ids (the relabel numbers
+// nodes by first occurrence), so a group's rows are taken a grid apart.  Rows that are too long for one workgroup as well
+// are cut into chunks (long_rows.hpp).
+//
+// Bound by rows of dz that come from beyond the L2 (300 MB for 123 k rows of 256 fp32 and 249 k edges, 4.6 TB/s), hence
+// group_row.  Sum with the ordering of the edges, before (rows dealt to the XCDs one by one, every hub to a whole
+// workgroup, bf16 rows converted where they were loaded) / now, us: 238 k sources 733 k edges 256 fp32 240 / 206, 256 bf16
+// 206 / 145, 64 bf16 212 / 145, 47 bf16 202 / 134; 123 k sources 249 k edges 97 / 92, 106 / 79, 103 / 82, 88 / 72.
 #include <algorithm>
 
 #include "common.hpp"
@@ -17,7 +22,11 @@
 namespace apt {
 
 constexpr int kHubEdges = 16;
-constexpr int kHubList = 1024;             // rows of a workgroup at the most, so its list of hubs never overflows
+// Edges of a hub that one lane group adds up by itself: with 128 instead of 32 a hub of 100 edges is the tail of a launch
+// (54 k sources, 256 fp32: 36 us instead of 27), with 32 instead of 128 the 32 groups of a workgroup meet for a few edges
+// each (238 k sources, 64 bf16, with the ordering: 204 us instead of 145).
+template <int LPR> constexpr int hub_shared() { return LPR <= 8 ? 128 : 32; }
+constexpr int kHubList = 1024;             // more than a workgroup has rows, so its list of hubs never overflows
 constexpr int kSourceBlocks = 2048;
 constexpr int kLongBlocks = 512;           // (without a long row the launch takes 3 us)
 
@@ -37,6 +46,35 @@ struct SourceSumParams {
   LongRows lng;
 };
 
+// First row of a lane group.  The groups that work side by side on one XCD (workgroups eight apart) take 64 neighbouring
+// rows: the relabel numbers sources by their first destination, so rows next to each other read the same rows of dz, and
+// that XCD's L2 has them.  (num_src rows are taken a grid apart: hubs have neighbouring ids too.)
+constexpr int kSlab = 64;
+template <int GROUPS> __host__ __device__ constexpr int slab_blocks() { return kSlab / GROUPS; }
+template <int GROUPS> __device__ __forceinline__ int64_t group_row(int grp) {
+  const uint32_t per = 8 * slab_blocks<GROUPS>();
+  const uint32_t whole = gridDim.x / per * per, b = blockIdx.x;
+  if (b >= whole) return static_cast<int64_t>(b) * GROUPS + grp;   // what is left of the grid: in a row
+  const uint32_t xcd = b % 8, j = b / 8;                           // the j-th workgroup of the XCD
+  return (static_cast<int64_t>(j / slab_blocks<GROUPS>()) * 8 + xcd) * kSlab + grp * slab_blocks<GROUPS>() + j % slab_blocks<GROUPS>();
+}
+
+// A value of lane `lane` of the group; a whole wavefront's is the same in all lanes and stands in a scalar register.
+template <int LPR> __device__ __forceinline__ int group_read(int v, int lane) {
+  if constexpr (LPR == kWave) return __builtin_amdgcn_readlane(v, lane);
+  else return __shfl(v, lane, LPR);
+}
+template <int LPR> __device__ __forceinline__ uint32_t group_read(uint32_t v, int lane) {
+  return static_cast<uint32_t>(group_read<LPR>(static_cast<int>(v), lane));
+}
+template <int LPR> __device__ __forceinline__ float group_read(float v, int lane) {
+  return __int_as_float(group_read<LPR>(__float_as_int(v), lane));
+}
+template <int LPR> __device__ __forceinline__ int64_t group_read(int64_t v, int lane) {
+  const uint32_t lo = group_read<LPR>(static_cast<uint32_t>(v), lane), hi = group_read<LPR>(static_cast<uint32_t>(v >> 32), lane);
+  return static_cast<int64_t>(static_cast<uint64_t>(hi) << 32 | lo);
+}
+
 // I: int64_t = a block's CSR (offsets, destinations), uint32_t = apt_block_transpose (offsets, slots).
 // LONG: the long rows alone, a launch after the one that takes all others (in one kernel with them, the compiler makes the
 // loop over the rows 18 % slower: 282 us instead of 239 for 500 k rows of 256 fp32).
@@ -45,8 +83,9 @@ __global__ __launch_bounds__(kAggBlock) void source_sum_kernel(SourceSumParams p
   constexpr int kGroups = kAggBlock / LPR;
   constexpr int kRows = 2;
   constexpr int kUnroll = 4;
+  constexpr int kChunk = LPR < 32 ? LPR : 32;   // edges of a hub that are looked up at once
   __shared__ int s_hub[LONG ? 1 : kHubList];
-  __shared__ int s_hubs;
+  __shared__ int s_hubs[2];
   __shared__ float s_sum[kGroups][LPR * VEC];
   __shared__ uint32_t s_wave[kAggWaves], s_where[2];   // LONG
   const int grp = threadIdx.x / LPR, l = threadIdx.x % LPR;
@@ -59,7 +98,7 @@ __global__ __launch_bounds__(kAggBlock) void source_sum_kernel(SourceSumParams p
     chunks.number(s_wave);
     if (blockIdx.x >= chunks.all) return;
   } else {
-    if (threadIdx.x == 0) s_hubs = 0;
+    if (threadIdx.x == 0) s_hubs[0] = s_hubs[1] = 0;
     __syncthreads();
   }
   struct Edge {      // lane j of a group: edge j of the row
@@ -82,42 +121,43 @@ __global__ __launch_bounds__(kAggBlock) void source_sum_kernel(SourceSumParams p
     return e;
   };
   const T* edata = static_cast<const T*>(p.edata);
-  // acc += the rows of up to LPR edges that the group's lanes hold
-  auto add_edges = [&](const Edge& my, int n, int64_t c, bool live, float (&acc)[VEC]) {
-    for (int e0 = 0; e0 < n; e0 += kUnroll) {
-      float v[kUnroll][VEC];
+  // acc += the rows of edges from .. n - 1 that the group's lanes hold, kUnroll on their way at once.  What is loaded in a
+  // branch is converted behind all of them: a conversion inside one waits for its load.
+  auto walk = [&](const Edge& my, int from, int n, int64_t c, bool live, float (&acc)[VEC]) {
+    for (int e0 = from; e0 < n; e0 += kUnroll) {
+      Row<T, VEC> v[kUnroll], m[EDATA ? kUnroll : 1];
       float w[kUnroll];
+      bool ok[kUnroll];
 #pragma unroll
       for (int u = 0; u < kUnroll; ++u) {
-#pragma unroll
-        for (int k = 0; k < VEC; ++k) v[u][k] = 0.f;
+        ok[u] = false;
         w[u] = 0.f;
-        if (e0 + u < n) {
-          const int64_t d = __shfl(my.dst, e0 + u, LPR);
-          w[u] = __shfl(my.scale, e0 + u, LPR);
-          const uint32_t slot = EDATA ? __shfl(my.slot, e0 + u, LPR) : 0u;
-          if (d >= 0 && live) {
-            load_vec<T, VEC>(dz, d * p.dim + c, v[u]);
-            if constexpr (EDATA) {
-              float m[VEC];
-              load_vec<T, VEC>(edata, static_cast<int64_t>(slot) * p.dim + c, m);
-#pragma unroll
-              for (int k = 0; k < VEC; ++k) v[u][k] *= m[k];
-            }
-          }
+        if (e0 + u < n) {   // group-uniform
+          const int64_t d = group_read<LPR>(my.dst, e0 + u);
+          w[u] = group_read<LPR>(my.scale, e0 + u);
+          ok[u] = d >= 0;
+          v[u] = load_row<T, VEC>(dz, (d >= 0 ? d * p.dim : 0) + (live ? c : 0));
+          if constexpr (EDATA)
+            m[u] = load_row<T, VEC>(edata, static_cast<int64_t>(group_read<LPR>(my.slot, e0 + u)) * p.dim + (live ? c : 0));
         }
       }
 #pragma unroll
-      for (int u = 0; u < kUnroll; ++u)
+      for (int u = 0; u < kUnroll; ++u) {
+        if (!ok[u]) continue;
 #pragma unroll
-        for (int k = 0; k < VEC; ++k) acc[k] += w[u] * v[u][k];
+        for (int k = 0; k < VEC; ++k) {
+          float f = row_elem<T, VEC>(v[u], k);
+          if constexpr (EDATA) f *= row_elem<T, VEC>(m[u], k);
+          acc[k] += w[u] * f;
+        }
+      }
     }
   };
   // acc += the edges [lo, hi), every kGroups-th by this group
   auto add_span = [&](int64_t lo, int64_t hi, int64_t c, bool live, float (&acc)[VEC]) {
     for (int64_t e = lo + grp; e < hi; e += kAggBlock) {
       const int64_t at = e + static_cast<int64_t>(l) * kGroups;
-      add_edges(edge(at, at < hi), static_cast<int>(min((hi - e + kGroups - 1) / kGroups, static_cast<int64_t>(LPR))), c, live, acc);
+      walk(edge(at, at < hi), 0, static_cast<int>(min((hi - e + kGroups - 1) / kGroups, static_cast<int64_t>(LPR))), c, live, acc);
     }
   };
   // The groups' sums together, in order, for the first group.
@@ -169,7 +209,7 @@ __global__ __launch_bounds__(kAggBlock) void source_sum_kernel(SourceSumParams p
     return;
   }
   const int64_t row_groups = static_cast<int64_t>(gridDim.x) * kGroups;
-  for (int64_t r0 = static_cast<int64_t>(grp) * gridDim.x + blockIdx.x; r0 < p.num_src; r0 += kRows * row_groups) {
+  for (int64_t r0 = group_row<kGroups>(grp); r0 < p.num_src; r0 += kRows * row_groups) {
     int64_t lo[kRows];
     int n[kRows];
 #pragma unroll
@@ -195,9 +235,9 @@ __global__ __launch_bounds__(kAggBlock) void source_sum_kernel(SourceSumParams p
         float acc[VEC];
 #pragma unroll
         for (int k = 0; k < VEC; ++k) acc[k] = 0.f;
-        add_edges(first[q], min(n[q], LPR), c, live, acc);
+        walk(first[q], 0, min(n[q], LPR), c, live, acc);
         for (int e = LPR; e < n[q]; e += LPR)   // LPR < kHubEdges only
-          add_edges(edge(lo[q] + e + l, e + l < n[q]), min(n[q] - e, LPR), c, live, acc);
+          walk(edge(lo[q] + e + l, e + l < n[q]), 0, min(n[q] - e, LPR), c, live, acc);
         if (live) {
 #pragma unroll
           for (int k = 0; k < VEC; ++k) acc[k] *= p.scale;
@@ -207,13 +247,45 @@ __global__ __launch_bounds__(kAggBlock) void source_sum_kernel(SourceSumParams p
     }
 #pragma unroll
     for (int q = 0; q < kRows; ++q)
-      if (n[q] > kHubEdges && l == 0 && (p.lng.slots == 0 || n[q] <= static_cast<int>(p.lng.longer)))
-        s_hub[atomicAdd(&s_hubs, 1)] = static_cast<int>(r0 + q * row_groups);
+      if (n[q] > kHubEdges && l == 0 && (p.lng.slots == 0 || n[q] <= static_cast<int>(p.lng.longer))) {
+        if (n[q] <= hub_shared<LPR>()) s_hub[atomicAdd(&s_hubs[0], 1)] = static_cast<int>(r0 + q * row_groups);
+        else s_hub[kHubList - 1 - atomicAdd(&s_hubs[1], 1)] = static_cast<int>(r0 + q * row_groups);
+      }
   }
   __syncthreads();
-  const int hubs = s_hubs;
-  for (int i = 0; i < hubs; ++i) {   // (in any order: every hub is summed on its own)
+  // (in any order: every hub is summed on its own)
+  const int hubs = s_hubs[0], shared = s_hubs[1];
+  for (int i = grp; i < hubs; i += kGroups) {
     const int64_t r = s_hub[i];
+    const int64_t lo = static_cast<int64_t>(indptr[r]);
+    const int n = static_cast<int>(static_cast<int64_t>(indptr[r + 1]) - lo);
+    for (int64_t c0 = 0; c0 < p.dim; c0 += LPR * VEC) {
+      const int64_t c = c0 + static_cast<int64_t>(l) * VEC;
+      const bool live = c < p.dim;
+      float acc[VEC];
+#pragma unroll
+      for (int k = 0; k < VEC; ++k) acc[k] = 0.f;
+      for (int k0 = 0; k0 < n; k0 += kChunk) {
+        const Edge my = edge(lo + k0 + l, l < kChunk && k0 + l < n);
+#pragma unroll 1
+        for (int e = 0; e < min(n - k0, kChunk); e += kHubEdges) {   // one rounding of the long sum for each of these
+          float run[VEC];
+#pragma unroll
+          for (int k = 0; k < VEC; ++k) run[k] = 0.f;
+          walk(my, e, min(min(n - k0, kChunk), e + kHubEdges), c, live, run);
+#pragma unroll
+          for (int k = 0; k < VEC; ++k) acc[k] += run[k];
+        }
+      }
+      if (live) {
+#pragma unroll
+        for (int k = 0; k < VEC; ++k) acc[k] *= p.scale;
+        store_vec<T, VEC>(dx, r * p.dim + c, acc);
+      }
+    }
+  }
+  for (int i = 0; i < shared; ++i) {
+    const int64_t r = s_hub[kHubList - 1 - i];
     const int64_t lo = static_cast<int64_t>(indptr[r]), hi = static_cast<int64_t>(indptr[r + 1]);
     for (int64_t c0 = 0; c0 < p.dim; c0 += LPR * VEC) {
       const int64_t c = c0 + static_cast<int64_t>(l) * VEC;
@@ -240,7 +312,7 @@ static void launch_source_sum(const SourceSumParams& p, int64_t num_edges, hipSt
 #define APT_SOURCE_SUM(LPR)                                                                                        \
   do {                                                                                                            \
     constexpr int64_t groups = kAggBlock / LPR;                                                                    \
-    const int64_t blocks = std::max(ceil_div(p.num_src, kHubList),                                                \
+    const int64_t blocks = std::max(ceil_div(p.num_src, kHubList / 2),                                            \
                                     std::min<int64_t>(std::max(ceil_div(p.num_src, groups * 2),                   \
                                                                std::min(p.num_src, num_edges / (groups * kHubEdges))), \
                                                       kSourceBlocks));                                            \

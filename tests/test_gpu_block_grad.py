@@ -138,3 +138,33 @@ def test_block_aggregate_empty_and_wrong_inputs():
         op(rel.cpu(), 3, 2, x, True, None, None)
     with pytest.raises(RuntimeError):
         op(rel, 4, 2, x, True, None, None)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("dim", [16, 47, 64, 128, 256, 300])
+@pytest.mark.parametrize("num_src", [40, 1100, 9000])
+def test_hubs_of_every_class(dim, dtype, num_src):
+    """Sources of 0 .. 600 edges around the lengths where another part of the kernel takes them (16, 32, 128 edges, 512 of a
+    long row), side by side, in launches with and without a whole slab of neighbouring rows for every XCD."""
+    import apt_amd  # noqa: F401  (loads the operators)
+    gen = torch.Generator(device=DEV).manual_seed(dim + num_src)
+    degrees = [0, 1, 2, 4, 5, 15, 16, 17, 18, 31, 32, 33, 47, 63, 64, 65, 127, 128, 129, 200, 513, 600]
+    slots = torch.cat([torch.full((n,), i * 7 % num_src if num_src > 154 else i, dtype=torch.int64) for i, n in enumerate(degrees)]
+                      + [torch.arange(num_src, dtype=torch.int64), torch.full((3,), -1, dtype=torch.int64)]).to(DEV)
+    fanout = 10
+    num_dst = -(-slots.numel() // fanout)
+    slots = torch.nn.functional.pad(slots, (0, num_dst * fanout - slots.numel()), value=-1)
+    slots = slots[torch.randperm(slots.numel(), generator=gen, device=DEV)].contiguous()
+    x = torch.randn(num_src, dim, generator=gen, device=DEV).to(dtype).requires_grad_(True)
+    up = torch.randn(num_dst, dim, generator=gen, device=DEV).to(dtype)
+    got, = torch.autograd.grad(torch.ops.npc.block_aggregate(slots, num_dst, fanout, x, True, None, None), x, up)
+    there = slots.view(num_dst, fanout) >= 0
+    weighted = up.double() / there.sum(1, keepdim=True).clamp(min=1)
+    edge = there.nonzero()[:, 0], slots[slots >= 0]
+    want = torch.zeros(num_src, dim, dtype=torch.float64, device=DEV).index_add_(0, edge[1], weighted[edge[0]])
+    size = torch.zeros_like(want).index_add_(0, edge[1], weighted[edge[0]].abs())
+    # fp32 sums of n terms in any order: n 2^-24 of the terms' absolute sum, one rounding more for the factor of each; a
+    # bf16 result is rounded at 2^-9
+    count = torch.bincount(edge[1], minlength=num_src).unsqueeze(1)
+    bound = (count + 3) * 2.0 ** -24 * size + (2.0 ** -8 if dtype == torch.bfloat16 else 0.0) * want.abs()
+    assert got.dtype == dtype and bool(((got.double() - want).abs() <= bound).all())
