@@ -17,16 +17,13 @@
 
 #include "common.hpp"
 #include "feature_rows.hpp"
+#include "grouped_rows.hpp"
 #include "long_rows.hpp"
 
 namespace apt {
 
 constexpr int kHubEdges = 16;
-// Edges of a hub that one lane group adds up by itself: with 128 instead of 32 a hub of 100 edges is the tail of a launch
-// (54 k sources, 256 fp32: 36 us instead of 27), with 32 instead of 128 the 32 groups of a workgroup meet for a few edges
-// each (238 k sources, 64 bf16, with the ordering: 204 us instead of 145).
-template <int LPR> constexpr int hub_shared() { return LPR <= 8 ? 128 : 32; }
-constexpr int kHubList = 1024;             // more than a workgroup has rows, so its list of hubs never overflows
+constexpr int kHubList = 1024;             // rows of a workgroup at the most, so its list of hubs never overflows
 constexpr int kSourceBlocks = 2048;
 constexpr int kLongBlocks = 512;           // (without a long row the launch takes 3 us)
 
@@ -45,19 +42,6 @@ struct SourceSumParams {
   void* dx;                // [num_src, dim]
   LongRows lng;
 };
-
-// First row of a lane group.  The groups that work side by side on one XCD (workgroups eight apart) take 64 neighbouring
-// rows: the relabel numbers sources by their first destination, so rows next to each other read the same rows of dz, and
-// that XCD's L2 has them.  (num_src rows are taken a grid apart: hubs have neighbouring ids too.)
-constexpr int kSlab = 64;
-template <int GROUPS> __host__ __device__ constexpr int slab_blocks() { return kSlab / GROUPS; }
-template <int GROUPS> __device__ __forceinline__ int64_t group_row(int grp) {
-  const uint32_t per = 8 * slab_blocks<GROUPS>();
-  const uint32_t whole = gridDim.x / per * per, b = blockIdx.x;
-  if (b >= whole) return static_cast<int64_t>(b) * GROUPS + grp;   // what is left of the grid: in a row
-  const uint32_t xcd = b % 8, j = b / 8;                           // the j-th workgroup of the XCD
-  return (static_cast<int64_t>(j / slab_blocks<GROUPS>()) * 8 + xcd) * kSlab + grp * slab_blocks<GROUPS>() + j % slab_blocks<GROUPS>();
-}
 
 // A value of lane `lane` of the group; a whole wavefront's is the same in all lanes and stands in a scalar register.
 template <int LPR> __device__ __forceinline__ int group_read(int v, int lane) {
@@ -312,7 +296,7 @@ static void launch_source_sum(const SourceSumParams& p, int64_t num_edges, hipSt
 #define APT_SOURCE_SUM(LPR)                                                                                        \
   do {                                                                                                            \
     constexpr int64_t groups = kAggBlock / LPR;                                                                    \
-    const int64_t blocks = std::max(ceil_div(p.num_src, kHubList / 2),                                            \
+    const int64_t blocks = std::max(ceil_div(p.num_src, kHubList),                                                \
                                     std::min<int64_t>(std::max(ceil_div(p.num_src, groups * 2),                   \
                                                                std::min(p.num_src, num_edges / (groups * kHubEdges))), \
                                                       kSourceBlocks));                                            \

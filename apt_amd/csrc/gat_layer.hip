@@ -18,6 +18,7 @@
 
 #include "common.hpp"
 #include "feature_rows.hpp"
+#include "grouped_rows.hpp"
 #include "long_rows.hpp"
 #include "partial_sums.hpp"
 
@@ -215,17 +216,20 @@ struct GatSourceParams {
 // Nearly all sources have one or two edges, so a row is a chain of three dependent reads (offsets, edges, rows of the
 // destinations) and little else: a group has kRows rows in flight with their first edges, loads stand outside branches
 // (a conversion inside one waits for its load), and what depends on the columns alone (heads, parameters) is taken out
-// of the loop over the rows.  124 k rows of 4 x 64 bf16, 261 k edges: 68 us; 193 us with a wavefront per row, loads in
-// branches and the heads worked out per row (63 MB written, 134 MB of destinations' rows read from the caches).
+// of the loop over the rows.  Rows and hubs are dealt as in block_grad.hip (grouped_rows.hpp).  124 k rows of 4 x 64 bf16,
+// 261 k edges (63 MB written, 134 MB of destinations' rows read): 61 us; 72 with four rows in flight (161 registers
+// instead of 111), neighbouring rows on different XCDs and every hub a workgroup's; 193 with a wavefront per row, loads in
+// branches and the heads worked out per row.
 // TWO: a lane's features may belong to two heads.
 template <typename T, int VEC, int LPR, typename I, bool TWO>
 __global__ __launch_bounds__(kAggBlock) void gat_source_kernel(GatSourceParams p) {
   constexpr int kGroups = kAggBlock / LPR;
-  constexpr int kRows = 4;     // rows of a group in flight,
+  constexpr int kRows = 2;     // rows of a group in flight,
   constexpr int kHead = 2;     // with their first edges
+  constexpr int kChunk = LPR < 32 ? LPR : 32;   // edges of a hub that are looked up at once
   constexpr int kUnroll = 4;
-  __shared__ int s_hub[kGatHubList];
-  __shared__ int s_hubs;
+  __shared__ int s_hub[kGatHubList];   // short hubs from the front, longer ones from the back
+  __shared__ int s_hubs[2];
   __shared__ float s_sum[kGroups][LPR * (VEC + 2)];
   __shared__ uint32_t s_wave[kAggWaves], s_where[2];
   const int grp = threadIdx.x / LPR, l = threadIdx.x % LPR;
@@ -235,7 +239,7 @@ __global__ __launch_bounds__(kAggBlock) void gat_source_kernel(GatSourceParams p
   T* d_ft = static_cast<T*>(p.d_ft);
   const int64_t row_len = p.heads * p.dim;
   const Terms<T> term(p.attn_l);
-  if (threadIdx.x == 0) s_hubs = 0;
+  if (threadIdx.x == 0) s_hubs[0] = s_hubs[1] = 0;
   __syncthreads();
   struct Cols {
     int64_t c;
@@ -369,7 +373,7 @@ __global__ __launch_bounds__(kAggBlock) void gat_source_kernel(GatSourceParams p
   const int64_t row_groups = static_cast<int64_t>(gridDim.x) * kGroups;
   for (int64_t c0 = 0; c0 < row_len; c0 += LPR * VEC) {
     const Cols col = columns(c0);
-    for (int64_t r0 = static_cast<int64_t>(grp) * gridDim.x + blockIdx.x; r0 < p.num_src; r0 += kRows * row_groups) {
+    for (int64_t r0 = group_row<kGroups>(grp); r0 < p.num_src; r0 += kRows * row_groups) {
       int64_t lo[kRows], hi[kRows], dst[kRows], weight[kRows];
       int n[kRows];     // edges; a hub's are left for later
 #pragma unroll
@@ -392,8 +396,10 @@ __global__ __launch_bounds__(kAggBlock) void gat_source_kernel(GatSourceParams p
         const int64_t r = r0 + q * row_groups;
         if (r >= p.num_src) break;
         if (hi[q] - lo[q] > kGatHubEdges) {
-          if (l == 0 && c0 == 0 && (p.lng.slots == 0 || hi[q] - lo[q] <= p.lng.longer))
-            s_hub[atomicAdd(&s_hubs, 1)] = static_cast<int>(r);
+          if (l == 0 && c0 == 0 && (p.lng.slots == 0 || hi[q] - lo[q] <= p.lng.longer)) {
+            if (hi[q] - lo[q] <= hub_shared<LPR>()) s_hub[atomicAdd(&s_hubs[0], 1)] = static_cast<int>(r);
+            else s_hub[kGatHubList - 1 - atomicAdd(&s_hubs[1], 1)] = static_cast<int>(r);
+          }
           continue;
         }
         Acc acc;
@@ -410,9 +416,34 @@ __global__ __launch_bounds__(kAggBlock) void gat_source_kernel(GatSourceParams p
     }
   }
   __syncthreads();
-  const int hubs = s_hubs;
-  for (int i = 0; i < hubs; ++i) {
+  const int hubs = s_hubs[0], shared = s_hubs[1];
+  for (int i = grp; i < hubs; i += kGroups) {
     const int64_t r = s_hub[i];
+    const int64_t lo = static_cast<int64_t>(indptr[r]), hi = static_cast<int64_t>(indptr[r + 1]);
+    for (int64_t c0 = 0; c0 < row_len; c0 += LPR * VEC) {
+      const Cols col = columns(c0);
+      Acc acc;
+      clear(acc);
+      for (int64_t e = lo; e < hi; e += kChunk) {
+        int64_t d, w;
+        edge_of(l < kChunk ? e + l : hi, hi, d, w);
+        const int n = static_cast<int>(min(hi - e, static_cast<int64_t>(kChunk)));
+#pragma unroll 1
+        for (int f = 0; f < n; f += kGatHubEdges) {   // one rounding of the long sum for each of these
+          Acc run;
+          clear(run);
+          add_edges(d, w, f, min(n, f + kGatHubEdges), col, run);
+#pragma unroll
+          for (int k = 0; k < VEC; ++k) acc.v[k] += run.v[k];
+          acc.el0 += run.el0;
+          acc.el1 += run.el1;
+        }
+      }
+      finish(r, col, acc);
+    }
+  }
+  for (int i = 0; i < shared; ++i) {
+    const int64_t r = s_hub[kGatHubList - 1 - i];
     const int64_t lo = static_cast<int64_t>(indptr[r]), hi = static_cast<int64_t>(indptr[r + 1]);
     for (int64_t c0 = 0; c0 < row_len; c0 += LPR * VEC) {
       const Cols col = columns(c0);
