@@ -148,6 +148,8 @@ SYMBOLS = {
     "apt_add_rows": (_I, [_P, _P, _I64, _I, _I, _P]),
     "apt_rows_gemm_workspace_bytes": (_SZ, [_I64, _I64, _I64]),
     "apt_rows_gemm": (_I, [_P, _I64, _P, _I64, _I64, _P, _I64, _P, _I64, _I64, _I64, _I64, _I64, _P, _I, _I, _P, _P, _SZ, _P]),
+    "apt_rows_product_fits": (_I, [_I64, _I64, _I64, _I64]),
+    "apt_rows_product": (_I, [_P, _I64, _P, _I64, _I64, _P, _I64, _P, _I64, _I64, _I64, _I64, _I64, _P, _I, _I, _P, _P]),
     "apt_linear_wgrad_workspace_bytes": (_SZ, [_I64, _I64, _I64, _I]),
     "apt_linear_wgrad": (_I, [_P, _P, _I64, _I64, _I64, _I, _P, _P, _P, _SZ, _P]),
     "apt_linear_wgrads_workspace_bytes": (_SZ, [C.POINTER(CWgradProduct), _I, _I]),
@@ -1092,11 +1094,14 @@ def linear_wgrads(products):
 
 
 def rows_gemm(x1, w1, x2=None, w2=None, bias=None, out=None, relu=False):
-    """x1 w1^T (+ x2 w2^T on the first rows) (+ bias) in fp32; out: added to.  Weights may have any strides."""
+    """x1 w1^T (+ x2 w2^T on the first rows) (+ bias) in fp32 or bf16; out: added to.  Weights may have any strides (bf16:
+    one of them 1)."""
     x1 = x1.contiguous()
     x2 = None if x2 is None else x2.contiguous()
-    if any(t is not None and (not t.is_cuda or t.dtype != torch.float32) for t in (x1, w1, x2, w2, bias, out)):
-        raise AptError("rows_gemm takes fp32 GPU tensors")
+    dtype = x1.dtype
+    if dtype not in (torch.float32, torch.bfloat16) or any(t is not None and (not t.is_cuda or t.dtype != dtype)
+                                                           for t in (x1, w1, x2, w2, bias, out)):
+        raise AptError("rows_gemm takes fp32 or bf16 GPU tensors")
     m, k1 = x1.shape
     n = w1.shape[0]
     k2, m2 = (0, 0) if x2 is None else (x2.shape[1], x2.shape[0])
@@ -1107,10 +1112,13 @@ def rows_gemm(x1, w1, x2=None, w2=None, bias=None, out=None, relu=False):
     bias = None if bias is None else bias.contiguous()
     accumulate = out is not None
     if out is None:
-        out = torch.empty((m, n), dtype=torch.float32, device=x1.device)
-    need = int(lib().apt_rows_gemm_workspace_bytes(n, k1, k2))
-    ws = torch.empty(max(need, 256), dtype=torch.uint8, device=x1.device)
+        out = torch.empty((m, n), dtype=dtype, device=x1.device)
     s2 = (0, 0) if w2 is None else w2.stride()
-    check(lib().apt_rows_gemm(_ptr(x1), k1, _ptr(w1), w1.stride(0), w1.stride(1), _ptr(x2), k2, _ptr(w2), s2[0], s2[1], m, m2,
-                              n, _ptr(bias), int(accumulate), int(relu), _ptr(out), _ptr(ws), ws.numel(), _stream()))
+    args = (_ptr(x1), k1, _ptr(w1), w1.stride(0), w1.stride(1), _ptr(x2), k2, _ptr(w2), s2[0], s2[1], m, m2, n, _ptr(bias),
+            int(accumulate), int(relu), _ptr(out))
+    if dtype == torch.bfloat16:
+        check(lib().apt_rows_product(*args, _stream()))
+        return out
+    ws = torch.empty(max(int(lib().apt_rows_gemm_workspace_bytes(n, k1, k2)), 256), dtype=torch.uint8, device=x1.device)
+    check(lib().apt_rows_gemm(*args, _ptr(ws), ws.numel(), _stream()))
     return out

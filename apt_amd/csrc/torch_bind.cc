@@ -1020,8 +1020,14 @@ std::tuple<Tensor, Tensor> linear_wgrad(const Tensor& dy, const Tensor& x, bool 
   return {g[0].dw, g[0].db};
 }
 
+// Whether apt_rows_product takes a weight [n, k]: contiguous along a side.
+bool product_takes(const Tensor& w) {
+  const int64_t n = w.size(0), k = w.size(1), sn = w.stride(0), sk = w.stride(1);
+  return (sk == 1 && sn >= k && (n + 256) * sn <= (1 << 30)) || (sn == 1 && sk >= n && (k + 32) * sk <= (1 << 30));
+}
+
 // x w^T (+ x2 w2^T on the first rows) (+ b) with w [n, k] of any strides; `onto`: added to (and returned).  fp32 rows
-// take apt_rows_gemm, bf16 rows, whose products are bound by memory in the library's kernels already, at::mm.
+// take apt_rows_gemm, bf16 rows apt_rows_product.
 Tensor dense(const Tensor& x_in, const Tensor& w, const Tensor& x2_in = Tensor(), const Tensor& w2 = Tensor(),
              const Tensor& b = Tensor(), Tensor onto = Tensor(), bool relu = false) {
   const int64_t m = x_in.size(0), k = x_in.size(1), n = w.size(0);
@@ -1043,20 +1049,32 @@ Tensor dense(const Tensor& x_in, const Tensor& w, const Tensor& x2_in = Tensor()
                         need, stream()));
     return y;
   }
+  if (x_in.scalar_type() == torch::kBFloat16 && apt_rows_product_fits(m, n, k, k2) && product_takes(w) &&
+      (!pair || product_takes(w2)) && (!b.defined() || b.scalar_type() == torch::kBFloat16)) {
+    auto x = x_in.contiguous();
+    Tensor x2 = pair ? x2_in.contiguous() : Tensor(), bias = b.defined() ? b.contiguous() : Tensor();
+    const bool accumulate = onto.defined();
+    auto y = accumulate ? onto : torch::empty({m, n}, x.options());
+    check(apt_rows_product(x.data_ptr(), k, w.data_ptr(), w.stride(0), w.stride(1), pair ? x2.data_ptr() : nullptr, k2,
+                           pair ? w2.data_ptr() : nullptr, pair ? w2.stride(0) : 0, pair ? w2.stride(1) : 0, m, m2, n,
+                           bias.defined() ? bias.data_ptr() : nullptr, accumulate, relu, y.data_ptr(), stream()));
+    return y;
+  }
   Tensor y = at::linear(x_in, w, b.defined() ? std::optional<Tensor>(b) : std::nullopt);
   if (pair) y.narrow(0, 0, m2).addmm_(x2_in, w2.t());
   if (onto.defined()) y = onto.add_(y);
   return relu ? y.relu_() : y;
 }
 
-// Whether a call is part of a training step.  Its fp32 products are the library's: they give the bits of nn.Linear, and a
+// Whether a call is part of a training step.  Its fp32 products are the library's (`exact` below): they give the bits of nn.Linear, and a
 // ReLU whose input changes sign with the last bit (one or two of 10^7) moves a weight's gradient by up to 6e-5.
 template <typename... Tensors>
 bool trains(const Tensors&... t) {
   return torch::GradMode::is_enabled() && (t.requires_grad() || ...);
 }
-Tensor product(bool train, const Tensor& x, const Tensor& w, const Tensor& b = Tensor()) {
-  return train ? at::linear(x, w, b.defined() ? std::optional<Tensor>(b) : std::nullopt)
+bool exact(bool train, const Tensor& x) { return train && x.scalar_type() == torch::kFloat32; }
+Tensor product(bool library, const Tensor& x, const Tensor& w, const Tensor& b = Tensor()) {
+  return library ? at::linear(x, w, b.defined() ? std::optional<Tensor>(b) : std::nullopt)
                : dense(x, w, Tensor(), Tensor(), b);
 }
 
@@ -1075,8 +1093,8 @@ struct BlockLinearFn : public torch::autograd::Function<BlockLinearFn> {
     ctx->save_for_backward({kept_if(w.requires_grad(), x), kept_if(x.requires_grad(), w)});
     ctx->saved_data["kn"] = kn;
     ctx->saved_data["bias"] = b.has_value() && b->requires_grad();
-    if (train && kn) return at::mm(x, w);
-    return product(train, x, kn ? w.t() : w, b.value_or(Tensor()));
+    if (exact(train, x) && kn) return at::mm(x, w);
+    return product(exact(train, x), x, kn ? w.t() : w, b.value_or(Tensor()));
   }
   static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx,
                                                  torch::autograd::variable_list grads) {
@@ -1309,7 +1327,7 @@ struct SageLayerFn : public torch::autograd::Function<SageLayerFn> {
     const Tensor b = bias.value_or(Tensor()), self = x.narrow(0, 0, num_dst);
     const bool first = x.size(1) > w_self.size(0);
     Tensor mean, inv, out;
-    const bool apart = train || x.scalar_type() != torch::kFloat32;   // the products by the library
+    const bool apart = train;   // the products by the library
     if (first) {
       const Tensor base = product(apart, self, w_self, b);
       std::tie(out, inv) = aggregate_forward(relabeled, num_dst, fanout, product(apart, x, w_neigh), true, 1.f, Tensor(), relu,
@@ -1373,8 +1391,7 @@ struct SageLayerFn : public torch::autograd::Function<SageLayerFn> {
       if (want_x)
         dx = first ? dense(dpre, w_neigh.t(), dz, w_self.t()) : [&] {
           Tensor d = spread(dense(dz, w_neigh.t()));
-          if (d.scalar_type() == torch::kFloat32) dense(dz, w_self.t(), Tensor(), Tensor(), Tensor(), d.narrow(0, 0, num_dst));
-          else d.narrow(0, 0, num_dst).addmm_(dz, w_self);
+          dense(dz, w_self.t(), Tensor(), Tensor(), Tensor(), d.narrow(0, 0, num_dst));
           return d;
         }();
     }
@@ -1415,11 +1432,11 @@ struct GcnLayerFn : public torch::autograd::Function<GcnLayerFn> {
                         double left, double right, const std::optional<Tensor>& csr_indptr,
                         const std::optional<Tensor>& csr_indices, bool relu, bool train) {
     const Tensor b = bias.has_value() ? bias->contiguous() : Tensor();
-    const bool exact = train && x.scalar_type() == torch::kFloat32;
-    const Tensor h = exact ? at::mm(left == 1.0 ? x : at::mul(x, left), w) : dense(x, w.t());
+    const bool as_mm = exact(train, x);
+    const Tensor h = as_mm ? at::mm(left == 1.0 ? x : at::mul(x, left), w) : dense(x, w.t());
     const double scale = left * right;
     const Tensor out = std::get<0>(aggregate_forward(relabeled, num_dst, fanout, h, false,
-                                                     static_cast<float>(exact ? right : scale), b, relu));
+                                                     static_cast<float>(as_mm ? right : scale), b, relu));
     ctx->save_for_backward({kept_if(w.requires_grad(), x), kept_if(x.requires_grad(), w), relabeled,
                             csr_indptr.value_or(Tensor()), csr_indices.value_or(Tensor()), relu ? out : Tensor()});
     ctx->saved_data["bias"] = bias.has_value() && bias->requires_grad();

@@ -40,11 +40,9 @@ class BlockAggregate:
 
 def _native_rows(x, weight):
     """Whether the library's products can take x (fp32 or bf16 GPU rows of the weight's dtype; autocast picks dtypes of
-    its own).  A bf16 product without gradients is the same one either way."""
-    if not (x.is_cuda and x.dim() == 2 and x.dtype == weight.dtype and weight.is_cuda and weight.numel() > 0
-            and not torch.is_autocast_enabled("cuda")):
-        return False
-    return x.dtype == torch.float32 or (x.dtype == torch.bfloat16 and torch.is_grad_enabled() and weight.requires_grad)
+    its own)."""
+    return (x.is_cuda and x.dim() == 2 and x.dtype == weight.dtype and x.dtype in (torch.float32, torch.bfloat16)
+            and weight.is_cuda and weight.numel() > 0 and not torch.is_autocast_enabled("cuda"))
 
 
 def _plain(layer):

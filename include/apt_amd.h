@@ -919,6 +919,15 @@ size_t apt_linear_wgrad_workspace_bytes(int64_t m, int64_t n, int64_t k, int ele
 int apt_linear_wgrad(const void* dy, const void* x, int64_t m, int64_t n, int64_t k, int elem_size,
                      void* dw, void* db, void* workspace, size_t workspace_bytes, void* stream);
 
+/* apt_rows_gemm in bf16 (fp32 sums, rounded once where they are stored; accumulate
+ * adds what y holds to the sum).  Weights must be contiguous along one of their
+ * sides; no workspace.  apt_rows_product_fits: 1 if the weights of a column tile
+ * fit LDS (k1 + k2 up to about 1000) and the sizes are in range. */
+int apt_rows_product_fits(int64_t m, int64_t n, int64_t k1, int64_t k2);
+int apt_rows_product(const void* x1, int64_t k1, const void* w1, int64_t w1_stride_n, int64_t w1_stride_k,
+                     const void* x2, int64_t k2, const void* w2, int64_t w2_stride_n, int64_t w2_stride_k,
+                     int64_t m, int64_t m2, int64_t n, const void* bias, int accumulate, int relu, void* y, void* stream);
+
 /* One or two such products (count) of one type in one launch, each with its own
  * rows and sizes.  out [m, n], optional: the result of a ReLU that dy is the
  * gradient of; dy counts where out > 0.  k = 0: the column sums alone (x and dw
