@@ -99,6 +99,72 @@ __device__ __forceinline__ gemm_f32x4 gemm_mfma(gemm_u32x4 a, gemm_u32x4 b, gemm
                                                  0, 0);
 }
 
+// Fragments of rows row0 .. and columns n0 .. with the fp32 instruction.
+template <int MF, int NF>
+__device__ __forceinline__ void gemm_again(const GemmParams& p, int64_t row0, int64_t n0, gemm_f32x4 (&acc)[MF][NF]) {
+  const int l16 = threadIdx.x % 16, group = threadIdx.x % kWave / 16;
+#pragma unroll 1
+  for (int t = 0; t < MF * NF; ++t) {
+    const int m = t / NF, f = t % NF;
+    const int64_t r = row0 + m * 16 + l16, n = n0 + f * 16 + l16;
+    // the operands apart: zeros in the place of a missing second row must not meet an infinite weight
+    gemm_f32x4 c = {0.f, 0.f, 0.f, 0.f}, c2 = {0.f, 0.f, 0.f, 0.f};
+    for (int64_t k0 = 0; k0 < p.k1; k0 += 4) {
+      const int64_t k = k0 + group;
+      const bool in = k < p.k1;
+      c = __builtin_amdgcn_mfma_f32_16x16x4f32(in ? gemm_weight(p, n, k) : 0.f, in && r < p.m ? p.x1[r * p.k1 + k] : 0.f, c, 0, 0, 0);
+    }
+    for (int64_t k0 = 0; k0 < (row0 < p.m2 ? p.k2 : 0); k0 += 4) {
+      const int64_t k = k0 + group;
+      const bool in = k < p.k2;
+      c2 = __builtin_amdgcn_mfma_f32_16x16x4f32(in ? gemm_weight(p, n, p.k1 + k) : 0.f,
+                                                in && r < p.m2 ? p.x2[r * p.k2 + k] : 0.f, c2, 0, 0, 0);
+    }
+    if (r < p.m2) c += c2;
+#pragma unroll
+    for (int mm = 0; mm < MF; ++mm)
+#pragma unroll
+      for (int ff = 0; ff < NF; ++ff)
+        if (mm == m && ff == f) acc[mm][ff] = c;
+  }
+}
+// Row r of fragments of columns n0 ..: a lane has four consecutive columns of each.
+template <int NF>
+__device__ __forceinline__ void gemm_store(const GemmParams& p, int64_t r, int64_t n0, const gemm_f32x4 (&acc)[NF]) {
+  const int group = threadIdx.x % kWave / 16;
+  const bool wide = p.n % 4 == 0;
+  if (r >= p.m) return;
+#pragma unroll
+  for (int f = 0; f < NF; ++f) {
+    const int64_t n = n0 + f * 16 + group * 4;
+    float* out = p.y + r * p.n + n;
+    if (wide) {
+      if (n >= p.n) continue;
+      gemm_f32x4 v = acc[f];
+      if (p.bias != nullptr) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) v[q] += p.bias[n + q];
+      }
+      if (p.accumulate) v += *reinterpret_cast<const gemm_f32x4*>(out);
+      if (p.relu) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) v[q] = relu(v[q]);
+      }
+      *reinterpret_cast<gemm_f32x4*>(out) = v;
+    } else {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        if (n + q >= p.n) continue;
+        float v = acc[f][q];
+        if (p.bias != nullptr) v += p.bias[n + q];
+        if (p.accumulate) v += out[q];
+        if (p.relu) v = relu(v);
+        out[q] = v;
+      }
+    }
+  }
+}
+
 // WN wavefronts side by side along the columns, the others along the rows; MF row fragments (of 16) per wavefront.
 // VEC: rows are read four elements at a time (k1, k2 multiples of four, aligned) or one.
 template <int WN, int MF, int VEC>
@@ -224,70 +290,16 @@ __global__ __launch_bounds__(kGemmBlock, 2) void rows_gemm_kernel(GemmParams p) 
     for (int f = 0; f < kGemmFragsN; ++f)
 #pragma unroll
       for (int q = 0; q < 4; ++q) finite &= __builtin_isfinite(acc[m][f][q]);
-  if (__any(!finite)) {
-#pragma unroll 1
-    for (int t = 0; t < MF * kGemmFragsN; ++t) {
-      const int m = t / kGemmFragsN, f = t % kGemmFragsN;
-      const int64_t r = row0 + (wm * MF + m) * 16 + l16, n = static_cast<int64_t>(frag_n + f) * 16 + l16;
-      // the operands apart: zeros in the place of a missing second row must not meet an infinite weight
-      gemm_f32x4 c = {0.f, 0.f, 0.f, 0.f}, c2 = {0.f, 0.f, 0.f, 0.f};
-      for (int64_t k0 = 0; k0 < p.k1; k0 += 4) {
-        const int64_t k = k0 + group;
-        const bool in = k < p.k1;
-        c = __builtin_amdgcn_mfma_f32_16x16x4f32(in ? gemm_weight(p, n, k) : 0.f, in && r < p.m ? p.x1[r * p.k1 + k] : 0.f, c,
-                                                 0, 0, 0);
-      }
-      for (int64_t k0 = 0; k0 < depth - p.k1; k0 += 4) {
-        const int64_t k = k0 + group;
-        const bool in = k < p.k2;
-        c2 = __builtin_amdgcn_mfma_f32_16x16x4f32(in ? gemm_weight(p, n, p.k1 + k) : 0.f,
-                                                  in && r < p.m2 ? p.x2[r * p.k2 + k] : 0.f, c2, 0, 0, 0);
-      }
-      if (r < p.m2) c += c2;
+  if (__any(!finite)) gemm_again<MF, kGemmFragsN>(p, row0 + wm * MF * 16, static_cast<int64_t>(frag_n) * 16, acc);
 #pragma unroll
-      for (int mm = 0; mm < MF; ++mm)
-#pragma unroll
-        for (int ff = 0; ff < kGemmFragsN; ++ff)
-          if (mm == m && ff == f) acc[mm][ff] = c;
-    }
-  }
-  // A lane has four consecutive columns of row l16 of its fragment.
-  const bool wide = p.n % 4 == 0;
-#pragma unroll
-  for (int m = 0; m < MF; ++m) {
-    const int64_t r = row0 + (wm * MF + m) * 16 + l16;
-    if (r >= p.m) continue;
-#pragma unroll
-    for (int f = 0; f < kGemmFragsN; ++f) {
-      const int64_t n = static_cast<int64_t>(frag_n + f) * 16 + group * 4;
-      float* out = p.y + r * p.n + n;
-      if (wide) {
-        if (n >= p.n) continue;
-        gemm_f32x4 v = acc[m][f];
-        if (p.bias != nullptr) {
-#pragma unroll
-          for (int q = 0; q < 4; ++q) v[q] += p.bias[n + q];
-        }
-        if (p.accumulate) v += *reinterpret_cast<const gemm_f32x4*>(out);
-        if (p.relu) {
-#pragma unroll
-          for (int q = 0; q < 4; ++q) v[q] = relu(v[q]);
-        }
-        *reinterpret_cast<gemm_f32x4*>(out) = v;
-      } else {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          if (n + q >= p.n) continue;
-          float v = acc[m][f][q];
-          if (p.bias != nullptr) v += p.bias[n + q];
-          if (p.accumulate) v += out[q];
-          if (p.relu) v = relu(v);
-          out[q] = v;
-        }
-      }
-    }
-  }
+  for (int m = 0; m < MF; ++m) gemm_store<kGemmFragsN>(p, row0 + (wm * MF + m) * 16 + l16, static_cast<int64_t>(frag_n) * 16, acc[m]);
 }
+
+}  // namespace apt
+
+#include "rows_gemm_resident.hpp"
+
+namespace apt {
 
 // The sum of two products that the library formed, with the ReLU: one pass instead of two.
 template <typename T, int VEC>
@@ -360,6 +372,15 @@ extern "C" int apt_rows_gemm(const float* x1, int64_t k1, const float* w1, int64
   hipStream_t st = static_cast<hipStream_t>(stream);
   GemmParams p{x1, x2, k1, k2, m, k2 > 0 ? m2 : 0, n, {w1, w1_stride_n, w1_stride_k}, {w2, w2_stride_n, w2_stride_k},
                static_cast<const gemm_u32x4*>(workspace), gemm_frags(n), bias, accumulate, relu, y};
+  const int64_t steps1 = ceil_div(k1, kGemmStep), steps2 = m2 > 0 ? ceil_div(k2, kGemmStep) : 0;
+  if (const int nf = resident_columns(m, n, steps1 + steps2)) {
+    ResidentParams q{p, static_cast<int>(steps1), static_cast<int>(steps2), 0, 0};
+    if (nf == 8) launch_resident<8>(q, st);
+    else if (nf == 4) launch_resident<4>(q, st);
+    else launch_resident<2>(q, st);
+    APT_LAUNCH_CHECK("rows_gemm_resident_kernel");
+    return APT_OK;
+  }
   const int steps = static_cast<int>(ceil_div(k1 + k2, kGemmStep));
   hipLaunchKernelGGL(rows_gemm_weights_kernel,
                      dim3(static_cast<unsigned>(ceil_div(static_cast<int64_t>(steps) * p.frags * kWave, kGemmBlock))),

@@ -263,20 +263,20 @@ __global__ __launch_bounds__(kProdBlock, 4) void rows_product_kernel(ProdParams 
   if (at.block >= p.row_blocks) return;
   load(at, x[0]);
   begin();
-  for (;;) {
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const At then = next(at);
-      load(then, x[(u + 1) & 1]);
-      __builtin_amdgcn_sched_barrier(0);   // (those of this chunk are waited for alone)
-      multiply(at, x[u]);
-      if (then.block != at.block) {
-        store(at);
-        if (then.block >= p.row_blocks) return;
-        begin();
-      }
-      at = then;
+  auto turn = [&](ProdRaw<ODD> (&now)[kProdChunk], ProdRaw<ODD> (&ahead)[kProdChunk]) {   // false: that was the last one
+    const At then = next(at);
+    load(then, ahead);
+    __builtin_amdgcn_sched_barrier(0);   // (those of this chunk are waited for alone)
+    multiply(at, now);
+    if (then.block != at.block) {
+      store(at);
+      if (then.block >= p.row_blocks) return false;
+      begin();
     }
+    at = then;
+    return true;
+  };
+  while (turn(x[0], x[1]) && turn(x[1], x[0])) {
   }
 }
 
