@@ -142,6 +142,7 @@ SYMBOLS = {
     "apt_coo_sum": (_I, [_I, _P, _P, _I64, _I, _I, _P, _I64, _P, _I64, _I, _P, _I64, _P, _SZ, _P]),
     "apt_coo_combine": (_I, [_I, _P, _P, _I64, _P, _I64, _P, _I64, _I64, _I, _P, _P, _P, _I, _P, _P]),
     "apt_gat_layer": (_I, [_P, _I64, _I, _P, _I64, _I, _I64, _I, _P, _P, _I, _P, _I, C.c_float, _I, _P, _P, _P, _P, _P]),
+    "apt_gat_layer_infer": (_I, [_P, _I64, _I, _P, _I64, _I, _I64, _I, _P, _P, _I, _P, _I, C.c_float, _P, _P, _P]),
     "apt_gat_layer_backward_workspace_bytes": (_SZ, [_I64, _I, _I64, _I, _I64, _I64]),
     "apt_gat_layer_backward": (_I, [_P, _I64, _I, _P, _I64, _I, _I64, _I, _P, _P, _I, C.c_float, _P, _P, _P, _P, _P, _P, _I, _P,
                                     _P, _I64, _P, _P, _P, _P, _P, _P, _SZ, _P]),

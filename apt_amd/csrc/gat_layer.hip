@@ -27,6 +27,9 @@ namespace apt {
 int gat_block(const char* who, const int64_t* neighbors, int64_t num_dst, const int64_t* num_dst_dev, int fanout,
               const void* ft, int64_t num_src, int heads, int64_t dim, int elem_size, const float* el, const float* er,
               float slope, void* out, bool like_input, float* attn_out, const void* bias, int act, hipStream_t st);
+bool gat_block_scores(const int64_t* neighbors, int64_t num_dst, int fanout, const void* ft, int64_t num_src, int heads,
+                      int64_t dim, int elem_size, const void* attn_l, const void* attn_r, int attn_elem_size, float slope,
+                      void* out, const void* bias, int act, hipStream_t st);
 int gat_edge_grad(const char* who, const int64_t* neighbors, int64_t num_dst, int fanout, const void* ft, int64_t num_src,
                   int heads, int64_t dim, int elem_size, const float* el, const float* er, float slope, const float* attn,
                   const void* d_out, bool like_input, const int64_t* csc_indptr, float* a_edge, float* dz_edge, float* d_er,
@@ -717,6 +720,23 @@ extern "C" int apt_gat_layer(const int64_t* neighbors, int64_t num_dst, int fano
   APT_LAUNCH_CHECK("gat_pair_scores_kernel");
   return gat_block(who, neighbors, num_dst, nullptr, fanout, ft, num_src, heads, dim, elem_size, el, er, negative_slope, out,
                    wide == 0, attn_out, bias, relu, st);
+}
+
+extern "C" int apt_gat_layer_infer(const int64_t* neighbors, int64_t num_dst, int fanout, const void* ft, int64_t num_src,
+                                   int heads, int64_t dim, int elem_size, const void* attn_l, const void* attn_r,
+                                   int attn_elem_size, const float* bias, int relu, float negative_slope, float* scratch,
+                                   float* out, void* stream) {
+  using namespace apt;
+  if (num_dst > 0 && num_dst <= num_src && fanout > 0 && heads > 0 && dim > 0 && (elem_size == 2 || elem_size == 4) &&
+      (attn_elem_size == 2 || attn_elem_size == 4) && neighbors != nullptr && ft != nullptr && attn_l != nullptr &&
+      attn_r != nullptr && out != nullptr &&
+      gat_block_scores(neighbors, num_dst, fanout, ft, num_src, heads, dim, elem_size, attn_l, attn_r, attn_elem_size,
+                       negative_slope, out, bias, relu, static_cast<hipStream_t>(stream))) {
+    APT_LAUNCH_CHECK("gat_ell_scores_kernel");
+    return APT_OK;
+  }
+  return apt_gat_layer(neighbors, num_dst, fanout, ft, num_src, heads, dim, elem_size, attn_l, attn_r, attn_elem_size, bias, relu,
+                       negative_slope, 1, scratch, scratch == nullptr ? nullptr : scratch + num_src * heads, out, nullptr, stream);
 }
 
 extern "C" size_t apt_gat_layer_backward_workspace_bytes(int64_t num_dst, int fanout, int64_t num_src, int heads, int64_t dim,

@@ -414,13 +414,15 @@ __global__ __launch_bounds__(kAggBlock) void gat_scores_vec_kernel(const T* __re
 // GATConv aggregation over a fixed-stride block (gatconv.py:118-126, DGL's
 // u_add_v -> LeakyReLU -> edge_softmax -> u_mul_e + sum): for destination i and
 // head h, e_k = leaky(el[src_k, h] + er[i, h]) over the row's slots, a = softmax(e),
-// out[i, h, :] = sum_k a_k * ft[src_k, h, :].  A lane group owns a destination
-// row (all heads); the softmax runs online over the slots (running maximum,
-// rescaled sum), so a row's features are read once and nothing is written but
-// the result: no per-edge score, exponent or weight arrays, no atomics.
+// out[i, h, :] = sum_k a_k * ft[src_k, h, :].  A thread has VEC features of a destination; the softmax runs online over
+// the slots (running maximum, rescaled sum), so a row's features are read once and nothing is written but
+// the result: no per-edge score, exponent or weight arrays, no atomics.  The lanes need nothing of each other, so the
+// features of all destinations are dealt out in one sequence, and kUnroll slots are on their way (loads outside branches).
+// 1024 destinations of 4 x 47 fp32, 10 slots: 6.3 us; 16.7 with a lane group a destination, which walks over 188
+// features in three turns.
 // OUT: fp32 or the input's type, with the layer's bias (optional, [heads, dim] of OUT) added to the result as it would
 // be stored without one.
-template <typename T, typename OUT, int VEC, int LPR>
+template <typename T, typename OUT, int VEC>
 __global__ __launch_bounds__(kAggBlock) void gat_ell_kernel(const int64_t* __restrict__ nbr, int64_t num_dst,
                                                             const int64_t* num_dst_dev, int fanout,
                                                             const T* __restrict__ ft, int64_t num_src,
@@ -430,39 +432,30 @@ __global__ __launch_bounds__(kAggBlock) void gat_ell_kernel(const int64_t* __res
                                                             OUT* __restrict__ out,
                                                             float* __restrict__ attn_out,
                                                             const OUT* __restrict__ bias, int act) {
-  constexpr int kGroups = kAggBlock / LPR;
   constexpr int kUnroll = 5;
   const int64_t n = actual_count(num_dst, num_dst_dev);
-  const int64_t row_len = static_cast<int64_t>(heads) * dim;
-  const int grp = threadIdx.x / LPR, l = threadIdx.x % LPR;
-  for (int64_t i = static_cast<int64_t>(blockIdx.x) * kGroups + grp; i < n;
-       i += static_cast<int64_t>(gridDim.x) * kGroups) {
+  const int64_t row_len = static_cast<int64_t>(heads) * dim, vecs = row_len / VEC;
+  for (int64_t item = static_cast<int64_t>(blockIdx.x) * kAggBlock + threadIdx.x; item < n * vecs;
+       item += static_cast<int64_t>(gridDim.x) * kAggBlock) {
+    const int64_t i = item / vecs, d = item % vecs * VEC;
     const int64_t* ids = nbr + i * fanout;
-    for (int64_t d = static_cast<int64_t>(l) * VEC; d < row_len; d += LPR * VEC) {
-      const int h = static_cast<int>(d / dim);   // VEC divides dim: a lane's features share a head
-      const float er_i = er[i * heads + h];
-      float acc[VEC];
+    const int h = static_cast<int>(d / dim);   // VEC divides dim: a thread's features share a head
+    const float er_i = er[i * heads + h];
+    float acc[VEC];
 #pragma unroll
-      for (int k = 0; k < VEC; ++k) acc[k] = 0.f;
-      float top = -INFINITY, denom = 0.f;
-      for (int s0 = 0; s0 < fanout; s0 += kUnroll) {
-        float v[kUnroll][VEC];
-        float sc[kUnroll];
-        bool ok[kUnroll];
+    for (int k = 0; k < VEC; ++k) acc[k] = 0.f;
+    float top = -INFINITY, denom = 0.f;
+    for (int s0 = 0; s0 < fanout; s0 += kUnroll) {
+      Row<T, VEC> v[kUnroll];
+      float sc[kUnroll];
+      bool ok[kUnroll];
+      if (num_src > 0) {   // (in the place of a missing row, the first one)
 #pragma unroll
         for (int u = 0; u < kUnroll; ++u) {
-          ok[u] = false;
-          sc[u] = 0.f;
-#pragma unroll
-          for (int k = 0; k < VEC; ++k) v[u][k] = 0.f;
-          if (s0 + u < fanout) {
-            const int64_t src = ids[s0 + u];
-            if (src >= 0 && src < num_src) {
-              ok[u] = true;
-              sc[u] = el[src * heads + h];
-              load_vec<T, VEC>(ft, src * row_len + d, v[u]);
-            }
-          }
+          const int64_t src = ids[min(s0 + u, fanout - 1)];
+          ok[u] = s0 + u < fanout && src >= 0 && src < num_src;
+          sc[u] = el[(ok[u] ? src : 0) * heads + h];
+          v[u] = load_row<T, VEC>(ft, (ok[u] ? src : 0) * row_len + d);
         }
 #pragma unroll
         for (int u = 0; u < kUnroll; ++u) {
@@ -479,29 +472,29 @@ __global__ __launch_bounds__(kAggBlock) void gat_ell_kernel(const int64_t* __res
           const float w = expf(e - top);
           denom += w;
 #pragma unroll
-          for (int k = 0; k < VEC; ++k) acc[k] += w * v[u][k];
+          for (int k = 0; k < VEC; ++k) acc[k] += w * row_elem<T, VEC>(v[u], k);
         }
       }
-      const float inv = denom > 0.f ? 1.0f / denom : 0.f;
+    }
+    const float inv = denom > 0.f ? 1.0f / denom : 0.f;
 #pragma unroll
-      for (int k = 0; k < VEC; ++k) {
-        acc[k] *= inv;
-        if (bias != nullptr) acc[k] = as_stored<OUT>(acc[k]) + to_float<OUT>(bias[d + k]);
-        if (act) acc[k] = relu(acc[k]);
-      }
-      store_vec<OUT, VEC>(out, i * row_len + d, acc);
-      // the lane that holds a head's first features also writes its attention weights
-      if (attn_out != nullptr && d % dim == 0) {
-        for (int s = 0; s < fanout; ++s) {
-          const int64_t src = ids[s];
-          float a = 0.f;
-          if (src >= 0 && src < num_src) {
-            float e = el[src * heads + h] + er_i;
-            e = e > 0.f ? e : e * slope;
-            a = expf(e - top) * inv;
-          }
-          attn_out[(i * fanout + s) * heads + h] = a;
+    for (int k = 0; k < VEC; ++k) {
+      acc[k] *= inv;
+      if (bias != nullptr) acc[k] = as_stored<OUT>(acc[k]) + to_float<OUT>(bias[d + k]);
+      if (act) acc[k] = relu(acc[k]);
+    }
+    store_vec<OUT, VEC>(out, i * row_len + d, acc);
+    // the thread that holds a head's first features also writes its attention weights
+    if (attn_out != nullptr && d % dim == 0) {
+      for (int s = 0; s < fanout; ++s) {
+        const int64_t src = ids[s];
+        float a = 0.f;
+        if (src >= 0 && src < num_src) {
+          float e = el[src * heads + h] + er_i;
+          e = e > 0.f ? e : e * slope;
+          a = expf(e - top) * inv;
         }
+        attn_out[(i * fanout + s) * heads + h] = a;
       }
     }
   }
@@ -600,22 +593,142 @@ static bool launch_gat_wave(const int64_t* nbr, int64_t num_dst, const int64_t* 
   return true;
 }
 
+// The same again with the scores formed where they are used: a layer whose scores nobody needs afterwards (no gradients)
+// saves the pass over all source rows that writes them.  The rows of up to ROWS slots stay in registers between their
+// product with attn_l (summed over the lanes of a head) and the weighted sum; attn_r meets the destination's own row.
+// 26 k destinations of 4 x 64 fp32, 10 slots, 122 k sources: 50 us; 61 in two kernels.
+constexpr int gat_scores_waves(int rows, int elem_size) {   // per SIMD: what the registers allow (bf16 rows are held converted)
+  return rows <= 5 ? 7 : (rows <= 10 ? 5 : 4) - (elem_size == 2 ? 1 : 0);
+}
+template <typename T, typename OUT, typename P, int VEC, int ROWS>
+__global__ __launch_bounds__(kAggBlock, gat_scores_waves(ROWS, sizeof(T))) void gat_ell_scores_kernel(
+    const int64_t* __restrict__ nbr, int64_t num_dst, int fanout, const T* __restrict__ ft, int64_t num_src, int heads,
+    int log2_heads, int64_t dim, const P* __restrict__ attn_l, const P* __restrict__ attn_r, float slope,
+    OUT* __restrict__ out, const OUT* __restrict__ bias, int act) {
+  const int lane = threadIdx.x % kWave;
+  const int lph = static_cast<int>(dim / VEC);
+  const int64_t row_len = static_cast<int64_t>(heads) * dim;
+  const bool live = lane < heads * lph;
+  const int hf = live ? lane / lph : 0;
+  const int64_t d = live ? static_cast<int64_t>(lane) * VEC : 0;
+  const int k = lane >> log2_heads, hs = lane & (heads - 1);
+  const bool slot = k < fanout;
+  float al[VEC], ar[VEC];
+#pragma unroll
+  for (int q = 0; q < VEC; ++q) {
+    al[q] = live ? to_float<P>(attn_l[d + q]) : 0.f;
+    ar[q] = live ? to_float<P>(attn_r[d + q]) : 0.f;
+  }
+  // a row's product with a head's vector, for the lanes of the slot layout that have the head (in gat_pair_scores_kernel's
+  // order and roundings: the layer gives the same bits with and without gradients)
+  auto score = [&](const Row<T, VEC>& row, const float (&w)[VEC]) {
+    float part = 0.f;
+#pragma unroll
+    for (int q = 0; q < VEC; ++q) part = __fadd_rn(part, live ? __fmul_rn(row_elem<T, VEC>(row, q), w[q]) : 0.f);
+    for (int off = lph / 2; off > 0; off >>= 1) part += __shfl_xor(part, off, kWave);
+    return __shfl(part, hs * lph, kWave);
+  };
+  for (int64_t i = static_cast<int64_t>(blockIdx.x) * kAggWaves + threadIdx.x / kWave; i < num_dst;
+       i += static_cast<int64_t>(gridDim.x) * kAggWaves) {
+    const int64_t id = slot ? nbr[i * fanout + k] : -1;
+    const bool valid = id >= 0 && id < num_src;
+    const Row<T, VEC> own = load_row<T, VEC>(ft, i * row_len + d);   // (num_dst <= num_src)
+    Row<T, VEC> v[ROWS];
+    bool ok[ROWS];
+#pragma unroll
+    for (int u = 0; u < ROWS; ++u) {
+      const int64_t src = wave_read(id, min(u, fanout - 1) << log2_heads);
+      ok[u] = u < fanout && src >= 0 && src < num_src;
+      if (ok[u]) v[u] = load_row<T, VEC>(ft, src * row_len + d);     // the same in all lanes; used behind all of them
+    }
+    const float er = score(own, ar);
+    float el = 0.f;
+#pragma unroll
+    for (int u = 0; u < ROWS; ++u) {
+      if (!ok[u]) continue;
+      const float got = score(v[u], al);
+      if (k == u) el = got;
+    }
+    float e = -INFINITY;
+    if (valid) {
+      e = el + er;
+      e = e > 0.f ? e : e * slope;
+    }
+    float top = e;
+    for (int off = heads; off < kWave; off <<= 1) top = fmaxf(top, __shfl_xor(top, off, kWave));
+    const float w = valid ? expf(e - top) : 0.f;
+    float denom = w;
+    for (int off = heads; off < kWave; off <<= 1) denom += __shfl_xor(denom, off, kWave);
+    const float a = denom > 0.f ? w / denom : 0.f;
+    float acc[VEC];
+#pragma unroll
+    for (int q = 0; q < VEC; ++q) acc[q] = 0.f;
+#pragma unroll
+    for (int u = 0; u < ROWS; ++u) {
+      if (!ok[u]) continue;
+      const float au = __shfl(a, (u << log2_heads) + hf, kWave);
+#pragma unroll
+      for (int q = 0; q < VEC; ++q) acc[q] += au * row_elem<T, VEC>(v[u], q);
+    }
+    if (live) {
+      if (bias != nullptr) {
+#pragma unroll
+        for (int q = 0; q < VEC; ++q) acc[q] = as_stored<OUT>(acc[q]) + to_float<OUT>(bias[d + q]);
+      }
+      if (act) {
+#pragma unroll
+        for (int q = 0; q < VEC; ++q) acc[q] = relu(acc[q]);
+      }
+      store_vec<OUT, VEC>(out, i * row_len + d, acc);
+    }
+  }
+}
+
+// Whether it was launched: heads and lanes per head powers of two, heads * fanout slots in a wavefront, as gat_ell_wave_kernel;
+// up to 16 slots (registers).
+template <typename T, typename OUT, typename P>
+static bool launch_gat_scores(const int64_t* nbr, int64_t num_dst, int fanout, const void* ft, int64_t num_src, int heads,
+                              int64_t dim, const void* attn_l, const void* attn_r, float slope, void* out, const void* bias,
+                              int act, hipStream_t st) {
+  constexpr int VEC = 4;
+  const int64_t lph = dim / VEC;
+  if (dim % VEC != 0 || (heads & (heads - 1)) != 0 || heads * fanout > kWave || fanout > 16 || (lph & (lph - 1)) != 0 ||
+      heads * lph > kWave || ((reinterpret_cast<uintptr_t>(ft) | reinterpret_cast<uintptr_t>(out)) & 15) != 0)
+    return false;
+  int log2_heads = 0;
+  while ((1 << log2_heads) < heads) ++log2_heads;
+  const dim3 grid(static_cast<unsigned>(std::min<int64_t>(ceil_div(num_dst, kAggWaves), 1 << 20))), block(kAggBlock);
+#define APT_GAT_SCORES(ROWS)                                                                                              \
+  hipLaunchKernelGGL((gat_ell_scores_kernel<T, OUT, P, VEC, ROWS>), grid, block, 0, st, nbr, num_dst, fanout,             \
+                     static_cast<const T*>(ft), num_src, heads, log2_heads, dim, static_cast<const P*>(attn_l),           \
+                     static_cast<const P*>(attn_r), slope, static_cast<OUT*>(out), static_cast<const OUT*>(bias), act)
+  if (fanout <= 5) APT_GAT_SCORES(5);
+  else if (fanout <= 10) APT_GAT_SCORES(10);
+  else APT_GAT_SCORES(16);
+#undef APT_GAT_SCORES
+  return true;
+}
+
+// A layer's result without the scores beside it; false: not of these shapes or types.
+bool gat_block_scores(const int64_t* neighbors, int64_t num_dst, int fanout, const void* ft, int64_t num_src, int heads,
+                      int64_t dim, int elem_size, const void* attn_l, const void* attn_r, int attn_elem_size, float slope,
+                      void* out, const void* bias, int act, hipStream_t st) {
+#define APT_GAT_SCORES_AS(T, P) \
+  launch_gat_scores<T, float, P>(neighbors, num_dst, fanout, ft, num_src, heads, dim, attn_l, attn_r, slope, out, bias, act, st)
+  if (elem_size == 4) return attn_elem_size == 4 ? APT_GAT_SCORES_AS(float, float) : APT_GAT_SCORES_AS(float, uint16_t);
+  return attn_elem_size == 4 ? APT_GAT_SCORES_AS(uint16_t, float) : APT_GAT_SCORES_AS(uint16_t, uint16_t);
+#undef APT_GAT_SCORES_AS
+}
+
 template <typename T, typename OUT, int VEC>
 static void launch_gat(const int64_t* nbr, int64_t num_dst, const int64_t* num_dst_dev, int fanout,
                        const void* ft, int64_t num_src, int heads, int64_t dim, const float* el,
                        const float* er, float slope, void* out, float* attn_out, const void* bias, int act, hipStream_t st) {
-  const int64_t per_row = ceil_div(static_cast<int64_t>(heads) * dim, VEC);
-  const T* x = static_cast<const T*>(ft);
-#define APT_GAT(LPR)                                                                                  \
-  hipLaunchKernelGGL((gat_ell_kernel<T, OUT, VEC, LPR>),                                              \
-                     dim3(static_cast<unsigned>(std::min<int64_t>(ceil_div(num_dst, kAggBlock / LPR), 1 << 20))), \
-                     dim3(kAggBlock), 0, st, nbr, num_dst, num_dst_dev, fanout, x, num_src, heads, dim, el, er, \
-                     slope, static_cast<OUT*>(out), attn_out, static_cast<const OUT*>(bias), act)
-  if (per_row <= 8) APT_GAT(8);
-  else if (per_row <= 16) APT_GAT(16);
-  else if (per_row <= 32) APT_GAT(32);
-  else APT_GAT(64);
-#undef APT_GAT
+  const int64_t items = num_dst * (heads * dim / VEC);
+  hipLaunchKernelGGL((gat_ell_kernel<T, OUT, VEC>),
+                     dim3(static_cast<unsigned>(std::min<int64_t>(ceil_div(items, kAggBlock), 1 << 20))), dim3(kAggBlock), 0, st,
+                     nbr, num_dst, num_dst_dev, fanout, static_cast<const T*>(ft), num_src, heads, dim, el, er, slope,
+                     static_cast<OUT*>(out), attn_out, static_cast<const OUT*>(bias), act);
 }
 
 // Backward of gat_ell_kernel, edge half.  A wavefront per (destination, head):

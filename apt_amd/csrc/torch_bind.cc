@@ -1538,6 +1538,13 @@ struct GatLayerFn : public torch::autograd::Function<GatLayerFn> {
     Tensor attn;
     if (want_grad) attn = torch::empty({num_dst * fanout, heads}, f32);
     Tensor b = bias.has_value() ? bias->to(out.scalar_type()).contiguous() : Tensor();
+    if (!want_grad && out.scalar_type() == torch::kFloat32) {
+      check(apt_gat_layer_infer(i64(relabeled), num_dst, static_cast<int>(fanout), ft.data_ptr(), n, static_cast<int>(heads), dim,
+                                static_cast<int>(ft.element_size()), attn_l.data_ptr(), attn_r.data_ptr(),
+                                static_cast<int>(attn_l.element_size()), b.defined() ? b.data_ptr<float>() : nullptr, relu,
+                                static_cast<float>(slope), el, out.data_ptr<float>(), stream()));
+      return out;
+    }
     check(apt_gat_layer(i64(relabeled), num_dst, static_cast<int>(fanout), ft.data_ptr(), n, static_cast<int>(heads), dim,
                         static_cast<int>(ft.element_size()), attn_l.data_ptr(), attn_r.data_ptr(),
                         static_cast<int>(attn_l.element_size()), b.defined() ? b.data_ptr() : nullptr, relu,

@@ -896,6 +896,13 @@ int apt_gat_layer(const int64_t* neighbors, int64_t num_dst, int fanout, const v
                   int heads, int64_t dim, int elem_size, const void* attn_l, const void* attn_r,
                   int attn_elem_size, const void* bias, int relu, float negative_slope, int wide, float* el, float* er,
                   void* out, float* attn_out, void* stream);
+/* apt_gat_layer with an fp32 result (wide) whose scores nobody needs afterwards:
+ * formed where they are used where the shape allows it.  scratch: fp32,
+ * (num_src + num_dst) * heads. */
+int apt_gat_layer_infer(const int64_t* neighbors, int64_t num_dst, int fanout, const void* ft, int64_t num_src,
+                        int heads, int64_t dim, int elem_size, const void* attn_l, const void* attn_r,
+                        int attn_elem_size, const float* bias, int relu, float negative_slope, float* scratch,
+                        float* out, void* stream);
 size_t apt_gat_layer_backward_workspace_bytes(int64_t num_dst, int fanout, int64_t num_src, int heads, int64_t dim,
                                               int64_t num_edges);
 int apt_gat_layer_backward(const int64_t* neighbors, int64_t num_dst, int fanout, const void* ft,

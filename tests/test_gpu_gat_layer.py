@@ -152,3 +152,33 @@ def test_gat_layer_sources_with_given_numbers_of_edges(capi, heads, dim, dtype, 
         assert bool((a - b).norm() <= tol * b.norm()), (name, ((a - b).norm() / b.norm()).item())
     for a, b in zip(got, grads()):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("dtype,attn_dtype", [(torch.float32, torch.float32), (torch.float32, torch.bfloat16),
+                                              (torch.bfloat16, torch.bfloat16), (torch.bfloat16, torch.float32)])
+@pytest.mark.parametrize("num_dst,fanout,num_src,heads,dim", [
+    (1, 1, 1, 1, 4), (70, 5, 400, 4, 64), (70, 6, 400, 4, 64), (33, 10, 300, 2, 128), (33, 11, 300, 1, 16), (50, 16, 300, 4, 8),
+    (50, 17, 300, 2, 8), (20, 8, 90, 8, 32), (40, 7, 200, 4, 47), (40, 3, 200, 1, 10)])
+def test_scores_formed_where_they_are_used(capi, num_dst, fanout, num_src, heads, dim, dtype, attn_dtype):
+    """Without gradients: the slots that a wavefront's registers hold (5, 10, 16, and one more), against float64; and fp32
+    with the bits of the layer that has gradients, rows with infinities and NaN included."""
+    import apt_amd  # noqa: F401
+    rng = np.random.default_rng(num_dst * fanout)
+    r = rng.integers(0, num_src, size=num_dst * fanout)
+    r[rng.random(r.size) < 0.25] = -1
+    r[-fanout:] = -1 if num_dst > 1 else 0
+    rel = torch.from_numpy(r.astype(np.int64)).to(DEV)
+    gen = torch.Generator(device=DEV).manual_seed(heads * dim)
+    ft = torch.randn(num_src, heads, dim, generator=gen, device=DEV).to(dtype)
+    al, ar = ((torch.randn(heads, dim, generator=gen, device=DEV) * 0.3).to(attn_dtype) for _ in range(2))
+    bias = torch.randn(heads, dim, generator=gen, device=DEV).to(dtype)
+    got = torch.ops.npc.gat_layer(rel, num_dst, fanout, ft, al, ar, bias, 0.2, None, None, None, None, False, True)
+    want = _separate(rel, num_dst, fanout, ft.double(), al.double(), ar.double(), bias.double(), 0.2)
+    # fp32: dots of up to 128 products move a weight by less than 1e-5, a sum of 16 rows adds 1e-6
+    assert got.dtype == torch.float32 and bool(((got.double() - want).abs() <= 2e-5 * (1 + want.abs().max())).all())
+    if dtype == torch.float32:
+        ft[0, 0, 0], ft[num_src // 2, heads - 1, dim - 1] = float("inf"), float("nan")
+        rest = (al, ar, bias, 0.2, None, None, None, None)
+        plain = torch.ops.npc.gat_layer(rel, num_dst, fanout, ft, *rest)
+        grad = torch.ops.npc.gat_layer(rel, num_dst, fanout, ft.clone().requires_grad_(True), *rest)
+        assert torch.equal(plain.isnan(), grad.isnan()) and torch.equal(plain.nan_to_num(7.0), grad.detach().nan_to_num(7.0))
