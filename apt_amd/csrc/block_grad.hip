@@ -25,7 +25,7 @@ namespace apt {
 constexpr int kHubEdges = 16;
 constexpr int kHubList = 1024;             // rows of a workgroup at the most, so its list of hubs never overflows
 constexpr int kSourceBlocks = 2048;
-constexpr int kLongBlocks = 512;           // (without a long row the launch takes 3 us)
+constexpr int kLongBlocks = 512;           // workgroups for long rows at the most
 
 struct SourceSumParams {
   const void* indptr;      // offsets of the sources in `index`
@@ -41,6 +41,7 @@ struct SourceSumParams {
   int64_t num_src;
   void* dx;                // [num_src, dim]
   LongRows lng;
+  uint32_t row_blocks;     // workgroups for the rows; those behind them take the long ones
 };
 
 // A value of lane `lane` of the group; a whole wavefront's is the same in all lanes and stands in a scalar register.
@@ -60,31 +61,24 @@ template <int LPR> __device__ __forceinline__ int64_t group_read(int64_t v, int 
 }
 
 // I: int64_t = a block's CSR (offsets, destinations), uint32_t = apt_block_transpose (offsets, slots).
-// LONG: the long rows alone, a launch after the one that takes all others (in one kernel with them, the compiler makes the
-// loop over the rows 18 % slower: 282 us instead of 239 for 500 k rows of 256 fp32).
+// LONG: workgroups behind those of the rows take the long rows.
 template <typename T, int VEC, int LPR, typename I, bool EDATA, bool LONG>
 __global__ __launch_bounds__(kAggBlock) void source_sum_kernel(SourceSumParams p) {
   constexpr int kGroups = kAggBlock / LPR;
   constexpr int kRows = 2;
   constexpr int kUnroll = 4;
   constexpr int kChunk = LPR < 32 ? LPR : 32;   // edges of a hub that are looked up at once
-  __shared__ int s_hub[LONG ? 1 : kHubList];
+  __shared__ int s_hub[kHubList];
   __shared__ int s_hubs[2];
   __shared__ float s_sum[kGroups][LPR * VEC];
-  __shared__ uint32_t s_wave[kAggWaves], s_where[2];   // LONG
+  __shared__ uint32_t s_wave[LONG ? kAggWaves : 1], s_where[LONG ? 2 : 1];
   const int grp = threadIdx.x / LPR, l = threadIdx.x % LPR;
   const I* indptr = static_cast<const I*>(p.indptr);
   const I* index = static_cast<const I*>(p.index);
   const T* dz = static_cast<const T*>(p.dz);
   T* dx = static_cast<T*>(p.dx);
-  LongChunks<kAggBlock, I> chunks(p.lng, indptr);
-  if constexpr (LONG) {
-    chunks.number(s_wave);
-    if (blockIdx.x >= chunks.all) return;
-  } else {
-    if (threadIdx.x == 0) s_hubs[0] = s_hubs[1] = 0;
-    __syncthreads();
-  }
+  if (threadIdx.x == 0) s_hubs[0] = s_hubs[1] = 0;
+  __syncthreads();
   struct Edge {      // lane j of a group: edge j of the row
     int64_t dst;     // -1: none
     uint32_t slot;   // EDATA only
@@ -160,8 +154,10 @@ __global__ __launch_bounds__(kAggBlock) void source_sum_kernel(SourceSumParams p
     }
     __syncthreads();
   };
-  if constexpr (LONG) {
-    for (uint32_t q = blockIdx.x; q < chunks.all; q += gridDim.x) {   // block-uniform
+  if (LONG && blockIdx.x >= p.row_blocks) {   // block-uniform
+    LongChunks<kAggBlock, I> chunks(p.lng, indptr);
+    chunks.number(s_wave);
+    for (uint32_t q = blockIdx.x - p.row_blocks; q < chunks.all; q += gridDim.x - p.row_blocks) {
       const auto chunk = chunks.find(q, s_where);
       const float* part = p.lng.part + static_cast<int64_t>(q - chunk.index) * p.dim;   // of the row's chunks
       bool whole = false;
@@ -192,8 +188,8 @@ __global__ __launch_bounds__(kAggBlock) void source_sum_kernel(SourceSumParams p
     }
     return;
   }
-  const int64_t row_groups = static_cast<int64_t>(gridDim.x) * kGroups;
-  for (int64_t r0 = group_row<kGroups>(grp); r0 < p.num_src; r0 += kRows * row_groups) {
+  const int64_t row_groups = static_cast<int64_t>(p.row_blocks) * kGroups;
+  for (int64_t r0 = group_row<kGroups>(grp, p.row_blocks); r0 < p.num_src; r0 += kRows * row_groups) {
     int64_t lo[kRows];
     int n[kRows];
 #pragma unroll
@@ -291,7 +287,7 @@ __global__ __launch_bounds__(kAggBlock) void source_sum_kernel(SourceSumParams p
 // A workgroup for two rows per lane group, or, where rows have many edges, for sixteen edges per lane group (1 M edges of
 // 16 fp32 into 4096 rows: 481 us with the 64 workgroups of the rows alone).
 template <typename T, int VEC, typename I, bool EDATA>
-static void launch_source_sum(const SourceSumParams& p, int64_t num_edges, hipStream_t st) {
+static void launch_source_sum(SourceSumParams p, int64_t num_edges, hipStream_t st) {
   const int64_t per_row = ceil_div(p.dim, VEC);
 #define APT_SOURCE_SUM(LPR)                                                                                        \
   do {                                                                                                            \
@@ -300,12 +296,11 @@ static void launch_source_sum(const SourceSumParams& p, int64_t num_edges, hipSt
                                     std::min<int64_t>(std::max(ceil_div(p.num_src, groups * 2),                   \
                                                                std::min(p.num_src, num_edges / (groups * kHubEdges))), \
                                                       kSourceBlocks));                                            \
-    hipLaunchKernelGGL((source_sum_kernel<T, VEC, LPR, I, EDATA, false>), dim3(static_cast<unsigned>(blocks)),    \
-                       dim3(kAggBlock), 0, st, p);                                                                \
-    if (p.lng.slots > 0)                                                                                          \
-      hipLaunchKernelGGL((source_sum_kernel<T, VEC, LPR, I, EDATA, true>),                                        \
-                         dim3(static_cast<unsigned>(std::min<int64_t>(long_chunks(num_edges), kLongBlocks))),     \
-                         dim3(kAggBlock), 0, st, p);                                                              \
+    const int64_t chunks = p.lng.slots > 0 ? std::min<int64_t>(long_chunks(num_edges), kLongBlocks) : 0;          \
+    p.row_blocks = static_cast<uint32_t>(blocks);                                                                 \
+    const dim3 grid(static_cast<unsigned>(blocks + chunks)), block(kAggBlock);                                    \
+    if (chunks > 0) hipLaunchKernelGGL((source_sum_kernel<T, VEC, LPR, I, EDATA, true>), grid, block, 0, st, p);  \
+    else hipLaunchKernelGGL((source_sum_kernel<T, VEC, LPR, I, EDATA, false>), grid, block, 0, st, p);            \
   } while (0)
   if (per_row <= 8) APT_SOURCE_SUM(8);
   else if (per_row <= 16) APT_SOURCE_SUM(16);

@@ -376,7 +376,7 @@ __global__ __launch_bounds__(kAggBlock) void gat_source_kernel(GatSourceParams p
   const int64_t row_groups = static_cast<int64_t>(gridDim.x) * kGroups;
   for (int64_t c0 = 0; c0 < row_len; c0 += LPR * VEC) {
     const Cols col = columns(c0);
-    for (int64_t r0 = group_row<kGroups>(grp); r0 < p.num_src; r0 += kRows * row_groups) {
+    for (int64_t r0 = group_row<kGroups>(grp, gridDim.x); r0 < p.num_src; r0 += kRows * row_groups) {
       int64_t lo[kRows], hi[kRows], dst[kRows], weight[kRows];
       int n[kRows];     // edges; a hub's are left for later
 #pragma unroll

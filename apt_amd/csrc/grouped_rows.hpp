@@ -10,9 +10,9 @@ namespace apt {
 // that XCD's L2 has them.  (num_src rows are taken a grid apart: hubs have neighbouring ids too.)
 constexpr int kSlab = 64;
 template <int GROUPS> __host__ __device__ constexpr int slab_blocks() { return kSlab / GROUPS; }
-template <int GROUPS> __device__ __forceinline__ int64_t group_row(int grp) {
+template <int GROUPS> __device__ __forceinline__ int64_t group_row(int grp, uint32_t blocks) {   // blocks: of the rows
   const uint32_t per = 8 * slab_blocks<GROUPS>();
-  const uint32_t whole = gridDim.x / per * per, b = blockIdx.x;
+  const uint32_t whole = blocks / per * per, b = blockIdx.x;
   if (b >= whole) return static_cast<int64_t>(b) * GROUPS + grp;   // what is left of the grid: in a row
   const uint32_t xcd = b % 8, j = b / 8;                           // the j-th workgroup of the XCD
   return (static_cast<int64_t>(j / slab_blocks<GROUPS>()) * 8 + xcd) * kSlab + grp * slab_blocks<GROUPS>() + j % slab_blocks<GROUPS>();
