@@ -162,6 +162,7 @@ SYMBOLS = {
     "apt_epoch_release": (_I, [_P, _P]),
     "apt_epoch_end": (_I, [_P]),
     "apt_epoch_destroy": (_I, [_P]),
+    "apt_publish_words": (_I, [_P, _I, _P, _I, _P, _I, _P, _P]),
     "apt_epoch_host_cost": (_I, [_P, C.POINTER(CEpochCost)]),
 }
 
@@ -634,6 +635,7 @@ class MinibatchPlan:
         self.counts = [torch.empty(max(self.caps[h], 1), **i64) for h in range(H)] if want_counts else None
         self.sizes = torch.zeros(H + 2, **i64)
         self.pending = PendingLookup()
+        self.launches = 0
         self.rng_seed_dev = torch.zeros(1, **i64)
         self.table = table if table is not None else rank_table(graph.num_total_nodes, dev)
         self.table_len = graph.num_total_nodes
@@ -659,6 +661,7 @@ class MinibatchPlan:
                 _ptr(self.nodes), self._nb, self._rl, self._ct, _ptr(self.sizes), _ptr(self.workspace),
                 self.workspace.numel(), _stream())
         self.pending.run()          # a pass still open from an earlier call goes first
+        self.launches += 1
         if defer_lookup:
             check(lib().apt_minibatch_sample_deferred(*args, C.addressof(self.pending.c)))
             self.pending.open = True
@@ -1072,6 +1075,13 @@ def linear_wgrad(dy, x, want_bias=True):
     check(lib().apt_linear_wgrad(_ptr(dy), _ptr(x), m, n, k, x.element_size(), _ptr(dw), _ptr(db), _ptr(ws), ws.numel(),
                                  _stream()))
     return dw, db
+
+
+def publish_words(arrays, host):
+    """Up to three int64 GPU tensors into the pinned tensor `host`, asynchronous."""
+    a, b, c = (list(arrays) + [None, None])[:3]
+    n = lambda t: 0 if t is None else t.numel()
+    check(lib().apt_publish_words(_ptr(a), n(a), _ptr(b), n(b), _ptr(c), n(c), C.c_void_p(host.data_ptr()), _stream()))
 
 
 def linear_wgrads(products):

@@ -97,7 +97,7 @@ class MiniBatchLoader:
         st = self.streams[k]
         st.wait_event(after)
         with torch.cuda.stream(st):
-            pipe.run(seeds, rng_seed)
+            pipe.run(seeds, rng_seed, publish=False)
             pipe.stage_sizes()
             self.done[k].record(st)
 

@@ -15,9 +15,15 @@ With use_graph=True the fused batch (and the gather) is captured once into a
 HIP graph and replayed; seeds and the rng seed are read from fixed device
 buffers that are refreshed before each replay.
 """
+import weakref
+
 import torch
 
 from . import capi
+
+
+def _settle(event, words):
+    event.synchronize()
 
 
 class MiniBatchPipeline:
@@ -119,6 +125,22 @@ class MiniBatchPipeline:
         self.seeds = None
         self.sizes_host = None
         self.format_edges_host = None
+        # run() leaves the batch's sizes (and request and edge counts) in pinned memory as soon as they are known
+        self.words = [t for t in (self.sizes, self.request_sizes if requests is not None else None,
+                                  self.format_edges if formats else None) if t is not None]
+        self.words_host = torch.zeros(sum(t.numel() for t in self.words), dtype=torch.int64, pin_memory=True)
+        self.words_view = self.words_host.numpy()
+        self.words_known, self.finished = torch.cuda.Event(), torch.cuda.Event()
+        self.words_pending = False      # they are those of the batch that result() is asked for
+        self.words_launch = 0
+        # Published where it replaces a second blocking read (20 us) or where the gather behind it is long enough to hide
+        # the host's work: with features of 64 MB at their upper bound (2048 seeds, two hops) 120 against 128 us, of 277 MB
+        # 202 against 217; at 1..9 MB both take the same, and among other programs' passes 35 MB took 75.7 against 73.1.
+        bound = 0 if self.features is None else self.features.numel() * self.features.element_size()
+        self.publishes = requests is not None or bool(formats) or bound >= 64_000_000
+        self.captured = False           # a replay of a caller's graph publishes nothing: no batch does from then on
+        # a kernel writes them: the memory stays until it has, also where the pipeline is dropped with a batch in flight
+        weakref.finalize(self, _settle, self.words_known, self.words_host).atexit = False
         self.graph_exec = None
         if use_graph:
             if not self.fused:
@@ -184,6 +206,7 @@ class MiniBatchPipeline:
         if seeds.numel() != self.caps[0]:
             raise ValueError(f"expected {self.caps[0]} seeds, got {seeds.numel()}")
         self.seeds = seeds
+        self.words_pending = False
         if self.fused:
             self.plan.launch(seeds, rng_seed, defer_lookup=defer_lookup and self.can_defer_lookup)
         else:
@@ -216,7 +239,11 @@ class MiniBatchPipeline:
             for e in self.format_done:
                 cur.wait_event(e)
 
-    def gather(self):
+    def _publish(self):
+        capi.publish_words(self.words, self.words_host)
+        self.words_known.record()
+
+    def gather(self, publish=False):
         """Features of the input nodes (the last hop's unique ids), asynchronous."""
         H = len(self.fanouts)
         index = self.nodes if self.fused else self.frontier[H]
@@ -230,22 +257,40 @@ class MiniBatchPipeline:
                           rq["world_size"], rq["num_remote_workers"], n_dev=self._size(H),
                           out=(self.request_sizes, self.request_offsets, self.request_ids,
                                self.request_perm), workspace=self.request_ws)
+        if publish:
+            self._publish()
         # rows that are here: features[k] belongs to request_ids[k], k < request_sizes[0]
         capi.gather_rows(self.feat, self.request_ids, num_index_dev=self.request_sizes[0:1],
                          out=self.features, miss_count=self.misses)
 
-    def run(self, seeds, rng_seed):
+    def run(self, seeds, rng_seed, publish=True):
+        """A whole batch, asynchronous.  publish: its sizes go to pinned memory on the way, so that result() cuts the
+        buffers while the features are still being gathered and waits once.  With its result(), against blocking reads
+        behind the gather: a batch of 4096 on the 111 M-node graph 225 us (238), one of a partition with request
+        buckets 117 (130), 1024 seeds with all formats 272 (289)."""
         if self.graph_exec is not None:
             self.static_seeds.copy_(seeds)
             self.plan.rng_seed_dev.fill_(int(rng_seed) & 0x7FFFFFFFFFFFFFFF)
             self.seeds = self.static_seeds
+            self.words_pending = False
             self.graph_exec.replay()
             return
+        self.captured |= torch.cuda.is_current_stream_capturing()
+        publish = publish and self.publishes and not self.captured
         self.sample(seeds, rng_seed, defer_lookup=True)
+        bucketed = self.features is not None and self.requests is not None
+        if publish and self.formats is None and not bucketed:
+            self._publish()
         self.emit_formats(join=False)
         if self.features is not None:
-            self.gather()
+            self.gather(publish and self.formats is None and bucketed)
         self.join_formats()
+        if publish:
+            if self.formats is not None:
+                self._publish()
+            self.finished.record()
+            self.words_pending = True
+            self.words_launch = self.plan.launches if self.fused else 0
 
     def stage_sizes(self):
         """Asynchronous copy of the batch's sizes (and request bucket sizes) to pinned
@@ -276,7 +321,19 @@ class MiniBatchPipeline:
         pipeline runs its next batch."""
         if self.fused and self.plan.pending.open:      # sampled with the last pass deferred and never gathered
             self.plan.pending.run()
-        if sizes is None:
+        published = (sizes is None and not staged and self.words_pending and
+                     (not self.fused or self.words_launch == self.plan.launches))
+        self.words_pending = False
+        if published:
+            self.words_known.synchronize()
+            words, at = self.words_view.tolist(), self.sizes.numel()
+            sizes = words[:at]
+            if self.requests is not None:
+                request_sizes = words[at:at + self.request_sizes.numel()] if request_sizes is None else request_sizes
+                at += self.request_sizes.numel()
+            if self.formats is not None and format_edges is None:
+                format_edges = words[at:]
+        elif sizes is None:
             sizes = self.sizes_host.tolist() if staged else self.sizes.cpu().tolist()
         fmt_edges = None
         if self.formats is not None:
@@ -310,4 +367,6 @@ class MiniBatchPipeline:
             out.update(request_sizes=rs, request_ids=self.request_ids[:sizes[H]],
                        request_perm=self.request_perm[:sizes[H]],
                        features=None if self.features is None else self.features[:rs[0]])
+        if published:
+            self.finished.synchronize()
         return out

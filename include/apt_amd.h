@@ -596,6 +596,11 @@ typedef struct apt_epoch_cost {
 } apt_epoch_cost;
 int apt_epoch_host_cost(apt_epoch* epoch, apt_epoch_cost* cost);
 
+/* Up to three short arrays of device memory, one behind the other, into pinned host
+ * memory by a kernel: readable once the stream has passed it (an event behind it). */
+int apt_publish_words(const int64_t* a, int na, const int64_t* b, int nb, const int64_t* c, int nc,
+                      int64_t* host_words, void* stream);
+
 /* Cache construction (the callers of the registries).
  *   apt_count_ids        freq[ids[i]] += 1 for ids in [0, num_total_nodes): the
  *                        access counting of a dry run (examples/dryrun.py:86-92,

@@ -447,6 +447,68 @@ def test_partitioned_store_pipeline(orc, capi):
         assert outside.any() and np.all(outer["counts"][outside] == 0)
 
 
+def _flat(x):
+    if isinstance(x, torch.Tensor):
+        return [x.clone()]
+    if isinstance(x, dict):
+        return [t for k in sorted(x) for t in _flat(x[k])]
+    if isinstance(x, (list, tuple)):
+        return [t for v in x for t in _flat(v)]
+    return _flat(vars(x)) if hasattr(x, "__dict__") else [x]
+
+
+@pytest.mark.parametrize("kind", ["plain", "unfused", "requests", "formats", "both", "no_features"])
+def test_published_sizes_are_those_of_the_batch_asked_for(capi, kind):
+    """result() from the words that run() publishes equals result() from the device's sizes, also where the
+    batch in the buffers is a later one: sampled alone, launched on the plan, or replayed in a caller's graph."""
+    from apt_amd.pipeline import MiniBatchPipeline
+    indptr, indices, feats = _setup(None, None, n=20000, deg=9, dim=16, seed=5)
+    n, W = 20000, 4
+    pos = dev(-np.arange(n) - 2)
+    pos[5000:] = -1
+    table = dev(feats[:5000])
+    rq = dict(feat_pos_map=pos, remote_worker_map=dev(np.arange(W)), min_vids=dev(np.arange(W + 1) * (n // W)),
+              world_size=W, num_remote_workers=W)
+    with_requests = kind in ("requests", "both")
+    store = capi.FeatStore(table, None, pos) if with_requests else capi.FeatStore(dev(feats))
+    pipe = MiniBatchPipeline(capi.Graph(dev(indptr), dev(indices)), None if kind == "no_features" else store, 128, [4, 6],
+                             fused=kind != "unfused", requests=rq if with_requests else None,
+                             formats=kind in ("formats", "both"))
+    pipe.publishes = True                                 # whatever the size
+    a, b = (torch.randperm(n, device=DEV)[:128] for _ in range(2))
+    want = []
+    for seeds in (a, b):
+        pipe.run(seeds, 7, publish=False)
+        want.append(_flat(pipe.result()))
+    same = lambda got, ref: len(got) == len(ref) and all(
+        torch.equal(x, y) if isinstance(x, torch.Tensor) else x == y for x, y in zip(got, ref))
+    assert not same(want[0], want[1])
+    pipe.run(a, 7)
+    assert same(_flat(pipe.result()), want[0]) and same(_flat(pipe.result()), want[0])
+    pipe.run(a, 7)
+    pipe.run(b, 7)                                        # the first one's result is never asked for
+    assert same(_flat(pipe.result()), want[1])
+    pipe.run(a, 7)
+    pipe.run(b, 7, publish=False)
+    assert same(_flat(pipe.result()), want[1])
+    if kind in ("plain", "no_features"):
+        pipe.run(b, 7)
+        pipe.seeds = a
+        pipe.plan.launch(a, 7)
+        if kind == "plain":
+            pipe.gather()
+        assert same(_flat(pipe.result()), want[0])
+        graph, static = torch.cuda.CUDAGraph(), a.clone()
+        with torch.cuda.graph(graph):
+            pipe.run(static, 7)
+        for seeds, ref in ((b, want[1]), (a, want[0]), (b, want[1])):
+            pipe.run(a, 7)
+            static.copy_(seeds)
+            graph.replay()
+            pipe.seeds = static
+            assert same(_flat(pipe.result()), ref)
+
+
 @pytest.mark.parametrize("fuse_mark", [1, 0])
 def test_rank_table_epochs_and_refill(orc, capi, fuse_mark):
     """Batches reuse the rank table without clearing it; with a 30-bit id field
