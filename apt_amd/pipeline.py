@@ -125,22 +125,16 @@ class MiniBatchPipeline:
         self.seeds = None
         self.sizes_host = None
         self.format_edges_host = None
-        # run() leaves the batch's sizes (and request and edge counts) in pinned memory as soon as they are known
-        self.words = [t for t in (self.sizes, self.request_sizes if requests is not None else None,
-                                  self.format_edges if formats else None) if t is not None]
-        self.words_host = torch.zeros(sum(t.numel() for t in self.words), dtype=torch.int64, pin_memory=True)
-        self.words_view = self.words_host.numpy()
-        self.words_known, self.finished = torch.cuda.Event(), torch.cuda.Event()
-        self.words_pending = False      # they are those of the batch that result() is asked for
-        self.words_launch = 0
-        # Published where it replaces a second blocking read (20 us) or where the gather behind it is long enough to hide
-        # the host's work: with features of 64 MB at their upper bound (2048 seeds, two hops) 120 against 128 us, of 277 MB
-        # 202 against 217; at 1..9 MB both take the same, and among other programs' passes 35 MB took 75.7 against 73.1.
+        # run() leaves the batch's sizes (and request sizes) in pinned memory as soon as they are known, where that replaces a
+        # second blocking read (requests: 117 against 137 us) or where the gather behind it is long enough to hide the host's
+        # work: with features of 64 MB at their upper bound (2048 seeds, two hops) 120 against 128 us, of 277 MB 202 against
+        # 217; at 1..9 MB both take the same, and among other passes 35 MB took 75.7 against 73.1.  With formats, whose counts
+        # come last, there is nothing left to hide it behind: 307 against 298 us.
         bound = 0 if self.features is None else self.features.numel() * self.features.element_size()
-        self.publishes = requests is not None or bool(formats) or bound >= 64_000_000
-        self.captured = False           # a replay of a caller's graph publishes nothing: no batch does from then on
-        # a kernel writes them: the memory stays until it has, also where the pipeline is dropped with a batch in flight
-        weakref.finalize(self, _settle, self.words_known, self.words_host).atexit = False
+        self.words_pending = False      # the words are those of the batch that result() is asked for
+        self.publishes = False
+        if not use_graph and not formats and (requests is not None or bound >= 64_000_000):
+            self._publish_sizes()
         self.graph_exec = None
         if use_graph:
             if not self.fused:
@@ -239,6 +233,17 @@ class MiniBatchPipeline:
             for e in self.format_done:
                 cur.wait_event(e)
 
+    def _publish_sizes(self):
+        self.words = [self.sizes] if self.requests is None else [self.sizes, self.request_sizes]
+        self.words_host = torch.zeros(sum(t.numel() for t in self.words), dtype=torch.int64, pin_memory=True)
+        self.words_view = self.words_host.numpy()
+        self.words_known, self.finished = torch.cuda.Event(), torch.cuda.Event()
+        self.words_launch = 0
+        self.captured = False           # a replay of a caller's graph publishes nothing: no batch does from then on
+        # a kernel writes them: the memory stays until it has, also where the pipeline is dropped with a batch in flight
+        weakref.finalize(self, _settle, self.words_known, self.words_host).atexit = False
+        self.publishes = True
+
     def _publish(self):
         capi.publish_words(self.words, self.words_host)
         self.words_known.record()
@@ -266,8 +271,8 @@ class MiniBatchPipeline:
     def run(self, seeds, rng_seed, publish=True):
         """A whole batch, asynchronous.  publish: its sizes go to pinned memory on the way, so that result() cuts the
         buffers while the features are still being gathered and waits once.  With its result(), against blocking reads
-        behind the gather: a batch of 4096 on the 111 M-node graph 225 us (238), one of a partition with request
-        buckets 117 (130), 1024 seeds with all formats 272 (289)."""
+        behind the gather: a batch of 4096 on the 111 M-node graph 230 us (244), one of a partition with request
+        buckets 117 (137)."""
         if self.graph_exec is not None:
             self.static_seeds.copy_(seeds)
             self.plan.rng_seed_dev.fill_(int(rng_seed) & 0x7FFFFFFFFFFFFFFF)
@@ -275,19 +280,18 @@ class MiniBatchPipeline:
             self.words_pending = False
             self.graph_exec.replay()
             return
-        self.captured |= torch.cuda.is_current_stream_capturing()
+        if self.publishes:
+            self.captured |= torch.cuda.is_current_stream_capturing()
         publish = publish and self.publishes and not self.captured
         self.sample(seeds, rng_seed, defer_lookup=True)
         bucketed = self.features is not None and self.requests is not None
-        if publish and self.formats is None and not bucketed:
+        if publish and not bucketed:
             self._publish()
         self.emit_formats(join=False)
         if self.features is not None:
-            self.gather(publish and self.formats is None and bucketed)
+            self.gather(publish and bucketed)
         self.join_formats()
         if publish:
-            if self.formats is not None:
-                self._publish()
             self.finished.record()
             self.words_pending = True
             self.words_launch = self.plan.launches if self.fused else 0
@@ -328,11 +332,8 @@ class MiniBatchPipeline:
             self.words_known.synchronize()
             words, at = self.words_view.tolist(), self.sizes.numel()
             sizes = words[:at]
-            if self.requests is not None:
-                request_sizes = words[at:at + self.request_sizes.numel()] if request_sizes is None else request_sizes
-                at += self.request_sizes.numel()
-            if self.formats is not None and format_edges is None:
-                format_edges = words[at:]
+            if request_sizes is None:
+                request_sizes = words[at:]
         elif sizes is None:
             sizes = self.sizes_host.tolist() if staged else self.sizes.cpu().tolist()
         fmt_edges = None

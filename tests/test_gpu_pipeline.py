@@ -457,7 +457,7 @@ def _flat(x):
     return _flat(vars(x)) if hasattr(x, "__dict__") else [x]
 
 
-@pytest.mark.parametrize("kind", ["plain", "unfused", "requests", "formats", "both", "no_features"])
+@pytest.mark.parametrize("kind", ["plain", "unfused", "requests", "no_features"])
 def test_published_sizes_are_those_of_the_batch_asked_for(capi, kind):
     """result() from the words that run() publishes equals result() from the device's sizes, also where the
     batch in the buffers is a later one: sampled alone, launched on the plan, or replayed in a caller's graph."""
@@ -469,12 +469,12 @@ def test_published_sizes_are_those_of_the_batch_asked_for(capi, kind):
     table = dev(feats[:5000])
     rq = dict(feat_pos_map=pos, remote_worker_map=dev(np.arange(W)), min_vids=dev(np.arange(W + 1) * (n // W)),
               world_size=W, num_remote_workers=W)
-    with_requests = kind in ("requests", "both")
+    with_requests = kind == "requests"
     store = capi.FeatStore(table, None, pos) if with_requests else capi.FeatStore(dev(feats))
     pipe = MiniBatchPipeline(capi.Graph(dev(indptr), dev(indices)), None if kind == "no_features" else store, 128, [4, 6],
-                             fused=kind != "unfused", requests=rq if with_requests else None,
-                             formats=kind in ("formats", "both"))
-    pipe.publishes = True                                 # whatever the size
+                             fused=kind != "unfused", requests=rq if with_requests else None)
+    if not with_requests:
+        pipe._publish_sizes()                             # whatever the size
     a, b = (torch.randperm(n, device=DEV)[:128] for _ in range(2))
     want = []
     for seeds in (a, b):
