@@ -15,7 +15,7 @@
 //
 // Measured (both launches; the library's products and the addition where there are two), error against 64 bits:
 //   170 k rows, 100 + 100 -> 256    173 us / 449 us    6e-8 / 1.5e-7
-//   270 k rows, 100 -> 256          158 / 218          5e-8 / 1.3e-7
+//   270 k rows, 100 -> 256          158 / 218          5e-8 / 1.3e-7     (up to four steps of depth: rows_gemm_resident.hpp)
 //   40 k rows, 256 -> 256            50 /  57          6e-8 / 2.0e-7
 //   170 k rows, 256 -> 47            76 /  75          5e-8 / 1.9e-7
 //   1 k rows, 256 + 256 -> 47        22 /  42          8e-8 / 2.4e-7
