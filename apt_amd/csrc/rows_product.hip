@@ -225,13 +225,13 @@ __global__ __launch_bounds__(kProdBlock, 4) void rows_product_kernel(ProdParams 
                                                          __builtin_bit_cast(prod_bf16x8, xs), acc[f], 0, 0, 0);
     }
   };
-  // A lane has, of row l16, columns 32 h + 8 group .. + 7 in the fragments 2 h and 2 h + 1.
-  auto store = [&](const At& at) {
+  // The rows from .. to - 1.  A lane has, of row l16, columns 32 h + 8 group .. + 7 in the fragments 2 h and 2 h + 1.
+  auto store = [&](const At& at, int64_t from, int64_t to) {
     const int64_t r = row0(at) + l16;
 #pragma unroll
     for (int h = 0; h < kFragsN / 2; ++h) {
       const int c = n0 + h * 32 + group * 8;
-      if (r >= p.m || c >= p.n) continue;
+      if (r < from || r >= to || c >= p.n) continue;
       uint16_t* out = p.y + r * p.n + c;
       float v[8];
 #pragma unroll
@@ -268,8 +268,11 @@ __global__ __launch_bounds__(kProdBlock, 4) void rows_product_kernel(ProdParams 
     load(then, ahead);
     __builtin_amdgcn_sched_barrier(0);   // (those of this chunk are waited for alone)
     multiply(at, now);
-    if (then.block != at.block) {
-      store(at);
+    // Rows of the fragment without the second operand are stored before it comes: their zeros must not meet a weight that is
+    // not finite.
+    const bool ends = then.block != at.block, parts = then.which > at.which && row0(at) + 16 > p.a[1].rows;   // wave-uniform
+    if (ends || parts) store(at, parts ? p.a[1].rows : 0, at.which == 1 ? p.a[1].rows : p.m);
+    if (ends) {
       if (then.block >= p.row_blocks) return false;
       begin();
     }

@@ -67,6 +67,27 @@ def test_rows_product_stays_inside_its_operands(capi, k, turned):
     assert bad[5] and bad[70] and int(bad.sum()) == 2
 
 
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+@pytest.mark.parametrize("turned", [False, True])
+@pytest.mark.parametrize("m,m2,n,k", [(200, 77, 40, 48), (200, 77, 40, 47), (2100, 1001, 188, 130), (300, 299, 256, 64)])
+def test_rows_product_second_weights_not_finite(capi, m, m2, n, k, turned, bad):
+    """The rows behind the second operand's last, in the same fragment of 16, have nothing of its weights."""
+    gen = torch.Generator(device=DEV).manual_seed(m + k)
+    draw = lambda *shape: torch.randn(*shape, generator=gen, device=DEV).bfloat16()
+    weight = lambda: draw(k, n).t() if turned else draw(n, k)
+    x1, x2, w1, w2, bias, y = draw(m, k), draw(m2, k), weight(), weight(), draw(n), draw(m, n)
+    w2[n // 2, k - 1], w2[3, 0] = bad, -bad
+    want, size = x1.double() @ w1.double().t(), x1.double().abs() @ w1.double().abs().t()
+    want[:m2] += x2.double() @ w2.double().t()
+    size[:m2] += x2.double().abs() @ w2.double().abs().t()
+    for got, ref, total in ((capi.rows_gemm(x1, w1, x2, w2, bias=bias, relu=True), torch.relu(want + bias.double()), size + bias.double().abs()),
+                            (capi.rows_gemm(x1, w1, x2, w2, out=y.clone()), want + y.double(), size + y.double().abs())):
+        fine = torch.isfinite(ref)
+        assert bool(fine[m2:].all()) and int((~fine).sum()) > 0
+        assert torch.equal(torch.isnan(got), torch.isnan(ref)) and torch.equal(got[torch.isinf(got)].double(), ref[torch.isinf(ref)])
+        _check(got[fine], ref[fine], total[fine], 2 * k)
+
+
 def test_rows_product_sizes(capi):
     import apt_amd  # noqa: F401  (loads the operators)
     L = capi.lib()
