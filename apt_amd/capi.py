@@ -636,6 +636,7 @@ class MinibatchPlan:
         self.sizes = torch.zeros(H + 2, **i64)
         self.pending = PendingLookup()
         self.launches = 0
+        self.watch_captures = self.captured = False     # whether launch() is to notice that it is being captured; it was
         self.rng_seed_dev = torch.zeros(1, **i64)
         self.table = table if table is not None else rank_table(graph.num_total_nodes, dev)
         self.table_len = graph.num_total_nodes
@@ -662,6 +663,8 @@ class MinibatchPlan:
                 self.workspace.numel(), _stream())
         self.pending.run()          # a pass still open from an earlier call goes first
         self.launches += 1
+        if self.watch_captures:
+            self.captured |= torch.cuda.is_current_stream_capturing()
         if defer_lookup:
             check(lib().apt_minibatch_sample_deferred(*args, C.addressof(self.pending.c)))
             self.pending.open = True

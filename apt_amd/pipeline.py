@@ -204,6 +204,8 @@ class MiniBatchPipeline:
         if self.fused:
             self.plan.launch(seeds, rng_seed, defer_lookup=defer_lookup and self.can_defer_lookup)
         else:
+            if self.publishes:
+                self.captured |= torch.cuda.is_current_stream_capturing()
             self._sample_unfused(seeds, rng_seed)
 
     def emit_formats(self, join=True):
@@ -239,7 +241,11 @@ class MiniBatchPipeline:
         self.words_view = self.words_host.numpy()
         self.words_known, self.finished = torch.cuda.Event(), torch.cuda.Event()
         self.words_launch = 0
-        self.captured = False           # a replay of a caller's graph publishes nothing: no batch does from then on
+        # A replay of a caller's graph publishes nothing and is seen by nobody here: once a sampling has been captured
+        # (through run(), sample() or the plan), sizes are read from the device.
+        self.captured = False
+        if self.fused:
+            self.plan.watch_captures = True
         # a kernel writes them: the memory stays until it has, also where the pipeline is dropped with a batch in flight
         weakref.finalize(self, _settle, self.words_known, self.words_host).atexit = False
         self.publishes = True
@@ -280,10 +286,8 @@ class MiniBatchPipeline:
             self.words_pending = False
             self.graph_exec.replay()
             return
-        if self.publishes:
-            self.captured |= torch.cuda.is_current_stream_capturing()
-        publish = publish and self.publishes and not self.captured
         self.sample(seeds, rng_seed, defer_lookup=True)
+        publish = publish and self.publishes and not (self.plan.captured if self.fused else self.captured)
         bucketed = self.features is not None and self.requests is not None
         if publish and not bucketed:
             self._publish()
