@@ -310,7 +310,8 @@ static void launch_source_sum(SourceSumParams p, int64_t num_edges, hipStream_t 
 }
 
 template <typename I, bool EDATA>
-static int source_sum(const SourceSumParams& p, int64_t num_edges, int elem_size, hipStream_t st) {
+static int source_sum(SourceSumParams p, int64_t num_edges, int elem_size, hipStream_t st) {
+  if (p.num_dst == 0) p.dz = p.dx;   // no edge counts then, but row 0 is read in the place of a missing one
   const bool aligned = ((reinterpret_cast<uintptr_t>(p.dz) | reinterpret_cast<uintptr_t>(p.dx) |
                          reinterpret_cast<uintptr_t>(p.edata)) & 15) == 0;
   if (elem_size == 4) {

@@ -168,3 +168,34 @@ def test_hubs_of_every_class(dim, dtype, num_src):
     count = torch.bincount(edge[1], minlength=num_src).unsqueeze(1)
     bound = (count + 3) * 2.0 ** -24 * size + (2.0 ** -8 if dtype == torch.bfloat16 else 0.0) * want.abs()
     assert got.dtype == dtype and bool(((got.double() - want).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("dim", [16, 33, 256])
+def test_edges_without_rows(capi, dim, dtype):
+    """No row on the other side, but edges (none of which counts then): zeros, and nothing is read in their place, through
+    the C interface as a NULL, or rows that nobody may read."""
+    L, es = capi.lib(), 2 if dtype == torch.bfloat16 else 4
+    i64 = dict(dtype=torch.int64, device=DEV)
+    num_src, counts = 50, torch.arange(50, device=DEV)
+    indptr = torch.zeros(num_src + 1, **i64)
+    indptr[1:] = torch.cumsum(counts, 0)
+    edges = int(indptr[-1])
+    index = torch.zeros(edges, **i64)
+    dx = torch.full((num_src, dim), 7.0, device=DEV, dtype=dtype)
+    stream = capi._stream()
+    capi.check(L.apt_block_aggregate_backward(indptr.data_ptr(), index.data_ptr(), 8, 5, num_src, edges, None, None, 1.0, None, 0,
+                                              dim, es, dx.data_ptr(), None, 0, stream))
+    assert not bool(dx.any())
+    keys = torch.repeat_interleave(torch.arange(num_src, device=DEV), counts)
+    unreadable = torch.full((1,), float("nan"), device=DEV)
+    edata = torch.ones(edges, dim, device=DEV, dtype=dtype)
+    for mode in (0, 2):
+        for grouped in (1, 0):
+            need = int(L.apt_coo_sum_workspace_bytes(edges, num_src, grouped, 0, dim))
+            ws = torch.empty(max(need, 256), dtype=torch.uint8, device=DEV)
+            dx.fill_(7.0)
+            capi.check(L.apt_coo_sum(mode, keys.data_ptr(), index.data_ptr(), edges, grouped, 0, unreadable.data_ptr(), 0,
+                                     edata.data_ptr() if mode == 2 else None, dim, es, dx.data_ptr(), num_src, ws.data_ptr(),
+                                     ws.numel(), stream))
+            assert not bool(dx.any())
