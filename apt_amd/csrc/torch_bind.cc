@@ -1060,9 +1060,14 @@ Tensor dense(const Tensor& x_in, const Tensor& w, const Tensor& x2_in = Tensor()
                            bias.defined() ? bias.data_ptr() : nullptr, accumulate, relu, y.data_ptr(), stream()));
     return y;
   }
-  Tensor y = at::linear(x_in, w, b.defined() ? std::optional<Tensor>(b) : std::nullopt);
+  Tensor y;
+  if (onto.defined()) {   // (in one rounding)
+    y = onto.addmm_(x_in, w.t());
+    if (b.defined()) y.add_(b);
+  } else {
+    y = at::linear(x_in, w, b.defined() ? std::optional<Tensor>(b) : std::nullopt);
+  }
   if (pair) y.narrow(0, 0, m2).addmm_(x2_in, w2.t());
-  if (onto.defined()) y = onto.add_(y);
   return relu ? y.relu_() : y;
 }
 
