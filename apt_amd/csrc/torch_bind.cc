@@ -980,6 +980,7 @@ template <size_t N>
 void weight_grads(std::array<WeightGrad, N>& all, size_t count = N) {
   apt_wgrad_product products[N] = {};
   int es = 0;
+  bool empty = false;
   for (size_t i = 0; i < count; ++i) {
     WeightGrad& g = all[i];
     g.dy = g.dy.contiguous();
@@ -989,9 +990,10 @@ void weight_grads(std::array<WeightGrad, N>& all, size_t count = N) {
     products[i].m = g.dy.size(0);
     products[i].n = g.dy.size(1);
     products[i].k = g.x.defined() ? g.x.size(1) : 0;
+    empty |= g.x.defined() && products[i].k == 0;
   }
-  const size_t need = apt_linear_wgrads_workspace_bytes(products, static_cast<int>(count), es);
-  if (need == 0) {   // a weight beyond the kernel's sizes
+  const size_t need = empty ? 0 : apt_linear_wgrads_workspace_bytes(products, static_cast<int>(count), es);
+  if (need == 0) {   // a weight beyond the kernel's sizes, or without elements
     for (size_t i = 0; i < count; ++i) {
       WeightGrad& g = all[i];
       const Tensor dy = g.relu.defined() ? at::threshold_backward(g.dy, g.relu, 0) : g.dy;

@@ -99,3 +99,16 @@ def test_weight_gradient_of_infinite_rows(capi):
     assert torch.equal(dw.isnan(), want.isnan()) and torch.equal(dw.isinf(), want.isinf())
     ok = want.isfinite()
     assert torch.allclose(dw[ok].double(), want[ok], atol=2.0 ** -22 * 500 ** 0.5 * 16) and db[3].isinf()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("bias", [False, True])
+def test_block_linear_without_columns(dtype, bias):
+    """A weight [3, 0]: the product is the bias, its gradients are empty and the column sums."""
+    import apt_amd  # noqa: F401
+    x, w = torch.zeros(5, 0, device=DEV, dtype=dtype, requires_grad=True), torch.zeros(3, 0, device=DEV, dtype=dtype, requires_grad=True)
+    b = torch.tensor([1.0, 2.0, 3.0], device=DEV, dtype=dtype, requires_grad=True) if bias else None
+    y = torch.ops.npc.block_linear(x, w, b, False)
+    assert torch.equal(y, b.expand(5, 3) if bias else torch.zeros_like(y))
+    got = torch.autograd.grad(y, [x, w] + ([b] if bias else []), torch.full_like(y, 2.0))
+    assert got[0].shape == (5, 0) and got[1].shape == (3, 0) and (not bias or got[2].tolist() == [10.0, 10.0, 10.0])
