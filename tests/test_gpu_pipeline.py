@@ -486,8 +486,16 @@ def test_published_sizes_are_those_of_the_batch_asked_for(capi, kind):
     pipe.run(a, 7)
     assert same(_flat(pipe.result()), want[0]) and same(_flat(pipe.result()), want[0])
     pipe.run(a, 7)
-    pipe.run(b, 7)                                        # the first one's result is never asked for
-    assert same(_flat(pipe.result()), want[1])
+    assert pipe.words_pending
+    pipe.run(b, 7)                                        # the first one's result is never asked for: no more is published,
+    assert not pipe.words_pending and same(_flat(pipe.result()), want[1])
+    pipe.run(a, 7)                                        # until one is again
+    assert pipe.words_pending
+    pipe.stage_sizes()
+    torch.cuda.synchronize()
+    assert same(_flat(pipe.result(staged=True)), want[0])
+    pipe.run(b, 7)                                        # that one's sizes were taken another way
+    assert not pipe.words_pending and same(_flat(pipe.result()), want[1])
     pipe.run(a, 7)
     pipe.run(b, 7, publish=False)
     assert same(_flat(pipe.result()), want[1])
