@@ -9,10 +9,12 @@
 // nodes by first occurrence), so a group's rows are taken a grid apart.  Rows that are too long for one workgroup as well
 // are cut into chunks (long_rows.hpp).
 //
-// Bound by rows of dz that come from beyond the L2 (300 MB for 123 k rows of 256 fp32 and 249 k edges, 4.6 TB/s), hence
-// group_row.  Sum with the ordering of the edges, before (rows dealt to the XCDs one by one, every hub to a whole
-// workgroup, bf16 rows converted where they were loaded) / now, us: 238 k sources 733 k edges 256 fp32 240 / 206, 256 bf16
-// 206 / 145, 64 bf16 212 / 145, 47 bf16 202 / 134; 123 k sources 249 k edges 97 / 92, 106 / 79, 103 / 82, 88 / 72.
+// Bound by rows of dz that come from beyond the L2 where blocks are large, hence group_row, and by chains of dependent reads
+// (offsets, edges, scales, rows) where they are not, hence eight wavefronts on a SIMD (kFullSgprs).  Sum with the ordering of
+// the edges, before (rows dealt to the XCDs one by one, every hub to a whole workgroup, bf16 rows converted where they were
+// loaded) / now, us, fanout 15 and 10, sources drawn with density r^(1/3 - 1) and r^(1/2 - 1): 240 k sources 750 k edges
+// 256 fp32 275 / 215, 256 bf16 233 / 138, 64 bf16 186 / 125, 47 bf16 264 / 175; 122 k sources 260 k edges 112 / 93, 104 / 69,
+// 91 / 66, 102 / 73.  Without any skew 500 k sources 1 M edges: 307 / 290, 221 / 175, 156 / 126, 180 / 174.
 #include <algorithm>
 
 #include "common.hpp"
@@ -24,7 +26,7 @@ namespace apt {
 
 constexpr int kHubEdges = 16;
 constexpr int kHubList = 1024;             // rows of a workgroup at the most, so its list of hubs never overflows
-constexpr int kSourceBlocks = 2048;
+constexpr int kSourceBlocks = 4096;
 constexpr int kLongBlocks = 512;           // workgroups for long rows at the most
 
 struct SourceSumParams {
@@ -63,7 +65,7 @@ template <int LPR> __device__ __forceinline__ int64_t group_read(int64_t v, int 
 // I: int64_t = a block's CSR (offsets, destinations), uint32_t = apt_block_transpose (offsets, slots).
 // LONG: workgroups behind those of the rows take the long rows.
 template <typename T, int VEC, int LPR, typename I, bool EDATA, bool LONG>
-__global__ __launch_bounds__(kAggBlock) void source_sum_kernel(SourceSumParams p) {
+__global__ __launch_bounds__(kAggBlock) __attribute__((amdgpu_num_sgpr(kFullSgprs))) void source_sum_kernel(SourceSumParams p) {
   constexpr int kGroups = kAggBlock / LPR;
   constexpr int kRows = 2;
   constexpr int kUnroll = 4;
@@ -84,24 +86,47 @@ __global__ __launch_bounds__(kAggBlock) void source_sum_kernel(SourceSumParams p
     uint32_t slot;   // EDATA only
     float scale;
   };
-  auto slot_of = [&](int64_t at) { return index != nullptr ? index[at] : static_cast<I>(at); };
-  auto edge = [&](int64_t at, bool mine) {
-    Edge e{-1, 0u, 1.f};
-    if (!mine) return e;
-    if constexpr (sizeof(I) == 8) {
-      e.dst = static_cast<int64_t>(index[at]);
+  // Edges at[q] of lists, where they exist (entry 0 is read in the place of others): all on their way together, step by step.
+  auto look_up = [&](auto& at, const auto& mine, auto& e) {
+    constexpr int kCount = sizeof(at) / sizeof(at[0]);
+    I v[kCount];
+    if (sizeof(I) == 8 || index != nullptr) {
+#pragma unroll
+      for (int q = 0; q < kCount; ++q) v[q] = index[mine[q] ? at[q] : 0];
     } else {
-      e.slot = static_cast<uint32_t>(slot_of(at));
-      e.dst = p.via != nullptr ? p.via[e.slot] : static_cast<int64_t>(e.slot / p.fanout);
+#pragma unroll
+      for (int q = 0; q < kCount; ++q) v[q] = static_cast<I>(mine[q] ? at[q] : 0);
     }
-    if (e.dst < 0 || e.dst >= p.num_dst) e.dst = -1;
-    if (p.dst_scale != nullptr && e.dst >= 0) e.scale = p.dst_scale[e.dst];
-    return e;
+    if (sizeof(I) == 4 && p.via != nullptr) {
+#pragma unroll
+      for (int q = 0; q < kCount; ++q) e[q].dst = p.via[mine[q] ? v[q] : I{0}];   // (a list without edges is not filled)
+    } else {
+#pragma unroll
+      for (int q = 0; q < kCount; ++q) e[q].dst = sizeof(I) == 8 ? static_cast<int64_t>(v[q]) : static_cast<int64_t>(v[q] / p.fanout);
+    }
+#pragma unroll
+    for (int q = 0; q < kCount; ++q) {
+      e[q].slot = static_cast<uint32_t>(v[q]);
+      if (!mine[q] || e[q].dst < 0 || e[q].dst >= p.num_dst) e[q].dst = -1;
+      e[q].scale = 1.f;
+    }
+    if (p.dst_scale != nullptr) {
+#pragma unroll
+      for (int q = 0; q < kCount; ++q) e[q].scale = p.dst_scale[e[q].dst >= 0 ? e[q].dst : 0];
+    }
+  };
+  auto edge = [&](int64_t at, bool mine) {
+    const int64_t ats[1] = {at};
+    const bool mines[1] = {mine};
+    Edge e[1];
+    look_up(ats, mines, e);
+    return e[0];
   };
   const T* edata = static_cast<const T*>(p.edata);
   // acc += the rows of edges from .. n - 1 that the group's lanes hold, kUnroll on their way at once.  What is loaded in a
   // branch is converted behind all of them: a conversion inside one waits for its load.
-  auto walk = [&](const Edge& my, int from, int n, int64_t c, bool live, float (&acc)[VEC]) {
+  auto walk = [&](const Edge& my, int from, int n, int64_t c, float (&acc)[VEC]) {
+    const int64_t col = min(c, p.dim - VEC);   // (lanes without columns read with the last one)
     for (int e0 = from; e0 < n; e0 += kUnroll) {
       Row<T, VEC> v[kUnroll], m[EDATA ? kUnroll : 1];
       float w[kUnroll];
@@ -114,9 +139,9 @@ __global__ __launch_bounds__(kAggBlock) void source_sum_kernel(SourceSumParams p
           const int64_t d = group_read<LPR>(my.dst, e0 + u);
           w[u] = group_read<LPR>(my.scale, e0 + u);
           ok[u] = d >= 0;
-          v[u] = load_row<T, VEC>(dz, (d >= 0 ? d * p.dim : 0) + (live ? c : 0));
+          v[u] = load_row<T, VEC>(dz, (d >= 0 ? d * p.dim : 0) + col);
           if constexpr (EDATA)
-            m[u] = load_row<T, VEC>(edata, static_cast<int64_t>(group_read<LPR>(my.slot, e0 + u)) * p.dim + (live ? c : 0));
+            m[u] = load_row<T, VEC>(edata, static_cast<int64_t>(group_read<LPR>(my.slot, e0 + u)) * p.dim + col);
         }
       }
 #pragma unroll
@@ -132,10 +157,10 @@ __global__ __launch_bounds__(kAggBlock) void source_sum_kernel(SourceSumParams p
     }
   };
   // acc += the edges [lo, hi), every kGroups-th by this group
-  auto add_span = [&](int64_t lo, int64_t hi, int64_t c, bool live, float (&acc)[VEC]) {
+  auto add_span = [&](int64_t lo, int64_t hi, int64_t c, float (&acc)[VEC]) {
     for (int64_t e = lo + grp; e < hi; e += kAggBlock) {
       const int64_t at = e + static_cast<int64_t>(l) * kGroups;
-      walk(edge(at, at < hi), 0, static_cast<int>(min((hi - e + kGroups - 1) / kGroups, static_cast<int64_t>(LPR))), c, live, acc);
+      walk(edge(at, at < hi), 0, static_cast<int>(min((hi - e + kGroups - 1) / kGroups, static_cast<int64_t>(LPR))), c, acc);
     }
   };
   // The groups' sums together, in order, for the first group.
@@ -168,7 +193,7 @@ __global__ __launch_bounds__(kAggBlock) void source_sum_kernel(SourceSumParams p
           float acc[VEC];
 #pragma unroll
           for (int k = 0; k < VEC; ++k) acc[k] = 0.f;
-          if (!whole) add_span(chunk.from, chunk.to, c, live, acc);
+          if (!whole) add_span(chunk.from, chunk.to, c, acc);
           for (uint32_t g = grp; whole && g < chunk.count && live; g += kGroups)
 #pragma unroll
             for (int k = 0; k < VEC; ++k) acc[k] += part[static_cast<int64_t>(g) * p.dim + c + k];
@@ -190,21 +215,23 @@ __global__ __launch_bounds__(kAggBlock) void source_sum_kernel(SourceSumParams p
   }
   const int64_t row_groups = static_cast<int64_t>(p.row_blocks) * kGroups;
   for (int64_t r0 = group_row<kGroups>(grp, p.row_blocks); r0 < p.num_src; r0 += kRows * row_groups) {
-    int64_t lo[kRows];
+    int64_t lo[kRows], at[kRows];
     int n[kRows];
+    bool mine[kRows];
 #pragma unroll
     for (int q = 0; q < kRows; ++q) {
       const int64_t r = r0 + q * row_groups;
-      lo[q] = 0;
-      n[q] = 0;
-      if (r < p.num_src) {
-        lo[q] = static_cast<int64_t>(indptr[r]);
-        n[q] = static_cast<int>(static_cast<int64_t>(indptr[r + 1]) - lo[q]);
-      }
+      const I a = indptr[min(r, p.num_src - 1)], b = indptr[min(r, p.num_src - 1) + 1];
+      lo[q] = static_cast<int64_t>(a);
+      n[q] = static_cast<int>(b - a) * (r < p.num_src);   // (a condition would wait for the load)
+    }
+#pragma unroll
+    for (int q = 0; q < kRows; ++q) {
+      at[q] = lo[q] + l;
+      mine[q] = l < n[q] && n[q] <= kHubEdges;
     }
     Edge first[kRows];
-#pragma unroll
-    for (int q = 0; q < kRows; ++q) first[q] = edge(lo[q] + l, l < n[q] && n[q] <= kHubEdges);
+    look_up(at, mine, first);
     for (int64_t c0 = 0; c0 < p.dim; c0 += LPR * VEC) {
       const int64_t c = c0 + static_cast<int64_t>(l) * VEC;
       const bool live = c < p.dim;
@@ -215,9 +242,9 @@ __global__ __launch_bounds__(kAggBlock) void source_sum_kernel(SourceSumParams p
         float acc[VEC];
 #pragma unroll
         for (int k = 0; k < VEC; ++k) acc[k] = 0.f;
-        walk(first[q], 0, min(n[q], LPR), c, live, acc);
+        walk(first[q], 0, min(n[q], LPR), c, acc);
         for (int e = LPR; e < n[q]; e += LPR)   // LPR < kHubEdges only
-          walk(edge(lo[q] + e + l, e + l < n[q]), 0, min(n[q] - e, LPR), c, live, acc);
+          walk(edge(lo[q] + e + l, e + l < n[q]), 0, min(n[q] - e, LPR), c, acc);
         if (live) {
 #pragma unroll
           for (int k = 0; k < VEC; ++k) acc[k] *= p.scale;
@@ -234,7 +261,9 @@ __global__ __launch_bounds__(kAggBlock) void source_sum_kernel(SourceSumParams p
   }
   __syncthreads();
   // (in any order: every hub is summed on its own)
-  const int hubs = s_hubs[0], shared = s_hubs[1];
+  // A group each for the shorter hubs if that keeps them busy; otherwise one after the other by all groups, as the longer.
+  const bool apiece = s_hubs[0] >= hubs_apiece<kGroups>();
+  const int hubs = apiece ? s_hubs[0] : 0, shared = s_hubs[1] + (apiece ? 0 : s_hubs[0]);
   for (int i = grp; i < hubs; i += kGroups) {
     const int64_t r = s_hub[i];
     const int64_t lo = static_cast<int64_t>(indptr[r]);
@@ -252,7 +281,7 @@ __global__ __launch_bounds__(kAggBlock) void source_sum_kernel(SourceSumParams p
           float run[VEC];
 #pragma unroll
           for (int k = 0; k < VEC; ++k) run[k] = 0.f;
-          walk(my, e, min(min(n - k0, kChunk), e + kHubEdges), c, live, run);
+          walk(my, e, min(min(n - k0, kChunk), e + kHubEdges), c, run);
 #pragma unroll
           for (int k = 0; k < VEC; ++k) acc[k] += run[k];
         }
@@ -265,7 +294,7 @@ __global__ __launch_bounds__(kAggBlock) void source_sum_kernel(SourceSumParams p
     }
   }
   for (int i = 0; i < shared; ++i) {
-    const int64_t r = s_hub[kHubList - 1 - i];
+    const int64_t r = i < s_hubs[1] ? s_hub[kHubList - 1 - i] : s_hub[i - s_hubs[1]];
     const int64_t lo = static_cast<int64_t>(indptr[r]), hi = static_cast<int64_t>(indptr[r + 1]);
     for (int64_t c0 = 0; c0 < p.dim; c0 += LPR * VEC) {
       const int64_t c = c0 + static_cast<int64_t>(l) * VEC;
@@ -273,7 +302,7 @@ __global__ __launch_bounds__(kAggBlock) void source_sum_kernel(SourceSumParams p
       float acc[VEC];
 #pragma unroll
       for (int k = 0; k < VEC; ++k) acc[k] = 0.f;
-      add_span(lo, hi, c, live, acc);   // (all groups have some of the edges)
+      add_span(lo, hi, c, acc);   // (all groups have some of the edges)
       over_groups(acc);
       if (grp == 0 && live) {
 #pragma unroll
@@ -292,10 +321,10 @@ static void launch_source_sum(SourceSumParams p, int64_t num_edges, hipStream_t 
 #define APT_SOURCE_SUM(LPR)                                                                                        \
   do {                                                                                                            \
     constexpr int64_t groups = kAggBlock / LPR;                                                                    \
-    const int64_t blocks = std::max(ceil_div(p.num_src, kHubList),                                                \
-                                    std::min<int64_t>(std::max(ceil_div(p.num_src, groups * 2),                   \
-                                                               std::min(p.num_src, num_edges / (groups * kHubEdges))), \
-                                                      kSourceBlocks));                                            \
+    const int64_t blocks = even_grid(std::max(ceil_div(p.num_src, kHubList),                                      \
+                                              std::min<int64_t>(std::max(ceil_div(p.num_src, groups * 2),         \
+                                                                         std::min(p.num_src, num_edges / (groups * kHubEdges))), \
+                                                                kSourceBlocks)));                                 \
     const int64_t chunks = p.lng.slots > 0 ? std::min<int64_t>(long_chunks(num_edges), kLongBlocks) : 0;          \
     p.row_blocks = static_cast<uint32_t>(blocks);                                                                 \
     const dim3 grid(static_cast<unsigned>(blocks + chunks)), block(kAggBlock);                                    \
@@ -311,7 +340,14 @@ static void launch_source_sum(SourceSumParams p, int64_t num_edges, hipStream_t 
 
 template <typename I, bool EDATA>
 static int source_sum(SourceSumParams p, int64_t num_edges, int elem_size, hipStream_t st) {
-  if (p.num_dst == 0) p.dz = p.dx;   // no edge counts then, but row 0 is read in the place of a missing one
+  if (p.num_dst == 0) {   // no edge counts then, but entry 0 is read in the place of a missing one
+    p.dz = p.dx;
+    p.dst_scale = nullptr;
+  }
+  if (num_edges == 0) {
+    p.via = nullptr;
+    if (p.index != nullptr) p.index = p.indptr;
+  }
   const bool aligned = ((reinterpret_cast<uintptr_t>(p.dz) | reinterpret_cast<uintptr_t>(p.dx) |
                          reinterpret_cast<uintptr_t>(p.edata)) & 15) == 0;
   if (elem_size == 4) {

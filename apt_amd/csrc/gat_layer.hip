@@ -195,7 +195,7 @@ static bool launch_pair_scores(const void* x, int64_t n, int64_t num_dst, int he
 // workgroup cut into chunks (long_rows.hpp; a chunk's sum: the row's features, then the heads' logit gradients).
 constexpr int kGatHubEdges = 16;
 constexpr int kGatHubList = 1024;
-constexpr int kGatSourceBlocks = 2048;
+constexpr int kGatSourceBlocks = 2048;      // twice as many where a lane reads single elements
 
 struct GatSourceParams {
   const void* indptr;       // offsets of the sources in `index`
@@ -222,7 +222,9 @@ struct GatSourceParams {
 // of the loop over the rows.  Rows and hubs are dealt as in block_grad.hip (grouped_rows.hpp).  124 k rows of 4 x 64 bf16,
 // 261 k edges (63 MB written, 134 MB of destinations' rows read): 61 us; 72 with four rows in flight (161 registers
 // instead of 111), neighbouring rows on different XCDs and every hub a workgroup's; 193 with a wavefront per row, loads in
-// branches and the heads worked out per row.
+// branches and the heads worked out per row.  (Three or four rows in flight where a lane reads one element: no faster.)
+// Workgroups, 2048 / 4096, whole backward pass of 240 k sources 500 k edges, us: 2 x 101 fp32 812 / 759, 4 x 64 fp32 361 / 369,
+// bf16 238 / 240; 124 k sampled rows of 4 x 64 bf16, the kernel alone, 41 / 43.
 // TWO: a lane's features may belong to two heads.
 template <typename T, int VEC, int LPR, typename I, bool TWO>
 __global__ __launch_bounds__(kAggBlock) void gat_source_kernel(GatSourceParams p) {
@@ -419,7 +421,8 @@ __global__ __launch_bounds__(kAggBlock) void gat_source_kernel(GatSourceParams p
     }
   }
   __syncthreads();
-  const int hubs = s_hubs[0], shared = s_hubs[1];
+  const bool apiece = s_hubs[0] >= hubs_apiece<kGroups>();
+  const int hubs = apiece ? s_hubs[0] : 0, shared = s_hubs[1] + (apiece ? 0 : s_hubs[0]);
   for (int i = grp; i < hubs; i += kGroups) {
     const int64_t r = s_hub[i];
     const int64_t lo = static_cast<int64_t>(indptr[r]), hi = static_cast<int64_t>(indptr[r + 1]);
@@ -446,7 +449,7 @@ __global__ __launch_bounds__(kAggBlock) void gat_source_kernel(GatSourceParams p
     }
   }
   for (int i = 0; i < shared; ++i) {
-    const int64_t r = s_hub[kGatHubList - 1 - i];
+    const int64_t r = i < s_hubs[1] ? s_hub[kGatHubList - 1 - i] : s_hub[i - s_hubs[1]];
     const int64_t lo = static_cast<int64_t>(indptr[r]), hi = static_cast<int64_t>(indptr[r + 1]);
     for (int64_t c0 = 0; c0 < row_len; c0 += LPR * VEC) {
       const Cols col = columns(c0);
@@ -503,9 +506,9 @@ static void launch_gat_source_as(const GatSourceParams& p, int64_t num_edges, hi
   do {                                                                                                            \
     const int64_t for_edges = std::max(std::min(p.num_src, num_edges / (kAggBlock / LPR * kGatHubEdges)),         \
                                        p.lng.slots > 0 ? long_chunks(num_edges) : 0);                             \
-    const int64_t blocks = std::max(ceil_div(p.num_src, kGatHubList),                                             \
-                                    std::min<int64_t>(std::max(ceil_div(p.num_src, 4 * kAggBlock / LPR), for_edges), \
-                                                      kGatSourceBlocks));                                         \
+    const int64_t blocks = even_grid(std::max(ceil_div(p.num_src, kGatHubList),                                   \
+                                              std::min<int64_t>(std::max(ceil_div(p.num_src, 4 * kAggBlock / LPR), for_edges), \
+                                                                kGatSourceBlocks * (VEC == 1 ? 2 : 1))));         \
     hipLaunchKernelGGL((gat_source_kernel<T, VEC, LPR, I, TWO>), dim3(static_cast<unsigned>(blocks)), dim3(kAggBlock), 0, st, p); \
   } while (0)
   if (per_row <= 8) APT_GAT_SOURCE(8);

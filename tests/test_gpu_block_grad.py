@@ -171,6 +171,33 @@ def test_hubs_of_every_class(dim, dtype, num_src):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("dim", [4, 8, 33, 64, 128, 256])
+@pytest.mark.parametrize("num_src,hubs", [(40, 40), (600, 90), (3000, 3000), (70000, 700)])
+def test_many_hubs(capi, num_src, hubs, dim, dtype):
+    """Neighbouring sources of 17 to 140 edges among those of two: whole workgroups of hubs, of which the lane groups take one
+    each, workgroups with one or two of them, and grids of rows that come out even and that do not."""
+    import apt_amd  # noqa: F401
+    rng = np.random.default_rng(num_src + dim)
+    counts = np.full(num_src, 2)
+    first = min(num_src // 3, num_src - hubs)
+    counts[first:first + hubs] = rng.integers(17, 141, size=hubs)
+    rel, num_dst = _counted_block(list(counts), 5, 100, num_src)
+    gen = torch.Generator(device=DEV).manual_seed(dim)
+    x = torch.zeros(num_src, dim, device=DEV, dtype=dtype, requires_grad=True)
+    up = torch.randn(num_dst, dim, generator=gen, device=DEV).to(dtype)
+    out = torch.ops.npc.block_aggregate(rel, num_dst, 5, x, False, None, None)
+    dx, = torch.autograd.grad(out, x, up, retain_graph=True)
+    keep = (rel >= 0).nonzero().flatten()
+    src, rows = rel[keep], up.double()[keep // 5]
+    want = torch.zeros(num_src, dim, device=DEV, dtype=torch.float64).index_add(0, src, rows)
+    size = torch.zeros(num_src, dim, device=DEV, dtype=torch.float64).index_add(0, src, rows.abs())
+    # fp32 sums of up to 140 terms, one rounding to the result's type
+    half = 2.0 ** -8 if dtype == torch.bfloat16 else 0.0      # (half a unit in the last of eight bits)
+    assert bool(((dx.double() - want).abs() <= 140 * 2.0 ** -24 * size + half * want.abs()).all())
+    assert torch.equal(dx, torch.autograd.grad(out, x, up)[0])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("dim", [16, 33, 256])
 def test_edges_without_rows(capi, dim, dtype):
     """No row on the other side, but edges (none of which counts then): zeros, and nothing is read in their place, through
