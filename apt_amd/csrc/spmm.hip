@@ -684,6 +684,23 @@ __global__ __launch_bounds__(kAggBlock, gat_scores_waves(ROWS, sizeof(T))) void 
   }
 }
 
+// Whether the one kernel is the faster.  It forms the scores of every edge, where the two form those of every source, and
+// keeps a destination's rows in registers: it wins where launches count, where few slots are held, and where all lanes of a
+// wavefront have features (fp32 rows of 256; a bf16 row is held converted, for half the bytes).  Two kernels / one, us,
+// 5 sources to a destination, fanout x heads x dim:
+//   2 k x 10    fp32 4x64 12/8, 2x64 10/8, 1x128 10/9     bf16 4x64 11/10, 1x64 10/10      (20 480 slots: 10 % either way)
+//   10 k x 10   fp32 4x64 31/24, 2x64 19/19, 4x16 16/14   bf16 4x64 23/29, 4x16 16/21
+//   100 k x 5   fp32 4x64 196/108, 1x64 70/70             bf16 4x64 124/108, 1x64 66/89, 4x16 63/77 (26 k: 23/25, 23/21)
+//   100 k x 10  fp32 4x64 273/191, 2x64 134/146, 4x16 85/111   bf16 4x64 163/259
+//   26 k x 15   fp32 4x64 87/74, 1x256 87/87, 2x64 46/66
+static bool gat_scores_pay(int64_t num_dst, int fanout, int heads, int64_t dim, int elem_size) {
+  const int64_t slots = num_dst * fanout;
+  const bool whole = heads * dim >= 256;
+  if (slots <= 20480) return true;
+  if (elem_size == 2) return fanout <= 5 && (whole || slots <= (dim <= 32 ? 131072 : 65536));
+  return fanout <= 5 || (fanout <= 10 && (whole || slots <= 80000)) || (whole && dim <= 64);
+}
+
 // Whether it was launched: heads and lanes per head powers of two, heads * fanout slots in a wavefront, as gat_ell_wave_kernel;
 // up to 16 slots (registers).
 template <typename T, typename OUT, typename P>
@@ -693,7 +710,8 @@ static bool launch_gat_scores(const int64_t* nbr, int64_t num_dst, int fanout, c
   constexpr int VEC = 4;
   const int64_t lph = dim / VEC;
   if (dim % VEC != 0 || (heads & (heads - 1)) != 0 || heads * fanout > kWave || fanout > 16 || (lph & (lph - 1)) != 0 ||
-      heads * lph > kWave || ((reinterpret_cast<uintptr_t>(ft) | reinterpret_cast<uintptr_t>(out)) & 15) != 0)
+      heads * lph > kWave || ((reinterpret_cast<uintptr_t>(ft) | reinterpret_cast<uintptr_t>(out)) & 15) != 0 ||
+      !gat_scores_pay(num_dst, fanout, heads, dim, sizeof(T)))
     return false;
   int log2_heads = 0;
   while ((1 << log2_heads) < heads) ++log2_heads;

@@ -182,3 +182,23 @@ def test_scores_formed_where_they_are_used(capi, num_dst, fanout, num_src, heads
         plain = torch.ops.npc.gat_layer(rel, num_dst, fanout, ft, *rest)
         grad = torch.ops.npc.gat_layer(rel, num_dst, fanout, ft.clone().requires_grad_(True), *rest)
         assert torch.equal(plain.isnan(), grad.isnan()) and torch.equal(plain.nan_to_num(7.0), grad.detach().nan_to_num(7.0))
+
+
+@pytest.mark.parametrize("num_dst,fanout,heads,dim", [(2048, 10, 2, 64), (2049, 10, 2, 64), (8000, 10, 4, 32), (8001, 10, 4, 32),
+                                                      (9000, 10, 1, 256), (3300, 5, 1, 64), (13200, 5, 1, 64), (13200, 5, 4, 64),
+                                                      (1500, 16, 4, 64), (1500, 16, 2, 128), (5, 16, 1, 4)])
+def test_scores_formed_where_they_are_used_or_before(num_dst, fanout, heads, dim):
+    """The two ways of a layer without gradients, on either side of where one becomes the faster: the bits of the layer with
+    gradients in fp32, and for bf16 rows those of an fp32 layer up to the order of a score's products."""
+    import apt_amd  # noqa: F401
+    gen = torch.Generator(device=DEV).manual_seed(num_dst)
+    num_src = num_dst + 500
+    rel = torch.randint(-1, num_src, (num_dst * fanout,), generator=gen, device=DEV)
+    ft, al, ar = (torch.randn(*s, heads, dim, generator=gen, device=DEV).bfloat16() for s in ((num_src,), (), ()))
+    call = lambda *v: torch.ops.npc.gat_layer(rel, num_dst, fanout, *v, None, 0.2, None, None, None, None, False, True)  # noqa: E731
+    whole = [t.float() for t in (ft, al, ar)]
+    with torch.no_grad():
+        got, half = call(*whole), call(ft, al, ar)
+    assert torch.equal(got, call(*(t.clone().requires_grad_(True) for t in whole)))
+    # a score is a sum of dim products (|products| up to about 4 sqrt(dim)): its error enters the weights as a factor
+    assert half.dtype == torch.float32 and torch.allclose(half, got, rtol=1e-5 * dim ** 0.5, atol=1e-5 * dim ** 0.5)

@@ -129,7 +129,8 @@ LAYER_BUDGETS = {
     "rows_gemm.hip": {"void apt::rows_gemm_kernel<4, 4, 4>(": 2, "void apt::rows_gemm_kernel<4, 1, 4>(": 3,
                       "void apt::rows_gemm_kernel<1, 2, 4>(": 2, "void apt::add_rows_kernel<float, 4>(": 8},
     "spmm.hip": {"void apt::spmm_ell_kernel<float, float, 4, 64>(": 8, "void apt::spmm_ell_kernel<unsigned short, unsigned short, 8, 32>(": 8,
-                 "void apt::gat_ell_wave_kernel<float, float, 4>(": 8, "void apt::gat_bwd_edge_wave_kernel<unsigned short, unsigned short, 4>(": 8},
+                 "void apt::gat_ell_wave_kernel<float, float, 4>(": 8,
+                 "void apt::gat_ell_scores_kernel<float, float, float, 4, 10>(": 5, "void apt::gat_ell_kernel<float, float, 1>(": 8, "void apt::gat_bwd_edge_wave_kernel<unsigned short, unsigned short, 4>(": 8},
 }
 
 
