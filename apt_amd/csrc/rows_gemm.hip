@@ -15,12 +15,12 @@
 //
 // Measured (both launches; the library's products and the addition where there are two), error against 64 bits:
 //   170 k rows, 100 + 100 -> 256    173 us / 449 us    6e-8 / 1.5e-7
-//   270 k rows, 100 -> 256          158 / 218          5e-8 / 1.3e-7     (up to four steps of depth: rows_gemm_resident.hpp)
 //   40 k rows, 256 -> 256            50 /  57          6e-8 / 2.0e-7
 //   170 k rows, 256 -> 47            76 /  75          5e-8 / 1.9e-7
 //   1 k rows, 256 + 256 -> 47        22 /  42          8e-8 / 2.4e-7
 // The first: 111 k of 306 k cycles on the matrix units (46 us at their rate), 72 k on the split and addresses, 310 MB of
-// rows and results (55 us); the workgroups of a launch read, multiply and write much in step.
+// rows and results (55 us); the workgroups of a launch read, multiply and write much in step.  Up to four steps of depth:
+// rows_gemm_resident.hpp (460 k rows, 100 -> 256 212 us, 230 here).
 #include <algorithm>
 
 #include "common.hpp"
@@ -373,8 +373,8 @@ extern "C" int apt_rows_gemm(const float* x1, int64_t k1, const float* w1, int64
   GemmParams p{x1, x2, k1, k2, m, k2 > 0 ? m2 : 0, n, {w1, w1_stride_n, w1_stride_k}, {w2, w2_stride_n, w2_stride_k},
                static_cast<const gemm_u32x4*>(workspace), gemm_frags(n), bias, accumulate, relu, y};
   const int64_t steps1 = ceil_div(k1, kGemmStep), steps2 = m2 > 0 ? ceil_div(k2, kGemmStep) : 0;
-  if (const int nf = resident_columns(m, n, steps1 + steps2)) {
-    ResidentParams q{p, static_cast<int>(steps1), static_cast<int>(steps2), 0, 0};
+  if (const int nf = resident_columns(m, n, steps1 + steps2, k1 % 32 != 0 || (m2 > 0 && k2 % 32 != 0))) {
+    ResidentParams q{p, static_cast<int>(steps1), static_cast<int>(steps2), 0, 0, 0};
     if (nf == 8) launch_resident<8>(q, st);
     else if (nf == 4) launch_resident<4>(q, st);
     else launch_resident<2>(q, st);

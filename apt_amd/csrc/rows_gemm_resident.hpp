@@ -19,7 +19,7 @@ using res_buffer_t = __amdgpu_buffer_rsrc_t;
 
 struct ResidentParams {
   GemmParams g;
-  int steps1, steps2, tiles_n;
+  int steps1, steps2, tiles_n, walkers;   // walkers: workgroups of a column tile
   int64_t row_blocks;
 };
 
@@ -32,11 +32,11 @@ __global__ __launch_bounds__(kResBlock, 2) void rows_gemm_resident_kernel(Reside
   const int lane = threadIdx.x % kWave;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int l16 = lane % 16, group = lane / 16;
-  // The workgroups of the same rows (other columns) are numbered eight apart, i.e. on one XCD.
-  const int i = blockIdx.x / 8;
+  // The workgroups of the same rows (other columns) follow each other on one XCD.
+  const int i = static_cast<int>(blockIdx.x % 8 * (gridDim.x / 8) + blockIdx.x / 8);
+  const int64_t first = __builtin_amdgcn_readfirstlane(i / p.tiles_n), stride = p.walkers;
   const int tile = __builtin_amdgcn_readfirstlane(i % p.tiles_n);
-  const int64_t first = __builtin_amdgcn_readfirstlane(i / p.tiles_n) * 8 + static_cast<int>(blockIdx.x % 8);
-  const int64_t stride = static_cast<int64_t>(gridDim.x / p.tiles_n);
+  if (first >= stride) return;   // block-uniform (the grid is a multiple of eight)
   const int64_t n0 = static_cast<int64_t>(tile) * NF * 16;
   const int steps = p.steps1 + p.steps2;
   constexpr int kBatch = 4;
@@ -211,16 +211,29 @@ __global__ __launch_bounds__(kResBlock, 2) void rows_gemm_resident_kernel(Reside
 }
 
 static int64_t resident_bytes(int64_t steps, int nf) { return steps * nf * kGemmParts * kWave * 16; }   // (96 KB at the most)
-// Column fragments of a tile; 0: the kernel without resident weights is the better one.  That is so for more than four
-// steps, whose weights leave room for 64 columns only, so that the rows are read and split once for each (26 k rows, 256 ->
-// 256: 32 us there, 40 here), and where the launch would leave CUs empty (11 k rows, 47 + 47 -> 256: 16 and 20) unless the
-// result is that narrow.  Here / there, us: 122 k rows 100 -> 256 65 / 75, 460 k 228 / 246, 300 k 64 -> 64 34 / 45, 200 k 128 ->
-// 128 60 / 65, 53 k 100 -> 16 11 / 15.
-static int resident_columns(int64_t m, int64_t n, int64_t steps) {
+// Turns of the loop over the rows: as many for every workgroup of a launch that the 256 CUs hold at once.
+static int64_t resident_turns(int64_t row_blocks, int64_t tiles_n) {
+  return ceil_div(row_blocks, std::max<int64_t>(256 / tiles_n, 1));
+}
+// Column fragments of a tile; 0: the kernel without resident weights is the better one.  That is so
+//   for more than four steps, whose weights leave room for 64 columns only, so that the rows are read and split once for each
+//     (26 k rows, 256 -> 256: 32 us there, 40 here);
+//   where the launch leaves many CUs idle, or has one turn only to pay for its weights with (the share of the CUs' turns that
+//     has work / turns; us here / there: 128 -> 256 26 k rows 0.8 / 1 26 / 21, 49 k 0.75 / 2 35 / 31, 53 k 0.81 / 2 35 / 35, 124 k
+//     0.95 / 4 57 / 63, 460 k 202 / 238; 100 -> 512 16 k 0.98 / 1 22 / 22, 26 k 0.8 / 2 32 / 35; 128 -> 1000 40 k 70 / 77);
+//   not so much for narrow results of few steps or of rows that begin inside a line, which the other kernel reads in more
+//     pieces (50 -> 100 32 k rows 0.5 / 1 14 / 13, 40 k 0.61 / 1 14 / 17, 124 k 22 / 33; 64 -> 64 100 k 0.76 / 2 17 / 22; 128 -> 128 as
+//     the wide ones, 65 k 1 / 1 27 / 26, 124 k 37 / 43);
+//   for a last tile that is nearly empty (128 -> 385, 100 k rows 148 / 129; 128 -> 300 65 / 81, 128 -> 301 106 / 121).
+// Up to 32 columns it is the better one throughout (100 -> 16: 5 k rows 10 / 13, 200 k 25 / 42).
+static int resident_columns(int64_t m, int64_t n, int64_t steps, bool broken) {   // broken: rows begin inside a line
   if (steps > 4) return 0;
   if (n <= 32) return 2;
   const int nf = n <= 64 ? 4 : 8;
-  return ceil_div(m, kResRows) * ceil_div(n, nf * 16) >= 128 ? nf : 0;
+  const int64_t tiles = ceil_div(n, nf * 16), row_blocks = ceil_div(m, kResRows), turns = resident_turns(row_blocks, tiles);
+  const double busy = static_cast<double>(row_blocks * tiles) / static_cast<double>(256 * turns);
+  if (n <= 128 && (steps <= 2 || broken)) return busy >= 0.6 ? nf : 0;
+  return turns >= 2 && busy >= 0.78 && n * 100 >= tiles * nf * 16 * 77 ? nf : 0;
 }
 
 template <int NF>
@@ -228,10 +241,9 @@ static void launch_resident(ResidentParams& p, hipStream_t st) {
   p.tiles_n = static_cast<int>(ceil_div(p.g.n, NF * 16));
   p.row_blocks = ceil_div(p.g.m, kResRows);
   const size_t lds = resident_bytes(p.steps1 + p.steps2, NF);
-  // as many turns of the loop over the rows for every workgroup; as many workgroups as the CUs hold
-  const int64_t most = std::max<int64_t>(256 / p.tiles_n, 8), turns = ceil_div(p.row_blocks, most);
-  const int64_t blocks = ceil_div(ceil_div(p.row_blocks, turns), 8) * 8;
-  hipLaunchKernelGGL((rows_gemm_resident_kernel<NF>), dim3(static_cast<unsigned>(blocks * p.tiles_n)), dim3(kResBlock), lds, st, p);
+  p.walkers = static_cast<int>(ceil_div(p.row_blocks, resident_turns(p.row_blocks, p.tiles_n)));
+  const int64_t grid = ceil_div(static_cast<int64_t>(p.walkers) * p.tiles_n, 8) * 8;
+  hipLaunchKernelGGL((rows_gemm_resident_kernel<NF>), dim3(static_cast<unsigned>(grid)), dim3(kResBlock), lds, st, p);
 }
 
 }  // namespace apt

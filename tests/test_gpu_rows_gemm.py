@@ -15,7 +15,8 @@ def _rand(gen, *shape):
 @pytest.mark.parametrize("m,m2,n,k1,k2", [(1, 0, 1, 1, 0), (17, 17, 47, 32, 1), (65, 40, 64, 33, 31), (1000, 1, 65, 100, 100),
                                           (1023, 64, 128, 4, 64), (2049, 2049, 129, 101, 3), (5000, 333, 256, 256, 256),
                                           (40001, 9000, 257, 12, 20), (70001, 70001, 47, 64, 4), (33000, 0, 100, 50, 0),
-                                          (300, 200, 600, 512, 40)])
+                                          (300, 200, 600, 512, 40), (40000, 77, 50, 50, 20), (40000, 40000, 100, 64, 0),
+                                          (53000, 52990, 300, 90, 20), (32769, 5, 1000, 70, 20)])
 @pytest.mark.parametrize("transposed,accumulate", [(False, False), (True, True)])
 def test_rows_gemm(capi, m, m2, n, k1, k2, transposed, accumulate):
     gen = torch.Generator(device=DEV).manual_seed(m + n)
@@ -36,12 +37,14 @@ def test_rows_gemm(capi, m, m2, n, k1, k2, transposed, accumulate):
     assert torch.equal(got, capi.rows_gemm(x1, at[0], x2, at[1], b, base))
 
 
-@pytest.mark.parametrize("k1", [100, 101])
-def test_rows_gemm_not_finite(capi, k1):
+# five steps of depth; four or fewer in the kernel with resident weights, by 32, 64 and 128 columns (200 of 256, of the fewest
+# rows that take it: two turns of the CUs, or a good part of one)
+@pytest.mark.parametrize("m,m2,n,k1", [(500, 203, 70, 100), (500, 203, 70, 101), (500, 203, 20, 50), (40000, 203, 60, 50),
+                                       (40000, 39999, 100, 51), (53000, 1003, 200, 96), (53000, 20, 256, 20)])
+def test_rows_gemm_not_finite(capi, m, m2, n, k1):
     gen = torch.Generator(device=DEV).manual_seed(3)
-    m, m2, n = 500, 203, 70
     x1, w1, x2, w2 = _rand(gen, m, k1), _rand(gen, n, k1), _rand(gen, m2, 8), _rand(gen, n, 8)
-    x1[3, 5], x1[7, 2], w1[10, 1], w2[20, 3] = float("inf"), float("nan"), float("-inf"), float("inf")
+    x1[3, 5], x1[7, 2], w1[10, 1], w2[n - 9, 3] = float("inf"), float("nan"), float("-inf"), float("inf")
     x1[9] = 0
     x1[9, 0] = torch.finfo(torch.float32).max            # rounds to an infinity in bf16
     w1[:, 0] = 1
