@@ -44,7 +44,7 @@ struct ProdOperand {
 struct ProdParams {
   ProdOperand a[2];
   int64_t m;
-  int n, tiles_n;
+  int n, tiles_n, walkers;   // walkers: workgroups of a column tile
   int64_t row_blocks;
   const uint16_t* bias;
   int accumulate, relu, wide;   // wide: results that can be stored at a time
@@ -151,11 +151,11 @@ __global__ __launch_bounds__(kProdBlock, 4) void rows_product_kernel(ProdParams 
   const int lane = threadIdx.x % kWave;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int l16 = lane % 16, group = lane / 16;
-  // The workgroups of the same rows (other columns) are numbered eight apart, i.e. on one XCD.
-  const int i = blockIdx.x / 8;
+  // The workgroups of the same rows (other columns) follow each other on one XCD.
+  const int i = static_cast<int>(blockIdx.x % 8 * (gridDim.x / 8) + blockIdx.x / 8);
+  const int64_t first = __builtin_amdgcn_readfirstlane(i / p.tiles_n), stride = p.walkers;
   const int tile = __builtin_amdgcn_readfirstlane(i % p.tiles_n);
-  const int64_t first = __builtin_amdgcn_readfirstlane(i / p.tiles_n) * 8 + static_cast<int>(blockIdx.x % 8);
-  const int64_t stride = static_cast<int64_t>(gridDim.x / p.tiles_n);
+  if (first >= stride) return;   // block-uniform (the grid is a multiple of eight)
   const int n0 = tile * WN * 64;
   const int steps = p.a[0].steps + p.a[1].steps;
   float* s_bias = reinterpret_cast<float*>(s_weights + steps * kFragsN * kWave);
@@ -295,11 +295,10 @@ static int prod_columns(int64_t n, int64_t steps) {
 template <int WN>
 static void launch_product(ProdParams& p, bool odd, hipStream_t st) {
   const size_t lds = prod_lds(p.a[0].steps + p.a[1].steps, WN);
-  // as many turns of the loop over the rows for every workgroup
-  const int64_t most = std::max<int64_t>(kProdGroups / (lds > 80 * 1024 ? 2 : 1) / p.tiles_n, 8);
-  const int64_t turns = ceil_div(p.row_blocks, most);
-  const int64_t blocks = ceil_div(ceil_div(p.row_blocks, turns), 8) * 8;
-  const dim3 grid(static_cast<unsigned>(blocks * p.tiles_n)), block(kProdBlock);
+  // as many turns of the loop over the rows for every workgroup of a launch that the CUs hold at once
+  const int64_t most = std::max<int64_t>(kProdGroups / (lds > 80 * 1024 ? 2 : 1) / p.tiles_n, 1);
+  p.walkers = static_cast<int>(ceil_div(p.row_blocks, ceil_div(p.row_blocks, most)));
+  const dim3 grid(static_cast<unsigned>(ceil_div(static_cast<int64_t>(p.walkers) * p.tiles_n, 8) * 8)), block(kProdBlock);
   if (odd) hipLaunchKernelGGL((rows_product_kernel<WN, true>), grid, block, lds, st, p);
   else hipLaunchKernelGGL((rows_product_kernel<WN, false>), grid, block, lds, st, p);
 }
