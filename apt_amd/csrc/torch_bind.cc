@@ -1028,8 +1028,25 @@ bool product_takes(const Tensor& w) {
   return (sk == 1 && sn >= k && (n + 256) * sn <= (1 << 30)) || (sn == 1 && sk >= n && (k + 32) * sk <= (1 << 30));
 }
 
+// Whether apt_rows_product is the faster for such sizes.  It reads the rows once for every column tile whose weights fit
+// LDS, and costs the host a third of a library product (6 us of 21): it wins where the rows are what counts, where a second
+// product and its sum are spared, and where both are short.  GPU us, library / here, 20 k | 54 k | 124 k | 460 k rows:
+//   100 -> 256 10/8 16/16 67/25 169/99     128 -> 64 5/5 7/8 27/12 59/32       128 -> 256 7/10 12/16 43/23 113/100
+//   128 -> 512 10/16 21/21 46/36 188/169   188 -> 256 12/11 19/21 78/33 215/101   256 -> 128 7/10 12/15 24/23 105/80
+//   256 -> 256 9/15 16/25 30/37 151/110    512 -> 128 9/15 18/21 34/34 160/118    512 -> 256 12/19 22/32 44/55 227/178
+//   1000 -> 64 16/16 28/27 74/51           1024 -> 128 12/24 23/42 57/76          1024 -> 1024 46/92 101/217 235/471
+//   333 -> 333 25/29 66/59 111/121         100 + 100 -> 256 23/13 35/23 142/40 403/113
+//   256 + 256 -> 256, 0.15 of the rows in the second: 15/18 24/26 43/41 193/125
+bool product_pays(int64_t m, int64_t n, int64_t k, int64_t k2) {
+  const int64_t steps = (k + 31) / 32 + (k2 + 31) / 32;
+  const bool once = n <= 64 || (n <= 128 && steps <= 16);   // one column tile, if any fits
+  if (steps <= 4 || (k2 > 0 && steps <= 16) || (k % 32 != 0 && k % 2 == 0 && steps <= 8)) return true;
+  if (m * n <= (k % 2 == 0 ? 1300000000 : 650000000) / k) return true;
+  return m >= 100000 && (once || (m >= 300000 && k % 32 == 0 && k <= 512 && n <= 256));
+}
+
 // x w^T (+ x2 w2^T on the first rows) (+ b) with w [n, k] of any strides; `onto`: added to (and returned).  fp32 rows
-// take apt_rows_gemm, bf16 rows apt_rows_product.
+// take apt_rows_gemm, bf16 rows apt_rows_product or the library's product.
 Tensor dense(const Tensor& x_in, const Tensor& w, const Tensor& x2_in = Tensor(), const Tensor& w2 = Tensor(),
              const Tensor& b = Tensor(), Tensor onto = Tensor(), bool relu = false) {
   const int64_t m = x_in.size(0), k = x_in.size(1), n = w.size(0);
@@ -1051,7 +1068,7 @@ Tensor dense(const Tensor& x_in, const Tensor& w, const Tensor& x2_in = Tensor()
                         need, stream()));
     return y;
   }
-  if (x_in.scalar_type() == torch::kBFloat16 && apt_rows_product_fits(m, n, k, k2) && product_takes(w) &&
+  if (x_in.scalar_type() == torch::kBFloat16 && apt_rows_product_fits(m, n, k, k2) && product_pays(m, n, k, k2) && product_takes(w) &&
       (!pair || product_takes(w2)) && (!b.defined() || b.scalar_type() == torch::kBFloat16)) {
     auto x = x_in.contiguous();
     Tensor x2 = pair ? x2_in.contiguous() : Tensor(), bias = b.defined() ? b.contiguous() : Tensor();

@@ -88,6 +88,20 @@ def test_rows_product_second_weights_not_finite(capi, m, m2, n, k, turned, bad):
         _check(got[fine], ref[fine], total[fine], 2 * k)
 
 
+@pytest.mark.parametrize("m,k,n", [(19000, 256, 256), (20000, 256, 256), (2000, 333, 970), (3000, 333, 970), (99999, 400, 100), (100000, 400, 100),
+                                   (30000, 512, 256), (40000, 129, 256), (70000, 258, 64), (500, 1500, 30)])
+def test_products_of_either_kind(m, k, n):
+    """A layer's product on both sides of where the resident weights begin to pay, with and without gradients."""
+    import apt_amd  # noqa: F401
+    gen = torch.Generator(device=DEV).manual_seed(m)
+    draw = lambda *shape: torch.randn(*shape, generator=gen, device=DEV).bfloat16()
+    x, w, b = draw(m, k), draw(n, k), draw(n)
+    want, size = x.double() @ w.double().t() + b.double(), x.double().abs() @ w.double().abs().t() + b.double().abs()
+    with torch.no_grad():
+        _check(torch.ops.npc.block_linear(x, w, b, False), want, size, k + 1)
+    _check(torch.ops.npc.block_linear(x, w.requires_grad_(True), b, False).detach(), want, size, k + 1)
+
+
 def test_rows_product_sizes(capi):
     import apt_amd  # noqa: F401  (loads the operators)
     L = capi.lib()
