@@ -127,7 +127,12 @@ LAYER_BUDGETS = {
                       "void apt::gat_param_grad_kernel<unsigned short, 8>(": 2, "void apt::gat_param_grad_kernel<float, 4>(": 3},
     "linear.hip": {"void apt::wgrad_kernel<float, 4, 4>(": 2, "void apt::wgrad_kernel<unsigned short, 4, 4>(": 2},
     "rows_gemm.hip": {"void apt::rows_gemm_kernel<4, 4, 4>(": 2, "void apt::rows_gemm_kernel<4, 1, 4>(": 3,
-                      "void apt::rows_gemm_kernel<1, 2, 4>(": 2, "void apt::add_rows_kernel<float, 4>(": 8},
+                      "void apt::rows_gemm_kernel<1, 2, 4>(": 2, "void apt::add_rows_kernel<float, 4>(": 8,
+                      "void apt::rows_gemm_resident_kernel<8>(": 2, "void apt::rows_gemm_resident_kernel<4>(": 3,
+                      "void apt::rows_gemm_resident_kernel<2>(": 3},
+    # eight wavefronts of a workgroup and, by LDS, up to two workgroups on a CU
+    "rows_product.hip": {"void apt::rows_product_kernel<1, false>(": 6, "void apt::rows_product_kernel<2, false>(": 5,
+                         "void apt::rows_product_kernel<4, false>(": 4, "void apt::rows_product_kernel<4, true>(": 4},
     "spmm.hip": {"void apt::spmm_ell_kernel<float, float, 4, 64>(": 8, "void apt::spmm_ell_kernel<unsigned short, unsigned short, 8, 32>(": 8,
                  "void apt::gat_ell_wave_kernel<float, float, 4>(": 8,
                  "void apt::gat_ell_scores_kernel<float, float, float, 4, 10>(": 5, "void apt::gat_ell_kernel<float, float, 1>(": 8, "void apt::gat_bwd_edge_wave_kernel<unsigned short, unsigned short, 4>(": 8},
