@@ -58,6 +58,8 @@ struct WgradJob {
 struct WgradParams {
   WgradJob job[kWgradJobs];
   int jobs, tiles;          // of all jobs
+  int common, longer;       // splits that all jobs have; the job that has more
+  int groups;               // workgroups
   int64_t rows_per_split;
 };
 
@@ -207,15 +209,17 @@ __global__ __launch_bounds__(kWgradBlock) void wgrad_kernel(WgradParams p) {
   const int lane = threadIdx.x % kWave;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int group = lane / 16, col16 = wgrad_col<T>(lane % 16);
-  // The workgroups of a split read the same rows: they are numbered eight apart, i.e. on one XCD, whose L2 then serves
-  // the others.
-  const int i = blockIdx.x / 8;
-  const int split = __builtin_amdgcn_readfirstlane((i / p.tiles) * 8 + blockIdx.x % 8);   // (a division leaves them in
-  int tile = __builtin_amdgcn_readfirstlane(i % p.tiles);                                  // vector registers)
-  const int which = p.jobs > 1 && tile >= p.job[0].tiles ? 1 : 0;
+  // The workgroups of a split read the same rows: they follow each other on one XCD, whose L2 then serves the others.  First
+  // the splits that all products have, then the others of the longer one.
+  const int w = static_cast<int>(blockIdx.x % 8 * (gridDim.x / 8) + blockIdx.x / 8);
+  if (w >= p.groups) return;   // block-uniform
+  const bool common = w < p.common * p.tiles;
+  const int in = common ? w : w - p.common * p.tiles, tiles = common ? p.tiles : p.job[p.longer].tiles;
+  const int split = __builtin_amdgcn_readfirstlane(in / tiles + (common ? 0 : p.common));   // (a division leaves them in
+  int tile = __builtin_amdgcn_readfirstlane(in % tiles);                                    // vector registers)
+  const int which = common ? (p.jobs > 1 && tile >= p.job[0].tiles ? 1 : 0) : p.longer;
   const WgradJob& job = p.job[which];
-  if (which == 1) tile -= p.job[0].tiles;
-  if (split >= job.splits) return;   // block-uniform
+  if (common && which == 1) tile -= p.job[0].tiles;
   const int tile_n = __builtin_amdgcn_readfirstlane(tile / job.tiles_k), tile_k = tile - tile_n * job.tiles_k;
   const int64_t n0 = static_cast<int64_t>(tile_n) * kTileN, k0 = static_cast<int64_t>(tile_k) * kTileK;
   const int64_t m0 = static_cast<int64_t>(split) * p.rows_per_split;
@@ -440,16 +444,19 @@ static bool wgrad_sizes_ok(int64_t m, int64_t n, int64_t k) {
 // read once) stay below half of the inputs they come from or a few megabytes.  Both launches; before: a wavefront for
 // itself loaded, regrouped and (fp32) split its operands, every tile's again.  us:
 //   rows n x k            fp32 before / now      bf16 before / now
-//   700 k 256 x 128           391 / 385              170 / 131
-//   124 k 256 x 128            74 /  71               38 /  29
-//   54 k  256 x 100            43 /  37               26 /  20
+//   460 k 256 x 128           228 / 209              113 /  81
+//   124 k 256 x 128            66 /  60               36 /  29
+//   54 k  256 x 100            38 /  33               25 /  20
 //   54 k  256 x (100 + 100)    87 /  60               53 /  26      (two products in one launch)
 //   11 k  256 x (256 + 256)    77 /  34               52 /  22
-//   11 k   47 x 256            21 /  12               18 /  14
-//   200 k  64 x 256            68 /  68               40 /  27
-//   460 k 256 x 64            166 / 178               77 /  62
-// fp32, 700 k rows: 3800 cycles a step and CU, of which 1540 on the matrix units, 770 in LDS and 1100 splitting; bf16:
-// 4.3 TB/s of rows.
+//   20 k   47 x 256            24 /  15               21 /  15
+//   20 k  256 x 602            62 /  51               37 /  26
+//   20 k 1024 x 1024          274 / 247              123 /  87
+//   460 k  47 x 256           129 / 138 to 147        68 / 154
+//   460 k 256 x 64            130 / 140               76 /  59
+//   460 k 512 x 64            234 / 267              131 / 120
+// Where one side is at most 64 wide the small tiles split an fp32 operand's rows for each of the tiles beside it, which over
+// long blocks costs more than the loads that they save (the last three rows); the larger tile would multiply padding.
 static bool wgrad_shape(WgradParams& p, int elem_size) {
   const int64_t step = elem_size == 4 ? 32 : 64;
   bool big = false;
@@ -478,9 +485,21 @@ static bool wgrad_shape(WgradParams& p, int elem_size) {
   rows = std::max(rows, ceil_div(part_row, std::max(kWgradPartBytes, bytes / 2)));
   rows = std::min(ceil_div(rows, step) * step, ceil_div(most, step) * step);
   // a split's rows are addressed with 32-bit offsets, and the loop reads up to 2 kWgradAhead steps past its last one
-  rows = std::min(rows, std::max<int64_t>((int64_t{1} << 30) / widest / step, 1) * step);
+  const int64_t limit = std::max<int64_t>((int64_t{1} << 30) / widest / step, 1) * step;
+  rows = std::min(rows, limit);
+  // ... nor more workgroups than aimed at (one of the larger tiles fills a CU)
+  const auto groups = [&](int64_t r) {
+    int64_t sum = 0;
+    for (int j = 0; j < p.jobs; ++j) sum += ceil_div(p.job[j].m, r) * p.job[j].tiles;
+    return sum;
+  };
+  while (big && p.tiles <= kWgradGroups && rows < most && groups(rows) > kWgradGroups && rows < limit)
+    rows = std::min(rows + ceil_div(rows, 64 * step) * step, limit);
   p.rows_per_split = rows;
   for (int j = 0; j < p.jobs; ++j) p.job[j].splits = static_cast<int>(ceil_div(p.job[j].m, rows));
+  p.longer = p.jobs > 1 && p.job[1].splits > p.job[0].splits ? 1 : 0;
+  p.common = p.jobs > 1 ? std::min(p.job[0].splits, p.job[1].splits) : p.job[0].splits;
+  p.groups = static_cast<int>(groups(rows));
   return big;
 }
 
@@ -495,10 +514,8 @@ static bool wgrad_pairs(const void* p, int64_t cols) { return cols % 2 == 0 && (
 
 template <typename T>
 static void launch_wgrad(const WgradParams& p, bool big, hipStream_t st) {
-  int splits = 0;
-  for (int j = 0; j < p.jobs; ++j) splits = std::max(splits, p.job[j].splits);
-  const dim3 grid(static_cast<unsigned>(ceil_div(splits, 8) * 8 * p.tiles)), block(kWgradBlock);
   const bool masked = p.job[0].out != nullptr || p.job[1].out != nullptr;
+  const dim3 grid(static_cast<unsigned>(ceil_div(p.groups, 8) * 8)), block(kWgradBlock);
 #define APT_WGRAD(TYPE, F) hipLaunchKernelGGL((wgrad_kernel<TYPE, F, F>), grid, block, (WgradTile<TYPE, F, F>::kLds), st, p)
   if (masked && big) APT_WGRAD(WgradRelu<T>, 4);
   else if (masked) APT_WGRAD(WgradRelu<T>, 2);

@@ -9,7 +9,8 @@ DEV = "cuda:0"
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("m,n,k", [(1, 1, 1), (31, 64, 64), (33, 65, 63), (64, 16, 50), (65, 10, 32), (1000, 47, 256),
-                                   (4099, 188, 101), (9001, 256, 100), (2500, 320, 514), (70000, 3, 7)])
+                                   (4099, 188, 101), (9001, 256, 100), (2500, 320, 514), (70000, 3, 7), (3000, 1030, 700),
+                                   (65, 47, 47), (8255, 47, 64), (40001, 130, 333)])
 def test_linear_wgrad(capi, m, n, k, dtype):
     gen = torch.Generator(device=DEV).manual_seed(m + n + k)
     dy = torch.randn(m, n, generator=gen, device=DEV).to(dtype)
@@ -112,3 +113,20 @@ def test_block_linear_without_columns(dtype, bias):
     assert torch.equal(y, b.expand(5, 3) if bias else torch.zeros_like(y))
     got = torch.autograd.grad(y, [x, w] + ([b] if bias else []), torch.full_like(y, 2.0))
     assert got[0].shape == (5, 0) and got[1].shape == (3, 0) and (not bias or got[2].tolist() == [10.0, 10.0, 10.0])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("sizes", [((20000, 256, 600), (3000, 256, 600)), ((500, 64, 64), (90000, 48, 60)), ((64, 300, 1000), (64, 300, 1000)),
+                                   ((5000, 256, 0), (30000, 200, 130))])
+def test_linear_wgrads_of_different_lengths(capi, sizes, dtype):
+    """Two products whose rows are split into different numbers of parts, and more tiles than workgroups."""
+    gen = torch.Generator(device=DEV).manual_seed(5)
+    draw = lambda *shape: torch.randn(*shape, generator=gen, device=DEV).to(dtype)  # noqa: E731
+    products = [(draw(m, n), draw(m, k) if k else None, None, True) for m, n, k in sizes]
+    half = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -23
+    for (dw, db), (dy, x, _, _) in zip(capi.linear_wgrads(products), products):
+        a, m = dy.double(), dy.shape[0]
+        if x is not None:
+            want, size = a.t() @ x.double(), a.abs().t() @ x.double().abs()
+            assert bool(((dw.double() - want).abs() <= (m / 32 + 40) * 2.0 ** -24 * size + half * want.abs()).all())
+        assert bool(((db.double() - a.sum(0)).abs() <= (m / 8 + 8) * 2.0 ** -24 * a.abs().sum(0) + half * a.sum(0).abs()).all())
