@@ -30,8 +30,12 @@ typedef uint32_t u32x2_v __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4_v __attribute__((ext_vector_type(4)));
 using buffer_t = __amdgpu_buffer_rsrc_t;
 
-__device__ __forceinline__ buffer_t make_buffer(const void* base, int64_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, static_cast<uint32_t>(bytes), 0x00020000);
+// It begins at a multiple of four bytes (`skip`: how far behind that the base is) and ends at one.
+__device__ __forceinline__ buffer_t make_buffer(const void* base, int64_t bytes, uint32_t& skip) {
+  const uintptr_t at = reinterpret_cast<uintptr_t>(base);
+  skip = static_cast<uint32_t>(at & 3);
+  return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(at - skip), 0,
+                                           bytes > 0 ? static_cast<uint32_t>(bytes + skip + 3) & ~3u : 0u, 0x00020000);
 }
 
 constexpr int kWgradWaves = 4;      // that multiply, two by two; as many more prepare their operands
@@ -64,7 +68,7 @@ struct WgradParams {
 };
 
 // Rows of a step and how a thread reads them: a unit is 8 rows (one lane's share of an MFMA operand) of kCols columns.
-// WgradOdd: bf16 rows of an odd length or address, whose elements are read one by one.
+// WgradOdd: bf16 rows of an odd length or address; a dword more is read, and the elements are taken out of the three.
 // WgradRelu: products may have a mask.
 struct WgradOdd {};
 template <typename T> struct WgradRelu {};
@@ -80,7 +84,7 @@ template <> struct WgradType<uint16_t> {
   static constexpr bool kMask = false;
 };
 template <> struct WgradType<WgradOdd> : WgradType<uint16_t> {
-  static constexpr int kWords = 4;
+  static constexpr int kWords = 3;
 };
 template <typename T> struct WgradType<WgradRelu<T>> : WgradType<T> {
   static constexpr bool kMask = true;
@@ -112,25 +116,29 @@ template <typename T> struct WgradUnit {
   __device__ __forceinline__ void load(buffer_t buf, uint32_t at, uint32_t row_bytes) {
 #pragma unroll
     for (int r = 0; r < kUnitRows; ++r, at += row_bytes) {
-      if constexpr (Type::kWords == 2) {
-        const u32x2_v w = __builtin_amdgcn_raw_buffer_load_b64(buf, at, 0, 0);
-        v[r][0] = w[0];
-        v[r][1] = w[1];
-      } else {
+      const uint32_t from = Type::kWords == 3 ? at & ~3u : at;
+      const u32x2_v w = __builtin_amdgcn_raw_buffer_load_b64(buf, from, 0, 0);
+      v[r][0] = w[0];
+      v[r][1] = w[1];
+      if constexpr (Type::kWords == 3) v[r][2] = __builtin_amdgcn_raw_buffer_load_b32(buf, from + 8, 0, 0);
+    }
+  }
+  // Elements where the even ones of the other kind are.  odd_at: the first row begins in the middle of a dword; odd_row: so does
+  // every other row.
+  __device__ __forceinline__ void align(uint32_t odd_at, uint32_t odd_row) {
+    if constexpr (Type::kWords == 3) {
 #pragma unroll
-        for (int c = 0; c < Type::kWords; ++c) v[r][c] = __builtin_amdgcn_raw_buffer_load_b16(buf, at + 2 * c, 0, 0);
+      for (int r = 0; r < kUnitRows; ++r) {
+        const uint32_t shift = 16 * ((odd_at ^ (r & odd_row)) & 1);
+        v[r][0] = __builtin_amdgcn_alignbit(v[r][1], v[r][0], shift);
+        v[r][1] = __builtin_amdgcn_alignbit(v[r][2], v[r][1], shift);
       }
     }
   }
-  // Single elements -> pairs of columns, as the wide loads leave them.
-  __device__ __forceinline__ void pack() {
-    if constexpr (Type::kWords == 4) {
+  // The first element of a row is none: what shares a dword with the last of the range.
+  __device__ __forceinline__ void drop_first(int row) {
 #pragma unroll
-      for (int r = 0; r < kUnitRows; ++r) {
-        v[r][0] |= v[r][1] << 16;
-        v[r][1] = v[r][2] | v[r][3] << 16;
-      }
-    }
+    for (int r = 0; r < kUnitRows; ++r) v[r][0] &= r == row ? 0xffff0000u : 0xffffffffu;
   }
   // Zero where the ReLU's result is (as torch has it: a NaN passes).
   __device__ __forceinline__ void mask(const WgradUnit& out) {
@@ -226,9 +234,11 @@ __global__ __launch_bounds__(kWgradBlock) void wgrad_kernel(WgradParams p) {
   const int64_t m1 = min(m0 + p.rows_per_split, job.m);
   const bool bias = job.db != nullptr && tile_k == 0;
   const bool masked = job.out != nullptr;
-  const buffer_t dy = make_buffer(static_cast<const Elem*>(job.dy) + m0 * job.n, (m1 - m0) * job.n * sizeof(Elem));
-  const buffer_t out = make_buffer(static_cast<const Elem*>(masked ? job.out : job.dy) + m0 * job.n, (m1 - m0) * job.n * sizeof(Elem));
-  const buffer_t x = make_buffer(static_cast<const Elem*>(job.x) + m0 * job.k, (m1 - m0) * job.k * sizeof(Elem));
+  uint32_t skip_a, skip_out, skip_b;
+  const buffer_t dy = make_buffer(static_cast<const Elem*>(job.dy) + m0 * job.n, (m1 - m0) * job.n * sizeof(Elem), skip_a);
+  const buffer_t out = make_buffer(static_cast<const Elem*>(masked ? job.out : job.dy) + m0 * job.n,
+                                   (m1 - m0) * job.n * sizeof(Elem), skip_out);
+  const buffer_t x = make_buffer(static_cast<const Elem*>(job.x) + m0 * job.k, (m1 - m0) * job.k * sizeof(Elem), skip_b);
   // (whole turns of the producers' loop; a step past the end reads zeros)
   const int steps = static_cast<int>((m1 - m0 + kWgradAhead * kRows - 1) / (kWgradAhead * kRows)) * kWgradAhead;
 
@@ -243,19 +253,29 @@ __global__ __launch_bounds__(kWgradBlock) void wgrad_kernel(WgradParams p) {
     const int col = u % (kTileN / kCols) * kCols, rg = u / (kTileN / kCols);
     const bool has_dy = kUnits == 2 || wave - kWgradWaves < kOperandUnits / kWave;   // wave-uniform; otherwise x alone
     const uint32_t row_a = static_cast<uint32_t>(job.n * sizeof(Elem)), row_b = static_cast<uint32_t>(job.k * sizeof(Elem));
-    const uint32_t at_a = static_cast<uint32_t>((rg * kUnitRows * job.n + n0 + col) * sizeof(Elem));
-    const uint32_t at_b = static_cast<uint32_t>((rg * kUnitRows * job.k + k0 + col) * sizeof(Elem));
+    const uint32_t at_a = static_cast<uint32_t>((rg * kUnitRows * job.n + n0 + col) * sizeof(Elem)) + skip_a;
+    const uint32_t at_b = static_cast<uint32_t>((rg * kUnitRows * job.k + k0 + col) * sizeof(Elem)) + skip_b;
     const bool sum_here = bias && has_dy;
+    // A range that ends in the middle of a dword holds an element too many, the first of the row behind it: in step `end`, if
+    // that is read at all.  (Its row and step in the range are the same for both operands.)
+    const int rows = static_cast<int>(m1 - m0), end = rows / kRows;
+    const bool end_here = rows % kRows / kUnitRows == rg;
     struct Source {
       buffer_t buffer;
       uint32_t row, at;
       int frag0;
+      uint32_t odd_at, odd_row;
+      bool cut;      // of this thread's unit
     } source[kUnits];
-    source[0] = has_dy ? Source{dy, row_a, at_a, 0} : Source{x, row_b, at_b, 2 * FN};
-    if constexpr (kUnits == 2) source[1] = Source{x, row_b, at_b, 2 * FN};
+    const auto operand = [&](buffer_t buffer, uint32_t row, uint32_t at, int frag0, uint32_t skip, int64_t cols, bool first) {
+      return Source{buffer, row, at, frag0, skip >> 1, row >> 1 & 1, first && end_here && ((rows * cols * 2 + skip) & 2) != 0};
+    };
+    const Source a = operand(dy, row_a, at_a, 0, skip_a, job.n, n0 + col == 0), b = operand(x, row_b, at_b, 2 * FN, skip_b, job.k, k0 + col == 0);
+    source[0] = has_dy ? a : b;
+    if constexpr (kUnits == 2) source[1] = b;
     WgradUnit<T> unit[kWgradAhead][kUnits], relu[kWgradAhead];
     auto load = [&](int q) {
-      if constexpr (Type::kMask) relu[q].load(has_dy ? out : x, source[0].at, source[0].row);
+      if constexpr (Type::kMask) relu[q].load(has_dy ? out : x, source[0].at + (has_dy ? skip_out - skip_a : 0u), source[0].row);
 #pragma unroll
       for (int i = 0; i < kUnits; ++i) {
         unit[q][i].load(source[i].buffer, source[i].at, source[i].row);
@@ -272,14 +292,15 @@ __global__ __launch_bounds__(kWgradBlock) void wgrad_kernel(WgradParams p) {
 #pragma unroll
         for (int i = 0; i < kUnits; ++i) {
           WgradUnit<T> now = unit[q][i];
-          now.pack();
+          now.align(source[i].odd_at, source[i].odd_row);
           if constexpr (Type::kMask) {
             if (i == 0 && masked && has_dy) {
               WgradUnit<T> result = relu[q];
-              result.pack();
+              result.align(skip_out >> 1, source[0].odd_row);
               now.mask(result);
             }
           }
+          if (Type::kWords == 3 && s + q == end && source[i].cut) now.drop_first(rows % kUnitRows);
           if (i == 0 && sum_here) now.add_to(sum);
 #pragma unroll
           for (int c = 0; c < kCols; ++c) {
@@ -452,11 +473,12 @@ static bool wgrad_sizes_ok(int64_t m, int64_t n, int64_t k) {
 //   20 k   47 x 256            24 /  15               21 /  15
 //   20 k  256 x 602            62 /  51               37 /  26
 //   20 k 1024 x 1024          274 / 247              123 /  87
-//   460 k  47 x 256           129 / 138 to 147        68 / 154
+//   460 k  47 x 256           129 / 138 to 147        68 /  63
 //   460 k 256 x 64            130 / 140               76 /  59
 //   460 k 512 x 64            234 / 267              131 / 120
+//   460 k  41 x 602           360 / 383              211 / 150
 // Where one side is at most 64 wide the small tiles split an fp32 operand's rows for each of the tiles beside it, which over
-// long blocks costs more than the loads that they save (the last three rows); the larger tile would multiply padding.
+// long blocks costs more than the loads that they save (the last four rows); the larger tile would multiply padding.
 static bool wgrad_shape(WgradParams& p, int elem_size) {
   const int64_t step = elem_size == 4 ? 32 : 64;
   bool big = false;

@@ -115,6 +115,30 @@ def test_block_linear_without_columns(dtype, bias):
     assert got[0].shape == (5, 0) and got[1].shape == (3, 0) and (not bias or got[2].tolist() == [10.0, 10.0, 10.0])
 
 
+@pytest.mark.parametrize("m", [1, 7, 63, 64, 65, 127, 129, 1000, 8193])
+@pytest.mark.parametrize("n,k", [(47, 31), (64, 47), (47, 64), (5, 66), (130, 101)])
+def test_linear_wgrad_between_what_is_not_finite(capi, m, n, k):
+    """bf16 rows of odd lengths and addresses: what shares a dword with their first and their last element is infinite, as is
+    what shares one with the ReLU's result."""
+    gen = torch.Generator(device=DEV).manual_seed(m + n)
+
+    def rows(cols, shift):
+        base = torch.full((m * cols + 8,), float("inf"), device=DEV, dtype=torch.bfloat16)
+        part = base[shift:shift + m * cols].view(m, cols)
+        part.copy_(torch.randn(m, cols, generator=gen, device=DEV).bfloat16())
+        return part
+
+    for shift in (0, 1, 3):
+        dy, x, y = rows(n, shift), rows(k, 4 - shift), rows(n, 1 if shift else 2)
+        for mask in (None, y):
+            (dw, db), = capi.linear_wgrads([(dy, x, mask, True)])
+            g = dy.double() if mask is None else torch.where(y.double() > 0, dy.double(), 0.0)
+            want, size = g.t() @ x.double(), g.abs().t() @ x.double().abs()
+            # fp32 sums of m products, one rounding to bf16
+            assert bool(((dw.double() - want).abs() <= (m + 2) * 2.0 ** -24 * size + 2.0 ** -8 * want.abs()).all())
+            assert bool(((db.double() - g.sum(0)).abs() <= (m + 2) * 2.0 ** -24 * g.abs().sum(0) + 2.0 ** -8 * g.sum(0).abs()).all())
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("sizes", [((20000, 256, 600), (3000, 256, 600)), ((500, 64, 64), (90000, 48, 60)), ((64, 300, 1000), (64, 300, 1000)),
                                    ((5000, 256, 0), (30000, 200, 130))])
