@@ -42,8 +42,9 @@ constexpr int kWgradWaves = 4;      // that multiply, two by two; as many more p
 constexpr int kWgradHalf = kWgradWaves * kWave;
 constexpr int kWgradBlock = 2 * kWgradHalf;
 constexpr int kWgradGroups = 256;   // workgroups aimed at: one per CU ...
-constexpr int kWgradSmallGroups = 512;   // ... or, of small tiles, two while each has kWgradSmallSteps of its loop
+constexpr int kWgradSmallGroups = 512;   // ... or, of smaller tiles, two while each has kWgradSmallSteps of its loop
 constexpr int kWgradSmallSteps = 16;
+constexpr int64_t kWgradLongRows = 1 << 19;   // times tiles: from here on oblong ones (see wgrad_shape)
 constexpr int kWgradJobs = 2;
 constexpr int64_t kWgradPartBytes = int64_t{16} << 20;
 
@@ -203,10 +204,9 @@ __global__ __launch_bounds__(kWgradBlock) void wgrad_kernel(WgradParams p) {
   constexpr int kRows = Type::kRows, kCols = Type::kCols, kParts = Type::kParts;
   constexpr int kGroups = Tile::kGroups, kSubs = kRows / 32;
   constexpr int kTileN = Tile::kTileN, kTileK = Tile::kTileK;
-  static_assert(FN == FK, "as many units of dy as of x");
-  constexpr int kOperandUnits = kTileN / kCols * kGroups;         // of dy, and of x
-  constexpr int kUnits = 2 * kOperandUnits / kWgradHalf;          // of a producer: 2 = one of either, 1 = of dy or of x
-  static_assert(kUnits == 1 || kUnits == 2);
+  constexpr int kUnitsN = kTileN / kCols * kGroups, kUnitsK = kTileK / kCols * kGroups;   // of dy and of x
+  constexpr int kUnits = FN + FK > 4 ? 2 : 1;                     // of a producer: 2 = one of either, 1 = of dy or of x
+  static_assert(std::max(kUnitsN, kUnitsK) * 2 == kUnits * kWgradHalf && std::min(kUnitsN, kUnitsK) % kWave == 0);
   constexpr int kFrags = 2 * FN + 2 * FK;                         // of the tile's operands: dy's, then x's
   constexpr int kFlip = kCols == 4 ? 4 : 0;                       // four lanes to a fragment: its neighbour the other way round
   static_assert(kWgradAhead % 2 == 0 && FN % 2 == 0);
@@ -249,30 +249,35 @@ __global__ __launch_bounds__(kWgradBlock) void wgrad_kernel(WgradParams p) {
   if (wave >= kWgradWaves) {
     // A thread's units: columns kCols * (u % units per row), rows 8 * (u / units per row) of a step.  Columns past the
     // edge read the row after (or zero): they only reach outputs past the edge, which are not stored.
-    const int u = (threadIdx.x - kWgradHalf) % kOperandUnits;
-    const int col = u % (kTileN / kCols) * kCols, rg = u / (kTileN / kCols);
-    const bool has_dy = kUnits == 2 || wave - kWgradWaves < kOperandUnits / kWave;   // wave-uniform; otherwise x alone
-    const uint32_t row_a = static_cast<uint32_t>(job.n * sizeof(Elem)), row_b = static_cast<uint32_t>(job.k * sizeof(Elem));
-    const uint32_t at_a = static_cast<uint32_t>((rg * kUnitRows * job.n + n0 + col) * sizeof(Elem)) + skip_a;
-    const uint32_t at_b = static_cast<uint32_t>((rg * kUnitRows * job.k + k0 + col) * sizeof(Elem)) + skip_b;
-    const bool sum_here = bias && has_dy;
+    // The narrow side of a tile that is not square has units for two of the wavefronts: of either pair in turn, since the
+    // workgroups of a CU come 256 apart and each has a wavefront on every SIMD.
+    const int pair = FN != FK && (wave / 2 & 1) != (blockIdx.x / kWgradGroups & 1) ? 1 : 0;      // wave-uniform; 1: none
+    const int thread = threadIdx.x - kWgradHalf, in_pair = threadIdx.x % (2 * kWave);
+    const bool has_dy = kUnits == 2 ? FN >= FK || pair == 0 : wave - kWgradWaves < kUnitsN / kWave;   // wave-uniform
+    const bool has_x = kUnits == 2 ? FN <= FK || pair == 0 : !has_dy;
     // A range that ends in the middle of a dword holds an element too many, the first of the row behind it: in step `end`, if
     // that is read at all.  (Its row and step in the range are the same for both operands.)
     const int rows = static_cast<int>(m1 - m0), end = rows / kRows;
-    const bool end_here = rows % kRows / kUnitRows == rg;
     struct Source {
       buffer_t buffer;
       uint32_t row, at;
-      int frag0;
+      int col, rg, frag0;
       uint32_t odd_at, odd_row;
       bool cut;      // of this thread's unit
     } source[kUnits];
-    const auto operand = [&](buffer_t buffer, uint32_t row, uint32_t at, int frag0, uint32_t skip, int64_t cols, bool first) {
-      return Source{buffer, row, at, frag0, skip >> 1, row >> 1 & 1, first && end_here && ((rows * cols * 2 + skip) & 2) != 0};
+    const auto operand = [&](buffer_t buffer, int64_t cols, int64_t col0, int u, int tile_cols, int frag0, uint32_t skip, bool here) {
+      const int col = u % (tile_cols / kCols) * kCols, rg = u / (tile_cols / kCols);
+      const uint32_t row = static_cast<uint32_t>(cols * sizeof(Elem));
+      // (a unit of another wavefront's is read past the range)
+      const uint32_t at = here ? static_cast<uint32_t>((rg * kUnitRows * cols + col0 + col) * sizeof(Elem)) + skip : 0x80000000u;
+      return Source{buffer, here ? row : 0u, at, col, rg, frag0, skip >> 1, row >> 1 & 1,
+                    col0 + col == 0 && rows % kRows / kUnitRows == rg && ((rows * cols * 2 + skip) & 2) != 0};
     };
-    const Source a = operand(dy, row_a, at_a, 0, skip_a, job.n, n0 + col == 0), b = operand(x, row_b, at_b, 2 * FN, skip_b, job.k, k0 + col == 0);
-    source[0] = has_dy ? a : b;
+    const Source a = operand(dy, job.n, n0, kUnits == 1 ? thread % kUnitsN : FN >= FK ? thread : in_pair, kTileN, 0, skip_a, has_dy);
+    const Source b = operand(x, job.k, k0, kUnits == 1 ? thread % kUnitsK : FN <= FK ? thread : in_pair, kTileK, 2 * FN, skip_b, has_x);
+    source[0] = kUnits == 2 || has_dy ? a : b;
     if constexpr (kUnits == 2) source[1] = b;
+    const bool sum_here = bias && has_dy;
     WgradUnit<T> unit[kWgradAhead][kUnits], relu[kWgradAhead];
     auto load = [&](int q) {
       if constexpr (Type::kMask) relu[q].load(has_dy ? out : x, source[0].at + (has_dy ? skip_out - skip_a : 0u), source[0].row);
@@ -291,6 +296,8 @@ __global__ __launch_bounds__(kWgradBlock) void wgrad_kernel(WgradParams p) {
       for (int q = 0; q < kWgradAhead; ++q) {
 #pragma unroll
         for (int i = 0; i < kUnits; ++i) {
+          if (FN < FK && i == 0 && !has_dy) continue;   // (wave-uniform)
+          if (FN > FK && i == 1 && !has_x) continue;
           WgradUnit<T> now = unit[q][i];
           now.align(source[i].odd_at, source[i].odd_row);
           if constexpr (Type::kMask) {
@@ -306,7 +313,7 @@ __global__ __launch_bounds__(kWgradBlock) void wgrad_kernel(WgradParams p) {
           for (int c = 0; c < kCols; ++c) {
             u32x4_v o[kParts];
             now.column(c, o);
-            const int frag = source[i].frag0 + col / 16;
+            const int col = source[i].col, rg = source[i].rg, frag = source[i].frag0 + col / 16;
             const int at = (q & 1) * kBufferVecs + ((rg / 4 * kFrags + frag) * 4 + rg % 4) * 16 + (wgrad_place<T>(col % 16 + c) ^ (frag & 1) * kFlip);
 #pragma unroll
             for (int d = 0; d < kParts; ++d) s_part[d * kPartVecs + at] = o[d];
@@ -318,7 +325,7 @@ __global__ __launch_bounds__(kWgradBlock) void wgrad_kernel(WgradParams p) {
     }
     if (sum_here)
 #pragma unroll
-      for (int q = 0; q < kCols; ++q) s_sum[rg][col + q] = sum[q];
+      for (int q = 0; q < kCols; ++q) s_sum[source[0].rg][source[0].col + q] = sum[q];
   } else {
     for (int s = 0; s < steps; ++s) {
       __syncthreads();
@@ -470,29 +477,42 @@ static bool wgrad_sizes_ok(int64_t m, int64_t n, int64_t k) {
 //   54 k  256 x 100            38 /  33               25 /  20
 //   54 k  256 x (100 + 100)    87 /  60               53 /  26      (two products in one launch)
 //   11 k  256 x (256 + 256)    77 /  34               52 /  22
-//   20 k   47 x 256            24 /  15               21 /  15
-//   20 k  256 x 602            62 /  51               37 /  26
+//   20 k   47 x 256            24 /  16               21 /  11
+//   20 k  256 x 602            62 /  52               37 /  26
 //   20 k 1024 x 1024          274 / 247              123 /  87
-//   460 k  47 x 256           129 / 138 to 147        68 /  63
-//   460 k 256 x 64            130 / 140               76 /  59
-//   460 k 512 x 64            234 / 267              131 / 120
-//   460 k  41 x 602           360 / 383              211 / 150
-// Where one side is at most 64 wide the small tiles split an fp32 operand's rows for each of the tiles beside it, which over
-// long blocks costs more than the loads that they save (the last four rows); the larger tile would multiply padding.
-static bool wgrad_shape(WgradParams& p, int elem_size) {
+//   460 k  47 x 256           135 / 142               70 /  63
+//   460 k 256 x 64            139 / 150               76 /  60
+//   460 k 512 x 64            248 / 272              129 / 117
+//   460 k  41 x 602           365 / 312              209 / 149
+// Where one side is at most 64 wide, the small tiles split an fp32 operand's rows for each of the tiles beside it.  Over long
+// blocks that costs more than what an oblong tile's wavefronts lose by unequal shares.  fp32, 64 x 64 / oblong, us (m: masked):
+//   60 k  47 x 256   28 /  30      124 k 512 x 64   85 /  84      300 k 256 x 64 m   152 / 140
+//   60 k 512 x 64    44 /  47      124 k  41 x 602  98 /  92      460 k  47 x 256 m  198 / 164
+//   124 k 256 x 64   44 /  46      460 k  47 x 256 153 / 142      460 k  41 x 602 m  657 / 360
+//   460 k 128 x 64   91 /  91      460 k 512 x 64  284 / 272      (one tile: nothing to gain)
+// bf16 has no split to save: 460 k rows of 256 x 64 61 / 67, of 128 x 64 35 / 39.
+struct WgradSides { int n, k; };   // of a tile
+
+static WgradSides wgrad_shape(WgradParams& p, int elem_size) {
   const int64_t step = elem_size == 4 ? 32 : 64;
-  bool big = false;
+  bool big = false, tall = elem_size == 4, wide = tall, is_long = false;
   for (int j = 0; j < p.jobs; ++j) {
     const WgradJob& w = p.job[j];
     big |= w.n > 64 && w.k > 64 && ceil_div(w.n, 128) * ceil_div(w.k, 128) * ceil_div(w.m, 2 * step) >= 256;
+    if (w.k == 0) continue;
+    tall &= w.n > 64 && w.k <= 64;
+    wide &= w.n <= 64 && w.k > 64;
+    is_long |= w.m * (ceil_div(w.n, 128) * ceil_div(w.k, 128)) >= kWgradLongRows;
   }
-  const int64_t tile = big ? 128 : 64;
+  tall &= is_long;
+  wide &= is_long && !tall;
+  const int64_t tile_n = big || tall ? 128 : 64, tile_k = big || wide ? 128 : 64;
   int64_t work = 0, part_row = 0, bytes = 0, most = 1, widest = 1;
   p.tiles = 0;
   for (int j = 0; j < p.jobs; ++j) {
     WgradJob& w = p.job[j];
-    w.tiles_k = static_cast<int>(std::max<int64_t>(ceil_div(w.k, tile), 1));
-    w.tiles = static_cast<int>(ceil_div(w.n, tile) * w.tiles_k);
+    w.tiles_k = static_cast<int>(std::max<int64_t>(ceil_div(w.k, tile_k), 1));
+    w.tiles = static_cast<int>(ceil_div(w.n, tile_n) * w.tiles_k);
     w.stride = ceil_div(w.n * w.k + w.n, 4) * 4;
     p.tiles += w.tiles;
     work += w.m * w.tiles;
@@ -509,20 +529,22 @@ static bool wgrad_shape(WgradParams& p, int elem_size) {
   // a split's rows are addressed with 32-bit offsets, and the loop reads up to 2 kWgradAhead steps past its last one
   const int64_t limit = std::max<int64_t>((int64_t{1} << 30) / widest / step, 1) * step;
   rows = std::min(rows, limit);
-  // ... nor more workgroups than aimed at (one of the larger tiles fills a CU)
+  // ... nor more workgroups than the CUs hold at a time: a few too many are a second round (300 k + 150 k masked rows of
+  // 256 x 64: 236 us with 514 of them, 174 with 512)
   const auto groups = [&](int64_t r) {
     int64_t sum = 0;
     for (int j = 0; j < p.jobs; ++j) sum += ceil_div(p.job[j].m, r) * p.job[j].tiles;
     return sum;
   };
-  while (big && p.tiles <= kWgradGroups && rows < most && groups(rows) > kWgradGroups && rows < limit)
+  const int64_t held = big ? kWgradGroups : kWgradSmallGroups;
+  while (p.tiles <= held && rows < most && groups(rows) > held && rows < limit)
     rows = std::min(rows + ceil_div(rows, 64 * step) * step, limit);
   p.rows_per_split = rows;
   for (int j = 0; j < p.jobs; ++j) p.job[j].splits = static_cast<int>(ceil_div(p.job[j].m, rows));
   p.longer = p.jobs > 1 && p.job[1].splits > p.job[0].splits ? 1 : 0;
   p.common = p.jobs > 1 ? std::min(p.job[0].splits, p.job[1].splits) : p.job[0].splits;
   p.groups = static_cast<int>(groups(rows));
-  return big;
+  return {static_cast<int>(tile_n), static_cast<int>(tile_k)};
 }
 
 static size_t wgrad_bytes(const WgradParams& p) {
@@ -535,14 +557,20 @@ static size_t wgrad_bytes(const WgradParams& p) {
 static bool wgrad_pairs(const void* p, int64_t cols) { return cols % 2 == 0 && (reinterpret_cast<uintptr_t>(p) & 3) == 0; }
 
 template <typename T>
-static void launch_wgrad(const WgradParams& p, bool big, hipStream_t st) {
+static void launch_wgrad(const WgradParams& p, WgradSides tile, hipStream_t st) {
   const bool masked = p.job[0].out != nullptr || p.job[1].out != nullptr;
   const dim3 grid(static_cast<unsigned>(ceil_div(p.groups, 8) * 8)), block(kWgradBlock);
-#define APT_WGRAD(TYPE, F) hipLaunchKernelGGL((wgrad_kernel<TYPE, F, F>), grid, block, (WgradTile<TYPE, F, F>::kLds), st, p)
-  if (masked && big) APT_WGRAD(WgradRelu<T>, 4);
-  else if (masked) APT_WGRAD(WgradRelu<T>, 2);
-  else if (big) APT_WGRAD(T, 4);
-  else APT_WGRAD(T, 2);
+#define APT_WGRAD(N, K) \
+  hipLaunchKernelGGL((masked ? wgrad_kernel<WgradRelu<T>, N, K> : wgrad_kernel<T, N, K>), grid, block, \
+                     (WgradTile<T, N, K>::kLds), st, p)
+  if (tile.n == 128 && tile.k == 128) {
+    APT_WGRAD(4, 4);
+  } else if (tile.n == tile.k) {
+    APT_WGRAD(2, 2);
+  } else if constexpr (WgradType<T>::kParts == 3) {
+    if (tile.n > tile.k) APT_WGRAD(4, 2);
+    else APT_WGRAD(2, 4);
+  }
 #undef APT_WGRAD
 }
 
@@ -583,7 +611,7 @@ extern "C" int apt_linear_wgrads(const apt_wgrad_product* products, int count, i
   const char* who = "apt_linear_wgrads";
   WgradParams p{};
   if (const int rc = wgrad_params(who, products, count, elem_size, p)) return rc;
-  const bool big = wgrad_shape(p, elem_size);
+  const WgradSides tile = wgrad_shape(p, elem_size);
   APT_REQUIRE(workspace != nullptr && workspace_bytes >= wgrad_bytes(p) && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0,
               APT_EWORKSPACE, "%s: workspace too small or not 16-byte aligned (see apt_linear_wgrads_workspace_bytes)", who);
   float* part = static_cast<float*>(workspace);
@@ -602,9 +630,9 @@ extern "C" int apt_linear_wgrads(const apt_wgrad_product* products, int count, i
   }
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (any) {
-    if (elem_size == 4) launch_wgrad<float>(p, big, st);
-    else if (odd) launch_wgrad<WgradOdd>(p, big, st);
-    else launch_wgrad<uint16_t>(p, big, st);
+    if (elem_size == 4) launch_wgrad<float>(p, tile, st);
+    else if (odd) launch_wgrad<WgradOdd>(p, tile, st);
+    else launch_wgrad<uint16_t>(p, tile, st);
     APT_LAUNCH_CHECK("wgrad_kernel");
   }
   const dim3 grid(static_cast<unsigned>(sum_blocks[0] + sum_blocks[1])), block(kWgradSumBlock);

@@ -154,3 +154,28 @@ def test_linear_wgrads_of_different_lengths(capi, sizes, dtype):
             want, size = a.t() @ x.double(), a.abs().t() @ x.double().abs()
             assert bool(((dw.double() - want).abs() <= (m / 32 + 40) * 2.0 ** -24 * size + half * want.abs()).all())
         assert bool(((db.double() - a.sum(0)).abs() <= (m / 8 + 8) * 2.0 ** -24 * a.abs().sum(0) + half * a.sum(0).abs()).all())
+
+
+@pytest.mark.parametrize("mask", [False, True])
+@pytest.mark.parametrize("sizes", [((16411, 33, 4090),), ((16411, 4100, 17),), ((131073, 64, 470), (1000, 3, 65)), ((131073, 470, 64), (77, 65, 1)),
+                                   ((131073, 470, 50), (9000, 470, 0)), ((262144, 129, 1),), ((262143, 1, 130),)])
+def test_linear_wgrads_of_oblong_tiles(capi, sizes, mask):
+    """Long blocks of which one side is at most 64 wide: tiles of 128 x 64 and 64 x 128.  With an infinite element the tiles it
+    reaches are formed again in fp32."""
+    gen = torch.Generator(device=DEV).manual_seed(9)
+    draw = lambda *shape: torch.randn(*shape, generator=gen, device=DEV)  # noqa: E731
+    for infinite in (False, True):
+        products = [(draw(m, n), draw(m, k) if k else None, draw(m, n) if mask else None, True) for m, n, k in sizes]
+        if infinite:
+            products[0][1][100, 0], products[0][0][100, 0] = float("inf"), 0.5
+            if mask:
+                products[0][2][100, 0] = 1.0
+        for (dw, db), (dy, x, y, _) in zip(capi.linear_wgrads(products), products):
+            a, m = dy.double() if y is None else torch.where(y > 0, dy, torch.zeros_like(dy)).double(), dy.shape[0]
+            if x is not None:
+                # a workgroup's rows (an LDS step of 32 at a time, or one by one) and the partials, each rounded once
+                want, size = a.t() @ x.double(), a.abs().t() @ x.double().abs()
+                ok = want.isfinite()
+                assert torch.equal(dw.isnan(), want.isnan()) and torch.equal(dw.isinf(), want.isinf()) and bool((~ok).any()) == (infinite and x is products[0][1])
+                assert bool(((dw.double() - want).abs() <= (m / 32 + 40) * 2.0 ** -24 * size + 2.0 ** -23 * want.abs())[ok].all())
+            assert bool(((db.double() - a.sum(0)).abs() <= (m / 8 + 8) * 2.0 ** -24 * a.abs().sum(0) + 2.0 ** -23 * a.sum(0).abs()).all())

@@ -125,7 +125,10 @@ LAYER_BUDGETS = {
                       "void apt::gat_pair_scores_kernel<unsigned short, 8, 8, 32>(": 6,
                       "void apt::gat_pair_scores_kernel<float, 4, 16, 64>(": 8,
                       "void apt::gat_param_grad_kernel<unsigned short, 8>(": 2, "void apt::gat_param_grad_kernel<float, 4>(": 3},
-    "linear.hip": {"void apt::wgrad_kernel<float, 4, 4>(": 2, "void apt::wgrad_kernel<unsigned short, 4, 4>(": 2},
+    "linear.hip": {"void apt::wgrad_kernel<float, 4, 4>(": 2, "void apt::wgrad_kernel<unsigned short, 4, 4>(": 2,
+                   # two workgroups on a CU
+                   "void apt::wgrad_kernel<apt::WgradRelu<float>, 2, 2>(": 4, "void apt::wgrad_kernel<apt::WgradRelu<float>, 2, 4>(": 4,
+                   "void apt::wgrad_kernel<apt::WgradRelu<float>, 4, 2>(": 4},
     "rows_gemm.hip": {"void apt::rows_gemm_kernel<4, 4, 4>(": 2, "void apt::rows_gemm_kernel<4, 1, 4>(": 3,
                       "void apt::rows_gemm_kernel<1, 2, 4>(": 2, "void apt::add_rows_kernel<float, 4>(": 8,
                       "void apt::rows_gemm_resident_kernel<8>(": 2, "void apt::rows_gemm_resident_kernel<4>(": 3,
