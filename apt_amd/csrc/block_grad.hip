@@ -163,7 +163,9 @@ __global__ __launch_bounds__(kAggBlock) __attribute__((amdgpu_num_sgpr(kFullSgpr
       walk(edge(at, at < hi), 0, static_cast<int>(min((hi - e + kGroups - 1) / kGroups, static_cast<int64_t>(LPR))), c, acc);
     }
   };
-  // The groups' sums together, in order, for the first group.
+  // The groups' sums together, in order, for the first group.  Many groups' are read eight at a time (256 workgroups of 32 groups
+  // and a hub or two each: 9 us, 17 one by one); for few groups the registers would cost more (8 bf16 a lane: 122 to 131 us).
+  constexpr int kMeeting = kGroups > 8 ? 8 : 1;
   auto over_groups = [&](float (&acc)[VEC]) {
 #pragma unroll
     for (int k = 0; k < VEC; ++k) s_sum[grp][l * VEC + k] = acc[k];
@@ -172,7 +174,7 @@ __global__ __launch_bounds__(kAggBlock) __attribute__((amdgpu_num_sgpr(kFullSgpr
 #pragma unroll
       for (int k = 0; k < VEC; ++k) {
         float sum = 0.f;
-#pragma unroll 1
+#pragma unroll kMeeting
         for (int g = 0; g < kGroups; ++g) sum += s_sum[g][l * VEC + k];
         acc[k] = sum;
       }
