@@ -30,8 +30,8 @@ template <int GROUPS> __device__ __forceinline__ int64_t group_row(int grp, uint
 // of a launch.  30 k rows of 25 edges, 47 / 256 bf16: 64 / 60 us, with 32 instead of 64 edges 67 / 70; 238 k sampled
 // sources, 64 bf16, 32 instead of 128 edges for the narrowest groups: 204 us instead of 145.  With hubs for a quarter / an
 // eighth / a sixteenth of the groups: 2 k skewed rows of 25 k edges, 16 bf16, 95 / 41 / 42 us; 8 k rows of 125 edges, 16 fp32,
-// 63 / 63 / 80.
+// 63 / 63 / 80.  A workgroup's only hub is always all groups' (256 x 10 skewed edges into 2 k rows of 100 fp32: 6.4 us, 12.2 alone).
 template <int LPR> constexpr int hub_shared() { return LPR <= 8 ? 128 : LPR >= 32 ? 64 : 32; }
-template <int GROUPS> constexpr int hubs_apiece() { return GROUPS / 8; }
+template <int GROUPS> constexpr int hubs_apiece() { return GROUPS > 16 ? GROUPS / 8 : 2; }
 
 }  // namespace apt
