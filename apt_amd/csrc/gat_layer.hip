@@ -220,9 +220,10 @@ struct GatSourceParams {
 // destinations) and little else: a group has kRows rows in flight with their first edges, loads stand outside branches
 // (a conversion inside one waits for its load), and what depends on the columns alone (heads, parameters) is taken out
 // of the loop over the rows.  Rows and hubs are dealt as in block_grad.hip (grouped_rows.hpp).  124 k rows of 4 x 64 bf16,
-// 261 k edges (63 MB written, 134 MB of destinations' rows read): 61 us; 72 with four rows in flight (161 registers
-// instead of 111), neighbouring rows on different XCDs and every hub a workgroup's; 193 with a wavefront per row, loads in
-// branches and the heads worked out per row.  (Three or four rows in flight where a lane reads one element: no faster.)
+// 261 k edges (63 MB written, 134 MB of destinations' rows read): 65 us, 61 when four neighbouring rows were a workgroup's
+// (grouped_rows.hpp says why they are not); 72 with four rows in flight (161 registers instead of 111), neighbouring rows on
+// different XCDs and every hub a workgroup's; 193 with a wavefront per row, loads in branches and the heads worked out per
+// row.  (Three or four rows in flight where a lane reads one element: no faster.)
 // Workgroups, 2048 / 4096, whole backward pass of 240 k sources 500 k edges, us: 2 x 101 fp32 812 / 759, 4 x 64 fp32 361 / 369,
 // bf16 238 / 240; 124 k sampled rows of 4 x 64 bf16, the kernel alone, 41 / 43.
 // TWO: a lane's features may belong to two heads.

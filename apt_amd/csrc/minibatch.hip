@@ -867,3 +867,25 @@ extern "C" int apt_relabel_ranked(const int64_t* seeds, int64_t num_seeds, const
   }
   return APT_OK;
 }
+
+namespace apt {
+
+__global__ void publish_words_kernel(const int64_t* __restrict__ a, int na, const int64_t* __restrict__ b, int nb,
+                                     const int64_t* __restrict__ c, int nc, int64_t* __restrict__ host_words) {
+  for (int t = threadIdx.x; t < na; t += kWave) host_words[t] = a[t];
+  for (int t = threadIdx.x; t < nb; t += kWave) host_words[na + t] = b[t];
+  for (int t = threadIdx.x; t < nc; t += kWave) host_words[na + nb + t] = c[t];
+}
+
+}  // namespace apt
+
+extern "C" int apt_publish_words(const int64_t* a, int na, const int64_t* b, int nb, const int64_t* c, int nc,
+                                 int64_t* host_words, void* stream) {
+  using namespace apt;
+  APT_REQUIRE(na >= 0 && nb >= 0 && nc >= 0 && (na == 0 || a != nullptr) && (nb == 0 || b != nullptr) &&
+                  (nc == 0 || c != nullptr) && host_words != nullptr,
+              APT_EINVAL, "apt_publish_words: a tensor is NULL or a count negative");
+  hipLaunchKernelGGL(publish_words_kernel, dim3(1), dim3(kWave), 0, static_cast<hipStream_t>(stream), a, na, b, nb, c, nc, host_words);
+  APT_LAUNCH_CHECK("publish_words_kernel");
+  return APT_OK;
+}

@@ -18,9 +18,9 @@
 //   40 k rows, 256 -> 256            50 /  57          6e-8 / 2.0e-7
 //   170 k rows, 256 -> 47            76 /  75          5e-8 / 1.9e-7
 //   1 k rows, 256 + 256 -> 47        22 /  42          8e-8 / 2.4e-7
-// The first: 111 k of 306 k cycles on the matrix units (46 us at their rate), 72 k on the split and addresses, 310 MB of
-// rows and results (55 us); the workgroups of a launch read, multiply and write much in step.  Up to four steps of depth:
-// rows_gemm_resident.hpp (460 k rows, 100 -> 256 212 us, 230 here).
+// The first has 46 us on the matrix units at their rate and 310 MB of rows and results (55 us); in the layers' passes the
+// matrix units work 39 % of this kernel's cycles and the vector units, which split, 33 %: the workgroups of a launch read,
+// multiply and write much in step.  Where the weights fit LDS: rows_gemm_resident.hpp (460 k rows, 100 -> 256 212 us, 230 here).
 #include <algorithm>
 
 #include "common.hpp"

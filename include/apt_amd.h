@@ -434,6 +434,12 @@ int apt_minibatch_sample(const apt_graph* graph, const int64_t* seeds, int64_t b
                          int64_t* const* counts, int64_t* sizes, void* workspace,
                          size_t workspace_bytes, void* stream);
 
+/* Up to three short arrays of device memory (a batch's sizes, its request sizes), one
+ * behind the other, into pinned host memory by a kernel: readable once the stream has
+ * passed it (an event behind it), without a copy that waits for the rest of the batch. */
+int apt_publish_words(const int64_t* a, int na, const int64_t* b, int nb, const int64_t* c, int nc,
+                      int64_t* host_words, void* stream);
+
 /* apt_minibatch_sample in two parts, for a caller that gathers the batch's
  * features right after sampling it (no counterpart in the reference, where
  * sampling and load_subtensor are separate operators, python/npc/sampler.py:
@@ -595,11 +601,6 @@ typedef struct apt_epoch_cost {
   double release_seconds;       /* apt_epoch_release, asking the consumer's stream whether it is idle */
 } apt_epoch_cost;
 int apt_epoch_host_cost(apt_epoch* epoch, apt_epoch_cost* cost);
-
-/* Up to three short arrays of device memory, one behind the other, into pinned host
- * memory by a kernel: readable once the stream has passed it (an event behind it). */
-int apt_publish_words(const int64_t* a, int na, const int64_t* b, int nb, const int64_t* c, int nc,
-                      int64_t* host_words, void* stream);
 
 /* Cache construction (the callers of the registries).
  *   apt_count_ids        freq[ids[i]] += 1 for ids in [0, num_total_nodes): the
@@ -931,15 +932,6 @@ size_t apt_linear_wgrad_workspace_bytes(int64_t m, int64_t n, int64_t k, int ele
 int apt_linear_wgrad(const void* dy, const void* x, int64_t m, int64_t n, int64_t k, int elem_size,
                      void* dw, void* db, void* workspace, size_t workspace_bytes, void* stream);
 
-/* apt_rows_gemm in bf16 (fp32 sums, rounded once where they are stored; accumulate
- * adds what y holds to the sum).  Weights must be contiguous along one of their
- * sides; no workspace.  apt_rows_product_fits: 1 if the weights of a column tile
- * fit LDS (k1 + k2 up to about 1000) and the sizes are in range. */
-int apt_rows_product_fits(int64_t m, int64_t n, int64_t k1, int64_t k2);
-int apt_rows_product(const void* x1, int64_t k1, const void* w1, int64_t w1_stride_n, int64_t w1_stride_k,
-                     const void* x2, int64_t k2, const void* w2, int64_t w2_stride_n, int64_t w2_stride_k,
-                     int64_t m, int64_t m2, int64_t n, const void* bias, int accumulate, int relu, void* y, void* stream);
-
 /* One or two such products (count) of one type in one launch, each with its own
  * rows and sizes.  out [m, n], optional: the result of a ReLU that dy is the
  * gradient of; dy counts where out > 0.  k = 0: the column sums alone (x and dw
@@ -956,6 +948,15 @@ typedef struct apt_wgrad_product {
 size_t apt_linear_wgrads_workspace_bytes(const apt_wgrad_product* products, int count, int elem_size);
 int apt_linear_wgrads(const apt_wgrad_product* products, int count, int elem_size, void* workspace,
                       size_t workspace_bytes, void* stream);
+
+/* apt_rows_gemm in bf16 (fp32 sums, rounded once where they are stored; accumulate
+ * adds what y holds to the sum).  Weights must be contiguous along one of their
+ * sides; no workspace.  apt_rows_product_fits: 1 if the weights of a column tile
+ * fit LDS (k1 + k2 up to about 1000) and the sizes are in range. */
+int apt_rows_product_fits(int64_t m, int64_t n, int64_t k1, int64_t k2);
+int apt_rows_product(const void* x1, int64_t k1, const void* w1, int64_t w1_stride_n, int64_t w1_stride_k,
+                     const void* x2, int64_t k2, const void* w2, int64_t w2_stride_n, int64_t w2_stride_k,
+                     int64_t m, int64_t m2, int64_t n, const void* bias, int accumulate, int relu, void* y, void* stream);
 
 #ifdef __cplusplus
 }
